@@ -74,7 +74,7 @@ def build(verbose=False):
     outs.append(_run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs))
     # host cells ("Frame_HIP" model): plain C++ over the C ABI
     glue = os.path.join(CSRC, "frame_hip")
-    outs.append(_run([os.environ.get("CXX", "g++"), "-std=c++14", "-O2", "-fPIC", "-Wall", "-Wextra", "-Wno-unused-parameter",
+    outs.append(_run([os.environ.get("CXX", "g++"), "-std=c++14", "-O2", "-fopenmp", "-fPIC", "-Wall", "-Wextra", "-Wno-unused-parameter",
                       "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + os.path.join(ROOT, "include"), "-shared",
                       os.path.join(glue, "frame_hip.cpp"), os.path.join(glue, "quantization.cpp"), os.path.join(glue, "qat_fuse.cpp"),
                       os.path.join(glue, "frame_hip_capi.cpp"),

@@ -127,7 +127,7 @@ void checkStatus(int status);
 // still read N2D2-style float tensors (the role CudaTensor plays, include/containers/CudaTensor.hpp:256-359).
 class HipTensor {
 public:
-    HipTensor() : mDesc(), mBytes(0), mHostValid(false) {}
+    HipTensor() : mDesc(), mBytes(0), mHostValid(false), mReadback(nullptr), mReadbackBytes(0) {}
     ~HipTensor();
     HipTensor(const HipTensor&) = delete;
     HipTensor& operator=(const HipTensor&) = delete;
@@ -150,6 +150,8 @@ private:
     size_t mBytes;
     Tensor<Float_T> mHost;
     bool mHostValid;
+    void* mReadback;           // pinned host memory the read-back of a small tensor goes through, kept from call to call
+    size_t mReadbackBytes;
 };
 
 // ---------------------------------------------------------------- ScalingMode
@@ -1107,6 +1109,9 @@ private:
 class DeepNet {
 public:
     DeepNet() {}
+    ~DeepNet();
+    DeepNet(const DeepNet&) = delete;
+    DeepNet& operator=(const DeepNet&) = delete;
     // parents empty = connected to the environment
     void addCell(const std::shared_ptr<Cell>& cell, const std::vector<std::shared_ptr<Cell> >& parents);
     std::shared_ptr<Cell> getCell(const std::string& name) const;
@@ -1114,6 +1119,8 @@ public:
     // environment: integer-valued stimuli {W,H,C,B}
     void setStimuli(unsigned int nbChannels, unsigned int height, unsigned int width, unsigned int batchSize);
     void setStimuliData(const Tensor<Float_T>& data);
+    // The same from plain memory that holds such a tensor
+    void setStimuliData(const Float_T* data, size_t dimX, size_t dimY, size_t dimZ, size_t dimB);
     HipTensor& getStimuli() { return mStimuli; }
     void initialize();
     void propagate(bool inference = true);
@@ -1136,7 +1143,13 @@ public:
 private:
     void planFusion();
     void layoutStimuli();
-    Tensor<Float_T> mStimuliHost;          // what setStimuliData() was given last
+    void convertStimuli();
+    // What setStimuliData() was given last, as byte planes {W,H,C,B} (uint8 or int8) on the device; mStimuliBytes is the
+    // pinned host memory they are narrowed into on their way there
+    n2d2hip_tensor mStimuliPlanes = {};
+    unsigned char* mStimuliBytes = nullptr;
+    size_t mStimuliCapacity = 0;
+    bool mStimuliValid = false;
     bool mFusion = true, mPlanned = false;
     std::vector<std::shared_ptr<Cell> > mOrder;
     std::vector<Cell_Frame_HIP*> mFrames;  // mOrder, as the cells' device side

@@ -126,9 +126,9 @@ int fh_net_propagate(void* net) { return guarded([&] { ((Net*)net)->deepNet->pro
 int fh_net_set_stimuli(void* net, const float* data, int C, int H, int W, int B)
 {
     return guarded([&] {
-        Tensor<Float_T> t({(size_t)W, (size_t)H, (size_t)C, (size_t)B});
-        std::memcpy(t.data(), data, t.size() * sizeof(float));
-        ((Net*)net)->deepNet->setStimuliData(t);
+        // (a view of the caller's values: nothing is copied before they are narrowed)
+        if (C < 0 || H < 0 || W < 0 || B < 0) throw std::runtime_error("fh_net_set_stimuli(): bad dimensions");
+        ((Net*)net)->deepNet->setStimuliData(data, (size_t)W, (size_t)H, (size_t)C, (size_t)B);
     });
 }
 

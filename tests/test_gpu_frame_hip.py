@@ -70,6 +70,26 @@ def cells_of(spec, x, keep):
     return cells.run_net(spec, x, keep=keep)
 
 
+@pytest.mark.parametrize("batch", [1, 64, 65])          # one slice of 64 K values, its last full one, one value into the next ones
+def test_stimuli_are_checked_and_narrowed_in_slices(fh, batch):
+    from n2d2_amd import nets
+    spec = nets.lenet()
+    x = np.random.default_rng(35).integers(0, 256, size=(batch, 1, 32, 32))
+    x[-1, 0, -1, -1] = 255
+    net = _compare(fh, spec, x, ["fc3"])
+    before = net.outputs("fc3")
+    for bad in (256.0, -1.0, 0.5, float("nan"), 3e9):
+        y = x.astype(np.float32)
+        y[-1, 0, -1, -2] = bad
+        with pytest.raises(fh.FrameHipError) as e:
+            net.set_stimuli(y)
+        assert "is not an integer in [0,255]" in str(e.value)
+    # a refused batch leaves the one before it in place, also through a change of the plan
+    net.set_fusion(False)
+    net.propagate()
+    assert np.array_equal(net.outputs("fc3"), before)
+
+
 def test_resnet50_through_the_registrar(fh):
     from n2d2_amd import nets
     spec = nets.resnet50()
