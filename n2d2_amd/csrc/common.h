@@ -109,6 +109,30 @@ const char* targs_of(const char* kernel)
 #define N2D2HIP_LAUNCH_T(K, TARGS, grid, block, lds, stream, ...)                                              \
     ::n2d2hip::launch_kernel<&K<N2D2HIP_UNPAREN TARGS>>(::n2d2hip::targs_of<&K<N2D2HIP_UNPAREN TARGS>, N2D2HIP_UNPAREN TARGS>(#K), grid, block, lds, stream, __VA_ARGS__)
 
+// (multiplier, shift) with n / d == umulhi(n, multiplier) >> shift for 0 <= n < 2^31; multiplier 0 stands for d == 1
+inline void magic_div(unsigned d, unsigned* mul, unsigned* sh)
+{
+    if (d <= 1) { *mul = 0; *sh = 0; return; }
+    unsigned s = 0;
+    while ((1ull << s) < d) ++s;
+    *mul = (unsigned)((1ull << (31 + s)) / d + 1);
+    *sh = s - 1;
+}
+
+// Compute units of the current device
+inline int num_cus()
+{
+    static int n = 0;
+    if (n == 0) {
+        hipDeviceProp_t prop;
+        int dev = 0;
+        if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
+            n = prop.multiProcessorCount;
+        if (n <= 0) n = 256;
+    }
+    return n;
+}
+
 // ---------------------------------------------------------------- epilogue
 // Device-side form of "Scaling::propagate, saturate, Rectifier/Linear" for one
 // cell.  Per-channel tables live in one device allocation of 5 int arrays of

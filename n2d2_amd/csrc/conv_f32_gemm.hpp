@@ -1,290 +1,959 @@
 // Float32 convolution (forward, backward-data, backward-filter) as an implicit GEMM on the fp32 matrix cores
 // (v_mfma_f32_32x32x2f32), for ungrouped convolutions without dilation on N2D2's NCHW / OCHW tensors.
 //
-// One kernel, three addressings.  The product is out[q][p] = sum_k Qop[q][k] * Pop[k][p], where p runs along the
-// dimension that is contiguous in the output tensor (so that the 32 lanes holding one accumulator row write 128
-// consecutive bytes) and q along the other one:
-//   forward          p = output pixel (b,oy,ox)   q = output channel   k = (c,ty,tx)      Pop = x gathered, Qop = w
-//   backward data    p = input pixel (b,iy,ix)    q = input channel    k = (o,ty,tx)      Pop = dy gathered, Qop = w
-//   backward filter  p = weight (c,ty,tx)         q = output channel   k = pixel (b,oy,ox) Pop = x gathered, Qop = dy
+// The product is out[q][p] = sum_k Qop[q][k] * Pop[k][p]:
+//   forward          p = output pixel   q = output channel   k = (input channel, tap)    Pop = x gathered, Qop = w
+//   backward data    p = input pixel    q = input channel    k = (output channel, tap)   Pop = dy gathered, Qop = w
+//   backward filter  p = (channel, tap) q = output channel   k = output pixel            Pop = x gathered, Qop = dy
 // Taps that fall outside the tensor contribute zero, which is what the reference's clipped window computes.
 //
-// A block of 256 threads (4 waves as 2 x 2) owns a 128 (q) x 128 (p) tile; each wave 64 x 64 as 2 x 2 MFMA tiles.  With at
-// most 64 rows of q (QT = 64) the four waves sit side by side along p instead, each 64 x 32.
-// K advances in steps of 16 through two LDS tiles [k][p] and [k][q] (row stride 129 floats); the next step's
-// elements are fetched into registers while the matrix cores work on the current one and are written to the other pair
-// of tiles, so one barrier per step suffices.  Backward-filter, whose K is
-// the whole batch of pixels and whose output is small, splits K over blockIdx.z into partial results that a second
-// kernel adds up in a fixed order; forward and backward-data do the same when their tiles alone would not fill the chip.
+// Bound by the matrix cores: an fp32 matrix instruction is 4096 flops in 64 cycles, which is the rate of the vector ALU, and
+// it runs on that ALU: every vector instruction beside it takes its 4 cycles from it (measured: loads and address
+// arithmetic left out, the products alone take as much less time as those take alone).  So:
+//  * operands go global -> LDS by direct loads (no registers on the way), into a ring of stages, and everything that does not
+//    differ from lane to lane is scalar: a load adds a scalar offset to a per-lane one.  What does not exist (padding, edges
+//    of tile and K range) is requested past the end of the buffer descriptor; the LDS receives 0.
+//  * 3x3 kernels, forward and at stride 1 backward, keep a lane's nine offsets in registers, so that a load costs no vector
+//    instruction; 1x1 kernels and strided backward-data run K over chunks of 16 channels at one tap, so that the test whether
+//    the tap lies inside the input is made once per step.  A small kernel lays the weights out for both first.  Any other
+//    forward kernel, and short passes, test every load.
+//  * backward-data of a strided convolution runs one residue class of input pixels at a time: the taps of a class form a
+//    dense stride-1 convolution of dy, so no tap is tried that cannot hit (a 3x3 of stride 2: 9 taps for 4 classes, where
+//    trying all of them is 36).
+//  * rows of LDS that hold consecutive k hold the even ones in front of the odd ones, or (filter) give the two lane halves of
+//    an instruction different groups of 4 k, so that a lane reads four instructions' operands in 16 bytes.
+// A forward sum is added in one order whatever kernel takes it: channel, tap, in pairs, in ranges that follow from the sizes.
+// Backward-filter, whose K is the whole batch of pixels and whose output is small, splits K over blockIdx.z into partial
+// results that a second kernel adds up in a fixed order; forward and backward-data do the same when their tiles alone would
+// not fill the chip.
+// Measured (us, forward / data / filter, before: 128 x 128 tiles, operands through registers, one test per load; now):
+//   64 -> 64, 3x3, 56 x 56, batch 64             236 / 284 / 263    149 / 157 / 180   (15 GFLOP: 99, 94, 82 TFLOP/s of 154)
+//   128 -> 256, 3x3 stride 2, 27 x 27, batch 33   80 / 277 /  76     55 /  53 /  58
+//   a layer spanning its input, 16384 -> 10, 64  2632 /  27 / 222    116 /   7 /   8
+// A CU takes whole tiles, so the last round costs its share: 64 -> 64 on 56 x 56 at batch 64 is 12.25 tiles for each.
 #pragma once
 
 #include "common.h"
+#include "mfma_util.hpp"
 
 namespace n2d2hip {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v2f __attribute__((ext_vector_type(2)));
 
-enum { GEMM_FWD = 0, GEMM_BWD_DATA = 1, GEMM_BWD_FILTER = 2 };
-
-struct GemmF32 {
-    int B, C, H, W, O, oH, oW, kW, kH;
-    int sx, sy, pl, pt;
-    int P, Q, K;          // GEMM extents
-    int kchunk;           // K range of one blockIdx.z (a multiple of 16)
-    unsigned bytesP, bytesQ;   // sizes of the two operand tensors (each at most 2 GiB)
+struct DivF32 {
+    unsigned mul, sh;
 };
 
-constexpr int GT = 128;       // tile edge (both p and q)
-constexpr int GK = 16;        // K step
-constexpr int GLD = GT + 1;   // LDS row stride in floats
+// The pixels of one launch: all output pixels (forward), or the input pixels of one residue class modulo the stride.
+struct PixelClass {
+    int tile0;                 // first tile of this class
+    int P, gW, gHW;            // pixels over all images; row length and pixels per image of the class's grid
+    int nx, nT;                // taps along x, taps
+    int ty0, tx0;              // first tap; the next one along an axis is osy / osx further in the kernel
+    int y0, x0;                // source position of tap (0, 0) for grid pixel (0, 0)
+    int stepy, stepx;          // element offset from one tap to the next in the source plane
+    int soff0, bias;           // element offset of tap (0, 0) against the moved base `src - bias`; both make every offset >= 0
+    int ry, rx;                // output position of grid pixel (py, px): (py * osy + ry, px * osx + rx)
+    DivF32 ghw, gw, nt, nxd;
+};
+constexpr int PIXEL_CLASSES = 4;
 
-template <int MODE, int QT>
-__global__ __launch_bounds__(256) void conv_f32_gemm_kernel(GemmF32 g, const float* __restrict__ srcP, const float* __restrict__ srcQ,
-                                                            const float* __restrict__ bias, float beta, float* __restrict__ out)
+struct PixelGemm {
+    int Q, Ch;                 // rows of q; channels that k runs over
+    int kchunk;                // a K range (a multiple of GK; chunked K: in steps of GK)
+    int nz;                    // K ranges of a block: blockIdx.z * nz ...
+    int sy, sx, d;             // source step per grid pixel (the strides; 1 for backward-data); +1 / -1: per tap
+    int Hs, Ws, planeS;        // source plane
+    int qs, chs, kW;           // weight element (q, ch, ty, tx) at q * qs + ch * chs + ty * kW + tx
+    int osy, osx;              // backward-data: the strides (1 forward)
+    int planeO, Wo;            // output plane and its row length
+    int ptiles, ptiles8, qtiles;
+    int qpad, T;               // chunked K: rows of q in the laid-out weights, taps of the kernel
+    unsigned bytesX, bytesW;   // sizes of the operand tensors (below 2 GiB)
+    int nclass;
+    PixelClass c[PIXEL_CLASSES];
+};
+
+struct FilterGemm {
+    int P, Q, K;
+    int kchunk;                // K range of one blockIdx.z (a multiple of FK)
+    int C, H, W, kW, kH, s_y, s_x, pt, pl;
+    int oW, plane;             // output row length and plane
+    int imgX, imgY;
+    int ctiles;                // by taps: tiles of channels
+    unsigned bytesX, bytesY;
+    DivF32 dplane, dow;
+};
+
+constexpr int GK = 16;         // K step of the pixel kernels
+constexpr int FK = 32;         // of the filter kernel
+constexpr unsigned F32_OOB = 0x80000000u;      // byte offset past the end of every operand
+
+__device__ __forceinline__ int div_f32(int n, DivF32 d) { return div_magic(n, d.mul, d.sh); }
+
+template <int OFF>
+__device__ __forceinline__ void lds_read128f(v4f& v, unsigned addr)
 {
-    __shared__ float Pbuf[2][GK * GLD];
-    __shared__ float Qbuf[2][GK * GLD];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    constexpr int NP = QT / 64;                 // 32-column MFMA tiles of p per wave
-    constexpr int NQL = QT / 16;                // q elements a thread fetches per step
-    const int wq = (QT == 128) ? (wave >> 1) : 0;
-    const int pw = (QT == 128) ? (wave & 1) * 64 : wave * 32;     // the wave's first p inside the tile
-    const int ptile = blockIdx.x * GT, qtile = blockIdx.y * QT;
-    const int kbeg = blockIdx.z * g.kchunk, kend = min(kbeg + g.kchunk, g.K);
-    const int kHW = g.kH * g.kW;
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF) : "memory");
+}
+template <int OFF>
+__device__ __forceinline__ void lds_read64f(v2f& v, unsigned addr)
+{
+    asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF) : "memory");
+}
+// two dwords, OFF0 and OFF1 in units of 256 bytes
+template <int OFF0, int OFF1>
+__device__ __forceinline__ void lds_read2st64f(v2f& v, unsigned addr)
+{
+    static_assert(OFF0 < 256 && OFF1 < 256, "8-bit offsets");
+    asm volatile("ds_read2st64_b32 %0, %1 offset0:%2 offset1:%3" : "=v"(v) : "v"(addr), "n"(OFF0), "n"(OFF1) : "memory");
+}
+__device__ __forceinline__ void tie(v4f& x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ void tie(v2f& x) { asm volatile("" : "+v"(x)); }
 
-    // ---- per-thread loader state.  FWD / BWD_DATA: thread owns one p (and one q) and 8 consecutive k of each step.
-    // BWD_FILTER: thread owns one k of each step and 8 p (and 8 q) spaced by 16.
-    const int lp = (MODE == GEMM_BWD_FILTER) ? (t >> 4) : (t & 127);     // first local p (and q for BWD_DATA / BWD_FILTER)
-    const int lk = (MODE == GEMM_BWD_FILTER) ? (t & 15) : ((t >> 7) * 8); // first local k
-    // Q operand of FWD (weights, contiguous along k): q = t / (16 / NQL), k = (t % (16 / NQL)) * NQL + i;
-    // of BWD_DATA: q = t % QT, k = (t / QT) * NQL + i
-    const int lq_w = (MODE == GEMM_FWD) ? t / (16 / NQL) : t % QT;
-    const int lk_w = (MODE == GEMM_FWD) ? (t % (16 / NQL)) * NQL : (t / QT) * NQL;
-
-    // Operands are read through buffer descriptors: an element that does not exist (padding, past the tile or the K
-    // range) is requested at an offset past the end and comes back as zero, so the loads need no branches.  All
-    // offsets fit 32 bits (checked by the host).
-    const __amdgpu_buffer_rsrc_t rsrcP = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(srcP), 0, g.bytesP, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rsrcQ = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(srcQ), 0, g.bytesQ, 0x00020000);
-    auto ldP = [&](int off, bool valid) -> float {
-        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrcP, valid ? (unsigned)off * 4u : 0x80000000u, 0, 0));
-    };
-    auto ldQ = [&](int off, bool valid) -> float {
-        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrcQ, valid ? (unsigned)off * 4u : 0x80000000u, 0, 0));
-    };
-    int pb = 0, py = 0, px = 0;             // decoded p (FWD: b,oy,ox; BWD_DATA: b,iy,ix)
-    bool pvalid = false;
-    int pbase = 0;                          // FWD: offset of tap (0,0) of channel 0 for this pixel; BWD_DATA: of (b, o = 0)
-    unsigned long long tapmask = 0;         // FWD: bit ty*kW+tx set if that tap lies inside the input (kH*kW <= 64)
-    int poff[8], pty[8], ptx[8];            // BWD_FILTER: p_i = (c,ty,tx): offset c*H*W + ty*W + tx (-1: no such p), ty, tx
-    if (MODE == GEMM_BWD_FILTER) {
+// Which tile a block of the forward / backward-data kernels takes.  Blocks 8 apart share an XCD and its L2: the q tiles of a
+// pixel tile come one behind the other on one XCD, and an XCD takes consecutive pixel tiles (they share their halo).  With
+// several classes, whose tiles differ in length, the tiles are dealt in turn instead.
+__device__ __forceinline__ bool pixel_tile(const PixelGemm& g, int* tile, int* qtile, int* ci)
+{
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, pt = slot / g.qtiles;
+    *qtile = slot - pt * g.qtiles;
+    *tile = g.nclass == 1 ? xcd * g.ptiles8 + pt : pt * 8 + xcd;
+    *ci = 0;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int p = ptile + lp + 16 * i;
-            const int pp = min(p, g.P - 1);
-            pty[i] = (pp % kHW) / g.kW;
-            ptx[i] = pp % g.kW;
-            poff[i] = (p < g.P) ? (pp / kHW) * g.H * g.W + pty[i] * g.W + ptx[i] : -1;
-        }
-    } else {
-        const int p = ptile + lp;
-        pvalid = p < g.P;
-        const int plane = (MODE == GEMM_FWD) ? g.oH * g.oW : g.H * g.W;
-        const int row = (MODE == GEMM_FWD) ? g.oW : g.W;
-        const int pp = pvalid ? p : 0;
-        pb = pp / plane;
-        py = (pp % plane) / row;
-        px = pp % row;
-        if (MODE == GEMM_FWD) {
-            const int iy0 = py * g.sy - g.pt, ix0 = px * g.sx - g.pl;
-            pbase = (pb * g.C * g.H + iy0) * g.W + ix0;
-            if (pvalid)
-                for (int ty = 0; ty < g.kH; ++ty)
-                    for (int tx = 0; tx < g.kW; ++tx)
-                        if (iy0 + ty >= 0 && iy0 + ty < g.H && ix0 + tx >= 0 && ix0 + tx < g.W)
-                            tapmask |= 1ull << (ty * g.kW + tx);
-        } else {
-            pbase = pb * g.O * g.oH * g.oW;
+    for (int i = 1; i < PIXEL_CLASSES; ++i)
+        if (i < g.nclass && *tile >= g.c[i].tile0) *ci = i;
+    return *tile < g.ptiles;
+}
+
+// A lane's pixel: byte offset of its tap (0, 0) (against the moved base), and which taps lie inside the source: bit j: tap
+// column j, bit nx + i: tap row i.
+__device__ __forceinline__ void pixel_source(const PixelGemm& g, const PixelClass& c, int p, unsigned* voff, unsigned* mask)
+{
+    const int pp = p < c.P ? p : 0;
+    const int b = div_f32(pp, c.ghw), rem = pp - b * c.gHW;
+    const int py = div_f32(rem, c.gw), px = rem - py * c.gW;
+    *voff = 4u * (unsigned)(b * g.Ch * g.planeS + py * g.sy * g.Ws + px * g.sx);
+    unsigned m = 0;
+    const int ny = c.nT > 0 ? div_f32(c.nT, c.nxd) : 0;
+    for (int j = 0; j < c.nx; ++j) {
+        const int x = px * g.sx + c.x0 + j * g.d;
+        m |= (unsigned)(x >= 0 && x < g.Ws) << j;
+    }
+    for (int i = 0; i < ny; ++i) {
+        const int y = py * g.sy + c.y0 + i * g.d;
+        m |= (unsigned)(y >= 0 && y < g.Hs) << (c.nx + i);
+    }
+    *mask = p < c.P ? m : 0u;
+}
+
+// The products of a wave's 32 x 32 tile from one stage: [16 k][PT pixels] and behind it [QT][16 k], the even k of a row in
+// front of the odd ones, in XOR-swizzled 16-byte slots.  A matrix instruction takes k = 2 j (lanes 0 .. 31) and 2 j + 1; group
+// gi of the step is j = 4 gi .. 4 gi + 3.
+template <int PT>
+struct PixelTile {
+    v16f acc;
+    double folded[16];         // several ranges in a block: their sums, as the partial results of several blocks are added
+    v4f fa[2];
+    v2f fb[2][2];
+    unsigned xaddr, waddr0, waddr1;
+    __device__ __forceinline__ void init(unsigned lds0, int wq, int wp, int lane)
+    {
+        const int l32 = lane & 31, lh = lane >> 5;
+        xaddr = lds0 + 4u * (lh * PT + wp * 32 + l32);
+        const unsigned wrow = lds0 + 4u * GK * PT + 64u * (wq * 32 + l32);
+        waddr0 = wrow + 16u * ((2 * lh) ^ ((l32 >> 2) & 3));
+        waddr1 = wrow + 16u * ((2 * lh + 1) ^ ((l32 >> 2) & 3));
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { acc[r] = 0.0f; folded[r] = 0.0; }
+    }
+    __device__ __forceinline__ void fold()
+    {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { folded[r] += (double)acc[r]; acc[r] = 0.0f; }
+    }
+    __device__ __forceinline__ void unfold()
+    {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = (float)folded[r];
+    }
+    template <bool LIVE, int gi>
+    __device__ __forceinline__ void read_group(unsigned sb)
+    {
+        constexpr int U = PT / 64;
+        if (!LIVE) return;
+        const unsigned xa = xaddr + sb;
+        lds_read128f<0>(fa[gi], (gi ? waddr1 : waddr0) + sb);
+        lds_read2st64f<8 * gi * U, (8 * gi + 2) * U>(fb[gi][0], xa);
+        lds_read2st64f<(8 * gi + 4) * U, (8 * gi + 6) * U>(fb[gi][1], xa);
+    }
+    template <bool LIVE>
+    __device__ __forceinline__ void wait_group(int gi)
+    {
+        if (!LIVE) return;
+        wait_lgkm<0>();
+        tie(fa[gi]);
+        tie(fb[gi][0]);
+        tie(fb[gi][1]);
+    }
+    template <bool LIVE>
+    __device__ __forceinline__ void mfma_half(int gi, int half)
+    {
+        if (!LIVE) return;
+#pragma unroll
+        for (int j = 2 * half; j < 2 * half + 2; ++j)
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[gi][j], fb[gi][j >> 1][j & 1], acc, 0, 0, 0);
+    }
+    // One step, with the loads of a coming stage (load_part(0..4)) spread between the matrix instructions, which run on for
+    // 64 cycles each while the wave issues them.
+    template <bool LIVE, class L>
+    __device__ __forceinline__ void step(unsigned sb, L&& load_part)
+    {
+        read_group<LIVE, 0>(sb);
+        load_part(0);
+        wait_group<LIVE>(0);
+        read_group<LIVE, 1>(sb);
+        __builtin_amdgcn_sched_barrier(0);
+        mfma_half<LIVE>(0, 0);
+        load_part(1);
+        __builtin_amdgcn_sched_barrier(0);
+        mfma_half<LIVE>(0, 1);
+        load_part(2);
+        wait_group<LIVE>(1);
+        __builtin_amdgcn_sched_barrier(0);
+        mfma_half<LIVE>(1, 0);
+        load_part(3);
+        __builtin_amdgcn_sched_barrier(0);
+        mfma_half<LIVE>(1, 1);
+        load_part(4);
+    }
+    // Lane holds column p = .. + lane % 32 and rows q = .. + 8 * (r / 4) + 4 * (lane / 32) + r % 4.  `partial`: elements of
+    // one K range's result, 0: one range.
+    __device__ __forceinline__ void store(const PixelGemm& g, const PixelClass& c, int p0, int q0, int lane, const float* bias, float beta, float* out,
+                                          size_t partial)
+    {
+        float* dst = out + (size_t)blockIdx.z * partial;
+        const int p = p0 + (lane & 31);
+        if (p >= c.P) return;
+        const int img = div_f32(p, c.ghw), rem = p - img * c.gHW;
+        const int py = div_f32(rem, c.gw), px = rem - py * c.gW;
+        const size_t base = (size_t)img * g.Q * g.planeO + (py * g.osy + c.ry) * g.Wo + px * g.osx + c.rx;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int q = q0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+            if (q >= g.Q) continue;
+            const size_t idx = base + (size_t)q * g.planeO;
+            float v = acc[r];
+            if (partial == 0) {
+                if (beta != 0.0f) v += beta * dst[idx];
+                if (bias) v = bias[q] + v;
+            }
+            dst[idx] = v;
         }
     }
+};
 
-    float rp[8], rq[8];
-    auto fetch = [&](int k0) {
-        if (MODE == GEMM_BWD_FILTER) {
-            const int k = k0 + lk;
-            const bool kv = k < kend;
-            const int kk = kv ? k : 0;
-            const int plane = g.oH * g.oW;
-            const int b = kk / plane, rem = kk % plane, oy = rem / g.oW, ox = rem % g.oW;
-            const int iy0 = oy * g.sy - g.pt, ix0 = ox * g.sx - g.pl;
-            const int xbase = (b * g.C * g.H + iy0) * g.W + ix0;
-            const int ybase = b * g.O * plane + rem;
+// Weights laid out for the chunked kernel: [chunk of 16 channels][tap][q, padded][16], a row's channels in the order they have
+// in LDS; channels and rows that do not exist are zero.
+__global__ __launch_bounds__(256) void conv_f32_lay_weights_kernel(const float* __restrict__ w, float* __restrict__ wt, int total, int Q, int qpad, int Ch,
+                                                                   int T, int qs, int chs)
+{
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+        const int q = (i >> 2) % qpad, rest = (i >> 2) / qpad, tap = rest % T, chunk = rest / T;
+        const int slot = (i & 3) ^ ((q >> 2) & 3), ch = chunk * GK + 8 * (slot & 1) + (slot >> 1);
+        v4f v;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int iy = iy0 + pty[i], ix = ix0 + ptx[i];
-                const bool v = kv && poff[i] >= 0 && iy >= 0 && iy < g.H && ix >= 0 && ix < g.W;
-                rp[i] = ldP(xbase + poff[i], v);
-                if (i < NQL) {
-                    const int q = qtile + lp + 16 * i;
-                    rq[i] = ldQ(ybase + q * plane, kv && q < g.Q);
-                }
-            }
-        } else {
-            // P operand: k = k0 + lk + i -> (channel-like, ty, tx), advanced with carries
-            const int k = k0 + lk;
-            int ch = k / kHW, tap = k % kHW, ty = tap / g.kW, tx = tap % g.kW;
-            if (MODE == GEMM_FWD) {
-                int off = pbase + ch * g.H * g.W + ty * g.W + tx;       // walks (c,ty,tx) with carries
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const bool v = ((tapmask >> tap) & 1) && k + i < kend;
-                    rp[i] = ldP(off, v);
-                    ++off; ++tap;
-                    if (++tx == g.kW) {
-                        tx = 0; off += g.W - g.kW;
-                        if (tap == kHW) { tap = 0; off += (g.H - g.kH) * g.W; }
-                    }
-                }
-            } else {
-                const bool unit = g.sx == 1 && g.sy == 1;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const int ny = py + g.pt - ty, nx = px + g.pl - tx;
-                    int oy = ny, ox = nx;
-                    bool v = pvalid && k + i < kend && ny >= 0 && nx >= 0;
-                    if (!unit) {
-                        oy = ny / g.sy; ox = nx / g.sx;
-                        v = v && oy * g.sy == ny && ox * g.sx == nx;
-                    }
-                    v = v && oy < g.oH && ox < g.oW;
-                    rp[i] = ldP(pbase + (ch * g.oH + oy) * g.oW + ox, v);
-                    if (++tx == g.kW) { tx = 0; if (++ty == g.kH) { ty = 0; ++ch; } }
-                }
-            }
-            if (MODE == GEMM_FWD) {
-                const int q = qtile + lq_w;
-#pragma unroll
-                for (int i = 0; i < NQL; ++i) {
-                    const int kq = k0 + lk_w + i;
-                    rq[i] = ldQ(q * g.K + kq, q < g.Q && kq < kend);
-                }
-            } else {
-                const int q = qtile + lq_w;         // input channel c; w[(o*C + c)*kHW + tap], k = o*kHW + tap
-#pragma unroll
-                for (int i = 0; i < NQL; ++i) {
-                    const int kq = k0 + lk_w + i;
-                    rq[i] = ldQ(((kq / kHW) * g.C + q) * kHW + kq % kHW, q < g.Q && kq < kend);
-                }
-            }
-        }
-    };
-    auto stage = [&](int buf) {
-        float* Ps = Pbuf[buf];
-        float* Qs = Qbuf[buf];
-        if (MODE == GEMM_BWD_FILTER) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                Ps[lk * GLD + lp + 16 * i] = rp[i];
-                if (i < NQL) Qs[lk * GLD + lp + 16 * i] = rq[i];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                Ps[(lk + i) * GLD + lp] = rp[i];
-                if (i < NQL) Qs[(lk_w + i) * GLD + lq_w] = rq[i];
-            }
-        }
-    };
-
-    v16f acc[2][NP];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < NP; ++b)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.0f;
-
-    if (kbeg < kend) {
-        fetch(kbeg);
-        stage(0);
-        __syncthreads();
-        int buf = 0;
-        for (int k0 = kbeg; k0 < kend; k0 += GK, buf ^= 1) {
-            const bool more = k0 + GK < kend;
-            if (more)
-                fetch(k0 + GK);         // in flight while the matrix cores run
-            const float* Ps = Pbuf[buf];
-            const float* Qs = Qbuf[buf];
-            const int kr = lane >> 5, col = lane & 31;
-#pragma unroll
-            for (int kk = 0; kk < GK / 2; ++kk) {
-                const float* qrow = Qs + (kk * 2 + kr) * GLD + wq * 64 + col;
-                const float* prow = Ps + (kk * 2 + kr) * GLD + pw + col;
-                const float a0 = qrow[0], a1 = qrow[32];
-#pragma unroll
-                for (int pi = 0; pi < NP; ++pi) {
-                    const float b = prow[32 * pi];
-                    acc[0][pi] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b, acc[0][pi], 0, 0, 0);
-                    acc[1][pi] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b, acc[1][pi], 0, 0, 0);
-                }
-            }
-            if (more)
-                stage(buf ^ 1);         // the other tile: its readers passed the barrier of the previous step
-            __syncthreads();
-        }
-    }
-
-    // ---- epilogue: lane holds column p = .. + lane % 32 and rows q = .. + 8 * (r / 4) + 4 * (lane / 32) + r % 4
-#pragma unroll
-    for (int pi = 0; pi < NP; ++pi) {
-        const int p = ptile + pw + pi * 32 + (lane & 31);
-        if (p >= g.P) continue;
-        size_t base, qstride;
-        if (MODE == GEMM_FWD) {
-            const int plane = g.oH * g.oW;
-            base = (size_t)(p / plane) * g.O * plane + p % plane;
-            qstride = plane;
-        } else if (MODE == GEMM_BWD_DATA) {
-            const int plane = g.H * g.W;
-            base = (size_t)(p / plane) * g.C * plane + p % plane;
-            qstride = plane;
-        } else {
-            base = p;
-            qstride = g.P;
-        }
-        const bool partial = MODE == GEMM_BWD_FILTER || gridDim.z > 1;     // `out` is then the buffer of partial results
-        if (partial)
-            base += (size_t)blockIdx.z * g.Q * g.P;
-#pragma unroll
-        for (int qi = 0; qi < 2; ++qi) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int q = qtile + wq * 64 + qi * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (q >= g.Q) continue;
-                const size_t idx = base + (size_t)q * qstride;
-                float v = acc[qi][pi][r];
-                if (!partial) {
-                    if (beta != 0.0f) v += beta * out[idx];
-                    if (MODE == GEMM_FWD && bias) v = bias[q] + v;
-                }
-                out[idx] = v;
-            }
-        }
+        for (int j = 0; j < 4; ++j)
+            v[j] = (q < Q && ch + 2 * j < Ch) ? w[(size_t)q * qs + (size_t)(ch + 2 * j) * chs + tap] : 0.0f;
+        ((v4f*)wt)[i] = v;
     }
 }
 
-// out[i] = sum over the K ranges, in their order, + beta * out[i] (+ bias of element i's channel, NCHW with `plane`
-// pixels per channel and O channels)
-__global__ __launch_bounds__(256) void conv_f32_reduce_partials_kernel(const float* __restrict__ partial, int splits, size_t n, float beta,
+// Forward and backward-data with K in chunks of 16 channels at one tap.
+template <int WQ, int WP, int S>
+__global__ __launch_bounds__(256) void conv_f32_chunk_kernel(PixelGemm g, const float* __restrict__ srcX, const float* __restrict__ wt,
+                                                             const float* __restrict__ bias, float beta, float* __restrict__ out, size_t partial)
+{
+    static_assert(WQ * WP == 4, "four waves");
+    constexpr int QT = 32 * WQ, PT = 32 * WP;
+    constexpr int PH = PT / 64;                  // loads per k row
+    constexpr int WJ = QT >= 64 ? QT / 64 : 1;   // weight loads of a wave per step (1 KB each)
+    constexpr int LPI = 4 * PH + WJ;
+    constexpr int STAGE = GK * PT + QT * GK;     // floats
+    static_assert(LPI * (S - 1) < 60, "vmcnt is a 6-bit counter");
+    __shared__ __attribute__((aligned(16))) float smem[S * STAGE];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wq = wave / WP, wp = wave % WP;
+    int tile, qtile, ci;
+    if (!pixel_tile(g, &tile, &qtile, &ci))
+        return;
+    const PixelClass& c = g.c[ci];
+    const int p0 = (tile - c.tile0) * PT, q0 = qtile * QT;
+    const int nT = c.nT, nchunks = (g.Ch + GK - 1) / GK;
+    const __amdgpu_buffer_rsrc_t rsrcX = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(srcX) - c.bias, 0, g.bytesX + 4u * c.bias, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrcW = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(wt), 0, nchunks * g.T * g.qpad * GK * 4, 0x00020000);
+    unsigned voff[PH], mask[PH], mv[PH];
+#pragma unroll
+    for (int h = 0; h < PH; ++h)
+        pixel_source(g, c, p0 + h * 64 + lane, &voff[h], &mask[h]);
+    // Tap t of this class lives in lane t, looked up with v_readlane: its offset in the source, its validity bits, its place
+    // in the weights.
+    const int tl = min(lane, max(nT - 1, 0)), ti = div_f32(tl, c.nxd), tj = tl - ti * c.nx;
+    const int tap_off = 4 * (c.soff0 + ti * c.stepy + tj * c.stepx);
+    const int tap_bit = (1 << tj) | (1 << (c.nx + ti));
+    const int tap_w = ((c.ty0 + ti * g.osy) * g.kW + c.tx0 + tj * g.osx) * g.qpad * (GK * 4);
+    const int plane4 = g.planeS * 4;
+    PixelTile<PT> tl_acc;
+    tl_acc.init((unsigned)(unsigned long)(__attribute__((address_space(3))) float*)smem, wq, wp, lane);
+    for (int z = blockIdx.z * g.nz; z < (int)(blockIdx.z + 1) * g.nz; ++z) {
+        const int sbeg = z * g.kchunk, nsteps = max(0, min(g.kchunk, nchunks * nT - sbeg));
+        int chunk = nT > 0 ? div_f32(sbeg, c.nt) : 0, t = sbeg - chunk * nT;
+        int ch_off = (chunk * GK + wave * 4) * plane4, ch_left = g.Ch - chunk * GK - wave * 4;
+        int w_off = chunk * g.T * g.qpad * (GK * 4) + q0 * (GK * 4) + (QT >= 64 ? wave : wave & 1) * 1024;
+        const int w_chunk = g.T * g.qpad * (GK * 4);
+        unsigned xdst = 0;                           // LDS bytes of the stage to load next
+        int soff = 0, left = nsteps;
+        auto load_part = [&](int part) {
+            if (part == 0) {
+                const unsigned bit = (unsigned)__builtin_amdgcn_readlane(tap_bit, t) | (left > 0 ? 0u : 0x80000000u);    // (bit 31: never valid)
+                soff = ch_off + __builtin_amdgcn_readlane(tap_off, t);
+#pragma unroll
+                for (int h = 0; h < PH; ++h) mv[h] = (mask[h] & bit) == bit ? voff[h] : F32_OOB;
+            }
+            if (part < 4) {
+#pragma unroll
+                for (int h = 0; h < PH; ++h) {
+                    const lds_ptr_t dst = (lds_ptr_t)((char*)smem + xdst + ((wave * 4 + part) * PT + h * 64) * 4);
+                    if (ch_left >= 4) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcX, dst, 4, mv[h], soff + part * plane4, 0, 0);
+                    else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcX, dst, 4, part < ch_left ? mv[h] : F32_OOB, soff + part * plane4, 0, 0);
+                }
+            } else {
+                const int wo = w_off + __builtin_amdgcn_readlane(tap_w, t);
+#pragma unroll
+                for (int j = 0; j < WJ; ++j)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcW, (lds_ptr_t)((char*)smem + xdst + GK * PT * 4 + ((QT >= 64 ? wave : wave & 1) + 4 * j) * 1024), 16,
+                                                             lane * 16, wo + j * 4096, 0, 0);
+                xdst = xdst == 4u * STAGE * (S - 1) ? 0u : xdst + 4u * STAGE;
+                --left;
+                if (++t >= nT) {
+                    t = 0;
+                    ch_off += GK * plane4;
+                    ch_left -= GK;
+                    w_off += w_chunk;
+                }
+            }
+        };
+
+        if (nsteps > 0) {
+#pragma unroll
+            for (int st = 0; st < S - 1; ++st)       // (steps past the range load zeros: the number in flight stays the same)
+#pragma unroll
+                for (int part = 0; part < 5; ++part) load_part(part);
+            auto k_loop = [&](auto live) {
+                unsigned sb = 0;
+                for (int st = 0; st < nsteps; ++st) {
+                    wait_loads_and_barrier<LPI*(S - 2)>();
+                    tl_acc.template step<decltype(live)::value>(sb, load_part);
+                    sb = sb == 4u * STAGE * (S - 1) ? 0u : sb + 4u * STAGE;
+                }
+            };
+            if (q0 + wq * 32 < g.Q) k_loop(std::true_type{});
+            else k_loop(std::false_type{});          // (rows past the last: only the loads)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        if (g.nz > 1) {
+            tl_acc.fold();
+            __syncthreads();                     // (the next range's loads go where slower waves may still read)
+        }
+    }
+    if (g.nz > 1) tl_acc.unfold();
+    tl_acc.store(g, c, p0 + wp * 32, q0 + wq * 32, lane, bias, beta, out, partial);
+}
+
+// Weights laid out for the 3x3 kernel: [chunk of 4 channels][q, padded][40], the 36 (channel, tap) products of a row of q with
+// the even ones at 0 .. 17 and the odd ones at 20 .. 37.
+constexpr int K33 = 36, W33 = 40;
+__global__ __launch_bounds__(256) void conv_f32_lay_weights3x3_kernel(const float* __restrict__ w, float* __restrict__ wt, int total, int Q, int qpad, int Ch,
+                                                                      int qs, int chs)
+{
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+        const int e = i % W33, rest = i / W33, q = rest % qpad, chunk = rest / qpad;
+        const int half = e >= 20, k = 2 * (e - 20 * half) + half, ch = chunk * 4 + k / 9;
+        wt[i] = (e - 20 * half < 18 && q < Q && ch < Ch) ? w[(size_t)q * qs + (size_t)ch * chs + k % 9] : 0.0f;
+    }
+}
+
+// Forward of a 3x3 kernel, and backward-data at stride 1, with K in the tensors' own order, 4 channels (36 products) a step.
+// A lane's nine source offsets, or the one past the end where the tap lies outside, are worked out once for the tile; a load
+// then adds only its channel's scalar offset, and between the matrix instructions there is no vector arithmetic left.  A
+// wave loads one channel.  Two stages of 19 KB and 4 blocks to a CU: the other blocks cover a step's loads.  (K ranges need
+// not start or end with a step: what lies outside is loaded as zero.)
+template <int WQ, int WP>
+__global__ __launch_bounds__(256) void conv_f32_3x3_kernel(PixelGemm g, const float* __restrict__ srcX, const float* __restrict__ wt,
+                                                           const float* __restrict__ bias, float beta, float* __restrict__ out, size_t partial)
+{
+    static_assert(WQ * WP == 4, "four waves");
+    constexpr int QT = 32 * WQ, PT = 32 * WP, PH = PT / 64, U = PT / 64;
+    constexpr int STAGE = K33 * PT + QT * W33;   // floats
+    constexpr int WL = QT * W33 * 4 / 1024;      // weight loads of a block per step
+    __shared__ __attribute__((aligned(16))) float smem[2 * STAGE];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31, lh = lane >> 5, wq = wave / WP, wp = wave % WP;
+    int tile, qtile, ci;
+    if (!pixel_tile(g, &tile, &qtile, &ci))
+        return;
+    const PixelClass& c = g.c[0];                // (one class)
+    const int p0 = tile * PT, q0 = qtile * QT;
+    const __amdgpu_buffer_rsrc_t rsrcX = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(srcX) - c.bias, 0, g.bytesX + 4u * c.bias, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrcW = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(wt), 0, (g.Ch + 3) / 4 * g.qpad * W33 * 4, 0x00020000);
+    unsigned tap[PH][9];
+#pragma unroll
+    for (int h = 0; h < PH; ++h) {
+        unsigned voff, mask;
+        pixel_source(g, c, p0 + h * 64 + lane, &voff, &mask);
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+            const unsigned bit = (1u << t % 3) | (8u << t / 3);
+            tap[h][t] = (mask & bit) == bit ? voff + 4 * (c.soff0 + t / 3 * c.stepy + t % 3 * c.stepx) : F32_OOB;
+        }
+    }
+    const int plane4 = g.planeS * 4, wstep = g.qpad * W33 * 4;
+    PixelTile<PT> acc;
+    acc.init(0, wq, wp, lane);
+    const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) float*)smem;
+    const unsigned xaddr = lds0 + 4u * (lh * PT + wp * 32 + l32), waddr = lds0 + 4u * (K33 * PT + (wq * 32 + l32) * W33 + 20 * lh);
+    for (int z = blockIdx.z * g.nz; z < (int)(blockIdx.z + 1) * g.nz; ++z) {
+        const int kbeg = z * g.kchunk, kend = min(kbeg + g.kchunk, g.Ch * 9);
+        const int step0 = kbeg / K33, nsteps = kend > kbeg ? (kend + K33 - 1) / K33 - step0 : 0;
+        int ch_off = (step0 * 4 + wave) * plane4, k_row = step0 * K33 + wave * 9 - kbeg, w_off = step0 * wstep + q0 * W33 * 4;
+        const unsigned krange = kend - kbeg;
+        unsigned xdst = 0;                           // LDS bytes of the stage to load next
+        auto load_part = [&](int part) {             // 0 .. 4
+#pragma unroll
+            for (int t = 2 * part; t < 2 * part + 2 && t < 9; ++t) {
+                // (a product outside the range: past the end of the tensor, which is shorter than 2 GiB)
+                const int soff = (unsigned)(k_row + t) < krange ? ch_off : 0x7ffffffc;
+#pragma unroll
+                for (int h = 0; h < PH; ++h)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcX, (lds_ptr_t)((char*)smem + xdst + ((wave * 9 + t) * PT + h * 64) * 4), 4, tap[h][t], soff, 0, 0);
+            }
+            if (part < (WL + 3) / 4 && wave + 4 * part < WL)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcW, (lds_ptr_t)((char*)smem + xdst + K33 * PT * 4 + (wave + 4 * part) * 1024), 16, lane * 16,
+                                                         w_off + (wave + 4 * part) * 1024, 0, 0);
+            if (part == 4) {
+                ch_off += 4 * plane4;
+                k_row += K33;
+                w_off += wstep;
+                xdst = xdst ? 0u : 4u * STAGE;
+            }
+        };
+
+        auto k_loop = [&](auto livec) {
+            constexpr bool LIVE = decltype(livec)::value;
+            v4f fa[2];
+            v2f fb[2][2], ta, tb;
+            auto read_group = [&](auto gic, unsigned sb) {       // products 8 gi .. 8 gi + 7 (the last: 32 .. 35)
+                constexpr int gi = decltype(gic)::value;
+                if (!LIVE) return;
+                if (gi < 4) {
+                    lds_read128f<16 * gi>(fa[gi & 1], waddr + sb);
+                    lds_read2st64f<8 * gi * U, (8 * gi + 2) * U>(fb[gi & 1][0], xaddr + sb);
+                    lds_read2st64f<(8 * gi + 4) * U, (8 * gi + 6) * U>(fb[gi & 1][1], xaddr + sb);
+                } else {
+                    lds_read64f<64>(ta, waddr + sb);
+                    lds_read2st64f<32 * U, 34 * U>(tb, xaddr + sb);
+                }
+            };
+            auto wait_group = [&](int gi) {
+                if (!LIVE) return;
+                wait_lgkm<0>();
+                if (gi < 4) {
+                    tie(fa[gi & 1]);
+                    tie(fb[gi & 1][0]);
+                    tie(fb[gi & 1][1]);
+                } else {
+                    tie(ta);
+                    tie(tb);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            unsigned sb = 0;
+            for (int st = 0; st < nsteps; ++st) {
+                const bool more = st + 1 < nsteps;
+                wait_loads_and_barrier<0>();
+                read_group(std::integral_constant<int, 0>{}, sb);
+                auto group = [&](auto gic) {
+                    constexpr int gi = decltype(gic)::value;
+                    wait_group(gi);
+                    read_group(std::integral_constant<int, gi + 1>{}, sb);
+                    if (LIVE) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) acc.acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[gi & 1][j], fb[gi & 1][j >> 1][j & 1], acc.acc, 0, 0, 0);
+                    }
+                    if (more) load_part(gi);
+                };
+                group(std::integral_constant<int, 0>{});
+                group(std::integral_constant<int, 1>{});
+                group(std::integral_constant<int, 2>{});
+                group(std::integral_constant<int, 3>{});
+                wait_group(4);
+                if (LIVE) {
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) acc.acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ta[j], tb[j], acc.acc, 0, 0, 0);
+                }
+                if (more) load_part(4);
+                sb = sb ? 0u : 4u * STAGE;
+            }
+        };
+        if (nsteps > 0) {
+#pragma unroll
+            for (int part = 0; part < 5; ++part) load_part(part);
+            if (q0 + wq * 32 < g.Q) k_loop(std::true_type{});
+            else k_loop(std::false_type{});          // (rows past the last: only the loads)
+        }
+        if (g.nz > 1) {
+            acc.fold();
+            __syncthreads();                     // (the next range's loads go where slower waves may still read)
+        }
+    }
+    if (g.nz > 1) acc.unfold();
+    acc.store(g, c, p0 + wp * 32, q0 + wq * 32, lane, bias, beta, out, partial);
+}
+
+// A layer that spans its input, forward, in the reference's order of terms: y[b][o] = sum over k of x[b][k] w[o][k], one
+// after the other in float.  The chain of additions is what takes the time (a product and an addition behind another: 5.3 ns
+// a term on one wave, of which the addition's latency is 3.6), so everything else is kept off it: a block is one wave with 8
+// images x 8 outputs, its 16 rows of operands arrive in LDS two stages of 256 terms ahead, and in registers 32 terms ahead.
+// 16384 -> 10, 64 images: 2632 -> 116 us.
+constexpr int CHAIN_K = 256, CHAIN_ROW = CHAIN_K + 4, CHAIN_STAGES = 3;      // (rows 16 bytes apart in the banks)
+__global__ __launch_bounds__(64) void conv_f32_chain_kernel(int B, int O, int K, const float* __restrict__ x, const float* __restrict__ w,
+                                                            const float* __restrict__ bias, float beta, float* __restrict__ y)
+{
+    __shared__ __attribute__((aligned(16))) float smem[CHAIN_STAGES * 16 * CHAIN_ROW];
+    const int lane = threadIdx.x, bi = lane >> 3, oi = lane & 7, b0 = blockIdx.x * 8, o0 = blockIdx.y * 8;
+    const __amdgpu_buffer_rsrc_t rsrcX = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x + (size_t)b0 * K), 0, min(8, B - b0) * K * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrcW = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(w + (size_t)o0 * K), 0, min(8, O - o0) * K * 4, 0x00020000);
+    int soff = 0;
+    unsigned dst = 0;
+    auto load = [&]() {                          // (terms past a row: zeros, or of the next row; rows past the last: zeros; not used)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const lds_ptr_t d = (lds_ptr_t)((char*)smem + dst + r * CHAIN_ROW * 4);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcX, d, 16, lane * 16, soff + r * K * 4, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcW, (lds_ptr_t)((char*)smem + dst + (r + 8) * CHAIN_ROW * 4), 16, lane * 16, soff + r * K * 4, 0, 0);
+        }
+        soff += CHAIN_K * 4;
+        dst = dst == (CHAIN_STAGES - 1) * 16u * CHAIN_ROW * 4u ? 0u : dst + 16u * CHAIN_ROW * 4u;
+    };
+    const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) float*)smem;
+    const unsigned xrow = lds0 + 4u * bi * CHAIN_ROW, wrow = lds0 + 4u * (8 + oi) * CHAIN_ROW;
+    const int full = K / 32, rest = K % 32, groups = full + (rest > 0);
+    v4f xv[2][8], wv[2][8];
+    unsigned src = 0;
+    auto read = [&](int buf, int h) {            // the operands of the h-th 32 terms
+        const unsigned off = src + 128u * (h & 7);
+        const unsigned xa = xrow + off, wa = wrow + off;
+        lds_read128f<0>(xv[buf][0], xa); lds_read128f<0>(wv[buf][0], wa);
+        lds_read128f<16>(xv[buf][1], xa); lds_read128f<16>(wv[buf][1], wa);
+        lds_read128f<32>(xv[buf][2], xa); lds_read128f<32>(wv[buf][2], wa);
+        lds_read128f<48>(xv[buf][3], xa); lds_read128f<48>(wv[buf][3], wa);
+        lds_read128f<64>(xv[buf][4], xa); lds_read128f<64>(wv[buf][4], wa);
+        lds_read128f<80>(xv[buf][5], xa); lds_read128f<80>(wv[buf][5], wa);
+        lds_read128f<96>(xv[buf][6], xa); lds_read128f<96>(wv[buf][6], wa);
+        lds_read128f<112>(xv[buf][7], xa); lds_read128f<112>(wv[buf][7], wa);
+    };
+    float sum = 0.0f;
+    auto group = [&](auto bufc, int h) {
+        constexpr int buf = decltype(bufc)::value;
+        wait_lgkm<0>();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) { tie(xv[buf][i]); tie(wv[buf][i]); }
+        if ((h & 7) == 7) {                      // the stage has been read: its place is free, and the next one is there
+            wait_loads_and_barrier<16 * (CHAIN_STAGES - 2)>();
+            load();
+            src = src == (CHAIN_STAGES - 1) * 16u * CHAIN_ROW * 4u ? 0u : src + 16u * CHAIN_ROW * 4u;
+        }
+        if (h + 1 < groups) read(1 - buf, h + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (h < full) {
+            float p[32];
+#pragma unroll
+            for (int i = 0; i < 32; ++i) p[i] = wv[buf][i >> 2][i & 3] * xv[buf][i >> 2][i & 3];
+#pragma unroll
+            for (int i = 0; i < 32; ++i) sum = sum + p[i];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 31; ++i) {
+                const float t = sum + wv[buf][i >> 2][i & 3] * xv[buf][i >> 2][i & 3];
+                sum = i < rest ? t : sum;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int st = 0; st < CHAIN_STAGES; ++st) load();
+    wait_loads_and_barrier<16 * (CHAIN_STAGES - 1)>();
+    read(0, 0);
+    for (int h = 0; h < groups; h += 2) {
+        group(std::integral_constant<int, 0>{}, h);
+        if (h + 1 < groups) group(std::integral_constant<int, 1>{}, h + 1);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const int b = b0 + bi, o = o0 + oi;
+    if (b >= B || o >= O) return;
+    const size_t idx = (size_t)b * O + o;
+    float r = sum + (beta != 0.0f ? beta * y[idx] : 0.0f);
+    if (bias) r = bias[o] + r;
+    y[idx] = r;
+}
+
+// Forward (BWD = false) and backward-data with K in the tensors' own order, (channel, tap).
+template <bool BWD, int WQ, int WP, int S>
+__global__ __launch_bounds__(256) void conv_f32_pixel_kernel(PixelGemm g, const float* __restrict__ srcX, const float* __restrict__ srcW,
+                                                             const float* __restrict__ bias, float beta, float* __restrict__ out, size_t partial)
+{
+    static_assert(WQ * WP == 4, "four waves");
+    constexpr int QT = 32 * WQ, PT = 32 * WP;
+    constexpr int PH = PT / 64;                  // loads per k row
+    constexpr int WJ = QT / 16;                  // weight loads of a wave per step
+    constexpr int LPI = 4 * PH + WJ;             // loads of a wave per step
+    constexpr int STAGE = GK * PT + QT * GK;     // floats
+    static_assert(LPI * (S - 1) < 60, "vmcnt is a 6-bit counter");
+    __shared__ __attribute__((aligned(16))) float smem[S * STAGE];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wq = wave / WP, wp = wave % WP;
+    int tile, qtile, ci;
+    if (!pixel_tile(g, &tile, &qtile, &ci))
+        return;
+    const PixelClass& c = g.c[ci];
+    const int p0 = (tile - c.tile0) * PT, q0 = qtile * QT;
+    const int nT = c.nT, K = g.Ch * nT;
+    const __amdgpu_buffer_rsrc_t rsrcX = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(srcX) - c.bias, 0, g.bytesX + 4u * c.bias, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrcW = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(srcW), 0, g.bytesW, 0x00020000);
+    unsigned voff[PH], mask[PH], wbase[WJ];
+#pragma unroll
+    for (int h = 0; h < PH; ++h)
+        pixel_source(g, c, p0 + h * 64 + lane, &voff[h], &mask[h]);
+    const int slot = ((lane & 15) >> 2) ^ wave, kk = 8 * (slot & 1) + 2 * (lane & 3) + (slot >> 1);    // this lane's k of a step in the weights
+#pragma unroll
+    for (int j = 0; j < WJ; ++j) {
+        const int q = q0 + 4 * (wave + 4 * j) + (lane >> 4);
+        wbase[j] = q < g.Q ? 4u * (unsigned)(q * g.qs) : F32_OOB;
+    }
+    // Tap t of this class lives in lane t; the running (channel, tap) of each of the wave's rows is scalar.
+    const int tl = min(lane, max(nT - 1, 0)), ti = div_f32(tl, c.nxd), tj = tl - ti * c.nx;
+    const int tap_off = 4 * (c.soff0 + ti * c.stepy + tj * c.stepx);
+    const int tap_bit = (1 << tj) | (1 << (c.nx + ti));
+    PixelTile<PT> tl_acc;
+    tl_acc.init((unsigned)(unsigned long)(__attribute__((address_space(3))) float*)smem, wq, wp, lane);
+    for (int z = blockIdx.z * g.nz; z < (int)(blockIdx.z + 1) * g.nz; ++z) {
+        const int kbeg = z * g.kchunk, kend = min(kbeg + g.kchunk, K);
+        const int nsteps = kend > kbeg ? (kend - kbeg + GK - 1) / GK : 0;
+        int row_t[4], row_ch[4];                     // row_ch: byte offset of the row's channel
+        const int plane4 = g.planeS * 4, adv = nT > 0 ? div_f32(GK, c.nt) : 0, adv_t = nT > 0 ? GK - adv * nT : 0, adv_ch = adv * plane4;
+        {
+            int ch = nT > 0 ? div_f32(kbeg + wave * 4, c.nt) : 0, t = nT > 0 ? kbeg + wave * 4 - ch * nT : 0;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                row_t[r] = t; row_ch[r] = ch * plane4;
+                if (++t >= nT) { t = 0; ++ch; }
+            }
+        }
+        int row_left = kend - kbeg - wave * 4, wk = kbeg + kk;
+        unsigned xdst = 0;                           // LDS bytes of the stage to load next
+        auto load_part = [&](int part) {
+            if (part < 4) {
+                const int t = row_t[part];
+                const int soff = row_ch[part] + __builtin_amdgcn_readlane(tap_off, t);
+                // (bit 31: never valid)
+                const unsigned bit = (unsigned)__builtin_amdgcn_readlane(tap_bit, t) | ((unsigned)(row_left - 1 - part) & 0x80000000u);
+#pragma unroll
+                for (int h = 0; h < PH; ++h)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcX, (lds_ptr_t)((char*)smem + xdst + ((wave * 4 + part) * PT + h * 64) * 4), 4,
+                                                             (mask[h] & bit) == bit ? voff[h] : F32_OOB, soff, 0, 0);
+                const int tn = t + adv_t;
+                const bool carry = tn >= nT;
+                row_t[part] = carry ? tn - nT : tn;
+                row_ch[part] += adv_ch + (carry ? plane4 : 0);
+            } else {
+                unsigned off = 4u * wk;
+                if (BWD) {
+                    const int ch = div_f32(wk, c.nt), t = wk - ch * nT;
+                    const int i = div_f32(t, c.nxd), j = t - i * c.nx;
+                    off = 4u * (ch * g.chs + (c.ty0 + i * g.osy) * g.kW + c.tx0 + j * g.osx);
+                }
+                const bool v = wk < kend;
+#pragma unroll
+                for (int j = 0; j < WJ; ++j)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcW, (lds_ptr_t)((char*)smem + xdst + (GK * PT + (wave + 4 * j) * 64) * 4), 4,
+                                                             v ? wbase[j] + off : F32_OOB, 0, 0, 0);
+                wk += GK;
+                row_left -= GK;
+                xdst = xdst == 4u * STAGE * (S - 1) ? 0u : xdst + 4u * STAGE;
+            }
+        };
+
+        if (nsteps > 0) {
+#pragma unroll
+            for (int st = 0; st < S - 1; ++st)       // (steps past the range load zeros: the number in flight stays the same)
+#pragma unroll
+                for (int part = 0; part < 5; ++part) load_part(part);
+            auto k_loop = [&](auto live) {
+                unsigned sb = 0;
+                for (int st = 0; st < nsteps; ++st) {
+                    wait_loads_and_barrier<LPI*(S - 2)>();
+                    tl_acc.template step<decltype(live)::value>(sb, load_part);
+                    sb = sb == 4u * STAGE * (S - 1) ? 0u : sb + 4u * STAGE;
+                }
+            };
+            if (q0 + wq * 32 < g.Q) k_loop(std::true_type{});
+            else k_loop(std::false_type{});          // (rows past the last: only the loads)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        if (g.nz > 1) {
+            tl_acc.fold();
+            __syncthreads();                     // (the next range's loads go where slower waves may still read)
+        }
+    }
+    if (g.nz > 1) tl_acc.unfold();
+    tl_acc.store(g, c, p0 + wp * 32, q0 + wq * 32, lane, BWD ? nullptr : bias, beta, out, partial);
+}
+
+// Backward-filter: both operands hold consecutive k (pixels), rows of 32 of them in LDS, two rows to a load.  Row pairs are
+// 272 bytes apart, so that 8 rows' 16-byte reads fall into different banks.
+template <int WQ, int WP, int S>
+__global__ __launch_bounds__(256) void conv_f32_filter_kernel(FilterGemm g, const float* __restrict__ srcX, const float* __restrict__ srcY,
+                                                              float* __restrict__ out)
+{
+    static_assert(WQ * WP == 4, "four waves");
+    constexpr int QT = 32 * WQ, PT = 32 * WP;
+    constexpr int PJ = PT / 8, QJ = QT / 8;      // loads of a wave per step (two rows each)
+    constexpr int PAIR = 68;                     // floats from one row pair to the next
+    constexpr int STAGE = (PT + QT) / 2 * PAIR;
+    static_assert((PJ + QJ) * (S - 1) < 60, "vmcnt is a 6-bit counter");
+    __shared__ __attribute__((aligned(16))) float smem[S * STAGE];
+    const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) float*)smem;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31, lh = lane >> 5;
+    const int wq = wave / WP, wp = wave % WP;
+    const int p0 = blockIdx.x * PT, q0 = blockIdx.y * QT;
+    const int kbeg = blockIdx.z * g.kchunk, kend = min(kbeg + g.kchunk, g.K);
+    const int nsteps = kend > kbeg ? (kend - kbeg + FK - 1) / FK : 0;
+    const int xbias = g.pt * g.W + g.pl;
+    const __amdgpu_buffer_rsrc_t rsrcX = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(srcX) - xbias, 0, g.bytesX + 4u * xbias, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrcY = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(srcY), 0, g.bytesY, 0x00020000);
+
+    // ---- loader state: this lane's half of the row pairs its wave loads
+    unsigned poff[PJ], pbit[PJ], qoff[QJ];
+    const int kHW = g.kH * g.kW;
+#pragma unroll
+    for (int j = 0; j < PJ; ++j) {
+        const int p = p0 + 2 * (wave + 4 * j) + lh, pp = min(p, g.P - 1);
+        const int ch = pp / kHW, t = pp - ch * kHW, ty = t / g.kW, tx = t - ty * g.kW;
+        poff[j] = 4u * (unsigned)(ch * g.H * g.W + ty * g.W + tx);
+        pbit[j] = p < g.P ? (1u << tx) | (1u << (g.kW + ty)) : 0x80000000u;
+    }
+#pragma unroll
+    for (int j = 0; j < QJ; ++j) {
+        const int q = q0 + 2 * (wave + 4 * j) + lh;
+        qoff[j] = q < g.Q ? 4u * (unsigned)(q * g.plane) : F32_OOB;
+    }
+    unsigned xo = 0, yo = 0, pmask = 0, dst_bytes = 0;
+    bool kv = false;
+    int k_next = kbeg + l32;
+    auto locate = [&]() {                        // this lane's pixel of the step to load next
+        kv = k_next < kend;
+        const int k = kv ? k_next : 0;
+        const int img = div_f32(k, g.dplane), rem = k - img * g.plane;
+        const int oy = div_f32(rem, g.dow), ox = rem - oy * g.oW;
+        const int iy0 = oy * g.s_y - g.pt, ix0 = ox * g.s_x - g.pl;
+        xo = 4u * (unsigned)(img * g.imgX + oy * g.s_y * g.W + ox * g.s_x);
+        yo = 4u * (unsigned)(img * g.imgY + rem);
+        // bits lo .. hi - 1 of the columns, then of the rows, that lie inside the input
+        const int xl = min(max(-ix0, 0), g.kW), xh = min(max(g.W - ix0, 0), g.kW), yl = min(max(-iy0, 0), g.kH), yh = min(max(g.H - iy0, 0), g.kH);
+        const unsigned mx = ((1u << xh) - 1u) & ~((1u << xl) - 1u), my = ((1u << yh) - 1u) & ~((1u << yl) - 1u);
+        pmask = kv ? mx | (my << g.kW) : 0u;
+        k_next += FK;
+    };
+    auto issue_part = [&](int part) {            // a quarter of a stage's loads
+#pragma unroll
+        for (int j = part * PJ / 4; j < (part + 1) * PJ / 4; ++j)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcX, (lds_ptr_t)((char*)smem + dst_bytes + (wave + 4 * j) * PAIR * 4), 4,
+                                                     (pmask & pbit[j]) == pbit[j] ? xo + poff[j] : F32_OOB, 0, 0, 0);
+#pragma unroll
+        for (int j = part * QJ / 4; j < (part + 1) * QJ / 4; ++j)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcY, (lds_ptr_t)((char*)smem + dst_bytes + (PT / 2 + wave + 4 * j) * PAIR * 4), 4,
+                                                     kv ? yo + qoff[j] : F32_OOB, 0, 0, 0);
+        if (part == 3)
+            dst_bytes = dst_bytes == 4u * STAGE * (S - 1) ? 0u : dst_bytes + 4u * STAGE;
+    };
+
+    v16f acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+
+    // ---- fragments: group gi of a step: k = 4 (2 gi + lh) + 0..3
+    const unsigned lrow = 4u * ((l32 >> 1) * PAIR + (l32 & 1) * 32) + 16u * lh;
+    const unsigned paddr = lds0 + 4u * (wp * 16 * PAIR) + lrow, qaddr = lds0 + 4u * (PT / 2 * PAIR + wq * 16 * PAIR) + lrow;
+    auto k_loop = [&](auto livec) {
+        constexpr bool LIVE = decltype(livec)::value;
+        v4f fa[2], fb[2];
+        auto read_group = [&](auto gic, unsigned sb) {
+            constexpr int gi = decltype(gic)::value;
+            if (!LIVE) return;
+            lds_read128f<32 * gi>(fa[gi & 1], qaddr + sb);
+            lds_read128f<32 * gi>(fb[gi & 1], paddr + sb);
+        };
+        auto wait_group = [&](int gi) {
+            if (!LIVE) return;
+            wait_lgkm<0>();
+            tie(fa[gi & 1]);
+            tie(fb[gi & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto mfma_group = [&](int gi) {
+            if (!LIVE) return;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[gi & 1][j], fb[gi & 1][j], acc, 0, 0, 0);
+        };
+        unsigned sb = 0;
+        for (int st = 0; st < nsteps; ++st) {
+            wait_loads_and_barrier<(PJ + QJ) * (S - 2)>();
+            read_group(std::integral_constant<int, 0>{}, sb);
+            locate();
+            issue_part(0);
+            wait_group(0);
+            read_group(std::integral_constant<int, 1>{}, sb);
+            mfma_group(0);
+            issue_part(1);
+            wait_group(1);
+            read_group(std::integral_constant<int, 2>{}, sb);
+            mfma_group(1);
+            issue_part(2);
+            wait_group(2);
+            read_group(std::integral_constant<int, 3>{}, sb);
+            mfma_group(2);
+            issue_part(3);
+            wait_group(3);
+            mfma_group(3);
+            sb = sb == 4u * STAGE * (S - 1) ? 0u : sb + 4u * STAGE;
+        }
+    };
+    if (nsteps > 0) {
+#pragma unroll
+        for (int st = 0; st < S - 1; ++st) {
+            locate();
+#pragma unroll
+            for (int part = 0; part < 4; ++part) issue_part(part);
+        }
+        if (p0 + wp * 32 < g.P && q0 + wq * 32 < g.Q) k_loop(std::true_type{});
+        else k_loop(std::false_type{});          // (past the last column or row: only the loads)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+
+    float* dst = out + (size_t)blockIdx.z * g.Q * g.P;
+    const int p = p0 + wp * 32 + l32;
+    if (p >= g.P) return;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int q = q0 + wq * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
+        if (q < g.Q) dst[(size_t)q * g.P + p] = acc[r];
+    }
+}
+
+// Backward-filter of small problems, in double on the fp64 matrix cores (16 x 16 x 4): a block is a 16 x 16 tile of dw and a
+// range of pixels, dealt to its four waves 16 at a time; a lane takes four consecutive pixels of its row of q and of its
+// column of p, one per matrix instruction.  Nothing here is near a rate: the time is that of the loads' latency and of two
+// launches, so the range is as short as fills the chip, and the next 16 pixels are on their way while these are multiplied.
+// Against one block per weight summing all pixels (32 images, 1 x 32 x 32 -> 6, 5x5): 46 -> 12 us; 16 -> 32 channels, 3x3 on
+// 16 x 16: 50 -> 12 us.
+typedef double v4d __attribute__((ext_vector_type(4)));
+__global__ __launch_bounds__(256) void conv_f32_filter_small_kernel(FilterGemm g, const float* __restrict__ srcX, const float* __restrict__ srcY,
+                                                                    double* __restrict__ partial, float beta, float* __restrict__ out)
+{
+    __shared__ double red[4][256];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane & 15, kg = lane >> 4;
+    const int p = blockIdx.x * 16 + row, q = blockIdx.y * 16 + row;
+    const int kbeg = blockIdx.z * g.kchunk, kend = min(kbeg + g.kchunk, g.K);
+    const int kHW = g.kH * g.kW, pp = min(p, g.P - 1);
+    const int ch = pp / kHW, t = pp - ch * kHW, ty = t / g.kW, tx = t - ty * g.kW;
+    const float* xb = srcX + (size_t)ch * g.H * g.W;
+    const float* yb = srcY + (size_t)min(q, g.Q - 1) * g.plane;
+    float a[2][4], b[2][4];
+    auto load = [&](int k0, float (&av)[4], float (&bv)[4]) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int k = k0 + j;
+            const bool kv = k < kend;
+            const int kk = kv ? k : 0;
+            const int img = div_f32(kk, g.dplane), rem = kk - img * g.plane;
+            const int oy = div_f32(rem, g.dow), ox = rem - oy * g.oW;
+            const int iy = oy * g.s_y - g.pt + ty, ix = ox * g.s_x - g.pl + tx;
+            const bool v = kv && iy >= 0 && iy < g.H && ix >= 0 && ix < g.W;
+            av[j] = kv ? yb[(size_t)img * g.imgY + rem] : 0.0f;
+            bv[j] = v ? xb[(size_t)img * g.imgX + iy * g.W + ix] : 0.0f;
+        }
+    };
+    v4d acc = {0.0, 0.0, 0.0, 0.0};
+    int k0 = kbeg + wave * 16 + kg * 4;
+    load(k0, a[0], b[0]);
+    for (int s = kbeg + wave * 16; s < kend; s += 128) {
+        load(k0 + 64, a[1], b[1]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[0][j], (double)b[0][j], acc, 0, 0, 0);
+        k0 += 128;
+        load(k0, a[0], b[0]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[1][j], (double)b[1][j], acc, 0, 0, 0);
+    }
+    // lane holds column p = lane % 16 and rows q = 4 r + lane / 16
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wave][(4 * r + kg) * 16 + row] = acc[r];
+    __syncthreads();
+    const int oq = blockIdx.y * 16 + threadIdx.x / 16, op = blockIdx.x * 16 + threadIdx.x % 16;
+    if (oq >= g.Q || op >= g.P) return;
+    const double v = ((red[0][threadIdx.x] + red[1][threadIdx.x]) + red[2][threadIdx.x]) + red[3][threadIdx.x];
+    const size_t idx = (size_t)oq * g.P + op;
+    if (gridDim.z > 1) partial[(size_t)blockIdx.z * g.Q * g.P + idx] = v;
+    else out[idx] = (float)v + (beta != 0.0f ? beta * out[idx] : 0.0f);
+}
+
+// out[i] = sum over the K ranges + beta * out[i] (+ bias of element i's channel, NCHW with `plane` pixels per channel and O
+// channels).  A block adds 64 elements: each of its four waves a quarter of the ranges in double, in their order, then the
+// four in order, so the result does not depend on timing.
+template <class T>
+__global__ __launch_bounds__(256) void conv_f32_reduce_partials_kernel(const T* __restrict__ partial, int splits, size_t n, float beta,
                                                                        float* __restrict__ out, const float* __restrict__ bias, int plane, int O)
 {
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+    __shared__ double red[4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int z0 = splits * w / 4, z1 = splits * (w + 1) / 4;
+    for (size_t i0 = (size_t)blockIdx.x * 64; i0 < n; i0 += (size_t)gridDim.x * 64) {
+        const size_t i = i0 + lane;
         double s = 0.0;
-        for (int z = 0; z < splits; ++z) s += (double)partial[(size_t)z * n + i];
-        float v = (float)s + (beta != 0.0f ? beta * out[i] : 0.0f);
-        if (bias) v = bias[(i / plane) % O] + v;
-        out[i] = v;
+        if (i < n) {
+            int z = z0;
+            for (; z + 8 <= z1; z += 8) {
+                T v[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v[j] = partial[(size_t)(z + j) * n + i];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) s += (double)v[j];
+            }
+            for (; z < z1; ++z) s += (double)partial[(size_t)z * n + i];
+        }
+        __syncthreads();
+        red[w][lane] = s;
+        __syncthreads();
+        if (w == 0 && i < n) {
+            const double t = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
+            float v = (float)t + (beta != 0.0f ? beta * out[i] : 0.0f);
+            if (bias) v = bias[(i / plane) % O] + v;
+            out[i] = v;
+        }
     }
 }
 

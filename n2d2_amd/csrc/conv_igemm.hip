@@ -430,29 +430,6 @@ void launch_pipe_res(ConvPipeArgs a, int grid, hipStream_t stream)
         N2D2HIP_LAUNCH_T(conv_pipe_kernel, (NW, BK, NI, NJ, WGM, EPI_I24, S, 1, true, false), dim3(grid), dim3(NW * 64), 0, stream, a);
 }
 
-// (multiplier, shift) with n / d == umulhi(n, multiplier) >> shift for 0 <= n < 2^31; multiplier 0 stands for d == 1
-void magic_div(unsigned d, unsigned* mul, unsigned* sh)
-{
-    if (d <= 1) { *mul = 0; *sh = 0; return; }
-    unsigned s = 0;
-    while ((1ull << s) < d) ++s;
-    *mul = (unsigned)((1ull << (31 + s)) / d + 1);
-    *sh = s - 1;
-}
-
-int num_cus()
-{
-    static int n = 0;
-    if (n == 0) {
-        hipDeviceProp_t prop;
-        int dev = 0;
-        if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
-            n = prop.multiProcessorCount;
-        if (n <= 0) n = 256;
-    }
-    return n;
-}
-
 int sext4(int n) { return (n & 8) ? (n | ~15) : (n & 15); }
 
 // Reads weight element `idx` of the caller's OCHW array (int8 or nibble-packed).

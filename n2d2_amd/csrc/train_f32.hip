@@ -2,10 +2,12 @@
 // the loss at the output and the SGD update.  Tensors are N2D2's own NCHW / OCHW float tensors (X fastest), so a
 // training graph exchanges them without conversion.
 //
-// These are direct kernels: one thread per produced element, walking channels and taps in the reference's order
-// (so forward and backward-data give the reference's float sums term for term), and one block per weight for
-// backward-filter, whose long sum over batch and pixels is wavefront-reduced in double.
-#include <cstdlib>
+// Convolutions run on the matrix cores (conv_f32_gemm.hpp) wherever they are neither grouped nor dilated.  The kernels here
+// are direct: one thread per produced element, walking channels and taps in the reference's order (so forward and
+// backward-data give the reference's float sums term for term), and one block per weight for backward-filter, whose long
+// sum over batch and pixels is wavefront-reduced in double.
+#include <algorithm>
+#include <vector>
 
 #include "common.h"
 #include "conv_f32_gemm.hpp"
@@ -111,6 +113,108 @@ __global__ __launch_bounds__(TBLOCK) void conv_f32_backward_data_kernel(ConvF32 
         }
         dx[idx] = g + (beta != 0.0f ? beta * dx[idx] : 0.0f);
     }
+}
+
+// The same two sums, term for term, with the loads of the next products requested together: the chain of additions is short
+// (4 cycles a term), waiting for each term's operands is what takes the time (0.14 us a term, one after the other).  A thread
+// is an element of the result; the walk over (channel, tap) is the same for all and scalar, a thread only adds its own base
+// and looks the tap up in its mask (bit j: column j inside, bit nj + i: row i inside).
+struct WalkF32 {
+    int n, ni, nj;                               // channels, tap rows, tap columns
+    int xo, xi, xj, wo, wi, wj;                  // offsets per channel, row, column in the source and in the weights
+    DivF32 dplane, dw, dch;                      // result: plane, row length, channels
+};
+
+constexpr int WALK = 16;                         // products in flight
+__device__ __forceinline__ float walk_f32(const WalkF32& k, const float* __restrict__ x, const float* __restrict__ w, int xb, int wb, unsigned mask)
+{
+    float sum = 0.0f;
+    const int total = k.n * k.ni * k.nj;
+    int xc = 0, wc = 0, i = 0, j = 0;            // the next product's channel offsets, row, column
+    for (int k0 = 0; k0 < total; k0 += WALK) {
+        float xv[WALK], wv[WALK];
+        unsigned ok = 0;
+#pragma unroll
+        for (int u = 0; u < WALK; ++u) {
+            const unsigned bit = (1u << j) | (1u << (k.nj + i)) | (k0 + u < total ? 0u : 0x80000000u);       // (bit 31: never set)
+            const bool v = (mask & bit) == bit;
+            ok |= v ? 1u << u : 0u;
+            xv[u] = x[v ? xb + xc + i * k.xi + j * k.xj : 0];
+            wv[u] = w[v ? wb + wc + i * k.wi + j * k.wj : 0];
+            if (++j == k.nj) {
+                j = 0;
+                if (++i == k.ni) { i = 0; xc += k.xo; wc += k.wo; }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < WALK; ++u) sum = ok & (1u << u) ? sum + wv[u] * xv[u] : sum;
+    }
+    return sum;
+}
+// Forward of a 3x3 kernel, CB channels at a time: a full window is summed row by row, then the rows.
+template <int CB>
+__device__ __forceinline__ float walk3x3_f32(const WalkF32& k, const float* __restrict__ x, const float* __restrict__ w, int xb, int wb, unsigned mask)
+{
+    float sum = 0.0f;
+    for (int c0 = 0; c0 < k.n; c0 += CB) {
+        float xv[CB][9], wv[CB][9];
+#pragma unroll
+        for (int c = 0; c < CB; ++c)
+#pragma unroll
+            for (int t = 0; t < 9; ++t) {
+                const unsigned bit = (1u << t % 3) | (8u << t / 3) | (c0 + c < k.n ? 0u : 0x80000000u);
+                const bool v = (mask & bit) == bit;
+                xv[c][t] = x[v ? xb + (c0 + c) * k.xo + t / 3 * k.xi + t % 3 * k.xj : 0];
+                wv[c][t] = w[v ? wb + (c0 + c) * k.wo + t / 3 * k.wi + t % 3 * k.wj : 0];
+            }
+#pragma unroll
+        for (int c = 0; c < CB; ++c) {
+            if (c0 + c >= k.n) break;
+            const float* a = wv[c];
+            const float* b = xv[c];
+            const float full = sum + (a[0] * b[0] + a[1] * b[1] + a[2] * b[2]) + (a[3] * b[3] + a[4] * b[4] + a[5] * b[5])
+                                   + (a[6] * b[6] + a[7] * b[7] + a[8] * b[8]);
+#pragma unroll
+            for (int t = 0; t < 9; ++t) {
+                const unsigned bit = (1u << t % 3) | (8u << t / 3);
+                sum = (mask & bit) == bit ? sum + a[t] * b[t] : sum;
+            }
+            sum = (mask & 63u) == 63u ? full : sum;
+        }
+    }
+    return sum;
+}
+
+// SHAPE: 0 any kernel, 1 / 4: forward of a 3x3 kernel, channels at a time.
+template <bool BWD, int SHAPE>
+__global__ __launch_bounds__(64) void conv_f32_walk_kernel(ConvF32 q, WalkF32 k, const float* __restrict__ x, const float* __restrict__ w,
+                                                           const float* __restrict__ bias, float beta, float* __restrict__ out, int total)
+{
+    const int idx = blockIdx.x * 64 + threadIdx.x;
+    if (idx >= total) return;
+    const int img = div_f32(idx, k.dplane);      // image and channel
+    const int b = div_f32(img, k.dch), ch = img - b * (BWD ? q.C : q.O);
+    const int rem = idx - img * (BWD ? q.H * q.W : q.oH * q.oW), py = div_f32(rem, k.dw), px = rem - py * (BWD ? q.W : q.oW);
+    const int T = q.kH * q.kW;
+    unsigned mask = 0;
+    int xb, wb;
+    if (BWD) {                                   // tap (ty0 + i sy, tx0 + j sx) reaches this element from output (oy0 - i, ox0 - j)
+        const int iyPad = py + q.pt, ixPad = px + q.pl, oy0 = iyPad / q.sy, ox0 = ixPad / q.sx, ty0 = iyPad - oy0 * q.sy, tx0 = ixPad - ox0 * q.sx;
+        for (int j = 0; j < k.nj; ++j) mask |= (unsigned)(tx0 + j * q.sx < q.kW && ox0 - j >= 0 && ox0 - j < q.oW) << j;
+        for (int i = 0; i < k.ni; ++i) mask |= (unsigned)(ty0 + i * q.sy < q.kH && oy0 - i >= 0 && oy0 - i < q.oH) << (k.nj + i);
+        xb = (b * q.O + (q.depthwise ? ch : 0)) * (q.oH * q.oW) + oy0 * q.oW + ox0;
+        wb = ch * T + ty0 * q.kW + tx0;
+    } else {
+        const int iy0 = py * q.sy - q.pt, ix0 = px * q.sx - q.pl;
+        for (int j = 0; j < k.nj; ++j) mask |= (unsigned)(ix0 + j >= 0 && ix0 + j < q.W) << j;
+        for (int i = 0; i < k.ni; ++i) mask |= (unsigned)(iy0 + i >= 0 && iy0 + i < q.H) << (k.nj + i);
+        xb = (b * q.C + (q.depthwise ? ch : 0)) * (q.H * q.W) + iy0 * q.W + ix0;
+        wb = ch * q.Cw * T;
+    }
+    const float sum = SHAPE == 0 ? walk_f32(k, x, w, xb, wb, mask) : walk3x3_f32<SHAPE ? SHAPE : 1>(k, x, w, xb, wb, mask);
+    float r = sum + (beta != 0.0f ? beta * out[idx] : 0.0f);
+    if (bias) r = bias[ch] + r;
+    out[idx] = r;
 }
 
 // dw[o,c',ty,tx] = sum over batch and the output pixels whose tap (ty,tx) falls inside the input + beta * dw.
@@ -599,56 +703,381 @@ static int make_conv(const n2d2hip_conv_desc* d, int B, int H, int W, bool backw
     return N2D2HIP_OK;
 }
 
-// The matrix-core kernel serves ungrouped convolutions without dilation that are worth a 128 x 128 tile; the direct
-// kernels keep the rest (depthwise, dilated, tiny).  The descriptor's kernel_choice (N2D2HIP_KERNEL_F32_DIRECT / _GEMM) overrides the size rule.
-static bool use_gemm(const ConvF32& q)
+static int ceil_div_i(long a, long b) { return (int)((a + b - 1) / b); }
+
+static bool spans_input(const ConvF32& q)
 {
-    if (q.depthwise || q.dx != 1 || q.dy != 1)
-        return false;
-    if (q.choice & N2D2HIP_KERNEL_F32_DIRECT) return false;
-    if (q.choice & N2D2HIP_KERNEL_F32_GEMM) return true;
-    return 2.0 * q.B * q.O * q.oH * q.oW * q.C * q.kH * q.kW >= 2.0e7;
+    return q.kH == q.H && q.kW == q.W && q.oH == 1 && q.oW == 1 && q.pl == 0 && q.pt == 0 && q.pr == 0 && q.pb == 0;
 }
 
-static GemmF32 make_gemm(const ConvF32& q, int mode)
+enum { PASS_FWD = 0, PASS_BWD_DATA = 1, PASS_BWD_FILTER = 2 };
+enum { F32_PATH_DIRECT, F32_PATH_GEMM, F32_PATH_SMALL };
+
+// The kernels of a pass.  The matrix cores serve ungrouped convolutions without dilation; the direct kernels keep the rest
+// (depthwise, dilated) and the forward sums below 2e7 flops or of kernels over 64 taps, which stay in the reference's order
+// of terms (quantizers turn the last bit of a sum into a level now and then).  Backward-filter below 2e7 flops stays in
+// double (F32_PATH_SMALL).  The descriptor's kernel_choice (N2D2HIP_KERNEL_F32_DIRECT / _GEMM) overrides the size rules.
+static int f32_path(const ConvF32& q, int pass)
 {
-    GemmF32 g = {q.B, q.C, q.H, q.W, q.O, q.oH, q.oW, q.kW, q.kH, q.sx, q.sy, q.pl, q.pt, 0, 0, 0, 0, 0, 0};
-    const unsigned xb = (unsigned)((size_t)q.B * q.C * q.H * q.W * 4), yb = (unsigned)((size_t)q.B * q.O * q.oH * q.oW * 4);
-    const unsigned wb = (unsigned)((size_t)q.O * q.C * q.kH * q.kW * 4);
-    if (mode == GEMM_FWD) { g.P = q.B * q.oH * q.oW; g.Q = q.O; g.K = q.C * q.kH * q.kW; g.bytesP = xb; g.bytesQ = wb; }
-    else if (mode == GEMM_BWD_DATA) { g.P = q.B * q.H * q.W; g.Q = q.C; g.K = q.O * q.kH * q.kW; g.bytesP = yb; g.bytesQ = wb; }
-    else { g.P = q.C * q.kH * q.kW; g.Q = q.O; g.K = q.B * q.oH * q.oW; g.bytesP = xb; g.bytesQ = yb; }
-    g.kchunk = round_up(g.K, GK);
+    if (q.depthwise || q.dx != 1 || q.dy != 1 || (q.choice & N2D2HIP_KERNEL_F32_DIRECT))
+        return F32_PATH_DIRECT;
+    // 32-bit byte offsets from a base moved back by the padding, and one validity bit per tap row and column
+    const size_t lim = ((size_t)1 << 29) - (size_t)(q.pt + q.kH) * (q.W + q.oW + q.pl + q.kW);
+    const bool many_taps = q.kH + q.kW > 31 || q.kH * q.kW > 64;
+    if ((size_t)q.B * q.C * q.H * q.W >= lim || (size_t)q.B * q.O * q.oH * q.oW >= lim || (size_t)q.O * q.C * q.kH * q.kW >= lim
+        || (many_taps && !spans_input(q)))
+        return F32_PATH_DIRECT;
+    if (q.choice & N2D2HIP_KERNEL_F32_GEMM) return F32_PATH_GEMM;
+    const bool small = 2.0 * q.B * q.O * q.oH * q.oW * q.C * q.kH * q.kW < 2.0e7;
+    if (pass == PASS_FWD) return small || many_taps ? F32_PATH_DIRECT : F32_PATH_GEMM;
+    return small && pass == PASS_BWD_FILTER ? F32_PATH_SMALL : F32_PATH_GEMM;
+}
+
+static DivF32 div_of(int d)
+{
+    DivF32 r;
+    magic_div((unsigned)d, &r.mul, &r.sh);
+    return r;
+}
+
+// The direct kernel of forward and backward-data: the walk with 32-bit offsets and one mask bit per tap row and column, or
+// (dilated, larger) one load after the other.
+static int run_direct(const ConvF32& q, int pass, const float* x, const float* w, const float* bias, float beta, float* out, hipStream_t st)
+{
+    const bool bwd = pass == PASS_BWD_DATA;
+    const size_t lim = (size_t)1 << 31, total = (size_t)q.B * (bwd ? (size_t)q.C * q.H * q.W : (size_t)q.O * q.oH * q.oW);
+    const size_t source = (size_t)q.B * (bwd ? (size_t)q.O * q.oH * q.oW : (size_t)q.C * q.H * q.W);
+    const int T = q.kH * q.kW;
+    const long K = (long)q.C * T;
+    // (a kernel of 3x3 has an order of its own; 16-byte loads)
+    if (!bwd && !q.depthwise && q.dx == 1 && q.dy == 1 && spans_input(q) && (q.kH != 3 || q.kW != 3) && K % 4 == 0 && K < (1 << 22)
+        && (((size_t)x | (size_t)w) & 15) == 0) {
+        hipLaunchKernelGGL(conv_f32_chain_kernel, dim3(ceil_div_i(q.B, 8), ceil_div_i(q.O, 8)), dim3(64), 0, st, q.B, q.O, (int)K, x, w, bias, beta, out);
+        N2D2HIP_HIP_CHECK(hipGetLastError());
+        return N2D2HIP_OK;
+    }
+    if (q.dx != 1 || q.dy != 1 || total >= lim - 64 || source >= lim || (size_t)q.O * q.Cw * T >= lim || q.kH + q.kW > 31) {
+        if (bwd) hipLaunchKernelGGL(conv_f32_backward_data_kernel, dim3(grid_for(total)), dim3(TBLOCK), 0, st, q, w, x, beta, out);
+        else hipLaunchKernelGGL(conv_f32_forward_kernel, dim3(grid_for(total)), dim3(TBLOCK), 0, st, q, x, w, bias, beta, out);
+        N2D2HIP_HIP_CHECK(hipGetLastError());
+        return N2D2HIP_OK;
+    }
+    WalkF32 k = {};
+    if (bwd) {
+        k = {q.depthwise ? 1 : q.O, ceil_div_i(q.kH, q.sy), ceil_div_i(q.kW, q.sx), q.oH * q.oW, -q.oW, -1, q.Cw * T, q.sy * q.kW, q.sx,
+             div_of(q.H * q.W), div_of(q.W), div_of(q.C)};
+        hipLaunchKernelGGL((conv_f32_walk_kernel<true, 0>), dim3((unsigned)((total + 63) / 64)), dim3(64), 0, st, q, k, x, w, bias, beta, out, (int)total);
+    } else {
+        k = {q.depthwise ? 1 : q.C, q.kH, q.kW, q.H * q.W, q.W, 1, T, q.kW, 1, div_of(q.oH * q.oW), div_of(q.oW), div_of(q.O)};
+        const dim3 grid((unsigned)((total + 63) / 64));
+        if (q.kH != 3 || q.kW != 3) hipLaunchKernelGGL((conv_f32_walk_kernel<false, 0>), grid, dim3(64), 0, st, q, k, x, w, bias, beta, out, (int)total);
+        else if (k.n == 1) hipLaunchKernelGGL((conv_f32_walk_kernel<false, 1>), grid, dim3(64), 0, st, q, k, x, w, bias, beta, out, (int)total);
+        else hipLaunchKernelGGL((conv_f32_walk_kernel<false, 4>), grid, dim3(64), 0, st, q, k, x, w, bias, beta, out, (int)total);
+    }
+    N2D2HIP_HIP_CHECK(hipGetLastError());
+    return N2D2HIP_OK;
+}
+
+// A kernel that spans its input (an FcCell) makes of each pass a plain matrix product, which is a 1x1 convolution with the
+// roles of the tensors exchanged so that the long contiguous dimension is the one the kernels read contiguously:
+//   forward          y[b][o] = sum_k x[b][k] w[o][k]     the filter pass of pixels k between "channels" w[o] and "outputs" x[b]
+//   backward data    dx[b][k] = sum_o dy[b][o] w[o][k]   the forward pass over one "image" w of O channels and K pixels
+//   backward filter  dw[o][k] = sum_b dy[b][o] x[b][k]   the data pass over one "image" x of B channels and K pixels
+static ConvF32 product_of(const ConvF32& q, int pass, int* as_pass)
+{
+    const int K = q.C * q.H * q.W;
+    *as_pass = pass == PASS_FWD ? PASS_BWD_FILTER : pass == PASS_BWD_DATA ? PASS_FWD : PASS_BWD_DATA;
+    return ConvF32{1, q.O, 1, K, q.B, 1, K, 1, 1, q.O, 1, 1, 0, 0, 0, 0, 1, 1, 0, q.choice};
+}
+
+// ---- forward and backward-data: tile shape and K ranges of a launch
+struct PixelPlan {
+    bool small_q;              // tiles of 32 q x 128 pixels instead of 64 x 64
+    int splits;                // K ranges that leave partial results
+    int kind;                  // PIXELS_*
+    PixelGemm g;
+};
+
+// Classes of pixels of one launch (backward-data of a strided convolution: s * s residue classes, those with the most taps
+// first).  Returns how many launches of up to PIXEL_CLASSES classes the pass takes.
+static std::vector<PixelClass> pixel_classes(const ConvF32& q, int pass)
+{
+    std::vector<PixelClass> v;
+    if (pass == PASS_FWD) {
+        PixelClass c = {};
+        c.gW = q.oW; c.gHW = q.oH * q.oW; c.P = q.B * c.gHW;
+        c.nx = q.kW; c.nT = q.kH * q.kW;
+        c.y0 = -q.pt; c.x0 = -q.pl;
+        c.stepy = q.W; c.stepx = 1;
+        c.bias = q.pt * q.W + q.pl; c.soff0 = 0;
+        v.push_back(c);
+    } else {
+        for (int ry = 0; ry < std::min(q.sy, q.H); ++ry)
+            for (int rx = 0; rx < std::min(q.sx, q.W); ++rx) {
+                PixelClass c = {};
+                c.gW = (q.W - rx + q.sx - 1) / q.sx;
+                c.gHW = ((q.H - ry + q.sy - 1) / q.sy) * c.gW;
+                c.P = q.B * c.gHW;
+                c.ty0 = (ry + q.pt) % q.sy; c.tx0 = (rx + q.pl) % q.sx;
+                const int ny = c.ty0 < q.kH ? (q.kH - 1 - c.ty0) / q.sy + 1 : 0;
+                c.nx = c.tx0 < q.kW ? (q.kW - 1 - c.tx0) / q.sx + 1 : 0;
+                c.nT = ny * c.nx;
+                c.y0 = (ry + q.pt) / q.sy; c.x0 = (rx + q.pl) / q.sx;
+                c.stepy = -q.oW; c.stepx = -1;
+                c.ry = ry; c.rx = rx;
+                const int first = c.y0 * q.oW + c.x0, last = first - std::max(ny - 1, 0) * q.oW - std::max(c.nx - 1, 0);
+                c.bias = std::max(0, -last);
+                c.soff0 = first + c.bias;
+                v.push_back(c);
+            }
+        std::stable_sort(v.begin(), v.end(), [](const PixelClass& a, const PixelClass& b) { return a.nT > b.nT; });
+    }
+    for (PixelClass& c : v) {
+        c.ghw = div_of(c.gHW); c.gw = div_of(c.gW); c.nt = div_of(c.nT); c.nxd = div_of(c.nx);
+    }
+    return v;
+}
+
+enum { PIXELS_TAPS, PIXELS_CHUNK, PIXELS_3X3 };
+static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass> cls, int kind)
+{
+    PixelPlan pl = {};
+    PixelGemm& g = pl.g;
+    const bool fwd = pass == PASS_FWD;
+    g.Q = fwd ? q.O : q.C;
+    g.Ch = fwd ? q.C : q.O;
+    g.sy = fwd ? q.sy : 1; g.sx = fwd ? q.sx : 1;
+    g.d = fwd ? 1 : -1;
+    g.Hs = fwd ? q.H : q.oH; g.Ws = fwd ? q.W : q.oW; g.planeS = g.Hs * g.Ws;
+    const int T = q.kH * q.kW;
+    g.qs = fwd ? q.C * T : T; g.chs = fwd ? T : q.C * T; g.kW = q.kW; g.osy = fwd ? 1 : q.sy; g.osx = fwd ? 1 : q.sx;
+    g.planeO = fwd ? q.oH * q.oW : q.H * q.W; g.Wo = fwd ? q.oW : q.W;
+    g.bytesX = (unsigned)(4 * (size_t)q.B * g.Ch * g.planeS);
+    g.bytesW = (unsigned)(4 * (size_t)q.O * q.C * T);
+    // tile shape
+    long P = 0, kmax = 0;
+    const int nchunks = ceil_div_i(g.Ch, GK);
+    for (const PixelClass& c : cls) { P += c.P; kmax = std::max<long>(kmax, (long)(kind == PIXELS_CHUNK && !fwd ? nchunks * GK : g.Ch) * c.nT); }
+    // (64 x 64 tiles, four to a CU, lost at most 4 % to the best of 32 x 128, 64 x 128 and 128 x 128 on every shape with Q
+    // over 32 that was timed, and gained up to 70 % where the larger tiles are few)
+    pl.small_q = g.Q <= 32;
+    const int PT = pl.small_q ? 128 : 64, QT = pl.small_q ? 32 : 64;
+    g.qtiles = ceil_div_i(g.Q, QT);
+    pl.kind = kind;
+    g.T = T;
+    g.qpad = g.qtiles * QT;
+    long tiles = 0;
+    g.nclass = (int)cls.size();
+    for (int i = 0; i < g.nclass; ++i) {
+        cls[i].tile0 = (int)tiles;
+        tiles += ceil_div_i(cls[i].P, PT);
+        g.c[i] = cls[i];
+    }
+    g.ptiles = (int)tiles;
+    g.ptiles8 = ceil_div_i(tiles, 8);
+    const long blocks = tiles * g.qtiles;
+    g.nz = 1;
+    long splits;
+    if (fwd) {
+        // The ranges of a forward sum follow from its sizes alone, as if tiles were 128 x 128: with another order of additions
+        // the quantizer behind it would give another level now and then.  With a block for every CU it takes all of them.
+        const long tiles128 = (long)ceil_div_i(P, 128) * (g.Q <= 64 ? 1 : ceil_div_i(g.Q, 128));
+        splits = tiles128 >= 384 ? 1 : std::max(1L, 768 / tiles128);
+        splits = std::min<long>(splits, std::max(1L, kmax / (16 * GK)));
+    } else {
+        // where the tiles do not fill the chip twice; none below four steps
+        splits = blocks >= 512 ? 1 : std::max(1L, 768 / blocks);
+        splits = std::min<long>(splits, std::max(1L, kmax / (4 * GK)));
+    }
+    g.kchunk = std::max(round_up((int)((kmax + splits - 1) / splits), GK), GK);
+    pl.splits = std::max(1, ceil_div_i(kmax, g.kchunk));
+    if (fwd && blocks >= 256) {
+        g.nz = pl.splits;
+        pl.splits = 1;
+    }
+    if (kind == PIXELS_CHUNK) g.kchunk /= GK;
+    return pl;
+}
+
+template <bool BWD>
+static void launch_pixels(PixelPlan& pl, int splits, const float* x, const float* w, const float* bias, float beta, float* out, size_t partial,
+                          hipStream_t st)
+{
+    const dim3 grid(pl.g.ptiles8 * 8 * pl.g.qtiles, 1, splits);
+    if (pl.kind == PIXELS_3X3) {
+        if (pl.small_q) hipLaunchKernelGGL((conv_f32_3x3_kernel<1, 4>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
+        else hipLaunchKernelGGL((conv_f32_3x3_kernel<2, 2>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
+        return;
+    }
+    if (pl.kind == PIXELS_CHUNK) {
+        if (pl.small_q) hipLaunchKernelGGL((conv_f32_chunk_kernel<1, 4, 3>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
+        else hipLaunchKernelGGL((conv_f32_chunk_kernel<2, 2, 3>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
+        return;
+    }
+    if (pl.small_q) hipLaunchKernelGGL((conv_f32_pixel_kernel<BWD, 1, 4, 3>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
+    else hipLaunchKernelGGL((conv_f32_pixel_kernel<BWD, 2, 2, 3>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
+}
+
+static unsigned reduce_grid(size_t n) { return (unsigned)std::min<size_t>((n + 63) / 64, 16384); }
+
+// ---- backward-filter
+struct FilterPlan {
+    bool small_q;              // tiles of 32 q x 128 columns instead of 64 x 64
+    int splits;
+    FilterGemm g;
+};
+static FilterGemm filter_gemm(const ConvF32& q)
+{
+    FilterGemm g = {};
+    g.P = q.C * q.kH * q.kW; g.Q = q.O; g.K = q.B * q.oH * q.oW;
+    g.C = q.C; g.H = q.H; g.W = q.W; g.kW = q.kW; g.kH = q.kH;
+    g.s_y = q.sy; g.s_x = q.sx; g.pt = q.pt; g.pl = q.pl;
+    g.oW = q.oW; g.plane = q.oH * q.oW;
+    g.imgX = q.C * q.H * q.W; g.imgY = q.O * g.plane;
+    g.bytesX = (unsigned)(4 * (size_t)q.B * g.imgX); g.bytesY = (unsigned)(4 * (size_t)q.B * g.imgY);
+    g.dplane = div_of(g.plane); g.dow = div_of(g.oW);
     return g;
 }
-
-// K ranges of backward-filter: enough blocks to fill the chip, each range at least 32 steps long
-static int filter_splits(GemmF32* g)
+static FilterPlan plan_filter(const ConvF32& q)
 {
-    const long tiles = (long)((g->P + GT - 1) / GT) * (g->Q <= 64 ? 1 : (g->Q + GT - 1) / GT);
-    long splits = std::max(1L, 1024 / tiles);
-    splits = std::min<long>(splits, std::max(1, g->K / (32 * GK)));
-    g->kchunk = round_up((int)((g->K + splits - 1) / splits), GK);
-    return (g->K + g->kchunk - 1) / g->kchunk;
+    FilterPlan pl = {};
+    FilterGemm& g = pl.g;
+    g = filter_gemm(q);
+    pl.small_q = g.Q <= 32;
+    const long tiles = (long)ceil_div_i(g.P, pl.small_q ? 128 : 64) * ceil_div_i(g.Q, pl.small_q ? 32 : 64);
+    // (few tiles: four blocks per CU, two of the wide ones, beyond which the partial results cost more than the last round of
+    // blocks; many: three blocks per tile or six per CU)
+    long splits = tiles <= 256 ? (pl.small_q ? 512 : 1024) / tiles : std::max(1L, (1535 + tiles) / tiles);
+    splits = std::min<long>(splits, std::max(1, g.K / (4 * FK)));
+    g.kchunk = round_up((int)((g.K + splits - 1) / splits), FK);
+    pl.splits = ceil_div_i(g.K, g.kchunk);
+    return pl;
+}
+// The small backward-filter: enough ranges for two blocks per CU, none below 128 pixels (two rounds of a wave's loads).
+static int small_filter_splits(const FilterGemm& g)
+{
+    const long tiles = (long)ceil_div_i(g.P, 16) * ceil_div_i(g.Q, 16);
+    return (int)std::max(1L, std::min<long>(512 / tiles, g.K / 128));
+}
+// (a workspace too small for the partial results: one range)
+static int run_small_filter(const ConvF32& q, const float* x, const float* dy, float beta, float* out, double* ws, size_t ws_bytes, hipStream_t st)
+{
+    FilterGemm g = filter_gemm(q);
+    const size_t n = (size_t)g.Q * g.P;
+    int splits = small_filter_splits(g);
+    if (splits * n * sizeof(double) > ws_bytes || ((size_t)ws & 7)) splits = 1;
+    g.kchunk = round_up(ceil_div_i(g.K, splits), 64);
+    splits = ceil_div_i(g.K, g.kchunk);
+    hipLaunchKernelGGL(conv_f32_filter_small_kernel, dim3(ceil_div_i(g.P, 16), ceil_div_i(g.Q, 16), splits), dim3(256), 0, st, g, x, dy, ws, beta, out);
+    if (splits > 1)
+        hipLaunchKernelGGL(conv_f32_reduce_partials_kernel<double>, dim3(reduce_grid(n)), dim3(256), 0, st, (const double*)ws, splits, n, beta, out,
+                           (const float*)nullptr, 1, 1);
+    N2D2HIP_HIP_CHECK(hipGetLastError());
+    return N2D2HIP_OK;
+}
+static void launch_filter(const FilterPlan& pl, const float* x, const float* dy, float* out, hipStream_t st)
+{
+    const dim3 grid(ceil_div_i(pl.g.P, pl.small_q ? 128 : 64), ceil_div_i(pl.g.Q, pl.small_q ? 32 : 64), pl.splits);
+    if (pl.small_q) hipLaunchKernelGGL((conv_f32_filter_kernel<1, 4, 2>), grid, dim3(256), 0, st, pl.g, x, dy, out);
+    else hipLaunchKernelGGL((conv_f32_filter_kernel<2, 2, 2>), grid, dim3(256), 0, st, pl.g, x, dy, out);
 }
 
-// K ranges of forward / backward-data when the tiles alone leave most of the chip idle (three blocks fit a CU): each
-// range at least 16 steps long
-static int pass_splits(GemmF32* g)
+// The order of K.  3x3 kernels, forward or at stride 1: four channels with their taps at a time.  Chunks of 16 channels at one
+// tap: 1x1 kernels, and backward-data, where padding the channels to them costs less than testing every load (about a
+// fifth).  Both lay the weights out first (a launch of 3 us: even at 3 to 7e8 flops).
+static int pixels_kind(const ConvF32& q, int pass)
 {
-    const long tiles = (long)((g->P + GT - 1) / GT) * (g->Q <= 64 ? 1 : (g->Q + GT - 1) / GT);
-    long splits = tiles >= 384 ? 1 : std::max(1L, 768 / tiles);
-    splits = std::min<long>(splits, std::max(1, g->K / (16 * GK)));
-    g->kchunk = round_up((int)((g->K + splits - 1) / splits), GK);
-    return (g->K + g->kchunk - 1) / g->kchunk;
+    const int ch = pass == PASS_FWD ? q.C : q.O, T = q.kH * q.kW;
+    if (2.0 * q.B * q.O * q.oH * q.oW * q.C * T < 5.0e8 || (size_t)(q.O + 64) * (q.C + 64) * (T + 2) >= ((size_t)1 << 28))
+        return PIXELS_TAPS;
+    if (q.kH == 3 && q.kW == 3 && (pass == PASS_FWD || (q.sx == 1 && q.sy == 1)) && round_up(ch, 4) * 5 <= ch * 7)
+        return PIXELS_3X3;
+    return (pass == PASS_BWD_DATA || T == 1) && round_up(ch, GK) * 5 <= ch * 6 ? PIXELS_CHUNK : PIXELS_TAPS;
+}
+static size_t laid_weights(const ConvF32& q, int pass, int kind)
+{
+    const int ch = pass == PASS_FWD ? q.C : q.O, rows = pass == PASS_FWD ? q.O : q.C, qpad = round_up(rows, rows <= 32 ? 32 : 64);
+    if (kind == PIXELS_TAPS) return 0;
+    return kind == PIXELS_3X3 ? (size_t)(ch + 3) / 4 * qpad * W33 : (size_t)round_up(ch, GK) * q.kH * q.kW * qpad;
 }
 
-static bool fits_int(const ConvF32& q)
+// Floats of workspace a pass takes when it may split its K
+static size_t pass_workspace(const ConvF32& q, int pass)
 {
-    // the GEMM kernel reads tensors of at most 2 GiB through buffer descriptors and keeps one validity bit per tap
-    const size_t lim = (size_t)1 << 29;
-    return (size_t)q.B * q.C * q.H * q.W < lim && (size_t)q.B * q.O * q.oH * q.oW < lim && (size_t)q.O * q.C * q.kH * q.kW < lim
-           && q.kH * q.kW <= 64;
+    if (pass == PASS_BWD_FILTER) {
+        const FilterPlan pl = plan_filter(q);
+        return (size_t)pl.splits * pl.g.Q * pl.g.P;
+    }
+    const int kind = pixels_kind(q, pass);
+    const std::vector<PixelClass> cls = pixel_classes(q, pass);
+    const size_t n = (size_t)q.B * (pass == PASS_FWD ? (size_t)q.O * q.oH * q.oW : (size_t)q.C * q.H * q.W);
+    int splits = 1;
+    for (size_t i = 0; i < cls.size(); i += PIXEL_CLASSES)
+        splits = std::max(splits, plan_pixels(q, pass, std::vector<PixelClass>(cls.begin() + i, cls.begin() + std::min(cls.size(), i + PIXEL_CLASSES)), kind).splits);
+    return (splits > 1 ? splits * n : 0) + laid_weights(q, pass, kind);
+}
+
+// Runs one pass of q (which qualifies for the matrix cores): out = pass(x, w) + beta * out (+ bias[channel] forward).
+// The tensors are the pass's own operands: forward (x, w), backward-data (dy, w), backward-filter (x, dy).
+static int run_pass(const ConvF32& q, int pass, const float* a, const float* b, const float* bias, int bias_plane, int bias_channels, float beta,
+                    float* out, float* ws, size_t ws_floats, hipStream_t st)
+{
+    if (pass == PASS_BWD_FILTER) {
+        FilterPlan pl = plan_filter(q);
+        const size_t n = (size_t)pl.g.Q * pl.g.P;
+        bool direct = false;
+        if (pl.splits * n > ws_floats) {
+            pl.splits = 1;
+            pl.g.kchunk = round_up(pl.g.K, FK);
+        }
+        direct = pl.splits == 1 && beta == 0.0f && !bias;
+        N2D2HIP_REQUIRE(direct || pl.splits * n <= ws_floats, N2D2HIP_ERR_WORKSPACE, "convolution: workspace of %zu bytes, %zu needed", 4 * ws_floats,
+                        4 * pl.splits * n);
+        launch_filter(pl, a, b, direct ? out : ws, st);
+        if (!direct)
+            hipLaunchKernelGGL(conv_f32_reduce_partials_kernel<float>, dim3(reduce_grid(n)), dim3(256), 0, st, (const float*)ws, pl.splits, n, beta, out, bias,
+                               bias_plane, bias_channels);
+        N2D2HIP_HIP_CHECK(hipGetLastError());
+        return N2D2HIP_OK;
+    }
+    const size_t n = (size_t)q.B * (pass == PASS_FWD ? (size_t)q.O * q.oH * q.oW : (size_t)q.C * q.H * q.W);
+    // (the weights laid out come first in the workspace; without room for them, K tap by tap)
+    int kind = pixels_kind(q, pass);
+    const size_t nlaid = laid_weights(q, pass, kind);
+    if (nlaid > ws_floats || ((size_t)ws & 15)) kind = PIXELS_TAPS;
+    const std::vector<PixelClass> cls = pixel_classes(q, pass);
+    std::vector<PixelPlan> plans;
+    int splits = 1;
+    for (size_t i = 0; i < cls.size(); i += PIXEL_CLASSES) {
+        plans.push_back(plan_pixels(q, pass, std::vector<PixelClass>(cls.begin() + i, cls.begin() + std::min(cls.size(), i + PIXEL_CLASSES)), kind));
+        splits = std::max(splits, plans.back().splits);
+    }
+    const float* w = b;
+    if (kind != PIXELS_TAPS) {
+        const PixelGemm& g = plans[0].g;
+        const int total = (int)(kind == PIXELS_3X3 ? nlaid : nlaid / 4);
+        const dim3 grid(std::min((total + 255) / 256, 4096));
+        if (kind == PIXELS_3X3) hipLaunchKernelGGL(conv_f32_lay_weights3x3_kernel, grid, dim3(256), 0, st, b, ws, total, g.Q, g.qpad, g.Ch, g.qs, g.chs);
+        else hipLaunchKernelGGL(conv_f32_lay_weights_kernel, grid, dim3(256), 0, st, b, ws, total, g.Q, g.qpad, g.Ch, g.T, g.qs, g.chs);
+        w = ws;
+        ws += nlaid;
+        ws_floats -= nlaid;
+    }
+    if (splits * n > ws_floats) {                           // no room for partial results: a block takes all ranges
+        for (PixelPlan& pl : plans) pl.g.nz *= pl.splits;
+        splits = 1;
+    }
+    for (PixelPlan& pl : plans) {
+        float* dst = splits > 1 ? ws : out;
+        // (every launch runs the ranges of the pass, so that each partial result is complete)
+        if (pass == PASS_FWD) launch_pixels<false>(pl, splits, a, w, splits > 1 ? nullptr : bias, splits > 1 ? 0.0f : beta, dst, splits > 1 ? n : 0, st);
+        else launch_pixels<true>(pl, splits, a, w, nullptr, splits > 1 ? 0.0f : beta, dst, splits > 1 ? n : 0, st);
+    }
+    if (splits > 1)
+        hipLaunchKernelGGL(conv_f32_reduce_partials_kernel<float>, dim3(reduce_grid(n)), dim3(256), 0, st, (const float*)ws, splits, n, beta, out, bias,
+                           bias_plane, bias_channels);
+    N2D2HIP_HIP_CHECK(hipGetLastError());
+    return N2D2HIP_OK;
 }
 
 } // namespace n2d2hip
@@ -664,31 +1093,19 @@ int n2d2hip_conv2d_f32_forward(const n2d2hip_conv_desc* desc, int B, int H, int 
     const int st = make_conv(desc, B, H, W, false, &q, "n2d2hip_conv2d_f32_forward");
     if (st != N2D2HIP_OK) return st;
     N2D2HIP_REQUIRE(x && w && y, N2D2HIP_ERR_INVALID, "n2d2hip_conv2d_f32_forward: null pointer");
-    if (use_gemm(q) && fits_int(q)) {
-        GemmF32 g = make_gemm(q, GEMM_FWD);
-        const size_t n = (size_t)g.P * g.Q;
-        int splits = pass_splits(&g);
-        if (splits > 1 && (!workspace || workspace_bytes < (size_t)splits * n * sizeof(float))) {
-            splits = 1;                                     // no room for partial results: one range
-            g.kchunk = round_up(g.K, GK);
+    if (f32_path(q, PASS_FWD) == F32_PATH_GEMM) {
+        float* ws = (float*)workspace;
+        const size_t nws = workspace ? workspace_bytes / sizeof(float) : 0;
+        if (spans_input(q)) {
+            int pass;
+            const ConvF32 m = product_of(q, PASS_FWD, &pass);
+            // (without a workspace that holds its partial results: the convolution as it stands)
+            if (pass_workspace(m, pass) <= nws)
+                return run_pass(m, pass, w, x, bias, 1, q.O, beta, y, ws, nws, (hipStream_t)stream);
         }
-        float* dst = splits > 1 ? (float*)workspace : y;
-        if (g.Q <= 64)
-            hipLaunchKernelGGL((conv_f32_gemm_kernel<GEMM_FWD, 64>), dim3((g.P + GT - 1) / GT, 1, splits), dim3(256), 0, (hipStream_t)stream,
-                               g, x, w, bias, beta, dst);
-        else
-            hipLaunchKernelGGL((conv_f32_gemm_kernel<GEMM_FWD, 128>), dim3((g.P + GT - 1) / GT, (g.Q + GT - 1) / GT, splits), dim3(256), 0,
-                               (hipStream_t)stream, g, x, w, bias, beta, dst);
-        if (splits > 1)
-            hipLaunchKernelGGL(conv_f32_reduce_partials_kernel, dim3(grid_for(n)), dim3(256), 0, (hipStream_t)stream, (const float*)workspace, splits, n,
-                               beta, y, bias, q.oH * q.oW, q.O);
-        N2D2HIP_HIP_CHECK(hipGetLastError());
-        return N2D2HIP_OK;
+        return run_pass(q, PASS_FWD, x, w, bias, q.oH * q.oW, q.O, beta, y, ws, nws, (hipStream_t)stream);
     }
-    hipLaunchKernelGGL(conv_f32_forward_kernel, dim3(grid_for((size_t)q.B * q.O * q.oH * q.oW)), dim3(TBLOCK), 0, (hipStream_t)stream,
-                       q, x, w, bias, beta, y);
-    N2D2HIP_HIP_CHECK(hipGetLastError());
-    return N2D2HIP_OK;
+    return run_direct(q, PASS_FWD, x, w, bias, beta, y, (hipStream_t)stream);
 }
 
 int n2d2hip_conv2d_f32_backward_data(const n2d2hip_conv_desc* desc, int B, int H, int W, const float* w, const float* diff_y, float beta,
@@ -698,45 +1115,37 @@ int n2d2hip_conv2d_f32_backward_data(const n2d2hip_conv_desc* desc, int B, int H
     const int st = make_conv(desc, B, H, W, true, &q, "n2d2hip_conv2d_f32_backward_data");
     if (st != N2D2HIP_OK) return st;
     N2D2HIP_REQUIRE(w && diff_y && diff_x, N2D2HIP_ERR_INVALID, "n2d2hip_conv2d_f32_backward_data: null pointer");
-    if (use_gemm(q) && fits_int(q)) {
-        GemmF32 g = make_gemm(q, GEMM_BWD_DATA);
-        const size_t n = (size_t)g.P * g.Q;
-        int splits = pass_splits(&g);
-        if (splits > 1 && (!workspace || workspace_bytes < (size_t)splits * n * sizeof(float))) {
-            splits = 1;
-            g.kchunk = round_up(g.K, GK);
+    if (f32_path(q, PASS_BWD_DATA) == F32_PATH_GEMM) {
+        float* ws = (float*)workspace;
+        const size_t nws = workspace ? workspace_bytes / sizeof(float) : 0;
+        if (spans_input(q)) {
+            int pass;
+            const ConvF32 m = product_of(q, PASS_BWD_DATA, &pass);
+            return run_pass(m, pass, w, diff_y, nullptr, 1, 1, beta, diff_x, ws, nws, (hipStream_t)stream);
         }
-        float* dst = splits > 1 ? (float*)workspace : diff_x;
-        if (g.Q <= 64)
-            hipLaunchKernelGGL((conv_f32_gemm_kernel<GEMM_BWD_DATA, 64>), dim3((g.P + GT - 1) / GT, 1, splits), dim3(256), 0, (hipStream_t)stream,
-                               g, diff_y, w, (const float*)nullptr, beta, dst);
-        else
-            hipLaunchKernelGGL((conv_f32_gemm_kernel<GEMM_BWD_DATA, 128>), dim3((g.P + GT - 1) / GT, (g.Q + GT - 1) / GT, splits), dim3(256), 0,
-                               (hipStream_t)stream, g, diff_y, w, (const float*)nullptr, beta, dst);
-        if (splits > 1)
-            hipLaunchKernelGGL(conv_f32_reduce_partials_kernel, dim3(grid_for(n)), dim3(256), 0, (hipStream_t)stream, (const float*)workspace, splits, n,
-                               beta, diff_x, (const float*)nullptr, 1, 1);
-        N2D2HIP_HIP_CHECK(hipGetLastError());
-        return N2D2HIP_OK;
+        return run_pass(q, PASS_BWD_DATA, diff_y, w, nullptr, 1, 1, beta, diff_x, ws, nws, (hipStream_t)stream);
     }
-    hipLaunchKernelGGL(conv_f32_backward_data_kernel, dim3(grid_for((size_t)q.B * q.C * q.H * q.W)), dim3(TBLOCK), 0, (hipStream_t)stream,
-                       q, w, diff_y, beta, diff_x);
-    N2D2HIP_HIP_CHECK(hipGetLastError());
-    return N2D2HIP_OK;
+    return run_direct(q, PASS_BWD_DATA, diff_y, w, nullptr, beta, diff_x, (hipStream_t)stream);
 }
 
 size_t n2d2hip_conv2d_f32_workspace_bytes(const n2d2hip_conv_desc* desc, int B, int H, int W)
 {
     ConvF32 q;
-    if (make_conv(desc, B, H, W, true, &q, "n2d2hip_conv2d_f32_workspace_bytes") != N2D2HIP_OK || !use_gemm(q) || !fits_int(q))
+    if (make_conv(desc, B, H, W, true, &q, "n2d2hip_conv2d_f32_workspace_bytes") != N2D2HIP_OK)
         return 0;
-    GemmF32 g = make_gemm(q, GEMM_BWD_FILTER);
-    size_t need = (size_t)filter_splits(&g) * g.Q * g.P;
-    for (int mode : {GEMM_FWD, GEMM_BWD_DATA}) {
-        g = make_gemm(q, mode);
-        const int splits = pass_splits(&g);
-        if (splits > 1)
-            need = std::max(need, (size_t)splits * g.Q * g.P);
+    size_t need = 0;
+    for (int pass : {PASS_FWD, PASS_BWD_DATA, PASS_BWD_FILTER}) {
+        const int path = f32_path(q, pass);
+        if (path == F32_PATH_SMALL) {
+            const FilterGemm g = filter_gemm(q);
+            const int splits = small_filter_splits(g);
+            need = std::max(need, splits > 1 ? splits * (size_t)g.Q * g.P * 2 : 0);
+        } else if (path == F32_PATH_GEMM) {
+            int as = pass;
+            const ConvF32 m = spans_input(q) ? product_of(q, pass, &as) : q;
+            need = std::max(need, pass_workspace(m, as));
+            if (pass == PASS_BWD_FILTER) need = std::max(need, (size_t)q.O * q.C * q.kH * q.kW);     // (always has one)
+        }
     }
     return need * sizeof(float);
 }
@@ -750,23 +1159,18 @@ int n2d2hip_conv2d_f32_backward_filter(const n2d2hip_conv_desc* desc, int B, int
     N2D2HIP_REQUIRE(x && diff_y && diff_w, N2D2HIP_ERR_INVALID, "n2d2hip_conv2d_f32_backward_filter: null pointer");
     const size_t nw = (size_t)q.O * q.Cw * q.kH * q.kW;
     N2D2HIP_REQUIRE(nw < ((size_t)1 << 31), N2D2HIP_ERR_INVALID, "n2d2hip_conv2d_f32_backward_filter: too many weights");
-    if (use_gemm(q) && fits_int(q)) {
-        GemmF32 g = make_gemm(q, GEMM_BWD_FILTER);
-        const int splits = filter_splits(&g);
-        const size_t need = (size_t)splits * nw * sizeof(float);
+    const int path = f32_path(q, PASS_BWD_FILTER);
+    if (path == F32_PATH_SMALL)
+        return run_small_filter(q, x, diff_y, beta, diff_w, (double*)workspace, workspace ? workspace_bytes : 0, (hipStream_t)stream);
+    if (path == F32_PATH_GEMM) {
+        int pass = PASS_BWD_FILTER;
+        const bool fc = spans_input(q);
+        const ConvF32 m = fc ? product_of(q, PASS_BWD_FILTER, &pass) : q;
+        const size_t need = std::max(nw, pass_workspace(m, pass)) * sizeof(float);
         N2D2HIP_REQUIRE(workspace && workspace_bytes >= need, N2D2HIP_ERR_WORKSPACE,
                         "n2d2hip_conv2d_f32_backward_filter: workspace of %zu bytes, %zu needed (n2d2hip_conv2d_f32_workspace_bytes)",
                         workspace_bytes, need);
-        if (g.Q <= 64)
-            hipLaunchKernelGGL((conv_f32_gemm_kernel<GEMM_BWD_FILTER, 64>), dim3((g.P + GT - 1) / GT, 1, splits), dim3(256), 0,
-                               (hipStream_t)stream, g, x, diff_y, (const float*)nullptr, 0.0f, (float*)workspace);
-        else
-            hipLaunchKernelGGL((conv_f32_gemm_kernel<GEMM_BWD_FILTER, 128>), dim3((g.P + GT - 1) / GT, (g.Q + GT - 1) / GT, splits), dim3(256), 0,
-                               (hipStream_t)stream, g, x, diff_y, (const float*)nullptr, 0.0f, (float*)workspace);
-        hipLaunchKernelGGL(conv_f32_reduce_partials_kernel, dim3(grid_for(nw)), dim3(256), 0, (hipStream_t)stream, (const float*)workspace, splits, nw,
-                           beta, diff_w, (const float*)nullptr, 1, 1);
-        N2D2HIP_HIP_CHECK(hipGetLastError());
-        return N2D2HIP_OK;
+        return run_pass(m, pass, x, diff_y, nullptr, 1, 1, beta, diff_w, (float*)workspace, workspace_bytes / sizeof(float), (hipStream_t)stream);
     }
     hipLaunchKernelGGL(conv_f32_backward_filter_kernel, dim3((unsigned)nw), dim3(TBLOCK), 0, (hipStream_t)stream, q, x, diff_y, beta, diff_w);
     N2D2HIP_HIP_CHECK(hipGetLastError());

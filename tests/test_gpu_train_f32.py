@@ -222,6 +222,45 @@ def test_conv_f32_random_rectangular_shapes(g, path):
                     np.maximum(orc.conv_backward_filter(np.abs(x64), np.abs(dy64), w.shape, **kw), 1e-3)) <= TOL
 
 
+# B, C, H, W, O, kH, kW, stride, pad: K in chunks of 16 channels with channels and rows left over, strides beyond the kernel,
+# tiles of 32 rows, kernels that span their input, and the small sums' own kernel from one weight upwards
+SIZES = [(10, 47, 33, 31, 97, 3, 3, 1, 1), (40, 128, 25, 26, 65, 2, 2, 3, 0), (31, 32, 40, 41, 31, 3, 3, 1, 1), (20, 160, 15, 17, 193, 3, 3, 2, 1),
+         (130, 120, 7, 5, 90, 7, 5, 1, 0), (33, 70, 7, 5, 65, 7, 5, 1, 0), (1, 1, 1, 1, 1, 1, 1, 1, 0), (3, 5, 9, 8, 17, 3, 3, 1, 1),
+         (32, 1, 32, 32, 6, 5, 5, 1, 0), (2, 16, 8, 8, 16, 3, 3, 2, 1)]
+
+
+@pytest.mark.parametrize("workspace", [True, False])
+@pytest.mark.parametrize("case", SIZES)
+def test_conv_kernels_chosen_by_size(g, case, workspace):
+    B, Cn, H, W, O, kH, kW, s, p = case
+    print("conv f32 by size", case, workspace, flush=True)
+    t, F = g.torch_, g.torch_.nn.functional
+    rng = np.random.default_rng(sum(case))
+    x, w = rng.normal(size=(B, Cn, H, W)).astype(np.float32), rng.normal(size=(O, Cn, kH, kW)).astype(np.float32)
+
+    def passes(x_, w_, dy_):
+        x64, w64 = (t.from_numpy(v).double().requires_grad_() for v in (x_, w_))
+        y = F.conv2d(x64, w64, stride=s, padding=p)
+        y.backward(t.from_numpy(dy_).double())
+        return [v.detach().numpy() for v in (y, x64.grad, w64.grad)]
+    oH, oW = (H + 2 * p - kH) // s + 1, (W + 2 * p - kW) // s + 1
+    dy = rng.normal(size=(B, O, oH, oW)).astype(np.float32)
+    want, mag = passes(x, w, dy), passes(np.abs(x), np.abs(w), np.abs(dy))
+    d = g.capi.ConvDesc(Cn, O, kW, kH, s, s, p, p, p, p, 1, 1, 1, 0, 0)
+    need = int(g.lib.n2d2hip_conv2d_f32_workspace_bytes(C.byref(d), B, H, W)) if workspace else 0
+    ws = g.torch_.empty(max(need, 4), dtype=t.uint8, device="cuda")
+    wp = ws.data_ptr() if need else None
+    x_, w_, dy_ = g.dev(x), g.dev(w), g.dev(dy)
+    y, dx, dw = (t.ones(v.shape, dtype=t.float32, device="cuda") for v in (dy, x, w))
+    g.check(g.lib.n2d2hip_conv2d_f32_forward(C.byref(d), B, H, W, x_.data_ptr(), w_.data_ptr(), None, 0.0, y.data_ptr(), wp, need, g.sp()))
+    g.check(g.lib.n2d2hip_conv2d_f32_backward_data(C.byref(d), B, H, W, w_.data_ptr(), dy_.data_ptr(), 1.0, dx.data_ptr(), wp, need, g.sp()))
+    assert _rel(g.host(y), want[0], np.maximum(mag[0], 1e-3)) <= TOL
+    assert _rel(g.host(dx), want[1] + 1, mag[1] + 1) <= TOL
+    if workspace or 2.0 * dy.size * Cn * kH * kW < 2e7:
+        g.check(g.lib.n2d2hip_conv2d_f32_backward_filter(C.byref(d), B, H, W, x_.data_ptr(), dy_.data_ptr(), 1.0, dw.data_ptr(), wp, need, g.sp()))
+        assert _rel(g.host(dw), want[2] + 1, mag[2] + 1) <= TOL
+
+
 def test_dilated_forward(g):
     from oracle import oracle as orc
     rng = np.random.default_rng(3)
