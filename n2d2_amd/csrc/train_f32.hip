@@ -7,10 +7,12 @@
 // backward-data give the reference's float sums term for term), and one block per weight for backward-filter, whose long
 // sum over batch and pixels is wavefront-reduced in double.
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
 #include "conv_f32_gemm.hpp"
+#include "depthwise_f32.hpp"
 
 namespace n2d2hip {
 
@@ -740,10 +742,45 @@ static DivF32 div_of(int d)
     return r;
 }
 
+// The strip kernels of depthwise layers (depthwise_f32.hpp): square kernels of 3 or 5 at one stride of 1 or 2, 32-bit offsets
+// (with room for a window past the end).  All forms that qualify are faster so: 128
+// channels, 3x3, 56 x 56, batch 32: backward-data 167.5 -> 19.4 us, backward-filter 407.8 -> 49.7.
+static bool depthwise_strips(const ConvF32& q)
+{
+    const size_t lim = ((size_t)1 << 31) - 4096;
+    return q.depthwise && q.dx == 1 && q.dy == 1 && q.kH == q.kW && (q.kH == 3 || q.kH == 5) && q.sx == q.sy && q.sx <= 2 && q.C <= 65535
+           && (size_t)q.B * q.C * (q.H + q.kH) * (q.W + q.kW + q.pl + 8) < lim && (size_t)q.B * q.C * (q.oH + q.kH) * (q.oW + q.pl + 8) < lim
+           && (size_t)q.pl + q.pt + q.pr + q.pb < 4096;
+}
+static int run_depthwise(const ConvF32& q, int pass, const float* a, const float* b, const float* bias, float beta, float* out, hipStream_t st)
+{
+    const int rows = pass == PASS_BWD_DATA ? q.H : q.oH, cols = pass == PASS_BWD_DATA ? q.W : q.oW, strips = ceil_div_i(cols, 4);
+    const DepthwiseF32 k = {q.C, q.H, q.W, q.oH, q.oW, q.pl, q.pt, q.B * rows * strips, strips, q.B * q.C * q.H * q.W, q.B * q.C * q.oH * q.oW,
+                            div_of(strips), div_of(rows)};
+    const dim3 grid(ceil_div_i(k.items, 256), q.C);
+    const auto run = [&](auto K_, auto S_) {
+        constexpr int K = decltype(K_)::value, S = decltype(S_)::value;
+        if (pass == PASS_FWD) hipLaunchKernelGGL((depthwise_f32_forward_kernel<K, S>), grid, dim3(256), 0, st, k, a, b, bias, beta, out);
+        else if (pass == PASS_BWD_FILTER)
+            hipLaunchKernelGGL((depthwise_f32_filter_kernel<K, S>), dim3(q.C, K), dim3(k.items >= 2048 ? 1024 : 256), 0, st, k, a, b, beta, out);
+        else if (S == 2 && (q.pl & 1)) hipLaunchKernelGGL((depthwise_f32_data_kernel<K, S, S == 2>), grid, dim3(256), 0, st, k, b, a, beta, out);
+        else hipLaunchKernelGGL((depthwise_f32_data_kernel<K, S, 0>), grid, dim3(256), 0, st, k, b, a, beta, out);
+    };
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I3 = std::integral_constant<int, 3>;
+    using I5 = std::integral_constant<int, 5>;
+    if (q.kH == 3) q.sx == 1 ? run(I3{}, I1{}) : run(I3{}, I2{});
+    else q.sx == 1 ? run(I5{}, I1{}) : run(I5{}, I2{});
+    N2D2HIP_HIP_CHECK(hipGetLastError());
+    return N2D2HIP_OK;
+}
+
 // The direct kernel of forward and backward-data: the walk with 32-bit offsets and one mask bit per tap row and column, or
 // (dilated, larger) one load after the other.
 static int run_direct(const ConvF32& q, int pass, const float* x, const float* w, const float* bias, float beta, float* out, hipStream_t st)
 {
+    if (depthwise_strips(q)) return run_depthwise(q, pass, x, w, bias, beta, out, st);
     const bool bwd = pass == PASS_BWD_DATA;
     const size_t lim = (size_t)1 << 31, total = (size_t)q.B * (bwd ? (size_t)q.C * q.H * q.W : (size_t)q.O * q.oH * q.oW);
     const size_t source = (size_t)q.B * (bwd ? (size_t)q.O * q.oH * q.oW : (size_t)q.C * q.H * q.W);
@@ -1172,6 +1209,7 @@ int n2d2hip_conv2d_f32_backward_filter(const n2d2hip_conv_desc* desc, int B, int
                         workspace_bytes, need);
         return run_pass(m, pass, x, diff_y, nullptr, 1, 1, beta, diff_w, (float*)workspace, workspace_bytes / sizeof(float), (hipStream_t)stream);
     }
+    if (depthwise_strips(q)) return run_depthwise(q, PASS_BWD_FILTER, x, diff_y, nullptr, beta, diff_w, (hipStream_t)stream);
     hipLaunchKernelGGL(conv_f32_backward_filter_kernel, dim3((unsigned)nw), dim3(TBLOCK), 0, (hipStream_t)stream, q, x, diff_y, beta, diff_w);
     N2D2HIP_HIP_CHECK(hipGetLastError());
     return N2D2HIP_OK;

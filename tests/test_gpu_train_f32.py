@@ -261,6 +261,44 @@ def test_conv_kernels_chosen_by_size(g, case, workspace):
         assert _rel(g.host(dw), want[2] + 1, mag[2] + 1) <= TOL
 
 
+# B, C, H, W, k, stride, pad: strips of four with every remainder, rows shorter than a strip or a window, windows past both
+# ends of the tensor, both parities of the padding at stride 2, blocks of 256 and of 1024 threads, outputs wider than the input
+DEPTHWISE = [(1, 1, 1, 1, 3, 1, 1), (2, 3, 2, 3, 3, 1, 1), (1, 1, 3, 3, 3, 1, 0), (3, 2, 5, 6, 3, 2, 0), (2, 5, 9, 7, 3, 2, 1), (1, 4, 6, 9, 3, 2, 2),
+             (2, 3, 7, 8, 5, 1, 2), (1, 2, 5, 5, 5, 1, 4), (3, 3, 11, 10, 5, 2, 1), (2, 2, 12, 13, 5, 2, 2), (40, 3, 31, 29, 3, 1, 1), (33, 2, 30, 31, 5, 2, 3)]
+
+
+@pytest.mark.parametrize("infinity", [False, True])
+@pytest.mark.parametrize("case", DEPTHWISE)
+def test_depthwise_strips(g, case, infinity):
+    B, Cn, H, W, k, s, p = case
+    print("depthwise conv f32", case, infinity, flush=True)
+    t, F = g.torch_, g.torch_.nn.functional
+    rng = np.random.default_rng(sum(case))
+    x, w = rng.normal(size=(B, Cn, H, W)).astype(np.float32), rng.normal(size=(Cn, 1, k, k)).astype(np.float32)
+    oH, oW = (H + 2 * p - k) // s + 1, (W + 2 * p - k) // s + 1
+    dy = rng.normal(size=(B, Cn, oH, oW)).astype(np.float32)
+    if infinity:                # at the end of a row: the window of the next row's first outputs reads it and must not use it
+        x[0, 0, H // 2, W - 1] = np.inf
+
+    def passes(x_, w_, dy_):
+        x64, w64 = (t.from_numpy(v).double().requires_grad_() for v in (x_, w_))
+        y = F.conv2d(x64, w64, stride=s, padding=p, groups=Cn)
+        y.backward(t.from_numpy(dy_).double())
+        return [v.detach().numpy() for v in (y, x64.grad, w64.grad)]
+    want, mag = passes(x, w, dy), passes(np.abs(x), np.abs(w), np.abs(dy))
+    d = g.desc(Cn, Cn, k, s, p, Cn)
+    x_, w_, dy_ = g.dev(x), g.dev(w), g.dev(dy)
+    y, dx, dw = (t.ones(v.shape, dtype=t.float32, device="cuda") for v in (dy, x, w))
+    g.check(g.lib.n2d2hip_conv2d_f32_forward(C.byref(d), B, H, W, x_.data_ptr(), w_.data_ptr(), None, 1.0, y.data_ptr(), None, 0, g.sp()))
+    g.check(g.lib.n2d2hip_conv2d_f32_backward_data(C.byref(d), B, H, W, w_.data_ptr(), dy_.data_ptr(), 1.0, dx.data_ptr(), None, 0, g.sp()))
+    g.check(g.lib.n2d2hip_conv2d_f32_backward_filter(C.byref(d), B, H, W, x_.data_ptr(), dy_.data_ptr(), 1.0, dw.data_ptr(), None, 0, g.sp()))
+    for got, ref, m in zip((y, dx, dw), want, mag):
+        got, finite = g.host(got), np.isfinite(ref)
+        np.testing.assert_array_equal(np.where(finite, 0, got), np.where(finite, 0, ref))
+        if finite.any():
+            assert _rel(got[finite], ref[finite] + 1, m[finite] + 1) <= TOL
+
+
 def test_dilated_forward(g):
     from oracle import oracle as orc
     rng = np.random.default_rng(3)
