@@ -440,6 +440,36 @@ def test_batchnorm_forward_backward(g, shape, with_workspace):
                                                1e-5, 0.1, 0, y.data_ptr(), None, 0, g.sp()) == g.capi.ERR_INVALID
 
 
+@pytest.mark.parametrize("shape", [(4, 3, 7, 9), (2, 2, 8, 8), (40, 2, 28, 28), (40, 3, 27, 25)])
+@pytest.mark.parametrize("kind", ["offset", "outlier", "constant", "nan"])
+def test_batchnorm_statistics_far_from_zero(g, shape, kind):
+    """One pass gives the variance about the mean as rounded to float: where the values are far from zero, where the first of a
+    channel (from which the pass counts) is far from the rest, and where they are all one value."""
+    B, Cn, H, W = shape
+    print("batchnorm statistics", shape, kind, flush=True)
+    rng = np.random.default_rng(B + W)
+    x = rng.normal(1000.0 if kind == "offset" else 0.5, 1e-2, size=shape).astype(np.float32)
+    if kind == "outlier":
+        x[0, :, 0, 0] = 3e5
+    if kind == "constant":
+        x[:] = np.float32(0.1)
+    if kind == "nan":
+        x[1, 0, 2, 3] = np.nan
+    z = lambda v=0.0: g.torch_.full((Cn,), v, dtype=g.torch_.float32, device="cuda")
+    smean, svar, mean, var, gamma, beta, x_ = z(), z(), z(), z(1.0), z(1.0), z(), g.dev(x)
+    y = g.torch_.empty(shape, dtype=g.torch_.float32, device="cuda")
+    ws = g.torch_.empty(int(g.lib.n2d2hip_batchnorm_f32_workspace_bytes(B, Cn, H, W)), dtype=g.torch_.uint8, device="cuda")
+    g.check(g.lib.n2d2hip_batchnorm_f32_forward(B, Cn, H, W, x_.data_ptr(), gamma.data_ptr(), beta.data_ptr(), mean.data_ptr(), var.data_ptr(),
+                                                smean.data_ptr(), svar.data_ptr(), 1e-5, 0.1, 0, y.data_ptr(), ws.data_ptr(), ws.numel(), g.sp()))
+    m = x.astype(np.float64).mean(axis=(0, 2, 3)).astype(np.float32)
+    # the mean may round to the float beside it; the variance then is that about the other float.  One rounding, and what
+    # cancels: n values times 2^-53
+    np.testing.assert_allclose(g.host(smean), m, rtol=2.0 ** -23)
+    got = g.host(smean).astype(np.float64)
+    v = ((x.astype(np.float64) - got[:, None, None]) ** 2).mean(axis=(0, 2, 3))
+    np.testing.assert_allclose(g.host(svar), v, rtol=2.0 ** -23 + 4 * B * H * W * 2.0 ** -53)
+
+
 @pytest.mark.parametrize("case", [(2, 3, 9, 8, 2, 2, 2, 2, 0, 0), (2, 3, 9, 8, 3, 3, 2, 2, 0, 0), (2, 3, 9, 8, 3, 3, 2, 2, 1, 1),
                                   (1, 2, 7, 10, 3, 2, 1, 2, 0, 0), (4, 16, 28, 28, 2, 2, 2, 2, 0, 0), (3, 5, 11, 11, 3, 3, 1, 1, 1, 1),
                                   (2, 2, 6, 6, 2, 2, 3, 3, 0, 0)])
