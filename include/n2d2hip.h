@@ -372,6 +372,10 @@ int n2d2hip_bottleneck_forward(n2d2hip_bottleneck_t bottleneck, const n2d2hip_te
  * the separate launches.  `in`: the 3x3 convolution's input, NHWC bytes that carry the padding as a border (halo >= 1);
  * `other`: the sum's other input; `out`: the sum's output; the last two with or without a border. */
 int n2d2hip_conv_chain_supported(n2d2hip_conv_t conv3x3, n2d2hip_conv_t expand);
+/* 1 where the one launch is expected to be faster than the two for `batch` images of in_h x in_w pixels (inputs of the 3x3
+ * convolution, without their border), else 0, also for a pair that cannot run so.  Planners ask this instead of restating
+ * the rule. */
+int n2d2hip_conv_chain_pays(n2d2hip_conv_t conv3x3, n2d2hip_conv_t expand, int batch, int in_h, int in_w);
 int n2d2hip_conv_chain_forward(n2d2hip_conv_t conv3x3, n2d2hip_conv_t expand, const n2d2hip_tensor* in, const n2d2hip_tensor* other,
                                const n2d2hip_tensor* out, n2d2hip_stream_t stream);
 

@@ -30,7 +30,7 @@ SYMBOLS = [
     "n2d2hip_launch_log_begin", "n2d2hip_launch_log_end", "n2d2hip_launch_log_entry", "n2d2hip_nhwc_cs", "n2d2hip_tensor_bytes", "n2d2hip_tensor_clear",
     "n2d2hip_convert", "n2d2hip_act_create", "n2d2hip_act_destroy", "n2d2hip_scaling_forward",
     "n2d2hip_conv_create", "n2d2hip_conv_destroy", "n2d2hip_conv_out_dims", "n2d2hip_conv_forward", "n2d2hip_conv_s2d_halo", "n2d2hip_conv_accepts_halo", "n2d2hip_conv_desc_reads_halo",
-    "n2d2hip_conv_fuse_sum", "n2d2hip_conv_forward_sum", "n2d2hip_conv_chain_supported", "n2d2hip_conv_chain_forward", "n2d2hip_bottleneck_create", "n2d2hip_bottleneck_destroy", "n2d2hip_bottleneck_pays", "n2d2hip_bottleneck_forward",
+    "n2d2hip_conv_fuse_sum", "n2d2hip_conv_forward_sum", "n2d2hip_conv_chain_supported", "n2d2hip_conv_chain_pays", "n2d2hip_conv_chain_forward", "n2d2hip_bottleneck_create", "n2d2hip_bottleneck_destroy", "n2d2hip_bottleneck_pays", "n2d2hip_bottleneck_forward",
     "n2d2hip_conv_accepts_maxpool", "n2d2hip_conv_forward_maxpool", 
     "n2d2hip_dw_pw_create", "n2d2hip_dw_pw_destroy", "n2d2hip_dw_pw_forward", "n2d2hip_dw_pw_pays",
     "n2d2hip_fc_create", "n2d2hip_fc_destroy", "n2d2hip_fc_forward", "n2d2hip_fc_chain_create", "n2d2hip_fc_chain_destroy", "n2d2hip_fc_chain_forward",
@@ -108,6 +108,7 @@ def load():
     lib.n2d2hip_concat_channels.argtypes = [I, P, P, P]
     lib.n2d2hip_conv_forward_sum.argtypes = [P, P, P, P, P]
     lib.n2d2hip_conv_chain_supported.argtypes = [P, P]
+    lib.n2d2hip_conv_chain_pays.argtypes = [P, P, C.c_int, C.c_int, C.c_int]
     lib.n2d2hip_conv_chain_forward.argtypes = [P, P, P, P, P, P]
     lib.n2d2hip_bottleneck_create.argtypes = [P, P, P, P, P]
     lib.n2d2hip_bottleneck_destroy.argtypes = [P]

@@ -1560,6 +1560,25 @@ int n2d2hip_conv_chain_supported(n2d2hip_conv_t conv3x3, n2d2hip_conv_t expand)
     return chain_ok(conv3x3, expand) ? 1 : 0;
 }
 
+// The one launch has 128-pixel tiles over all channels, so ceil(pixels / 128) blocks; the two launches also cut the channels
+// into tiles.  ResNet-50 (us for the whole net; the pairs of a size in two launches / in one):
+//  64 middle channels: one launch is never slower (batch 1 347 / 342, batch 24 550 / 528, batch 128 1226 / 1204).
+//  128: one launch loses while a good part of the compute units has no tile (98 tiles 454 / 467, 147 tiles 544 / 560 and
+//  550 / 541); from three quarters on it is level or ahead (196 tiles 616 / 611, 392 812 / 805, 980 1456 / 1426).
+//  256: a work-group of eight waves has a compute unit to itself; one launch pays where its tiles make one nearly full round
+//  (245 tiles 1426 / 1389) and else loses (8 tiles 347 / 448, 196 1205 / 1227, 392 2066 / 2123, 612 3307 / 3349).
+int n2d2hip_conv_chain_pays(n2d2hip_conv_t c3, n2d2hip_conv_t ce, int batch, int in_h, int in_w)
+{
+    if (!chain_ok(c3, ce) || batch <= 0 || in_h <= 0 || in_w <= 0)
+        return 0;
+    int OH, OW;
+    if (n2d2hip_conv_out_dims(&c3->desc, in_h, in_w, &OH, &OW) != N2D2HIP_OK)
+        return 0;
+    const long long tiles = ((long long)batch * OH * OW + 127) / 128;
+    const int cus = num_cus();
+    return (c3->desc.C == 64 || (c3->desc.C == 128 ? 4 * tiles >= 3 * cus : 8 * tiles >= 7 * cus && tiles <= cus)) ? 1 : 0;
+}
+
 int n2d2hip_conv_chain_forward(n2d2hip_conv_t c3, n2d2hip_conv_t ce, const n2d2hip_tensor* in, const n2d2hip_tensor* other,
                                const n2d2hip_tensor* out, n2d2hip_stream_t stream)
 {

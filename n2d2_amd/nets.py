@@ -410,7 +410,8 @@ class GpuNet:
         fc_chains: run two or three fully-connected cells, each the only reader of the one before, as one launch
         (n2d2hip_fc_chain_*) where the library takes them.
         chains: run a block's 3x3 convolution in the launch of the expanding 1x1 convolution + sum that alone reads it
-        (n2d2hip_conv_chain_*) where the library takes the pair: the 3x3 convolution's output stays on the chip."""
+        (n2d2hip_conv_chain_*) where the library takes the pair: the 3x3 convolution's output stays on the chip.  Where the
+        library expects two launches to be faster (n2d2hip_conv_chain_pays) the step makes two."""
         from . import capi, runtime as rt
         self.spec, self.B, self.rt, self.capi = spec, batch, rt, capi
         consumers = {}
@@ -619,7 +620,7 @@ class GpuNet:
         if fuse and halo and bottlenecks:
             self._plan_bottlenecks(consumers, by_name, ins_of)
         # 3x3 convolutions computed by the launch of the expansion and sum that alone read them (their tensors are never written)
-        self.chains = {}
+        self.chains, self.chains_apart = {}, set()
         if fuse and halo and chains:
             self._plan_chains(consumers, by_name, ins_of)
         # fully-connected cells in a row as one launch (the vectors between them are never written)
@@ -680,8 +681,14 @@ class GpuNet:
             x = ins_of[c3.name][0]
             if x.halo < 1 or ins_of[sum_name][0] is not self.tensors[c3.name]:
                 continue
+            if expand_cell.chain_pays(c3_cell, self.B, x.H, x.W):
+                step = lambda c, i, o, c3c=c3_cell: c.forward_chain(c3c, i[0], i[1], o)     # noqa: E731
+            else:                   # the same step in two launches, through the 3x3 convolution's own tensor
+                mid = ins_of[sum_name][0]
+                self.chains_apart.add(sum_name)
+                step = lambda c, i, o, c3c=c3_cell, m=mid: c.forward_sum(c3c.forward(i[0], m), i[1], o)     # noqa: E731
             ins_of[sum_name] = [x, ins_of[sum_name][1]]
-            self.steps[k] = (self.steps[k][0], expand_cell, (lambda c, i, o, c3c=c3_cell: c.forward_chain(c3c, i[0], i[1], o)))
+            self.steps[k] = (self.steps[k][0], expand_cell, step)
             self.folded.add(c3.name)
             self.chains[sum_name] = c3
 
@@ -859,8 +866,9 @@ class GpuNet:
             total += sum(m.w.size for m in self.bottleneck_layers[l.name])
         elif l.name in self.fused_sums:
             total += self.fused_sums[l.name][1].w.size
-        if l.name in self.chains:           # the 3x3 convolution's weights; its output never leaves the chip
-            total += self.chains[l.name].w.size
+        if l.name in self.chains:           # the 3x3 convolution's weights; its output never leaves the chip in one launch
+            c3 = self.chains[l.name]
+            total += c3.w.size + (2 * self.B * math.prod(c3.out_shape) if l.name in self.chains_apart else 0)
         if l.name in self.fc_chains:        # the earlier cells' weights; their outputs never leave the chip
             total += sum(m.w.size for m in self.fc_chains[l.name])
         if l.name in self.stem_pools:       # the convolution's weights; its output never leaves the chip

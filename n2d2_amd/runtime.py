@@ -281,6 +281,10 @@ class Conv:
         """Can `conv3x3`, whose output only this 1x1 expansion (with its folded sum) reads, run in this cell's launch?"""
         return bool(lib.n2d2hip_conv_chain_supported(conv3x3.handle, self.handle))
 
+    def chain_pays(self, conv3x3, batch, H, W):
+        """Is that one launch expected to be faster than the two for `batch` inputs of H x W pixels?"""
+        return bool(lib.n2d2hip_conv_chain_pays(conv3x3.handle, self.handle, batch, H, W))
+
     def forward_chain(self, conv3x3, x, other, out):
         """out = sum(self(conv3x3(x)), other) in one launch; x carries conv3x3's padding as a border."""
         check(lib.n2d2hip_conv_chain_forward(conv3x3.handle, self.handle, x.ref, other.ref, out.ref, stream_ptr()))

@@ -111,3 +111,4 @@ def test_planning_questions_answered_from_descriptors_alone():
     assert wh(pool(capi.POOL_MAX, 3, 2, 3), 28, 28, 16) == 0                # padding as large as the window
     assert lib.n2d2hip_pool_writes_halo(None, 28, 28, 16) == 0
     assert lib.n2d2hip_bottleneck_pays(None, 128, 56, 56) == 0
+    assert lib.n2d2hip_conv_chain_pays(None, None, 128, 56, 56) == 0

@@ -1100,6 +1100,24 @@ def test_conv3x3_expansion_and_sum_in_one_launch_bit_exact(rt):
     assert not c2.chain_supported(cb)
 
 
+@pytest.mark.parametrize("cm,stride,batch,size,pays", [
+    (64, 1, 1, 1, True), (128, 1, 1, 28, False), (128, 1, 95, 16, False), (128, 1, 96, 16, True), (128, 2, 96, 31, True), (128, 1, 128, 28, True),
+    (256, 1, 1, 14, False), (256, 1, 128, 14, False), (256, 1, 112, 16, True), (256, 1, 128, 16, True), (256, 1, 129, 16, False), (128, 1, 0, 28, False)])
+def test_where_the_chain_launch_pays(rt, cm, stride, batch, size, pays):
+    """n2d2hip_conv_chain_pays on 256 compute units: with 64 middle channels always, with 128 from 192 tiles of 128 pixels, with
+    256 for 224 to 256 tiles."""
+    from n2d2_amd import capi
+    from oracle.cells import ActSpec
+    rng = np.random.default_rng(cm)
+    act = lambda O, kind: rt.Act(O, **ActSpec(kind, "SingleShift", rng.integers(8, 12, size=O), nb_bits=8, unsigned_out=kind == "Rectifier").kwargs())
+    w = lambda *shape: rng.integers(-20, 21, size=shape)
+    conv = rt.Conv(w(cm, cm, 3, 3), None, act(cm, "Rectifier"), capi.U8B, stride=(stride, stride), pad=(1, 1, 1, 1))
+    expand = rt.Conv(w(4 * cm, cm, 1, 1), None, act(4 * cm, "Linear"), capi.U8B)
+    ew = rt.ElemWiseSum(2, 4 * cm, rt.Act(4 * cm, **ActSpec("Rectifier", "SingleShift", rng.integers(0, 3, size=4 * cm), nb_bits=8, unsigned_out=True).kwargs()))
+    assert expand.fuse_sum(ew, 0, capi.U8B) and expand.chain_supported(conv)
+    assert expand.chain_pays(conv, batch, size, size) == pays
+
+
 def conv_spec_for(O, rng):
     from oracle.cells import ActSpec
     return ActSpec("Linear", "DoubleShift", np.stack([rng.integers(0, 3, size=O), rng.integers(8, 12, size=O)], 1), nb_bits=8, unsigned_out=False)
