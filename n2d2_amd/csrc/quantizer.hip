@@ -6,6 +6,7 @@
 // result does not depend on scheduling.  Sums are carried in double.
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 #include "epilogue.hpp"
@@ -31,27 +32,54 @@ __device__ __forceinline__ float wave_max(float v)
 }
 __device__ __forceinline__ double block_sum(double v)
 {
-    __shared__ double red[QBLOCK / 64];
+    __shared__ double red[16];
     v = wave_sum(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     double t = 0.0;
-#pragma unroll
-    for (int i = 0; i < QBLOCK / 64; ++i) t += red[i];
+    for (int i = 0; i < (int)(blockDim.x >> 6); ++i) t += red[i];
     return t;
 }
 __device__ __forceinline__ float block_max(float v)
 {
-    __shared__ float redm[QBLOCK / 64];
+    __shared__ float redm[16];
     v = wave_max(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) redm[threadIdx.x >> 6] = v;
     __syncthreads();
     float t = redm[0];
-#pragma unroll
-    for (int i = 1; i < QBLOCK / 64; ++i) t = fmaxf(t, redm[i]);
+    for (int i = 1; i < (int)(blockDim.x >> 6); ++i) t = fmaxf(t, redm[i]);
     return t;
+}
+
+// A grid's walk over n values: in quads of 16 bytes where the tensors' addresses allow it, the rest one by one.  Memory bounds
+// the passes that use it; at 4 bytes a load their at most 1024 blocks had too little in flight (SAT backward of 12.8 M values:
+// 40.3 us, now 30.2).  f(number of values as a type, index of the first); a value is read before its place is written, so
+// input and output may be one tensor.
+template <class F>
+__device__ __forceinline__ void for_quads(size_t n, int quads, F f)
+{
+    const size_t step = (size_t)gridDim.x * QBLOCK, first = (size_t)blockIdx.x * QBLOCK + threadIdx.x, n4 = quads ? n / 4 : 0;
+#pragma unroll 2
+    for (size_t i = first; i < n4; i += step) f(std::integral_constant<int, 4>{}, i * 4);
+    for (size_t i = n4 * 4 + first; i < n; i += step) f(std::integral_constant<int, 1>{}, i);
+}
+template <int N>
+__device__ __forceinline__ void quad_load(float* dst, const float* p, size_t i)
+{
+    if (N == 4) {
+        const float4 v = *(const float4*)(p + i);
+        dst[0] = v.x; dst[1] = v.y; dst[2] = v.z; dst[3] = v.w;
+    } else {
+        dst[0] = p[i];
+    }
+}
+template <int N>
+__device__ __forceinline__ void quad_store(float* p, size_t i, const float* v)
+{
+    if (N == 4) *(float4*)(p + i) = make_float4(v[0], v[1], v[2], v[3]);
+    else p[i] = v[0];
 }
 
 // ------------------------------------------------------------ SAT weights
@@ -72,50 +100,99 @@ __global__ __launch_bounds__(QBLOCK) void sat_absmax_final(const float* __restri
     if (threadIdx.x == 0) { stats[0] = m; stats[1] = 1.0f; }
 }
 
-// ref: src/Quantizer/QAT/Kernel/SATQuantizer_Frame_Kernels.cpp:66-238
-__global__ __launch_bounds__(QBLOCK) void sat_weight_quantize(const float* __restrict__ w, float* __restrict__ wq, size_t n,
-                                                              float range, int mode, const float* __restrict__ stats)
-{
-    const float tmax = stats[0];
-    if (mode == N2D2HIP_SAT_SYMRANGE || mode == N2D2HIP_SAT_ASYMRANGE || mode == N2D2HIP_SAT_NONE_ASYM)
-        range = floorf(range / 2.0f);
-    const float inv_range = 1.0f / range;
-    const float full_a = 1.0f + 0.9998f / range, full_b = 0.4999f / range;
-    const float asym_a = 1.0f + 1.0f / (2.0f * range), asym_b = 1.0f / (2.0f * range);
-    for (size_t i = (size_t)blockIdx.x * QBLOCK + threadIdx.x; i < n; i += (size_t)gridDim.x * QBLOCK) {
-        const float t = tanhf(w[i]);
+// The weights' quantization levels from tanh(w), ref: src/Quantizer/QAT/Kernel/SATQuantizer_Frame_Kernels.cpp:66-238
+struct SatLevels {
+    int mode;
+    float range, tmax, inv_range, full_a, full_b, asym_a, asym_b;
+    __device__ SatLevels(float r, int m, float t) : mode(m), range(r), tmax(t)
+    {
+        if (mode == N2D2HIP_SAT_SYMRANGE || mode == N2D2HIP_SAT_ASYMRANGE || mode == N2D2HIP_SAT_NONE_ASYM)
+            range = floorf(range / 2.0f);
+        inv_range = 1.0f / range;
+        full_a = 1.0f + 0.9998f / range;
+        full_b = 0.4999f / range;
+        asym_a = 1.0f + 1.0f / (2.0f * range);
+        asym_b = 1.0f / (2.0f * range);
+    }
+    __device__ float operator()(float t) const
+    {
         float q;
         switch (mode) {
         case N2D2HIP_SAT_NONE:
-            q = t / tmax;
-            break;
+            return t / tmax;
         case N2D2HIP_SAT_DEFAULT:
             q = __fmul_rn(0.5f, __fadd_rn(t / tmax, 1.0f));
             q = __fmul_rn(inv_range, rintf(__fmul_rn(q, range)));
-            q = __fsub_rn(__fmul_rn(q, 2.0f), 1.0f);
-            break;
+            return __fsub_rn(__fmul_rn(q, 2.0f), 1.0f);
         case N2D2HIP_SAT_FULLRANGE:
             q = __fmul_rn(0.5f, __fadd_rn(t / tmax, 1.0f));
             q = __fsub_rn(__fmul_rn(full_a, q), full_b);
             q = __fmul_rn(inv_range, rintf(__fmul_rn(q, range)));
-            q = __fsub_rn(__fmul_rn(q, 2.0f), 1.0f);
-            break;
+            return __fsub_rn(__fmul_rn(q, 2.0f), 1.0f);
         case N2D2HIP_SAT_SYMRANGE:
             q = t / tmax;
-            q = __fmul_rn(inv_range, rintf(__fmul_rn(q, range)));
-            break;
+            return __fmul_rn(inv_range, rintf(__fmul_rn(q, range)));
         case N2D2HIP_SAT_ASYMRANGE:
             q = t / tmax;
             q = __fsub_rn(__fmul_rn(asym_a, q), asym_b);
-            q = __fmul_rn(inv_range, rintf(__fmul_rn(q, range)));
-            break;
+            return __fmul_rn(inv_range, rintf(__fmul_rn(q, range)));
         default:
             q = t / tmax;
-            q = __fsub_rn(__fmul_rn(asym_a, q), asym_b);
-            break;
+            return __fsub_rn(__fmul_rn(asym_a, q), asym_b);
         }
-        wq[i] = q;
     }
+};
+__global__ __launch_bounds__(QBLOCK) void sat_weight_quantize(const float* __restrict__ w, float* __restrict__ wq, size_t n,
+                                                              float range, int mode, const float* __restrict__ stats)
+{
+    const SatLevels level(range, mode, stats[0]);
+    for (size_t i = (size_t)blockIdx.x * QBLOCK + threadIdx.x; i < n; i += (size_t)gridDim.x * QBLOCK)
+        wq[i] = level(tanhf(w[i]));
+}
+
+// Small tensors: the whole quantizer in one launch of one block, the weights in its registers.  One kernel per pass is bound
+// by the launches there (3 of 2 to 4 us, 8 with the scaling); one compute unit has done up to 1024 weights
+// in 3.7 us, 2400 in 4.2 and 10080, scaling included, in 11.5.  (Instances by the weights per thread: skipping unused ones
+// inside one instance made the compiler spill.)
+constexpr int SAT_SMALL = 16;                    // weights per thread at most; K: of this launch
+template <int K>
+__global__ __launch_bounds__(1024) void sat_weight_small_kernel(const float* __restrict__ w, float* __restrict__ wq, int n, float range, int mode,
+                                                                int apply_scaling, unsigned factor, float* __restrict__ stats)
+{
+    float v[K];
+    float m = 0.0f;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int i = k * 1024 + threadIdx.x;
+        v[k] = i < n ? tanhf(w[i]) : 0.0f;
+        m = fmaxf(m, fabsf(v[k]));
+    }
+    m = block_max(m);
+    const SatLevels level(range, mode, m);
+    double sum = 0.0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        v[k] = level(v[k]);
+        if (k * 1024 + (int)threadIdx.x < n) sum += (double)v[k];
+    }
+    float scaling = 1.0f;
+    if (apply_scaling) {                         // (the formulas of mean_final, sqdev_partial and sat_scaling_final)
+        const float mean = (float)block_sum(sum) / (float)n;
+        double squares = 0.0;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+                const float d = __fsub_rn(v[k], mean);
+            if (k * 1024 + (int)threadIdx.x < n) squares += (double)__fmul_rn(d, d);
+        }
+        const float var = (float)block_sum(squares) / ((float)n - 1.0f);
+        scaling = sqrtf(var * (float)factor);
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int i = k * 1024 + threadIdx.x;
+        if (i < n) wq[i] = apply_scaling ? v[k] / scaling : v[k];
+    }
+    if (threadIdx.x == 0) { stats[0] = m; stats[1] = scaling; }
 }
 
 // SAT scaling, ref: SATQuantizer_Frame_Kernels.cpp:244-262: mean, unbiased variance about that
@@ -198,40 +275,61 @@ __global__ __launch_bounds__(QBLOCK) void sat_act_forward_kernel(float* __restri
     }
 }
 
-// ref: SATQuantizer_Frame_Kernels.cpp:410-448; the alpha-gradient terms are summed instead of stored
-__global__ __launch_bounds__(QBLOCK) void sat_act_backward_kernel(const float* dy, const float* __restrict__ fp,
-                                                                  float* dx, size_t n, float range,
-                                                                  const float* __restrict__ alpha, double* __restrict__ partial)
-{
-    const float a = fabsf(alpha[0]);
-    double s = 0.0;
-    for (size_t i = (size_t)blockIdx.x * QBLOCK + threadIdx.x; i < n; i += (size_t)gridDim.x * QBLOCK) {
-        const float x = fp[i];
-        const float g = dy[i];
-        const float xc = (x < 0.0f) ? 0.0f : (x < a) ? x : a;
-        const float q = xc / a;
-        const float qd = round_half_away(__fmul_rn(range, q)) / range;
-        const float dqa = (x >= a) ? 1.0f : __fsub_rn(qd, q);
-        s += (double)__fmul_rn(dqa, g);
-        const float dact = (x <= 0.0f) ? 0.0f : (x > a) ? 0.0f : 1.0f;
-        dx[i] = __fmul_rn(dact, g);
-    }
-    s = block_sum(s);
-    if (threadIdx.x == 0) partial[blockIdx.x] = s;
-}
 // result[0] = (sum + beta * result[0]) * scale
-__global__ __launch_bounds__(QBLOCK) void accumulate_final(const double* __restrict__ partial, int count, float beta, float scale,
-                                                           float* __restrict__ result)
-{
-    double s = 0.0;
-    for (int i = threadIdx.x; i < count; i += QBLOCK) s += partial[i];
-    s = block_sum(s);
-    if (threadIdx.x == 0) {
+struct Accumulate {
+    float beta, scale;
+    float* result;
+    __device__ void operator()(double s) const
+    {
         float acc = (float)s;
         if (beta != 0.0f)
             acc = __fadd_rn(acc, __fmul_rn(beta, result[0]));
         result[0] = __fmul_rn(acc, scale);
     }
+};
+// The end of a reducing pass: a single block (up to ONE_BLOCK values: a second launch would take longer than the rest of its
+// loop) accumulates by itself, several leave their sums to accumulate_final
+constexpr size_t ONE_BLOCK = 4096;
+__device__ __forceinline__ void end_of_pass(double s, double* __restrict__ partial, const Accumulate& acc)
+{
+    s = block_sum(s);
+    if (threadIdx.x) return;
+    if (gridDim.x == 1) acc(s);
+    else partial[blockIdx.x] = s;
+}
+
+// ref: SATQuantizer_Frame_Kernels.cpp:410-448; the alpha-gradient terms are summed instead of stored
+__global__ __launch_bounds__(QBLOCK) void sat_act_backward_kernel(const float* dy, const float* __restrict__ fp,
+                                                                  float* dx, size_t n, float range,
+                                                                  const float* __restrict__ alpha, double* __restrict__ partial, int quads, Accumulate accumulate)
+{
+    const float a = fabsf(alpha[0]);
+    double s = 0.0;
+    for_quads(n, quads, [&](auto k, size_t i) {
+        constexpr int N = decltype(k)::value;
+        float x[N], g[N], d[N];
+        quad_load<N>(x, fp, i);
+        quad_load<N>(g, dy, i);
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const float xc = (x[j] < 0.0f) ? 0.0f : (x[j] < a) ? x[j] : a;
+            const float q = xc / a;
+            const float qd = round_half_away(__fmul_rn(range, q)) / range;
+            const float dqa = (x[j] >= a) ? 1.0f : __fsub_rn(qd, q);
+            s += (double)__fmul_rn(dqa, g[j]);
+            const float dact = (x[j] <= 0.0f) ? 0.0f : (x[j] > a) ? 0.0f : 1.0f;
+            d[j] = __fmul_rn(dact, g[j]);
+        }
+        quad_store<N>(dx, i, d);
+    });
+    end_of_pass(s, partial, accumulate);
+}
+__global__ __launch_bounds__(QBLOCK) void accumulate_final(const double* __restrict__ partial, int count, Accumulate acc)
+{
+    double s = 0.0;
+    for (int i = threadIdx.x; i < count; i += QBLOCK) s += partial[i];
+    s = block_sum(s);
+    if (threadIdx.x == 0) acc(s);
 }
 
 // -------------------------------------------------------------------- LSQ
@@ -250,20 +348,26 @@ __global__ __launch_bounds__(QBLOCK) void lsq_forward_kernel(const float* __rest
 // ref: LSQQuantizerCell_Frame.cpp:234-303, LSQQuantizerActivation_Frame.cpp:193-262
 __global__ __launch_bounds__(QBLOCK) void lsq_backward_kernel(const float* dq, const float* __restrict__ fp,
                                                               float* dfp, size_t n, const float* __restrict__ step,
-                                                              int lo, int hi, double* __restrict__ partial)
+                                                              int lo, int hi, double* __restrict__ partial, int quads, Accumulate accumulate)
 {
     const float s = step[0];
     double acc = 0.0;
-    for (size_t i = (size_t)blockIdx.x * QBLOCK + threadIdx.x; i < n; i += (size_t)gridDim.x * QBLOCK) {
-        const float q = fp[i] / s;
-        const float g = dq[i];
-        const bool below = q <= (float)lo, above = q >= (float)hi;
-        dfp[i] = __fmul_rn(g, (below || above) ? 0.0f : 1.0f);
-        const float term = below ? (float)lo : above ? (float)hi : __fsub_rn(round_half_away(q), q);
-        acc += (double)__fmul_rn(term, g);
-    }
-    acc = block_sum(acc);
-    if (threadIdx.x == 0) partial[blockIdx.x] = acc;
+    for_quads(n, quads, [&](auto k, size_t i) {
+        constexpr int N = decltype(k)::value;
+        float x[N], g[N], d[N];
+        quad_load<N>(x, fp, i);
+        quad_load<N>(g, dq, i);
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const float q = x[j] / s;
+            const bool below = q <= (float)lo, above = q >= (float)hi;
+            d[j] = __fmul_rn(g[j], (below || above) ? 0.0f : 1.0f);
+            const float term = below ? (float)lo : above ? (float)hi : __fsub_rn(round_half_away(q), q);
+            acc += (double)__fmul_rn(term, g[j]);
+        }
+        quad_store<N>(dfp, i, d);
+    });
+    end_of_pass(acc, partial, accumulate);
 }
 
 } // namespace n2d2hip
@@ -276,6 +380,7 @@ int blocks_for(size_t n)
     size_t b = (n + QBLOCK - 1) / QBLOCK;
     return (int)std::max<size_t>(1, std::min<size_t>(b, PARTIALS));
 }
+int quads_of(const float* a, const float* b, const float* c) { return (((size_t)a | (size_t)b | (size_t)c) & 15) == 0; }
 unsigned ew_grid(size_t n)
 {
     size_t b = (n + QBLOCK - 1) / QBLOCK;
@@ -324,6 +429,12 @@ static int sat_weight_forward_impl(const char* who, const float* w, float* wq, s
     N2D2HIP_REQUIRE(mode >= N2D2HIP_SAT_NONE && mode <= N2D2HIP_SAT_NONE_ASYM, N2D2HIP_ERR_INVALID, "%s: bad mode %d", who, mode);
     N2D2HIP_REQUIRE(range >= 1.0f, N2D2HIP_ERR_INVALID, "%s: range %g", who, (double)range);
     N2D2HIP_REQUIRE(!apply_scaling || n > 1, N2D2HIP_ERR_INVALID, "%s: SAT scaling needs more than one weight", who);
+    if (n <= (size_t)SAT_SMALL * 1024) {
+        const auto kernel = n <= 1024 ? sat_weight_small_kernel<1> : n <= 4 * 1024 ? sat_weight_small_kernel<4> : sat_weight_small_kernel<SAT_SMALL>;
+        hipLaunchKernelGGL(kernel, dim3(1), dim3(1024), 0, st, w, wq, (int)n, range, mode, apply_scaling, outputs_size, stats);
+        N2D2HIP_HIP_CHECK(hipGetLastError());
+        return N2D2HIP_OK;
+    }
     const int nb = blocks_for(n);
     double* partial = (double*)workspace;
     float* mean = (float*)((char*)workspace + (size_t)PARTIALS * sizeof(double));
@@ -401,10 +512,12 @@ int n2d2hip_sat_act_backward(const float* diff_in, const float* fp_x, float* dif
     N2D2HIP_REQUIRE(n > 0, N2D2HIP_ERR_INVALID, "sat_act_backward: empty tensor");
     N2D2HIP_REQUIRE(workspace_bytes >= n2d2hip_quantizer_workspace_bytes(n), N2D2HIP_ERR_WORKSPACE, "sat_act_backward: workspace of %zu bytes needed",
                     n2d2hip_quantizer_workspace_bytes(n));
-    const int nb = blocks_for(n);
+    const int nb = n <= ONE_BLOCK ? 1 : blocks_for(n);
+    const Accumulate acc = {beta, 1.0f, diff_alpha};
     double* partial = (double*)workspace;
-    hipLaunchKernelGGL(sat_act_backward_kernel, dim3(nb), dim3(QBLOCK), 0, st, diff_in, fp_x, diff_out, n, range, alpha, partial);
-    hipLaunchKernelGGL(accumulate_final, dim3(1), dim3(QBLOCK), 0, st, (const double*)partial, nb, beta, 1.0f, diff_alpha);
+    hipLaunchKernelGGL(sat_act_backward_kernel, dim3(nb), dim3(QBLOCK), 0, st, diff_in, fp_x, diff_out, n, range, alpha, partial,
+                       quads_of(diff_in, fp_x, diff_out), acc);
+    if (nb > 1) hipLaunchKernelGGL(accumulate_final, dim3(1), dim3(QBLOCK), 0, st, (const double*)partial, nb, acc);
     N2D2HIP_HIP_CHECK(hipGetLastError());
     return N2D2HIP_OK;
 }
@@ -426,10 +539,12 @@ int n2d2hip_lsq_backward(const float* diff_q, const float* fp_x, float* diff_fp,
     N2D2HIP_REQUIRE(n > 0 && lo < hi, N2D2HIP_ERR_INVALID, "lsq_backward: empty tensor or empty range [%d,%d]", lo, hi);
     N2D2HIP_REQUIRE(workspace_bytes >= n2d2hip_quantizer_workspace_bytes(n), N2D2HIP_ERR_WORKSPACE, "lsq_backward: workspace of %zu bytes needed",
                     n2d2hip_quantizer_workspace_bytes(n));
-    const int nb = blocks_for(n);
+    const int nb = n <= ONE_BLOCK ? 1 : blocks_for(n);
+    const Accumulate acc = {beta, grad_scale, diff_step};
     double* partial = (double*)workspace;
-    hipLaunchKernelGGL(lsq_backward_kernel, dim3(nb), dim3(QBLOCK), 0, st, diff_q, fp_x, diff_fp, n, step, lo, hi, partial);
-    hipLaunchKernelGGL(accumulate_final, dim3(1), dim3(QBLOCK), 0, st, (const double*)partial, nb, beta, grad_scale, diff_step);
+    hipLaunchKernelGGL(lsq_backward_kernel, dim3(nb), dim3(QBLOCK), 0, st, diff_q, fp_x, diff_fp, n, step, lo, hi, partial,
+                       quads_of(diff_q, fp_x, diff_fp), acc);
+    if (nb > 1) hipLaunchKernelGGL(accumulate_final, dim3(1), dim3(QBLOCK), 0, st, (const double*)partial, nb, acc);
     N2D2HIP_HIP_CHECK(hipGetLastError());
     return N2D2HIP_OK;
 }

@@ -157,3 +157,44 @@ def test_lsq_forward_backward(q, lo, hi):
     q.check(q.lib.n2d2hip_lsq_backward(dg.data_ptr(), dx.data_ptr(), ddfp.data_ptr(), n, dstep.data_ptr(), lo, hi, float(grad_scale), 0.0,
                                        dds2.data_ptr(), ws.data_ptr(), ws.numel(), q.sp()))
     assert abs(q.host(dds2)[0] - want_sum * grad_scale) <= TOL * summed * grad_scale
+
+
+@pytest.mark.parametrize("n", [2, 1023, 1024, 1025, 10080, 16384, 16385])
+@pytest.mark.parametrize("mode", ["default", "none"])
+def test_sat_weights_around_the_one_launch_size(q, n, mode):
+    """Up to 16 weights for each of 1024 threads run in one launch: both sides of that and of a thread's share, with scaling."""
+    from oracle import oracle as orc
+    w = np.random.default_rng(n).normal(0, 0.05, size=n).astype(np.float32)
+    want, tmax, scal = orc.sat_weight_forward(w.astype(np.float64), 15.0, mode, apply_scaling=True, outputs_size=7)
+    dw_, dwq_, dstats, ws = q.dev(w), q.empty(n), q.empty(2), q.ws(n)
+    q.check(q.lib.n2d2hip_sat_weight_forward(dw_.data_ptr(), dwq_.data_ptr(), n, 15.0, MODES[mode], 1, 7, dstats.data_ptr(), ws.data_ptr(), ws.numel(),
+                                             q.sp()))
+    got, stats = q.host(dwq_), q.host(dstats)
+    assert abs(stats[0] - tmax) <= TOL * tmax
+    moved = ~_close(got * stats[1], want * scal, scale=1.0)
+    # a weight on a rounding edge moves by a level, 2 / 15, and the variance (of order 0.05) by up to 2 * 2 / 15 / n
+    assert moved.sum() <= 2 and np.all(np.abs(got[moved] * stats[1] - want[moved] * scal) <= 2.0 / 15.0 + 1e-4)
+    assert abs(stats[1] - scal) <= (TOL + 3.0 * moved.sum() / n) * scal
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("n", [1, 3, 4, 1027, 4096, 4097, 9002])
+def test_quantizer_backward_sizes_and_alignments(q, n, shift):
+    """Quads and what is left of them, one block and several, tensors that start beside a 16-byte boundary, in place."""
+    from oracle import oracle as orc
+    rng = np.random.default_rng(n)
+    x, g = rng.normal(1.0, 2.0, size=n).astype(np.float32), rng.normal(size=n).astype(np.float32)
+    at = lambda a: q.dev(np.concatenate([np.zeros(shift, dtype=np.float32), a]))[shift:]
+    dx_, ws = at(x), q.ws(n)
+    want_dx, want_da, terms = orc.sat_act_backward(g.astype(np.float64), x.astype(np.float64), 15.0, 1.5, beta=1.0, prev_diff_alpha=3.0)
+    dg, dda, dalpha, dstep = at(g), q.dev([3.0]), q.dev([1.5]), q.dev([0.25])
+    q.check(q.lib.n2d2hip_sat_act_backward(dg.data_ptr(), dx_.data_ptr(), dg.data_ptr(), n, 15.0, dalpha.data_ptr(), 1.0, dda.data_ptr(),
+                                           ws.data_ptr(), ws.numel(), q.sp()))
+    assert np.array_equal(q.host(dg), want_dx.astype(np.float32))
+    assert abs(q.host(dda)[0] - want_da) <= TOL * (np.abs(terms).sum() + 3.0)
+    want_dfp, want_sum = orc.lsq_backward(g.astype(np.float64), x.astype(np.float64), 0.25, -8, 7)
+    dg, dds = at(g), q.dev([0.5])
+    q.check(q.lib.n2d2hip_lsq_backward(dg.data_ptr(), dx_.data_ptr(), dg.data_ptr(), n, dstep.data_ptr(), -8, 7, 0.5, 1.0, dds.data_ptr(),
+                                       ws.data_ptr(), ws.numel(), q.sp()))
+    assert np.array_equal(q.host(dg), want_dfp.astype(np.float32))
+    assert abs(q.host(dds)[0] - (want_sum + 0.5) * 0.5) <= TOL * (8 * np.abs(g).sum() + 1.0)
