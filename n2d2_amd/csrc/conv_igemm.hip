@@ -1152,9 +1152,13 @@ static int conv_forward_impl(n2d2hip_conv_t c, const n2d2hip_tensor* in, const n
                                                                                             : tiles128 < (3 * num_cus()) / 2);
         // 64-channel layers whose K advances in 64-byte steps take 256-pixel tiles: twice the MFMAs per ring stage
         const bool wide64 = !w4 && !bn128 && !other && d.C % 128 != 0 && Mll >= 256ll * 4 * num_cus();
-        // A handful of tiles (the classifier's FC): 64 x 64 tiles, four times as many blocks share the long K
-        const bool tiny = !w4 && small_m && !other && ((Mll + 63) / 64) * a.ntiles_n * 8 < num_cus();
-        if (tiny) a.ntiles_n = (round_up(d.O, 16) + 63) / 64;
+        // Fewer 64 x 128 tiles than compute units: 64 x 64 tiles, twice as many blocks share the layer (a folded sum is written
+        // for two channel tiles a wave and keeps its 128 channels).  Whole nets, us, with the line at an eighth / a half / one /
+        // two times the compute units: ResNet-50 batch 1 343 / 339 / 338 / 338, 8 388 / 363 / 364 / 363, 32 596 / 582 / 577 /
+        // 578, 64 798 / - / 789 / 794; MobileNet batch 4 134 / 124 / 124 / 124; ResNet-18 W4A4 (before: never) batch 1 215 / - /
+        // 196 / 196, 32 276 / - / 265 / 269.
+        const bool tiny = small_m && !other && ((Mll + 63) / 64) * a.ntiles_n < num_cus();
+        if (tiny) q.c.ntiles_n = a.ntiles_n = (round_up(d.O, 16) + 63) / 64;
         const int BMp = small_m ? 64 : wide64 ? 256 : 128;
         q.mtiles = (int)((Mll + BMp - 1) / BMp);
         const int per_xcd = std::max(1, std::min((q.mtiles + 7) / 8, 2 * num_cus() / (8 * a.ntiles_n)));
@@ -1171,7 +1175,7 @@ static int conv_forward_impl(n2d2hip_conv_t c, const n2d2hip_tensor* in, const n
         if (w4 && !other) {
             // 4-bit weights, packed in memory and in LDS
             q.c.w = c->d_w4img;
-            return conv_pipe_w4_launch(q, small_m ? 2 : bn128 ? 1 : 0, all_valid, hi16, grid, stream);
+            return conv_pipe_w4_launch(q, tiny ? 3 : small_m ? 2 : bn128 ? 1 : 0, all_valid, hi16, grid, stream);
         }
         if (other) {
             const int cp = c->sum->act->cpad;
@@ -1209,7 +1213,6 @@ static int conv_forward_impl(n2d2hip_conv_t c, const n2d2hip_tensor* in, const n
         } else if (wide64) {
             launch_pipe<4, 64, 2, 2, 4, 3>(q, all_valid, hi16, grid, stream);
         } else if (tiny) {
-            q.c.ntiles_n = a.ntiles_n;
             launch_pipe<4, 128, 1, 1, 2, 3>(q, all_valid, hi16, grid, stream);
         } else if (small_m) {
             launch_pipe<4, 128, 2, 1, 2, 3>(q, all_valid, hi16, grid, stream);

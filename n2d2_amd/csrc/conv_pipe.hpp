@@ -896,7 +896,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     asm volatile("s_waitcnt vmcnt(0)\n\ts_waitcnt lgkmcnt(0)" ::: "memory");
 }
 
-// 4-bit weights (conv_pipe_w4.hip).  tile: 0 = 128 pixels x 64 channels, 1 = 128 x 128, 2 = 64 x 128; `a.c.w` is the image
+// 4-bit weights (conv_pipe_w4.hip).  tile: 0 = 128 pixels x 64 channels, 1 = 128 x 128, 2 = 64 x 128, 3 = 64 x 64 (no
+// folded sum); `a.c.w` is the image
 // conv_pipe_w4_image() makes; hi16 selects the scaled-up tables.
 size_t conv_pipe_w4_image_bytes(int rows, int ktot);
 void conv_pipe_w4_image(const signed char* w, int rows, int ktot, signed char* image);

@@ -43,7 +43,10 @@ template <int BK, int S, int NI, int NJ, int WGM, int V>
 void launch_valid(const ConvPipeArgs& a, bool hi16, int grid, hipStream_t stream)
 {
     constexpr int NW = 4;
-    if (a.res) {
+    if constexpr (NI == 1) {                     // (a folded sum is written for two channel tiles a wave)
+        if (hi16) N2D2HIP_LAUNCH_T(conv_pipe_kernel, (NW, BK, NI, NJ, WGM, EPI_I24, S, V, false, true, true), dim3(grid), dim3(NW * 64), 0, stream, a);
+        else N2D2HIP_LAUNCH_T(conv_pipe_kernel, (NW, BK, NI, NJ, WGM, EPI_I24, S, V, false, false, true), dim3(grid), dim3(NW * 64), 0, stream, a);
+    } else if (a.res) {
         // residual sum in the epilogue; 16-bit pairs when the host has shown that they hold every intermediate
         if (a.sum16) N2D2HIP_LAUNCH_T(conv_pipe_kernel, (NW, BK, NI, NJ, WGM, EPI_I24, S, V, true, true, true), dim3(grid), dim3(NW * 64), 0, stream, a);
         else N2D2HIP_LAUNCH_T(conv_pipe_kernel, (NW, BK, NI, NJ, WGM, EPI_I24, S, V, true, false, true), dim3(grid), dim3(NW * 64), 0, stream, a);
@@ -78,9 +81,11 @@ int conv_pipe_w4_launch(ConvPipeArgs a, int tile, int valid, bool hi16, int grid
 {
     N2D2HIP_REQUIRE(a.c.epi.kind == EPI_I24 && a.c.ktot % 64 == 0 && a.c.in_cs % 64 == 0, N2D2HIP_ERR_INVALID,
                     "conv_pipe_w4: integer rescale and a multiple of 64 channels expected");
+    N2D2HIP_REQUIRE(tile != 3 || !a.res, N2D2HIP_ERR_INVALID, "conv_pipe_w4: no folded sum on 64 x 64 tiles");
     if (tile == 0) launch<2, 1, 4>(a, valid, hi16, grid, stream);
     else if (tile == 1) launch<2, 2, 2>(a, valid, hi16, grid, stream);
-    else launch<2, 1, 2>(a, valid, hi16, grid, stream);
+    else if (tile == 2) launch<2, 1, 2>(a, valid, hi16, grid, stream);
+    else launch<1, 1, 2>(a, valid, hi16, grid, stream);
     N2D2HIP_HIP_CHECK(hipGetLastError());
     return N2D2HIP_OK;
 }

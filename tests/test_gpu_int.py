@@ -1118,6 +1118,24 @@ def test_where_the_chain_launch_pays(rt, cm, stride, batch, size, pays):
     assert expand.chain_pays(conv, batch, size, size) == pays
 
 
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("B,H,W,Cc,O,k", [(1, 120, 136, 128, 128, 1), (1, 128, 128, 128, 128, 1), (5, 29, 113, 128, 128, 1), (3, 7, 5, 128, 320, 3),
+                                          (1, 1, 1, 256, 200, 1), (2, 13, 9, 192, 136, 3)])
+def test_channel_tiles_of_64_for_few_pixels(rt, bits, B, H, W, Cc, O, k):
+    """Both sides of the line (255, 256 and 257 tiles of 64 pixels x 128 channels) and channel counts that end inside a tile."""
+    from n2d2_amd import capi
+    from oracle import cells as cells_ref
+    rng = np.random.default_rng(B * H * W + O)
+    print("tiles", bits, B, H, W, Cc, O, k, flush=True)
+    x = rng.integers(0, 256, size=(B, Cc, H, W))
+    top = 7 if bits == 4 else 40
+    w, bias = rng.integers(-top - 1, top + 1, size=(O, Cc, k, k)), rng.integers(-2000, 2000, size=O)
+    spec = conv_spec_for(O, rng)
+    conv = rt.Conv(w, bias, rt.Act(O, **spec.kwargs()), capi.U8B, pad=(k // 2,) * 4, weight_bits=bits)
+    got = conv.forward(rt.DTensor.from_numpy(x, capi.U8B)).to_numpy()
+    assert np.array_equal(got, cells_ref.conv_cell(x, w, bias, spec, pad=(k // 2,) * 4).astype(np.int64))
+
+
 def conv_spec_for(O, rng):
     from oracle.cells import ActSpec
     return ActSpec("Linear", "DoubleShift", np.stack([rng.integers(0, 3, size=O), rng.integers(8, 12, size=O)], 1), nb_bits=8, unsigned_out=False)
