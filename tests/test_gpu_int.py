@@ -1118,6 +1118,27 @@ def test_where_the_chain_launch_pays(rt, cm, stride, batch, size, pays):
     assert expand.chain_pays(conv, batch, size, size) == pays
 
 
+@pytest.mark.parametrize("src", ["U8", "U8B", "I8"])
+@pytest.mark.parametrize("W", [3, 4, 5, 6, 7, 9, 127, 129, 193])
+def test_space_to_depth_of_rows_of_any_length(rt, W, src):
+    """Byte planes into 16-byte pixels of 2 x 2: rows that end one, two or three columns into a dword, or are shorter than one."""
+    from n2d2_amd import capi
+    for B, Cc, H, halo, dst in ((2, 3, 5, 2, "U8B"), (1, 1, 4, 0, "I8" if src == "I8" else "U8B"), (3, 4, 3, 4, "I8" if src == "I8" else "U8"),
+                                (2, 3, 4, 1, "U8B")):
+        print("s2d convert", W, src, B, Cc, H, halo, dst, flush=True)
+        v = np.random.default_rng(W).integers(-128 if src == "I8" else 0, 128 if src == "I8" else 256, size=(B, Cc, H, W))
+        into = lambda a, t: {"U8": a.astype(np.uint8).view(np.int8), "U8B": (a - 128).astype(np.int8), "I8": a.astype(np.int8)}[t]
+        x = rt.DTensor(B, Cc, H, W, getattr(capi, src), capi.NCHW)
+        x.buf.copy_(rt.torch.from_numpy(into(v, src).reshape(-1)).view(x.buf.dtype))
+        out = rt.DTensor(B, Cc, H, W, getattr(capi, dst), capi.S2D, halo=halo).convert_from(x)
+        Hp, Wp = (H + 1) // 2, (W + 1) // 2
+        want = np.zeros((B, 2 * (Hp + 2 * halo), 2 * (Wp + 2 * halo), 4), dtype=np.int64)
+        kept = v if dst == "I8" or src != "I8" else np.maximum(v, 0)        # (unsigned forms hold no negative values)
+        want[:, 2 * halo:2 * halo + H, 2 * halo:2 * halo + W, :Cc] = kept.transpose(0, 2, 3, 1)
+        want = want.reshape(B, Hp + 2 * halo, 2, Wp + 2 * halo, 2, 4).transpose(0, 1, 3, 2, 4, 5)
+        assert np.array_equal(out.raw().view(np.int8), into(want, dst).reshape(-1)), (B, Cc, H, halo, dst)
+
+
 @pytest.mark.parametrize("bits", [8, 4])
 @pytest.mark.parametrize("B,H,W,Cc,O,k", [(1, 120, 136, 128, 128, 1), (1, 128, 128, 128, 128, 1), (5, 29, 113, 128, 128, 1), (3, 7, 5, 128, 320, 3),
                                           (1, 1, 1, 256, 200, 1), (2, 13, 9, 192, 136, 3)])
