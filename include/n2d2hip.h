@@ -559,6 +559,17 @@ int n2d2hip_loss_f32(const float* target, const float* output, float* diff, size
 int n2d2hip_sgd_update_f32(float* data, const float* diff, size_t n, float rate_diff, float momentum,
                            float decay_times_rate, float* momentum_data, int clamp, float clamp_min, float clamp_max,
                            n2d2hip_stream_t stream);
+/* The same for `count` tensors, 32 to a launch: what a net's solvers do after one backward pass.  The tensors of a call do
+ * not overlap; the results are those of one call for each. */
+typedef struct {
+    float* data;
+    const float* diff;
+    size_t n;
+    float* momentum_data;
+    float rate_diff, momentum, decay_times_rate, clamp_min, clamp_max;
+    int clamp;
+} n2d2hip_sgd_item;
+int n2d2hip_sgd_update_f32_batch(const n2d2hip_sgd_item* items, int count, n2d2hip_stream_t stream);
 
 #ifdef __cplusplus
 }

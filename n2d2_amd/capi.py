@@ -40,7 +40,7 @@ SYMBOLS = [
     "n2d2hip_sat_act_forward", "n2d2hip_sat_act_backward", "n2d2hip_lsq_forward", "n2d2hip_lsq_backward",
     "n2d2hip_conv2d_f32_forward", "n2d2hip_conv2d_f32_backward_data", "n2d2hip_conv2d_f32_backward_filter", "n2d2hip_conv2d_f32_workspace_bytes",
     "n2d2hip_conv2d_f32_backward_bias", "n2d2hip_softmax_f32_forward", "n2d2hip_loss_workspace_bytes", "n2d2hip_loss_f32",
-    "n2d2hip_sgd_update_f32", "n2d2hip_rectifier_f32_forward", "n2d2hip_rectifier_f32_backward",
+    "n2d2hip_sgd_update_f32", "n2d2hip_sgd_update_f32_batch", "n2d2hip_rectifier_f32_forward", "n2d2hip_rectifier_f32_backward",
     "n2d2hip_batchnorm_f32_workspace_bytes", "n2d2hip_batchnorm_f32_forward", "n2d2hip_batchnorm_f32_backward", "n2d2hip_pool_max_f32_forward", "n2d2hip_pool_max_f32_backward",
     "n2d2hip_pool_average_f32_forward", "n2d2hip_pool_average_f32_backward", "n2d2hip_elemwise_sum_f32_forward", "n2d2hip_elemwise_sum_f32_backward",
 ]
@@ -55,6 +55,11 @@ class Activation(C.Structure):
     _fields_ = [("kind", C.c_int), ("leak_slope", C.c_float), ("scaling_mode", C.c_int), ("scaling", C.c_void_p),
                 ("frac_bits", C.c_int), ("is_clipped", C.c_int), ("clipping", C.c_void_p),
                 ("nb_bits", C.c_int), ("unsigned_out", C.c_int)]
+
+
+class SgdItem(C.Structure):
+    _fields_ = [("data", C.c_void_p), ("diff", C.c_void_p), ("n", C.c_size_t), ("momentum_data", C.c_void_p), ("rate_diff", C.c_float),
+                ("momentum", C.c_float), ("decay_times_rate", C.c_float), ("clamp_min", C.c_float), ("clamp_max", C.c_float), ("clamp", C.c_int)]
 
 
 class ConvDesc(C.Structure):
@@ -152,6 +157,7 @@ def load():
     lib.n2d2hip_loss_workspace_bytes.argtypes = [SZ]
     lib.n2d2hip_loss_f32.argtypes = [P, P, P, SZ, I, P, P, SZ, P]
     lib.n2d2hip_sgd_update_f32.argtypes = [P, P, SZ, F, F, F, P, I, F, F, P]
+    lib.n2d2hip_sgd_update_f32_batch.argtypes = [C.POINTER(SgdItem), I, P]
     lib.n2d2hip_rectifier_f32_forward.argtypes = [P, SZ, F, F, P]
     lib.n2d2hip_rectifier_f32_backward.argtypes = [P, P, P, SZ, F, F, P]
     D = C.c_double

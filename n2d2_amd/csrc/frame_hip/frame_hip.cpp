@@ -1289,6 +1289,9 @@ template <> Registrar<ScalingCell> ScalingCell_Frame_HIP<float>::mRegistrar("Fra
 // ------------------------------------------------------------------- SGDSolver
 SGDSolver::~SGDSolver()
 {
+    if (mMomentumData && SGDUpdateScope::current()) {
+        try { SGDUpdateScope::current()->flush(); } catch (const std::exception&) {}
+    }
     if (mMomentumData) (void)hipFree(mMomentumData);
 }
 
@@ -1325,6 +1328,42 @@ void SGDSolver::update(float& data, float diff, unsigned int batchSize)
     data += rateDiff * diff;
 }
 
+static thread_local SGDUpdateScope* sgdScope = nullptr;
+
+SGDUpdateScope::SGDUpdateScope() : mOuter(sgdScope == nullptr), mStream(nullptr)
+{
+    if (mOuter) sgdScope = this;
+}
+
+SGDUpdateScope::~SGDUpdateScope()
+{
+    if (!mOuter) return;
+    sgdScope = nullptr;
+    // (left by an exception: what came before it is still done; its own error is the one to report)
+    if (!mItems.empty()) (void)n2d2hip_sgd_update_f32_batch(mItems.data(), (int)mItems.size(), mStream);
+}
+
+void SGDUpdateScope::flush()
+{
+    if (!mOuter && sgdScope) sgdScope->flush();
+    if (mItems.empty()) return;
+    std::vector<n2d2hip_sgd_item> items;
+    items.swap(mItems);
+    checkStatus(n2d2hip_sgd_update_f32_batch(items.data(), (int)items.size(), mStream));
+}
+
+SGDUpdateScope* SGDUpdateScope::current() { return sgdScope; }
+
+void SGDUpdateScope::add(const n2d2hip_sgd_item& item, void* stream)
+{
+    bool apart = stream != mStream;
+    for (const n2d2hip_sgd_item& i : mItems)
+        apart = apart || i.data == item.data || (item.momentum_data && i.momentum_data == item.momentum_data);
+    if (apart) flush();
+    mStream = stream;
+    mItems.push_back(item);
+}
+
 void SGDSolver::update(float* data, const float* diff, std::size_t n, unsigned int batchSize, void* stream)
 {
     const float rate = (float)getLearningRate();
@@ -1333,14 +1372,16 @@ void SGDSolver::update(float* data, const float* diff, std::size_t n, unsigned i
     const float rateDiff = rate / ((float)batchSize * (float)mIterationSize);
     const bool plain = (mMomentum == 0.0 && mDecay == 0.0);
     if (!plain && mMomentumSize != n) {
+        if (SGDUpdateScope* scope = SGDUpdateScope::current()) scope->flush();
         if (mMomentumData) (void)hipFree(mMomentumData);
         mMomentumData = nullptr;
         checkHip(hipMalloc((void**)&mMomentumData, n * sizeof(float)), "SGDSolver::update()");
         checkHip(hipMemsetAsync(mMomentumData, 0, n * sizeof(float), (hipStream_t)stream), "SGDSolver::update()");
         mMomentumSize = n;
     }
-    checkStatus(n2d2hip_sgd_update_f32(data, diff, n, rateDiff, (float)mMomentum, (float)mDecay * rate, plain ? nullptr : mMomentumData,
-                                       0, 0.0f, 0.0f, stream));
+    const n2d2hip_sgd_item item = {data, diff, n, plain ? nullptr : mMomentumData, rateDiff, (float)mMomentum, (float)mDecay * rate, 0.0f, 0.0f, 0};
+    if (SGDUpdateScope* scope = SGDUpdateScope::current()) scope->add(item, stream);
+    else checkStatus(n2d2hip_sgd_update_f32_batch(&item, 1, stream));
 }
 
 template <> Registrar<SGDSolver> SGDSolver_Frame_HIP<float>::mRegistrar("Frame_HIP", SGDSolver_Frame_HIP<float>::create,

@@ -852,6 +852,27 @@ private:
 // ------------------------------------------------------------------ quantizers
 // Solver used by the quantizers' update() (include/Solver/SGDSolver_Frame.hpp:84-109: N2D2 ADDS
 // rate/(batch*iterationSize)*diff, because its diffInputs carry target - output).
+// While one lives, the device updates of the calling thread's solvers are gathered and launched together: when it ends, when
+// an update is for another stream or for a tensor already in the list, and before a solver frees its momentum.  A scope inside
+// another leaves the launch to the outer one.
+class SGDUpdateScope {
+public:
+    SGDUpdateScope();
+    ~SGDUpdateScope();
+    SGDUpdateScope(const SGDUpdateScope&) = delete;
+    SGDUpdateScope& operator=(const SGDUpdateScope&) = delete;
+    // launches what has been gathered, by an outer scope too
+    void flush();
+    // the calling thread's outermost scope, or null
+    static SGDUpdateScope* current();
+    void add(const n2d2hip_sgd_item& item, void* stream);
+
+private:
+    bool mOuter;
+    void* mStream;
+    std::vector<n2d2hip_sgd_item> mItems;
+};
+
 class SGDSolver {
 public:
     typedef std::function<std::shared_ptr<SGDSolver>()> RegistryCreate_T;

@@ -374,7 +374,9 @@ int fh_train_learn(void* net, const float* targets, size_t nTargets, int iterati
                 throw std::runtime_error("fh_train_learn(): copy of the targets failed");
             l = last->applyLoss();
             for (auto c = n.cells.rbegin(); c != n.cells.rend(); ++c) (*c)->backPropagate();
+            SGDUpdateScope updates;              // (all tensors of the net in one launch)
             for (auto c = n.cells.rbegin(); c != n.cells.rend(); ++c) (*c)->update();
+            updates.flush();
         }
         if (hipDeviceSynchronize() != hipSuccess) throw std::runtime_error("fh_train_learn(): device error");
         if (loss) *loss = l;

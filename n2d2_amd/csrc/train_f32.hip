@@ -294,21 +294,40 @@ __global__ __launch_bounds__(TBLOCK) void loss_finish_kernel(const double* __res
 }
 
 // SGDSolver_Frame::update for one tensor.
-__global__ __launch_bounds__(TBLOCK) void sgd_f32_kernel(float* __restrict__ data, const float* __restrict__ diff, size_t n, float rate_diff,
-                                                         float momentum, float decay_rate, float* __restrict__ mom, float lo, float hi, int clamp)
+// SGD updates of up to SGD_ITEMS tensors.  Most tensors of a net are small (scales, biases, steps), and a launch for each is
+// what bounds an update; the blocks of one launch find their tensor in the table that comes with the arguments.  16 tensors
+// of a small LeNet (61 k values): 16 launches of 1.7 us, now one of 3.8.  N: room in the table (2 KB of arguments for 32; a
+// single tensor does not pay for them).
+constexpr int SGD_ITEMS = 32;
+template <int N>
+struct SgdBatch {
+    n2d2hip_sgd_item item[N];
+    unsigned first[N + 1];                       // first block of a tensor; the grid behind the last
+    int count;
+};
+template <int N>
+__global__ __launch_bounds__(TBLOCK) void sgd_f32_kernel(SgdBatch<N> b)
 {
-    for (size_t i = (size_t)blockIdx.x * TBLOCK + threadIdx.x; i < n; i += (size_t)gridDim.x * TBLOCK) {
+    int k = 0;
+    if (N > 1)
+        while (k + 1 < b.count && blockIdx.x >= b.first[k + 1]) ++k;
+    const n2d2hip_sgd_item& t = b.item[k];
+    float* __restrict__ data = t.data;
+    const float* __restrict__ diff = t.diff;
+    float* __restrict__ mom = t.momentum_data;
+    const size_t n = t.n, step = (size_t)(b.first[k + 1] - b.first[k]) * TBLOCK;
+    for (size_t i = (size_t)(blockIdx.x - b.first[k]) * TBLOCK + threadIdx.x; i < n; i += step) {
         float v;
         if (mom) {
-            float m = mom[i] * momentum;
-            m += rate_diff * diff[i];
-            if (decay_rate != 0.0f) m += -decay_rate * data[i];
+            float m = mom[i] * t.momentum;
+            m += t.rate_diff * diff[i];
+            if (t.decay_times_rate != 0.0f) m += -t.decay_times_rate * data[i];
             mom[i] = m;
             v = data[i] + m;
         } else {
-            v = data[i] + rate_diff * diff[i];
+            v = data[i] + t.rate_diff * diff[i];
         }
-        data[i] = clamp ? fminf(fmaxf(v, lo), hi) : v;
+        data[i] = t.clamp ? fminf(fmaxf(v, t.clamp_min), t.clamp_max) : v;
     }
 }
 
@@ -1608,16 +1627,38 @@ int n2d2hip_loss_f32(const float* target, const float* output, float* diff, size
     return N2D2HIP_OK;
 }
 
+int n2d2hip_sgd_update_f32_batch(const n2d2hip_sgd_item* items, int count, n2d2hip_stream_t stream)
+{
+    N2D2HIP_REQUIRE(items && count > 0, N2D2HIP_ERR_INVALID, "n2d2hip_sgd_update_f32: bad argument");
+    for (int k = 0; k < count; ++k) {
+        N2D2HIP_REQUIRE(items[k].data && items[k].diff && items[k].n > 0, N2D2HIP_ERR_INVALID, "n2d2hip_sgd_update_f32: bad argument");
+        N2D2HIP_REQUIRE(items[k].momentum_data || (items[k].momentum == 0.0f && items[k].decay_times_rate == 0.0f), N2D2HIP_ERR_INVALID,
+                        "n2d2hip_sgd_update_f32: momentum or decay without a momentum buffer");
+    }
+    const auto launch = [&](auto N_, const n2d2hip_sgd_item* item, int nb) {
+        constexpr int N = decltype(N_)::value;
+        SgdBatch<N> b = {};
+        b.count = nb;
+        for (int i = 0; i < nb; ++i) {
+            b.item[i] = item[i];
+            b.first[i + 1] = b.first[i] + (unsigned)grid_for(item[i].n);
+        }
+        hipLaunchKernelGGL(sgd_f32_kernel<N>, dim3(b.first[nb]), dim3(TBLOCK), 0, (hipStream_t)stream, b);
+    };
+    for (int k = 0; k < count; k += SGD_ITEMS) {
+        const int nb = std::min(count - k, SGD_ITEMS);
+        if (nb == 1) launch(std::integral_constant<int, 1>{}, items + k, nb);
+        else launch(std::integral_constant<int, SGD_ITEMS>{}, items + k, nb);
+    }
+    N2D2HIP_HIP_CHECK(hipGetLastError());
+    return N2D2HIP_OK;
+}
+
 int n2d2hip_sgd_update_f32(float* data, const float* diff, size_t n, float rate_diff, float momentum, float decay_times_rate,
                            float* momentum_data, int clamp, float clamp_min, float clamp_max, n2d2hip_stream_t stream)
 {
-    N2D2HIP_REQUIRE(data && diff && n > 0, N2D2HIP_ERR_INVALID, "n2d2hip_sgd_update_f32: bad argument");
-    N2D2HIP_REQUIRE(momentum_data || (momentum == 0.0f && decay_times_rate == 0.0f), N2D2HIP_ERR_INVALID,
-                    "n2d2hip_sgd_update_f32: momentum or decay without a momentum buffer");
-    hipLaunchKernelGGL(sgd_f32_kernel, dim3(grid_for(n)), dim3(TBLOCK), 0, (hipStream_t)stream, data, diff, n, rate_diff, momentum,
-                       decay_times_rate, momentum_data, clamp_min, clamp_max, clamp);
-    N2D2HIP_HIP_CHECK(hipGetLastError());
-    return N2D2HIP_OK;
+    const n2d2hip_sgd_item item = {data, diff, n, momentum_data, rate_diff, momentum, decay_times_rate, clamp_min, clamp_max, clamp};
+    return n2d2hip_sgd_update_f32_batch(&item, 1, stream);
 }
 
 } // extern "C"

@@ -567,3 +567,33 @@ def test_elemwise_sum_float_forward_backward(g, shape, n_in):
             assert np.array_equal(g.host(out).reshape(shape), wdx)
     assert g.lib.n2d2hip_elemwise_sum_f32_forward(9, ptrs, n, wa, sa, y.data_ptr(), g.sp()) == g.capi.ERR_UNSUPPORTED
     assert g.lib.n2d2hip_elemwise_sum_f32_forward(0, ptrs, n, wa, sa, y.data_ptr(), g.sp()) == g.capi.ERR_INVALID
+
+
+@pytest.mark.parametrize("count", [1, 3, 32, 33, 70])
+def test_sgd_update_of_many_tensors(g, count):
+    """Launches of up to 32 tensors: sizes around a block, with and without momentum, decay and clamping; a refused item touches none."""
+    rng = np.random.default_rng(count)
+    items, want, keep = (g.capi.SgdItem * count)(), [], []
+    for k in range(count):
+        n = [1, 255, 256, 257, 5000][k % 5]
+        data, diff, mom = (rng.normal(size=n).astype(np.float32) for _ in range(3))
+        rate, momentum, decay = np.float32(0.05 + 0.01 * k), np.float32(0.9 if k % 2 else 0.0), np.float32(0.001 if k % 4 == 1 else 0.0)
+        dev = [g.dev(data), g.dev(diff), g.dev(mom) if k % 2 else None]
+        keep.append(dev)
+        items[k] = g.capi.SgdItem(dev[0].data_ptr(), dev[1].data_ptr(), n, dev[2].data_ptr() if k % 2 else None, rate, momentum, decay, -1.0, 1.0, k % 3 == 0)
+        v = data + rate * diff
+        if k % 2:
+            mom = mom * momentum + rate * diff
+            mom = mom + -decay * data if decay else mom
+            v = data + mom
+        want.append((np.clip(v, -1, 1) if k % 3 == 0 else v, mom))
+    bad = g.capi.SgdItem.from_buffer_copy(items[count - 1])
+    bad.diff, good = None, g.capi.SgdItem.from_buffer_copy(items[count - 1])
+    items[count - 1] = bad
+    assert g.lib.n2d2hip_sgd_update_f32_batch(items, count, g.sp()) == g.capi.ERR_INVALID
+    items[count - 1] = good
+    g.check(g.lib.n2d2hip_sgd_update_f32_batch(items, count, g.sp()))
+    for (data, _, mom), (v, m) in zip(keep, want):
+        assert np.array_equal(g.host(data), v)
+        assert mom is None or np.array_equal(g.host(mom), m)
+    assert g.lib.n2d2hip_sgd_update_f32_batch(None, 1, g.sp()) == g.capi.ERR_INVALID
