@@ -731,6 +731,9 @@ static bool spans_input(const ConvF32& q)
 enum { PASS_FWD = 0, PASS_BWD_DATA = 1, PASS_BWD_FILTER = 2 };
 enum { F32_PATH_DIRECT, F32_PATH_GEMM, F32_PATH_SMALL };
 
+// More than the pixel and filter kernels have lanes and mask bits for
+static bool many_taps(const ConvF32& q) { return q.kH + q.kW > 31 || q.kH * q.kW > 64; }
+
 // The kernels of a pass.  The matrix cores serve ungrouped convolutions without dilation; the direct kernels keep the rest
 // (depthwise, dilated) and the forward sums below 2e7 flops or of kernels over 64 taps, which stay in the reference's order
 // of terms (quantizers turn the last bit of a sum into a level now and then).  Backward-filter below 2e7 flops stays in
@@ -741,13 +744,12 @@ static int f32_path(const ConvF32& q, int pass)
         return F32_PATH_DIRECT;
     // 32-bit byte offsets from a base moved back by the padding, and one validity bit per tap row and column
     const size_t lim = ((size_t)1 << 29) - (size_t)(q.pt + q.kH) * (q.W + q.oW + q.pl + q.kW);
-    const bool many_taps = q.kH + q.kW > 31 || q.kH * q.kW > 64;
     if ((size_t)q.B * q.C * q.H * q.W >= lim || (size_t)q.B * q.O * q.oH * q.oW >= lim || (size_t)q.O * q.C * q.kH * q.kW >= lim
-        || (many_taps && !spans_input(q)))
+        || (many_taps(q) && !spans_input(q)))
         return F32_PATH_DIRECT;
     if (q.choice & N2D2HIP_KERNEL_F32_GEMM) return F32_PATH_GEMM;
     const bool small = 2.0 * q.B * q.O * q.oH * q.oW * q.C * q.kH * q.kW < 2.0e7;
-    if (pass == PASS_FWD) return small || many_taps ? F32_PATH_DIRECT : F32_PATH_GEMM;
+    if (pass == PASS_FWD) return small || many_taps(q) ? F32_PATH_DIRECT : F32_PATH_GEMM;
     return small && pass == PASS_BWD_FILTER ? F32_PATH_SMALL : F32_PATH_GEMM;
 }
 
@@ -1152,9 +1154,11 @@ int n2d2hip_conv2d_f32_forward(const n2d2hip_conv_desc* desc, int B, int H, int 
         if (spans_input(q)) {
             int pass;
             const ConvF32 m = product_of(q, PASS_FWD, &pass);
-            // (without a workspace that holds its partial results: the convolution as it stands)
+            // (without a workspace that holds its partial results: the convolution as it stands, whose kernels keep a tap in each
+            // of a wave's 64 lanes, or the direct kernels)
             if (pass_workspace(m, pass) <= nws)
                 return run_pass(m, pass, w, x, bias, 1, q.O, beta, y, ws, nws, (hipStream_t)stream);
+            if (many_taps(q)) return run_direct(q, PASS_FWD, x, w, bias, beta, y, (hipStream_t)stream);
         }
         return run_pass(q, PASS_FWD, x, w, bias, q.oH * q.oW, q.O, beta, y, ws, nws, (hipStream_t)stream);
     }

@@ -261,6 +261,31 @@ def test_conv_kernels_chosen_by_size(g, case, workspace):
         assert _rel(g.host(dw), want[2] + 1, mag[2] + 1) <= TOL
 
 
+# B, C, H, W, O of layers that span their input with 64 taps, 65 and more, up to more columns than a mask word has bits
+SPANNING = [(5, 3, 8, 8, 7), (3, 2, 5, 13, 4), (2, 3, 9, 9, 4), (70, 5, 16, 16, 33), (4, 6, 1, 70, 9)]
+
+
+@pytest.mark.parametrize("workspace", [True, False])
+@pytest.mark.parametrize("case", SPANNING)
+def test_forward_of_a_spanning_layer(g, case, path, workspace):
+    """The forward sums of a kernel as large as its input on the kernels asked for, with and without a workspace."""
+    B, Cn, H, W, O = case
+    print("spanning forward", case, path, workspace, flush=True)
+    rng = np.random.default_rng(sum(case))
+    x, w = rng.normal(size=(B, Cn, H, W)).astype(np.float32), rng.normal(size=(O, Cn, H, W)).astype(np.float32)
+    bias = rng.normal(size=O).astype(np.float32)
+    x64, w64 = (v.astype(np.float64).reshape(v.shape[0], -1) for v in (x, w))
+    want, mag = x64 @ w64.T + bias, np.abs(x64) @ np.abs(w64).T + np.abs(bias)
+    d = g.capi.ConvDesc(Cn, O, W, H, 1, 1, 0, 0, 0, 0, 1, 1, 1, 0, {"direct": g.capi.KERNEL_F32_DIRECT, "gemm": g.capi.KERNEL_F32_GEMM}[path])
+    need = int(g.lib.n2d2hip_conv2d_f32_workspace_bytes(C.byref(d), B, H, W)) if workspace else 0
+    ws = g.torch_.empty(max(need, 4), dtype=g.torch_.uint8, device="cuda")
+    x_, w_, b_ = g.dev(x), g.dev(w), g.dev(bias)
+    y = g.torch_.ones((B, O), dtype=g.torch_.float32, device="cuda")
+    g.check(g.lib.n2d2hip_conv2d_f32_forward(C.byref(d), B, H, W, x_.data_ptr(), w_.data_ptr(), b_.data_ptr(), 0.0, y.data_ptr(),
+                                             ws.data_ptr() if need else None, need, g.sp()))
+    assert _rel(g.host(y), want, mag) <= TOL
+
+
 # B, C, H, W, k, stride, pad: strips of four with every remainder, rows shorter than a strip or a window, windows past both
 # ends of the tensor, both parities of the padding at stride 2, blocks of 256 and of 1024 threads, outputs wider than the input
 DEPTHWISE = [(1, 1, 1, 1, 3, 1, 1), (2, 3, 2, 3, 3, 1, 1), (1, 1, 3, 3, 3, 1, 0), (3, 2, 5, 6, 3, 2, 0), (2, 5, 9, 7, 3, 2, 1), (1, 4, 6, 9, 3, 2, 2),
