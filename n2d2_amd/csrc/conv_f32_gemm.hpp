@@ -864,12 +864,13 @@ __global__ __launch_bounds__(256) void conv_f32_filter_kernel(FilterGemm g, cons
     }
 }
 
-// Backward-filter of small problems, in double on the fp64 matrix cores (16 x 16 x 4): a block is a 16 x 16 tile of dw and a
-// range of pixels, dealt to its four waves 16 at a time; a lane takes four consecutive pixels of its row of q and of its
+// Backward-filter of small problems, and of spanning kernels of more than 64 taps, in double on the fp64 matrix cores
+// (16 x 16 x 4): a block is a 16 x 16 tile of dw and a range of pixels, dealt to its four waves 16 at a time; a lane takes four consecutive pixels of its row of q and of its
 // column of p, one per matrix instruction.  Nothing here is near a rate: the time is that of the loads' latency and of two
 // launches, so the range is as short as fills the chip, and the next 16 pixels are on their way while these are multiplied.
 // Against one block per weight summing all pixels (32 images, 1 x 32 x 32 -> 6, 5x5): 46 -> 12 us; 16 -> 32 channels, 3x3 on
-// 16 x 16: 50 -> 12 us.
+// 16 x 16: 50 -> 12 us.  Spanning layers, whose K is the batch: 16384 -> 10, 64 images: 211 -> 8.2 us; 20736 -> 64, 64 images:
+// 1690 -> 22 (fp32 matrix instructions take 10, with four times the error of a sum in double: 1.4e-7 against 2.5e-8).
 typedef double v4d __attribute__((ext_vector_type(4)));
 __global__ __launch_bounds__(256) void conv_f32_filter_small_kernel(FilterGemm g, const float* __restrict__ srcX, const float* __restrict__ srcY,
                                                                     double* __restrict__ partial, float beta, float* __restrict__ out)

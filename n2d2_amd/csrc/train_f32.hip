@@ -736,8 +736,9 @@ static bool many_taps(const ConvF32& q) { return q.kH + q.kW > 31 || q.kH * q.kW
 
 // The kernels of a pass.  The matrix cores serve ungrouped convolutions without dilation; the direct kernels keep the rest
 // (depthwise, dilated) and the forward sums below 2e7 flops or of kernels over 64 taps, which stay in the reference's order
-// of terms (quantizers turn the last bit of a sum into a level now and then).  Backward-filter below 2e7 flops stays in
-// double (F32_PATH_SMALL).  The descriptor's kernel_choice (N2D2HIP_KERNEL_F32_DIRECT / _GEMM) overrides the size rules.
+// of terms (quantizers turn the last bit of a sum into a level now and then).  Backward-filter below 2e7 flops, and of a
+// spanning kernel over 64 taps, adds in double (F32_PATH_SMALL).  The descriptor's kernel_choice (N2D2HIP_KERNEL_F32_DIRECT /
+// _GEMM) overrides the size rules.
 static int f32_path(const ConvF32& q, int pass)
 {
     if (q.depthwise || q.dx != 1 || q.dy != 1 || (q.choice & N2D2HIP_KERNEL_F32_DIRECT))
@@ -747,6 +748,7 @@ static int f32_path(const ConvF32& q, int pass)
     if ((size_t)q.B * q.C * q.H * q.W >= lim || (size_t)q.B * q.O * q.oH * q.oW >= lim || (size_t)q.O * q.C * q.kH * q.kW >= lim
         || (many_taps(q) && !spans_input(q)))
         return F32_PATH_DIRECT;
+    if (pass == PASS_BWD_FILTER && q.kH * q.kW > 64) return F32_PATH_SMALL;
     if (q.choice & N2D2HIP_KERNEL_F32_GEMM) return F32_PATH_GEMM;
     const bool small = 2.0 * q.B * q.O * q.oH * q.oW * q.C * q.kH * q.kW < 2.0e7;
     if (pass == PASS_FWD) return small || many_taps(q) ? F32_PATH_DIRECT : F32_PATH_GEMM;

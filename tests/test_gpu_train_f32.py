@@ -286,6 +286,29 @@ def test_forward_of_a_spanning_layer(g, case, path, workspace):
     assert _rel(g.host(y), want, mag) <= TOL
 
 
+@pytest.mark.parametrize("workspace", [True, False])
+@pytest.mark.parametrize("case", [(64, 16, 9, 9, 123), (129, 3, 16, 16, 103), (1000, 2, 5, 13, 97), (2, 3, 9, 9, 4)])
+def test_filter_gradient_of_a_spanning_layer_is_added_in_double(g, case, path, workspace):
+    """More than 64 taps, on both sides of 2e7 flops: one rounding to float and what sums of B terms in double lose; a caller
+    without a workspace is served as well."""
+    B, Cn, H, W, O = case
+    print("spanning filter gradient", case, path, workspace, flush=True)
+    rng = np.random.default_rng(sum(case))
+    x, dy = rng.normal(size=(B, Cn, H, W)).astype(np.float32), rng.normal(size=(B, O)).astype(np.float32)
+    x64, dy64 = x.astype(np.longdouble).reshape(B, -1), dy.astype(np.longdouble)
+    want, mag = dy64.T @ x64, np.abs(dy64).T @ np.abs(x64)
+    d = g.capi.ConvDesc(Cn, O, W, H, 1, 1, 0, 0, 0, 0, 1, 1, 1, 0, {"direct": g.capi.KERNEL_F32_DIRECT, "gemm": g.capi.KERNEL_F32_GEMM}[path])
+    need = int(g.lib.n2d2hip_conv2d_f32_workspace_bytes(C.byref(d), B, H, W)) if workspace else 0
+    ws = g.torch_.empty(max(need, 4), dtype=g.torch_.uint8, device="cuda")
+    x_, dy_ = g.dev(x), g.dev(dy)
+    dw = g.torch_.ones(want.shape, dtype=g.torch_.float32, device="cuda")
+    g.check(g.lib.n2d2hip_conv2d_f32_backward_filter(C.byref(d), B, H, W, x_.data_ptr(), dy_.data_ptr(), 0.0, dw.data_ptr(),
+                                                     ws.data_ptr() if need else None, need, g.sp()))
+    # (the direct kernel rounds each product to float)
+    bound = np.abs(want) * 2.0 ** -24 + mag * ((2.0 ** -24 if path == "direct" else 0.0) + B * 2.0 ** -52)
+    assert (np.abs(g.host(dw).astype(np.longdouble) - want) <= bound).all()
+
+
 # B, C, H, W, k, stride, pad: strips of four with every remainder, rows shorter than a strip or a window, windows past both
 # ends of the tensor, both parities of the padding at stride 2, blocks of 256 and of 1024 threads, outputs wider than the input
 DEPTHWISE = [(1, 1, 1, 1, 3, 1, 1), (2, 3, 2, 3, 3, 1, 1), (1, 1, 3, 3, 3, 1, 0), (3, 2, 5, 6, 3, 2, 0), (2, 5, 9, 7, 3, 2, 1), (1, 4, 6, 9, 3, 2, 2),
