@@ -82,7 +82,7 @@ struct FilterGemm {
     int C, H, W, kW, kH, s_y, s_x, pt, pl;
     int oW, plane;             // output row length and plane
     int imgX, imgY;
-    int ctiles;                // by taps: tiles of channels
+    int rowY;                  // from one row of q to the next in Y (the small kernel; others: plane)
     unsigned bytesX, bytesY;
     DivF32 dplane, dow;
 };
@@ -864,8 +864,9 @@ __global__ __launch_bounds__(256) void conv_f32_filter_kernel(FilterGemm g, cons
     }
 }
 
-// Backward-filter of small problems, and of spanning kernels of more than 64 taps, in double on the fp64 matrix cores
-// (16 x 16 x 4): a block is a 16 x 16 tile of dw and a range of pixels, dealt to its four waves 16 at a time; a lane takes four consecutive pixels of its row of q and of its
+// Backward-filter of small problems, and of spanning kernels of more than 64 taps (backward-data of spanning kernels of up to
+// 64 as well, which is such a sum over the outputs), in double on the fp64 matrix cores (16 x 16 x 4): a block is a 16 x 16
+// tile of dw and a range of pixels, dealt to its four waves 16 at a time; a lane takes four consecutive pixels of its row of q and of its
 // column of p, one per matrix instruction.  Nothing here is near a rate: the time is that of the loads' latency and of two
 // launches, so the range is as short as fills the chip, and the next 16 pixels are on their way while these are multiplied.
 // Against one block per weight summing all pixels (32 images, 1 x 32 x 32 -> 6, 5x5): 46 -> 12 us; 16 -> 32 channels, 3x3 on
@@ -882,7 +883,7 @@ __global__ __launch_bounds__(256) void conv_f32_filter_small_kernel(FilterGemm g
     const int kHW = g.kH * g.kW, pp = min(p, g.P - 1);
     const int ch = pp / kHW, t = pp - ch * kHW, ty = t / g.kW, tx = t - ty * g.kW;
     const float* xb = srcX + (size_t)ch * g.H * g.W;
-    const float* yb = srcY + (size_t)min(q, g.Q - 1) * g.plane;
+    const float* yb = srcY + (size_t)min(q, g.Q - 1) * g.rowY;
     float a[2][4], b[2][4];
     auto load = [&](int k0, float (&av)[4], float (&bv)[4]) {
 #pragma unroll

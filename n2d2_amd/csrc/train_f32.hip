@@ -23,6 +23,7 @@ struct ConvF32 {
     int sx, sy, pl, pt, pr, pb, dx, dy;
     int depthwise;                                // groups == C == O
     int choice;                                   // the descriptor's kernel_choice bits
+    int ranges = 0;                               // a product that stands for a pass: least number of K ranges
 };
 
 __device__ __forceinline__ double wave_sum_d(double v)
@@ -749,8 +750,16 @@ static int f32_path(const ConvF32& q, int pass)
         || (many_taps(q) && !spans_input(q)))
         return F32_PATH_DIRECT;
     if (pass == PASS_BWD_FILTER && q.kH * q.kW > 64) return F32_PATH_SMALL;
-    if (q.choice & N2D2HIP_KERNEL_F32_GEMM) return F32_PATH_GEMM;
-    const bool small = 2.0 * q.B * q.O * q.oH * q.oW * q.C * q.kH * q.kW < 2.0e7;
+    const double flops = 2.0 * q.B * q.O * q.oH * q.oW * q.C * q.kH * q.kW;
+    const bool forced = q.choice & N2D2HIP_KERNEL_F32_GEMM, small = flops < 2.0e7;
+    // As a convolution the K of a spanning layer's backward-data runs over all taps of an output, one of which is not zero: few
+    // terms to a range.  As a product it has as many terms as outputs, so it adds in double up to 5e8 flops (64 images,
+    // 64 x 4 x 4 <- 256: 2.5e-8 from 64 bits and 10 us; convolution 7.7e-8, 41 us; product in float 2.9e-7, 14 us) and beyond
+    // takes as many ranges as the convolution would (128 images, 512 x 2 x 2 <- 1000: 1.5e-7 and 26 us; in double 36; convolution
+    // 1.5e-7, 64; 64 images, 512 x 7 x 7 <- 4096: 179 us, in double 1019, convolution 9566).
+    if (pass == PASS_BWD_DATA && (forced || !small) && flops < 5.0e8 && q.kH * q.kW > 1 && q.kH * q.kW <= 64 && spans_input(q))
+        return F32_PATH_SMALL;
+    if (forced) return F32_PATH_GEMM;
     if (pass == PASS_FWD) return small || many_taps(q) ? F32_PATH_DIRECT : F32_PATH_GEMM;
     return small && pass == PASS_BWD_FILTER ? F32_PATH_SMALL : F32_PATH_GEMM;
 }
@@ -835,16 +844,26 @@ static int run_direct(const ConvF32& q, int pass, const float* x, const float* w
     return N2D2HIP_OK;
 }
 
+// K ranges of P pixels x Q channels over K terms, from the sizes alone, as if tiles were 128 x 128: 768 blocks, none below 256
+// terms.
+static int pass_ranges(long P, int Q, long K)
+{
+    const long tiles = ((P + 127) / 128) * (Q <= 64 ? 1 : ceil_div_i(Q, 128));
+    return (int)std::min<long>(tiles >= 384 ? 1 : std::max(1L, 768 / tiles), std::max(1L, K / (16 * GK)));
+}
+
 // A kernel that spans its input (an FcCell) makes of each pass a plain matrix product, which is a 1x1 convolution with the
 // roles of the tensors exchanged so that the long contiguous dimension is the one the kernels read contiguously:
 //   forward          y[b][o] = sum_k x[b][k] w[o][k]     the filter pass of pixels k between "channels" w[o] and "outputs" x[b]
 //   backward data    dx[b][k] = sum_o dy[b][o] w[o][k]   the forward pass over one "image" w of O channels and K pixels
 //   backward filter  dw[o][k] = sum_b dy[b][o] x[b][k]   the data pass over one "image" x of B channels and K pixels
+// Backward data runs at least as many ranges as the convolution itself would, so that no float sum is longer.
 static ConvF32 product_of(const ConvF32& q, int pass, int* as_pass)
 {
-    const int K = q.C * q.H * q.W;
+    const int K = q.C * q.H * q.W, T = q.H * q.W;
+    const int ranges = pass == PASS_BWD_DATA && T > 1 && T <= 64 ? pass_ranges((long)q.B * T, q.C, (long)q.O * T) : 0;
     *as_pass = pass == PASS_FWD ? PASS_BWD_FILTER : pass == PASS_BWD_DATA ? PASS_FWD : PASS_BWD_DATA;
-    return ConvF32{1, q.O, 1, K, q.B, 1, K, 1, 1, q.O, 1, 1, 0, 0, 0, 0, 1, 1, 0, q.choice};
+    return ConvF32{1, q.O, 1, K, q.B, 1, K, 1, 1, q.O, 1, 1, 0, 0, 0, 0, 1, 1, 0, q.choice, ranges};
 }
 
 // ---- forward and backward-data: tile shape and K ranges of a launch
@@ -936,17 +955,15 @@ static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass>
     g.nz = 1;
     long splits;
     if (fwd) {
-        // The ranges of a forward sum follow from its sizes alone, as if tiles were 128 x 128: with another order of additions
-        // the quantizer behind it would give another level now and then.  With a block for every CU it takes all of them.
-        const long tiles128 = (long)ceil_div_i(P, 128) * (g.Q <= 64 ? 1 : ceil_div_i(g.Q, 128));
-        splits = tiles128 >= 384 ? 1 : std::max(1L, 768 / tiles128);
-        splits = std::min<long>(splits, std::max(1L, kmax / (16 * GK)));
+        // The ranges of a forward sum follow from its sizes alone: with another order of additions the quantizer behind it would
+        // give another level now and then.  With a block for every CU it takes all of them.
+        splits = pass_ranges(P, g.Q, kmax);
     } else {
         // where the tiles do not fill the chip twice; none below four steps
         splits = blocks >= 512 ? 1 : std::max(1L, 768 / blocks);
         splits = std::min<long>(splits, std::max(1L, kmax / (4 * GK)));
     }
-    g.kchunk = std::max(round_up((int)((kmax + splits - 1) / splits), GK), GK);
+    g.kchunk = std::max(q.ranges > splits ? (int)(kmax / q.ranges) / GK * GK : round_up((int)((kmax + splits - 1) / splits), GK), GK);
     pl.splits = std::max(1, ceil_div_i(kmax, g.kchunk));
     if (fwd && blocks >= 256) {
         g.nz = pl.splits;
@@ -990,7 +1007,7 @@ static FilterGemm filter_gemm(const ConvF32& q)
     g.C = q.C; g.H = q.H; g.W = q.W; g.kW = q.kW; g.kH = q.kH;
     g.s_y = q.sy; g.s_x = q.sx; g.pt = q.pt; g.pl = q.pl;
     g.oW = q.oW; g.plane = q.oH * q.oW;
-    g.imgX = q.C * q.H * q.W; g.imgY = q.O * g.plane;
+    g.imgX = q.C * q.H * q.W; g.imgY = q.O * g.plane; g.rowY = g.plane;
     g.bytesX = (unsigned)(4 * (size_t)q.B * g.imgX); g.bytesY = (unsigned)(4 * (size_t)q.B * g.imgY);
     g.dplane = div_of(g.plane); g.dow = div_of(g.oW);
     return g;
@@ -1010,16 +1027,27 @@ static FilterPlan plan_filter(const ConvF32& q)
     pl.splits = ceil_div_i(g.K, g.kchunk);
     return pl;
 }
-// The small backward-filter: enough ranges for two blocks per CU, none below 128 pixels (two rounds of a wave's loads).
+// What the small filter kernel runs of a pass: backward-filter, or backward-data of a spanning kernel as a sum over "pixels" o,
+// dx[b][k] = sum_o dy[b][o] w[o][k], with the images as rows of q and the weights of an output as columns of p.
+static FilterGemm small_gemm(const ConvF32& q, int pass)
+{
+    if (pass == PASS_BWD_FILTER) return filter_gemm(q);
+    FilterGemm g = {};
+    g.P = q.C * q.kH * q.kW; g.Q = q.B; g.K = q.O;
+    g.C = g.P; g.H = g.W = g.kW = g.kH = g.s_y = g.s_x = g.oW = g.plane = 1;
+    g.imgX = g.P; g.imgY = 1; g.rowY = q.O;
+    g.dplane = div_of(1); g.dow = div_of(1);
+    return g;
+}
+// The small kernel: enough ranges for two blocks per CU, none below 128 pixels (two rounds of a wave's loads).
 static int small_filter_splits(const FilterGemm& g)
 {
     const long tiles = (long)ceil_div_i(g.P, 16) * ceil_div_i(g.Q, 16);
     return (int)std::max(1L, std::min<long>(512 / tiles, g.K / 128));
 }
 // (a workspace too small for the partial results: one range)
-static int run_small_filter(const ConvF32& q, const float* x, const float* dy, float beta, float* out, double* ws, size_t ws_bytes, hipStream_t st)
+static int run_small_filter(FilterGemm g, const float* x, const float* dy, float beta, float* out, double* ws, size_t ws_bytes, hipStream_t st)
 {
-    FilterGemm g = filter_gemm(q);
     const size_t n = (size_t)g.Q * g.P;
     int splits = small_filter_splits(g);
     if (splits * n * sizeof(double) > ws_bytes || ((size_t)ws & 7)) splits = 1;
@@ -1174,7 +1202,10 @@ int n2d2hip_conv2d_f32_backward_data(const n2d2hip_conv_desc* desc, int B, int H
     const int st = make_conv(desc, B, H, W, true, &q, "n2d2hip_conv2d_f32_backward_data");
     if (st != N2D2HIP_OK) return st;
     N2D2HIP_REQUIRE(w && diff_y && diff_x, N2D2HIP_ERR_INVALID, "n2d2hip_conv2d_f32_backward_data: null pointer");
-    if (f32_path(q, PASS_BWD_DATA) == F32_PATH_GEMM) {
+    const int path = f32_path(q, PASS_BWD_DATA);
+    if (path == F32_PATH_SMALL)
+        return run_small_filter(small_gemm(q, PASS_BWD_DATA), w, diff_y, beta, diff_x, (double*)workspace, workspace ? workspace_bytes : 0, (hipStream_t)stream);
+    if (path == F32_PATH_GEMM) {
         float* ws = (float*)workspace;
         const size_t nws = workspace ? workspace_bytes / sizeof(float) : 0;
         if (spans_input(q)) {
@@ -1196,7 +1227,7 @@ size_t n2d2hip_conv2d_f32_workspace_bytes(const n2d2hip_conv_desc* desc, int B, 
     for (int pass : {PASS_FWD, PASS_BWD_DATA, PASS_BWD_FILTER}) {
         const int path = f32_path(q, pass);
         if (path == F32_PATH_SMALL) {
-            const FilterGemm g = filter_gemm(q);
+            const FilterGemm g = small_gemm(q, pass);
             const int splits = small_filter_splits(g);
             need = std::max(need, splits > 1 ? splits * (size_t)g.Q * g.P * 2 : 0);
         } else if (path == F32_PATH_GEMM) {
@@ -1220,7 +1251,7 @@ int n2d2hip_conv2d_f32_backward_filter(const n2d2hip_conv_desc* desc, int B, int
     N2D2HIP_REQUIRE(nw < ((size_t)1 << 31), N2D2HIP_ERR_INVALID, "n2d2hip_conv2d_f32_backward_filter: too many weights");
     const int path = f32_path(q, PASS_BWD_FILTER);
     if (path == F32_PATH_SMALL)
-        return run_small_filter(q, x, diff_y, beta, diff_w, (double*)workspace, workspace ? workspace_bytes : 0, (hipStream_t)stream);
+        return run_small_filter(small_gemm(q, PASS_BWD_FILTER), x, diff_y, beta, diff_w, (double*)workspace, workspace ? workspace_bytes : 0, (hipStream_t)stream);
     if (path == F32_PATH_GEMM) {
         int pass = PASS_BWD_FILTER;
         const bool fc = spans_input(q);

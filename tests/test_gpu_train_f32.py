@@ -309,6 +309,31 @@ def test_filter_gradient_of_a_spanning_layer_is_added_in_double(g, case, path, w
     assert (np.abs(g.host(dw).astype(np.longdouble) - want) <= bound).all()
 
 
+# The longest float sum `terms` that the layer's convolution has (0: sums in double); rounding a float loses 2.53e-8 in the
+# root mean square (mantissas spread over a logarithm), and of the partial sums of L equal terms the i-th is sqrt(i / L) of the
+# last: sqrt(1 + L / 2) such losses.
+@pytest.mark.parametrize("case,terms", [((8, 32, 8, 8, 700), 0), ((100, 3, 2, 1, 40000), 0), ((17, 65, 7, 5, 300), 0), ((128, 512, 2, 2, 1000), 66),
+                                        ((64, 256, 7, 7, 512), 34), ((32, 512, 7, 7, 1000), 71)])
+@pytest.mark.parametrize("workspace", [True, False])
+def test_data_gradient_of_a_spanning_layer(g, case, terms, workspace):
+    B, Cn, H, W, O = case
+    print("spanning data gradient", case, workspace, flush=True)
+    rng = np.random.default_rng(sum(case))
+    w, dy = rng.normal(size=(O, Cn, H, W)).astype(np.float32), rng.normal(size=(B, O)).astype(np.float32)
+    want = dy.astype(np.float64) @ w.astype(np.float64).reshape(O, -1)
+    d = g.capi.ConvDesc(Cn, O, W, H, 1, 1, 0, 0, 0, 0, 1, 1, 1, 0, 0)
+    need = int(g.lib.n2d2hip_conv2d_f32_workspace_bytes(C.byref(d), B, H, W)) if workspace else 0
+    ws = g.torch_.empty(max(need, 4), dtype=g.torch_.uint8, device="cuda")
+    w_, dy_ = g.dev(w), g.dev(dy)
+    dx = g.torch_.ones(want.shape, dtype=g.torch_.float32, device="cuda")
+    g.check(g.lib.n2d2hip_conv2d_f32_backward_data(C.byref(d), B, H, W, w_.data_ptr(), dy_.data_ptr(), 0.0, dx.data_ptr(),
+                                                   ws.data_ptr() if need else None, need, g.sp()))
+    err = np.abs(g.host(dx) - want)
+    mag = np.abs(dy.astype(np.float64)) @ np.abs(w.astype(np.float64)).reshape(O, -1)
+    assert (err <= np.abs(want) * 2.0 ** -24 + mag * max(terms * 2.0 ** -24, O * 2.0 ** -52)).all()
+    assert np.linalg.norm(err) <= 1.1 * 2.53e-8 * np.sqrt(1 + terms / 2) * np.linalg.norm(want)
+
+
 # B, C, H, W, k, stride, pad: strips of four with every remainder, rows shorter than a strip or a window, windows past both
 # ends of the tensor, both parities of the padding at stride 2, blocks of 256 and of 1024 threads, outputs wider than the input
 DEPTHWISE = [(1, 1, 1, 1, 3, 1, 1), (2, 3, 2, 3, 3, 1, 1), (1, 1, 3, 3, 3, 1, 0), (3, 2, 5, 6, 3, 2, 0), (2, 5, 9, 7, 3, 2, 1), (1, 4, 6, 9, 3, 2, 2),
