@@ -857,11 +857,11 @@ static int pass_ranges(long P, int Q, long K)
 //   forward          y[b][o] = sum_k x[b][k] w[o][k]     the filter pass of pixels k between "channels" w[o] and "outputs" x[b]
 //   backward data    dx[b][k] = sum_o dy[b][o] w[o][k]   the forward pass over one "image" w of O channels and K pixels
 //   backward filter  dw[o][k] = sum_b dy[b][o] x[b][k]   the data pass over one "image" x of B channels and K pixels
-// Backward data runs at least as many ranges as the convolution itself would, so that no float sum is longer.
+// Forward and backward data run at least as many ranges as the convolution itself would, so that no float sum is longer.
 static ConvF32 product_of(const ConvF32& q, int pass, int* as_pass)
 {
     const int K = q.C * q.H * q.W, T = q.H * q.W;
-    const int ranges = pass == PASS_BWD_DATA && T > 1 && T <= 64 ? pass_ranges((long)q.B * T, q.C, (long)q.O * T) : 0;
+    const int ranges = pass == PASS_FWD ? pass_ranges(q.B, q.O, K) : pass == PASS_BWD_DATA && T > 1 && T <= 64 ? pass_ranges((long)q.B * T, q.C, (long)q.O * T) : 0;
     *as_pass = pass == PASS_FWD ? PASS_BWD_FILTER : pass == PASS_BWD_DATA ? PASS_FWD : PASS_BWD_DATA;
     return ConvF32{1, q.O, 1, K, q.B, 1, K, 1, 1, q.O, 1, 1, 0, 0, 0, 0, 1, 1, 0, q.choice, ranges};
 }
@@ -1023,7 +1023,7 @@ static FilterPlan plan_filter(const ConvF32& q)
     // blocks; many: three blocks per tile or six per CU)
     long splits = tiles <= 256 ? (pl.small_q ? 512 : 1024) / tiles : std::max(1L, (1535 + tiles) / tiles);
     splits = std::min<long>(splits, std::max(1, g.K / (4 * FK)));
-    g.kchunk = round_up((int)((g.K + splits - 1) / splits), FK);
+    g.kchunk = q.ranges > splits ? std::max(g.K / q.ranges / FK * FK, FK) : round_up((int)((g.K + splits - 1) / splits), FK);
     pl.splits = ceil_div_i(g.K, g.kchunk);
     return pl;
 }

@@ -334,6 +334,22 @@ def test_data_gradient_of_a_spanning_layer(g, case, terms, workspace):
     assert np.linalg.norm(err) <= 1.1 * 2.53e-8 * np.sqrt(1 + terms / 2) * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("case,terms", [((32, 512, 7, 7, 1000), 272), ((64, 256, 6, 6, 2048), 256), ((48, 300, 5, 7, 500), 256)])
+def test_forward_sums_of_a_spanning_layer_are_no_longer_than_the_convolutions(g, case, terms):
+    B, Cn, H, W, O = case
+    print("spanning forward sums", case, flush=True)
+    rng = np.random.default_rng(sum(case))
+    x, w = rng.normal(size=(B, Cn, H, W)).astype(np.float32), rng.normal(size=(O, Cn, H, W)).astype(np.float32)
+    want = x.astype(np.float64).reshape(B, -1) @ w.astype(np.float64).reshape(O, -1).T
+    d = g.capi.ConvDesc(Cn, O, W, H, 1, 1, 0, 0, 0, 0, 1, 1, 1, 0, 0)
+    need = int(g.lib.n2d2hip_conv2d_f32_workspace_bytes(C.byref(d), B, H, W))
+    ws = g.torch_.empty(need, dtype=g.torch_.uint8, device="cuda")
+    w_, x_ = g.dev(w), g.dev(x)
+    y = g.torch_.ones(want.shape, dtype=g.torch_.float32, device="cuda")
+    g.check(g.lib.n2d2hip_conv2d_f32_forward(C.byref(d), B, H, W, x_.data_ptr(), w_.data_ptr(), None, 0.0, y.data_ptr(), ws.data_ptr(), need, g.sp()))
+    assert np.linalg.norm(g.host(y) - want) <= 1.1 * 2.53e-8 * np.sqrt(1 + terms / 2) * np.linalg.norm(want)
+
+
 # B, C, H, W, k, stride, pad: strips of four with every remainder, rows shorter than a strip or a window, windows past both
 # ends of the tensor, both parities of the padding at stride 2, blocks of 256 and of 1024 threads, outputs wider than the input
 DEPTHWISE = [(1, 1, 1, 1, 3, 1, 1), (2, 3, 2, 3, 3, 1, 1), (1, 1, 3, 3, 3, 1, 0), (3, 2, 5, 6, 3, 2, 0), (2, 5, 9, 7, 3, 2, 1), (1, 4, 6, 9, 3, 2, 2),
