@@ -16,7 +16,8 @@
 //  * 3x3 kernels, forward and at stride 1 backward, keep a lane's nine offsets in registers, so that a load costs no vector
 //    instruction; 1x1 kernels and strided backward-data run K over chunks of 16 channels at one tap, so that the test whether
 //    the tap lies inside the input is made once per step.  A small kernel lays the weights out for both first.  Any other
-//    forward kernel, and short passes, test every load.
+//    forward kernel, and short passes, test every load.  Kernels of more than 31 rows and columns, up to 64 taps (time series),
+//    run on variants of the chunk, pixel and filter kernels that hold a bit per tap instead of one per row and column.
 //  * backward-data of a strided convolution runs one residue class of input pixels at a time: the taps of a class form a
 //    dense stride-1 convolution of dy, so no tap is tried that cannot hit (a 3x3 of stride 2: 9 taps for 4 classes, where
 //    trying all of them is 36).
@@ -30,6 +31,8 @@
 //   64 -> 64, 3x3, 56 x 56, batch 64             236 / 284 / 263    149 / 157 / 180   (15 GFLOP: 99, 94, 82 TFLOP/s of 154)
 //   128 -> 256, 3x3 stride 2, 27 x 27, batch 33   80 / 277 /  76     55 /  53 /  58
 //   a layer spanning its input, 16384 -> 10, 64  2632 /  27 / 222    116 /   7 /   8
+//   64 -> 64, 1 x 40, 1 x 512, batch 32            94 / 110 /  98     86 /  82 /  70
+//   128 -> 128, 1 x 64, 1 x 256, batch 16         120 / 134 / 124    113 / 106 / 104
 // A CU takes whole tiles, so the last round costs its share: 64 -> 64 on 56 x 56 at batch 64 is 12.25 tiles for each.
 #pragma once
 
@@ -128,16 +131,57 @@ __device__ __forceinline__ bool pixel_tile(const PixelGemm& g, int* tile, int* q
     return *tile < g.ptiles;
 }
 
-// A lane's pixel: byte offset of its tap (0, 0) (against the moved base), and which taps lie inside the source: bit j: tap
-// column j, bit nx + i: tap row i.
-__device__ __forceinline__ void pixel_source(const PixelGemm& g, const PixelClass& c, int p, unsigned* voff, unsigned* mask)
+// Which taps lie inside the source.  Bit j: tap column j, bit nx + i: tap row i; bit 31 is never set.  LONG, for kernels of more
+// rows and columns than that (1 x 40): a bit for each of up to 64 taps.
+template <bool LONG>
+struct TapMask {
+    unsigned m[LONG ? 2 : 1];
+    // `bit`: LONG: bit t of its word, or 0 past the range; else the tap's column and row, and bit 31 past the range
+    __device__ __forceinline__ bool inside(int t, unsigned bit) const
+    {
+        if (LONG) return ((t & 32 ? m[LONG] : m[0]) & bit) != 0;
+        return (m[0] & bit) == bit;
+    }
+};
+// The first tap of each of a kernel's rows, and of the taps those in columns xl .. xh - 1 and rows yl .. yh - 1.
+__device__ __forceinline__ unsigned long long long_rows(int ny, int nx)
+{
+    unsigned long long m = 0;
+    for (int i = 0; i < ny; ++i) m |= 1ull << (i * nx);
+    return m;
+}
+__device__ __forceinline__ unsigned long long long_taps(int xl, int xh, int yl, int yh, int nx, unsigned long long rows)
+{
+    auto below = [](int n) { return n >= 64 ? ~0ull : (1ull << n) - 1; };
+    return ((below(xh) & ~below(xl)) * rows) & below(yh * nx) & ~below(yl * nx);
+}
+// (`left`: negative past the range)
+template <bool LONG>
+__device__ __forceinline__ unsigned tap_test(int t, int tap_bit, int left)
+{
+    if (LONG) return (1u << (t & 31)) & ~(unsigned)(left >> 31);
+    return (unsigned)__builtin_amdgcn_readlane(tap_bit, t) | ((unsigned)left & 0x80000000u);
+}
+
+// A lane's pixel: byte offset of its tap (0, 0) (against the moved base), and its taps inside the source.
+template <bool LONG>
+__device__ __forceinline__ void pixel_source(const PixelGemm& g, const PixelClass& c, int p, unsigned* voff, TapMask<LONG>* mask)
 {
     const int pp = p < c.P ? p : 0;
     const int b = div_f32(pp, c.ghw), rem = pp - b * c.gHW;
     const int py = div_f32(rem, c.gw), px = rem - py * c.gW;
     *voff = 4u * (unsigned)(b * g.Ch * g.planeS + py * g.sy * g.Ws + px * g.sx);
-    unsigned m = 0;
     const int ny = c.nT > 0 ? div_f32(c.nT, c.nxd) : 0;
+    if (LONG) {
+        const int x = px * g.sx + c.x0, y = py * g.sy + c.y0;
+        auto first = [&](int v, int size, int n) { return min(max(g.d > 0 ? -v : v - size + 1, 0), n); };
+        auto end = [&](int v, int size, int n) { return min(max(g.d > 0 ? size - v : v + 1, 0), n); };
+        const unsigned long long m = long_taps(first(x, g.Ws, c.nx), end(x, g.Ws, c.nx), first(y, g.Hs, ny), end(y, g.Hs, ny), c.nx, long_rows(ny, c.nx));
+        mask->m[0] = p < c.P ? (unsigned)m : 0u;
+        mask->m[LONG] = p < c.P ? (unsigned)(m >> 32) : 0u;
+        return;
+    }
+    unsigned m = 0;
     for (int j = 0; j < c.nx; ++j) {
         const int x = px * g.sx + c.x0 + j * g.d;
         m |= (unsigned)(x >= 0 && x < g.Ws) << j;
@@ -146,7 +190,7 @@ __device__ __forceinline__ void pixel_source(const PixelGemm& g, const PixelClas
         const int y = py * g.sy + c.y0 + i * g.d;
         m |= (unsigned)(y >= 0 && y < g.Hs) << (c.nx + i);
     }
-    *mask = p < c.P ? m : 0u;
+    mask->m[0] = p < c.P ? m : 0u;
 }
 
 // The products of a wave's 32 x 32 tile from one stage: [16 k][PT pixels] and behind it [QT][16 k], the even k of a row in
@@ -272,7 +316,7 @@ __global__ __launch_bounds__(256) void conv_f32_lay_weights_kernel(const float* 
 }
 
 // Forward and backward-data with K in chunks of 16 channels at one tap.
-template <int WQ, int WP, int S>
+template <int WQ, int WP, int S, bool LONG>
 __global__ __launch_bounds__(256) void conv_f32_chunk_kernel(PixelGemm g, const float* __restrict__ srcX, const float* __restrict__ wt,
                                                              const float* __restrict__ bias, float beta, float* __restrict__ out, size_t partial)
 {
@@ -294,7 +338,8 @@ __global__ __launch_bounds__(256) void conv_f32_chunk_kernel(PixelGemm g, const 
     const int nT = c.nT, nchunks = (g.Ch + GK - 1) / GK;
     const __amdgpu_buffer_rsrc_t rsrcX = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(srcX) - c.bias, 0, g.bytesX + 4u * c.bias, 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrcW = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(wt), 0, nchunks * g.T * g.qpad * GK * 4, 0x00020000);
-    unsigned voff[PH], mask[PH], mv[PH];
+    unsigned voff[PH], mv[PH];
+    TapMask<LONG> mask[PH];
 #pragma unroll
     for (int h = 0; h < PH; ++h)
         pixel_source(g, c, p0 + h * 64 + lane, &voff[h], &mask[h]);
@@ -302,7 +347,7 @@ __global__ __launch_bounds__(256) void conv_f32_chunk_kernel(PixelGemm g, const 
     // in the weights.
     const int tl = min(lane, max(nT - 1, 0)), ti = div_f32(tl, c.nxd), tj = tl - ti * c.nx;
     const int tap_off = 4 * (c.soff0 + ti * c.stepy + tj * c.stepx);
-    const int tap_bit = (1 << tj) | (1 << (c.nx + ti));
+    const int tap_bit = LONG ? 0 : (1 << tj) | (1 << (c.nx + ti));
     const int tap_w = ((c.ty0 + ti * g.osy) * g.kW + c.tx0 + tj * g.osx) * g.qpad * (GK * 4);
     const int plane4 = g.planeS * 4;
     PixelTile<PT> tl_acc;
@@ -317,10 +362,10 @@ __global__ __launch_bounds__(256) void conv_f32_chunk_kernel(PixelGemm g, const 
         int soff = 0, left = nsteps;
         auto load_part = [&](int part) {
             if (part == 0) {
-                const unsigned bit = (unsigned)__builtin_amdgcn_readlane(tap_bit, t) | (left > 0 ? 0u : 0x80000000u);    // (bit 31: never valid)
+                const unsigned bit = tap_test<LONG>(t, tap_bit, left - 1);
                 soff = ch_off + __builtin_amdgcn_readlane(tap_off, t);
 #pragma unroll
-                for (int h = 0; h < PH; ++h) mv[h] = (mask[h] & bit) == bit ? voff[h] : F32_OOB;
+                for (int h = 0; h < PH; ++h) mv[h] = mask[h].inside(t, bit) ? voff[h] : F32_OOB;
             }
             if (part < 4) {
 #pragma unroll
@@ -411,12 +456,13 @@ __global__ __launch_bounds__(256) void conv_f32_3x3_kernel(PixelGemm g, const fl
     unsigned tap[PH][9];
 #pragma unroll
     for (int h = 0; h < PH; ++h) {
-        unsigned voff, mask;
+        unsigned voff;
+        TapMask<false> mask;
         pixel_source(g, c, p0 + h * 64 + lane, &voff, &mask);
 #pragma unroll
         for (int t = 0; t < 9; ++t) {
             const unsigned bit = (1u << t % 3) | (8u << t / 3);
-            tap[h][t] = (mask & bit) == bit ? voff + 4 * (c.soff0 + t / 3 * c.stepy + t % 3 * c.stepx) : F32_OOB;
+            tap[h][t] = mask.inside(t, bit) ? voff + 4 * (c.soff0 + t / 3 * c.stepy + t % 3 * c.stepx) : F32_OOB;
         }
     }
     const int plane4 = g.planeS * 4, wstep = g.qpad * W33 * 4;
@@ -610,7 +656,7 @@ __global__ __launch_bounds__(64) void conv_f32_chain_kernel(int B, int O, int K,
 }
 
 // Forward (BWD = false) and backward-data with K in the tensors' own order, (channel, tap).
-template <bool BWD, int WQ, int WP, int S>
+template <bool BWD, int WQ, int WP, int S, bool LONG>
 __global__ __launch_bounds__(256) void conv_f32_pixel_kernel(PixelGemm g, const float* __restrict__ srcX, const float* __restrict__ srcW,
                                                              const float* __restrict__ bias, float beta, float* __restrict__ out, size_t partial)
 {
@@ -632,7 +678,8 @@ __global__ __launch_bounds__(256) void conv_f32_pixel_kernel(PixelGemm g, const 
     const int nT = c.nT, K = g.Ch * nT;
     const __amdgpu_buffer_rsrc_t rsrcX = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(srcX) - c.bias, 0, g.bytesX + 4u * c.bias, 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrcW = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(srcW), 0, g.bytesW, 0x00020000);
-    unsigned voff[PH], mask[PH], wbase[WJ];
+    unsigned voff[PH], wbase[WJ];
+    TapMask<LONG> mask[PH];
 #pragma unroll
     for (int h = 0; h < PH; ++h)
         pixel_source(g, c, p0 + h * 64 + lane, &voff[h], &mask[h]);
@@ -645,7 +692,7 @@ __global__ __launch_bounds__(256) void conv_f32_pixel_kernel(PixelGemm g, const 
     // Tap t of this class lives in lane t; the running (channel, tap) of each of the wave's rows is scalar.
     const int tl = min(lane, max(nT - 1, 0)), ti = div_f32(tl, c.nxd), tj = tl - ti * c.nx;
     const int tap_off = 4 * (c.soff0 + ti * c.stepy + tj * c.stepx);
-    const int tap_bit = (1 << tj) | (1 << (c.nx + ti));
+    const int tap_bit = LONG ? 0 : (1 << tj) | (1 << (c.nx + ti));
     PixelTile<PT> tl_acc;
     tl_acc.init((unsigned)(unsigned long)(__attribute__((address_space(3))) float*)smem, wq, wp, lane);
     for (int z = blockIdx.z * g.nz; z < (int)(blockIdx.z + 1) * g.nz; ++z) {
@@ -667,12 +714,11 @@ __global__ __launch_bounds__(256) void conv_f32_pixel_kernel(PixelGemm g, const 
             if (part < 4) {
                 const int t = row_t[part];
                 const int soff = row_ch[part] + __builtin_amdgcn_readlane(tap_off, t);
-                // (bit 31: never valid)
-                const unsigned bit = (unsigned)__builtin_amdgcn_readlane(tap_bit, t) | ((unsigned)(row_left - 1 - part) & 0x80000000u);
+                const unsigned bit = tap_test<LONG>(t, tap_bit, row_left - 1 - part);
 #pragma unroll
                 for (int h = 0; h < PH; ++h)
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcX, (lds_ptr_t)((char*)smem + xdst + ((wave * 4 + part) * PT + h * 64) * 4), 4,
-                                                             (mask[h] & bit) == bit ? voff[h] : F32_OOB, soff, 0, 0);
+                                                             mask[h].inside(t, bit) ? voff[h] : F32_OOB, soff, 0, 0);
                 const int tn = t + adv_t;
                 const bool carry = tn >= nT;
                 row_t[part] = carry ? tn - nT : tn;
@@ -723,7 +769,7 @@ __global__ __launch_bounds__(256) void conv_f32_pixel_kernel(PixelGemm g, const 
 
 // Backward-filter: both operands hold consecutive k (pixels), rows of 32 of them in LDS, two rows to a load.  Row pairs are
 // 272 bytes apart, so that 8 rows' 16-byte reads fall into different banks.
-template <int WQ, int WP, int S>
+template <int WQ, int WP, int S, bool LONG>
 __global__ __launch_bounds__(256) void conv_f32_filter_kernel(FilterGemm g, const float* __restrict__ srcX, const float* __restrict__ srcY,
                                                               float* __restrict__ out)
 {
@@ -746,21 +792,26 @@ __global__ __launch_bounds__(256) void conv_f32_filter_kernel(FilterGemm g, cons
     const __amdgpu_buffer_rsrc_t rsrcY = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(srcY), 0, g.bytesY, 0x00020000);
 
     // ---- loader state: this lane's half of the row pairs its wave loads
-    unsigned poff[PJ], pbit[PJ], qoff[QJ];
+    typedef std::conditional_t<LONG, unsigned long long, unsigned> Mask;
+    unsigned poff[PJ], qoff[QJ];
+    Mask pbit[PJ];
     const int kHW = g.kH * g.kW;
+    const unsigned long long rows = LONG ? long_rows(g.kH, g.kW) : 0;
 #pragma unroll
     for (int j = 0; j < PJ; ++j) {
         const int p = p0 + 2 * (wave + 4 * j) + lh, pp = min(p, g.P - 1);
         const int ch = pp / kHW, t = pp - ch * kHW, ty = t / g.kW, tx = t - ty * g.kW;
         poff[j] = 4u * (unsigned)(ch * g.H * g.W + ty * g.W + tx);
-        pbit[j] = p < g.P ? (1u << tx) | (1u << (g.kW + ty)) : 0x80000000u;
+        if (LONG) pbit[j] = p < g.P ? (Mask)1 << t : 0;
+        else pbit[j] = p < g.P ? (1u << tx) | (1u << (g.kW + ty)) : 0x80000000u;
     }
 #pragma unroll
     for (int j = 0; j < QJ; ++j) {
         const int q = q0 + 2 * (wave + 4 * j) + lh;
         qoff[j] = q < g.Q ? 4u * (unsigned)(q * g.plane) : F32_OOB;
     }
-    unsigned xo = 0, yo = 0, pmask = 0, dst_bytes = 0;
+    unsigned xo = 0, yo = 0, dst_bytes = 0;
+    Mask pmask = 0;
     bool kv = false;
     int k_next = kbeg + l32;
     auto locate = [&]() {                        // this lane's pixel of the step to load next
@@ -773,15 +824,19 @@ __global__ __launch_bounds__(256) void conv_f32_filter_kernel(FilterGemm g, cons
         yo = 4u * (unsigned)(img * g.imgY + rem);
         // bits lo .. hi - 1 of the columns, then of the rows, that lie inside the input
         const int xl = min(max(-ix0, 0), g.kW), xh = min(max(g.W - ix0, 0), g.kW), yl = min(max(-iy0, 0), g.kH), yh = min(max(g.H - iy0, 0), g.kH);
-        const unsigned mx = ((1u << xh) - 1u) & ~((1u << xl) - 1u), my = ((1u << yh) - 1u) & ~((1u << yl) - 1u);
-        pmask = kv ? mx | (my << g.kW) : 0u;
+        if (LONG) {
+            pmask = kv ? (Mask)long_taps(xl, xh, yl, yh, g.kW, rows) : 0;
+        } else {
+            const unsigned mx = ((1u << xh) - 1u) & ~((1u << xl) - 1u), my = ((1u << yh) - 1u) & ~((1u << yl) - 1u);
+            pmask = kv ? (Mask)(mx | (my << g.kW)) : 0;
+        }
         k_next += FK;
     };
     auto issue_part = [&](int part) {            // a quarter of a stage's loads
 #pragma unroll
         for (int j = part * PJ / 4; j < (part + 1) * PJ / 4; ++j)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcX, (lds_ptr_t)((char*)smem + dst_bytes + (wave + 4 * j) * PAIR * 4), 4,
-                                                     (pmask & pbit[j]) == pbit[j] ? xo + poff[j] : F32_OOB, 0, 0, 0);
+                                                     (LONG ? (pmask & pbit[j]) != 0 : (pmask & pbit[j]) == pbit[j]) ? xo + poff[j] : F32_OOB, 0, 0, 0);
 #pragma unroll
         for (int j = part * QJ / 4; j < (part + 1) * QJ / 4; ++j)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcY, (lds_ptr_t)((char*)smem + dst_bytes + (PT / 2 + wave + 4 * j) * PAIR * 4), 4,

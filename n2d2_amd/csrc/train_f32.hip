@@ -732,8 +732,8 @@ static bool spans_input(const ConvF32& q)
 enum { PASS_FWD = 0, PASS_BWD_DATA = 1, PASS_BWD_FILTER = 2 };
 enum { F32_PATH_DIRECT, F32_PATH_GEMM, F32_PATH_SMALL };
 
-// More than the pixel and filter kernels have lanes and mask bits for
-static bool many_taps(const ConvF32& q) { return q.kH + q.kW > 31 || q.kH * q.kW > 64; }
+// More than the pixel kernels have lanes and the filter kernel has mask bits for
+static bool many_taps(const ConvF32& q) { return (long)q.kH * q.kW > 64; }
 
 // The kernels of a pass.  The matrix cores serve ungrouped convolutions without dilation; the direct kernels keep the rest
 // (depthwise, dilated) and the forward sums below 2e7 flops or of kernels over 64 taps, which stay in the reference's order
@@ -749,7 +749,7 @@ static int f32_path(const ConvF32& q, int pass)
     if ((size_t)q.B * q.C * q.H * q.W >= lim || (size_t)q.B * q.O * q.oH * q.oW >= lim || (size_t)q.O * q.C * q.kH * q.kW >= lim
         || (many_taps(q) && !spans_input(q)))
         return F32_PATH_DIRECT;
-    if (pass == PASS_BWD_FILTER && q.kH * q.kW > 64) return F32_PATH_SMALL;
+    if (pass == PASS_BWD_FILTER && many_taps(q)) return F32_PATH_SMALL;
     const double flops = 2.0 * q.B * q.O * q.oH * q.oW * q.C * q.kH * q.kW;
     const bool forced = q.choice & N2D2HIP_KERNEL_F32_GEMM, small = flops < 2.0e7;
     // As a convolution the K of a spanning layer's backward-data runs over all taps of an output, one of which is not zero: few
@@ -757,7 +757,7 @@ static int f32_path(const ConvF32& q, int pass)
     // 64 x 4 x 4 <- 256: 2.5e-8 from 64 bits and 10 us; convolution 7.7e-8, 41 us; product in float 2.9e-7, 14 us) and beyond
     // takes as many ranges as the convolution would (128 images, 512 x 2 x 2 <- 1000: 1.5e-7 and 26 us; in double 36; convolution
     // 1.5e-7, 64; 64 images, 512 x 7 x 7 <- 4096: 179 us, in double 1019, convolution 9566).
-    if (pass == PASS_BWD_DATA && (forced || !small) && flops < 5.0e8 && q.kH * q.kW > 1 && q.kH * q.kW <= 64 && spans_input(q))
+    if (pass == PASS_BWD_DATA && (forced || !small) && flops < 5.0e8 && !many_taps(q) && q.kH * q.kW > 1 && spans_input(q))
         return F32_PATH_SMALL;
     if (forced) return F32_PATH_GEMM;
     if (pass == PASS_FWD) return small || many_taps(q) ? F32_PATH_DIRECT : F32_PATH_GEMM;
@@ -871,6 +871,7 @@ struct PixelPlan {
     bool small_q;              // tiles of 32 q x 128 pixels instead of 64 x 64
     int splits;                // K ranges that leave partial results
     int kind;                  // PIXELS_*
+    bool many;                 // a class has more tap rows and columns than a mask of 31 bits
     PixelGemm g;
 };
 
@@ -933,7 +934,7 @@ static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass>
     // tile shape
     long P = 0, kmax = 0;
     const int nchunks = ceil_div_i(g.Ch, GK);
-    for (const PixelClass& c : cls) { P += c.P; kmax = std::max<long>(kmax, (long)(kind == PIXELS_CHUNK && !fwd ? nchunks * GK : g.Ch) * c.nT); }
+    for (const PixelClass& c : cls) { P += c.P; kmax = std::max<long>(kmax, (long)(kind == PIXELS_CHUNK && (!fwd || T > 1) ? nchunks * GK : g.Ch) * c.nT); }
     // (64 x 64 tiles, four to a CU, lost at most 4 % to the best of 32 x 128, 64 x 128 and 128 x 128 on every shape with Q
     // over 32 that was timed, and gained up to 70 % where the larger tiles are few)
     pl.small_q = g.Q <= 32;
@@ -946,6 +947,7 @@ static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass>
     g.nclass = (int)cls.size();
     for (int i = 0; i < g.nclass; ++i) {
         cls[i].tile0 = (int)tiles;
+        pl.many = pl.many || cls[i].nx + (cls[i].nT > 0 ? cls[i].nT / cls[i].nx : 0) > 31;
         tiles += ceil_div_i(cls[i].P, PT);
         g.c[i] = cls[i];
     }
@@ -956,7 +958,8 @@ static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass>
     long splits;
     if (fwd) {
         // The ranges of a forward sum follow from its sizes alone: with another order of additions the quantizer behind it would
-        // give another level now and then.  With a block for every CU it takes all of them.
+        // give another level now and then.  With a block for every CU it takes all of them (long kernels: with two; 64 -> 64,
+        // 1 x 31, 256 tiles: 102 us with one, 82 with partial results).
         splits = pass_ranges(P, g.Q, kmax);
     } else {
         // where the tiles do not fill the chip twice; none below four steps
@@ -965,7 +968,7 @@ static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass>
     }
     g.kchunk = std::max(q.ranges > splits ? (int)(kmax / q.ranges) / GK * GK : round_up((int)((kmax + splits - 1) / splits), GK), GK);
     pl.splits = std::max(1, ceil_div_i(kmax, g.kchunk));
-    if (fwd && blocks >= 256) {
+    if (fwd && blocks >= (pl.many ? 512 : 256)) {
         g.nz = pl.splits;
         pl.splits = 1;
     }
@@ -983,13 +986,17 @@ static void launch_pixels(PixelPlan& pl, int splits, const float* x, const float
         else hipLaunchKernelGGL((conv_f32_3x3_kernel<2, 2>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
         return;
     }
-    if (pl.kind == PIXELS_CHUNK) {
-        if (pl.small_q) hipLaunchKernelGGL((conv_f32_chunk_kernel<1, 4, 3>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
-        else hipLaunchKernelGGL((conv_f32_chunk_kernel<2, 2, 3>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
-        return;
-    }
-    if (pl.small_q) hipLaunchKernelGGL((conv_f32_pixel_kernel<BWD, 1, 4, 3>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
-    else hipLaunchKernelGGL((conv_f32_pixel_kernel<BWD, 2, 2, 3>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
+    const auto run = [&](auto long_) {
+        constexpr bool LONG = decltype(long_)::value;
+        if (pl.kind == PIXELS_CHUNK) {
+            if (pl.small_q) hipLaunchKernelGGL((conv_f32_chunk_kernel<1, 4, 3, LONG>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
+            else hipLaunchKernelGGL((conv_f32_chunk_kernel<2, 2, 3, LONG>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
+            return;
+        }
+        if (pl.small_q) hipLaunchKernelGGL((conv_f32_pixel_kernel<BWD, 1, 4, 3, LONG>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
+        else hipLaunchKernelGGL((conv_f32_pixel_kernel<BWD, 2, 2, 3, LONG>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
+    };
+    pl.many ? run(std::true_type{}) : run(std::false_type{});
 }
 
 static unsigned reduce_grid(size_t n) { return (unsigned)std::min<size_t>((n + 63) / 64, 16384); }
@@ -1063,13 +1070,17 @@ static int run_small_filter(FilterGemm g, const float* x, const float* dy, float
 static void launch_filter(const FilterPlan& pl, const float* x, const float* dy, float* out, hipStream_t st)
 {
     const dim3 grid(ceil_div_i(pl.g.P, pl.small_q ? 128 : 64), ceil_div_i(pl.g.Q, pl.small_q ? 32 : 64), pl.splits);
-    if (pl.small_q) hipLaunchKernelGGL((conv_f32_filter_kernel<1, 4, 2>), grid, dim3(256), 0, st, pl.g, x, dy, out);
-    else hipLaunchKernelGGL((conv_f32_filter_kernel<2, 2, 2>), grid, dim3(256), 0, st, pl.g, x, dy, out);
+    const auto run = [&](auto long_) {
+        constexpr bool LONG = decltype(long_)::value;
+        if (pl.small_q) hipLaunchKernelGGL((conv_f32_filter_kernel<1, 4, 2, LONG>), grid, dim3(256), 0, st, pl.g, x, dy, out);
+        else hipLaunchKernelGGL((conv_f32_filter_kernel<2, 2, 2, LONG>), grid, dim3(256), 0, st, pl.g, x, dy, out);
+    };
+    pl.g.kH + pl.g.kW > 31 ? run(std::true_type{}) : run(std::false_type{});
 }
 
 // The order of K.  3x3 kernels, forward or at stride 1: four channels with their taps at a time.  Chunks of 16 channels at one
-// tap: 1x1 kernels, and backward-data, where padding the channels to them costs less than testing every load (about a
-// fifth).  Both lay the weights out first (a launch of 3 us: even at 3 to 7e8 flops).
+// tap: 1x1 kernels, kernels of more than 31 rows and columns (1 x 64, 128 -> 128: 138 -> 113 us) and backward-data, where padding
+// the channels to them costs less than testing every load (about a fifth).  Both lay the weights out first (a launch of 3 us: even at 3 to 7e8 flops).
 static int pixels_kind(const ConvF32& q, int pass)
 {
     const int ch = pass == PASS_FWD ? q.C : q.O, T = q.kH * q.kW;
@@ -1077,7 +1088,7 @@ static int pixels_kind(const ConvF32& q, int pass)
         return PIXELS_TAPS;
     if (q.kH == 3 && q.kW == 3 && (pass == PASS_FWD || (q.sx == 1 && q.sy == 1)) && round_up(ch, 4) * 5 <= ch * 7)
         return PIXELS_3X3;
-    return (pass == PASS_BWD_DATA || T == 1) && round_up(ch, GK) * 5 <= ch * 6 ? PIXELS_CHUNK : PIXELS_TAPS;
+    return (pass == PASS_BWD_DATA || T == 1 || q.kH + q.kW > 31) && round_up(ch, GK) * 5 <= ch * 6 ? PIXELS_CHUNK : PIXELS_TAPS;
 }
 static size_t laid_weights(const ConvF32& q, int pass, int kind)
 {

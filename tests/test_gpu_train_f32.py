@@ -350,6 +350,44 @@ def test_forward_sums_of_a_spanning_layer_are_no_longer_than_the_convolutions(g,
     assert np.linalg.norm(g.host(y) - want) <= 1.1 * 2.53e-8 * np.sqrt(1 + terms / 2) * np.linalg.norm(want)
 
 
+# B, C, H, W, O, kH, kW, stride, pad y, pad x: kernels of more rows and columns than a mask word has bits and at most 64 taps
+LONG = [(4, 20, 3, 90, 40, 1, 40, 1, 0, 0), (3, 17, 70, 5, 33, 64, 1, 1, 31, 0), (2, 16, 4, 100, 70, 2, 31, 1, 1, 15), (5, 12, 40, 9, 18, 32, 2, 1, 3, 1),
+        (2, 9, 1, 300, 35, 1, 64, 3, 0, 32), (6, 8, 1, 40, 12, 1, 40, 1, 0, 0), (2, 40, 65, 66, 30, 31, 1, 2, 15, 0), (33, 64, 1, 200, 64, 1, 33, 1, 0, 16),
+        (40, 60, 1, 200, 80, 1, 40, 1, 0, 0), (6, 30, 5, 120, 64, 2, 31, 1, 1, 15)]
+
+
+@pytest.mark.parametrize("path", [None, "gemm"])
+@pytest.mark.parametrize("case", LONG)
+def test_long_kernels_on_the_matrix_cores(g, case, path):
+    B, Cn, H, W, O, kH, kW, s, py, px = case
+    print("long kernel", case, path, flush=True)
+    t, F = g.torch_, g.torch_.nn.functional
+    rng = np.random.default_rng(sum(case))
+    x, w = rng.normal(size=(B, Cn, H, W)).astype(np.float32), rng.normal(size=(O, Cn, kH, kW)).astype(np.float32)
+
+    def passes(x_, w_, dy_):
+        x64, w64 = (t.from_numpy(v).double().requires_grad_() for v in (x_, w_))
+        y = F.conv2d(x64, w64, stride=s, padding=(py, px))
+        y.backward(t.from_numpy(dy_).double())
+        return [v.detach().numpy() for v in (y, x64.grad, w64.grad)]
+    dy = rng.normal(size=(B, O, (H + 2 * py - kH) // s + 1, (W + 2 * px - kW) // s + 1)).astype(np.float32)
+    want, mag = passes(x, w, dy), passes(np.abs(x), np.abs(w), np.abs(dy))
+    d = g.capi.ConvDesc(Cn, O, kW, kH, s, s, px, py, px, py, 1, 1, 1, 0, g.capi.KERNEL_F32_GEMM if path else 0)
+    need = int(g.lib.n2d2hip_conv2d_f32_workspace_bytes(C.byref(d), B, H, W))
+    assert need > 0 or not path             # (the direct kernels take none)
+    ws = g.torch_.empty(max(need, 4), dtype=t.uint8, device="cuda")
+    x_, w_, dy_ = g.dev(x), g.dev(w), g.dev(dy)
+    for wp, n in ((ws.data_ptr(), need), (None, 0)):
+        y, dx, dw = (t.ones(v.shape, dtype=t.float32, device="cuda") for v in (dy, x, w))
+        g.check(g.lib.n2d2hip_conv2d_f32_forward(C.byref(d), B, H, W, x_.data_ptr(), w_.data_ptr(), None, 1.0, y.data_ptr(), wp, n, g.sp()))
+        g.check(g.lib.n2d2hip_conv2d_f32_backward_data(C.byref(d), B, H, W, w_.data_ptr(), dy_.data_ptr(), 1.0, dx.data_ptr(), wp, n, g.sp()))
+        assert _rel(g.host(y), want[0] + 1, mag[0] + 1) <= TOL
+        assert _rel(g.host(dx), want[1] + 1, mag[1] + 1) <= TOL
+        if n:
+            g.check(g.lib.n2d2hip_conv2d_f32_backward_filter(C.byref(d), B, H, W, x_.data_ptr(), dy_.data_ptr(), 1.0, dw.data_ptr(), wp, n, g.sp()))
+            assert _rel(g.host(dw), want[2] + 1, mag[2] + 1) <= TOL
+
+
 # B, C, H, W, k, stride, pad: strips of four with every remainder, rows shorter than a strip or a window, windows past both
 # ends of the tensor, both parities of the padding at stride 2, blocks of 256 and of 1024 threads, outputs wider than the input
 DEPTHWISE = [(1, 1, 1, 1, 3, 1, 1), (2, 3, 2, 3, 3, 1, 1), (1, 1, 3, 3, 3, 1, 0), (3, 2, 5, 6, 3, 2, 0), (2, 5, 9, 7, 3, 2, 1), (1, 4, 6, 9, 3, 2, 2),
