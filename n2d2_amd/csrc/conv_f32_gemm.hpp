@@ -54,6 +54,7 @@ struct PixelClass {
     int tile0;                 // first tile of this class
     int P, gW, gHW;            // pixels over all images; row length and pixels per image of the class's grid
     int nx, nT;                // taps along x, taps
+    int kchunk;                // a K range (a multiple of GK or K33; chunked K: in steps of GK)
     int ty0, tx0;              // first tap; the next one along an axis is osy / osx further in the kernel
     int y0, x0;                // source position of tap (0, 0) for grid pixel (0, 0)
     int stepy, stepx;          // element offset from one tap to the next in the source plane
@@ -65,7 +66,6 @@ constexpr int PIXEL_CLASSES = 4;
 
 struct PixelGemm {
     int Q, Ch;                 // rows of q; channels that k runs over
-    int kchunk;                // a K range (a multiple of GK; chunked K: in steps of GK)
     int nz;                    // K ranges of a block: blockIdx.z * nz ...
     int sy, sx, d;             // source step per grid pixel (the strides; 1 for backward-data); +1 / -1: per tap
     int Hs, Ws, planeS;        // source plane
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(256) void conv_f32_chunk_kernel(PixelGemm g, const 
     PixelTile<PT> tl_acc;
     tl_acc.init((unsigned)(unsigned long)(__attribute__((address_space(3))) float*)smem, wq, wp, lane);
     for (int z = blockIdx.z * g.nz; z < (int)(blockIdx.z + 1) * g.nz; ++z) {
-        const int sbeg = z * g.kchunk, nsteps = max(0, min(g.kchunk, nchunks * nT - sbeg));
+        const int sbeg = z * c.kchunk, nsteps = max(0, min(c.kchunk, nchunks * nT - sbeg));
         int chunk = nT > 0 ? div_f32(sbeg, c.nt) : 0, t = sbeg - chunk * nT;
         int ch_off = (chunk * GK + wave * 4) * plane4, ch_left = g.Ch - chunk * GK - wave * 4;
         int w_off = chunk * g.T * g.qpad * (GK * 4) + q0 * (GK * 4) + (QT >= 64 ? wave : wave & 1) * 1024;
@@ -471,7 +471,7 @@ __global__ __launch_bounds__(256) void conv_f32_3x3_kernel(PixelGemm g, const fl
     const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) float*)smem;
     const unsigned xaddr = lds0 + 4u * (lh * PT + wp * 32 + l32), waddr = lds0 + 4u * (K33 * PT + (wq * 32 + l32) * W33 + 20 * lh);
     for (int z = blockIdx.z * g.nz; z < (int)(blockIdx.z + 1) * g.nz; ++z) {
-        const int kbeg = z * g.kchunk, kend = min(kbeg + g.kchunk, g.Ch * 9);
+        const int kbeg = z * c.kchunk, kend = min(kbeg + c.kchunk, g.Ch * 9);
         const int step0 = kbeg / K33, nsteps = kend > kbeg ? (kend + K33 - 1) / K33 - step0 : 0;
         int ch_off = (step0 * 4 + wave) * plane4, k_row = step0 * K33 + wave * 9 - kbeg, w_off = step0 * wstep + q0 * W33 * 4;
         const unsigned krange = kend - kbeg;
@@ -696,7 +696,7 @@ __global__ __launch_bounds__(256) void conv_f32_pixel_kernel(PixelGemm g, const 
     PixelTile<PT> tl_acc;
     tl_acc.init((unsigned)(unsigned long)(__attribute__((address_space(3))) float*)smem, wq, wp, lane);
     for (int z = blockIdx.z * g.nz; z < (int)(blockIdx.z + 1) * g.nz; ++z) {
-        const int kbeg = z * g.kchunk, kend = min(kbeg + g.kchunk, K);
+        const int kbeg = z * c.kchunk, kend = min(kbeg + c.kchunk, K);
         const int nsteps = kend > kbeg ? (kend - kbeg + GK - 1) / GK : 0;
         int row_t[4], row_ch[4];                     // row_ch: byte offset of the row's channel
         const int plane4 = g.planeS * 4, adv = nT > 0 ? div_f32(GK, c.nt) : 0, adv_t = nT > 0 ? GK - adv * nT : 0, adv_ch = adv * plane4;

@@ -934,7 +934,8 @@ static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass>
     // tile shape
     long P = 0, kmax = 0;
     const int nchunks = ceil_div_i(g.Ch, GK);
-    for (const PixelClass& c : cls) { P += c.P; kmax = std::max<long>(kmax, (long)(kind == PIXELS_CHUNK && (!fwd || T > 1) ? nchunks * GK : g.Ch) * c.nT); }
+    const int kch = kind == PIXELS_CHUNK && (!fwd || T > 1) ? nchunks * GK : g.Ch;
+    for (const PixelClass& c : cls) { P += c.P; kmax = std::max(kmax, (long)kch * c.nT); }
     // (64 x 64 tiles, four to a CU, lost at most 4 % to the best of 32 x 128, 64 x 128 and 128 x 128 on every shape with Q
     // over 32 that was timed, and gained up to 70 % where the larger tiles are few)
     pl.small_q = g.Q <= 32;
@@ -949,30 +950,38 @@ static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass>
         cls[i].tile0 = (int)tiles;
         pl.many = pl.many || cls[i].nx + (cls[i].nT > 0 ? cls[i].nT / cls[i].nx : 0) > 31;
         tiles += ceil_div_i(cls[i].P, PT);
-        g.c[i] = cls[i];
     }
     g.ptiles = (int)tiles;
     g.ptiles8 = ceil_div_i(tiles, 8);
     const long blocks = tiles * g.qtiles;
     g.nz = 1;
-    long splits;
+    long splits, least = q.ranges;
     if (fwd) {
         // The ranges of a forward sum follow from its sizes alone: with another order of additions the quantizer behind it would
         // give another level now and then.  With a block for every CU it takes all of them (long kernels: with two; 64 -> 64,
         // 1 x 31, 256 tiles: 102 us with one, 82 with partial results).
         splits = pass_ranges(P, g.Q, kmax);
     } else {
-        // where the tiles do not fill the chip twice; none below four steps
+        // where the tiles do not fill the chip twice; none below four steps.  And as many ranges as over all taps at 128 x 128
+        // tiles: the longer a float sum, the more it loses (256 -> 256, 3x3, 14 x 14, batch 32: one range 8.3e-7 from 64 bits and
+        // 89 us, seven folded in double 3.1e-7 and 96).
         splits = blocks >= 512 ? 1 : std::max(1L, 768 / blocks);
         splits = std::min<long>(splits, std::max(1L, kmax / (4 * GK)));
+        least = pass_ranges((long)q.B * q.H * q.W, q.C, (long)q.O * T);
     }
-    g.kchunk = std::max(q.ranges > splits ? (int)(kmax / q.ranges) / GK * GK : round_up((int)((kmax + splits - 1) / splits), GK), GK);
-    pl.splits = std::max(1, ceil_div_i(kmax, g.kchunk));
-    if (fwd && blocks >= (pl.many ? 512 : 256)) {
+    const int step = !fwd && kind == PIXELS_3X3 ? K33 : GK;
+    pl.splits = 1;
+    for (int i = 0; i < g.nclass; ++i) {         // (the ranges of a class of fewer taps are as many, and shorter)
+        const long K = (long)kch * cls[i].nT;
+        cls[i].kchunk = std::max(least > splits ? (int)(K / least) / step * step : round_up((int)((K + splits - 1) / splits), GK), step);
+        pl.splits = std::max(pl.splits, ceil_div_i(K, cls[i].kchunk));
+        if (kind == PIXELS_CHUNK) cls[i].kchunk /= GK;
+        g.c[i] = cls[i];
+    }
+    if (blocks >= (fwd && !pl.many ? 256 : 512)) {
         g.nz = pl.splits;
         pl.splits = 1;
     }
-    if (kind == PIXELS_CHUNK) g.kchunk /= GK;
     return pl;
 }
 

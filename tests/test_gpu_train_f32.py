@@ -388,6 +388,32 @@ def test_long_kernels_on_the_matrix_cores(g, case, path):
             assert _rel(g.host(dw), want[2] + 1, mag[2] + 1) <= TOL
 
 
+# `terms`: the longest float sum of the data gradient and of the filter gradient (the losses of such sums: as for the spanning
+# layers above)
+@pytest.mark.parametrize("case,terms", [((32, 256, 14, 14, 256, 3, 1), (330, 0)), ((33, 128, 27, 27, 256, 3, 2), (256, 0)),
+                                        ((32, 128, 14, 14, 128, 5, 1), (256, 0))])
+def test_error_of_the_gradients(g, case, terms):
+    B, Cn, H, W, O, k, s = case
+    print("error of the gradients", case, flush=True)
+    t, F = g.torch_, g.torch_.nn.functional
+    gen = t.Generator().manual_seed(sum(case))
+    x, w = t.randn(B, Cn, H, W, generator=gen), t.randn(O, Cn, k, k, generator=gen)
+    x64, w64 = x.double().requires_grad_(), w.double().requires_grad_()
+    y64 = F.conv2d(x64, w64, stride=s, padding=k // 2)
+    dy = t.randn(y64.shape, generator=gen)
+    y64.backward(dy.double())
+    d = g.desc(Cn, O, k, s, k // 2, 1)
+    need = int(g.lib.n2d2hip_conv2d_f32_workspace_bytes(C.byref(d), B, H, W))
+    ws = t.empty(need, dtype=t.uint8, device="cuda")
+    x_, w_, dy_ = x.cuda(), w.cuda(), dy.cuda()
+    dx, dw = t.empty_like(x_), t.empty_like(w_)
+    g.check(g.lib.n2d2hip_conv2d_f32_backward_data(C.byref(d), B, H, W, w_.data_ptr(), dy_.data_ptr(), 0.0, dx.data_ptr(), ws.data_ptr(), need, g.sp()))
+    g.check(g.lib.n2d2hip_conv2d_f32_backward_filter(C.byref(d), B, H, W, x_.data_ptr(), dy_.data_ptr(), 0.0, dw.data_ptr(), ws.data_ptr(), need, g.sp()))
+    for got, want, n in ((dx, x64.grad, terms[0]), (dw, w64.grad, terms[1])):
+        if n:
+            assert float((got.cpu().double() - want).norm()) <= 1.1 * 2.53e-8 * np.sqrt(1 + n / 2) * float(want.norm())
+
+
 # B, C, H, W, k, stride, pad: strips of four with every remainder, rows shorter than a strip or a window, windows past both
 # ends of the tensor, both parities of the padding at stride 2, blocks of 256 and of 1024 threads, outputs wider than the input
 DEPTHWISE = [(1, 1, 1, 1, 3, 1, 1), (2, 3, 2, 3, 3, 1, 1), (1, 1, 3, 3, 3, 1, 0), (3, 2, 5, 6, 3, 2, 0), (2, 5, 9, 7, 3, 2, 1), (1, 4, 6, 9, 3, 2, 2),
