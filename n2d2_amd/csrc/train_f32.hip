@@ -744,8 +744,11 @@ static int f32_path(const ConvF32& q, int pass)
 {
     if (q.depthwise || q.dx != 1 || q.dy != 1 || (q.choice & N2D2HIP_KERNEL_F32_DIRECT))
         return F32_PATH_DIRECT;
-    // 32-bit byte offsets from a base moved back by the padding, and one validity bit per tap row and column
-    const size_t lim = ((size_t)1 << 29) - (size_t)(q.pt + q.kH) * (q.W + q.oW + q.pl + q.kW);
+    // 32-bit byte offsets from a base moved back by the padding
+    const size_t most = (size_t)1 << 29, rows = (size_t)q.pt + q.kH, cols = (size_t)q.W + q.oW + q.pl + q.kW;
+    if (rows >= most || cols >= most || rows * cols >= most)
+        return F32_PATH_DIRECT;
+    const size_t lim = most - rows * cols;
     if ((size_t)q.B * q.C * q.H * q.W >= lim || (size_t)q.B * q.O * q.oH * q.oW >= lim || (size_t)q.O * q.C * q.kH * q.kW >= lim
         || (many_taps(q) && !spans_input(q)))
         return F32_PATH_DIRECT;

@@ -112,3 +112,19 @@ def test_planning_questions_answered_from_descriptors_alone():
     assert lib.n2d2hip_pool_writes_halo(None, 28, 28, 16) == 0
     assert lib.n2d2hip_bottleneck_pays(None, 128, 56, 56) == 0
     assert lib.n2d2hip_conv_chain_pays(None, None, 128, 56, 56) == 0
+
+
+def test_float_convolutions_too_large_for_32_bit_offsets_ask_for_no_workspace():
+    """Tensors of 2 GiB and more, and rows so long that a kernel's reach alone passes the offsets, run on the direct kernels,
+    whatever the descriptor asks for.  The workspace query answers from sizes alone: 0 there."""
+    from n2d2_amd import capi
+    lib = capi.lib
+    need = lambda B, Cc, H, W, O, kH, kW, pt=0, pl=0: lib.n2d2hip_conv2d_f32_workspace_bytes(  # noqa: E731
+        C.byref(capi.ConvDesc(Cc, O, kW, kH, 1, 1, pl, pt, pl, pt, 1, 1, 1, 0, capi.KERNEL_F32_GEMM)), B, H, W)
+    assert need(1, 1, 3, 1000, 1, 3, 3) > 0 and need(1, 1, 3, 10 ** 7, 1, 3, 3) > 0
+    for W in (9 * 10 ** 7, 10 ** 8, 2 * 10 ** 8, 5 * 10 ** 8, 10 ** 9, 2 * 10 ** 9):        # 3 (W + W - 2 + 3) > 2^29
+        assert need(1, 1, 3, W, 1, 3, 3) == 0
+    assert need(2, 300, 30, 40000, 1, 3, 3) == 0                                            # 720 M inputs
+    assert need(1, 1, 10, 10, 1, 2, 2, pt=10 ** 4, pl=10 ** 5) == 0                         # 4.0 G outputs
+    assert need(1, 1, 1, 2 ** 29, 1, 1, 1) == 0 and need(1, 2, 1, 2 ** 28, 1, 1, 1) == 0
+    assert need(1, 1, 2, 1, 1, 4, 1, pt=10 ** 9) == 0                                       # rows of padding alone
