@@ -735,6 +735,9 @@ enum { F32_PATH_DIRECT, F32_PATH_GEMM, F32_PATH_SMALL };
 // More than the pixel kernels have lanes and the filter kernel has mask bits for
 static bool many_taps(const ConvF32& q) { return (long)q.kH * q.kW > 64; }
 
+// Largest second dimension of a grid.  Layers of more outputs or images than it covers take kernels with those in the first.
+constexpr long GRID_Y = 65535;
+
 // The kernels of a pass.  The matrix cores serve ungrouped convolutions without dilation; the direct kernels keep the rest
 // (depthwise, dilated) and the forward sums below 2e7 flops or of kernels over 64 taps, which stay in the reference's order
 // of terms (quantizers turn the last bit of a sum into a level now and then).  Backward-filter below 2e7 flops, and of a
@@ -752,7 +755,8 @@ static int f32_path(const ConvF32& q, int pass)
     if ((size_t)q.B * q.C * q.H * q.W >= lim || (size_t)q.B * q.O * q.oH * q.oW >= lim || (size_t)q.O * q.C * q.kH * q.kW >= lim
         || (many_taps(q) && !spans_input(q)))
         return F32_PATH_DIRECT;
-    if (pass == PASS_BWD_FILTER && many_taps(q)) return F32_PATH_SMALL;
+    if (pass == PASS_BWD_FILTER && many_taps(q)) return q.O <= 16 * GRID_Y ? F32_PATH_SMALL : F32_PATH_DIRECT;
+    if (pass == PASS_BWD_FILTER && q.O > 64 * GRID_Y && !spans_input(q)) return F32_PATH_DIRECT;
     const double flops = 2.0 * q.B * q.O * q.oH * q.oW * q.C * q.kH * q.kW;
     const bool forced = q.choice & N2D2HIP_KERNEL_F32_GEMM, small = flops < 2.0e7;
     // As a convolution the K of a spanning layer's backward-data runs over all taps of an output, one of which is not zero: few
@@ -760,11 +764,12 @@ static int f32_path(const ConvF32& q, int pass)
     // 64 x 4 x 4 <- 256: 2.5e-8 from 64 bits and 10 us; convolution 7.7e-8, 41 us; product in float 2.9e-7, 14 us) and beyond
     // takes as many ranges as the convolution would (128 images, 512 x 2 x 2 <- 1000: 1.5e-7 and 26 us; in double 36; convolution
     // 1.5e-7, 64; 64 images, 512 x 7 x 7 <- 4096: 179 us, in double 1019, convolution 9566).
-    if (pass == PASS_BWD_DATA && (forced || !small) && flops < 5.0e8 && !many_taps(q) && q.kH * q.kW > 1 && spans_input(q))
+    if (pass == PASS_BWD_DATA && (forced || !small) && flops < 5.0e8 && !many_taps(q) && q.kH * q.kW > 1 && q.B <= 16 * GRID_Y && spans_input(q))
         return F32_PATH_SMALL;
     if (forced) return F32_PATH_GEMM;
     if (pass == PASS_FWD) return small || many_taps(q) ? F32_PATH_DIRECT : F32_PATH_GEMM;
-    return small && pass == PASS_BWD_FILTER ? F32_PATH_SMALL : F32_PATH_GEMM;
+    if (small && pass == PASS_BWD_FILTER) return q.O <= 16 * GRID_Y ? F32_PATH_SMALL : F32_PATH_DIRECT;
+    return F32_PATH_GEMM;
 }
 
 static DivF32 div_of(int d)
@@ -819,7 +824,7 @@ static int run_direct(const ConvF32& q, int pass, const float* x, const float* w
     const int T = q.kH * q.kW;
     const long K = (long)q.C * T;
     // (a kernel of 3x3 has an order of its own; 16-byte loads)
-    if (!bwd && !q.depthwise && q.dx == 1 && q.dy == 1 && spans_input(q) && (q.kH != 3 || q.kW != 3) && K % 4 == 0 && K < (1 << 22)
+    if (!bwd && !q.depthwise && q.dx == 1 && q.dy == 1 && spans_input(q) && (q.kH != 3 || q.kW != 3) && K % 4 == 0 && K < (1 << 22) && q.O <= 8 * GRID_Y
         && (((size_t)x | (size_t)w) & 15) == 0) {
         hipLaunchKernelGGL(conv_f32_chain_kernel, dim3(ceil_div_i(q.B, 8), ceil_div_i(q.O, 8)), dim3(64), 0, st, q.B, q.O, (int)K, x, w, bias, beta, out);
         N2D2HIP_HIP_CHECK(hipGetLastError());
@@ -1213,7 +1218,7 @@ int n2d2hip_conv2d_f32_forward(const n2d2hip_conv_desc* desc, int B, int H, int 
             const ConvF32 m = product_of(q, PASS_FWD, &pass);
             // (without a workspace that holds its partial results: the convolution as it stands, whose kernels keep a tap in each
             // of a wave's 64 lanes, or the direct kernels)
-            if (pass_workspace(m, pass) <= nws)
+            if (q.B <= 64 * GRID_Y && pass_workspace(m, pass) <= nws)
                 return run_pass(m, pass, w, x, bias, 1, q.O, beta, y, ws, nws, (hipStream_t)stream);
             if (many_taps(q)) return run_direct(q, PASS_FWD, x, w, bias, beta, y, (hipStream_t)stream);
         }

@@ -413,6 +413,27 @@ def test_error_of_the_gradients(g, case, terms):
         assert float((got.cpu().double() - want).norm()) <= 1.1 * 2.53e-8 * np.sqrt(1 + n / 2) * float(want.norm())
 
 
+# B, C, O: layers on one pixel with more images or outputs than the second dimension of a grid covers in tiles
+@pytest.mark.parametrize("case", [(1, 4, 8 * 65535 + 9), (1, 1, 16 * 65535 + 17), (64 * 65535 + 65, 3, 5), (16 * 65535 + 17, 2, 1)])
+def test_layers_of_millions_of_outputs_or_images(g, case):
+    B, Cn, O = case
+    print("wide layer", case, flush=True)
+    t = g.torch_
+    gen = t.Generator(device="cuda").manual_seed(sum(case))
+    x, w, dy = (t.randn(*s, generator=gen, device="cuda") for s in ((B, Cn), (O, Cn), (B, O)))
+    d = g.capi.ConvDesc(Cn, O, 1, 1, 1, 1, 0, 0, 0, 0, 1, 1, 1, 0, 0)
+    need = int(g.lib.n2d2hip_conv2d_f32_workspace_bytes(C.byref(d), B, 1, 1))
+    ws = t.empty(max(need, 4), dtype=t.uint8, device="cuda")
+    y, dx, dw = t.empty_like(dy), t.empty_like(x), t.empty_like(w)
+    g.check(g.lib.n2d2hip_conv2d_f32_forward(C.byref(d), B, 1, 1, x.data_ptr(), w.data_ptr(), None, 0.0, y.data_ptr(), ws.data_ptr(), need, g.sp()))
+    g.check(g.lib.n2d2hip_conv2d_f32_backward_data(C.byref(d), B, 1, 1, w.data_ptr(), dy.data_ptr(), 0.0, dx.data_ptr(), ws.data_ptr(), need, g.sp()))
+    g.check(g.lib.n2d2hip_conv2d_f32_backward_filter(C.byref(d), B, 1, 1, x.data_ptr(), dy.data_ptr(), 0.0, dw.data_ptr(), ws.data_ptr(), need, g.sp()))
+    x, w, dy = x.double(), w.double(), dy.double()
+    for got, a, b in ((y, x, w.T), (dx, dy, w), (dw, dy.T, x)):
+        want, mag = a @ b.contiguous(), a.abs() @ b.abs().contiguous()
+        assert float(((got.double() - want).abs() / mag.clamp(min=1e-3)).max()) <= TOL
+
+
 # B, C, H, W, k, stride, pad: strips of four with every remainder, rows shorter than a strip or a window, windows past both
 # ends of the tensor, both parities of the padding at stride 2, blocks of 256 and of 1024 threads, outputs wider than the input
 DEPTHWISE = [(1, 1, 1, 1, 3, 1, 1), (2, 3, 2, 3, 3, 1, 1), (1, 1, 3, 3, 3, 1, 0), (3, 2, 5, 6, 3, 2, 0), (2, 5, 9, 7, 3, 2, 1), (1, 4, 6, 9, 3, 2, 2),
