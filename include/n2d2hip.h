@@ -452,9 +452,14 @@ int n2d2hip_lsq_backward(const float* diff_q, const float* fp_x, float* diff_fp,
 /* The float32 cells a quantization-aware training graph runs between the fake-quant kernels above.  Tensors are
  * N2D2's own: activations NCHW ({X,Y,Z,B}, X fastest), weights OCHW ({kW,kH,C/groups,O}); `desc->weight_bits` is not
  * read; groups is 1 or C == O (depthwise).  "diff" tensors carry the descent direction, as in the reference
- * (target - output at the loss), so the solver adds rate * diff.  Ungrouped convolutions without dilation of at
- * least 2e7 flops run as an implicit GEMM on the fp32 matrix cores, the others on direct kernels that add their terms
- * in the reference's order.
+ * (target - output at the loss), so the solver adds rate * diff.
+ *
+ * Ungrouped convolutions without dilation, of up to 64 taps or spanning their input, run on the matrix cores: forward from
+ * 2e7 flops (spanning: up to 64 taps), backward-data, and backward-filter (in double below 2e7 flops and for spanning
+ * kernels of more than 64 taps).  There sums are added in an order that follows from the sizes, not in the reference's.
+ * All others, and tensors of 2 GiB and more, run on direct kernels, which add forward and backward-data in the
+ * reference's order and backward-filter in double.  kernel_choice N2D2HIP_KERNEL_F32_DIRECT asks for the direct
+ * kernels, N2D2HIP_KERNEL_F32_GEMM for the matrix cores at any size.
  *
  * y = conv(x, w) (+ bias[o] if bias != NULL) + beta * y; the window is clipped at the borders (ref: src/Cell/ConvCell_Frame_Kernels.cpp:26-174, called from
  * ConvCell_Frame<T>::propagate, src/Cell/ConvCell_Frame.cpp:418-473). */
@@ -469,10 +474,9 @@ int n2d2hip_conv2d_f32_backward_data(const n2d2hip_conv_desc* desc, int B, int H
 /* diff_w = backwardFilter(x, diff_y) + beta * diff_w (ref: src/Cell/ConvCell_Frame_Kernels.cpp:335-427).
  *
  * `workspace` (device memory) of the three passes: n2d2hip_conv2d_f32_workspace_bytes bytes (may be 0) serve all of
- * them.  Backward-filter splits its sum over batch and pixels into ranges whose partial results go through the
- * workspace and are added in a fixed order; it fails with N2D2HIP_ERR_WORKSPACE when the workspace is too small.
- * Forward and backward-data do the same to fill the chip when their output is small, and run as one range when the
- * workspace is NULL or too small. */
+ * them.  Sums are split into ranges whose partial results go through the workspace and are added in a fixed order.
+ * Backward-filter in float needs it and fails with N2D2HIP_ERR_WORKSPACE when it is too small.  Where it adds in double,
+ * and in forward and backward-data, a block takes all ranges when the workspace is NULL or too small. */
 size_t n2d2hip_conv2d_f32_workspace_bytes(const n2d2hip_conv_desc* desc, int B, int H, int W);
 int n2d2hip_conv2d_f32_backward_filter(const n2d2hip_conv_desc* desc, int B, int H, int W, const float* x,
                                        const float* diff_y, float beta, float* diff_w, void* workspace,

@@ -23,7 +23,10 @@
 //    trying all of them is 36).
 //  * rows of LDS that hold consecutive k hold the even ones in front of the odd ones, or (filter) give the two lane halves of
 //    an instruction different groups of 4 k, so that a lane reads four instructions' operands in 16 bytes.
-// A forward sum is added in one order whatever kernel takes it: channel, tap, in pairs, in ranges that follow from the sizes.
+// A forward sum is added in one order by the 3x3, the chunk (1x1) and the pixel kernel: channel, tap, in pairs, in ranges that
+// follow from the sizes.  Two forms have an order of their own: long kernels in chunks of 16 channels at one tap, and layers
+// that span their input with up to 64 taps and have room for partial results, which are plain products on the filter kernel
+// (its instructions pair k with k + 4).
 // Backward-filter, whose K is the whole batch of pixels and whose output is small, splits K over blockIdx.z into partial
 // results that a second kernel adds up in a fixed order; forward and backward-data do the same when their tiles alone would
 // not fill the chip.

@@ -1566,10 +1566,14 @@ int n2d2hip_conv_chain_supported(n2d2hip_conv_t conv3x3, n2d2hip_conv_t expand)
 // The one launch has 128-pixel tiles over all channels, so ceil(pixels / 128) blocks; the two launches also cut the channels
 // into tiles.  ResNet-50 (us for the whole net; the pairs of a size in two launches / in one):
 //  64 middle channels: one launch is never slower (batch 1 347 / 342, batch 24 550 / 528, batch 128 1226 / 1204).
-//  128: one launch loses while a good part of the compute units has no tile (98 tiles 454 / 467, 147 tiles 544 / 560 and
-//  550 / 541); from three quarters on it is level or ahead (196 tiles 616 / 611, 392 812 / 805, 980 1456 / 1426).
+//  128: one launch loses while a good part of the compute units has no tile (25 tiles 350 / 373, 74 401 / 414, 98 413 / 423,
+//  123 437 / 446); between half and three quarters it is one or the other (147 tiles 530 / 519 and 544 / 560, 160 538 / 541,
+//  172 557 / 550, 184 573 / 556), from there on level or ahead (196 593 / 584, 252 638 / 632, 258 714 / 716, 294 736 / 738,
+//  392 807 / 800, 490 931 / 901, 980 1456 / 1426).
 //  256: a work-group of eight waves has a compute unit to itself; one launch pays where its tiles make one nearly full round
-//  (245 tiles 1426 / 1389) and else loses (8 tiles 347 / 448, 196 1205 / 1227, 392 2066 / 2123, 612 3307 / 3349).
+//  (226 tiles 1427 / 1369, 238 1451 / 1404, 250 1496 / 1450, 256 1510 / 1468; already 215 1370 / 1334) and else loses (2 tiles
+//  365 / 468, 49 588 / 682, 98 801 / 854, 154 1098 / 1121, 196 1241 / 1252, 258 1630 / 1723, 276 1704 / 1798, 392 2140 / 2186);
+//  of two nearly full rounds it gains too little to be asked for (460 2515 / 2503, 490 2634 / 2610, 512 2725 / 2699).
 int n2d2hip_conv_chain_pays(n2d2hip_conv_t c3, n2d2hip_conv_t ce, int batch, int in_h, int in_w)
 {
     if (!chain_ok(c3, ce) || batch <= 0 || in_h <= 0 || in_w <= 0)

@@ -2,8 +2,8 @@
 // the loss at the output and the SGD update.  Tensors are N2D2's own NCHW / OCHW float tensors (X fastest), so a
 // training graph exchanges them without conversion.
 //
-// Convolutions run on the matrix cores (conv_f32_gemm.hpp) wherever they are neither grouped nor dilated.  The kernels here
-// are direct: one thread per produced element, walking channels and taps in the reference's order (so forward and
+// Convolutions run on the matrix cores (conv_f32_gemm.hpp) wherever they are neither grouped nor dilated, but for small forward
+// sums (f32_path).  The kernels here are direct: one thread per produced element, walking channels and taps in the reference's order (so forward and
 // backward-data give the reference's float sums term for term), and one block per weight for backward-filter, whose long
 // sum over batch and pixels is wavefront-reduced in double.
 #include <algorithm>
