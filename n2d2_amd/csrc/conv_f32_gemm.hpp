@@ -32,7 +32,7 @@
 // not fill the chip.
 // Measured (us, forward / data / filter, before: 128 x 128 tiles, operands through registers, one test per load; now):
 //   64 -> 64, 3x3, 56 x 56, batch 64             236 / 284 / 263    149 / 157 / 180   (15 GFLOP: 99, 94, 82 TFLOP/s of 154)
-//   128 -> 256, 3x3 stride 2, 27 x 27, batch 33   80 / 277 /  76     55 /  53 /  58
+//   128 -> 256, 3x3 stride 2, 27 x 27, batch 33   80 / 277 /  76     55 /  54 /  58
 //   a layer spanning its input, 16384 -> 10, 64  2632 /  27 / 222    116 /   7 /   8
 //   64 -> 64, 1 x 40, 1 x 512, batch 32            94 / 110 /  98     86 /  82 /  70
 //   128 -> 128, 1 x 64, 1 x 256, batch 16         120 / 134 / 124    113 / 106 / 104
