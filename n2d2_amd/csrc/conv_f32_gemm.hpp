@@ -138,12 +138,14 @@ __device__ __forceinline__ bool pixel_tile(const PixelGemm& g, int* tile, int* q
 // rows and columns than that (1 x 40): a bit for each of up to 64 taps.
 template <bool LONG>
 struct TapMask {
-    unsigned m[LONG ? 2 : 1];
+    unsigned m, high;
     // `bit`: LONG: bit t of its word, or 0 past the range; else the tap's column and row, and bit 31 past the range
     __device__ __forceinline__ bool inside(int t, unsigned bit) const
     {
-        if (LONG) return ((t & 32 ? m[LONG] : m[0]) & bit) != 0;
-        return (m[0] & bit) == bit;
+        // (chosen by bits: a choice between two members goes through their addresses, and the masks live in scratch memory)
+        const unsigned upper = t & 32 ? ~0u : 0u;
+        if (LONG) return (((high & upper) | (m & ~upper)) & bit) != 0;
+        return (m & bit) == bit;
     }
 };
 // The first tap of each of a kernel's rows, and of the taps those in columns xl .. xh - 1 and rows yl .. yh - 1.
@@ -180,8 +182,8 @@ __device__ __forceinline__ void pixel_source(const PixelGemm& g, const PixelClas
         auto first = [&](int v, int size, int n) { return min(max(g.d > 0 ? -v : v - size + 1, 0), n); };
         auto end = [&](int v, int size, int n) { return min(max(g.d > 0 ? size - v : v + 1, 0), n); };
         const unsigned long long m = long_taps(first(x, g.Ws, c.nx), end(x, g.Ws, c.nx), first(y, g.Hs, ny), end(y, g.Hs, ny), c.nx, long_rows(ny, c.nx));
-        mask->m[0] = p < c.P ? (unsigned)m : 0u;
-        mask->m[LONG] = p < c.P ? (unsigned)(m >> 32) : 0u;
+        mask->m = p < c.P ? (unsigned)m : 0u;
+        mask->high = p < c.P ? (unsigned)(m >> 32) : 0u;
         return;
     }
     unsigned m = 0;
@@ -193,7 +195,8 @@ __device__ __forceinline__ void pixel_source(const PixelGemm& g, const PixelClas
         const int y = py * g.sy + c.y0 + i * g.d;
         m |= (unsigned)(y >= 0 && y < g.Hs) << (c.nx + i);
     }
-    mask->m[0] = p < c.P ? m : 0u;
+    mask->m = p < c.P ? m : 0u;
+    mask->high = 0;
 }
 
 // The products of a wave's 32 x 32 tile from one stage: [16 k][PT pixels] and behind it [QT][16 k], the even k of a row in
