@@ -27,6 +27,7 @@
 // follow from the sizes.  Two forms have an order of their own: long kernels in chunks of 16 channels at one tap, and layers
 // that span their input with up to 64 taps and have room for partial results, which are plain products on the filter kernel
 // (its instructions pair k with k + 4).
+// Within a block, float sums are added to sums in double after as many steps as keep them no longer than 128 x 128 tiles would.
 // Backward-filter, whose K is the whole batch of pixels and whose output is small, splits K over blockIdx.z into partial
 // results that a second kernel adds up in a fixed order; forward and backward-data do the same when their tiles alone would
 // not fill the chip.
@@ -34,8 +35,8 @@
 //   64 -> 64, 3x3, 56 x 56, batch 64             236 / 284 / 263    149 / 157 / 180   (15 GFLOP: 99, 94, 82 TFLOP/s of 154)
 //   128 -> 256, 3x3 stride 2, 27 x 27, batch 33   80 / 277 /  76     55 /  54 /  58
 //   a layer spanning its input, 16384 -> 10, 64  2632 /  27 / 222    116 /   7 /   8
-//   64 -> 64, 1 x 40, 1 x 512, batch 32            94 / 110 /  98     86 /  82 /  70
-//   128 -> 128, 1 x 64, 1 x 256, batch 16         120 / 134 / 124    113 / 106 / 104
+//   64 -> 64, 1 x 40, 1 x 512, batch 32            94 / 110 /  98     76 /  72 /  70
+//   128 -> 128, 1 x 64, 1 x 256, batch 16         120 / 134 / 124    101 /  96 / 105
 // A CU takes whole tiles, so the last round costs its share: 64 -> 64 on 56 x 56 at batch 64 is 12.25 tiles for each.
 #pragma once
 
@@ -57,7 +58,8 @@ struct PixelClass {
     int tile0;                 // first tile of this class
     int P, gW, gHW;            // pixels over all images; row length and pixels per image of the class's grid
     int nx, nT;                // taps along x, taps
-    int kchunk;                // a K range (a multiple of GK or K33; chunked K: in steps of GK)
+    int kchunk;                // a K range (a multiple of GK; chunked K: in steps of GK)
+    int fold;                  // steps of a range after which its float sums are added to those in double; 0: all of it
     int ty0, tx0;              // first tap; the next one along an axis is osy / osx further in the kernel
     int y0, x0;                // source position of tap (0, 0) for grid pixel (0, 0)
     int stepy, stepx;          // element offset from one tap to the next in the source plane
@@ -85,6 +87,7 @@ struct PixelGemm {
 struct FilterGemm {
     int P, Q, K;
     int kchunk;                // K range of one blockIdx.z (a multiple of FK)
+    int fold;                  // steps of it after which the float sums are added to those in double; 0: all of it
     int C, H, W, kW, kH, s_y, s_x, pt, pl;
     int oW, plane;             // output row length and plane
     int imgX, imgY;
@@ -205,7 +208,7 @@ __device__ __forceinline__ void pixel_source(const PixelGemm& g, const PixelClas
 template <int PT>
 struct PixelTile {
     v16f acc;
-    double folded[16];         // several ranges in a block: their sums, as the partial results of several blocks are added
+    double folded[16];         // several ranges or folds in a block: their sums, as the partial results of several blocks are added
     v4f fa[2];
     v2f fb[2][2];
     unsigned xaddr, waddr0, waddr1;
@@ -404,22 +407,26 @@ __global__ __launch_bounds__(256) void conv_f32_chunk_kernel(PixelGemm g, const 
                 for (int part = 0; part < 5; ++part) load_part(part);
             auto k_loop = [&](auto live) {
                 unsigned sb = 0;
-                for (int st = 0; st < nsteps; ++st) {
-                    wait_loads_and_barrier<LPI*(S - 2)>();
-                    tl_acc.template step<decltype(live)::value>(sb, load_part);
-                    sb = sb == 4u * STAGE * (S - 1) ? 0u : sb + 4u * STAGE;
+                for (int st = 0; st < nsteps;) {
+                    const int end = c.fold ? min(st + c.fold, nsteps) : nsteps;
+                    for (; st < end; ++st) {
+                        wait_loads_and_barrier<LPI*(S - 2)>();
+                        tl_acc.template step<decltype(live)::value>(sb, load_part);
+                        sb = sb == 4u * STAGE * (S - 1) ? 0u : sb + 4u * STAGE;
+                    }
+                    if (decltype(live)::value && c.fold) tl_acc.fold();      // (not in both loops: that doubles the registers)
                 }
             };
             if (q0 + wq * 32 < g.Q) k_loop(std::true_type{});
             else k_loop(std::false_type{});          // (rows past the last: only the loads)
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
-        if (g.nz > 1) {
+        if (g.nz > 1 || c.fold) {
             tl_acc.fold();
             __syncthreads();                     // (the next range's loads go where slower waves may still read)
         }
     }
-    if (g.nz > 1) tl_acc.unfold();
+    if (g.nz > 1 || c.fold) tl_acc.unfold();
     tl_acc.store(g, c, p0 + wp * 32, q0 + wq * 32, lane, bias, beta, out, partial);
 }
 
@@ -532,6 +539,7 @@ __global__ __launch_bounds__(256) void conv_f32_3x3_kernel(PixelGemm g, const fl
                 __builtin_amdgcn_sched_barrier(0);
             };
             unsigned sb = 0;
+            int until = c.fold;
             for (int st = 0; st < nsteps; ++st) {
                 const bool more = st + 1 < nsteps;
                 wait_loads_and_barrier<0>();
@@ -557,6 +565,10 @@ __global__ __launch_bounds__(256) void conv_f32_3x3_kernel(PixelGemm g, const fl
                 }
                 if (more) load_part(4);
                 sb = sb ? 0u : 4u * STAGE;
+                if (LIVE && --until == 0) {
+                    acc.fold();
+                    until = c.fold;
+                }
             }
         };
         if (nsteps > 0) {
@@ -565,12 +577,12 @@ __global__ __launch_bounds__(256) void conv_f32_3x3_kernel(PixelGemm g, const fl
             if (q0 + wq * 32 < g.Q) k_loop(std::true_type{});
             else k_loop(std::false_type{});          // (rows past the last: only the loads)
         }
-        if (g.nz > 1) {
+        if (g.nz > 1 || c.fold) {
             acc.fold();
             __syncthreads();                     // (the next range's loads go where slower waves may still read)
         }
     }
-    if (g.nz > 1) acc.unfold();
+    if (g.nz > 1 || c.fold) acc.unfold();
     acc.store(g, c, p0 + wp * 32, q0 + wq * 32, lane, bias, beta, out, partial);
 }
 
@@ -686,6 +698,7 @@ __global__ __launch_bounds__(256) void conv_f32_pixel_kernel(PixelGemm g, const 
     const __amdgpu_buffer_rsrc_t rsrcW = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(srcW), 0, g.bytesW, 0x00020000);
     unsigned voff[PH], wbase[WJ];
     TapMask<LONG> mask[PH];
+    const int fold = BWD ? c.fold : 0;           // (forward: ranges)
 #pragma unroll
     for (int h = 0; h < PH; ++h)
         pixel_source(g, c, p0 + h * 64 + lane, &voff[h], &mask[h]);
@@ -754,28 +767,32 @@ __global__ __launch_bounds__(256) void conv_f32_pixel_kernel(PixelGemm g, const 
                 for (int part = 0; part < 5; ++part) load_part(part);
             auto k_loop = [&](auto live) {
                 unsigned sb = 0;
-                for (int st = 0; st < nsteps; ++st) {
-                    wait_loads_and_barrier<LPI*(S - 2)>();
-                    tl_acc.template step<decltype(live)::value>(sb, load_part);
-                    sb = sb == 4u * STAGE * (S - 1) ? 0u : sb + 4u * STAGE;
+                for (int st = 0; st < nsteps;) {
+                    const int end = fold ? min(st + fold, nsteps) : nsteps;
+                    for (; st < end; ++st) {
+                        wait_loads_and_barrier<LPI*(S - 2)>();
+                        tl_acc.template step<decltype(live)::value>(sb, load_part);
+                        sb = sb == 4u * STAGE * (S - 1) ? 0u : sb + 4u * STAGE;
+                    }
+                    if (decltype(live)::value && fold) tl_acc.fold();      // (not in both loops: that doubles the registers)
                 }
             };
             if (q0 + wq * 32 < g.Q) k_loop(std::true_type{});
             else k_loop(std::false_type{});          // (rows past the last: only the loads)
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
-        if (g.nz > 1) {
+        if (g.nz > 1 || fold) {
             tl_acc.fold();
             __syncthreads();                     // (the next range's loads go where slower waves may still read)
         }
     }
-    if (g.nz > 1) tl_acc.unfold();
+    if (g.nz > 1 || fold) tl_acc.unfold();
     tl_acc.store(g, c, p0 + wp * 32, q0 + wq * 32, lane, BWD ? nullptr : bias, beta, out, partial);
 }
 
 // Backward-filter: both operands hold consecutive k (pixels), rows of 32 of them in LDS, two rows to a load.  Row pairs are
 // 272 bytes apart, so that 8 rows' 16-byte reads fall into different banks.
-template <int WQ, int WP, int S, bool LONG>
+template <int WQ, int WP, int S, bool LONG, bool FOLD>
 __global__ __launch_bounds__(256) void conv_f32_filter_kernel(FilterGemm g, const float* __restrict__ srcX, const float* __restrict__ srcY,
                                                               float* __restrict__ out)
 {
@@ -852,8 +869,13 @@ __global__ __launch_bounds__(256) void conv_f32_filter_kernel(FilterGemm g, cons
     };
 
     v16f acc;
+    double folded[16];                           // (FOLD)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    for (int r = 0; r < 16; ++r) { acc[r] = 0.0f; folded[r] = 0.0; }
+    auto fold = [&]() {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { folded[r] += (double)acc[r]; acc[r] = 0.0f; }
+    };
 
     // ---- fragments: group gi of a step: k = 4 (2 gi + lh) + 0..3
     const unsigned lrow = 4u * ((l32 >> 1) * PAIR + (l32 & 1) * 32) + 16u * lh;
@@ -881,26 +903,30 @@ __global__ __launch_bounds__(256) void conv_f32_filter_kernel(FilterGemm g, cons
                 acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[gi & 1][j], fb[gi & 1][j], acc, 0, 0, 0);
         };
         unsigned sb = 0;
-        for (int st = 0; st < nsteps; ++st) {
-            wait_loads_and_barrier<(PJ + QJ) * (S - 2)>();
-            read_group(std::integral_constant<int, 0>{}, sb);
-            locate();
-            issue_part(0);
-            wait_group(0);
-            read_group(std::integral_constant<int, 1>{}, sb);
-            mfma_group(0);
-            issue_part(1);
-            wait_group(1);
-            read_group(std::integral_constant<int, 2>{}, sb);
-            mfma_group(1);
-            issue_part(2);
-            wait_group(2);
-            read_group(std::integral_constant<int, 3>{}, sb);
-            mfma_group(2);
-            issue_part(3);
-            wait_group(3);
-            mfma_group(3);
-            sb = sb == 4u * STAGE * (S - 1) ? 0u : sb + 4u * STAGE;
+        for (int st = 0; st < nsteps;) {
+            const int end = FOLD ? min(st + g.fold, nsteps) : nsteps;
+            for (; st < end; ++st) {
+                wait_loads_and_barrier<(PJ + QJ) * (S - 2)>();
+                read_group(std::integral_constant<int, 0>{}, sb);
+                locate();
+                issue_part(0);
+                wait_group(0);
+                read_group(std::integral_constant<int, 1>{}, sb);
+                mfma_group(0);
+                issue_part(1);
+                wait_group(1);
+                read_group(std::integral_constant<int, 2>{}, sb);
+                mfma_group(1);
+                issue_part(2);
+                wait_group(2);
+                read_group(std::integral_constant<int, 3>{}, sb);
+                mfma_group(2);
+                issue_part(3);
+                wait_group(3);
+                mfma_group(3);
+                sb = sb == 4u * STAGE * (S - 1) ? 0u : sb + 4u * STAGE;
+            }
+            if (FOLD && LIVE) fold();
         }
     };
     if (nsteps > 0) {
@@ -921,7 +947,7 @@ __global__ __launch_bounds__(256) void conv_f32_filter_kernel(FilterGemm g, cons
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int q = q0 + wq * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-        if (q < g.Q) dst[(size_t)q * g.P + p] = acc[r];
+        if (q < g.Q) dst[(size_t)q * g.P + p] = FOLD ? (float)(folded[r] + (double)acc[r]) : acc[r];
     }
 }
 

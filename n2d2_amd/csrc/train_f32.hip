@@ -23,7 +23,7 @@ struct ConvF32 {
     int sx, sy, pl, pt, pr, pb, dx, dy;
     int depthwise;                                // groups == C == O
     int choice;                                   // the descriptor's kernel_choice bits
-    int ranges = 0;                               // a product that stands for a pass: least number of K ranges
+    int ranges = 0;                               // a product that stands for a pass: float sums of K / ranges terms at most
 };
 
 __device__ __forceinline__ double wave_sum_d(double v)
@@ -762,8 +762,8 @@ static int f32_path(const ConvF32& q, int pass)
     // As a convolution the K of a spanning layer's backward-data runs over all taps of an output, one of which is not zero: few
     // terms to a range.  As a product it has as many terms as outputs, so it adds in double up to 5e8 flops (64 images,
     // 64 x 4 x 4 <- 256: 2.5e-8 from 64 bits and 10 us; convolution 7.7e-8, 41 us; product in float 2.9e-7, 14 us) and beyond
-    // takes as many ranges as the convolution would (128 images, 512 x 2 x 2 <- 1000: 1.5e-7 and 26 us; in double 36; convolution
-    // 1.5e-7, 64; 64 images, 512 x 7 x 7 <- 4096: 179 us, in double 1019, convolution 9566).
+    // has float sums as short as the convolution's (128 images, 512 x 2 x 2 <- 1000: 1.5e-7 and 22 us; in double 36; convolution
+    // 1.5e-7, 64; 64 images, 512 x 7 x 7 <- 4096: 177 us, in double 1019, convolution 9566).
     if (pass == PASS_BWD_DATA && (forced || !small) && flops < 5.0e8 && !many_taps(q) && q.kH * q.kW > 1 && q.B <= 16 * GRID_Y && spans_input(q))
         return F32_PATH_SMALL;
     if (forced) return F32_PATH_GEMM;
@@ -865,7 +865,7 @@ static int pass_ranges(long P, int Q, long K)
 //   forward          y[b][o] = sum_k x[b][k] w[o][k]     the filter pass of pixels k between "channels" w[o] and "outputs" x[b]
 //   backward data    dx[b][k] = sum_o dy[b][o] w[o][k]   the forward pass over one "image" w of O channels and K pixels
 //   backward filter  dw[o][k] = sum_b dy[b][o] x[b][k]   the data pass over one "image" x of B channels and K pixels
-// Forward and backward data run at least as many ranges as the convolution itself would, so that no float sum is longer.
+// Forward and backward data have no longer float sums than the convolution itself would.
 static ConvF32 product_of(const ConvF32& q, int pass, int* as_pass)
 {
     const int K = q.C * q.H * q.W, T = q.H * q.W;
@@ -970,23 +970,25 @@ static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass>
         // 1 x 31, 256 tiles: 102 us with one, 82 with partial results).
         splits = pass_ranges(P, g.Q, kmax);
     } else {
-        // where the tiles do not fill the chip twice; none below four steps.  And as many ranges as over all taps at 128 x 128
-        // tiles: the longer a float sum, the more it loses (256 -> 256, 3x3, 14 x 14, batch 32: one range 8.3e-7 from 64 bits and
-        // 89 us, seven folded in double 3.1e-7 and 96).
+        // where the tiles do not fill the chip twice; none below four steps.  And no float sum longer than over all taps at 128 x
+        // 128 tiles: the longer, the more it loses (256 -> 256, 3x3, 14 x 14, batch 32: one sum 8.3e-7 from 64 bits and 89 us,
+        // seven added in double as the steps go 3.1e-7 and 91, as ranges that each fill the ring anew 97).
         splits = blocks >= 512 ? 1 : std::max(1L, 768 / blocks);
         splits = std::min<long>(splits, std::max(1L, kmax / (4 * GK)));
         least = pass_ranges((long)q.B * q.H * q.W, q.C, (long)q.O * T);
     }
-    const int step = !fwd && kind == PIXELS_3X3 ? K33 : GK;
+    const int step = kind == PIXELS_3X3 ? K33 : GK;
     pl.splits = 1;
     for (int i = 0; i < g.nclass; ++i) {         // (the ranges of a class of fewer taps are as many, and shorter)
         const long K = (long)kch * cls[i].nT;
-        cls[i].kchunk = std::max(least > splits ? (int)(K / least) / step * step : round_up((int)((K + splits - 1) / splits), GK), step);
+        const bool ranges = fwd && kind == PIXELS_TAPS && least > splits;        // (the forward pixel kernel does not fold)
+        cls[i].kchunk = std::max(ranges ? (int)(K / least) / GK * GK : round_up((int)((K + splits - 1) / splits), GK), GK);
+        cls[i].fold = least > splits && !ranges ? std::max((int)(K / least) / step, 1) : 0;
         pl.splits = std::max(pl.splits, ceil_div_i(K, cls[i].kchunk));
         if (kind == PIXELS_CHUNK) cls[i].kchunk /= GK;
         g.c[i] = cls[i];
     }
-    if (blocks >= (fwd && !pl.many ? 256 : 512)) {
+    if (fwd && blocks >= (pl.many ? 512 : 256)) {
         g.nz = pl.splits;
         pl.splits = 1;
     }
@@ -1047,11 +1049,13 @@ static FilterPlan plan_filter(const ConvF32& q)
     // blocks; many: three blocks per tile or six per CU)
     long splits = tiles <= 256 ? (pl.small_q ? 512 : 1024) / tiles : std::max(1L, (1535 + tiles) / tiles);
     splits = std::min<long>(splits, std::max(1, g.K / (4 * FK)));
-    // At least as many as 128 x 128 tiles would take, none of those below 512 pixels: the longer a float sum, the more it loses
-    // (256 -> 256, 3x3, 14 x 14, batch 32: 7 ranges 5.1e-7 from 64 bits and 90 us, 13 ranges 3.8e-7 and 95).
+    // No float sum longer than the ranges that 128 x 128 tiles would take, none of those below 512 pixels: the longer, the more
+    // it loses (256 -> 256, 3x3, 14 x 14, batch 32: sums of 896 pixels 5.1e-7 from 64 bits and 89 us, of 512 3.7e-7 and 90, with
+    // as many partial results 95).
     const long tiles128 = (long)ceil_div_i(g.P, 128) * (g.Q <= 64 ? 1 : ceil_div_i(g.Q, 128));
     const long least = q.ranges ? q.ranges : std::min<long>(std::max(1L, 1024 / tiles128), std::max(1, g.K / (16 * FK)));
-    g.kchunk = least > splits ? std::max((int)(g.K / least) / FK * FK, FK) : round_up((int)((g.K + splits - 1) / splits), FK);
+    g.kchunk = round_up((int)((g.K + splits - 1) / splits), FK);
+    g.fold = least > splits ? std::max((int)(g.K / least) / FK, 1) : 0;
     pl.splits = ceil_div_i(g.K, g.kchunk);
     return pl;
 }
@@ -1091,12 +1095,13 @@ static int run_small_filter(FilterGemm g, const float* x, const float* dy, float
 static void launch_filter(const FilterPlan& pl, const float* x, const float* dy, float* out, hipStream_t st)
 {
     const dim3 grid(ceil_div_i(pl.g.P, pl.small_q ? 128 : 64), ceil_div_i(pl.g.Q, pl.small_q ? 32 : 64), pl.splits);
-    const auto run = [&](auto long_) {
-        constexpr bool LONG = decltype(long_)::value;
-        if (pl.small_q) hipLaunchKernelGGL((conv_f32_filter_kernel<1, 4, 2, LONG>), grid, dim3(256), 0, st, pl.g, x, dy, out);
-        else hipLaunchKernelGGL((conv_f32_filter_kernel<2, 2, 2, LONG>), grid, dim3(256), 0, st, pl.g, x, dy, out);
+    const auto run = [&](auto long_, auto fold_) {
+        constexpr bool LONG = decltype(long_)::value, FOLD = decltype(fold_)::value;
+        if (pl.small_q) hipLaunchKernelGGL((conv_f32_filter_kernel<1, 4, 2, LONG, FOLD>), grid, dim3(256), 0, st, pl.g, x, dy, out);
+        else hipLaunchKernelGGL((conv_f32_filter_kernel<2, 2, 2, LONG, FOLD>), grid, dim3(256), 0, st, pl.g, x, dy, out);
     };
-    pl.g.kH + pl.g.kW > 31 ? run(std::true_type{}) : run(std::false_type{});
+    const auto pick = [&](auto long_) { pl.g.fold ? run(long_, std::true_type{}) : run(long_, std::false_type{}); };
+    pl.g.kH + pl.g.kW > 31 ? pick(std::true_type{}) : pick(std::false_type{});
 }
 
 // The order of K.  3x3 kernels, forward or at stride 1: four channels with their taps at a time.  Chunks of 16 channels at one
