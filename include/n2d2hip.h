@@ -296,6 +296,31 @@ int n2d2hip_conv_accepts_maxpool(n2d2hip_conv_t conv, const n2d2hip_pool_desc* p
 int n2d2hip_conv_forward_maxpool(n2d2hip_conv_t conv, const n2d2hip_pool_desc* pool, const n2d2hip_tensor* in,
                                  const n2d2hip_tensor* out, n2d2hip_stream_t stream);
 
+/* Graph-level fusion of a small network's first cells (a whole LeNet): up to 8 convolutions and max poolings, each reading
+ * the one before, and the run of fully-connected cells behind them if there is one, in one launch; that is their propagate()
+ * in turn (ref: src/Cell/ConvCell_Frame.cpp:418-473, src/Cell/PoolCell_Frame.cpp:123-174, src/Cell/FcCell_Frame.cpp:234-340),
+ * results bit for bit those of the separate launches, and every output tensor is written as they write it (but the vectors
+ * between the fully-connected cells, as with n2d2hip_fc_chain_forward).  H x W: the size of the first cell's input.  The
+ * handles are borrowed and must outlive the run.  Returns N2D2HIP_ERR_UNSUPPORTED (the caller keeps the separate launches)
+ * unless the first cell is a convolution, every convolution has 8-bit weights, at most 16 inputs, 32 outputs and 64 taps and
+ * an output of bytes, no pooling window is empty, and tensors and weights fit 64 KB. */
+typedef struct n2d2hip_run_cell { /* one of the three, the others NULL; fcs only as the last */
+    n2d2hip_conv_t conv;
+    const n2d2hip_pool_desc* pool;
+    n2d2hip_fc_chain_t fcs;
+    int out_dtype;                /* storage type of the cell's output: U8B or I8 (the last cell's: any it can store) */
+} n2d2hip_run_cell;
+typedef struct n2d2hip_cell_run_s* n2d2hip_cell_run_t;
+int n2d2hip_cell_run_create(int nb_cells, const n2d2hip_run_cell* cells, int H, int W, n2d2hip_cell_run_t* run);
+int n2d2hip_cell_run_destroy(n2d2hip_cell_run_t run);
+/* 1 when the library expects the launch to be faster than the cells' own for this batch, else 0. */
+int n2d2hip_cell_run_pays(n2d2hip_cell_run_t run, int batch);
+/* `in`: the first cell's input (NHWC, no halo); `outs`: the output of every cell (nb_cells of them).  `edge`: NULL, or the
+ * network's byte planes (NCHW U8 for a U8B input, I8 for I8, at most 4 channels): `in` is then written from them first, as
+ * n2d2hip_convert(edge, in) does, in the same launch. */
+int n2d2hip_cell_run_forward(n2d2hip_cell_run_t run, const n2d2hip_tensor* edge, const n2d2hip_tensor* in,
+                             const n2d2hip_tensor* outs, n2d2hip_stream_t stream);
+
 /* -------------------------------------------------------------- elemwise */
 enum { N2D2HIP_COEFF_PER_LAYER = 0, N2D2HIP_COEFF_PER_INPUT = 1, N2D2HIP_COEFF_PER_CHANNEL = 2 };
 typedef struct n2d2hip_elemwise_s* n2d2hip_elemwise_t;

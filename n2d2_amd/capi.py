@@ -34,6 +34,7 @@ SYMBOLS = [
     "n2d2hip_conv_accepts_maxpool", "n2d2hip_conv_forward_maxpool", 
     "n2d2hip_dw_pw_create", "n2d2hip_dw_pw_destroy", "n2d2hip_dw_pw_forward", "n2d2hip_dw_pw_pays",
     "n2d2hip_fc_create", "n2d2hip_fc_destroy", "n2d2hip_fc_forward", "n2d2hip_fc_chain_create", "n2d2hip_fc_chain_destroy", "n2d2hip_fc_chain_forward",
+    "n2d2hip_cell_run_create", "n2d2hip_cell_run_destroy", "n2d2hip_cell_run_pays", "n2d2hip_cell_run_forward",
     "n2d2hip_pool_out_dims", "n2d2hip_pool_forward", "n2d2hip_pool_writes_halo", "n2d2hip_pool_forward_mapped",
     "n2d2hip_elemwise_create", "n2d2hip_elemwise_destroy", "n2d2hip_elemwise_forward", "n2d2hip_elemwise_fold_input_scaling", "n2d2hip_concat_channels",
     "n2d2hip_quantizer_workspace_bytes", "n2d2hip_sat_weight_forward", "n2d2hip_sat_weight_forward_static", "n2d2hip_sat_weight_backward",
@@ -71,6 +72,10 @@ class ConvDesc(C.Structure):
 class PoolDesc(C.Structure):
     _fields_ = [("pooling", C.c_int), ("poolW", C.c_int), ("poolH", C.c_int), ("strideX", C.c_int), ("strideY", C.c_int),
                 ("padX", C.c_int), ("padY", C.c_int)]
+
+
+class RunCell(C.Structure):
+    _fields_ = [("conv", C.c_void_p), ("pool", C.POINTER(PoolDesc)), ("fcs", C.c_void_p), ("out_dtype", C.c_int)]
 
 
 class N2D2HipError(RuntimeError):
@@ -131,6 +136,10 @@ def load():
     lib.n2d2hip_fc_chain_create.argtypes = [I, P, P]
     lib.n2d2hip_fc_chain_destroy.argtypes = [P]
     lib.n2d2hip_fc_chain_forward.argtypes = [P, P, P, P]
+    lib.n2d2hip_cell_run_create.argtypes = [I, P, I, I, P]
+    lib.n2d2hip_cell_run_destroy.argtypes = [P]
+    lib.n2d2hip_cell_run_pays.argtypes = [P, I]
+    lib.n2d2hip_cell_run_forward.argtypes = [P, P, P, P, P]
     lib.n2d2hip_pool_out_dims.argtypes = [P, I, I, P, P]
     lib.n2d2hip_pool_forward.argtypes = [P, P, P, P]
     lib.n2d2hip_pool_writes_halo.argtypes = [P, I, I, I]

@@ -46,6 +46,10 @@ struct n2d2hip_conv_s {
     signed char* d_w4img;
     // direct kernel for layers with a handful of channels: [tap][8 | 16 | 32 output rows][input channel stride]
     signed char* d_wsmall;
+    // what a run of small cells copies into its own image (cell_run.hip), kept on the host: the biases of a cell of at most 128
+    // outputs, and the direct kernel's weights
+    std::vector<int> hbias;
+    std::vector<signed char> hsmall;
     bool is_fc;
     int fcH, fcW;
     // sub-sampling (desc.subX or subY > 1): the convolution proper is a handle of its own that stores raw sums without a

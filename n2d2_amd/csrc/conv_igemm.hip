@@ -767,6 +767,8 @@ int n2d2hip_conv_create(const n2d2hip_conv_desc* d, const void* weights, const i
     if (e == hipSuccess) e = hipMemcpy(c->d_w, hw.data(), hw.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMalloc((void**)&c->d_bias, hbias.size() * sizeof(int));
     if (e == hipSuccess) e = hipMemcpy(c->d_bias, hbias.data(), hbias.size() * sizeof(int), hipMemcpyHostToDevice);
+    if (d->O <= 128)
+        c->hbias.assign(hbias.begin(), hbias.begin() + d->O);
     if (e == hipSuccess && c->pix4 && d->weight_bits == 8 && d->strideX == 2 && d->dilX == 1 && d->dilY == 1 && d->kW <= 8
         && (d->kH == 3 || d->kH == 5 || d->kH == 7)) {
         // [channel][kernel row][8 tap slots][4 channel slots], zero where the kernel has nothing
@@ -804,6 +806,7 @@ int n2d2hip_conv_create(const n2d2hip_conv_desc* d, const void* weights, const i
         conv_small_weight_layout(ohwc.data(), d->C, d->O, taps, img.data());
         e = hipMalloc((void**)&c->d_wsmall, img.size());
         if (e == hipSuccess) e = hipMemcpy(c->d_wsmall, img.data(), img.size(), hipMemcpyHostToDevice);
+        c->hsmall.swap(img);
     }
     if (e == hipSuccess && !hfrag.empty()) {
         e = hipMalloc((void**)&c->d_wfrag, hfrag.size());

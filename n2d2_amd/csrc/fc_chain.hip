@@ -13,10 +13,9 @@
 #include "common.h"
 #include "conv_handle.hpp"
 #include "epilogue.hpp"
+#include "fc_chain.hpp"
 
 namespace n2d2hip {
-
-enum { FC_CHAIN_MAX = 3, FC_CHAIN_K4 = 256 /* dwords of K per cell at most */, FC_CHAIN_O = 128 };
 
 struct FcChainArgs {
     const signed char* in;      // B images of in_bytes contiguous bytes (NHWC with the channel stride equal to the channels)
@@ -93,13 +92,6 @@ __global__ __launch_bounds__(FC_CHAIN_O) void fc_chain_kernel(const FcChainArgs 
 
 using namespace n2d2hip;
 
-struct n2d2hip_fc_chain_s {
-    int n;
-    n2d2hip_fc_t fc[FC_CHAIN_MAX];
-    unsigned* d_wt[FC_CHAIN_MAX];
-    int k4[FC_CHAIN_MAX];
-};
-
 extern "C" {
 
 int n2d2hip_fc_chain_destroy(n2d2hip_fc_chain_t h)
@@ -144,6 +136,7 @@ int n2d2hip_fc_chain_create(int n, const n2d2hip_fc_t* fcs, n2d2hip_fc_chain_t* 
             e = hipMalloc((void**)&h->d_wt[l], wt.size() * sizeof(unsigned));
         }
         if (e == hipSuccess) e = hipMemcpy(h->d_wt[l], wt.data(), wt.size() * sizeof(unsigned), hipMemcpyHostToDevice);
+        h->hwt[l].swap(wt);
         if (e != hipSuccess) {
             n2d2hip_fc_chain_destroy(h);
             return fail(N2D2HIP_ERR_HIP, "fc_chain_create: moving the weights failed: %s", hipGetErrorString(e));

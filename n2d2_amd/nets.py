@@ -391,7 +391,7 @@ class GpuNet:
     Activations stay on the device in the private NHWC form between cells; all buffers are allocated once."""
 
     def __init__(self, spec, batch, fuse=True, halo=True, kernel_choice=0, bottlenecks="projection", stem_pool=True,
-                 dw_pw=True, s2d=True, chains=True, fc_chains=True):
+                 dw_pw=True, s2d=True, chains=True, fc_chains=True, cell_runs=True):
         """fuse: fold a ScalingCell whose only consumer is an ElemWise sum into that sum (one pass instead of two;
         the rescaled tensor is never written), and a two-input sum into the 1x1 convolution that feeds it.
         halo: a tensor written by a convolution and read only by convolutions is stored with the readers' padding as
@@ -409,6 +409,9 @@ class GpuNet:
         one cell reading it is a first-layer convolution the library serves that way (n2d2hip_conv_s2d_halo).
         fc_chains: run two or three fully-connected cells, each the only reader of the one before, as one launch
         (n2d2hip_fc_chain_*) where the library takes them.
+        cell_runs: forward() runs the small convolutions, max poolings and fully-connected cells a network begins with as one
+        launch (n2d2hip_cell_run_*) where the library takes them; every tensor is written all the same, and what addresses
+        the cells one by one (forward_subset, forward_timed, kernel_names) still launches them one by one.
         chains: run a block's 3x3 convolution in the launch of the expanding 1x1 convolution + sum that alone reads it
         (n2d2hip_conv_chain_*) where the library takes the pair: the 3x3 convolution's output stays on the chip.  Where the
         library expects two launches to be faster (n2d2hip_conv_chain_pays) the step makes two."""
@@ -661,6 +664,30 @@ class GpuNet:
         self.steps = [self.steps[k] for k in keep]
         self._io = [self._io[k] for k in keep]
         self.launched = [spec.layers[k] for k in keep]
+        # the cells the network begins with, each reading the one before, as one launch
+        self.cell_run, self._run_steps = None, 0
+        if fuse and cell_runs:
+            self._plan_cell_run()
+
+    def _plan_cell_run(self):
+        rt, run, src = self.rt, [], self.input
+        for (l, cell, fn), (ins, out) in zip(self.steps, self._io):
+            if (len(ins) != 1 or ins[0] is not src or src.halo or out.halo or src.layout != self.capi.NHWC or l.name in self.stem_pools
+                    or type(cell) not in (rt.Conv, rt.Pool, rt.FcChain)):
+                break
+            run.append((cell, out))
+            src = out
+        # (a shorter run where the library declines the last cells; a run of one or two cells is left to their launches)
+        while len(run) > 2:
+            self.cell_run = rt.CellRun.create([c for c, o in run], self.input, [o for c, o in run])
+            if self.cell_run is not None:
+                # (with thousands of images the cells' own launches fill the chip)
+                if not self.cell_run.pays(self.B):
+                    self.cell_run = None
+                else:
+                    self._run_steps = len(run)
+                return
+            run.pop()
 
     def _plan_chains(self, consumers, by_name, ins_of):
         """For every sum folded into the expanding 1x1 convolution of a block (and not part of a whole-block launch): the 3x3
@@ -794,9 +821,24 @@ class GpuNet:
             self.input.convert_from(self.input_src)
 
     def forward(self):
-        for (l, cell, fn), (ins, out) in zip(self.steps, self._io):
+        if self.cell_run is not None:
+            self.cell_run.forward()
+        return self._forward_rest()
+
+    def _forward_rest(self):
+        for k in range(self._run_steps, len(self.steps)):
+            l, cell, fn = self.steps[k]
+            ins, out = self._io[k]
             fn(cell, ins, out)
         return self.tensors[self.spec.output]
+
+    def _convert_and_forward(self):
+        """convert_input() and forward(), the conversion in the launch of the first cells where that takes it."""
+        if self.cell_run is not None and self._input_plain is None and self.cell_run.takes_edge(self.input_src):
+            self.cell_run.forward(self.input_src)
+            return self._forward_rest()
+        self.convert_input()
+        return self.forward()
 
     def capture(self, forwards=1, with_input_conversion=False):
         """Records `forwards` forwards, one behind the other, into a HIP graph (every launch of the C ABI goes to the
@@ -813,13 +855,21 @@ class GpuNet:
             with torch.cuda.graph(graph, stream=side):
                 for _ in range(forwards):
                     if with_input_conversion:
-                        self.convert_input()
-                    self.forward()
+                        self._convert_and_forward()
+                    else:
+                        self.forward()
         torch.cuda.synchronize()
         self._graph = graph
+        replay_graph = graph.replay
+        if forwards == 1 and self._run_steps == len(self.steps) and self._run_steps > 0:
+            # a graph of one launch costs more than the launch (14.1 against 8.6 us for one LeNet image): the same launch, with
+            # the same buffers, without it
+            src = self.input_src if with_input_conversion else None
+            if src is None or (self._input_plain is None and self.cell_run.takes_edge(src)):
+                replay_graph = lambda: self.cell_run.forward(src)      # noqa: E731
 
         def replay():
-            graph.replay()
+            replay_graph()
             return self.tensors[self.spec.output]
         return replay
 

@@ -351,6 +351,53 @@ class FcChain:
             self.handle = None
 
 
+class CellRun:
+    """n2d2hip_cell_run_t: the convolutions, max poolings and fully-connected cells of a small network as one launch."""
+
+    def __init__(self, handle, cells, in_edge, outs):
+        self.handle, self.cells = handle, cells     # the cells' handles are borrowed: keep them alive
+        self.in_edge, self.outs = in_edge, outs
+        self._outs = (capi.Tensor * len(outs))(*[o.desc for o in outs])
+
+    @staticmethod
+    def create(cells, x, outs):
+        """cells: Conv and Pool objects in order, a FcChain possibly last; x: the first one's input; outs: their outputs.
+        None when the library keeps the cells apart."""
+        arr = (capi.RunCell * len(cells))()
+        for k, c in enumerate(cells):
+            arr[k].out_dtype = outs[k].dtype
+            if isinstance(c, Pool):
+                arr[k].pool = C.pointer(c.desc)
+            elif isinstance(c, FcChain):
+                arr[k].fcs = c.handle
+            else:
+                arr[k].conv = c.handle
+        h = C.c_void_p()
+        rc = lib.n2d2hip_cell_run_create(len(cells), arr, x.H, x.W, C.byref(h))
+        if rc == capi.ERR_UNSUPPORTED:
+            return None
+        check(rc)
+        return CellRun(h, list(cells), x, list(outs))
+
+    def pays(self, batch):
+        return bool(lib.n2d2hip_cell_run_pays(self.handle, batch))
+
+    def takes_edge(self, src):
+        """True when the conversion of these byte planes into the first cell's input can be part of the launch."""
+        x = self.in_edge
+        return (src.layout == capi.NCHW and x.cs == 4 and (src.B, src.C, src.H, src.W) == (x.B, x.C, x.H, x.W)
+                and src.dtype == (capi.U8 if x.dtype == capi.U8B else capi.I8))
+
+    def forward(self, edge=None):
+        """edge: the network's byte planes, converted into the first cell's input on the way, or None."""
+        check(lib.n2d2hip_cell_run_forward(self.handle, None if edge is None else edge.ref, self.in_edge.ref, self._outs, stream_ptr()))
+
+    def __del__(self):
+        if getattr(self, "handle", None) and lib is not None:
+            lib.n2d2hip_cell_run_destroy(self.handle)
+            self.handle = None
+
+
 class Pool:
     def __init__(self, kind, pool, stride, pad=(0, 0), maps=None):
         """maps: None for one output per channel, else a bool array [channels, outputs] (maps[c, o]: output o pools channel c)."""

@@ -1,0 +1,75 @@
+"""The first cells of a small network in one launch (n2d2hip_cell_run_*): every tensor against the cells launched one by one,
+the outputs against the CPU oracle.  Integers: bit for bit."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# name, input shape, input unsigned, rescale mode, cells: ("conv", outputs, kernel, stride, pad) / ("pool", kernel, stride, pad) / ("fc", outputs)
+NETS = [
+    ("lenet_like", (1, 28, 28), True, "FixedMult32", [("conv", 6, 5, 1, 0), ("pool", 2, 2, 0), ("conv", 16, 5, 1, 0), ("pool", 2, 2, 0),
+                                                     ("fc", 120), ("fc", 84), ("fc", 10)]),
+    # padded windows, 32 outputs (two blocks), overlapping padded pooling, sizes that fill no tile, signed input
+    ("padded", (3, 13, 11), False, "SingleShift", [("conv", 16, 4, 2, 1), ("conv", 32, 3, 1, 1), ("pool", 3, 2, 1), ("fc", 128), ("fc", 7)]),
+    # one pixel left, four channels all the way (channel stride 4), 8 x 8 kernel of 64 taps, float rescale
+    ("four_channels", (4, 17, 19), True, "FloatMult", [("conv", 4, 8, 1, 0), ("conv", 3, 7, 3, 3), ("pool", 4, 4, 0), ("conv", 9, 1, 1, 0)]),
+    # 16 input channels, the largest K, no fully-connected cell
+    ("wide", (16, 9, 21), True, "DoubleShift", [("conv", 16, 7, 2, 3), ("conv", 17, 2, 1, 0), ("pool", 2, 1, 0)]),
+    # a first fully-connected cell of 1024 inputs
+    ("long_vector", (2, 10, 10), False, "FixedMult16", [("conv", 16, 3, 1, 0), ("pool", 1, 1, 0), ("conv", 16, 1, 1, 0), ("fc", 100), ("fc", 33)]),
+]
+
+
+@pytest.mark.parametrize("batch", [1, 3, 261])
+@pytest.mark.parametrize("case", NETS, ids=[c[0] for c in NETS])
+def test_cells_in_one_launch_bit_exact(case, batch):
+    from n2d2_amd import capi, nets
+    from oracle import cells
+    name, shape, unsigned, mode, plan = case
+    b = nets._Builder(name, shape, 5, mode, unsigned_data=unsigned)
+    b.spec.input_unsigned = unsigned
+    b.spec.unsigned["input"] = unsigned
+    x = "input"
+    for k, c in enumerate(plan):
+        if c[0] == "conv":
+            x = b.conv("c%d" % k, x, c[1], c[2], c[3], c[4])
+        elif c[0] == "pool":
+            x = b.pool("p%d" % k, x, "max", c[1], c[2], c[3])
+        else:
+            last = k + 1 == len(plan)
+            x = b.fc("f%d" % k, x, c[1], kind="Linear" if last else "Rectifier", **({"mode": "None"} if last else {}))
+    lo, hi = (0, 256) if unsigned else (-128, 128)
+    img = np.random.default_rng(batch).integers(lo, hi, size=(batch,) + shape)
+    print(name, batch, flush=True)
+    run = nets.GpuNet(b.spec, batch)
+    apart = nets.GpuNet(b.spec, batch, cell_runs=False)
+    assert run.cell_run is not None and run._run_steps == len(run.steps)
+    for net in (run, apart):
+        net.set_input(img)
+    with capi.launch_log() as log:
+        run.forward()
+    assert [e[0] for e in log.entries] and all("cell_run_kernel" in e[0] for e in log.entries) and len(log.entries) == 1
+    apart.forward()
+    for n, t in apart.tensors.items():
+        used = t.cs if t.dtype != capi.I32 else t.C         # (channels past the last one: the stored 0, but not behind integers)
+        a, b2 = (net.tensors[n].buf.cpu().numpy().reshape(-1, t.cs)[:, :used] for net in (run, apart))
+        assert np.array_equal(a, b2), n
+    got = run.tensors[b.spec.output].to_numpy()
+    want = cells.run_net(b.spec, img[:3])[b.spec.output].astype(np.int64)
+    assert np.array_equal(got[:3], want)
+    # from the byte planes, replayed from a graph with other work between the replays
+    edge_in_launch = run.cell_run.takes_edge(run.input_src)
+    assert edge_in_launch == (shape[0] <= 4)
+    replay = run.capture(1, with_input_conversion=True)
+    for _ in range(3):
+        for n in run.tensors:
+            run.tensors[n].buf.fill_(7)
+        assert np.array_equal(replay().to_numpy(), got)
+        assert np.array_equal(run.input.buf.cpu().numpy(), apart.input.buf.cpu().numpy())
+
+
+def test_large_batches_keep_their_own_launches():
+    from n2d2_amd import nets
+    spec = nets.lenet()
+    assert nets.GpuNet(spec, 4096).cell_run is not None
+    assert nets.GpuNet(spec, 4097).cell_run is None
