@@ -313,8 +313,6 @@ typedef struct n2d2hip_run_cell { /* one of the three, the others NULL; fcs only
 typedef struct n2d2hip_cell_run_s* n2d2hip_cell_run_t;
 int n2d2hip_cell_run_create(int nb_cells, const n2d2hip_run_cell* cells, int H, int W, n2d2hip_cell_run_t* run);
 int n2d2hip_cell_run_destroy(n2d2hip_cell_run_t run);
-/* 1 when the library expects the launch to be faster than the cells' own for this batch, else 0. */
-int n2d2hip_cell_run_pays(n2d2hip_cell_run_t run, int batch);
 /* `in`: the first cell's input (NHWC, no halo); `outs`: the output of every cell (nb_cells of them).  `edge`: NULL, or the
  * network's byte planes (NCHW U8 for a U8B input, I8 for I8, at most 4 channels): `in` is then written from them first, as
  * n2d2hip_convert(edge, in) does, in the same launch. */

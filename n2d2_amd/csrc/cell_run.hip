@@ -6,7 +6,8 @@
 // a work-group of 8 waves takes one image through all the cells with its tensors in LDS; what a cell hands to the next
 // costs a barrier instead of a launch.  Each cell's output is also stored to its tensor, as the cells run in turn do (the
 // stores wait for nobody), so a caller finds the same values everywhere.  LeNet, conversion of the bytes included: one image
-// 33.9 -> 8.6 us, 256 images launched one by one 45.7 -> 15.8 us.  Of the launch's 8 us, 2 go by until the image and the weights
+// 33.9 -> 8.6 us, 256 images launched one by one 45.7 -> 14.8 us, 2048 images 82 -> 66 us, 16384 images (64 one after the other on
+// a compute unit) 463 -> 456 us: the cells' own launches, which then fill the chip, are never ahead.  Of the launch's 8 us, 2 go by until the image and the weights
 // are there, 3 in the first convolution (instruction issue), and the other five cells take about 0.5 each: a descriptor, a
 // few dependent LDS reads and a barrier.  16 waves took as long (each pays for its cells' descriptors and set-up).
 //
@@ -730,15 +731,6 @@ int n2d2hip_cell_run_create(int nb_cells, const n2d2hip_run_cell* cells, int H, 
     r->long_fc = a.kper > 32;
     *out = r;
     return N2D2HIP_OK;
-}
-
-int n2d2hip_cell_run_pays(n2d2hip_cell_run_t r, int batch)
-{
-    // An image is one work-group's, 8 us on a compute unit whatever the batch: LeNet's forward with its conversion takes 8.6 us
-    // against 34 for one image, 10 against 42 for 256, 64 against 113 for 2048, and from 16 images a compute unit on the cells'
-    // own launches, which use every one of its lanes, draw level (4096: 179 against 180 launched one by one; 16384: 693
-    // against 659).
-    return r && batch > 0 && batch <= 16 * num_cus() ? 1 : 0;
 }
 
 int n2d2hip_cell_run_forward(n2d2hip_cell_run_t r, const n2d2hip_tensor* edge, const n2d2hip_tensor* in, const n2d2hip_tensor* outs, n2d2hip_stream_t stream)

@@ -681,11 +681,7 @@ class GpuNet:
         while len(run) > 2:
             self.cell_run = rt.CellRun.create([c for c, o in run], self.input, [o for c, o in run])
             if self.cell_run is not None:
-                # (with thousands of images the cells' own launches fill the chip)
-                if not self.cell_run.pays(self.B):
-                    self.cell_run = None
-                else:
-                    self._run_steps = len(run)
+                self._run_steps = len(run)
                 return
             run.pop()
 

@@ -379,9 +379,6 @@ class CellRun:
         check(rc)
         return CellRun(h, list(cells), x, list(outs))
 
-    def pays(self, batch):
-        return bool(lib.n2d2hip_cell_run_pays(self.handle, batch))
-
     def takes_edge(self, src):
         """True when the conversion of these byte planes into the first cell's input can be part of the launch."""
         x = self.in_edge

@@ -68,8 +68,22 @@ def test_cells_in_one_launch_bit_exact(case, batch):
         assert np.array_equal(run.input.buf.cpu().numpy(), apart.input.buf.cpu().numpy())
 
 
-def test_large_batches_keep_their_own_launches():
-    from n2d2_amd import nets
-    spec = nets.lenet()
-    assert nets.GpuNet(spec, 4096).cell_run is not None
-    assert nets.GpuNet(spec, 4097).cell_run is None
+@pytest.mark.parametrize("shape", [(1, 1, 2, 2), (3, 1, 32, 32), (5, 3, 7, 4), (2, 4, 6, 10), (2, 2, 5, 5), (513, 3, 33, 36)])
+@pytest.mark.parametrize("src,dst", [("U8", "U8B"), ("U8", "U8"), ("I8", "I8"), ("U8", "I8"), ("I8", "U8B")])
+def test_byte_planes_to_pixels_of_four_channels(shape, src, dst):
+    """The graph edge's conversion: every stored byte, from aligned planes, and from planes that begin at an odd address."""
+    import torch
+    from n2d2_amd import capi, runtime as rt
+    B, C, H, W = shape
+    x = np.random.default_rng(7).integers(*((0, 256) if src == "U8" else (-128, 128)), size=shape)
+    lo, hi, off = {"U8B": (0, 255, -128), "U8": (0, 255, 0), "I8": (-128, 127, 0)}[dst]
+    want = np.zeros((B, H, W, 4), np.int64)
+    want[..., :C] = np.clip(x, lo, hi).transpose(0, 2, 3, 1)
+    want = (want + off).astype(np.uint8).reshape(-1)
+    flat = torch.from_numpy(x.astype(np.uint8 if src == "U8" else np.int8).reshape(-1))
+    for shift in (0, 1):
+        buf = torch.zeros(flat.numel() + 16, dtype=flat.dtype, device="cuda")[shift:shift + flat.numel()]
+        buf.copy_(flat)
+        t = rt.DTensor(B, C, H, W, getattr(capi, src), capi.NCHW, buf)
+        out = rt.DTensor(B, C, H, W, getattr(capi, dst)).convert_from(t)
+        assert np.array_equal(out.buf.cpu().numpy().view(np.uint8).reshape(-1), want), shift
