@@ -287,6 +287,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 
 } // namespace n2d2hip
 #include "conv_pipe.hpp"
+#include "conv_split.hpp"
 #include "conv_stem.hpp"
 #include "conv_small.hpp"
 namespace n2d2hip {
@@ -1162,6 +1163,11 @@ static int conv_forward_impl(n2d2hip_conv_t c, const n2d2hip_tensor* in, const n
         // 196 / 196, 32 276 / - / 265 / 269.
         const bool tiny = small_m && !other && ((Mll + 63) / 64) * a.ntiles_n < num_cus();
         if (tiny) q.c.ntiles_n = a.ntiles_n = (round_up(d.O, 16) + 63) / 64;
+        // Few tiles and a long K: smaller tiles whose waves share K
+        const int kind = c->act->args.kind;
+        const bool split = conv_split_takes(d, kind, all_valid) && (kind != EPI_I24 || c->bias_folded)
+            && !(d.kernel_choice & (N2D2HIP_KERNEL_TILE_M64 | N2D2HIP_KERNEL_TILE_M128 | N2D2HIP_KERNEL_NO_SPLIT))
+            && ((d.kernel_choice & N2D2HIP_KERNEL_SPLIT) || conv_split_pays(Mll, d.O, c->ktot, w4, other != nullptr));
         const int BMp = small_m ? 64 : wide64 ? 256 : 128;
         q.mtiles = (int)((Mll + BMp - 1) / BMp);
         const int per_xcd = std::max(1, std::min((q.mtiles + 7) / 8, 2 * num_cus() / (8 * a.ntiles_n)));
@@ -1171,15 +1177,6 @@ static int conv_forward_impl(n2d2hip_conv_t c, const n2d2hip_tensor* in, const n
         q.res = nullptr; q.res_cs = 0; q.res_halo = 0; q.res_flip = 0; q.has_pre = q.pre_clamp = q.sum_clamp = 0;
         q.sum16 = nullptr; q.sum16_stride = 0; q.pre_in_range = 0;
         q.sum = EpiArgs(); q.pre = EpiArgs();
-        // Byte outputs of an integer rescale whose scaled-up tables fit: the rescaled value is read from the upper half of
-        // the multiply-add's result
-        const bool hi16 = !other && c->hi16 && c->act->args.kind == EPI_I24 && is_byte_type(out->dtype) && !(d.kernel_choice & N2D2HIP_KERNEL_NO_HI16);
-        if (hi16) { q.c.epi.c = c->d_epi_tab + 5 * c->act->cpad; q.c.epi.d = c->d_epi_tab + 6 * c->act->cpad; }
-        if (w4 && !other) {
-            // 4-bit weights, packed in memory and in LDS
-            q.c.w = c->d_w4img;
-            return conv_pipe_w4_launch(q, tiny ? 3 : small_m ? 2 : bn128 ? 1 : 0, all_valid, hi16, grid, stream);
-        }
         if (other) {
             const int cp = c->sum->act->cpad;
             q.res = (const signed char*)other->data;
@@ -1197,9 +1194,28 @@ static int conv_forward_impl(n2d2hip_conv_t c, const n2d2hip_tensor* in, const n
                 q.pre = c->sum->pre_act->args;
                 q.pre.a = c->d_res_tab + 5 * cp; q.pre.b = c->d_res_tab + 6 * cp; q.pre.c = c->d_res_tab + 7 * cp;
                 q.pre.d = c->d_res_tab + 8 * cp; q.pre.e = c->d_res_tab + 9 * cp;
-                if (c->sum16) { q.pre.c = c->d_res_tab + 12 * cp; q.pre.d = c->d_res_tab + 13 * cp; }
             }
-            if (c->sum16) { q.c.epi.c = c->d_epi_tab + 5 * c->act->cpad; q.c.epi.d = c->d_epi_tab + 6 * c->act->cpad; }
+        }
+        if (split) {
+            q.c.ntiles_n = (round_up(d.O, 16) + 31) / 32;
+            if (w4) q.c.w = c->d_w4img;
+            return conv_split_launch(q, all_valid, w4, stream);
+        }
+        // Byte outputs of an integer rescale whose scaled-up tables fit: the rescaled value is read from the upper half of
+        // the multiply-add's result
+        const bool hi16 = !other && c->hi16 && c->act->args.kind == EPI_I24 && is_byte_type(out->dtype) && !(d.kernel_choice & N2D2HIP_KERNEL_NO_HI16);
+        if (hi16) { q.c.epi.c = c->d_epi_tab + 5 * c->act->cpad; q.c.epi.d = c->d_epi_tab + 6 * c->act->cpad; }
+        if (w4 && !other) {
+            // 4-bit weights, packed in memory and in LDS
+            q.c.w = c->d_w4img;
+            return conv_pipe_w4_launch(q, tiny ? 3 : small_m ? 2 : bn128 ? 1 : 0, all_valid, hi16, grid, stream);
+        }
+        if (other) {
+            if (c->sum16) {
+                const int cp = c->sum->act->cpad;
+                if (c->has_pre) { q.pre.c = c->d_res_tab + 12 * cp; q.pre.d = c->d_res_tab + 13 * cp; }
+                q.c.epi.c = c->d_epi_tab + 5 * c->act->cpad; q.c.epi.d = c->d_epi_tab + 6 * c->act->cpad;
+            }
             if (w4) {
                 q.c.w = c->d_w4img;
                 return conv_pipe_w4_launch(q, small_m ? 2 : bn128 ? 1 : 0, all_valid, false, grid, stream);

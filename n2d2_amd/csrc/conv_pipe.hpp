@@ -64,6 +64,9 @@ struct ConvPipeArgs {
     // sum16_stride dwords, when the host has shown that the sum's arithmetic stays inside 16 bits; else null.
     const int* sum16;
     int sum16_stride;
+    // conv_split_kernel: division by the pixel tiles, by the K steps per tap and by kW
+    unsigned xcd_mul, xcd_sh, cper_mul, cper_sh;
+    int kw_mul;
     int pre_in_range;            // with sum16: the ScalingCell's result cannot leave its range, no saturation needed
 #ifdef N2D2HIP_PROFILE
     long long* prof;             // one 16-counter record per block
