@@ -1543,6 +1543,14 @@ float SATQuantizerActivation_Frame_HIP<T>::getDiffAlpha()
     return h;
 }
 template <class T>
+std::pair<float, float> SATQuantizerActivation_Frame_HIP<T>::getAlphaAndGradient()
+{
+    lazyInit(0, false);
+    float h[2] = {0, 0};
+    checkHip(hipMemcpy(h, mDev, sizeof(h), hipMemcpyDeviceToHost), "getAlphaAndGradient");
+    return std::make_pair(h[0], h[1]);
+}
+template <class T>
 void SATQuantizerActivation_Frame_HIP<T>::update(unsigned int batchSize)
 {
     if (!mSolver) return;
@@ -1714,6 +1722,13 @@ float LSQQuantizerActivation_Frame_HIP<T>::getDiffStepSize()
     float h = 0;
     checkHip(hipMemcpy(&h, mDev + 1, sizeof(float), hipMemcpyDeviceToHost), "getDiffStepSize");
     return h;
+}
+template <class T>
+std::pair<float, float> LSQQuantizerActivation_Frame_HIP<T>::getStepSizeAndGradient()
+{
+    float h[2] = {0, 0};
+    checkHip(hipMemcpy(h, mDev, sizeof(h), hipMemcpyDeviceToHost), "getStepSizeAndGradient");
+    return std::make_pair(h[0], h[1]);
 }
 template <class T>
 void LSQQuantizerActivation_Frame_HIP<T>::update(unsigned int batchSize)

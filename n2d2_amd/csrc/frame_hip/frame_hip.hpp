@@ -1031,6 +1031,7 @@ public:
     void update(unsigned int batchSize);
     float getAlpha();
     float getDiffAlpha();
+    std::pair<float, float> getAlphaAndGradient();       // both in one copy from the device
 
 private:
     void lazyInit(std::size_t size, bool needCopy);
@@ -1113,6 +1114,7 @@ public:
     void update(unsigned int batchSize);
     float getStepSize();
     float getDiffStepSize();
+    std::pair<float, float> getStepSizeAndGradient();    // both in one copy from the device
 
 private:
     float mGradScale;

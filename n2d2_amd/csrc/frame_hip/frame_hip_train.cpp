@@ -14,21 +14,32 @@ static void checkHipT(hipError_t e, const char* what)
 // --------------------------------------------------------------- DeviceFloats
 DeviceFloats::~DeviceFloats()
 {
-    if (mData) (void)hipFree(mData);
+    if (mData && mOwned) (void)hipFree(mData);
 }
 
 void DeviceFloats::resize(const std::vector<size_t>& dims)
 {
     std::vector<size_t> d = dims;
     while (d.size() < 4) d.push_back(1);
-    if (mData) (void)hipFree(mData);
+    if (mData && mOwned) (void)hipFree(mData);
     mData = nullptr;
+    mOwned = true;
     mDims = d;
     mValid = false;
     if (size() == 0)
         return;
     checkHipT(hipMalloc((void**)&mData, size() * sizeof(float)), "DeviceFloats::resize()");
     checkHipT(hipMemset(mData, 0, size() * sizeof(float)), "DeviceFloats::resize()");
+}
+
+void DeviceFloats::within(float* memory, const std::vector<size_t>& dims)
+{
+    if (mData && mOwned) (void)hipFree(mData);
+    mData = memory;
+    mOwned = false;
+    mDims = dims;
+    while (mDims.size() < 4) mDims.push_back(1);
+    mValid = false;
 }
 
 void DeviceFloats::fromHost(const float* host, size_t n)
@@ -51,6 +62,13 @@ Tensor<Float_T> DeviceFloats::toHost() const
     if (size() > 0)
         checkHipT(hipMemcpy(host.data(), mData, size() * sizeof(float), hipMemcpyDeviceToHost), "DeviceFloats::toHost()");
     return host;
+}
+
+void DeviceFloats::toHost(float* host, size_t n) const
+{
+    if (n != size())
+        throw std::runtime_error("DeviceFloats::toHost(): size mismatch");
+    checkHipT(hipMemcpy(host, mData, n * sizeof(float), hipMemcpyDeviceToHost), "DeviceFloats::toHost()");
 }
 
 // -------------------------------------------------------- Cell_FrameTrain_HIP
@@ -138,24 +156,30 @@ void Cell_FrameTrain_HIP::activationUpdate()
         mActivation->getQuantizer()->update((unsigned int)mIn->dimB());
 }
 
-double Cell_FrameTrain_HIP::applyLoss()
+void Cell_FrameTrain_HIP::launchLoss(const float* targets)
 {
     const size_t n = mOutputs.size();
     if (!mLoss)
-        checkHipT(hipMalloc((void**)&mLoss, sizeof(double)), "Cell_FrameTrain_HIP::applyLoss()");
+        checkHipT(hipMalloc((void**)&mLoss, sizeof(double)), "Cell_FrameTrain_HIP::launchLoss()");
     const size_t need = n2d2hip_loss_workspace_bytes(n);
     if (mLossWorkspaceBytes < need) {
         if (mLossWorkspace) (void)hipFree(mLossWorkspace);
         mLossWorkspace = nullptr;
-        checkHipT(hipMalloc(&mLossWorkspace, need), "Cell_FrameTrain_HIP::applyLoss()");
+        checkHipT(hipMalloc(&mLossWorkspace, need), "Cell_FrameTrain_HIP::launchLoss()");
         mLossWorkspaceBytes = need;
     }
-    // target and diff are the same buffer: each element is read, then written, by one thread
-    checkStatus(n2d2hip_loss_f32(mDiffInputs.data(), mOutputs.data(), mDiffInputs.data(), n, (int)mOutputs.dimB(), mLoss,
+    // (target and diff may be the same buffer: each element is read, then written, by one thread)
+    checkStatus(n2d2hip_loss_f32(targets, mOutputs.data(), mDiffInputs.data(), n, (int)mOutputs.dimB(), mLoss,
                                  mLossWorkspace, mLossWorkspaceBytes, mStream));
     mDiffInputs.setValid();
+}
+
+double Cell_FrameTrain_HIP::readLoss() const
+{
+    if (!mLoss)
+        throw std::runtime_error("Cell_FrameTrain_HIP::readLoss(): no loss has been computed");
     double loss = 0.0;
-    checkHipT(hipMemcpy(&loss, mLoss, sizeof(double), hipMemcpyDeviceToHost), "Cell_FrameTrain_HIP::applyLoss()");
+    checkHipT(hipMemcpy(&loss, mLoss, sizeof(double), hipMemcpyDeviceToHost), "Cell_FrameTrain_HIP::readLoss()");
     return loss;
 }
 
@@ -484,6 +508,17 @@ std::vector<Float_T> BatchNormCell_FrameTrain_HIP<T>::get(const DeviceFloats& de
 }
 
 template <class T>
+void BatchNormCell_FrameTrain_HIP<T>::readParameters(float* host) const
+{
+    if (mParameters.empty())
+        throw std::runtime_error("BatchNormCell_FrameTrain_HIP " + mName + ": readParameters() before initialize()");
+    checkHipT(hipStreamSynchronize((hipStream_t)mStream), "BatchNormCell_FrameTrain_HIP: synchronize");
+    const Tensor<Float_T> all = mParameters.toHost();
+    for (size_t k = 0; k < 6; ++k)
+        std::copy(all.data() + k * parameterStride(), all.data() + k * parameterStride() + mNbOutputs, host + k * mNbOutputs);
+}
+
+template <class T>
 BatchNormParameters BatchNormCell_FrameTrain_HIP<T>::getBatchNormParameters() const
 {
     BatchNormParameters p;
@@ -510,14 +545,17 @@ void BatchNormCell_FrameTrain_HIP<T>::initialize()
     allocateOutputs();
     const std::vector<size_t> dims = {1, 1, (size_t)mNbOutputs, 1};
     struct Init { DeviceFloats* dev; std::vector<Float_T>* host; Float_T value; };
+    mParameters.resize({6 * parameterStride(), 1, 1, 1});
+    size_t part = 0;
+    for (DeviceFloats* d : {&mScale, &mBias, &mMean, &mVariance, &mDiffScale, &mDiffBias})
+        d->within(mParameters.data() + parameterStride() * part++, dims);
     const Init params[] = {{&mScale, &mHostScale, 1.0f}, {&mBias, &mHostBias, 0.0f}, {&mMean, &mHostMean, 0.0f}, {&mVariance, &mHostVariance, 0.0f}};
     for (const Init& p : params) {
-        p.dev->resize(dims);
         if (p.host->empty())
             p.host->assign(mNbOutputs, p.value);
         p.dev->fromHost(p.host->data(), p.host->size());
     }
-    for (DeviceFloats* d : {&mSavedMean, &mSavedVariance, &mDiffScale, &mDiffBias, &mDiffSavedMean, &mDiffSavedVariance})
+    for (DeviceFloats* d : {&mSavedMean, &mSavedVariance, &mDiffSavedMean, &mDiffSavedVariance})
         d->resize(dims);
     const size_t bytes = n2d2hip_batchnorm_f32_workspace_bytes((int)mIn->dimB(), (int)mNbOutputs, (int)mInH, (int)mInW);
     mWorkspace.resize({(bytes + sizeof(float) - 1) / sizeof(float), 1, 1, 1});

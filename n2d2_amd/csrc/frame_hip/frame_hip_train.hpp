@@ -16,11 +16,12 @@ namespace N2D2 {
 // (BaseTensor::isValid / setValid / clearValid, include/containers/Tensor.hpp:137-139).
 class DeviceFloats {
 public:
-    DeviceFloats() : mData(nullptr), mDims{0, 0, 0, 0}, mValid(false) {}
+    DeviceFloats() : mData(nullptr), mOwned(true), mDims{0, 0, 0, 0}, mValid(false) {}
     ~DeviceFloats();
     DeviceFloats(const DeviceFloats&) = delete;
     DeviceFloats& operator=(const DeviceFloats&) = delete;
     void resize(const std::vector<size_t>& dims);        // zero-filled
+    void within(float* memory, const std::vector<size_t>& dims);        // part of memory that another tensor owns
     bool empty() const { return mData == nullptr; }
     size_t dimX() const { return mDims[0]; }
     size_t dimY() const { return mDims[1]; }
@@ -36,9 +37,11 @@ public:
     void fromHost(const Tensor<Float_T>& host);
     void fromHost(const float* host, size_t n);
     Tensor<Float_T> toHost() const;
+    void toHost(float* host, size_t n) const;
 
 private:
     float* mData;
+    bool mOwned;
     std::vector<size_t> mDims;
     bool mValid;
 };
@@ -61,7 +64,11 @@ public:
     // Cell_Frame<T>::applyLoss() (src/Cell/Cell_Frame.cpp:646-650 over Cell_Frame_Top::applyLoss,
     // src/Cell/Cell_Frame_Top.cpp:27-40): diffInputs, holding the targets, becomes targets - outputs; returns the sum of
     // squares over the batch size
-    double applyLoss();
+    double applyLoss() { launchLoss(mDiffInputs.data()); return readLoss(); }
+    // Its two halves: the launches, from targets in device memory of the outputs' size (diffInputs itself is fine), and the
+    // wait for the value.  A learning loop that reads only its last loss need not stop the device for the others.
+    void launchLoss(const float* targets);
+    double readLoss() const;
     bool isCuda() const { return false; }
     std::string getPyModel() const { return "Frame_HIP_QAT"; }
     // The stream this cell's kernels are launched on: whatever a caller copies into the cell's tensors between two of its
@@ -104,6 +111,8 @@ public:
     QATCellParameters getQATCellParameters();
     // refreshes the host tensors getWeights() / getBiases() return from the device
     virtual void synchronizeWeightsToHost() = 0;
+    // the device's weights, without the host tensors
+    void readWeights(float* host, size_t n) const { mDevW.toHost(host, n); }
 
 protected:
     WeightedCell_FrameTrain_HIP();
@@ -253,6 +262,8 @@ public:
     std::vector<Float_T> getVariances() const { return get(mVariance, mHostVariance); }
     std::vector<Float_T> getDiffScales() const { return get(mDiffScale, std::vector<Float_T>()); }
     std::vector<Float_T> getDiffBiases() const { return get(mDiffBias, std::vector<Float_T>()); }
+    // the six vectors above, one behind the other (6 x nbOutputs values), in one copy from the device
+    void readParameters(float* host) const;
     void setScaleSolver(const std::shared_ptr<SGDSolver>& solver) { mScaleSolver = solver; }
     void setBiasSolver(const std::shared_ptr<SGDSolver>& solver) { mBiasSolver = solver; }
     const std::shared_ptr<SGDSolver>& getScaleSolver() const { return mScaleSolver; }
@@ -267,6 +278,8 @@ protected:
 private:
     void set(DeviceFloats& dev, std::vector<Float_T>& host, const std::vector<Float_T>& v);
     std::vector<Float_T> get(const DeviceFloats& dev, const std::vector<Float_T>& host) const;
+    size_t parameterStride() const { return ((size_t)mNbOutputs + 63) / 64 * 64; }
+    DeviceFloats mParameters;           // scales, biases, means, variances, gradients of scales and biases: parts of one tensor
     DeviceFloats mScale, mBias, mMean, mVariance, mSavedMean, mSavedVariance, mDiffScale, mDiffBias, mDiffSavedMean, mDiffSavedVariance;
     DeviceFloats mDiffOwn;      // this cell's part of the input gradient while another consumer's is already there
     DeviceFloats mWorkspace;            // partial sums of the split reductions

@@ -259,6 +259,17 @@ int fh_train_get_batchnorm(void* net, const char* cell, int what, float* out, si
     });
 }
 
+// all of them, 6 x n values in that order, in one copy from the device
+int fh_train_get_batchnorm_all(void* net, const char* cell, float* out, size_t n)
+{
+    return guardedT([&] {
+        auto bn = dynamic_cast<BatchNormCell_FrameTrain_HIP<float>*>(find(*(TrainNet*)net, cell));
+        if (!bn) throw std::runtime_error("Not a BatchNorm cell: " + std::string(cell));
+        if (n != bn->getNbOutputs()) throw std::runtime_error("fh_train_get_batchnorm_all(): size mismatch");
+        bn->readParameters(out);
+    });
+}
+
 // Max (pooling 0) or Average (pooling 1) pooling, one output per channel
 int fh_train_add_pool(void* net, const char* name, int poolW, int poolH, int strideX, int strideY, int padX, int padY, int pooling)
 {
@@ -341,7 +352,7 @@ int fh_train_set_solver_parameter(void* net, const char* cell, const char* name,
 }
 
 // targets: HOST float, the shape of the last cell's outputs.  Runs `iterations` times what the reference's learning
-// loop runs: propagate front to back, targets into the last cell's diffInputs, applyLoss, backPropagate back to front,
+// loop runs: propagate front to back, the last cell's applyLoss on the targets, backPropagate back to front,
 // update back to front.  loss receives the last iteration's.
 int fh_train_learn(void* net, const float* targets, size_t nTargets, int iterations, double* loss)
 {
@@ -352,7 +363,6 @@ int fh_train_learn(void* net, const float* targets, size_t nTargets, int iterati
         if (nTargets != last->getOutputs().size()) throw std::runtime_error("fh_train_learn(): wrong number of targets");
         n.targets.resize(last->getOutputs().dims());
         n.targets.fromHost(targets, nTargets);
-        double l = 0.0;
         for (int it = 0; it < iterations; ++it) {
             // the gradient towards the net's input is this iteration's: empty, or what another consumer of the input has
             // already put there (fh_train_preset_input_gradient)
@@ -369,15 +379,14 @@ int fh_train_learn(void* net, const float* targets, size_t nTargets, int iterati
                 }
             }
             for (auto& c : n.cells) c->propagate(false);
-            if (hipMemcpyAsync(last->getDiffInputs().data(), n.targets.data(), nTargets * sizeof(float), hipMemcpyDeviceToDevice,
-                               (hipStream_t)last->stream()) != hipSuccess)
-                throw std::runtime_error("fh_train_learn(): copy of the targets failed");
-            l = last->applyLoss();
+            last->launchLoss(n.targets.data());
             for (auto c = n.cells.rbegin(); c != n.cells.rend(); ++c) (*c)->backPropagate();
             SGDUpdateScope updates;              // (all tensors of the net in one launch)
             for (auto c = n.cells.rbegin(); c != n.cells.rend(); ++c) (*c)->update();
             updates.flush();
         }
+        // (only the last iteration's loss is asked for: the device runs through the others without a stop)
+        const double l = iterations > 0 ? last->readLoss() : 0.0;
         if (hipDeviceSynchronize() != hipSuccess) throw std::runtime_error("fh_train_learn(): device error");
         if (loss) *loss = l;
     });
@@ -455,14 +464,13 @@ int fh_train_get(void* net, const char* cell, int what, float* out, size_t n)
         Cell_FrameTrain_HIP* c = find(*(TrainNet*)net, cell);
         Tensor<Float_T> t;
         auto conv = dynamic_cast<WeightedCell_FrameTrain_HIP*>(c);
+        if (what == 2 && conv) {
+            conv->readWeights(out, n);
+            return;
+        }
         if (what == 0) t = c->getOutputs().toHost();
         else if (what == 1) t = c->getDiffInputs().toHost();
         else if (!conv) throw std::runtime_error("Not a cell with weights: " + std::string(cell));
-        else if (what == 2) {
-            conv->synchronizeWeightsToHost();
-            if (auto cc = dynamic_cast<ConvCell*>(c)) t = cc->getWeights();
-            else t = dynamic_cast<FcCell*>(c)->getWeights();
-        }
         else if (what == 3) t = conv->getDiffWeights();
         else t = conv->getQuantizedWeights();
         if (t.size() != n) throw std::runtime_error("fh_train_get(): size mismatch");
@@ -498,8 +506,8 @@ int fh_train_get_activation_quantizer(void* net, const char* cell, float* value,
         TrainNet& n = *(TrainNet*)net;
         auto s = n.satAct.find(cell);
         auto l = n.lsqAct.find(cell);
-        if (s != n.satAct.end()) { *value = s->second->getAlpha(); if (grad) *grad = s->second->getDiffAlpha(); }
-        else if (l != n.lsqAct.end()) { *value = l->second->getStepSize(); if (grad) *grad = l->second->getDiffStepSize(); }
+        if (s != n.satAct.end()) { const auto v = s->second->getAlphaAndGradient(); *value = v.first; if (grad) *grad = v.second; }
+        else if (l != n.lsqAct.end()) { const auto v = l->second->getStepSizeAndGradient(); *value = v.first; if (grad) *grad = v.second; }
         else throw std::runtime_error("No activation quantizer on cell \"" + std::string(cell) + "\"");
     });
 }

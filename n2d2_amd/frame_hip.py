@@ -396,6 +396,7 @@ lib.fh_train_set_next_inputs.argtypes = [_P, C.c_char_p]
 lib.fh_train_add_elemwise.argtypes = [_P, C.c_char_p, _P, _P, _I, _I, _I, _I, C.c_float]
 lib.fh_train_add_batchnorm.argtypes = [_P, C.c_char_p, _P, C.c_double, C.c_double, _I, _I, _I, _F]
 lib.fh_train_get_batchnorm.argtypes = [_P, C.c_char_p, _I, _P, _SZ]
+lib.fh_train_get_batchnorm_all.argtypes = [_P, C.c_char_p, _P, _SZ]
 lib.fh_train_add_pool.argtypes = [_P, C.c_char_p, _I, _I, _I, _I, _I, _I, _I]
 lib.fh_net_deepnet.argtypes = [_P]
 lib.fh_net_deepnet.restype = C.c_void_p
@@ -486,12 +487,9 @@ class TrainNet:
 
     def batchnorm(self, name):
         """dict of the cell's scales, biases, running means and variances, and the last gradients of scales and biases."""
-        out = {}
-        for k, what in (("scales", 0), ("biases", 1), ("means", 2), ("variances", 3), ("diff_scales", 4), ("diff_biases", 5)):
-            v = np.empty(self._shapes[name][1], dtype=np.float32)
-            _check_train(lib.fh_train_get_batchnorm(self._h, name.encode(), what, v.ctypes.data, v.size))
-            out[k] = v
-        return out
+        v = np.empty((6, self._shapes[name][1]), dtype=np.float32)
+        _check_train(lib.fh_train_get_batchnorm_all(self._h, name.encode(), v.ctypes.data, v.shape[1]))
+        return dict(zip(("scales", "biases", "means", "variances", "diff_scales", "diff_biases"), v))
 
     def add_pool(self, name, pool, stride, pad=(0, 0), pooling="Max"):
         """Max or Average pooling, one output per channel; pool / stride / pad as (x, y)."""
