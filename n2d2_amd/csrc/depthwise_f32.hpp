@@ -163,47 +163,63 @@ __global__ __launch_bounds__(256) void depthwise_f32_data_kernel(DepthwiseF32 q,
     strip_store(dx, (img * q.H + iy) * q.W + ix0, q.W - ix0, sum, beta, nullptr, c);
 }
 
-// Backward-filter: block (channel, tap row) adds the K taps of its row in double.  The blocks of a channel's tap rows read the
-// same two tensors at about the same pace, and all but the first find them in the caches.  A channel's sum is not split
-// further (the workspace query answers 0 for depthwise layers), so few channels leave most of the chip idle.  The same layer:
-// one block per weight 407.8 us, now 49.7; 8 channels, 56 x 56, batch 32, which are 24 blocks: 233 us, now 25.
-template <int K, int S>
-__global__ __launch_bounds__(1024) void depthwise_f32_filter_kernel(DepthwiseF32 q, const float* __restrict__ x, const float* __restrict__ dy, float beta,
-                                                                    float* __restrict__ dw)
+// Backward-filter: a block adds the products of all K^2 taps over one range of a channel's strips in double, so both tensors
+// are read once (x's rows K times, out of the caches).  gridDim.y is the number of ranges; one: the sums are the gradient,
+// more: they go to partial[range][channel][tap], which conv_f32_reduce_partials_kernel adds up.
+// What bounds it is the vector ALU: four instructions a product (multiply, select, conversion, addition in double).
+// 128 channels, 3x3, 56 x 56, batch 32: a block per channel and tap row, which loaded and converted dy's strip once per row
+// and stood on 384 blocks, 48.6 us; now 31.1 with the launch that adds the ranges up.
+// THREADS: 256; more where a range is a whole channel because the caller gave no workspace.  ROWS: tap rows of a block, all K or
+// one (blockIdx.z is which).
+template <int K, int S, int THREADS, int ROWS>
+__global__ __launch_bounds__(THREADS) void depthwise_f32_filter_kernel(DepthwiseF32 q, int per_range, const float* __restrict__ x, const float* __restrict__ dy,
+                                                                   float beta, float* __restrict__ dw, double* __restrict__ partial)
 {
     constexpr int NX = 3 * S + K;
-    const int c = blockIdx.x, ty = blockIdx.y;
-    double acc[K] = {};
-    for (int i = threadIdx.x; i < q.items; i += blockDim.x) {
+    const int c = blockIdx.x, end = min(q.items, ((int)blockIdx.y + 1) * per_range), ty0 = ROWS == K ? 0 : (int)blockIdx.z;
+    double acc[ROWS][K] = {};
+    for (int i = (int)blockIdx.y * per_range + threadIdx.x; i < end; i += THREADS) {
         const int r = div_f32(i, q.dstrips), ox0 = (i - r * q.strips) * 4, b = div_f32(r, q.drows), oy = r - b * q.oH;
-        const int iy = oy * S + ty - q.pt, ix0 = ox0 * S - q.pl, img = b * q.C + c;
-        if ((unsigned)iy >= (unsigned)q.H) continue;
-        float xv[NX], dv[4];
+        const int iy0 = oy * S - q.pt + ty0, ix0 = ox0 * S - q.pl, img = b * q.C + c;
+        float xv[ROWS][NX], dv[4];
         strip_load<4>(dv, dy, (img * q.oH + oy) * q.oW + ox0, q.ny);
-        strip_load<NX>(xv, x, (img * q.H + iy) * q.W + ix0, q.nx);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const bool pixel = ox0 + u < q.oW;
+        for (int ty = 0; ty < ROWS; ++ty)
+            if ((unsigned)(iy0 + ty) < (unsigned)q.H)
+                strip_load<NX>(xv[ty], x, (img * q.H + iy0 + ty) * q.W + ix0, q.nx);
+        bool inside[4][K];
 #pragma unroll
-            for (int t = 0; t < K; ++t) {
-                const float p = xv[u * S + t] * dv[u];
-                acc[t] += (double)(pixel && (unsigned)(ix0 + u * S + t) < (unsigned)q.W ? p : 0.0f);
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int t = 0; t < K; ++t)
+                inside[u][t] = ox0 + u < q.oW && (unsigned)(ix0 + u * S + t) < (unsigned)q.W;
+#pragma unroll
+        for (int ty = 0; ty < ROWS; ++ty)
+            if ((unsigned)(iy0 + ty) < (unsigned)q.H) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int t = 0; t < K; ++t) {
+                        const float p = xv[ty][u * S + t] * dv[u];
+                        acc[ty][t] += (double)(inside[u][t] ? p : 0.0f);
+                    }
             }
-        }
     }
-    __shared__ double red[16][K];
+    __shared__ double red[THREADS / 64][ROWS * K];
 #pragma unroll
-    for (int t = 0; t < K; ++t) {
+    for (int t = 0; t < ROWS * K; ++t) {
+        double a = acc[t / K][t % K];
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) acc[t] += __shfl_xor(acc[t], off, 64);
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][t] = acc[t];
+        for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][t] = a;
     }
     __syncthreads();
-    if (threadIdx.x < K) {
+    if (threadIdx.x < ROWS * K) {
         double s = 0.0;
-        for (int wv = 0; wv < (int)(blockDim.x >> 6); ++wv) s += red[wv][threadIdx.x];
-        const int idx = (c * K + ty) * K + threadIdx.x;
-        dw[idx] = (float)s + (beta != 0.0f ? beta * dw[idx] : 0.0f);
+        for (int wv = 0; wv < THREADS / 64; ++wv) s += red[wv][threadIdx.x];
+        const int idx = (c * K + ty0) * K + threadIdx.x;
+        if (gridDim.y == 1) dw[idx] = (float)s + (beta != 0.0f ? beta * dw[idx] : 0.0f);
+        else partial[(size_t)blockIdx.y * q.C * K * K + idx] = s;
     }
 }
 

@@ -789,7 +789,29 @@ static bool depthwise_strips(const ConvF32& q)
            && (size_t)q.B * q.C * (q.H + q.kH) * (q.W + q.kW + q.pl + 8) < lim && (size_t)q.B * q.C * (q.oH + q.kH) * (q.oW + q.pl + 8) < lim
            && (size_t)q.pl + q.pt + q.pr + q.pb < 4096;
 }
-static int run_depthwise(const ConvF32& q, int pass, const float* a, const float* b, const float* bias, float beta, float* out, hipStream_t st)
+static unsigned reduce_grid(size_t n) { return (unsigned)std::min<size_t>((n + 63) / 64, 16384); }
+
+// Short sums of a few dozen channels: a block of 1024 per channel and tap row, whose blocks find each other's strips in the
+// caches, is ahead of ranges and the launch that adds them up (64 channels, 112 x 112, stride 2, batch 8: 10.1 against 12.7 us),
+// while it has blocks for the chip and all run side by side.
+static bool depthwise_filter_by_rows(const ConvF32& q)
+{
+    const int items = q.B * q.oH * ceil_div_i(q.oW, 4), blocks = q.C * q.kH;
+    return items > 6 * 256 && items <= 8 * 1024 && 2 * blocks >= num_cus() && blocks <= 2 * num_cus();
+}
+// Ranges the strips of a channel are split into for its filter gradient: enough for eight blocks of 256 on every compute unit,
+// but no fewer than six strips a thread.  us, at 2 / 3 / 6 / 12 strips: 128 channels, 56 x 56, batch 32 30.8 / 31.4 / 31.1 / 32.6;
+// 512, 14 x 14, batch 64 20.0 / 20.2 / 20.0 / 20.3; 8, 56 x 56, batch 32 10.3 / 10.0 / 11.9 / 15.4; 96, 5x5, 56 x 56, batch 16
+// 41.8 / 37.0 / 33.9 / 33.1 (a block per channel and tap row: 48.6, 27.6, 25.4, 36.2).
+static int depthwise_filter_ranges(const ConvF32& q)
+{
+    const int items = q.B * q.oH * ceil_div_i(q.oW, 4);
+    return depthwise_filter_by_rows(q) ? 1 : std::max(1, std::min(ceil_div_i(items, 6 * 256), ceil_div_i(8 * num_cus(), q.C)));
+}
+static size_t depthwise_filter_bytes(const ConvF32& q, int ranges) { return ranges > 1 ? (size_t)ranges * q.C * q.kH * q.kW * sizeof(double) : 0; }
+
+static int run_depthwise(const ConvF32& q, int pass, const float* a, const float* b, const float* bias, float beta, float* out, void* workspace,
+                         size_t workspace_bytes, hipStream_t st)
 {
     const int rows = pass == PASS_BWD_DATA ? q.H : q.oH, cols = pass == PASS_BWD_DATA ? q.W : q.oW, strips = ceil_div_i(cols, 4);
     const DepthwiseF32 k = {q.C, q.H, q.W, q.oH, q.oW, q.pl, q.pt, q.B * rows * strips, strips, q.B * q.C * q.H * q.W, q.B * q.C * q.oH * q.oW,
@@ -798,8 +820,25 @@ static int run_depthwise(const ConvF32& q, int pass, const float* a, const float
     const auto run = [&](auto K_, auto S_) {
         constexpr int K = decltype(K_)::value, S = decltype(S_)::value;
         if (pass == PASS_FWD) hipLaunchKernelGGL((depthwise_f32_forward_kernel<K, S>), grid, dim3(256), 0, st, k, a, b, bias, beta, out);
-        else if (pass == PASS_BWD_FILTER)
-            hipLaunchKernelGGL((depthwise_f32_filter_kernel<K, S>), dim3(q.C, K), dim3(k.items >= 2048 ? 1024 : 256), 0, st, k, a, b, beta, out);
+        else if (pass == PASS_BWD_FILTER) {
+            // (without the workspace that the query names, or with one that holds no doubles: one range)
+            int ranges = depthwise_filter_ranges(q);
+            if (workspace_bytes < depthwise_filter_bytes(q, ranges) || (size_t)workspace % sizeof(double)) ranges = 1;
+            const int per_range = ceil_div_i(k.items, ranges);
+            ranges = ceil_div_i(k.items, per_range);
+            constexpr int WIDE = K == 3 ? 1024 : 512;
+            if (depthwise_filter_by_rows(q))
+                hipLaunchKernelGGL((depthwise_f32_filter_kernel<K, S, 1024, 1>), dim3(q.C, 1, K), dim3(1024), 0, st, k, per_range, a, b, beta, out, nullptr);
+            else if (ranges == 1 && k.items > 6 * 256)
+                hipLaunchKernelGGL((depthwise_f32_filter_kernel<K, S, WIDE, K>), dim3(q.C), dim3(WIDE), 0, st, k, per_range, a, b, beta, out, nullptr);
+            else
+                hipLaunchKernelGGL((depthwise_f32_filter_kernel<K, S, 256, K>), dim3(q.C, ranges), dim3(256), 0, st, k, per_range, a, b, beta, out,
+                                   (double*)workspace);
+            const size_t n = (size_t)q.C * K * K;
+            if (ranges > 1)
+                hipLaunchKernelGGL(conv_f32_reduce_partials_kernel<double>, dim3(reduce_grid(n)), dim3(256), 0, st, (const double*)workspace, ranges, n, beta, out,
+                                   (const float*)nullptr, 1, 1);
+        }
         else if (S == 2 && (q.pl & 1)) hipLaunchKernelGGL((depthwise_f32_data_kernel<K, S, S == 2>), grid, dim3(256), 0, st, k, b, a, beta, out);
         else hipLaunchKernelGGL((depthwise_f32_data_kernel<K, S, 0>), grid, dim3(256), 0, st, k, b, a, beta, out);
     };
@@ -817,7 +856,7 @@ static int run_depthwise(const ConvF32& q, int pass, const float* a, const float
 // (dilated, larger) one load after the other.
 static int run_direct(const ConvF32& q, int pass, const float* x, const float* w, const float* bias, float beta, float* out, hipStream_t st)
 {
-    if (depthwise_strips(q)) return run_depthwise(q, pass, x, w, bias, beta, out, st);
+    if (depthwise_strips(q)) return run_depthwise(q, pass, x, w, bias, beta, out, nullptr, 0, st);
     const bool bwd = pass == PASS_BWD_DATA;
     const size_t lim = (size_t)1 << 31, total = (size_t)q.B * (bwd ? (size_t)q.C * q.H * q.W : (size_t)q.O * q.oH * q.oW);
     const size_t source = (size_t)q.B * (bwd ? (size_t)q.O * q.oH * q.oW : (size_t)q.C * q.H * q.W);
@@ -1018,7 +1057,6 @@ static void launch_pixels(PixelPlan& pl, int splits, const float* x, const float
     pl.many ? run(std::true_type{}) : run(std::false_type{});
 }
 
-static unsigned reduce_grid(size_t n) { return (unsigned)std::min<size_t>((n + 63) / 64, 16384); }
 
 // ---- backward-filter
 struct FilterPlan {
@@ -1274,6 +1312,8 @@ size_t n2d2hip_conv2d_f32_workspace_bytes(const n2d2hip_conv_desc* desc, int B, 
             if (pass == PASS_BWD_FILTER) need = std::max(need, (size_t)q.O * q.C * q.kH * q.kW);     // (always has one)
         }
     }
+    if (depthwise_strips(q) && f32_path(q, PASS_BWD_FILTER) == F32_PATH_DIRECT)
+        need = std::max(need, depthwise_filter_bytes(q, depthwise_filter_ranges(q)) / sizeof(float));
     return need * sizeof(float);
 }
 
@@ -1299,7 +1339,8 @@ int n2d2hip_conv2d_f32_backward_filter(const n2d2hip_conv_desc* desc, int B, int
                         workspace_bytes, need);
         return run_pass(m, pass, x, diff_y, nullptr, 1, 1, beta, diff_w, (float*)workspace, workspace_bytes / sizeof(float), (hipStream_t)stream);
     }
-    if (depthwise_strips(q)) return run_depthwise(q, PASS_BWD_FILTER, x, diff_y, nullptr, beta, diff_w, (hipStream_t)stream);
+    if (depthwise_strips(q))
+        return run_depthwise(q, PASS_BWD_FILTER, x, diff_y, nullptr, beta, diff_w, workspace, workspace ? workspace_bytes : 0, (hipStream_t)stream);
     hipLaunchKernelGGL(conv_f32_backward_filter_kernel, dim3((unsigned)nw), dim3(TBLOCK), 0, (hipStream_t)stream, q, x, diff_y, beta, diff_w);
     N2D2HIP_HIP_CHECK(hipGetLastError());
     return N2D2HIP_OK;
