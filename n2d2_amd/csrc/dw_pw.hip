@@ -1,21 +1,33 @@
 // A 3x3 depthwise convolution and the 1x1 convolution that reads it, in one launch (the building block of the MobileNets).
 // Launched cell by cell, the depthwise output is written by one launch and read back by the next, and at 14 x 14 and
-// below both launches are mostly their fixed cost.  Here a work-group owns a tile of 8 rows x 16 columns of output pixels:
-// for each chunk of 64 (or 32) channels it computes the depthwise convolution on the vector ALU exactly as the stand-alone
-// kernel does (a thread owns 4 channels of one column and walks down the rows, every tap a byte of a 4-way dot product),
-// rescales it to bytes, writes them to LDS as the pixel operand of the matrix cores and multiplies them into the 1x1
-// convolution's accumulators, of which that chunk is one slice of K; the depthwise output never reaches memory.
+// below both launches are mostly their fixed cost.  Here a work-group takes tiles of 8 rows x 16 columns of output pixels, and
+// of a tile one chunk of 64 (or 32) channels a step: the depthwise convolution of the chunk is rescaled to bytes, written to
+// LDS as the pixel operand of the 1x1 convolution, of which the chunk is one slice of K, and multiplied there; the depthwise
+// output never reaches memory.
 //
-// LDS: the pixel operand (128 pixels x 64 bytes, 16-byte slots XOR-swizzled by the row so that the 32 rows of a fragment
-// read spread over the banks) and the 1x1 weights of the chunk in matrix-core fragment order (copied by direct-to-LDS
-// loads while the vector ALU works on the chunk), both twice, so that a chunk is written while slower waves still
-// multiply the one before: one barrier per chunk.  The 1x1 convolution's tables are resident in LDS.
+// The depthwise convolution runs on the matrix cores as well, though its matrix is mostly zeros: of 16 channels x 16 pixels, one
+// 16x16x64 instruction a tap row, whose 64 terms are 16 channels at 4 columns (three taps, the fourth weighing 0) and whose
+// weights for a channel are zero but for that channel's bytes.  Its pixel operand is 16 bytes of one pixel as they lie in
+// memory, read once for the three output rows that use it.  On the vector ALU, 4 outputs took 12 dot products and about 20
+// instructions of transposes, borders and addresses.  What is left there are the two rescales, 14 instructions for 4 outputs.
+//
+// LDS: the input of a chunk (the tile and its border, by loads that go there directly; a pixel outside the image comes from a
+// line of the stored 0), the pixel operand, the 1x1 weights and the depthwise tables, each twice: while step n is computed,
+// the input of step n + 1 is on its way, and the multiplication is one step behind the depthwise part, so that one barrier a
+// step is enough.  A work-group stays for a run of tiles.  All slots of 16 bytes are swizzled by the pixel so that 16
+// pixels' slots of one channel group lie in different banks.
+//
+// Batch of 64, MobileNet-v1's sizes, before (depthwise on the vector ALU, one tile a work-group, no loads ahead) and now, us:
+// 32 -> 64 channels at 112 x 112 34.6 and 19.5 (77 MB, 4.0 TB/s: near the rate of a copy), 64 -> 128 from 112 to 56 30.9 and 19.5
+// (77 MB), 128 -> 128 at 56 29.4 and 20.7, 128 -> 256 from 56 to 28 26.6 and 15.8, 256 -> 256 at 28 27.7 and 18.4.  The last three
+// have less to move (51, 38 and 26 MB); vector ALU and LDS are each about half busy there, and a step's parts wait for
+// each other.  Measured and not kept: half of the waves multiplying first (+2 us), the multiplication before the depthwise
+// part (0), 4 waves in place of 8 (+1 to 3 us); 16 waves only where a work-group has 256 outputs (-0.5 us).
 #include <algorithm>
 #include <vector>
 
 #include "common.h"
 #include "conv_handle.hpp"
-#include "depthwise_math.hpp"
 #include "epilogue.hpp"
 #include "mfma_util.hpp"
 
@@ -24,255 +36,363 @@ namespace n2d2hip {
 struct DwPwArgs {
     const signed char* in;    // B x H x W x C bytes
     signed char* out;         // B x OH x OW x O bytes
-    const int* wdw;           // depthwise: [3][C] dwords (w[ky][0], w[ky][1], w[ky][2], 0), then [C] biases, zero point folded in
-    EpiArgs dwe;              // depthwise rescale, tables by channel
+    const int* dwt;           // depthwise tables: [chunk][DWT_ROWS][KC] ints, see DWT_*
     const signed char* wpw;   // 1x1 weights: [channel tile of 32*NB][chunk][K step of 32][32-channel block][lane][16 bytes]
-    const int* pwt;           // 1x1 rescale with the bias folded in: a, b, c, d, e, each [O]
+    const int* pwt;           // 1x1 rescale with the bias folded in: c and e, d, a, b, each [O]
+    const signed char* fill_line;   // 16 bytes of the input's stored form of 0
     int C, O;
-    int B, H, W, OH, OW, padL, padT;
+    int H, W, OH, OW, padL, padT;
     int tw;                   // valid columns of a tile (at most 16)
     int tiles_x, tiles_y, ntiles;
-    unsigned fill;            // the stored form of 0 in all four bytes of the input
+    int per_xcd, per_block, extra_tiles;   // tiles of an XCD; of those, of one work-group; the first so many have one more
     unsigned mid_xor;         // 0x80808080 when the depthwise output is stored as value - 128
     unsigned out_xor;
+    int dw_lo, dw_hi;
     int pw_lo, pw_hi;
     unsigned out_bytes;
 };
 
 namespace {
 
+// Rows of a chunk's depthwise tables: the tap columns as dwords (w[0][kx], w[1][kx], w[2][kx], 0), the rescale, and what only
+// the general rescale needs (the bias with the zero point folded in, and the bounds).
+enum { DWT_W, DWT_CE = 3, DWT_D, DWT_BIAS, DWT_A, DWT_B, DWT_USED, DWT_ROWS = 8 };
+
+// 16 bytes a lane from its own address to 16 * lane bytes past LDS offset `lds`, which is the same in all lanes.  As text,
+// because the compiler would wait for every such load of the wave before the next LDS read of any buffer.
+__device__ __forceinline__ void load_to_lds(const void* src, unsigned lds)
+{
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds) : "memory");
+}
+
+// (acc * c + d) >> e of the rescales on 32 bits.  acc comes from an instruction of the compiler's: it waits for a matrix
+// instruction's result before its own instructions only, not before text (so the clamp before this is not med3_i32 either).  c fits 24 bits, of which alone the multiply-add reads: its word carries e in
+// the top byte, so that a table costs one LDS read less.
+__device__ __forceinline__ int scale24(int acc, int ce, int d)
+{
+    int r;
+    asm("v_ashrrev_i32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3 src1_sel:DWORD" : "=v"(r) : "v"(ce), "v"(__mul24(acc, ce) + d));
+    return r;
+}
+
+// What a variant needs of a compute unit.  SINGLE: the layer is one chunk, whose weights and tables stay for all tiles.
+template <int S, int KC, int NB, int WAVES, bool SINGLE, bool FAST>
+struct DwPwShape {
+    static constexpr int TCOLS = S == 1 ? 18 : 33, TROWS = S == 1 ? 10 : 17;        // input pixels of a tile
+    static constexpr int IN_LOADS = (TROWS * TCOLS * KC + 1023) / 1024;             // of 1 KB each
+    static constexpr int IN_BYTES = IN_LOADS * 1024;
+    static_assert(IN_BYTES >= (TROWS * TCOLS + 1) * KC, "the fourth tap of the last pixel, which weighs 0, reads one pixel past the tile");
+    static constexpr int A_BYTES = 128 * KC;
+    static constexpr int B_BYTES = KC * NB * 32;
+    static constexpr int NT = NB * 32;              // output channels of the work-group
+    static constexpr int DWT_LOADS = ((FAST ? (int)DWT_BIAS : (int)DWT_USED) * KC * 4 + 1023) / 1024;
+    static constexpr int DWT_BYTES = DWT_LOADS * 1024;
+    static_assert(DWT_BYTES <= DWT_ROWS * KC * 4, "the loads stay within the chunk's rows");
+    static constexpr int A_OFF = 2 * IN_BYTES, B_OFF = A_OFF + 2 * A_BYTES;
+    static constexpr int D_OFF = B_OFF + (SINGLE ? 1 : 2) * B_BYTES, T_OFF = D_OFF + (SINGLE ? 1 : 2) * DWT_BYTES;
+    static constexpr int PW_ROWS = FAST ? 2 : 4;    // rows of the 1x1 tables that are read
+    static constexpr int LDS = T_OFF + PW_ROWS * NT * 4;
+    // work-groups on a compute unit: by LDS, and by registers (5 waves a SIMD have 96 each, 4 have 128, 2 have 256)
+    static constexpr int MAX_GROUPS = (2 * NB / WAVES == 1 ? 20 : 8) / WAVES;
+    static constexpr int GROUPS = 163840 / LDS < MAX_GROUPS ? 163840 / LDS : MAX_GROUPS;
+};
+
 // S: stride of the depthwise convolution; KC: channels per chunk (64, or 32 for a 32-channel layer); NB: 32-channel blocks
-// of the 1x1 convolution's outputs a work-group computes (blockIdx.y selects which 32 * NB of them); WAVES: 4, or 8 with
-// the channel blocks split between the two halves of the work-group (half the accumulators per wave, half the rows per
-// thread in the depthwise part).
+// of the 1x1 convolution's outputs a work-group computes (blockIdx.y selects which 32 * NB of them); WAVES: 4, 8 or 16.
 // FAST: neither cell needs a clamp before its multiply and both saturate to [0, 255]: the depthwise tables c, d, e are then
 // the ones with the bias folded in (accumulators start from zero), and both rescales saturate while they pack.
-template <int S, int KC, int NB, int WAVES, bool FAST>
-__global__ __launch_bounds__(64 * WAVES) void dw_pw_kernel(const DwPwArgs q)
+template <int S, int KC, int NB, int WAVES, bool SINGLE, bool FAST>
+__global__ __launch_bounds__(64 * WAVES, (DwPwShape<S, KC, NB, WAVES, SINGLE, FAST>::GROUPS * WAVES / 4)) void dw_pw_kernel(const DwPwArgs q)
 {
+    typedef DwPwShape<S, KC, NB, WAVES, SINGLE, FAST> Z;
     constexpr int THREADS = 64 * WAVES;
-    constexpr int NBW = NB / (WAVES / 4);    // channel blocks of a wave
-    static_assert(NBW >= 2 && NBW % 2 == 0, "a wave stores pairs of channel blocks");
-    constexpr int CG = KC / 4;               // channel groups of a chunk
-    constexpr int RH = THREADS / (CG * 16);  // the tile's rows are split over this many groups of threads
-    constexpr int ROWS = 8 / RH;             // output rows a thread walks down
+    constexpr int PB = 2;                    // a wave multiplies 2 blocks of 32 pixels ...
+    constexpr int NBW = NB / (WAVES / 2);    // ... with 1 or 2 blocks of 32 channels
+    static_assert(NBW == 1 || NBW == 2, "a wave stores one channel block or a pair");
+    constexpr int SL = KC / 16;              // 16-channel groups of a chunk = 16-byte slots of a pixel
+    constexpr int RP = WAVES / SL;           // the tile's rows are split over this many sets of waves
+    constexpr int ROWS = 8 / RP;             // output rows a wave walks down
     constexpr int KS = KC / 32;
-    constexpr int A_BYTES = 128 * 64;
-    constexpr int B_BYTES = KC * NB * 32;
-    constexpr int NT = NB * 32;              // output channels of the work-group
-    constexpr int A_OFF = 0, B_OFF = 2 * A_BYTES, T_OFF = B_OFF + 2 * B_BYTES;
-    __shared__ __attribute__((aligned(16))) unsigned char smem[T_OFF + 5 * NT * 4];
+    constexpr int TCOLS = Z::TCOLS, NT = Z::NT;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[Z::LDS];
+    const unsigned lds0 = (unsigned)(unsigned long long)(lds_ptr_t)smem;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, lh = lane >> 5;
 
-    // blocks 8 apart run on the same XCD: give each XCD a run of consecutive tiles (neighbours share input rows)
-    const int per_xcd = (q.ntiles + 7) / 8;
-    const int tile = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-    if (tile >= q.ntiles)
+    // blocks 8 apart run on the same XCD: give each XCD a run of consecutive tiles (neighbours share input rows), and each
+    // work-group a run of those
+    const int xcd = (int)(blockIdx.x & 7), i = (int)(blockIdx.x >> 3);
+    const int extra = min(i, q.extra_tiles);
+    const int tile0 = xcd * q.per_xcd + i * q.per_block + extra;
+    const int ntile = min(q.per_block + (i < q.extra_tiles ? 1 : 0), min((xcd + 1) * q.per_xcd, q.ntiles) - tile0);
+    if (ntile <= 0)
         return;
     const int n0 = (int)blockIdx.y * NT;
-    const int tx = tile % q.tiles_x;
-    const int ty = (tile / q.tiles_x) % q.tiles_y;
-    const int b = tile / (q.tiles_x * q.tiles_y);
+    const int nchunks = SINGLE ? 1 : q.C / KC;
+    const int nsteps = ntile * nchunks;
+    struct Tile { int x, y, b; };
+    Tile lt = {tile0 % q.tiles_x, (tile0 / q.tiles_x) % q.tiles_y, tile0 / (q.tiles_x * q.tiles_y)};     // the tile that is loaded
+    Tile et = lt;                                                                                         // the one that is written
+    auto advance = [&](Tile& t) {
+        if (++t.x == q.tiles_x) {
+            t.x = 0;
+            if (++t.y == q.tiles_y) {
+                t.y = 0;
+                ++t.b;
+            }
+        }
+    };
+
+    // swizzle of a pixel's slots: 16 consecutive pixels of one slot lie in 16 different 16-byte columns of the 64 banks
+    auto swizzle = [](int pos) { return (pos / (16 / SL)) & (SL - 1); };
+
+    // ---- input loads: load j of this wave brings slots 64 * (wave + WAVES * j) + lane of the tile.  A row holds its pixels in
+    // order (stride 2: the even columns first), a pixel its 16-channel groups swizzled; outside the image the fill is read.
+    constexpr int NLD = (Z::IN_LOADS + WAVES - 1) / WAVES;
+    int ld_pos[NLD], ld_off[NLD];      // the slot's row (16 bits up) and column, its bytes from the tile's first pixel
+    int in_off[NLD];
+#pragma unroll
+    for (int j = 0; j < NLD; ++j) {
+        const unsigned idx = (wave + WAVES * j) * 64 + lane;
+        const unsigned pix = idx / SL, slot = idx % SL;
+        const unsigned r = pix / TCOLS, pos = pix % TCOLS;
+        const int col = S == 1 ? pos : pos < 17 ? 2 * pos : 2 * (pos - 17) + 1;
+        ld_pos[j] = (int)r << 16 | col;         // (the last load ends in a row below the tile)
+        ld_off[j] = ((int)r * q.W + col) * q.C + ((slot ^ swizzle(pos)) << 4);
+    }
+    auto place_tile = [&]() {
+        const int ix0 = lt.x * q.tw * S - q.padL, iy0 = lt.y * 8 * S - q.padT;
+        const int base = ((lt.b * q.H + iy0) * q.W + ix0) * q.C;
+#pragma unroll
+        for (int j = 0; j < NLD; ++j)
+            in_off[j] = (unsigned)(ix0 + (ld_pos[j] & 0xffff)) < (unsigned)q.W && (unsigned)(iy0 + (ld_pos[j] >> 16)) < (unsigned)q.H ? base + ld_off[j] : -1;
+    };
+    auto issue_tables = [&](int kc, int step) {
+        if (wave < Z::DWT_LOADS)
+            load_to_lds((const char*)q.dwt + kc * (DWT_ROWS * KC * 4) + wave * 1024 + lane * 16,
+                        lds0 + Z::D_OFF + (SINGLE ? 0 : (step & 1) * Z::DWT_BYTES) + wave * 1024);
+    };
+    int lkc = 0;                             // the chunk that is loaded
+    auto issue_input = [&](int step) {
+        if (lkc == 0)
+            place_tile();
+        const unsigned dst = lds0 + (step & 1) * Z::IN_BYTES;
+        const signed char* base = q.in + lkc * KC;
+#pragma unroll
+        for (int j = 0; j < NLD; ++j)
+            if (wave + WAVES * j < Z::IN_LOADS)
+                load_to_lds(in_off[j] >= 0 ? base + in_off[j] : q.fill_line, dst + (wave + WAVES * j) * 1024);
+        if (!SINGLE)
+            issue_tables(lkc, step);
+        if (++lkc == nchunks) {
+            lkc = 0;
+            advance(lt);
+        }
+    };
+    auto issue_weights = [&](int kc, int step) {     // B_BYTES contiguous bytes, 1 KB per load
+        const signed char* src = q.wpw + ((long long)blockIdx.y * nchunks + kc) * Z::B_BYTES + lane * 16;
+        const unsigned dst = lds0 + Z::B_OFF + (SINGLE ? 0 : (step & 1) * Z::B_BYTES);
+#pragma unroll
+        for (int j = 0; j < (Z::B_BYTES / 1024 + WAVES - 1) / WAVES; ++j) {
+            const int c = wave + WAVES * j;
+            if (c < Z::B_BYTES / 1024)
+                load_to_lds(src + c * 1024, dst + c * 1024);
+        }
+    };
+    issue_input(0);
+    if (SINGLE) {
+        issue_weights(0, 0);
+        issue_tables(0, 0);
+    }
+
+    // ---- depthwise side: this wave's 16 channels and rows; lane (p, g): output column p, tap column g (the fourth tap weighs 0)
+    const int cgid = wave % SL, rp = wave / SL;
+    const int p = lane & 15, g = lane >> 4;
+    // the matrix of a tap row weighs, for channel p, that channel's bytes only: byte p % 4 of dword p / 4 is w[ky][g]
+    const unsigned select = g == 3 ? 0x0c0c0c0cu : 0x0c0c0c0cu & ~(255u << (8 * (p & 3)));
+    const unsigned select1 = g == 3 ? 0u : 1u << (8 * (p & 3));
+    struct Chunk { v4i w[3], ce, d, bias, a, b; };
+    auto read_chunk = [&](const int* t, Chunk& k) {
+        const int* tc = t + cgid * 16 + 4 * g;
+        const unsigned taps = (unsigned)t[DWT_W * KC + g * KC + cgid * 16 + p];      // (the row after them for the fourth)
+#pragma unroll
+        for (int ky = 0; ky < 3; ++ky) {
+            const int byte = (int)__builtin_amdgcn_perm(0u, taps, select + ky * select1);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                k.w[ky][e] = (p >> 2) == e ? byte : 0;
+        }
+        k.ce = *(const v4i*)(tc + DWT_CE * KC);
+        k.d = *(const v4i*)(tc + DWT_D * KC);
+        if (!FAST) {
+            k.bias = *(const v4i*)(tc + DWT_BIAS * KC);
+            k.a = *(const v4i*)(tc + DWT_A * KC);
+            k.b = *(const v4i*)(tc + DWT_B * KC);
+        }
+    };
 
     // ---- the 1x1 convolution's tables
-    {
-        int* tab = (int*)(smem + T_OFF);
-        for (int i = tid; i < 5 * NT; i += THREADS) {
-            const int row = i / NT, ch = i - row * NT;
-            tab[i] = q.pwt[row * q.O + n0 + ch];
-        }
-    }
+    int* const tab = (int*)(smem + Z::T_OFF);
+    for (int i = tid; i < Z::PW_ROWS * NT; i += THREADS)
+        tab[i] = q.pwt[i / NT * q.O + n0 + i % NT];
 
-    // ---- depthwise side: this thread's column and channel group
-    const int cg = tid % CG;
-    const int x = (tid / CG) % 16;
-    const int rh = tid / (CG * 16);
-    const int ox = min(tx * q.tw + x, q.OW - 1);
-    const int oy0 = ty * 8 + rh * ROWS;
-    const int ix0 = ox * S - q.padL;
-    const bool vm = ix0 >= 0 && ix0 < q.W, v0 = ix0 + 1 >= 0 && ix0 + 1 < q.W, vp = ix0 + 2 >= 0 && ix0 + 2 < q.W;
-    const unsigned fill = q.fill;
-    const int om = min(max(ix0, 0), q.W - 1) * q.C, oc = min(max(ix0 + 1, 0), q.W - 1) * q.C, op = min(max(ix0 + 2, 0), q.W - 1) * q.C;
-    const long long row_bytes = (long long)q.W * q.C;
-    const signed char* img = q.in + (long long)b * q.H * row_bytes + cg * 4;
-    const int iy0 = oy0 * S - q.padT;
-    typedef const unsigned __attribute__((address_space(1))) * GlobalWord;
-    struct Raw3 { unsigned m, c, p; };
+    const int wm = wave & 1, wn = wave >> 1;     // this wave's 64 pixels and its channel blocks
+    v16i acc[PB][NBW];
+#pragma unroll
+    for (int u = 0; u < PB; ++u)
+#pragma unroll
+        for (int i = 0; i < NBW; ++i)
+            acc[u][i] = v16i{};
+    const __amdgpu_buffer_rsrc_t out_rsrc = __builtin_amdgcn_make_buffer_rsrc(q.out, 0, q.out_bytes, 0x00020000);
 
-    const int wm = wave & 3, wn = wave >> 2;     // this wave's 32 pixels and its run of channel blocks
-    v16i acc[NBW];
-#pragma unroll
-    for (int i = 0; i < NBW; ++i)
-        acc[i] = v16i{};
+    const int pos0 = S == 1 ? p + g : (g & 1) * 17 + p + (g >> 1);
+    const int in_addr = ((rp * ROWS * S) * TCOLS + pos0) * KC + ((cgid ^ swizzle(pos0)) << 4);
+    const int mid_addr = rp * ROWS * 16 * KC + p * KC + ((cgid ^ swizzle(p)) << 4) + 4 * g;       // (16 rows further the swizzle is the same)
+    const int m0 = 64 * wm + l32;                // this lane's pixels of the 1x1 convolution: m0 and m0 + 32
+    const int pf_addr = m0 * KC;
 
-    const int nchunks = q.C / KC;
-    for (int kc = 0; kc < nchunks; ++kc) {
-        unsigned char* abuf = smem + A_OFF + (kc & 1) * A_BYTES;
-        unsigned char* bbuf = smem + B_OFF + (kc & 1) * B_BYTES;
-        // ---- the chunk's 1x1 weights: B_BYTES contiguous bytes, 1 KB per load
-        {
-            const signed char* src = q.wpw + ((long long)blockIdx.y * nchunks + kc) * B_BYTES;
+    bool stored = false;                         // the last iteration stored
+    int kc = 0, pkc = 0;                         // chunk of the depthwise part, chunk of the multiplication (one step behind)
+    for (int step = 0; step <= nsteps; ++step) {
+        // This step's input and the weights of the one before have arrived (a wave's stores were issued last and may be on their
+        // way), and every wave is past what it read from the buffers that are filled next.
+        if (stored) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(PB * NBW) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
+        if (step + 1 < nsteps)
+            issue_input(step + 1);
+        if (step < nsteps) {
+            if (!SINGLE)
+                issue_weights(kc, step);
+            Chunk k;
+            read_chunk((const int*)(smem + Z::D_OFF + (SINGLE ? 0 : (step & 1) * Z::DWT_BYTES)), k);
+            const unsigned char* ib = smem + (step & 1) * Z::IN_BYTES + in_addr;
+            unsigned char* ab = smem + Z::A_OFF + (step & 1) * Z::A_BYTES + mid_addr;
+            v4i f[ROWS * S + 3 - S];
 #pragma unroll
-            for (int j = 0; j < (B_BYTES / 1024 + WAVES - 1) / WAVES; ++j) {
-                const int c = wave + WAVES * j;
-                if (c < B_BYTES / 1024)
-                    __builtin_amdgcn_global_load_lds((gbl_ptr_t)(src + c * 1024 + lane * 16), (lds_ptr_t)(bbuf + c * 1024), 16, 0, 0);
-            }
-        }
-        // ---- depthwise convolution of the chunk's channels
-        {
-            const int ch = kc * KC + cg * 4;
-            const signed char* cimg = img + kc * KC;
-            const int4 w0 = *(const int4*)(q.wdw + ch);
-            const int4 w1 = *(const int4*)(q.wdw + q.C + ch);
-            const int4 w2 = *(const int4*)(q.wdw + 2 * q.C + ch);
-            int4 bias = {}, ta = {}, tb = {};
-            if (!FAST) {
-                bias = *(const int4*)(q.wdw + 3 * q.C + ch);
-                ta = *(const int4*)(q.dwe.a + ch);
-                tb = *(const int4*)(q.dwe.b + ch);
-            }
-            const int4 tc = *(const int4*)(q.dwe.c + ch);
-            const int4 td = *(const int4*)(q.dwe.d + ch);
-            const int4 te = *(const int4*)(q.dwe.e + ch);
-            auto fetch_row = [&](int iy) -> Raw3 {
-                const signed char* rp = cimg + min(max(iy, 0), q.H - 1) * row_bytes;
-                Raw3 r;
-                r.m = *(GlobalWord)(rp + om);
-                r.c = *(GlobalWord)(rp + oc);
-                r.p = *(GlobalWord)(rp + op);
-                return r;
-            };
-            auto settle_row = [&](const Raw3& r, int iy) -> Row4 {
-                const bool row_ok = iy >= 0 && iy < q.H;
-                return transpose3((row_ok && vm) ? r.m : fill, (row_ok && v0) ? r.c : fill, (row_ok && vp) ? r.p : fill);
-            };
-            Row4 t0 = settle_row(fetch_row(iy0), iy0);
-            Row4 t1 = {};
-            if (S == 1)
-                t1 = settle_row(fetch_row(iy0 + 1), iy0 + 1);
-            // this thread's dword of row m of the pixel operand: slot (cg / 4) of the row, swizzled, byte 4 * (cg % 4)
-            constexpr int R = S == 1 ? (ROWS < 4 ? ROWS : 4) : 2;
+            for (int r = 0; r < ROWS * S + 3 - S; ++r)
+                f[r] = *(const v4i*)(ib + r * TCOLS * KC);
 #pragma unroll
-            for (int r0 = 0; r0 < ROWS; r0 += R) {
-                const int base = iy0 + S * r0 + (S == 1 ? 2 : 1);
-                Raw3 raw[R * S];
+            for (int r = 0; r < ROWS; ++r) {
+                v4i s = FAST ? v4i{} : k.bias;
 #pragma unroll
-                for (int i = 0; i < R * S; ++i)
-                    raw[i] = fetch_row(base + i);
-#pragma unroll
-                for (int i = 0; i < R; ++i) {
-                    if (S != 1)
-                        t1 = settle_row(raw[2 * i], base + 2 * i);
-                    const Row4 t2 = settle_row(raw[S * i + S - 1], base + S * i + S - 1);
-                    int a0 = __builtin_amdgcn_sdot4(t0.c[0], w0.x, bias.x, false);
-                    int a1 = __builtin_amdgcn_sdot4(t0.c[1], w0.y, bias.y, false);
-                    int a2 = __builtin_amdgcn_sdot4(t0.c[2], w0.z, bias.z, false);
-                    int a3 = __builtin_amdgcn_sdot4(t0.c[3], w0.w, bias.w, false);
-                    a0 = __builtin_amdgcn_sdot4(t1.c[0], w1.x, a0, false);
-                    a1 = __builtin_amdgcn_sdot4(t1.c[1], w1.y, a1, false);
-                    a2 = __builtin_amdgcn_sdot4(t1.c[2], w1.z, a2, false);
-                    a3 = __builtin_amdgcn_sdot4(t1.c[3], w1.w, a3, false);
-                    a0 = __builtin_amdgcn_sdot4(t2.c[0], w2.x, a0, false);
-                    a1 = __builtin_amdgcn_sdot4(t2.c[1], w2.y, a1, false);
-                    a2 = __builtin_amdgcn_sdot4(t2.c[2], w2.z, a2, false);
-                    a3 = __builtin_amdgcn_sdot4(t2.c[3], w2.w, a3, false);
-                    unsigned packed;
-                    if (FAST) {
-                        packed = sat_bytes_u8((__mul24(a0, tc.x) + td.x) >> te.x, (__mul24(a1, tc.y) + td.y) >> te.y,
-                                              (__mul24(a2, tc.z) + td.z) >> te.z, (__mul24(a3, tc.w) + td.w) >> te.w);
-                    } else {
-                        const int v0r = epi_apply<EPI_I24>(a0, ta.x, tb.x, tc.x, td.x, te.x, q.dwe.lo, q.dwe.hi, 0);
-                        const int v1r = epi_apply<EPI_I24>(a1, ta.y, tb.y, tc.y, td.y, te.y, q.dwe.lo, q.dwe.hi, 0);
-                        const int v2r = epi_apply<EPI_I24>(a2, ta.z, tb.z, tc.z, td.z, te.z, q.dwe.lo, q.dwe.hi, 0);
-                        const int v3r = epi_apply<EPI_I24>(a3, ta.w, tb.w, tc.w, td.w, te.w, q.dwe.lo, q.dwe.hi, 0);
-                        packed = ((unsigned)v0r & 255u) | (((unsigned)v1r & 255u) << 8) | (((unsigned)v2r & 255u) << 16) | ((unsigned)v3r << 24);
-                    }
-                    packed ^= q.mid_xor;
-                    const int m = (rh * ROWS + r0 + i) * 16 + x;
-                    *(unsigned*)(abuf + m * 64 + (((cg >> 2) ^ ((m >> 1) & 3)) << 4) + ((cg & 3) << 2)) = packed;
-                    if (S == 1) {
-                        t0 = t1;
-                        t1 = t2;
-                    } else {
-                        t0 = t2;
-                    }
-                }
-            }
-        }
-        // the chunk's pixel bytes and weights are in LDS for every wave; the chunk before this one has been multiplied by
-        // every wave, so its buffers may be written again after this barrier
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        // ---- multiply: this wave's 32 pixels against all NB channel blocks
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const int m = 32 * wm + l32;
-            const v4i pf = *(const v4i*)(abuf + m * 64 + (((2 * ks + lh) ^ ((m >> 1) & 3)) << 4));
-#pragma unroll
-            for (int nb = 0; nb < NBW; ++nb) {
-                const v4i wf = *(const v4i*)(bbuf + ((ks * NB + wn * NBW + nb) * 64 + lane) * 16);
-                acc[nb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wf, pf, acc[nb], 0, 0, 0);
-            }
-        }
-    }
-
-    // ---- epilogue: lane (l32, lh) holds, for pixel 32 * wm + l32, channels 32 * (wn * NBW + nb) + 8 * g + 4 * lh + e in
-    // acc[nb][4 * g + e]
-    const int m = 32 * wm + l32;
-    const int px = m & 15, py = m >> 4;
-    const int oxo = tx * q.tw + px, oyo = ty * 8 + py;
-    const bool pix_ok = px < q.tw && oxo < q.OW && oyo < q.OH;
-    const int* tab = (const int*)(smem + T_OFF);
-    signed char* orow = q.out + (((long long)b * q.OH + oyo) * q.OW + oxo) * q.O + n0 + wn * NBW * 32 + 32 * lh;
-#pragma unroll
-    for (int j = 0; j < NBW / 2; ++j) {
-        unsigned pk[2][4];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int ch = (wn * NBW + 2 * j + i) * 32 + 8 * g + 4 * lh;
-                const v4i tc = *(const v4i*)(tab + 2 * NT + ch), td = *(const v4i*)(tab + 3 * NT + ch), te = *(const v4i*)(tab + 4 * NT + ch);
-                int r[4];
+                for (int ky = 0; ky < 3; ++ky)
+                    s = __builtin_amdgcn_mfma_i32_16x16x64_i8(k.w[ky], f[S * r + ky], s, 0, 0, 0);
+                int v[4];
+                unsigned packed;
                 if (FAST) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        r[e] = (__mul24(acc[2 * j + i][4 * g + e], tc[e]) + td[e]) >> te[e];
-                    pk[i][g] = sat_bytes_u8(r[0], r[1], r[2], r[3]) ^ q.out_xor;
+                        v[e] = scale24(s[e], k.ce[e], k.d[e]);
+                    packed = sat_bytes_u8(v[0], v[1], v[2], v[3]);
                 } else {
-                    const v4i ta = *(const v4i*)(tab + ch), tb = *(const v4i*)(tab + NT + ch);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int t = med3_i32(acc[2 * j + i][4 * g + e], ta[e], tb[e]);
-                        r[e] = med3_i32((__mul24(t, tc[e]) + td[e]) >> te[e], q.pw_lo, q.pw_hi);
-                    }
-                    pk[i][g] = pack_bytes(r[0], r[1], r[2], r[3]) ^ q.out_xor;
+                    for (int e = 0; e < 4; ++e)
+                        v[e] = med3_i32(scale24(clamp_i32(s[e], k.a[e], k.b[e]), k.ce[e], k.d[e]), q.dw_lo, q.dw_hi);
+                    packed = pack_bytes(v[0], v[1], v[2], v[3]);
                 }
+                *(unsigned*)(ab + r * 16 * KC) = packed ^ q.mid_xor;
+            }
+            if (++kc == nchunks)
+                kc = 0;
+        }
+        stored = false;
+        if (step == 0)
+            continue;
+        __builtin_amdgcn_sched_barrier(0);       // (registers: nothing of this part is read early)
+        // ---- multiply the chunk before: this wave's 32 pixels against all its channel blocks
+        const unsigned char* abuf = smem + Z::A_OFF + ((step - 1) & 1) * Z::A_BYTES;
+        const unsigned char* bbuf = smem + Z::B_OFF + (SINGLE ? 0 : ((step - 1) & 1) * Z::B_BYTES);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            v4i pf[PB];
+#pragma unroll
+            for (int u = 0; u < PB; ++u)
+                pf[u] = *(const v4i*)(abuf + pf_addr + u * 32 * KC + (((2 * ks + lh) ^ swizzle(l32)) << 4));
+#pragma unroll
+            for (int nb = 0; nb < NBW; ++nb) {
+                const v4i wf = *(const v4i*)(bbuf + ((ks * NB + wn * NBW + nb) * 64 + lane) * 16);
+#pragma unroll
+                for (int u = 0; u < PB; ++u)
+                    acc[u][nb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wf, pf[u], SINGLE && ks == 0 ? v16i{} : acc[u][nb], 0, 0, 0);
             }
         }
-        // exchange between the lane halves until a lane owns 32 consecutive channels of the pair of blocks
-        unsigned qd[2][4];
+        if (++pkc < nchunks)
+            continue;
+        pkc = 0;
+        stored = true;
+
+        // ---- epilogue: lane (l32, lh) holds, for pixel m0 + 32 * u, channels 32 * (wn * NBW + nb) + 8 * h + 4 * lh + e in
+        // acc[u][nb][4 * h + e]
+        unsigned qd[PB][NBW][4];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const auto s02 = __builtin_amdgcn_permlane32_swap(pk[i][0], pk[i][2], false, false);
-            const auto s13 = __builtin_amdgcn_permlane32_swap(pk[i][1], pk[i][3], false, false);
-            qd[i][0] = s02[0]; qd[i][1] = s02[1]; qd[i][2] = s13[0]; qd[i][3] = s13[1];
-        }
-        v4i first, second;
+        for (int i = 0; i < NBW; ++i) {
+            if (!FAST)
+                __builtin_amdgcn_sched_barrier(0);
+            unsigned pk[PB][4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const auto xw = __builtin_amdgcn_permlane32_swap(qd[0][e], qd[1][e], false, false);
-            first[e] = (int)xw[0];
-            second[e] = (int)xw[1];
+            for (int h = 0; h < 4; ++h) {
+                const int ch = (wn * NBW + i) * 32 + 8 * h + 4 * lh;
+                const v4i tce = *(const v4i*)(tab + ch), td = *(const v4i*)(tab + NT + ch);
+                v4i ta, tb;
+                if (!FAST) {
+                    ta = *(const v4i*)(tab + 2 * NT + ch);
+                    tb = *(const v4i*)(tab + 3 * NT + ch);
+                }
+#pragma unroll
+                for (int u = 0; u < PB; ++u) {
+                    int r[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (FAST) r[e] = scale24(acc[u][i][4 * h + e], tce[e], td[e]);
+                        else r[e] = med3_i32(scale24(clamp_i32(acc[u][i][4 * h + e], ta[e], tb[e]), tce[e], td[e]), q.pw_lo, q.pw_hi);
+                    }
+                    pk[u][h] = (FAST ? sat_bytes_u8(r[0], r[1], r[2], r[3]) : pack_bytes(r[0], r[1], r[2], r[3])) ^ q.out_xor;
+                }
+            }
+            // exchange between the lane halves: the lower lane owns the block's first 16 channels, the upper one the others
+#pragma unroll
+            for (int u = 0; u < PB; ++u) {
+                const auto s02 = __builtin_amdgcn_permlane32_swap(pk[u][0], pk[u][2], false, false);
+                const auto s13 = __builtin_amdgcn_permlane32_swap(pk[u][1], pk[u][3], false, false);
+                qd[u][i][0] = s02[0]; qd[u][i][1] = s02[1]; qd[u][i][2] = s13[0]; qd[u][i][3] = s13[1];
+            }
         }
-        if (pix_ok) {
-            *(v4i*)(orow + 64 * j) = first;
-            *(v4i*)(orow + 64 * j + 16) = second;
+#pragma unroll
+        for (int u = 0; u < PB; ++u) {
+            const int m = m0 + 32 * u, px = m & 15, py = m >> 4;
+            const int oxo = et.x * q.tw + px, oyo = et.y * 8 + py;
+            const bool pix_ok = px < q.tw && oxo < q.OW && oyo < q.OH;
+            // (a store outside the tensor is dropped by its bounds: every wave issues all of them, which the wait above counts)
+            const unsigned out_off = pix_ok ? (unsigned)((((et.b * q.OH + oyo) * q.OW + oxo) * q.O) + n0 + wn * NBW * 32 + 16 * NBW * lh) : 0x80000000u;
+            typedef unsigned v4u __attribute__((ext_vector_type(4)));
+            v4u first, second;
+            if constexpr (NBW == 1) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    first[e] = qd[u][0][e];
+                __builtin_amdgcn_raw_buffer_store_b128(first, out_rsrc, out_off, 0, 0);
+            } else {
+                // ... of a pair: the lower lane owns the first block's 32 channels
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const auto xw = __builtin_amdgcn_permlane32_swap(qd[u][0][e], qd[u][1][e], false, false);
+                    first[e] = xw[0];
+                    second[e] = xw[1];
+                }
+                __builtin_amdgcn_raw_buffer_store_b128(first, out_rsrc, out_off, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b128(second, out_rsrc, out_off + 16, 0, 0);
+            }
+        }
+        advance(et);
+        if (!SINGLE) {
+#pragma unroll
+            for (int u = 0; u < PB; ++u)
+#pragma unroll
+                for (int i = 0; i < NBW; ++i)
+                    acc[u][i] = v16i{};
         }
     }
 }
@@ -285,18 +405,43 @@ bool plain_1x1(const n2d2hip_conv_desc& d)
 
 int byte_type_of(const n2d2hip_act_s* a) { return a->min_out >= 0 ? N2D2HIP_U8B : N2D2HIP_I8; }
 
-template <int S, int KC, bool FAST>
-void launch_nb(const DwPwArgs& a, int nb, dim3 grid, hipStream_t stream)
+
+template <int S, int KC, int NB, int WAVES, bool SINGLE, bool FAST>
+void launch_one(DwPwArgs a, int ytiles, hipStream_t stream)
 {
-    if (nb == 8) N2D2HIP_LAUNCH_T(dw_pw_kernel, (S, KC, 8, 8, FAST), grid, dim3(512), 0, stream, a);
-    else if (nb == 4) N2D2HIP_LAUNCH_T(dw_pw_kernel, (S, KC, 4, 4, FAST), grid, dim3(256), 0, stream, a);
-    else N2D2HIP_LAUNCH_T(dw_pw_kernel, (S, KC, 2, 4, FAST), grid, dim3(256), 0, stream, a);
+    // as many work-groups as the chip holds at a time, each with a run of tiles: their loads overlap the tile before, and
+    // tables, addresses and (one chunk) weights are prepared once
+    typedef DwPwShape<S, KC, NB, WAVES, SINGLE, FAST> Z;
+    const int slots = std::max(1, num_cus() / 8 * Z::GROUPS / ytiles);       // work-groups of an XCD at a time
+    a.per_xcd = (a.ntiles + 7) / 8;
+    const int groups = std::min(slots, a.per_xcd);
+    a.per_block = a.per_xcd / groups;
+    a.extra_tiles = a.per_xcd % groups;          // to the first work-groups, each of which shares its unit with a later one
+    const dim3 grid((unsigned)(8 * groups), (unsigned)ytiles);
+    N2D2HIP_LAUNCH_T(dw_pw_kernel, (S, KC, NB, WAVES, SINGLE, FAST), grid, dim3(64 * WAVES), 0, stream, a);
 }
 
-template <int S, int KC>
-void launch_fast(const DwPwArgs& a, bool fast, int nb, dim3 grid, hipStream_t stream)
+template <int S, int KC, bool SINGLE, bool FAST>
+void launch_nb(const DwPwArgs& a, int nb, hipStream_t stream)
 {
-    if (fast) launch_nb<S, KC, true>(a, nb, grid, stream); else launch_nb<S, KC, false>(a, nb, grid, stream);
+    const int ytiles = a.O / (nb * 32);
+    if (nb == 8) launch_one<S, KC, 8, 16, SINGLE, FAST>(a, ytiles, stream);
+    else if (nb == 4) launch_one<S, KC, 4, 8, SINGLE, FAST>(a, ytiles, stream);
+    else launch_one<S, KC, 2, 4, SINGLE, FAST>(a, ytiles, stream);
+}
+
+template <int S, int KC, bool SINGLE>
+void launch_fast(const DwPwArgs& a, bool fast, int nb, hipStream_t stream)
+{
+    if (fast) launch_nb<S, KC, SINGLE, true>(a, nb, stream); else launch_nb<S, KC, SINGLE, false>(a, nb, stream);
+}
+
+template <int S>
+void launch_chunks(const DwPwArgs& a, bool fast, int nb, hipStream_t stream)
+{
+    if (a.C == 32) launch_fast<S, 32, true>(a, fast, nb, stream);
+    else if (a.C == 64) launch_fast<S, 64, true>(a, fast, nb, stream);
+    else launch_fast<S, 64, false>(a, fast, nb, stream);
 }
 
 } // namespace
@@ -306,10 +451,10 @@ using namespace n2d2hip;
 
 struct n2d2hip_dw_pw_s {
     n2d2hip_conv_t dw, pw;
-    int kc, nb;               // channels per chunk, 32-channel blocks per work-group
+    int nb;                   // 32-channel blocks per work-group
     bool fast;                // neither rescale clamps before its multiply, both saturate to [0, 255]
     signed char* d_w;
-    int* d_tab;
+    int* d_tab;               // 1x1 tables, [4][O]; 4 ints of the depthwise input's stored 0; depthwise tables by chunk
 };
 
 extern "C" {
@@ -339,7 +484,7 @@ int n2d2hip_dw_pw_create(n2d2hip_conv_t dw, n2d2hip_conv_t pw, n2d2hip_dw_pw_t* 
                     "dw_pw_create: needs a 3x3 undilated depthwise convolution of stride 1 or 2 over 32 or a multiple of 64 channels and an "
                     "unpadded 1x1 convolution of stride 1 reading it, to 64, 128 or a multiple of 256 channels, both 8-bit with integer "
                     "rescales (32-bit multiply-add) and byte outputs, the second without a folded sum");
-    const int kc = C == 32 ? 32 : 64, nb = std::min(O, 256) / 32, nt = nb * 32;
+    const int kc = C == 32 ? 32 : 64, nb = std::min(O, 256) / 32;
     const int nchunks = C / kc, ks = kc / 32;
     std::vector<signed char> w((size_t)pw->opad * pw->ktot);
     const int cp = pw->act->cpad;
@@ -363,21 +508,44 @@ int n2d2hip_dw_pw_create(n2d2hip_conv_t dw, n2d2hip_conv_t pw, n2d2hip_dw_pw_t* 
         return img;
     };
     const std::vector<signed char> img = fragment_image(nb);
-    (void)nt;
-    // a, b, c, d, e by channel; a cell that needs no clamp before its multiply gets bounds that clamp nothing
-    std::vector<int> tab(5 * (size_t)O);
-    for (int r = 0; r < 5; ++r)
-        for (int o = 0; o < O; ++o)
-            tab[(size_t)r * O + o] = tab5[(size_t)r * cp + o];
-    if (!pw->preclamp)
-        for (int o = 0; o < O; ++o) {
-            tab[o] = std::numeric_limits<int>::min();
-            tab[(size_t)O + o] = std::numeric_limits<int>::max();
-        }
-    n2d2hip_dw_pw_s* h = new n2d2hip_dw_pw_s();
-    h->dw = dw; h->pw = pw; h->kc = kc; h->nb = nb; h->d_w = nullptr; h->d_tab = nullptr;
-    h->fast = dw->bias_folded && dw->d_epi_tab && !dw->preclamp && dw->act->args.lo == 0 && dw->act->args.hi == 255
+    // c and e, d, a, b by channel; a cell that needs no clamp before its multiply gets bounds that clamp nothing
+    auto with_shift = [](int c, int e) { return (int)(((unsigned)c & 0xffffffu) | (unsigned)e << 24); };
+    std::vector<int> tab(4 * (size_t)O);
+    for (int o = 0; o < O; ++o) {
+        tab[o] = with_shift(tab5[2 * (size_t)cp + o], tab5[4 * (size_t)cp + o]);
+        tab[(size_t)O + o] = tab5[3 * (size_t)cp + o];
+        tab[2 * (size_t)O + o] = pw->preclamp ? tab5[o] : std::numeric_limits<int>::min();
+        tab[3 * (size_t)O + o] = pw->preclamp ? tab5[(size_t)cp + o] : std::numeric_limits<int>::max();
+    }
+    // 16 bytes of the depthwise input's stored 0 behind them, then the depthwise tables
+    tab.insert(tab.end(), 4, zero_point(dw->in_dtype) ? (int)0x80808080u : 0);
+    const bool fast = dw->bias_folded && dw->d_epi_tab && !dw->preclamp && dw->act->args.lo == 0 && dw->act->args.hi == 255
         && !pw->preclamp && pw->act->args.lo == 0 && pw->act->args.hi == 255;
+    {
+        const EpiArgs& t = dw->act->args;
+        const int cpd = dw->act->cpad;
+        const int* w = dw->d_wdw;
+        const int* rows[] = {w, w + C, w + 2 * (size_t)C, fast ? dw->d_epi_tab + 2 * cpd : t.c, fast ? dw->d_epi_tab + 3 * cpd : t.d,
+                             w + 3 * (size_t)C, t.a, t.b, fast ? dw->d_epi_tab + 4 * cpd : t.e};     // in the order of DWT_*, then e
+        const size_t base = tab.size();
+        tab.resize(base + (size_t)nchunks * DWT_ROWS * kc);
+        std::vector<int> row(C);
+        for (int r = 0; r <= DWT_USED; ++r) {
+            e = hipMemcpy(row.data(), rows[r], C * sizeof(int), hipMemcpyDeviceToHost);
+            if (e != hipSuccess)
+                return fail(N2D2HIP_ERR_HIP, "dw_pw_create: reading the depthwise tables back failed: %s", hipGetErrorString(e));
+            for (int c = 0; c < C; ++c) {
+                int* const t0 = tab.data() + base + (size_t)(c / kc) * DWT_ROWS * kc + c % kc;
+                if (r < 3)
+                    for (int kx = 0; kx < 3; ++kx)
+                        t0[(DWT_W + kx) * kc] |= (row[c] >> (8 * kx) & 255) << (8 * r);
+                else if (r == DWT_USED) t0[DWT_CE * kc] = with_shift(t0[DWT_CE * kc], row[c]);
+                else t0[r * kc] = row[c];
+            }
+        }
+    }
+    n2d2hip_dw_pw_s* h = new n2d2hip_dw_pw_s();
+    h->dw = dw; h->pw = pw; h->nb = nb; h->fast = fast; h->d_w = nullptr; h->d_tab = nullptr;
     e = hipMalloc((void**)&h->d_w, img.size());
     if (e == hipSuccess) e = hipMemcpy(h->d_w, img.data(), img.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMalloc((void**)&h->d_tab, tab.size() * sizeof(int));
@@ -427,14 +595,12 @@ int n2d2hip_dw_pw_forward(n2d2hip_dw_pw_t h, const n2d2hip_tensor* in, const n2d
                     N2D2HIP_ERR_UNSUPPORTED, "dw_pw_forward: tensor too large");
     DwPwArgs a;
     a.in = (const signed char*)in->data; a.out = (signed char*)out->data;
-    a.wdw = h->dw->d_wdw; a.dwe = h->dw->act->args;
-    if (h->fast) {
-        const int cpd = h->dw->act->cpad;
-        a.dwe.c = h->dw->d_epi_tab + 2 * cpd; a.dwe.d = h->dw->d_epi_tab + 3 * cpd; a.dwe.e = h->dw->d_epi_tab + 4 * cpd;
-    }
     a.wpw = h->d_w; a.pwt = h->d_tab;
+    a.fill_line = (const signed char*)(h->d_tab + 4 * dp.O);
+    a.dwt = h->d_tab + 4 * dp.O + 4;
+    a.dw_lo = h->dw->act->args.lo; a.dw_hi = h->dw->act->args.hi;
     a.C = dd.C; a.O = dp.O;
-    a.B = in->B; a.H = in->H; a.W = in->W; a.OH = OH; a.OW = OW; a.padL = dd.padL; a.padT = dd.padT;
+    a.H = in->H; a.W = in->W; a.OH = OH; a.OW = OW; a.padL = dd.padL; a.padT = dd.padT;
     // columns of a tile: 16, or fewer when that leaves fewer idle columns in the last tile of a row
     int best_tw = 16;
     long long best_cols = ((OW + 15) / 16) * 16;
@@ -448,17 +614,12 @@ int n2d2hip_dw_pw_forward(n2d2hip_dw_pw_t h, const n2d2hip_tensor* in, const n2d
     const long long ntiles = (long long)in->B * a.tiles_y * a.tiles_x;
     N2D2HIP_REQUIRE(ntiles < (1 << 28), N2D2HIP_ERR_UNSUPPORTED, "dw_pw_forward: tensor too large");
     a.ntiles = (int)ntiles;
-    a.fill = zero_point(in->dtype) ? 0x80808080u : 0u;
     a.mid_xor = h->pw->in_dtype == N2D2HIP_U8B ? 0x80808080u : 0u;
     a.out_xor = out_dtype == N2D2HIP_U8B ? 0x80808080u : 0u;
     a.pw_lo = h->pw->act->args.lo; a.pw_hi = h->pw->act->args.hi;
     a.out_bytes = (unsigned)((long long)out->B * OH * OW * out->cs);
-    const dim3 grid((unsigned)(((a.ntiles + 7) / 8) * 8), (unsigned)(dp.O / (h->nb * 32)));
-    if (dd.strideX == 1) {
-        if (h->kc == 32) launch_fast<1, 32>(a, h->fast, h->nb, grid, stream); else launch_fast<1, 64>(a, h->fast, h->nb, grid, stream);
-    } else {
-        if (h->kc == 32) launch_fast<2, 32>(a, h->fast, h->nb, grid, stream); else launch_fast<2, 64>(a, h->fast, h->nb, grid, stream);
-    }
+    if (dd.strideX == 1) launch_chunks<1>(a, h->fast, h->nb, stream);
+    else launch_chunks<2>(a, h->fast, h->nb, stream);
     N2D2HIP_HIP_CHECK(hipGetLastError());
     return N2D2HIP_OK;
 }
