@@ -176,12 +176,24 @@ int depthwise3x3_launch(DepthwiseArgs a, int stride, int num_cus, hipStream_t st
 {
     N2D2HIP_REQUIRE((stride == 1 || stride == 2) && a.cs % 4 == 0, N2D2HIP_ERR_INVALID, "depthwise3x3: stride %d, channel stride %d", stride, a.cs);
     a.cq = (unsigned)(a.cs / 4);
-    // Strips short enough that every compute unit holds about 1024 threads: a strip re-reads the two input rows above it.
+    // A strip re-reads the two input rows above it and computes whole turns of the kernel's loop, and a compute unit needs
+    // some waves: strips of a multiple of a turn's rows, up to 8 (14 rows gain 2 % more on large planes and lose 4 % at
+    // 64 x 256 x 28 x 28), as long as the chip holds 400 threads a unit.  Strips that filled 1024 threads a unit were up to
+    // four times as many, and of rows that left turns half empty.  us by rows of a strip, images x channels x height x width:
+    //   64 x 512 x 14 x 14   2: 11.6   4: 7.7   5 (the former rule): 9.1   8: 7.3
+    //   64 x 1024 x 7 x 7    2: 7.2    4: 5.2   3 (the former rule): 6.5   8: 4.9
+    //   64 x 128 x 56 x 56   2: 37.5   4: 21.5  28 (the former rule): 18.7  8: 18.4
+    //   8 x 256 x 28 x 28    2: 4.8    4: 3.7   2 (the former rule): 4.9   8: 3.9
+    //   stride 2, 64 x 256 x 28 x 28   2: 6.2   4: 5.9   3 (the former rule): 6.3   8: 5.7
+    // (What is left is the vector ALU: the same on the matrix cores, 16 channels x 16 pixels an instruction with operands
+    // straight from memory, took 8.7 where this takes 7.3, and 5.3 for 4.9; the next turn's rows requested a turn ahead +4 %.)
     const long long columns = (long long)a.B * a.OW * a.cq;
-    const long long want = (long long)num_cus * 1024;
-    long long nstrips = std::min<long long>((want + columns - 1) / columns, (a.OH + 1) / 2);
-    nstrips = std::max<long long>(nstrips, 1);
-    a.rows = (int)((a.OH + nstrips - 1) / nstrips);
+    const long long want = (long long)num_cus * 400;
+    const int turn = stride == 1 ? 4 : 2;
+    const long long nstrips = std::max<long long>(std::min<long long>((want + columns - 1) / columns, (a.OH + 1) / 2), 1);
+    const long long rows = (a.OH + nstrips - 1) / nstrips, whole = (rows + turn - 1) / turn * turn;
+    // (with less than 100 threads a unit left, a turn is time to wait for and no work: 1 x 512 x 14 x 14 3.00 at 2 rows, 3.04 at 4)
+    a.rows = (int)std::min<long long>(columns * ((a.OH + whole - 1) / whole) * 4 >= want ? whole : rows, 8);
     a.nstrips = (a.OH + a.rows - 1) / a.rows;
     const long long nthreads = columns * a.nstrips;
     N2D2HIP_REQUIRE(nthreads < (1ll << 31), N2D2HIP_ERR_UNSUPPORTED, "depthwise3x3: tensor too large");
