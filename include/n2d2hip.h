@@ -407,7 +407,7 @@ int n2d2hip_conv_chain_forward(n2d2hip_conv_t conv3x3, n2d2hip_conv_t expand, co
 /* Graph-level fusion of the MobileNet building block: `depthwise` (3x3, groups == channels, stride 1 or 2, undilated) and
  * `pointwise` (1x1, stride 1, unpadded), the only reader of its output.  That is ConvCell_Frame::propagate twice
  * (ref: src/Cell/ConvCell_Frame.cpp:418-473, kernels src/Cell/ConvCell_Frame_Kernels.cpp:26-179) in one launch: the
- * depthwise output goes from the vector ALU through LDS straight into the matrix cores and is never written to memory;
+ * depthwise output goes through LDS straight into the 1x1 convolution and is never written to memory;
  * results are those of the separate cells, bit for bit.  The handles are borrowed, must outlive this one and stay usable
  * on their own.  Returns N2D2HIP_ERR_UNSUPPORTED (the caller keeps the separate launches) unless both cells are 8-bit
  * with integer rescales (32-bit multiply-add) and byte outputs, over 32 or a multiple of 64 channels, to 64, 128 or a
@@ -416,12 +416,22 @@ typedef struct n2d2hip_dw_pw_s* n2d2hip_dw_pw_t;
 int n2d2hip_dw_pw_create(n2d2hip_conv_t depthwise, n2d2hip_conv_t pointwise, n2d2hip_dw_pw_t* fused);
 int n2d2hip_dw_pw_destroy(n2d2hip_dw_pw_t fused);
 /* 1 when the one launch is expected to be faster than the two cells' own on `batch` inputs of in_h x in_w (measured rule:
- * at most 256 outputs and at least 32768 output pixels), else 0.  No counterpart in the reference: a planner's question
- * (DeepNet::planFusion asks it). */
+ * at most 256 outputs and at least 32768 output pixels, 9216 with more than 128 outputs), else 0.  No counterpart in the
+ * reference: a planner's question (DeepNet::planFusion asks it). */
 int n2d2hip_dw_pw_pays(n2d2hip_dw_pw_t fused, int batch, int in_h, int in_w);
 /* `in`: input of `depthwise`; `out`: output of `pointwise`.  NHWC bytes without a border, channel stride equal to the
  * channel count. */
 int n2d2hip_dw_pw_forward(n2d2hip_dw_pw_t fused, const n2d2hip_tensor* in, const n2d2hip_tensor* out, n2d2hip_stream_t stream);
+/* The same for few pixels: work-groups of 16 pixels x 32 outputs, each of which computes the depthwise convolution of its
+ * pixels itself, or the kernel above where that is faster (up to 128 outputs).  Taken are 8-bit cells with integer rescales
+ * (of either width) and byte outputs, over 32 or a multiple of 64 channels, to a multiple of 32; tensors, results and the
+ * handles' lifetimes as above.  _pays: 1 where the one launch is expected to be faster than the two cells' own (measured
+ * rule, at the function). */
+typedef struct n2d2hip_dw_pw_small_s* n2d2hip_dw_pw_small_t;
+int n2d2hip_dw_pw_small_create(n2d2hip_conv_t depthwise, n2d2hip_conv_t pointwise, n2d2hip_dw_pw_small_t* fused);
+int n2d2hip_dw_pw_small_destroy(n2d2hip_dw_pw_small_t fused);
+int n2d2hip_dw_pw_small_pays(n2d2hip_dw_pw_small_t fused, int batch, int in_h, int in_w);
+int n2d2hip_dw_pw_small_forward(n2d2hip_dw_pw_small_t fused, const n2d2hip_tensor* in, const n2d2hip_tensor* out, n2d2hip_stream_t stream);
 
 /* --------------------------------------------------- SAT / LSQ fake-quant */
 /* Weight quantizer modes, numbered as SATQuantizerCell_Frame::propagate selects them

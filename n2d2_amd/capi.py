@@ -34,6 +34,7 @@ SYMBOLS = [
     "n2d2hip_conv_fuse_sum", "n2d2hip_conv_forward_sum", "n2d2hip_conv_chain_supported", "n2d2hip_conv_chain_pays", "n2d2hip_conv_chain_forward", "n2d2hip_bottleneck_create", "n2d2hip_bottleneck_destroy", "n2d2hip_bottleneck_pays", "n2d2hip_bottleneck_forward",
     "n2d2hip_conv_accepts_maxpool", "n2d2hip_conv_forward_maxpool", 
     "n2d2hip_dw_pw_create", "n2d2hip_dw_pw_destroy", "n2d2hip_dw_pw_forward", "n2d2hip_dw_pw_pays",
+    "n2d2hip_dw_pw_small_create", "n2d2hip_dw_pw_small_destroy", "n2d2hip_dw_pw_small_forward", "n2d2hip_dw_pw_small_pays",
     "n2d2hip_fc_create", "n2d2hip_fc_destroy", "n2d2hip_fc_forward", "n2d2hip_fc_chain_create", "n2d2hip_fc_chain_destroy", "n2d2hip_fc_chain_forward",
     "n2d2hip_cell_run_create", "n2d2hip_cell_run_destroy", "n2d2hip_cell_run_forward",
     "n2d2hip_pool_out_dims", "n2d2hip_pool_forward", "n2d2hip_pool_writes_halo", "n2d2hip_pool_forward_mapped",
@@ -127,10 +128,11 @@ def load():
     lib.n2d2hip_bottleneck_forward.argtypes = [P, P, P, P]
     lib.n2d2hip_conv_accepts_maxpool.argtypes = [P, P, C.c_int, C.c_int]
     lib.n2d2hip_conv_forward_maxpool.argtypes = [P, P, P, P, P]
-    lib.n2d2hip_dw_pw_create.argtypes = [P, P, P]
-    lib.n2d2hip_dw_pw_destroy.argtypes = [P]
-    lib.n2d2hip_dw_pw_forward.argtypes = [P, P, P, P]
-    lib.n2d2hip_dw_pw_pays.argtypes = [P, C.c_int, C.c_int, C.c_int]
+    for size in ("dw_pw", "dw_pw_small"):
+        getattr(lib, "n2d2hip_%s_create" % size).argtypes = [P, P, P]
+        getattr(lib, "n2d2hip_%s_destroy" % size).argtypes = [P]
+        getattr(lib, "n2d2hip_%s_forward" % size).argtypes = [P, P, P, P]
+        getattr(lib, "n2d2hip_%s_pays" % size).argtypes = [P, C.c_int, C.c_int, C.c_int]
     lib.n2d2hip_fc_create.argtypes = [I, I, I, I, I, P, P, P, I, P]
     lib.n2d2hip_fc_destroy.argtypes = [P]
     lib.n2d2hip_fc_forward.argtypes = [P, P, P, P]

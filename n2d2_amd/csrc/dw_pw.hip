@@ -566,10 +566,11 @@ int n2d2hip_dw_pw_pays(n2d2hip_dw_pw_t h, int batch, int in_h, int in_w)
     if (n2d2hip_conv_out_dims(&h->dw->desc, in_h, in_w, &OH, &OW) != N2D2HIP_OK)
         return 0;
     const long long pixels = (long long)batch * OH * OW;
-    // One work-group holds all output channels of its pixels and the tensor between the cells is large: with more than 256
-    // output channels the depthwise part is computed once per 256 of them, and on small images the launch has too few
-    // work-groups to fill the chip.
-    return h->pw->desc.O <= 256 && pixels >= 32768 ? 1 : 0;
+    // With more than 256 outputs the depthwise part is computed once per 256 of them.  A work-group of 256 outputs takes 9 us for
+    // its first tile, so that launches of fewer than two thirds of a tile a unit lose: 256 -> 256 at 28 x 28, this and two
+    // launches, us: 8 images 9.4 8.4, 12 9.6 10.6, 16 9.8 10.9, 64 18.4 and 35.  Up to 128 outputs it wins at every size; below
+    // 32768 pixels n2d2hip_dw_pw_small_*, which knows one more kernel, decides.
+    return h->pw->desc.O <= 256 && pixels >= (h->pw->desc.O > 128 ? 9216 : 32768) ? 1 : 0;
 }
 
 int n2d2hip_dw_pw_forward(n2d2hip_dw_pw_t h, const n2d2hip_tensor* in, const n2d2hip_tensor* out, n2d2hip_stream_t stream_)

@@ -1,0 +1,354 @@
+// A 3x3 depthwise convolution and the 1x1 convolution that reads it, in one launch, for few pixels: MobileNet-v1 on one
+// image.  There both launches are mostly their fixed cost (2.5 us of 4 on this chip), and the kernel for many pixels
+// (dw_pw.hip), whose work-groups own 128 pixels and all their outputs, would leave most of the chip idle.
+//
+// A work-group owns 16 pixels x 32 outputs and computes the depthwise convolution of its pixels itself, once per 32 outputs:
+// what is computed again is 9 products an element, and shared are the latencies of one launch.  Its waves share the channels,
+// a chunk of 64 each (or two, past 512 channels), and work alone until their sums meet in LDS:
+//  * the 9 pixels of each output pixel and the chunk's tables go to the wave's own part of LDS by direct loads, 64 contiguous
+//    bytes a pixel (16 bytes a lane of scattered pixels, straight to registers, took 10.4 us for 512 -> 512 channels at
+//    14 x 14: the address unit takes a cycle for each line a load touches);
+//  * the depthwise convolution of 16 channels x 16 pixels is a 16x16x64 instruction a tap row, whose 64 terms are 16 channels
+//    at 4 columns (three taps, the fourth weighing 0);
+//  * of its result a lane holds 4 channels of one pixel, and the rescaled bytes of 4 channel groups are, as they lie, the
+//    pixel operand of the 1x1 convolution's 16x16x64 instruction, whose weights are laid out for that order of the channels.
+#include <algorithm>
+#include <vector>
+
+#include "common.h"
+#include "conv_handle.hpp"
+#include "epilogue.hpp"
+#include "mfma_util.hpp"
+
+namespace n2d2hip {
+
+namespace {
+
+// rows of a chunk's depthwise tables: tap columns as dwords (w[0][kx], w[1][kx], w[2][kx], 0), the rescale, and what only the
+// general rescale needs
+enum { DWS_W, DWS_C = 3, DWS_D, DWS_E, DWS_BIAS, DWS_A, DWS_B, DWS_ROWS = 12 };
+constexpr int OUTS = 32, PIXELS = 16, MAX_PARTS = 8;
+constexpr int TILES_OUTS = 128;           // up to so many outputs the kernel for many pixels is considered too
+constexpr int STAGE_PIXELS = 9 * PIXELS * 64, STAGE = STAGE_PIXELS + DWS_ROWS * 64 * 4;      // bytes of LDS of a wave
+
+struct DwPwSmallArgs {
+    const signed char* in;
+    signed char* out;
+    const int* dwt;               // [chunk][DWS_ROWS][64]
+    const signed char* wpw;       // [block of 16 outputs][chunk][lane][16 bytes]
+    const int* pwt;               // bias, a, b, c, d, e, each [O]
+    const signed char* fill_line; // C bytes of the input's stored 0
+    int C, O, nchunks, parts;
+    int H, W, OH, OW, stride, padL, padT;
+    int ntasks;                   // output pixels
+    unsigned ow_mul, ow_sh, oh_mul, oh_sh;
+    unsigned mid_xor, out_xor;
+    int dw_lo, dw_hi;
+    int pw_kind, pw_lo, pw_hi;
+};
+
+// KIND of the depthwise cell's rescale (FAST: EPI_I24 with the bias folded in, no clamp before it, saturating to [0, 255]); GN:
+// groups of 16 channels in a chunk
+template <int KIND, bool FAST, int GN>
+__global__ __launch_bounds__(64 * MAX_PARTS) void dw_pw_small_kernel(const DwPwSmallArgs q)
+{
+    typedef const v4i __attribute__((address_space(1))) * GlobalQuad;
+    constexpr int OB = OUTS / 16;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];       // STAGE bytes a wave
+    const int lane = threadIdx.x & 63, p = lane & 15, g = lane >> 4;
+    const int part = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    unsigned char* const stage = smem + part * STAGE;
+
+    // the pixel this lane brings 16 bytes of, 4 lanes a pixel; a pixel's 16-channel groups are swizzled so that 16 pixels' bytes
+    // of one group lie in different banks
+    const int pl = lane >> 2, group = (lane & 3) ^ (pl >> 2 & 3);
+    const int task = min((int)blockIdx.y * PIXELS + pl, q.ntasks - 1);
+    const int t1 = div_magic(task, q.ow_mul, q.ow_sh), ox = task - t1 * q.OW;
+    const int b = div_magic(t1, q.oh_mul, q.oh_sh), oy = t1 - b * q.OH;
+    const int ix = ox * q.stride - q.padL, iy = oy * q.stride - q.padT;
+    const signed char* tap[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        const bool ok = group < GN && (unsigned)(ix + i % 3) < (unsigned)q.W && (unsigned)(iy + i / 3) < (unsigned)q.H;
+        tap[i] = (ok ? q.in + ((long long)(b * q.H + iy + i / 3) * q.W + ix + i % 3) * q.C : q.fill_line) + 16 * (group % GN);
+    }
+
+    // the matrix of a tap row weighs, for channel p, that channel's bytes only: byte p % 4 of dword p / 4 is w[ky][g]
+    const unsigned select = g == 3 ? 0x0c0c0c0cu : 0x0c0c0c0cu & ~(255u << (8 * (p & 3)));
+    const unsigned select1 = g == 3 ? 0u : 1u << (8 * (p & 3));
+    const int n0 = (int)blockIdx.x * OB;          // first block of 16 outputs
+    v4i acc[OB];
+#pragma unroll
+    for (int o = 0; o < OB; ++o)
+        acc[o] = v4i{};
+    for (int k = part; k < q.nchunks; k += q.parts) {
+        v4i wp[OB];
+#pragma unroll
+        for (int i = 0; i < 9; ++i)
+            __builtin_amdgcn_global_load_lds((gbl_ptr_t)(tap[i] + k * 64), (lds_ptr_t)(stage + i * 1024), 16, 0, 0);
+#pragma unroll
+        for (int i = 0; i < (FAST ? 2 : 3); ++i)
+            __builtin_amdgcn_global_load_lds((gbl_ptr_t)(q.dwt + ((size_t)k * DWS_ROWS + 4 * i) * 64 + 4 * lane),
+                                             (lds_ptr_t)(stage + STAGE_PIXELS + i * 1024), 16, 0, 0);
+#pragma unroll
+        for (int o = 0; o < OB; ++o)
+            wp[o] = *(GlobalQuad)(q.wpw + (((size_t)(n0 + o) * q.nchunks + k) * 64 + lane) * 16);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const int* const t = (const int*)(stage + STAGE_PIXELS);
+        const unsigned char* const px = stage + ((g < 3 ? g : 2) * PIXELS + p) * 64;
+        v4i mid = {};
+#pragma unroll
+        for (int G = 0; G < GN; ++G) {
+            const int* const tg = t + 16 * G + 4 * g;
+            const unsigned taps = (unsigned)t[g * 64 + 16 * G + p];              // (the row after the taps for the fourth column)
+            const v4i tc = *(const v4i*)(tg + DWS_C * 64), td = *(const v4i*)(tg + DWS_D * 64), te = *(const v4i*)(tg + DWS_E * 64);
+            v4i s = {}, ta = {}, tb = {};
+            if (!FAST) {
+                s = *(const v4i*)(tg + DWS_BIAS * 64);
+                ta = *(const v4i*)(tg + DWS_A * 64);
+                tb = *(const v4i*)(tg + DWS_B * 64);
+            }
+#pragma unroll
+            for (int ky = 0; ky < 3; ++ky) {
+                const v4i f = *(const v4i*)(px + ky * 3 * PIXELS * 64 + ((G ^ (p >> 2 & 3)) << 4));
+                const int byte = (int)__builtin_amdgcn_perm(0u, taps, select + ky * select1);
+                v4i w;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    w[e] = (p >> 2) == e ? byte : 0;
+                s = __builtin_amdgcn_mfma_i32_16x16x64_i8(w, f, s, 0, 0, 0);
+            }
+            int v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                v[e] = FAST ? (__mul24(s[e], tc[e]) + td[e]) >> te[e]
+                            : epi_apply<KIND>(s[e], ta[e], tb[e], tc[e], td[e], te[e], q.dw_lo, q.dw_hi, 0);
+            mid[G] = (int)((FAST ? sat_bytes_u8(v[0], v[1], v[2], v[3]) : pack_bytes(v[0], v[1], v[2], v[3])) ^ q.mid_xor);
+        }
+#pragma unroll
+        for (int o = 0; o < OB; ++o)
+            acc[o] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wp[o], mid, acc[o], 0, 0, 0);
+        if (k + q.parts < q.nchunks)              // the next chunk's loads write what this one's reads have read
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    // the sums of the waves meet where each kept its pixels
+#pragma unroll
+    for (int o = 0; o < OB; ++o)
+        *(v4i*)(stage + (o * 64 + lane) * 16) = acc[o];
+    __syncthreads();
+    // 16 pixels x 16 outputs a wave: lane (p, g) holds outputs 4 g .. 4 g + 3 of pixel p
+    for (int o = part; o < OB; o += q.parts) {
+        v4i s = *(const v4i*)(smem + (o * 64 + lane) * 16);
+        for (int i = 1; i < q.parts; ++i)
+            s += *(const v4i*)(smem + i * STAGE + (o * 64 + lane) * 16);
+        const int ch = (n0 + o) * 16 + 4 * g;
+        const v4i bias = *(const v4i*)(q.pwt + ch), a = *(const v4i*)(q.pwt + q.O + ch), bb = *(const v4i*)(q.pwt + 2 * q.O + ch);
+        const v4i c = *(const v4i*)(q.pwt + 3 * q.O + ch), d = *(const v4i*)(q.pwt + 4 * q.O + ch), e5 = *(const v4i*)(q.pwt + 5 * q.O + ch);
+        int v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            v[e] = q.pw_kind == EPI_I24 ? epi_apply<EPI_I24>(s[e] + bias[e], a[e], bb[e], c[e], d[e], e5[e], q.pw_lo, q.pw_hi, 0)
+                                        : epi_apply<EPI_I64>(s[e] + bias[e], a[e], bb[e], c[e], 0, e5[e], q.pw_lo, q.pw_hi, 0);
+        const int pix = (int)blockIdx.y * PIXELS + p;
+        if (pix < q.ntasks)
+            *(unsigned*)(q.out + (long long)pix * q.O + ch) = pack_bytes(v[0], v[1], v[2], v[3]) ^ q.out_xor;
+    }
+}
+
+template <int KIND, bool FAST>
+void launch_groups(const DwPwSmallArgs& a, dim3 grid, hipStream_t stream)
+{
+    if (a.C == 32) N2D2HIP_LAUNCH_T(dw_pw_small_kernel, (KIND, FAST, 2), grid, dim3(64 * a.parts), a.parts * STAGE, stream, a);
+    else N2D2HIP_LAUNCH_T(dw_pw_small_kernel, (KIND, FAST, 4), grid, dim3(64 * a.parts), a.parts * STAGE, stream, a);
+}
+
+bool integer_bytes(const n2d2hip_act_s* a)
+{
+    return (a->args.kind == EPI_I24 || a->args.kind == EPI_I64) && a->min_out >= -128 && a->max_out <= 255;
+}
+
+int byte_type_of(const n2d2hip_act_s* a) { return a->min_out >= 0 ? N2D2HIP_U8B : N2D2HIP_I8; }
+
+} // namespace
+} // namespace n2d2hip
+
+using namespace n2d2hip;
+
+struct n2d2hip_dw_pw_small_s {
+    n2d2hip_conv_t dw, pw;
+    n2d2hip_dw_pw_t tiles;        // the kernel for many pixels, where this handle may choose it, or null
+    bool fast;
+    int nchunks;
+    signed char* d_image;         // 1x1 weights, depthwise tables, 1x1 tables, the stored 0
+    size_t dwt_at, pwt_at, fill_at;
+};
+
+extern "C" {
+
+int n2d2hip_dw_pw_small_destroy(n2d2hip_dw_pw_small_t h)
+{
+    if (!h) return N2D2HIP_OK;
+    if (h->d_image) (void)hipFree(h->d_image);
+    if (h->tiles) n2d2hip_dw_pw_destroy(h->tiles);
+    delete h;
+    return N2D2HIP_OK;
+}
+
+int n2d2hip_dw_pw_small_create(n2d2hip_conv_t dw, n2d2hip_conv_t pw, n2d2hip_dw_pw_small_t* out)
+{
+    N2D2HIP_REQUIRE(dw && pw && out, N2D2HIP_ERR_INVALID, "dw_pw_small_create: null argument");
+    const n2d2hip_conv_desc& dd = dw->desc;
+    const n2d2hip_conv_desc& dp = pw->desc;
+    const int C = dd.C, O = dp.O;
+    const bool ok = dw->depthwise && dw->d_wdw && dd.kW == 3 && dd.kH == 3 && dd.dilX == 1 && dd.dilY == 1 && dd.strideX == dd.strideY
+        && (dd.strideX == 1 || dd.strideX == 2) && integer_bytes(dw->act) && dw->act->cpad >= C && dw->in_cs == C && (C == 32 || C % 64 == 0)
+        && dp.kW == 1 && dp.kH == 1 && dp.strideX == 1 && dp.strideY == 1 && dp.padL == 0 && dp.padT == 0 && dp.padR == 0 && dp.padB == 0
+        && dp.dilX == 1 && dp.dilY == 1 && dp.groups == 1 && dp.weight_bits == 8 && !pw->depthwise && !pw->sub_inner && !pw->is_fc
+        && dp.C == C && pw->in_cs == C && pw->in_dtype == byte_type_of(dw->act) && O % OUTS == 0 && integer_bytes(pw->act) && !pw->sum
+        && pw->ktot >= C && pw->d_bias && (int)dw->act->htab.size() >= 5 * dw->act->cpad && (int)pw->act->htab.size() >= 5 * pw->act->cpad;
+    N2D2HIP_REQUIRE(ok, N2D2HIP_ERR_UNSUPPORTED,
+                    "dw_pw_small_create: needs a 3x3 undilated depthwise convolution of stride 1 or 2 over 32 or a multiple of 64 channels and an "
+                    "unpadded 1x1 convolution of stride 1 reading it, to a multiple of 32 channels, both 8-bit with integer rescales and byte "
+                    "outputs, the second without a folded sum");
+    const int nchunks = (C + 63) / 64;
+    std::vector<signed char> w((size_t)pw->opad * pw->ktot);
+    std::vector<int> wdw(4 * (size_t)C), bias(O), fold;
+    hipError_t e = hipMemcpy(w.data(), pw->d_w, w.size(), hipMemcpyDeviceToHost);
+    if (e == hipSuccess) e = hipMemcpy(wdw.data(), dw->d_wdw, wdw.size() * sizeof(int), hipMemcpyDeviceToHost);
+    if (e == hipSuccess) e = hipMemcpy(bias.data(), pw->d_bias, bias.size() * sizeof(int), hipMemcpyDeviceToHost);
+    const bool fast = dw->bias_folded && dw->d_epi_tab && !dw->preclamp && dw->act->args.kind == EPI_I24 && dw->act->args.lo == 0
+        && dw->act->args.hi == 255;
+    const int cpd = dw->act->cpad, cpp = pw->act->cpad;
+    if (fast) {                                   // a - bias, b - bias, c, d + bias * c, e
+        fold.resize(5 * (size_t)cpd);
+        if (e == hipSuccess) e = hipMemcpy(fold.data(), dw->d_epi_tab, fold.size() * sizeof(int), hipMemcpyDeviceToHost);
+    }
+    if (e != hipSuccess)
+        return fail(N2D2HIP_ERR_HIP, "dw_pw_small_create: reading the cells back failed: %s", hipGetErrorString(e));
+    n2d2hip_dw_pw_small_s* h = new n2d2hip_dw_pw_small_s();
+    h->dw = dw; h->pw = pw; h->fast = fast; h->nchunks = nchunks; h->d_image = nullptr; h->tiles = nullptr;
+    h->dwt_at = (size_t)(O / 16) * nchunks * 1024;
+    h->pwt_at = h->dwt_at + (size_t)nchunks * DWS_ROWS * 64 * sizeof(int);
+    h->fill_at = h->pwt_at + 6 * (size_t)O * sizeof(int);
+    std::vector<signed char> img(h->fill_at + (size_t)nchunks * 64, 0);
+    // lane (p, g) of an output block: output p, and in byte 4 * G + i channel 16 * G + 4 * g + i of the chunk
+    for (int o = 0; o < O; ++o)
+        for (int c = 0; c < C; c += 4) {
+            const int k = c / 64, G = c / 16 % 4, g = c / 4 % 4;
+            memcpy(img.data() + (((size_t)(o / 16) * nchunks + k) * 64 + g * 16 + o % 16) * 16 + 4 * G, w.data() + (size_t)o * pw->ktot + c, 4);
+        }
+    int* const dwt = (int*)(img.data() + h->dwt_at);
+    const std::vector<int>& tab = fast ? fold : dw->act->htab;
+    for (int c = 0; c < C; ++c) {
+        int* const t = dwt + (size_t)(c / 64) * DWS_ROWS * 64 + c % 64;
+        for (int kx = 0; kx < 3; ++kx)
+            for (int ky = 0; ky < 3; ++ky)
+                t[(DWS_W + kx) * 64] |= (wdw[(size_t)ky * C + c] >> (8 * kx) & 255) << (8 * ky);
+        t[DWS_BIAS * 64] = wdw[3 * (size_t)C + c];
+        const int rows[5] = {DWS_A, DWS_B, DWS_C, DWS_D, DWS_E};
+        for (int r = 0; r < 5; ++r)
+            t[rows[r] * 64] = tab[(size_t)r * cpd + c];
+    }
+    int* const pwt = (int*)(img.data() + h->pwt_at);
+    for (int o = 0; o < O; ++o) {
+        pwt[o] = bias[o];
+        for (int r = 0; r < 5; ++r)
+            pwt[(size_t)(r + 1) * O + o] = pw->act->htab[(size_t)r * cpp + o];
+    }
+    memset(img.data() + h->fill_at, zero_point(dw->in_dtype) ? 0x80 : 0, img.size() - h->fill_at);
+    e = hipMalloc((void**)&h->d_image, img.size());
+    if (e == hipSuccess) e = hipMemcpy(h->d_image, img.data(), img.size(), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        n2d2hip_dw_pw_small_destroy(h);
+        return fail(N2D2HIP_ERR_HIP, "dw_pw_small_create: device upload failed: %s", hipGetErrorString(e));
+    }
+    if (O <= TILES_OUTS) {
+        const int rc = n2d2hip_dw_pw_create(dw, pw, &h->tiles);
+        if (rc != N2D2HIP_OK && rc != N2D2HIP_ERR_UNSUPPORTED) {
+            n2d2hip_dw_pw_small_destroy(h);
+            return rc;
+        }
+        if (rc != N2D2HIP_OK)
+            h->tiles = nullptr;
+    }
+    *out = h;
+    return N2D2HIP_OK;
+}
+
+// 32 pixels' worth of outputs and more channels than a chunk fill the chip only with many pixels, 8 x 16 of which the other kernel
+// gives to a work-group; up to 128 outputs it needs no more of them than one image has.  us, that kernel / this one / two
+// launches: 32 -> 64 channels, 112 x 112 3.6 / 4.8 / 7.6, two images of 48 x 48 3.4 / 4.1 / 7.5; 64 -> 128 stride 2, 56 x 56
+// 4.6 / 4.3 / 8.1, two 4.6 / 5.1 / 8.2; 128 -> 128, 56 x 56 5.1 / 4.6 / 6.6, two 5.2 / 6.7 / 7.0, four 5.3 / 10.0 / 8.0, two of 24 x 24
+// 5.7 / 4.1 / 5.9.
+static bool choose_tiles(n2d2hip_dw_pw_small_t h, long long groups)
+{
+    return h->tiles && (h->dw->desc.C == 32 || groups > 1024);
+}
+
+static long long work_groups(n2d2hip_dw_pw_small_t h, long long pixels) { return (pixels + PIXELS - 1) / PIXELS * (h->pw->desc.O / OUTS); }
+
+int n2d2hip_dw_pw_small_pays(n2d2hip_dw_pw_small_t h, int batch, int in_h, int in_w)
+{
+    if (!h || batch <= 0)
+        return 0;
+    int OH, OW;
+    if (n2d2hip_conv_out_dims(&h->dw->desc, in_h, in_w, &OH, &OW) != N2D2HIP_OK)
+        return 0;
+    const long long groups = work_groups(h, (long long)batch * OH * OW);
+    if (choose_tiles(h, groups))
+        return 1;
+    // Where all work-groups are on the chip at once (by their LDS, 12 KB a wave).  us, one launch and two, for output planes of
+    // 112 / 56 / 56 / 28 / 28 / 14 / 14 / 7 and 32 -> 64, 64 -> 128, 128 -> 128, 128 -> 256, 256 -> 256, 256 -> 512, 512 -> 512, 512 -> 1024 channels:
+    //   one image    4.8 7.6   4.3 8.1   4.6 6.6   4.1 5.8   4.6 6.1   4.2 5.7   5.2 6.1   4.7 5.8
+    //   two images   7.2 7.8   5.0 8.2   6.7 7.0*  4.6 6.3   6.8 6.9*  4.6 5.9   8.8 6.2*  4.8 5.9     * the rule declines
+    //   four        11.0 9.3*  7.6 8.7  10.0 8.0*  6.7 6.8*  9.8 7.2*  6.8 6.4* 16.0 7.3*  8.0 5.9*
+    return groups <= (long long)num_cus() * (163840 / (std::min(MAX_PARTS, h->nchunks) * STAGE)) ? 1 : 0;
+}
+
+int n2d2hip_dw_pw_small_forward(n2d2hip_dw_pw_small_t h, const n2d2hip_tensor* in, const n2d2hip_tensor* out, n2d2hip_stream_t stream_)
+{
+    hipStream_t stream = (hipStream_t)stream_;
+    N2D2HIP_REQUIRE(h && in && out && in->data && out->data, N2D2HIP_ERR_INVALID, "dw_pw_small_forward: null argument");
+    const n2d2hip_conv_desc& dd = h->dw->desc;
+    const n2d2hip_conv_desc& dp = h->pw->desc;
+    int OH, OW;
+    const int rc = n2d2hip_conv_out_dims(&dd, in->H, in->W, &OH, &OW);
+    if (rc != N2D2HIP_OK)
+        return rc;
+    const long long pixels = (long long)in->B * OH * OW;
+    if (choose_tiles(h, work_groups(h, pixels)))
+        return n2d2hip_dw_pw_forward(h->tiles, in, out, stream_);
+    const int out_dtype = byte_type_of(h->pw->act);
+    N2D2HIP_REQUIRE(in->layout == N2D2HIP_NHWC && out->layout == N2D2HIP_NHWC && in->halo == 0 && out->halo == 0, N2D2HIP_ERR_UNSUPPORTED,
+                    "dw_pw_small_forward: tensors must be NHWC without a border");
+    N2D2HIP_REQUIRE(in->dtype == h->dw->in_dtype && in->C == dd.C && in->cs == dd.C, N2D2HIP_ERR_INVALID,
+                    "dw_pw_small_forward: input has %d channels (stride %d) of type %d, the depthwise convolution expects %d of type %d", in->C,
+                    in->cs, in->dtype, dd.C, h->dw->in_dtype);
+    N2D2HIP_REQUIRE(out->B == in->B && out->C == dp.O && out->cs == dp.O && out->H == OH && out->W == OW && out->dtype == out_dtype,
+                    N2D2HIP_ERR_INVALID, "dw_pw_small_forward: output must be %dx%dx%dx%d bytes of type %d with a channel stride of %d", in->B,
+                    dp.O, OH, OW, out_dtype, dp.O);
+    N2D2HIP_REQUIRE(pixels > 0 && (pixels + PIXELS - 1) / PIXELS <= 65535 && (long long)in->B * in->H * in->W * in->cs < (1ll << 31),
+                    N2D2HIP_ERR_UNSUPPORTED, "dw_pw_small_forward: tensor too large");
+    DwPwSmallArgs a;
+    a.in = (const signed char*)in->data; a.out = (signed char*)out->data;
+    a.wpw = h->d_image; a.dwt = (const int*)(h->d_image + h->dwt_at); a.pwt = (const int*)(h->d_image + h->pwt_at);
+    a.fill_line = h->d_image + h->fill_at;
+    a.C = dd.C; a.O = dp.O; a.nchunks = h->nchunks; a.parts = std::min(MAX_PARTS, h->nchunks);
+    a.H = in->H; a.W = in->W; a.OH = OH; a.OW = OW; a.stride = dd.strideX; a.padL = dd.padL; a.padT = dd.padT;
+    a.ntasks = (int)pixels;
+    magic_div((unsigned)OW, &a.ow_mul, &a.ow_sh);
+    magic_div((unsigned)OH, &a.oh_mul, &a.oh_sh);
+    a.mid_xor = h->pw->in_dtype == N2D2HIP_U8B ? 0x80808080u : 0u;
+    a.out_xor = out_dtype == N2D2HIP_U8B ? 0x80808080u : 0u;
+    a.dw_lo = h->dw->act->args.lo; a.dw_hi = h->dw->act->args.hi;
+    a.pw_kind = h->pw->act->args.kind; a.pw_lo = h->pw->act->args.lo; a.pw_hi = h->pw->act->args.hi;
+    // (output tiles first: work-groups 8 apart share an XCD, whose L2 then holds an eighth of the 1x1 weights)
+    const dim3 grid((unsigned)(dp.O / OUTS), (unsigned)((pixels + PIXELS - 1) / PIXELS));
+    if (h->fast) launch_groups<EPI_I24, true>(a, grid, stream);
+    else if (h->dw->act->args.kind == EPI_I24) launch_groups<EPI_I24, false>(a, grid, stream);
+    else launch_groups<EPI_I64, false>(a, grid, stream);
+    N2D2HIP_HIP_CHECK(hipGetLastError());
+    return N2D2HIP_OK;
+}
+
+} // extern "C"

@@ -545,7 +545,7 @@ class GpuNet:
                 self.stem_pools[l.name] = conv
         # a 3x3 depthwise convolution and the 1x1 convolution that alone reads it as one launch (the depthwise output is
         # never written)
-        self.dw_pws = {}
+        self.dw_pws, self.dw_pws_small = {}, {}
         if fuse and dw_pw:
             step_index = {l.name: k for k, (l, c, f) in enumerate(self.steps)}
             for l in spec.layers:
@@ -555,18 +555,18 @@ class GpuNet:
                 if (dw is None or dw.type != "conv" or len(dw.inputs) != 1 or dw.groups == 1 or len(consumers[dw.name]) != 1 or dw.name in self.folded
                         or ins_of[dw.name][0].halo or self.tensors[l.name].halo):
                     continue
-                fused_cell = rt.DwPw.create(self.steps[step_index[dw.name]][1], self.steps[step_index[l.name]][1])
-                if fused_cell is None:
-                    continue
-                # the library knows where one launch is faster than two (large tensors between the cells; small images
-                # with 512 outputs per work-group)
+                # the library knows where one launch is faster than two: large tensors between the cells, and few pixels
                 x = ins_of[dw.name][0]
-                if dw_pw != "all" and not fused_cell.pays(batch, x.H, x.W):
+                for kind, pairs in ((rt.DwPw, self.dw_pws), (rt.DwPwSmall, self.dw_pws_small)):
+                    fused_cell = kind.create(self.steps[step_index[dw.name]][1], self.steps[step_index[l.name]][1])
+                    if fused_cell is not None and (fused_cell.pays(batch, x.H, x.W) or dw_pw == "all" and kind is rt.DwPw):
+                        break
+                else:
                     continue
                 self.steps[step_index[l.name]] = (l, fused_cell, (lambda c, i, o: c.forward(i[0], o)))
                 ins_of[l.name] = ins_of[dw.name]
                 self.folded.add(dw.name)
-                self.dw_pws[l.name] = dw
+                pairs[l.name] = dw
         # A tensor read by padded convolutions and, as the other input, by sums that a convolution has taken into its
         # epilogue may carry the convolutions' padding too (the epilogue finds the other input's pixels past its borders),
         # when its producer can write it: ResNet-18's block inputs, which a max pooling or such a sum produces.
@@ -919,8 +919,9 @@ class GpuNet:
             total += sum(m.w.size for m in self.fc_chains[l.name])
         if l.name in self.stem_pools:       # the convolution's weights; its output never leaves the chip
             total += self.stem_pools[l.name].w.size
-        if l.name in self.dw_pws:           # the depthwise weights; its output never leaves the chip
-            total += self.dw_pws[l.name].w.size
+        dw = self.dw_pws.get(l.name) or self.dw_pws_small.get(l.name)
+        if dw is not None:                  # the depthwise weights; its output never leaves the chip
+            total += dw.w.size
         return total
 
     def layer_macs(self, l):
@@ -931,8 +932,8 @@ class GpuNet:
             return self.layer_macs(self.fused_sums[l.name][1]) + (self.layer_macs(c3) if c3 is not None else 0)
         if l.name in self.stem_pools:
             return self.layer_macs(self.stem_pools[l.name])
-        if l.name in self.dw_pws:
-            dw = self.dw_pws[l.name]
+        dw = self.dw_pws.get(l.name) or self.dw_pws_small.get(l.name)
+        if dw is not None:
             return self.B * l.out_shape[1] * l.out_shape[2] * l.w.size + self.B * dw.out_shape[1] * dw.out_shape[2] * dw.w.size
         if l.type == "conv":
             return self.B * l.out_shape[1] * l.out_shape[2] * l.w.size

@@ -169,30 +169,38 @@ class DwPw:
     """n2d2hip_dw_pw_t: a 3x3 depthwise convolution and the 1x1 convolution reading it in one launch; None when the library
     keeps the cells apart."""
 
+    _NAME = "n2d2hip_dw_pw"
+
     def __init__(self, handle, cells):
         self.handle, self._cells = handle, cells
 
-    @staticmethod
-    def create(depthwise, pointwise):
+    @classmethod
+    def create(cls, depthwise, pointwise):
         h = C.c_void_p()
-        rc = lib.n2d2hip_dw_pw_create(depthwise.handle, pointwise.handle, C.byref(h))
+        rc = getattr(lib, cls._NAME + "_create")(depthwise.handle, pointwise.handle, C.byref(h))
         if rc == capi.ERR_UNSUPPORTED:
             return None
         check(rc)
-        return DwPw(h, (depthwise, pointwise))
+        return cls(h, (depthwise, pointwise))
 
     def forward(self, x, out):
-        check(lib.n2d2hip_dw_pw_forward(self.handle, x.ref, out.ref, stream_ptr()))
+        check(getattr(lib, self._NAME + "_forward")(self.handle, x.ref, out.ref, stream_ptr()))
         return out
 
     def pays(self, batch, in_h, in_w):
         """Does the library expect the one launch to be faster than the two cells' own on inputs of this size?"""
-        return bool(lib.n2d2hip_dw_pw_pays(self.handle, batch, in_h, in_w))
+        return bool(getattr(lib, self._NAME + "_pays")(self.handle, batch, in_h, in_w))
 
     def __del__(self):
         if getattr(self, "handle", None) and lib is not None:
-            lib.n2d2hip_dw_pw_destroy(self.handle)
+            getattr(lib, self._NAME + "_destroy")(self.handle)
             self.handle = None
+
+
+class DwPwSmall(DwPw):
+    """n2d2hip_dw_pw_small_t: the same for few pixels."""
+
+    _NAME = "n2d2hip_dw_pw_small"
 
 
 def scaling_forward(act, x, out_dtype=None):

@@ -1,0 +1,64 @@
+"""The one-launch depthwise + 1x1 kernel for few pixels against the two separate launches, byte for byte: remainders of its 16 pixels,
+one and several chunks of 64 channels a wave, both strides, every rescale it takes, and the sizes where it hands over."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,C,O,stride,H,W,pad", [
+    (1, 64, 32, 1, 1, 1, 1),           # one pixel
+    (1, 32, 96, 1, 7, 5, 1),           # half a chunk; 96 outputs (the other kernel does not take them)
+    (3, 64, 64, 2, 9, 11, 0),          # pixels of three images in one work-group, no padding
+    (2, 192, 160, 1, 6, 9, 1),         # three waves
+    (1, 512, 64, 2, 14, 14, 1),        # eight waves
+    (1, 640, 32, 1, 5, 4, 1),          # ten chunks: two waves have two
+    (2, 1024, 1024, 1, 7, 7, 1),
+    (2, 64, 128, 1, 33, 31, 1),        # 256 + groups: all on the chip
+    (2, 64, 128, 1, 48, 47, 1),        # 1128 work-groups: the kernel for many pixels
+    (1, 32, 64, 1, 20, 9, 1),          # 32 channels: the kernel for many pixels
+])
+@pytest.mark.parametrize("rescale", ["plain", "clamped", "wide"])
+def test_small_equals_separate_launches(B, C, O, stride, H, W, pad, rescale):
+    from n2d2_amd import capi, runtime as rt
+    from oracle.cells import ActSpec
+    print("dw_pw_small", B, C, O, stride, H, W, pad, rescale, flush=True)
+    rng = np.random.default_rng(C + O + H)
+    x = rng.integers(0, 256, size=(B, C, H, W))
+    wd, bd = rng.integers(-128, 128, size=(C, 1, 3, 3)), rng.integers(-2000, 2001, size=C)
+    wp, bp = rng.integers(-128, 128, size=(O, C, 1, 1)), rng.integers(-20000, 20001, size=O)
+    unsigned = dict(nb_bits=8, unsigned_out=True)
+    if rescale == "plain":
+        sd = ActSpec("Rectifier", "FixedMult32", rng.integers(2 ** 11, 2 ** 12, size=C), frac_bits=18, **unsigned)
+        sp = ActSpec("Rectifier", "FixedMult32", rng.integers(2 ** 7, 2 ** 8, size=O), frac_bits=16, **unsigned)
+    elif rescale == "clamped":         # a signed tensor between the cells
+        sd = ActSpec("Linear", "FixedMult32", rng.integers(2 ** 13, 2 ** 14, size=C), frac_bits=21, nb_bits=8, unsigned_out=False)
+        sp = ActSpec("Linear", "FixedMult32", rng.integers(2 ** 13, 2 ** 14, size=O), frac_bits=21, nb_bits=8, unsigned_out=False)
+    else:                              # multipliers past 24 bits: 64-bit rescales
+        sd = ActSpec("Rectifier", "FixedMult32", rng.integers(2 ** 25, 2 ** 26, size=C), frac_bits=33, **unsigned)
+        sp = ActSpec("Rectifier", "FixedMult32", rng.integers(2 ** 25, 2 ** 26, size=O), frac_bits=35, **unsigned)
+    dw = rt.Conv(wd, bd, rt.Act(C, **sd.kwargs()), capi.U8B, stride=(stride, stride), pad=(pad,) * 4, groups=C)
+    pw = rt.Conv(wp, bp, rt.Act(O, **sp.kwargs()), capi.I8 if rescale == "clamped" else capi.U8B)
+    xin = rt.DTensor.from_numpy(x, capi.U8B)
+    want = pw.forward(dw.forward(xin))
+    fused = rt.DwPwSmall.create(dw, pw)
+    assert fused is not None
+    out = rt.DTensor(B, O, want.H, want.W, want.dtype)
+    assert np.array_equal(fused.forward(xin, out).to_numpy(), want.to_numpy())
+
+
+def test_small_declines_what_it_is_not_written_for():
+    from n2d2_amd import capi, runtime as rt
+    from oracle.cells import ActSpec
+    rng = np.random.default_rng(5)
+    act = lambda n: rt.Act(n, **ActSpec("Rectifier", "SingleShift", rng.integers(8, 12, size=n), nb_bits=8, unsigned_out=True).kwargs())
+    conv = lambda O, C, k, g=1, **kw: rt.Conv(rng.integers(-9, 10, size=(O, C // g, k, k)), None, act(O), capi.U8B, groups=g, **kw)
+    dw = conv(64, 64, 3, 64, pad=(1,) * 4)
+    assert rt.DwPwSmall.create(dw, conv(32, 64, 1)) is not None
+    assert rt.DwPwSmall.create(dw, conv(40, 64, 1)) is None                                  # outputs not in 32s
+    assert rt.DwPwSmall.create(conv(48, 48, 3, 48, pad=(1,) * 4), conv(32, 48, 1)) is None   # channels not in 64s
+    assert rt.DwPwSmall.create(conv(64, 64, 3, 64, pad=(2,) * 4, dil=(2, 2)), conv(32, 64, 1)) is None
+    assert rt.DwPwSmall.create(dw, conv(32, 64, 3, pad=(1,) * 4)) is None
+    # one pixel pays, a batch that does not fit the chip does not
+    h = rt.DwPwSmall.create(conv(512, 512, 3, 512, pad=(1,) * 4), conv(512, 512, 1))
+    assert h.pays(1, 14, 14) and not h.pays(8, 14, 14)
