@@ -461,6 +461,30 @@ int n2d2hip_sat_weight_forward_static(const float* w, float* wq, size_t n, float
 /* ref: SATQuantizer_Frame_Kernels.cpp:349-404; factor = tanh_max * scaling read from stats */
 int n2d2hip_sat_weight_backward(const float* diff_wq, const float* w, float* diff_w, size_t n, float range,
                                 int mode, int apply_scaling, const float* stats, n2d2hip_stream_t stream);
+/* The same for `count` tensors, 16 to a launch: the weights of all cells of a learning net before a pass, and their gradients
+ * after one.  The tensors and workspaces of a call do not overlap; the results are those of one call for each. */
+typedef struct {
+    const float* w;
+    float* wq;
+    size_t n;
+    float range;
+    int mode, apply_scaling;
+    unsigned outputs_size;
+    float* stats;
+    void* workspace;
+    size_t workspace_bytes;
+} n2d2hip_sat_weight_item;
+int n2d2hip_sat_weight_forward_batch(const n2d2hip_sat_weight_item* items, int count, n2d2hip_stream_t stream);
+typedef struct {
+    const float* diff_wq;
+    const float* w;
+    float* diff_w;
+    size_t n;
+    float range;
+    int mode, apply_scaling;
+    const float* stats;
+} n2d2hip_sat_weight_grad_item;
+int n2d2hip_sat_weight_backward_batch(const n2d2hip_sat_weight_grad_item* items, int count, n2d2hip_stream_t stream);
 /* ref: SATQuantizer_Frame_Kernels.cpp:268-322; alpha: device float[1]; fp_copy NULL when inference */
 int n2d2hip_sat_act_forward(float* x, float* fp_copy, size_t n, float range, const float* alpha,
                             n2d2hip_stream_t stream);

@@ -39,7 +39,8 @@ SYMBOLS = [
     "n2d2hip_cell_run_create", "n2d2hip_cell_run_destroy", "n2d2hip_cell_run_forward",
     "n2d2hip_pool_out_dims", "n2d2hip_pool_forward", "n2d2hip_pool_writes_halo", "n2d2hip_pool_forward_mapped",
     "n2d2hip_elemwise_create", "n2d2hip_elemwise_destroy", "n2d2hip_elemwise_forward", "n2d2hip_elemwise_fold_input_scaling", "n2d2hip_concat_channels",
-    "n2d2hip_quantizer_workspace_bytes", "n2d2hip_sat_weight_forward", "n2d2hip_sat_weight_forward_static", "n2d2hip_sat_weight_backward",
+    "n2d2hip_quantizer_workspace_bytes", "n2d2hip_sat_weight_forward_batch", "n2d2hip_sat_weight_backward_batch",
+    "n2d2hip_sat_weight_forward", "n2d2hip_sat_weight_forward_static", "n2d2hip_sat_weight_backward",
     "n2d2hip_sat_act_forward", "n2d2hip_sat_act_backward", "n2d2hip_lsq_forward", "n2d2hip_lsq_backward",
     "n2d2hip_conv2d_f32_forward", "n2d2hip_conv2d_f32_backward_data", "n2d2hip_conv2d_f32_backward_filter", "n2d2hip_conv2d_f32_workspace_bytes",
     "n2d2hip_conv2d_f32_backward_bias", "n2d2hip_softmax_f32_forward", "n2d2hip_loss_workspace_bytes", "n2d2hip_loss_f32",
@@ -63,6 +64,16 @@ class Activation(C.Structure):
 class SgdItem(C.Structure):
     _fields_ = [("data", C.c_void_p), ("diff", C.c_void_p), ("n", C.c_size_t), ("momentum_data", C.c_void_p), ("rate_diff", C.c_float),
                 ("momentum", C.c_float), ("decay_times_rate", C.c_float), ("clamp_min", C.c_float), ("clamp_max", C.c_float), ("clamp", C.c_int)]
+
+
+class SatWeightItem(C.Structure):
+    _fields_ = [("w", C.c_void_p), ("wq", C.c_void_p), ("n", C.c_size_t), ("range", C.c_float), ("mode", C.c_int), ("apply_scaling", C.c_int),
+                ("outputs_size", C.c_uint), ("stats", C.c_void_p), ("workspace", C.c_void_p), ("workspace_bytes", C.c_size_t)]
+
+
+class SatWeightGradItem(C.Structure):
+    _fields_ = [("diff_wq", C.c_void_p), ("w", C.c_void_p), ("diff_w", C.c_void_p), ("n", C.c_size_t), ("range", C.c_float), ("mode", C.c_int),
+                ("apply_scaling", C.c_int), ("stats", C.c_void_p)]
 
 
 class ConvDesc(C.Structure):
@@ -150,6 +161,8 @@ def load():
     lib.n2d2hip_elemwise_destroy.argtypes = [P]
     lib.n2d2hip_elemwise_fold_input_scaling.argtypes = [P, I, P]
     lib.n2d2hip_elemwise_forward.argtypes = [P, P, P, P]
+    lib.n2d2hip_sat_weight_forward_batch.argtypes = [C.POINTER(SatWeightItem), I, P]
+    lib.n2d2hip_sat_weight_backward_batch.argtypes = [C.POINTER(SatWeightGradItem), I, P]
     lib.n2d2hip_sat_weight_forward.argtypes = [P, P, SZ, F, I, I, U, P, P, SZ, P]
     lib.n2d2hip_sat_weight_forward_static.argtypes = [P, P, SZ, F, I, I, U, P, P]
     lib.n2d2hip_sat_weight_backward.argtypes = [P, P, P, SZ, F, I, I, P, P]

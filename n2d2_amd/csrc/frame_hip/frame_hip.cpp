@@ -1410,9 +1410,68 @@ static void ensureWorkspace(void*& ws, size_t& bytes, size_t n)
     bytes = need;
 }
 
+static thread_local SATWeightsScope* satScope = nullptr;
+
+SATWeightsScope::SATWeightsScope() : mOuter(satScope == nullptr), mStream(nullptr)
+{
+    if (mOuter) satScope = this;
+}
+
+SATWeightsScope::~SATWeightsScope()
+{
+    if (!mOuter) return;
+    satScope = nullptr;
+    // (left by an exception: what came before it is still done; its own error is the one to report)
+    launch(mItems, mGrads, false);
+}
+
+void SATWeightsScope::launch(const std::vector<n2d2hip_sat_weight_item>& items, const std::vector<n2d2hip_sat_weight_grad_item>& grads, bool throws)
+{
+    const int rc = items.empty() ? N2D2HIP_OK : n2d2hip_sat_weight_forward_batch(items.data(), (int)items.size(), mStream);
+    if (throws) checkStatus(rc);
+    const int rcGrads = grads.empty() ? N2D2HIP_OK : n2d2hip_sat_weight_backward_batch(grads.data(), (int)grads.size(), mStream);
+    if (throws) checkStatus(rcGrads);
+}
+
+void SATWeightsScope::flush()
+{
+    if (!mOuter && satScope) satScope->flush();
+    std::vector<n2d2hip_sat_weight_item> items;
+    std::vector<n2d2hip_sat_weight_grad_item> grads;
+    items.swap(mItems);
+    grads.swap(mGrads);
+    launch(items, grads, true);
+}
+
+SATWeightsScope* SATWeightsScope::current() { return satScope; }
+
+void SATWeightsScope::add(const n2d2hip_sat_weight_item& item, void* stream)
+{
+    // (a gradient reads what its forward pass has left; a tensor's second pass is a launch of its own)
+    bool apart = stream != mStream || !mGrads.empty();
+    for (const n2d2hip_sat_weight_item& i : mItems)
+        apart = apart || i.wq == item.wq || i.stats == item.stats || i.workspace == item.workspace;
+    if (apart) flush();
+    mStream = stream;
+    mItems.push_back(item);
+}
+
+void SATWeightsScope::add(const n2d2hip_sat_weight_grad_item& item, void* stream)
+{
+    bool apart = stream != mStream;
+    for (const n2d2hip_sat_weight_grad_item& i : mGrads)
+        apart = apart || i.diff_w == item.diff_w;
+    if (apart) flush();
+    mStream = stream;
+    mGrads.push_back(item);
+}
+
 template <class T>
 SATQuantizerCell_Frame_HIP<T>::~SATQuantizerCell_Frame_HIP()
 {
+    if (SATWeightsScope::current()) {
+        try { SATWeightsScope::current()->flush(); } catch (const std::exception&) {}
+    }
     for (auto& b : mW) { (void)hipFree(b.q); (void)hipFree(b.diffFp); }
     if (mStats) (void)hipFree(mStats);
     if (mWorkspace) (void)hipFree(mWorkspace);
@@ -1452,10 +1511,24 @@ void SATQuantizerCell_Frame_HIP<T>::propagate()
 {
     if (!mStats && !mW.empty())
         mStats = deviceFloats(2 * mW.size(), "SATQuantizerCell_Frame_HIP::propagate()");
+    SATWeightsScope* const scope = SATWeightsScope::current();
+    // (a part of the workspace for each tensor: the tensors of a scope are quantized together)
+    size_t each = 0;
+    for (size_t k = 0; k < mW.size(); ++k)
+        each = std::max(each, (n2d2hip_quantizer_workspace_bytes(mW[k].size) + 255) / 256 * 256);
+    if (each * mW.size() > mWorkspaceBytes) {
+        if (scope) scope->flush();
+        if (mWorkspace) (void)hipFree(mWorkspace);
+        mWorkspace = nullptr;
+        mWorkspaceBytes = 0;
+        checkHip(hipMalloc(&mWorkspace, each * mW.size()), "quantizer workspace");
+        mWorkspaceBytes = each * mW.size();
+    }
     for (size_t k = 0; k < mW.size(); ++k) {
-        ensureWorkspace(mWorkspace, mWorkspaceBytes, mW[k].size);
-        checkStatus(n2d2hip_sat_weight_forward(mW[k].fp, mW[k].q, mW[k].size, (float)mRange, satMode(), mApplyScaling ? 1 : 0,
-                                               (unsigned)mOutputsSize, mStats + 2 * k, mWorkspace, mWorkspaceBytes, mStream));
+        const n2d2hip_sat_weight_item item = {mW[k].fp, mW[k].q, mW[k].size, (float)mRange, satMode(), mApplyScaling ? 1 : 0, (unsigned)mOutputsSize,
+                                              mStats + 2 * k, (char*)mWorkspace + each * k, each};
+        if (scope) scope->add(item, mStream);
+        else checkStatus(n2d2hip_sat_weight_forward_batch(&item, 1, mStream));
     }
 }
 
@@ -1467,8 +1540,10 @@ void SATQuantizerCell_Frame_HIP<T>::back_propagate()
         int mode = N2D2HIP_SAT_DEFAULT;
         if (mQuantMode == QuantizerCell::Asymmetric) mode = N2D2HIP_SAT_ASYMRANGE;
         else if (mQuantMode == QuantizerCell::FullRange) mode = N2D2HIP_SAT_FULLRANGE;
-        checkStatus(n2d2hip_sat_weight_backward(mW[k].diffQ, mW[k].fp, mW[k].diffFp, mW[k].size, (float)mRange, mode, mApplyScaling ? 1 : 0,
-                                                mStats + 2 * k, mStream));
+        const n2d2hip_sat_weight_grad_item item = {mW[k].diffQ, mW[k].fp, mW[k].diffFp, mW[k].size, (float)mRange, mode, mApplyScaling ? 1 : 0,
+                                                   mStats + 2 * k};
+        if (SATWeightsScope* scope = SATWeightsScope::current()) scope->add(item, mStream);
+        else checkStatus(n2d2hip_sat_weight_backward_batch(&item, 1, mStream));
     }
 }
 

@@ -873,6 +873,28 @@ private:
     std::vector<n2d2hip_sgd_item> mItems;
 };
 
+// The same for the SAT quantizers of weights: while a scope lives, what the calling thread's propagate() and back_propagate()
+// would launch is gathered, up to 16 tensors a launch.  The quantized weights, and the gradients, are there after flush().
+class SATWeightsScope {
+public:
+    SATWeightsScope();
+    ~SATWeightsScope();
+    SATWeightsScope(const SATWeightsScope&) = delete;
+    SATWeightsScope& operator=(const SATWeightsScope&) = delete;
+    void flush();
+    // the calling thread's outermost scope, or null
+    static SATWeightsScope* current();
+    void add(const n2d2hip_sat_weight_item& item, void* stream);
+    void add(const n2d2hip_sat_weight_grad_item& item, void* stream);
+
+private:
+    void launch(const std::vector<n2d2hip_sat_weight_item>& items, const std::vector<n2d2hip_sat_weight_grad_item>& grads, bool throws);
+    bool mOuter;
+    void* mStream;
+    std::vector<n2d2hip_sat_weight_item> mItems;
+    std::vector<n2d2hip_sat_weight_grad_item> mGrads;
+};
+
 class SGDSolver {
 public:
     typedef std::function<std::shared_ptr<SGDSolver>()> RegistryCreate_T;

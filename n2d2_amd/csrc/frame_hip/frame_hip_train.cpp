@@ -185,7 +185,8 @@ double Cell_FrameTrain_HIP::readLoss() const
 
 // ------------------------------------------------ WeightedCell_FrameTrain_HIP
 WeightedCell_FrameTrain_HIP::WeightedCell_FrameTrain_HIP()
-    : mWeightsSolver(std::make_shared<SGDSolver_Frame_HIP<float> >()), mBiasSolver(std::make_shared<SGDSolver_Frame_HIP<float> >())
+    : mWeightsSolver(std::make_shared<SGDSolver_Frame_HIP<float> >()), mBiasSolver(std::make_shared<SGDSolver_Frame_HIP<float> >()),
+      mWeightsQuantized(false)
 {
 }
 
@@ -210,10 +211,18 @@ void WeightedCell_FrameTrain_HIP::initializeWeights(const Tensor<Float_T>& weigh
     }
 }
 
-void WeightedCell_FrameTrain_HIP::propagateWeighted(bool inference, bool noBias)
+void WeightedCell_FrameTrain_HIP::quantizeWeights()
 {
     if (mQuantizer)
         mQuantizer->propagate();
+    mWeightsQuantized = true;
+}
+
+void WeightedCell_FrameTrain_HIP::propagateWeighted(bool inference, bool noBias)
+{
+    if (mQuantizer && !mWeightsQuantized)
+        mQuantizer->propagate();
+    mWeightsQuantized = false;
     const n2d2hip_conv_desc d = desc();
     const float* w = mQuantizer ? mQuantizer->getQuantizedWeights(0) : mDevW.data();
     const size_t need = n2d2hip_conv2d_f32_workspace_bytes(&d, (int)mIn->dimB(), (int)mInH, (int)mInW);

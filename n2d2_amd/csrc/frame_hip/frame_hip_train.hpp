@@ -57,6 +57,10 @@ public:
     virtual void addInput(DeviceFloats& inputs, DeviceFloats& diffOutputs);
     virtual void initialize() = 0;
     virtual void propagate(bool inference = false) = 0;
+    // The part of the next propagate() that needs no inputs: its weights' quantizer.  A net does it for all cells at once
+    // (SATWeightsScope); forgetQuantizedWeights() before the weights may change.
+    virtual void quantizeWeights() {}
+    virtual void forgetQuantizedWeights() {}
     virtual void backPropagate() = 0;
     virtual void update() = 0;
     DeviceFloats& getOutputs() { return mOutputs; }
@@ -111,6 +115,8 @@ public:
     QATCellParameters getQATCellParameters();
     // refreshes the host tensors getWeights() / getBiases() return from the device
     virtual void synchronizeWeightsToHost() = 0;
+    void quantizeWeights();
+    void forgetQuantizedWeights() { mWeightsQuantized = false; }
     // the device's weights, without the host tensors
     void readWeights(float* host, size_t n) const { mDevW.toHost(host, n); }
 
@@ -126,6 +132,7 @@ protected:
     std::shared_ptr<SGDSolver> mWeightsSolver, mBiasSolver;
     DeviceFloats mDevW, mDevDiffW, mDevBias, mDevDiffBias;
     DeviceFloats mWorkspace;        // partial sums of the convolution passes
+    bool mWeightsQuantized;         // by quantizeWeights(), for the next propagate()
 };
 
 // src/Cell/ConvCell_Frame.cpp:418-597 for one input tensor.

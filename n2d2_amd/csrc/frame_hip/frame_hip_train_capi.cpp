@@ -89,6 +89,24 @@ void connect(TrainNet& n, const std::shared_ptr<Cell_FrameTrain_HIP>& cell)
     n.cells.push_back(cell);
 }
 
+// The weights of all cells quantized for the propagation that follows, however that ends
+struct QuantizedWeights {
+    explicit QuantizedWeights(TrainNet& net) : n(net)
+    {
+        try {
+            SATWeightsScope weights;
+            for (auto& c : n.cells) c->quantizeWeights();
+            weights.flush();
+        } catch (...) {
+            forget();
+            throw;
+        }
+    }
+    ~QuantizedWeights() { forget(); }
+    void forget() { for (auto& c : n.cells) c->forgetQuantizedWeights(); }
+    TrainNet& n;
+};
+
 Cell_FrameTrain_HIP* find(TrainNet& n, const char* name)
 {
     for (auto& c : n.cells)
@@ -378,9 +396,16 @@ int fh_train_learn(void* net, const float* targets, size_t nTargets, int iterati
                     n.inputDiff.setValid();
                 }
             }
-            for (auto& c : n.cells) c->propagate(false);
+            {
+                QuantizedWeights quantized(n);   // (all cells' in one launch or two)
+                for (auto& c : n.cells) c->propagate(false);
+            }
             last->launchLoss(n.targets.data());
-            for (auto c = n.cells.rbegin(); c != n.cells.rend(); ++c) (*c)->backPropagate();
+            {
+                SATWeightsScope gradients;
+                for (auto c = n.cells.rbegin(); c != n.cells.rend(); ++c) (*c)->backPropagate();
+                gradients.flush();
+            }
             SGDUpdateScope updates;              // (all tensors of the net in one launch)
             for (auto c = n.cells.rbegin(); c != n.cells.rend(); ++c) (*c)->update();
             updates.flush();

@@ -84,22 +84,6 @@ __device__ __forceinline__ void quad_store(float* p, size_t i, const float* v)
 
 // ------------------------------------------------------------ SAT weights
 
-__global__ __launch_bounds__(QBLOCK) void sat_absmax_partial(const float* __restrict__ w, size_t n, float* __restrict__ partial)
-{
-    float m = 0.0f;
-    for (size_t i = (size_t)blockIdx.x * QBLOCK + threadIdx.x; i < n; i += (size_t)gridDim.x * QBLOCK)
-        m = fmaxf(m, fabsf(tanhf(w[i])));
-    m = block_max(m);
-    if (threadIdx.x == 0) partial[blockIdx.x] = m;
-}
-__global__ __launch_bounds__(QBLOCK) void sat_absmax_final(const float* __restrict__ partial, int count, float* __restrict__ stats)
-{
-    float m = 0.0f;
-    for (int i = threadIdx.x; i < count; i += QBLOCK) m = fmaxf(m, partial[i]);
-    m = block_max(m);
-    if (threadIdx.x == 0) { stats[0] = m; stats[1] = 1.0f; }
-}
-
 // The weights' quantization levels from tanh(w), ref: src/Quantizer/QAT/Kernel/SATQuantizer_Frame_Kernels.cpp:66-238
 struct SatLevels {
     int mode;
@@ -142,23 +126,31 @@ struct SatLevels {
         }
     }
 };
-__global__ __launch_bounds__(QBLOCK) void sat_weight_quantize(const float* __restrict__ w, float* __restrict__ wq, size_t n,
-                                                              float range, int mode, const float* __restrict__ stats)
-{
-    const SatLevels level(range, mode, stats[0]);
-    for (size_t i = (size_t)blockIdx.x * QBLOCK + threadIdx.x; i < n; i += (size_t)gridDim.x * QBLOCK)
-        wq[i] = level(tanhf(w[i]));
-}
+// SAT weights of several tensors, in two launches at most: a learning net quantizes the weights of all its cells before a pass,
+// most of them few, and a launch each (three for many weights) was what bounded them.  16 tensors fit a launch's arguments.
+//  * Up to 16384 weights: one block computes the tensor, in the first launch.  Its tanh stay in registers (they were computed
+//    twice, and each pass went through memory): up to 1024 weights 3.7 us, 2400 4.2 and 10080, scaling included, 11.5; the blocks
+//    of several tensors run side by side.  (Instances by the weights per thread: skipping unused ones inside one instance
+//    made the compiler spill.)
+//  * More: the first launch leaves each block's max |tanh w|, and every block of the second one takes the maximum of those,
+//    at most 256, itself, instead of a launch of one block in between (48120 weights: 3 launches of 2.8, 1.8 and 2.4 us).
+constexpr int SAT_SMALL = 16;                    // weights per thread of a block of 1024 at most
+constexpr int SAT_BLOCKS = 256;                  // blocks of a larger tensor's first launch at most
+constexpr int SAT_ITEMS = 16;
+template <int N>
+struct SatBatch {
+    n2d2hip_sat_weight_item item[N];
+    unsigned first[N + 1], first2[N + 1];        // first block of a tensor in the first and the second launch
+    int count;
+};
+__host__ __device__ inline bool sat_small(size_t n) { return n <= (size_t)SAT_SMALL * 1024; }
 
-// Small tensors: the whole quantizer in one launch of one block, the weights in its registers.  One kernel per pass is bound
-// by the launches there (3 of 2 to 4 us, 8 with the scaling); one compute unit has done up to 1024 weights
-// in 3.7 us, 2400 in 4.2 and 10080, scaling included, in 11.5.  (Instances by the weights per thread: skipping unused ones
-// inside one instance made the compiler spill.)
-constexpr int SAT_SMALL = 16;                    // weights per thread at most; K: of this launch
 template <int K>
-__global__ __launch_bounds__(1024) void sat_weight_small_kernel(const float* __restrict__ w, float* __restrict__ wq, int n, float range, int mode,
-                                                                int apply_scaling, unsigned factor, float* __restrict__ stats)
+__device__ __forceinline__ void sat_weight_small(const n2d2hip_sat_weight_item& t)
 {
+    const float* __restrict__ w = t.w;
+    float* __restrict__ wq = t.wq;
+    const int n = (int)t.n;
     float v[K];
     float m = 0.0f;
 #pragma unroll
@@ -168,7 +160,7 @@ __global__ __launch_bounds__(1024) void sat_weight_small_kernel(const float* __r
         m = fmaxf(m, fabsf(v[k]));
     }
     m = block_max(m);
-    const SatLevels level(range, mode, m);
+    const SatLevels level(t.range, t.mode, m);
     double sum = 0.0;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -176,23 +168,57 @@ __global__ __launch_bounds__(1024) void sat_weight_small_kernel(const float* __r
         if (k * 1024 + (int)threadIdx.x < n) sum += (double)v[k];
     }
     float scaling = 1.0f;
-    if (apply_scaling) {                         // (the formulas of mean_final, sqdev_partial and sat_scaling_final)
+    if (t.apply_scaling) {                       // (the formulas of mean_final, sqdev_partial and sat_scaling_final)
         const float mean = (float)block_sum(sum) / (float)n;
         double squares = 0.0;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-                const float d = __fsub_rn(v[k], mean);
+            const float d = __fsub_rn(v[k], mean);
             if (k * 1024 + (int)threadIdx.x < n) squares += (double)__fmul_rn(d, d);
         }
         const float var = (float)block_sum(squares) / ((float)n - 1.0f);
-        scaling = sqrtf(var * (float)factor);
+        scaling = sqrtf(var * (float)t.outputs_size);
     }
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const int i = k * 1024 + threadIdx.x;
-        if (i < n) wq[i] = apply_scaling ? v[k] / scaling : v[k];
+        if (i < n) wq[i] = t.apply_scaling ? v[k] / scaling : v[k];
     }
-    if (threadIdx.x == 0) { stats[0] = m; stats[1] = scaling; }
+    if (threadIdx.x == 0) { t.stats[0] = m; t.stats[1] = scaling; }
+}
+template <int N>
+__global__ __launch_bounds__(1024) void sat_weight_first_kernel(const SatBatch<N> b)
+{
+    int k = 0;
+    if (N > 1)
+        while (k + 1 < b.count && blockIdx.x >= b.first[k + 1]) ++k;
+    const n2d2hip_sat_weight_item& t = b.item[k];
+    if (t.n <= 1024) sat_weight_small<1>(t);
+    else if (t.n <= 4 * 1024) sat_weight_small<4>(t);
+    else if (sat_small(t.n)) sat_weight_small<SAT_SMALL>(t);
+    else {
+        float m = 0.0f;
+        for (size_t i = (size_t)(blockIdx.x - b.first[k]) * 1024 + threadIdx.x; i < t.n; i += (size_t)(b.first[k + 1] - b.first[k]) * 1024)
+            m = fmaxf(m, fabsf(tanhf(t.w[i])));
+        m = block_max(m);
+        if (threadIdx.x == 0) ((float*)t.workspace)[blockIdx.x - b.first[k]] = m;
+    }
+}
+template <int N>
+__global__ __launch_bounds__(QBLOCK) void sat_weight_second_kernel(const SatBatch<N> b)
+{
+    int k = 0;
+    if (N > 1)
+        while (k + 1 < b.count && blockIdx.x >= b.first2[k + 1]) ++k;
+    const n2d2hip_sat_weight_item& t = b.item[k];
+    const float* __restrict__ w = t.w;
+    float* __restrict__ wq = t.wq;
+    static_assert(SAT_BLOCKS <= QBLOCK, "a thread takes one block's maximum");
+    const float m = block_max(threadIdx.x < b.first[k + 1] - b.first[k] ? ((const float*)t.workspace)[threadIdx.x] : 0.0f);
+    const SatLevels level(t.range, t.mode, m);
+    for (size_t i = (size_t)(blockIdx.x - b.first2[k]) * QBLOCK + threadIdx.x; i < t.n; i += (size_t)(b.first2[k + 1] - b.first2[k]) * QBLOCK)
+        wq[i] = level(tanhf(w[i]));
+    if (blockIdx.x == b.first2[k] && threadIdx.x == 0) { t.stats[0] = m; t.stats[1] = 1.0f; }
 }
 
 // SAT scaling, ref: SATQuantizer_Frame_Kernels.cpp:244-262: mean, unbiased variance about that
@@ -243,16 +269,30 @@ __global__ __launch_bounds__(QBLOCK) void divide_by_stat(float* __restrict__ x, 
 }
 
 // ref: SATQuantizer_Frame_Kernels.cpp:349-404
-__global__ __launch_bounds__(QBLOCK) void sat_weight_backward_kernel(const float* __restrict__ dq, const float* __restrict__ w,
-                                                                     float* __restrict__ dw, size_t n, float mode_factor, int use_mode_factor,
-                                                                     int apply_scaling, const float* __restrict__ stats)
+template <int N>
+struct SatGradBatch {
+    n2d2hip_sat_weight_grad_item item[N];
+    float mode_factor[N];                        // slope of the quantizer's line, 0: none
+    unsigned first[N + 1];
+    int count;
+};
+template <int N>
+__global__ __launch_bounds__(QBLOCK) void sat_weight_backward_kernel(const SatGradBatch<N> b)
 {
-    const float factor = apply_scaling ? __fmul_rn(stats[0], stats[1]) : stats[0];
+    int k = 0;
+    if (N > 1)
+        while (k + 1 < b.count && blockIdx.x >= b.first[k + 1]) ++k;
+    const n2d2hip_sat_weight_grad_item& t = b.item[k];
+    const float* __restrict__ dq = t.diff_wq;
+    const float* __restrict__ w = t.w;
+    float* __restrict__ dw = t.diff_w;
+    const float mode_factor = b.mode_factor[k];
+    const float factor = t.apply_scaling ? __fmul_rn(t.stats[0], t.stats[1]) : t.stats[0];
     const float inv_factor = 1.0f / factor;
-    for (size_t i = (size_t)blockIdx.x * QBLOCK + threadIdx.x; i < n; i += (size_t)gridDim.x * QBLOCK) {
+    for (size_t i = (size_t)(blockIdx.x - b.first[k]) * QBLOCK + threadIdx.x; i < t.n; i += (size_t)(b.first[k + 1] - b.first[k]) * QBLOCK) {
         const float inv_cosh = 1.0f / coshf(w[i]);
         float grad = __fmul_rn(__fmul_rn(inv_cosh, inv_cosh), inv_factor);
-        if (use_mode_factor)
+        if (mode_factor != 0.0f)
             grad = __fmul_rn(grad, mode_factor);
         dw[i] = __fmul_rn(dq[i], grad);
     }
@@ -417,39 +457,83 @@ int static_scratch(void** ptr)
 }
 } // namespace
 
+// The launches of up to SAT_ITEMS tensors' SAT weight quantizers, each over a workspace of n2d2hip_quantizer_workspace_bytes().
+template <int N>
+static void sat_weight_launch(const n2d2hip_sat_weight_item* items, int count, hipStream_t st)
+{
+    SatBatch<N> b = {};
+    b.count = count;
+    for (int i = 0; i < count; ++i) {
+        const size_t n = items[i].n;
+        b.item[i] = items[i];
+        b.first[i + 1] = b.first[i] + (sat_small(n) ? 1u : (unsigned)std::min<size_t>((n + 1023) / 1024, SAT_BLOCKS));
+        b.first2[i + 1] = b.first2[i] + (sat_small(n) ? 0u : (unsigned)blocks_for(n));
+    }
+    hipLaunchKernelGGL(sat_weight_first_kernel<N>, dim3(b.first[count]), dim3(1024), 0, st, b);
+    if (b.first2[count])
+        hipLaunchKernelGGL(sat_weight_second_kernel<N>, dim3(b.first2[count]), dim3(QBLOCK), 0, st, b);
+    for (int i = 0; i < count; ++i) {
+        const n2d2hip_sat_weight_item& t = items[i];
+        if (!t.apply_scaling || sat_small(t.n))
+            continue;
+        const int nb = blocks_for(t.n);
+        double* partial = (double*)t.workspace;
+        float* mean = (float*)((char*)t.workspace + (size_t)PARTIALS * sizeof(double));
+        hipLaunchKernelGGL(sum_partial, dim3(nb), dim3(QBLOCK), 0, st, (const float*)t.wq, t.n, partial);
+        hipLaunchKernelGGL(mean_final, dim3(1), dim3(QBLOCK), 0, st, (const double*)partial, nb, t.n, mean);
+        hipLaunchKernelGGL(sqdev_partial, dim3(nb), dim3(QBLOCK), 0, st, (const float*)t.wq, t.n, (const float*)mean, partial);
+        hipLaunchKernelGGL(sat_scaling_final, dim3(1), dim3(QBLOCK), 0, st, (const double*)partial, nb, t.n, t.outputs_size, t.stats);
+        hipLaunchKernelGGL(divide_by_stat, dim3(ew_grid(t.n)), dim3(QBLOCK), 0, st, t.wq, t.n, (const float*)(t.stats + 1));
+    }
+}
+
+template <int N>
+static void sat_weight_backward_launch(const n2d2hip_sat_weight_grad_item* items, int count, hipStream_t st)
+{
+    SatGradBatch<N> b = {};
+    b.count = count;
+    for (int i = 0; i < count; ++i) {
+        const n2d2hip_sat_weight_grad_item& t = items[i];
+        b.item[i] = t;
+        b.first[i + 1] = b.first[i] + ew_grid(t.n);
+        // ref: SATQuantizerCell_Frame.cpp:249-283: Asymmetric and FullRange have their own slope factor
+        if (t.mode == N2D2HIP_SAT_FULLRANGE) b.mode_factor[i] = 1.0f + 0.9998f / t.range;
+        else if (t.mode == N2D2HIP_SAT_ASYMRANGE || t.mode == N2D2HIP_SAT_NONE_ASYM) { const float r2 = floorf(t.range / 2.0f); b.mode_factor[i] = 1.0f + 1.0f / (2.0f * r2); }
+    }
+    hipLaunchKernelGGL(sat_weight_backward_kernel<N>, dim3(b.first[count]), dim3(QBLOCK), 0, st, b);
+}
+
 extern "C" {
 
 size_t n2d2hip_quantizer_workspace_bytes(size_t) { return (size_t)PARTIALS * sizeof(double) + 256; }
 
-// The kernel sequence of the SAT weight quantizer over a workspace of n2d2hip_quantizer_workspace_bytes() bytes.
-static int sat_weight_forward_impl(const char* who, const float* w, float* wq, size_t n, float range, int mode, int apply_scaling,
-                                   unsigned outputs_size, float* stats, void* workspace, hipStream_t st)
+static int sat_weight_forward_impl(const char* who, const n2d2hip_sat_weight_item* items, int count, hipStream_t st)
 {
-    N2D2HIP_REQUIRE(n > 0, N2D2HIP_ERR_INVALID, "%s: empty tensor", who);
-    N2D2HIP_REQUIRE(mode >= N2D2HIP_SAT_NONE && mode <= N2D2HIP_SAT_NONE_ASYM, N2D2HIP_ERR_INVALID, "%s: bad mode %d", who, mode);
-    N2D2HIP_REQUIRE(range >= 1.0f, N2D2HIP_ERR_INVALID, "%s: range %g", who, (double)range);
-    N2D2HIP_REQUIRE(!apply_scaling || n > 1, N2D2HIP_ERR_INVALID, "%s: SAT scaling needs more than one weight", who);
-    if (n <= (size_t)SAT_SMALL * 1024) {
-        const auto kernel = n <= 1024 ? sat_weight_small_kernel<1> : n <= 4 * 1024 ? sat_weight_small_kernel<4> : sat_weight_small_kernel<SAT_SMALL>;
-        hipLaunchKernelGGL(kernel, dim3(1), dim3(1024), 0, st, w, wq, (int)n, range, mode, apply_scaling, outputs_size, stats);
-        N2D2HIP_HIP_CHECK(hipGetLastError());
-        return N2D2HIP_OK;
+    for (int i = 0; i < count; ++i) {
+        const n2d2hip_sat_weight_item& t = items[i];
+        N2D2HIP_REQUIRE(t.n > 0, N2D2HIP_ERR_INVALID, "%s: empty tensor", who);
+        N2D2HIP_REQUIRE(t.mode >= N2D2HIP_SAT_NONE && t.mode <= N2D2HIP_SAT_NONE_ASYM, N2D2HIP_ERR_INVALID, "%s: bad mode %d", who, t.mode);
+        N2D2HIP_REQUIRE(t.range >= 1.0f, N2D2HIP_ERR_INVALID, "%s: range %g", who, (double)t.range);
+        N2D2HIP_REQUIRE(!t.apply_scaling || t.n > 1, N2D2HIP_ERR_INVALID, "%s: SAT scaling needs more than one weight", who);
     }
-    const int nb = blocks_for(n);
-    double* partial = (double*)workspace;
-    float* mean = (float*)((char*)workspace + (size_t)PARTIALS * sizeof(double));
-    hipLaunchKernelGGL(sat_absmax_partial, dim3(nb), dim3(QBLOCK), 0, st, w, n, (float*)partial);
-    hipLaunchKernelGGL(sat_absmax_final, dim3(1), dim3(QBLOCK), 0, st, (const float*)partial, nb, stats);
-    hipLaunchKernelGGL(sat_weight_quantize, dim3(ew_grid(n)), dim3(QBLOCK), 0, st, w, wq, n, range, mode, (const float*)stats);
-    if (apply_scaling) {
-        hipLaunchKernelGGL(sum_partial, dim3(nb), dim3(QBLOCK), 0, st, (const float*)wq, n, partial);
-        hipLaunchKernelGGL(mean_final, dim3(1), dim3(QBLOCK), 0, st, (const double*)partial, nb, n, mean);
-        hipLaunchKernelGGL(sqdev_partial, dim3(nb), dim3(QBLOCK), 0, st, (const float*)wq, n, (const float*)mean, partial);
-        hipLaunchKernelGGL(sat_scaling_final, dim3(1), dim3(QBLOCK), 0, st, (const double*)partial, nb, n, outputs_size, stats);
-        hipLaunchKernelGGL(divide_by_stat, dim3(ew_grid(n)), dim3(QBLOCK), 0, st, wq, n, (const float*)(stats + 1));
+    for (int i = 0; i < count; i += SAT_ITEMS) {
+        const int nb = std::min(count - i, SAT_ITEMS);
+        if (nb == 1) sat_weight_launch<1>(items + i, nb, st);
+        else sat_weight_launch<SAT_ITEMS>(items + i, nb, st);
     }
     N2D2HIP_HIP_CHECK(hipGetLastError());
     return N2D2HIP_OK;
+}
+
+int n2d2hip_sat_weight_forward_batch(const n2d2hip_sat_weight_item* items, int count, n2d2hip_stream_t stream_)
+{
+    N2D2HIP_REQUIRE(items && count > 0, N2D2HIP_ERR_INVALID, "sat_weight_forward_batch: bad argument");
+    for (int i = 0; i < count; ++i) {
+        N2D2HIP_REQUIRE(items[i].w && items[i].wq && items[i].stats && items[i].workspace, N2D2HIP_ERR_INVALID, "sat_weight_forward_batch: null argument");
+        N2D2HIP_REQUIRE(items[i].workspace_bytes >= n2d2hip_quantizer_workspace_bytes(items[i].n), N2D2HIP_ERR_WORKSPACE,
+                        "sat_weight_forward_batch: workspace of %zu bytes needed", n2d2hip_quantizer_workspace_bytes(items[i].n));
+    }
+    return sat_weight_forward_impl("sat_weight_forward_batch", items, count, (hipStream_t)stream_);
 }
 
 int n2d2hip_sat_weight_forward(const float* w, float* wq, size_t n, float range, int mode, int apply_scaling,
@@ -458,7 +542,8 @@ int n2d2hip_sat_weight_forward(const float* w, float* wq, size_t n, float range,
     N2D2HIP_REQUIRE(w && wq && stats && workspace, N2D2HIP_ERR_INVALID, "sat_weight_forward: null argument");
     N2D2HIP_REQUIRE(workspace_bytes >= n2d2hip_quantizer_workspace_bytes(n), N2D2HIP_ERR_WORKSPACE, "sat_weight_forward: workspace of %zu bytes needed",
                     n2d2hip_quantizer_workspace_bytes(n));
-    return sat_weight_forward_impl("sat_weight_forward", w, wq, n, range, mode, apply_scaling, outputs_size, stats, workspace, (hipStream_t)stream_);
+    const n2d2hip_sat_weight_item item = {w, wq, n, range, mode, apply_scaling, outputs_size, stats, workspace, workspace_bytes};
+    return sat_weight_forward_impl("sat_weight_forward", &item, 1, (hipStream_t)stream_);
 }
 
 int n2d2hip_sat_weight_forward_static(const float* w, float* wq, size_t n, float range, int mode, int apply_scaling,
@@ -475,24 +560,33 @@ int n2d2hip_sat_weight_forward_static(const float* w, float* wq, size_t n, float
         return rc;
     // Nothing in the scratch has to start from zero: every pass writes the partials it then reads (the same block count
     // both times), and the mean is written before it is read.
-    return sat_weight_forward_impl("sat_weight_forward_static", w, wq, n, range, mode, apply_scaling, outputs_size, stats, ws, (hipStream_t)stream_);
+    const n2d2hip_sat_weight_item item = {w, wq, n, range, mode, apply_scaling, outputs_size, stats, ws, STATIC_SCRATCH_BYTES};
+    return sat_weight_forward_impl("sat_weight_forward_static", &item, 1, (hipStream_t)stream_);
+}
+
+int n2d2hip_sat_weight_backward_batch(const n2d2hip_sat_weight_grad_item* items, int count, n2d2hip_stream_t stream_)
+{
+    N2D2HIP_REQUIRE(items && count > 0, N2D2HIP_ERR_INVALID, "sat_weight_backward: bad argument");
+    for (int i = 0; i < count; ++i) {
+        const n2d2hip_sat_weight_grad_item& t = items[i];
+        N2D2HIP_REQUIRE(t.diff_wq && t.w && t.diff_w && t.stats, N2D2HIP_ERR_INVALID, "sat_weight_backward: null argument");
+        N2D2HIP_REQUIRE(t.n > 0, N2D2HIP_ERR_INVALID, "sat_weight_backward: empty tensor");
+        N2D2HIP_REQUIRE(t.mode >= N2D2HIP_SAT_NONE && t.mode <= N2D2HIP_SAT_NONE_ASYM, N2D2HIP_ERR_INVALID, "sat_weight_backward: bad mode %d", t.mode);
+    }
+    for (int i = 0; i < count; i += SAT_ITEMS) {
+        const int nb = std::min(count - i, SAT_ITEMS);
+        if (nb == 1) sat_weight_backward_launch<1>(items + i, nb, (hipStream_t)stream_);
+        else sat_weight_backward_launch<SAT_ITEMS>(items + i, nb, (hipStream_t)stream_);
+    }
+    N2D2HIP_HIP_CHECK(hipGetLastError());
+    return N2D2HIP_OK;
 }
 
 int n2d2hip_sat_weight_backward(const float* diff_wq, const float* w, float* diff_w, size_t n, float range, int mode,
                                 int apply_scaling, const float* stats, n2d2hip_stream_t stream_)
 {
-    N2D2HIP_REQUIRE(diff_wq && w && diff_w && stats, N2D2HIP_ERR_INVALID, "sat_weight_backward: null argument");
-    N2D2HIP_REQUIRE(n > 0, N2D2HIP_ERR_INVALID, "sat_weight_backward: empty tensor");
-    N2D2HIP_REQUIRE(mode >= N2D2HIP_SAT_NONE && mode <= N2D2HIP_SAT_NONE_ASYM, N2D2HIP_ERR_INVALID, "sat_weight_backward: bad mode %d", mode);
-    // ref: SATQuantizerCell_Frame.cpp:249-283: Asymmetric and FullRange have their own slope factor
-    float mf = 1.0f;
-    int use = 0;
-    if (mode == N2D2HIP_SAT_FULLRANGE) { mf = 1.0f + 0.9998f / range; use = 1; }
-    else if (mode == N2D2HIP_SAT_ASYMRANGE || mode == N2D2HIP_SAT_NONE_ASYM) { const float r2 = floorf(range / 2.0f); mf = 1.0f + 1.0f / (2.0f * r2); use = 1; }
-    hipLaunchKernelGGL(sat_weight_backward_kernel, dim3(ew_grid(n)), dim3(QBLOCK), 0, (hipStream_t)stream_, diff_wq, w, diff_w, n, mf, use,
-                       apply_scaling, stats);
-    N2D2HIP_HIP_CHECK(hipGetLastError());
-    return N2D2HIP_OK;
+    const n2d2hip_sat_weight_grad_item item = {diff_wq, w, diff_w, n, range, mode, apply_scaling, stats};
+    return n2d2hip_sat_weight_backward_batch(&item, 1, stream_);
 }
 
 int n2d2hip_sat_act_forward(float* x, float* fp_copy, size_t n, float range, const float* alpha, n2d2hip_stream_t stream_)
