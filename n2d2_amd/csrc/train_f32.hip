@@ -220,6 +220,53 @@ __global__ __launch_bounds__(64) void conv_f32_walk_kernel(ConvF32 q, WalkF32 k,
     out[idx] = r;
 }
 
+// Forward of a square kernel whose windows all lie inside the input (no padding), term for term the same sums again.  There is
+// nothing to mask, so a product takes its two loads, at scalar addresses with the lane's offset, a multiplication and an
+// addition (the walk above: about 14 instructions, which a wave alone on its SIMD issues one in 8 cycles), and the next
+// channel's window is requested before this one's is added up.  32 x 6 x 14 x 14 -> 16 channels, 5x5: 20.1 us, now 6.0;
+// 32 x 1 x 32 x 32 -> 6, 5x5: 8.6 and 4.0.
+template <int KS>
+__global__ __launch_bounds__(64) void conv_f32_window_kernel(ConvF32 q, WalkF32 k, const float* __restrict__ x, const float* __restrict__ w,
+                                                             const float* __restrict__ bias, float beta, float* __restrict__ out, int total)
+{
+    constexpr int T = KS * KS;
+    const int idx = blockIdx.x * 64 + threadIdx.x;
+    if (idx >= total) return;
+    const int img = div_f32(idx, k.dplane);      // image and channel
+    const int b = div_f32(img, k.dch), ch = img - b * q.O;
+    const int rem = idx - img * (q.oH * q.oW), py = div_f32(rem, k.dw), px = rem - py * q.oW;
+    const unsigned xb = 4u * (unsigned)((b * q.C + (q.depthwise ? ch : 0)) * (q.H * q.W) + py * q.sy * q.W + px * q.sx), wb = 4u * (unsigned)(ch * q.Cw * T);
+    struct Window { float x[T], w[T]; };
+    const auto request = [&](int c, Window& v) {
+        const char* const xc = (const char*)(x + (size_t)c * k.xo);
+        const char* const wc = (const char*)(w + (size_t)c * T);
+#pragma unroll
+        for (int i = 0; i < KS; ++i)
+#pragma unroll
+            for (int j = 0; j < KS; ++j) {
+                v.x[i * KS + j] = *(const float*)(xc + (size_t)i * q.W * 4 + 4 * j + xb);
+                v.w[i * KS + j] = *(const float*)(wc + 4 * (i * KS + j) + wb);
+            }
+    };
+    float sum = 0.0f;
+    const auto add = [&](const Window& v) {
+#pragma unroll
+        for (int t = 0; t < T; ++t) sum = sum + v.w[t] * v.x[t];
+    };
+    Window even, odd;
+    request(0, even);
+    for (int c = 0; c < k.n; c += 2) {
+        if (c + 1 < k.n) request(c + 1, odd);
+        add(even);
+        if (c + 1 >= k.n) break;
+        if (c + 2 < k.n) request(c + 2, even);
+        add(odd);
+    }
+    float r = sum + (beta != 0.0f ? beta * out[idx] : 0.0f);
+    if (bias) r = bias[ch] + r;
+    out[idx] = r;
+}
+
 // dw[o,c',ty,tx] = sum over batch and the output pixels whose tap (ty,tx) falls inside the input + beta * dw.
 // One block per weight.
 __global__ __launch_bounds__(TBLOCK) void conv_f32_backward_filter_kernel(ConvF32 q, const float* __restrict__ x, const float* __restrict__ dy,
@@ -883,7 +930,14 @@ static int run_direct(const ConvF32& q, int pass, const float* x, const float* w
     } else {
         k = {q.depthwise ? 1 : q.C, q.kH, q.kW, q.H * q.W, q.W, 1, T, q.kW, 1, div_of(q.oH * q.oW), div_of(q.oW), div_of(q.O)};
         const dim3 grid((unsigned)((total + 63) / 64));
-        if (q.kH != 3 || q.kW != 3) hipLaunchKernelGGL((conv_f32_walk_kernel<false, 0>), grid, dim3(64), 0, st, q, k, x, w, bias, beta, out, (int)total);
+        // (windows inside the input, byte offsets of 32 bits; kernels of 4 to 7, whose windows the registers hold twice)
+        const bool inside = q.pt == 0 && q.pl == 0 && (q.oH - 1) * q.sy + q.kH <= q.H && (q.oW - 1) * q.sx + q.kW <= q.W && source < lim / 2
+            && (size_t)q.O * q.Cw * T < lim / 2;
+        if (inside && q.kH == q.kW && q.kH >= 4 && q.kH <= 7) {
+            const auto kernel = q.kH == 4 ? conv_f32_window_kernel<4> : q.kH == 5 ? conv_f32_window_kernel<5> : q.kH == 6 ? conv_f32_window_kernel<6>
+                                                                                                                      : conv_f32_window_kernel<7>;
+            hipLaunchKernelGGL(kernel, grid, dim3(64), 0, st, q, k, x, w, bias, beta, out, (int)total);
+        } else if (q.kH != 3 || q.kW != 3) hipLaunchKernelGGL((conv_f32_walk_kernel<false, 0>), grid, dim3(64), 0, st, q, k, x, w, bias, beta, out, (int)total);
         else if (k.n == 1) hipLaunchKernelGGL((conv_f32_walk_kernel<false, 1>), grid, dim3(64), 0, st, q, k, x, w, bias, beta, out, (int)total);
         else hipLaunchKernelGGL((conv_f32_walk_kernel<false, 4>), grid, dim3(64), 0, st, q, k, x, w, bias, beta, out, (int)total);
     }
