@@ -563,6 +563,14 @@ int n2d2hip_batchnorm_f32_forward(int B, int C, int H, int W, const float* x, co
                                   float* mean, float* variance, float* saved_mean, float* saved_variance, double epsilon,
                                   double moving_average_momentum, int use_running, float* y, void* workspace,
                                   size_t workspace_bytes, n2d2hip_stream_t stream);
+/* The same with the SAT activation quantizer of n2d2hip_sat_act_forward() behind it: y receives the quantized values,
+ * full_precision (or NULL) the normalised ones, as n2d2hip_sat_act_forward(y, full_precision, ...) would leave them.
+ * full_precision is neither x nor y. */
+int n2d2hip_batchnorm_f32_forward_sat(int B, int C, int H, int W, const float* x, const float* scale, const float* bias,
+                                      float* mean, float* variance, float* saved_mean, float* saved_variance, double epsilon,
+                                      double moving_average_momentum, int use_running, float* y, float* full_precision,
+                                      float range, const float* alpha, void* workspace, size_t workspace_bytes,
+                                      n2d2hip_stream_t stream);
 /* Its backward, from the x and the saved statistics of the learning pass: diff_scale[c] = sum(diff_y * x_hat) +
  * beta_scale * diff_scale[c], diff_bias[c] = sum(diff_y) + beta_bias * diff_bias[c], the gradients of the saved mean and
  * variance ({C} each, always written), and, when diff_x != NULL, diff_x = diff_y * scale / sigma + dVar * 2 (x - m) / n

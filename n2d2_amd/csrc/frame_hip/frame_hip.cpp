@@ -1584,10 +1584,17 @@ void SATQuantizerActivation_Frame_HIP<T>::lazyInit(std::size_t size, bool needCo
 }
 
 template <class T>
-void SATQuantizerActivation_Frame_HIP<T>::propagate(float* inOut, std::size_t size, bool inference)
+typename SATQuantizerActivation_Frame_HIP<T>::Prepared SATQuantizerActivation_Frame_HIP<T>::prepare(std::size_t size, bool inference)
 {
     lazyInit(size, !inference);
-    checkStatus(n2d2hip_sat_act_forward(inOut, inference ? nullptr : mFp, size, (float)mRange, mDev, mStream));
+    return Prepared{inference ? nullptr : mFp, (float)mRange, mDev};
+}
+
+template <class T>
+void SATQuantizerActivation_Frame_HIP<T>::propagate(float* inOut, std::size_t size, bool inference)
+{
+    const Prepared to = prepare(size, inference);
+    checkStatus(n2d2hip_sat_act_forward(inOut, to.fullPrecision, size, to.range, to.alpha, mStream));
 }
 
 template <class T>

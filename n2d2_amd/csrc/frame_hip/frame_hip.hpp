@@ -1054,6 +1054,10 @@ public:
     float getAlpha();
     float getDiffAlpha();
     std::pair<float, float> getAlphaAndGradient();       // both in one copy from the device
+    // For a cell whose own last launch does what propagate(inOut, size, inference) would: where the full-precision copy goes
+    // (null in inference), the range and the device's alpha
+    struct Prepared { float* fullPrecision; float range; const float* alpha; };
+    Prepared prepare(std::size_t size, bool inference);
 
 private:
     void lazyInit(std::size_t size, bool needCopy);

@@ -137,6 +137,14 @@ void Cell_FrameTrain_HIP::activationPropagate(bool inference)
         mActivation->getQuantizer()->propagate(mOutputs.data(), mOutputs.size(), inference);
 }
 
+std::shared_ptr<SATQuantizerActivation_Frame_HIP<float> > Cell_FrameTrain_HIP::lonelySatQuantizer() const
+{
+    if (!mActivation || mActivation->abiKind() == N2D2HIP_ACT_RECTIFIER || mActivation->clipping() != 0.0
+        || mActivation->getActivationScaling().getMode() != ScalingMode::NONE)
+        return nullptr;
+    return std::dynamic_pointer_cast<SATQuantizerActivation_Frame_HIP<float> >(mActivation->getQuantizer());
+}
+
 void Cell_FrameTrain_HIP::activationBackPropagate()
 {
     if (!mActivation)
@@ -573,12 +581,24 @@ void BatchNormCell_FrameTrain_HIP<T>::initialize()
 template <class T>
 void BatchNormCell_FrameTrain_HIP<T>::propagate(bool inference)
 {
-    checkStatus(n2d2hip_batchnorm_f32_forward((int)mIn->dimB(), (int)mNbOutputs, (int)mInH, (int)mInW, mIn->data(), mScale.data(), mBias.data(),
-                                              mMean.data(), mVariance.data(), mSavedMean.data(), mSavedVariance.data(), mEpsilon, mMovingAverageMomentum,
-                                              inference ? 1 : 0, mOutputs.data(), mWorkspace.data(), mWorkspace.size() * sizeof(float), mStream));
+    // (a SAT quantizer alone behind the normalisation is applied as that leaves)
+    const std::shared_ptr<SATQuantizerActivation_Frame_HIP<float> > sat = lonelySatQuantizer();
+    if (sat) {
+        const auto to = sat->prepare(mOutputs.size(), inference);
+        checkStatus(n2d2hip_batchnorm_f32_forward_sat((int)mIn->dimB(), (int)mNbOutputs, (int)mInH, (int)mInW, mIn->data(), mScale.data(), mBias.data(),
+                                                      mMean.data(), mVariance.data(), mSavedMean.data(), mSavedVariance.data(), mEpsilon,
+                                                      mMovingAverageMomentum, inference ? 1 : 0, mOutputs.data(), to.fullPrecision, to.range, to.alpha,
+                                                      mWorkspace.data(), mWorkspace.size() * sizeof(float), mStream));
+    } else {
+        checkStatus(n2d2hip_batchnorm_f32_forward((int)mIn->dimB(), (int)mNbOutputs, (int)mInH, (int)mInW, mIn->data(), mScale.data(), mBias.data(),
+                                                  mMean.data(), mVariance.data(), mSavedMean.data(), mSavedVariance.data(), mEpsilon,
+                                                  mMovingAverageMomentum, inference ? 1 : 0, mOutputs.data(), mWorkspace.data(),
+                                                  mWorkspace.size() * sizeof(float), mStream));
+    }
     if (!inference && mMovingAverageMomentum != 0.0)
         mLearned = true;
-    activationPropagate(inference);
+    if (!sat)
+        activationPropagate(inference);
     mDiffInputs.clearValid();
     mDiffScale.clearValid();
     mDiffBias.clearValid();

@@ -88,6 +88,8 @@ protected:
     void activationPropagate(bool inference);
     void activationBackPropagate();
     void activationUpdate();
+    // the activation's SAT quantizer, if the activation does nothing else
+    std::shared_ptr<SATQuantizerActivation_Frame_HIP<float> > lonelySatQuantizer() const;
     DeviceFloats* mIn;
     DeviceFloats* mDiffOut;
     DeviceFloats mOutputs, mDiffInputs;

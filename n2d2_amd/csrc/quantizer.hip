@@ -10,6 +10,7 @@
 
 #include "common.h"
 #include "epilogue.hpp"
+#include "sat_math.hpp"
 
 namespace n2d2hip {
 
@@ -308,10 +309,7 @@ __global__ __launch_bounds__(QBLOCK) void sat_act_forward_kernel(float* __restri
     for (size_t i = (size_t)blockIdx.x * QBLOCK + threadIdx.x; i < n; i += (size_t)gridDim.x * QBLOCK) {
         const float v = x[i];
         if (fp) fp[i] = v;
-        const float xc = (v < 0.0f) ? 0.0f : (v < a) ? v : a;
-        float q = xc / a;
-        q = round_half_away(__fmul_rn(range, q)) / range;
-        x[i] = __fmul_rn(q, a);
+        x[i] = sat_quantize(v, range, a);
     }
 }
 

@@ -12,6 +12,7 @@
 
 #include "common.h"
 #include "conv_f32_gemm.hpp"
+#include "sat_math.hpp"
 #include "depthwise_f32.hpp"
 
 namespace n2d2hip {
@@ -464,13 +465,16 @@ __device__ __forceinline__ void bn_partial_sums(double* v, const double* __restr
 // beside the sum of x it adds x - s and its square in double, s being the channel's first value, and moves the squares from s to
 // the mean afterwards.  As s is one of the n values, (s - mean)^2 is at most n variances, so what cancels costs at most n times
 // 2^-53 of the variance.  64 channels, 56 x 56, batch 64: two passes and the last step 56.8 us, now 12.4 and 4.8.
-__device__ __forceinline__ void bn_finish_stats(int c, double n, float shift, const double* t, float* __restrict__ mean, float* __restrict__ variance,
-                                                float* __restrict__ saved_mean, float* __restrict__ saved_variance, double momentum)
+__device__ __forceinline__ void bn_stats(double n, float shift, const double* t, float* m, float* v)
 {
-    const float m = (float)(t[0] / n);
-    const double e = (double)m - (double)shift;
+    *m = (float)(t[0] / n);
+    const double e = (double)*m - (double)shift;
     const double squares = t[2] - 2.0 * e * t[1] + n * e * e;
-    const float v = (float)((squares < 0.0 ? 0.0 : squares) / n);
+    *v = (float)((squares < 0.0 ? 0.0 : squares) / n);
+}
+__device__ __forceinline__ void bn_write_stats(int c, double n, float m, float v, float* __restrict__ mean, float* __restrict__ variance,
+                                               float* __restrict__ saved_mean, float* __restrict__ saved_variance, double momentum)
+{
     saved_mean[c] = m;
     saved_variance[c] = v;
     const float unbiased = v * ((float)n / ((float)n - 1.0f));
@@ -501,89 +505,141 @@ __global__ __launch_bounds__(1024) void batchnorm_f32_stats_kernel(BnRange q, do
     bn_block_sums<3>(t);
     if (threadIdx.x) return;
     if (gridDim.y == 1) {
-        bn_finish_stats(c, n, shift, t, mean, variance, saved_mean, saved_variance, momentum);
+        float m, v;
+        bn_stats(n, shift, t, &m, &v);
+        bn_write_stats(c, n, m, v, mean, variance, saved_mean, saved_variance, momentum);
     } else {
-        double* o = ws + ((size_t)c * gridDim.y + blockIdx.y) * 3;
-        o[0] = t[0]; o[1] = t[1]; o[2] = t[2];
+        double* o = ws + ((size_t)c * gridDim.y + blockIdx.y) * 4;
+        o[0] = t[0]; o[1] = t[1]; o[2] = t[2]; o[3] = (double)shift;
     }
 }
-__global__ __launch_bounds__(64) void batchnorm_f32_stats_finish_kernel(int plane, double n, int splits, const float* __restrict__ x,
-                                                                        const double* __restrict__ ws, float* __restrict__ mean, float* __restrict__ variance,
-                                                                        float* __restrict__ saved_mean, float* __restrict__ saved_variance, double momentum)
+// The statistics of a channel from its blocks' sums, by the first wavefront of the block that asks
+__device__ __forceinline__ void bn_split_stats(int c, double n, int splits, const double* __restrict__ ws, float* m, float* v)
+{
+    const double* p = ws + (size_t)c * splits * 4;
+    double t[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        t[k] = wave_sum_d((int)threadIdx.x < splits ? p[(size_t)threadIdx.x * 4 + k] : 0.0);
+    bn_stats(n, (float)p[3], t, m, v);
+}
+__global__ __launch_bounds__(64) void batchnorm_f32_stats_finish_kernel(double n, int splits, const double* __restrict__ ws, float* __restrict__ mean,
+                                                                        float* __restrict__ variance, float* __restrict__ saved_mean,
+                                                                        float* __restrict__ saved_variance, double momentum)
 {
     const int c = blockIdx.x;
-    double t[3];
-    bn_partial_sums<3>(t, ws + (size_t)c * splits * 3, splits);
-    if (threadIdx.x == 0) bn_finish_stats(c, n, x[(size_t)c * plane], t, mean, variance, saved_mean, saved_variance, momentum);
+    float m, v;
+    bn_split_stats(c, n, splits, ws, &m, &v);
+    if (threadIdx.x == 0) bn_write_stats(c, n, m, v, mean, variance, saved_mean, saved_variance, momentum);
+}
+
+// The SAT activation quantizer behind a normalisation: fp receives what goes into it (or null), the output what comes out;
+// alpha null: no quantizer
+struct BnSat {
+    float* fp;
+    float range;
+    const float* alpha;
+};
+template <int V>
+__device__ __forceinline__ void bn_store(float* p, size_t idx, const float* v)
+{
+    if (V == 4) *(float4*)(p + idx) = make_float4(v[0], v[1], v[2], v[3]);
+    else p[idx] = v[0];
 }
 
 // y = scale * (x - mean) / sqrt(variance + epsilon) + bias.  eps_in_float: the inference branch of the reference adds
 // the epsilon in float and takes a float square root; the learning branch adds the double and rounds the root.
-__global__ __launch_bounds__(TBLOCK) void batchnorm_f32_apply_kernel(int planes, int C, int plane, const float* __restrict__ x,
-                                                                     const float* __restrict__ scale, const float* __restrict__ bias,
-                                                                     const float* __restrict__ mean, const float* __restrict__ variance, double epsilon,
-                                                                     int eps_in_float, int vec, float* __restrict__ y)
+// A channel per blockIdx.x, in ranges of its units as the sums: what a channel needs is worked out once a block, from the sums
+// of the statistics' blocks too (splits > 1), for which a launch of C blocks stood in between.  The block of a channel's first
+// range writes the statistics.  The quantizer that follows a normalisation in a learning net is applied on the way out; it read
+// and wrote the tensor again.  64 x 64 x 32 x 32, us: statistics, their end, this and the quantizer 5.8 + 4.8 + 6.1 + 10.5, now
+// 6.0 + 12.9, of which 10 are the 50 MB.
+template <int V, bool SAT>
+__global__ __launch_bounds__(TBLOCK) void batchnorm_f32_apply_kernel(BnRange q, int splits, double n, const double* __restrict__ ws, float* __restrict__ mean,
+                                                                     float* __restrict__ variance, float* __restrict__ saved_mean,
+                                                                     float* __restrict__ saved_variance, double momentum, int running,
+                                                                     const float* __restrict__ x, const float* __restrict__ scale, const float* __restrict__ bias, double epsilon,
+                                                                     BnSat sat, float* __restrict__ y)
 {
-    // blockIdx.y walks the (batch, channel) planes, so that the channel's constants are worked out once per plane;
-    // planes whose size is a multiple of 4 move 16 bytes per lane
-    for (int bc = blockIdx.y; bc < planes; bc += gridDim.y) {
-        const int c = bc % C;
-        const float var = eps_in_float ? sqrtf(variance[c] + (float)epsilon) : (float)sqrt((double)variance[c] + epsilon);
-        const float m = mean[c], g = scale[c], b = bias[c];
-        const float* xp = x + (size_t)bc * plane;
-        float* yp = y + (size_t)bc * plane;
-        if (vec) {
-            for (int i = blockIdx.x * TBLOCK + threadIdx.x; i < plane / 4; i += gridDim.x * TBLOCK) {
-                const float4 v = ((const float4*)xp)[i];
-                float4 o;
-                o.x = g * ((v.x - m) / var) + b;
-                o.y = g * ((v.y - m) / var) + b;
-                o.z = g * ((v.z - m) / var) + b;
-                o.w = g * ((v.w - m) / var) + b;
-                ((float4*)yp)[i] = o;
+    const int c = blockIdx.x;
+    float m, v;
+    if (splits > 1) {
+        __shared__ float stats[2];
+        if (threadIdx.x < 64) {
+            bn_split_stats(c, n, splits, ws, &m, &v);
+            if (threadIdx.x == 0) {
+                stats[0] = m; stats[1] = v;
+                if (blockIdx.y == 0) bn_write_stats(c, n, m, v, mean, variance, saved_mean, saved_variance, momentum);
             }
-        } else {
-            for (int i = blockIdx.x * TBLOCK + threadIdx.x; i < plane; i += gridDim.x * TBLOCK)
-                yp[i] = g * ((xp[i] - m) / var) + b;
         }
+        __syncthreads();
+        m = stats[0]; v = stats[1];
+    } else {
+        m = running ? mean[c] : saved_mean[c];
+        v = running ? variance[c] : saved_variance[c];
     }
+    const float var = running ? sqrtf(v + (float)epsilon) : (float)sqrt((double)v + epsilon);
+    const float g = scale[c], b = bias[c];
+    const float a = SAT ? fabsf(sat.alpha[0]) : 0.0f;
+    bn_walk<V>(q, c, [&](size_t idx) {
+        float t[V];
+        bn_load<V>(t, x, idx);
+#pragma unroll
+        for (int k = 0; k < V; ++k) t[k] = g * ((t[k] - m) / var) + b;
+        if (SAT) {
+            if (sat.fp) bn_store<V>(sat.fp, idx, t);
+#pragma unroll
+            for (int k = 0; k < V; ++k) t[k] = sat_quantize(t[k], sat.range, a);
+        }
+        bn_store<V>(y, idx, t);
+    });
 }
 
-// The same for small planes: one lane per value, the channel found by division.
+// The same for small planes, whose channels lie in pieces, and for channels past 32-bit counts: one lane per value, the
+// channel found by division.
 __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_apply_flat_kernel(size_t total, int C, int plane, const float* __restrict__ x,
                                                                      const float* __restrict__ scale, const float* __restrict__ bias,
                                                                      const float* __restrict__ mean, const float* __restrict__ variance, double epsilon,
-                                                                     int eps_in_float, float* __restrict__ y)
+                                                                     int eps_in_float, BnSat sat, float* __restrict__ y)
 {
+    const float a = sat.alpha ? fabsf(sat.alpha[0]) : 0.0f;
     for (size_t i = (size_t)blockIdx.x * TBLOCK + threadIdx.x; i < total; i += (size_t)gridDim.x * TBLOCK) {
         const int c = (int)((i / plane) % C);
         const float var = eps_in_float ? sqrtf(variance[c] + (float)epsilon) : (float)sqrt((double)variance[c] + epsilon);
         const float normalized = (x[i] - mean[c]) / var;
-        y[i] = scale[c] * normalized + bias[c];
+        float o = scale[c] * normalized + bias[c];
+        if (sat.alpha) {
+            if (sat.fp) sat.fp[i] = o;
+            o = sat_quantize(o, sat.range, a);
+        }
+        y[i] = o;
     }
 }
 
 // The five sums of BatchNormCell_Frame<T>::backPropagate over one channel, and what follows from them, in blocks as above.
 // 128 channels, 56 x 56, batch 32: 40.7 us and the last step 7.0, now 20.6 and 4.9.
-__device__ __forceinline__ void bn_finish_backward(int c, double n, const double* t, const float* __restrict__ saved_variance, double epsilon,
-                                                   float beta_scale, float* __restrict__ diff_scale, float beta_bias, float* __restrict__ diff_bias,
-                                                   float* __restrict__ diff_saved_mean, float* __restrict__ diff_saved_variance)
+struct BnGrads { float* diff_scale; float* diff_bias; float* diff_saved_mean; float* diff_saved_variance; float beta_scale, beta_bias; };
+__device__ __forceinline__ void bn_stats_grads(double n, const double* t, float saved_variance, double epsilon, float* dmean, float* dvariance)
 {
-    const float sum_scale = (float)t[0], sum_bias = (float)t[1], sum_mean1 = (float)t[2], sum_mean2 = (float)t[3], sum_var = (float)t[4];
-    const float var = (float)sqrt((double)saved_variance[c] + epsilon);
-    const float dv = (float)((double)sum_var * (-1.0 / 2.0) * pow((double)saved_variance[c] + epsilon, -3.0 / 2.0));
-    diff_saved_variance[c] = dv;
-    diff_saved_mean[c] = (float)((double)sum_mean1 * (-1.0 / (double)var) + (double)(dv * sum_mean2 / (float)n));
-    diff_scale[c] = sum_scale + (beta_scale != 0.0f ? beta_scale * diff_scale[c] : 0.0f);
-    diff_bias[c] = sum_bias + (beta_bias != 0.0f ? beta_bias * diff_bias[c] : 0.0f);
+    const float sum_mean1 = (float)t[2], sum_mean2 = (float)t[3], sum_var = (float)t[4];
+    const double square = (double)saved_variance + epsilon, root = sqrt(square);
+    const float var = (float)root;
+    *dvariance = (float)((double)sum_var * (-1.0 / 2.0) / (square * root));      // (to the power -3/2; pow() took longer than the sums)
+    *dmean = (float)((double)sum_mean1 * (-1.0 / (double)var) + (double)(*dvariance * sum_mean2 / (float)n));
+}
+__device__ __forceinline__ void bn_write_grads(int c, const double* t, float dmean, float dvariance, const BnGrads& o)
+{
+    const float sum_scale = (float)t[0], sum_bias = (float)t[1];
+    o.diff_saved_variance[c] = dvariance;
+    o.diff_saved_mean[c] = dmean;
+    o.diff_scale[c] = sum_scale + (o.beta_scale != 0.0f ? o.beta_scale * o.diff_scale[c] : 0.0f);
+    o.diff_bias[c] = sum_bias + (o.beta_bias != 0.0f ? o.beta_bias * o.diff_bias[c] : 0.0f);
 }
 template <int V>
 __global__ __launch_bounds__(1024) void batchnorm_f32_backward_sums_kernel(BnRange q, double n, const float* __restrict__ x,
                                                                            const float* __restrict__ scale, const float* __restrict__ saved_mean,
                                                                            const float* __restrict__ saved_variance, double epsilon,
-                                                                           const float* __restrict__ dy, double* __restrict__ ws, float beta_scale,
-                                                                           float* __restrict__ diff_scale, float beta_bias, float* __restrict__ diff_bias,
-                                                                           float* __restrict__ diff_saved_mean, float* __restrict__ diff_saved_variance)
+                                                                           const float* __restrict__ dy, double* __restrict__ ws, BnGrads grads)
 {
     constexpr int N = V ? V : 1;
     const int c = blockIdx.x;
@@ -609,60 +665,72 @@ __global__ __launch_bounds__(1024) void batchnorm_f32_backward_sums_kernel(BnRan
     bn_block_sums<5>(t);
     if (threadIdx.x) return;
     if (gridDim.y == 1) {
-        bn_finish_backward(c, n, t, saved_variance, epsilon, beta_scale, diff_scale, beta_bias, diff_bias, diff_saved_mean, diff_saved_variance);
+        float dmean, dvariance;
+        bn_stats_grads(n, t, saved_variance[c], epsilon, &dmean, &dvariance);
+        bn_write_grads(c, t, dmean, dvariance, grads);
     } else {
         double* o = ws + ((size_t)c * gridDim.y + blockIdx.y) * 5;
         o[0] = t[0]; o[1] = t[1]; o[2] = t[2]; o[3] = t[3]; o[4] = t[4];
     }
 }
 __global__ __launch_bounds__(64) void batchnorm_f32_backward_finish_kernel(double n, int splits, const double* __restrict__ ws,
-                                                                           const float* __restrict__ saved_variance, double epsilon, float beta_scale,
-                                                                           float* __restrict__ diff_scale, float beta_bias, float* __restrict__ diff_bias,
-                                                                           float* __restrict__ diff_saved_mean, float* __restrict__ diff_saved_variance)
+                                                                           const float* __restrict__ saved_variance, double epsilon, BnGrads grads)
 {
     const int c = blockIdx.x;
     double t[5];
     bn_partial_sums<5>(t, ws + (size_t)c * splits * 5, splits);
-    if (threadIdx.x == 0)
-        bn_finish_backward(c, n, t, saved_variance, epsilon, beta_scale, diff_scale, beta_bias, diff_bias, diff_saved_mean, diff_saved_variance);
+    if (threadIdx.x) return;
+    float dmean, dvariance;
+    bn_stats_grads(n, t, saved_variance[c], epsilon, &dmean, &dvariance);
+    bn_write_grads(c, t, dmean, dvariance, grads);
 }
 
-// dx = dy * scale / sigma + dVar * 2 (x - mean) / size + dMean / size, plane by plane as the apply kernel
+// dx = dy * scale / sigma + dVar * 2 (x - mean) / size + dMean / size, in ranges of a channel as the apply kernel, the end of the
+// sums before it with it: 4.8 + 8.7 us at 64 x 64 x 32 x 32, now 10.5
 __device__ __forceinline__ float bn_dx(float x, float d, float g, float var, float m, double dv2, double size, double dmean_over_size)
 {
     const float diff_normalized = d * g;
     return (float)((double)(diff_normalized / var) + dv2 * (double)(x - m) / size + dmean_over_size);
 }
-__global__ __launch_bounds__(TBLOCK) void batchnorm_f32_backward_data_kernel(int planes, int C, int plane, float size, const float* __restrict__ x,
-                                                                            const float* __restrict__ scale, const float* __restrict__ saved_mean,
-                                                                            const float* __restrict__ saved_variance, double epsilon, const float* dy,
-                                                                            const float* __restrict__ diff_saved_mean,
-                                                                            const float* __restrict__ diff_saved_variance, int vec, float* dx)
+template <int V>
+__global__ __launch_bounds__(TBLOCK) void batchnorm_f32_backward_data_kernel(BnRange q, int splits, double n, const double* __restrict__ ws, float size,
+                                                                            const float* __restrict__ x, const float* __restrict__ scale,
+                                                                            const float* __restrict__ saved_mean, const float* __restrict__ saved_variance,
+                                                                            double epsilon, const float* dy, BnGrads grads, float* dx)
 {
-    for (int bc = blockIdx.y; bc < planes; bc += gridDim.y) {
-        const int c = bc % C;
-        const float var = (float)sqrt((double)saved_variance[c] + epsilon);
-        const float m = saved_mean[c], g = scale[c];
-        const double dv2 = (double)diff_saved_variance[c] * 2.0, sz = (double)size, dm = (double)(diff_saved_mean[c] / size);
-        const float* xp = x + (size_t)bc * plane;
-        const float* dp = dy + (size_t)bc * plane;
-        float* op = dx + (size_t)bc * plane;
-        if (vec) {
-            for (int i = blockIdx.x * TBLOCK + threadIdx.x; i < plane / 4; i += gridDim.x * TBLOCK) {
-                const float4 v = ((const float4*)xp)[i];
-                const float4 d = ((const float4*)dp)[i];
-                float4 o;
-                o.x = bn_dx(v.x, d.x, g, var, m, dv2, sz, dm);
-                o.y = bn_dx(v.y, d.y, g, var, m, dv2, sz, dm);
-                o.z = bn_dx(v.z, d.z, g, var, m, dv2, sz, dm);
-                o.w = bn_dx(v.w, d.w, g, var, m, dv2, sz, dm);
-                ((float4*)op)[i] = o;
+    const int c = blockIdx.x;
+    float dmean, dvariance;
+    if (splits > 1) {
+        __shared__ float of_stats[2];
+        if (threadIdx.x < 64) {
+            double t[5];
+            const double* const p = ws + (size_t)c * splits * 5;
+#pragma unroll
+            for (int k = 0; k < 5; ++k)           // (the first two are the scale's and the bias's)
+                if (k >= 2 || blockIdx.y == 0) t[k] = wave_sum_d((int)threadIdx.x < splits ? p[(size_t)threadIdx.x * 5 + k] : 0.0);
+            if (threadIdx.x == 0) {
+                bn_stats_grads(n, t, saved_variance[c], epsilon, &dmean, &dvariance);
+                of_stats[0] = dmean; of_stats[1] = dvariance;
+                if (blockIdx.y == 0) bn_write_grads(c, t, dmean, dvariance, grads);
             }
-        } else {
-            for (int i = blockIdx.x * TBLOCK + threadIdx.x; i < plane; i += gridDim.x * TBLOCK)
-                op[i] = bn_dx(xp[i], dp[i], g, var, m, dv2, sz, dm);
         }
+        __syncthreads();
+        dmean = of_stats[0]; dvariance = of_stats[1];
+    } else {
+        dmean = grads.diff_saved_mean[c];
+        dvariance = grads.diff_saved_variance[c];
     }
+    const float var = (float)sqrt((double)saved_variance[c] + epsilon);
+    const float m = saved_mean[c], g = scale[c];
+    const double dv2 = (double)dvariance * 2.0, sz = (double)size, dm = (double)(dmean / size);
+    bn_walk<V>(q, c, [&](size_t idx) {
+        float xv[V], dv[V];
+        bn_load<V>(xv, x, idx);
+        bn_load<V>(dv, dy, idx);
+#pragma unroll
+        for (int k = 0; k < V; ++k) dv[k] = bn_dx(xv[k], dv[k], g, var, m, dv2, sz, dm);
+        bn_store<V>(dx, idx, dv);
+    });
 }
 
 // The same for small planes: one lane per value.
@@ -1467,43 +1535,72 @@ size_t n2d2hip_batchnorm_f32_workspace_bytes(int B, int C, int H, int W)
     return (size_t)C * bn_splits(B, C, H, W) * 5 * sizeof(double);
 }
 
+// Blocks a channel for the passes that write a tensor: about 2048 in all, none for less than a value or quad a thread.  Planes below
+// 64 values (a channel's values of one image are less than a cache line or two) go value by value instead.
+constexpr int BN_WALK_PLANE = 64;
+static int bn_ranges(int B, int C, int plane, int V)
+{
+    const size_t blocks = ((size_t)B * plane / std::max(V, 1) + TBLOCK - 1) / TBLOCK;
+    return (int)std::min<size_t>(std::max(2048 / C, 1), blocks);
+}
+
+static int batchnorm_forward(const char* who, int B, int C, int H, int W, const float* x, const float* scale, const float* bias, float* mean, float* variance,
+                             float* saved_mean, float* saved_variance, double epsilon, double moving_average_momentum, int use_running, float* y,
+                             const BnSat& sat, void* workspace, size_t workspace_bytes, hipStream_t stream)
+{
+    N2D2HIP_REQUIRE(B > 0 && C > 0 && H > 0 && W > 0 && x && scale && bias && mean && variance && y && epsilon > 0.0, N2D2HIP_ERR_INVALID,
+                    "%s: bad argument", who);
+    N2D2HIP_REQUIRE((size_t)B * C < ((size_t)1 << 31) && (size_t)H * W < ((size_t)1 << 31), N2D2HIP_ERR_INVALID, "%s: tensor too large", who);
+    const bool running = use_running || moving_average_momentum == 0.0;
+    const double n = (double)B * H * W;
+    const int plane = H * W;
+    const int V = bn_launch(B, C, plane, 1, (uintptr_t)x | (uintptr_t)y | (uintptr_t)sat.fp).V;
+    const bool walk = plane >= BN_WALK_PLANE && V != 0;
+    int splits = 1;
+    if (!running) {
+        N2D2HIP_REQUIRE(saved_mean && saved_variance, N2D2HIP_ERR_INVALID, "%s: the learning pass needs saved_mean and saved_variance", who);
+        N2D2HIP_REQUIRE((size_t)B * H * W > 1, N2D2HIP_ERR_INVALID, "%s: batch statistics need more than one value per channel", who);
+        splits = workspace && workspace_bytes >= n2d2hip_batchnorm_f32_workspace_bytes(B, C, H, W) ? bn_splits(B, C, H, W) : 1;
+        const BnLaunch l = bn_launch(B, C, plane, splits, (uintptr_t)x);
+        const auto kernel = l.V == 4 ? batchnorm_f32_stats_kernel<4> : l.V == 1 ? batchnorm_f32_stats_kernel<1> : batchnorm_f32_stats_kernel<0>;
+        hipLaunchKernelGGL(kernel, dim3(C, splits), dim3(l.block), 0, stream, l.q, n, x, (double*)workspace, mean, variance, saved_mean, saved_variance,
+                           moving_average_momentum);
+        if (splits > 1 && !walk)
+            hipLaunchKernelGGL(batchnorm_f32_stats_finish_kernel, dim3(C), dim3(64), 0, stream, n, splits, (const double*)workspace, mean, variance,
+                               saved_mean, saved_variance, moving_average_momentum);
+    }
+    if (walk) {
+        const int ranges = bn_ranges(B, C, plane, V);
+        const BnLaunch l = bn_launch(B, C, plane, ranges, (uintptr_t)x | (uintptr_t)y | (uintptr_t)sat.fp);
+        const auto kernel = V == 4 ? (sat.alpha ? batchnorm_f32_apply_kernel<4, true> : batchnorm_f32_apply_kernel<4, false>)
+                                   : (sat.alpha ? batchnorm_f32_apply_kernel<1, true> : batchnorm_f32_apply_kernel<1, false>);
+        hipLaunchKernelGGL(kernel, dim3(C, ranges), dim3(TBLOCK), 0, stream, l.q, splits, n, (const double*)workspace, mean, variance, saved_mean,
+                           saved_variance, moving_average_momentum, running ? 1 : 0, x, scale, bias, epsilon, sat, y);
+    } else {
+        hipLaunchKernelGGL(batchnorm_f32_apply_flat_kernel, dim3(grid_for((size_t)B * C * plane)), dim3(TBLOCK), 0, stream, (size_t)B * C * plane, C, plane, x,
+                           scale, bias, running ? (const float*)mean : (const float*)saved_mean, running ? (const float*)variance : (const float*)saved_variance,
+                           epsilon, running ? 1 : 0, sat, y);
+    }
+    N2D2HIP_HIP_CHECK(hipGetLastError());
+    return N2D2HIP_OK;
+}
+
 int n2d2hip_batchnorm_f32_forward(int B, int C, int H, int W, const float* x, const float* scale, const float* bias, float* mean,
                                   float* variance, float* saved_mean, float* saved_variance, double epsilon, double moving_average_momentum,
                                   int use_running, float* y, void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream)
 {
-    N2D2HIP_REQUIRE(B > 0 && C > 0 && H > 0 && W > 0 && x && scale && bias && mean && variance && y && epsilon > 0.0, N2D2HIP_ERR_INVALID,
-                    "n2d2hip_batchnorm_f32_forward: bad argument");
-    N2D2HIP_REQUIRE((size_t)B * C < ((size_t)1 << 31) && (size_t)H * W < ((size_t)1 << 31), N2D2HIP_ERR_INVALID,
-                    "n2d2hip_batchnorm_f32_forward: tensor too large");
-    const bool running = use_running || moving_average_momentum == 0.0;
-    if (!running) {
-        N2D2HIP_REQUIRE(saved_mean && saved_variance, N2D2HIP_ERR_INVALID, "n2d2hip_batchnorm_f32_forward: the learning pass needs saved_mean and saved_variance");
-        N2D2HIP_REQUIRE((size_t)B * H * W > 1, N2D2HIP_ERR_INVALID, "n2d2hip_batchnorm_f32_forward: batch statistics need more than one value per channel");
-        const double n = (double)B * H * W;
-        const int splits = workspace && workspace_bytes >= n2d2hip_batchnorm_f32_workspace_bytes(B, C, H, W) ? bn_splits(B, C, H, W) : 1;
-        const BnLaunch l = bn_launch(B, C, H * W, splits, (uintptr_t)x);
-        const auto kernel = l.V == 4 ? batchnorm_f32_stats_kernel<4> : l.V == 1 ? batchnorm_f32_stats_kernel<1> : batchnorm_f32_stats_kernel<0>;
-        hipLaunchKernelGGL(kernel, dim3(C, splits), dim3(l.block), 0, (hipStream_t)stream, l.q, n, x, (double*)workspace, mean, variance, saved_mean,
-                           saved_variance, moving_average_momentum);
-        if (splits > 1)
-            hipLaunchKernelGGL(batchnorm_f32_stats_finish_kernel, dim3(C), dim3(64), 0, (hipStream_t)stream, H * W, n, splits, x,
-                               (const double*)workspace, mean, variance, saved_mean, saved_variance, moving_average_momentum);
-    }
-    const int plane = H * W;
-    // 16 bytes per lane when every plane starts on a 16-byte boundary
-    const int vec = plane % 4 == 0 && ((uintptr_t)x | (uintptr_t)y) % 16 == 0;
-    const dim3 plane_grid((unsigned)std::max(1, std::min(((vec ? plane / 4 : plane) + TBLOCK - 1) / TBLOCK, 64)),
-                          (unsigned)std::min<size_t>((size_t)B * C, 32768));
-    if (plane >= 512)
-        hipLaunchKernelGGL(batchnorm_f32_apply_kernel, plane_grid, dim3(TBLOCK), 0, (hipStream_t)stream, B * C, C, plane, x, scale, bias,
-                           running ? (const float*)mean : (const float*)saved_mean, running ? (const float*)variance : (const float*)saved_variance,
-                           epsilon, running ? 1 : 0, vec, y);
-    else
-        hipLaunchKernelGGL(batchnorm_f32_apply_flat_kernel, dim3(grid_for((size_t)B * C * plane)), dim3(TBLOCK), 0, (hipStream_t)stream,
-                           (size_t)B * C * plane, C, plane, x, scale, bias, running ? (const float*)mean : (const float*)saved_mean,
-                           running ? (const float*)variance : (const float*)saved_variance, epsilon, running ? 1 : 0, y);
-    N2D2HIP_HIP_CHECK(hipGetLastError());
-    return N2D2HIP_OK;
+    return batchnorm_forward("n2d2hip_batchnorm_f32_forward", B, C, H, W, x, scale, bias, mean, variance, saved_mean, saved_variance, epsilon,
+                             moving_average_momentum, use_running, y, BnSat{nullptr, 0.0f, nullptr}, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+int n2d2hip_batchnorm_f32_forward_sat(int B, int C, int H, int W, const float* x, const float* scale, const float* bias, float* mean,
+                                      float* variance, float* saved_mean, float* saved_variance, double epsilon, double moving_average_momentum,
+                                      int use_running, float* y, float* full_precision, float range, const float* alpha, void* workspace,
+                                      size_t workspace_bytes, n2d2hip_stream_t stream)
+{
+    N2D2HIP_REQUIRE(alpha && range >= 1.0f && full_precision != y, N2D2HIP_ERR_INVALID, "n2d2hip_batchnorm_f32_forward_sat: bad argument");
+    return batchnorm_forward("n2d2hip_batchnorm_f32_forward_sat", B, C, H, W, x, scale, bias, mean, variance, saved_mean, saved_variance, epsilon,
+                             moving_average_momentum, use_running, y, BnSat{full_precision, range, alpha}, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 int n2d2hip_batchnorm_f32_backward(int B, int C, int H, int W, const float* x, const float* scale, const float* saved_mean,
@@ -1517,23 +1614,25 @@ int n2d2hip_batchnorm_f32_backward(int B, int C, int H, int W, const float* x, c
     N2D2HIP_REQUIRE((size_t)B * C < ((size_t)1 << 31) && (size_t)H * W < ((size_t)1 << 31), N2D2HIP_ERR_INVALID,
                     "n2d2hip_batchnorm_f32_backward: tensor too large");
     const double n = (double)B * H * W;
+    const int plane = H * W;
+    const BnGrads grads = {diff_scale, diff_bias, diff_saved_mean, diff_saved_variance, beta_scale, beta_bias};
     const int splits = workspace && workspace_bytes >= n2d2hip_batchnorm_f32_workspace_bytes(B, C, H, W) ? bn_splits(B, C, H, W) : 1;
-    const BnLaunch l = bn_launch(B, C, H * W, splits, (uintptr_t)x | (uintptr_t)diff_y);
+    const BnLaunch l = bn_launch(B, C, plane, splits, (uintptr_t)x | (uintptr_t)diff_y);
     const auto kernel = l.V == 4 ? batchnorm_f32_backward_sums_kernel<4> : l.V == 1 ? batchnorm_f32_backward_sums_kernel<1> : batchnorm_f32_backward_sums_kernel<0>;
     hipLaunchKernelGGL(kernel, dim3(C, splits), dim3(l.block), 0, (hipStream_t)stream, l.q, n, x, scale, saved_mean, saved_variance, epsilon, diff_y,
-                       (double*)workspace, beta_scale, diff_scale, beta_bias, diff_bias, diff_saved_mean, diff_saved_variance);
-    if (splits > 1)
+                       (double*)workspace, grads);
+    const int V = bn_launch(B, C, plane, 1, (uintptr_t)x | (uintptr_t)diff_y | (uintptr_t)diff_x).V;
+    const bool walk = diff_x && plane >= BN_WALK_PLANE && V != 0;
+    if (splits > 1 && !walk)
         hipLaunchKernelGGL(batchnorm_f32_backward_finish_kernel, dim3(C), dim3(64), 0, (hipStream_t)stream, n, splits, (const double*)workspace,
-                           saved_variance, epsilon, beta_scale, diff_scale, beta_bias, diff_bias, diff_saved_mean, diff_saved_variance);
-    const int plane = H * W;
-    const int vec = plane % 4 == 0 && ((uintptr_t)x | (uintptr_t)diff_y | (uintptr_t)diff_x) % 16 == 0;
-    const dim3 plane_grid((unsigned)std::max(1, std::min(((vec ? plane / 4 : plane) + TBLOCK - 1) / TBLOCK, 64)),
-                          (unsigned)std::min<size_t>((size_t)B * C, 32768));
-    if (diff_x && plane >= 512)
-        hipLaunchKernelGGL(batchnorm_f32_backward_data_kernel, plane_grid, dim3(TBLOCK), 0, (hipStream_t)stream, B * C, C, plane,
-                           (float)((size_t)B * H * W), x, scale, saved_mean, saved_variance, epsilon, diff_y, (const float*)diff_saved_mean,
-                           (const float*)diff_saved_variance, vec, diff_x);
-    else if (diff_x)
+                           saved_variance, epsilon, grads);
+    if (walk) {
+        const int ranges = bn_ranges(B, C, plane, V);
+        const BnLaunch d = bn_launch(B, C, plane, ranges, (uintptr_t)x | (uintptr_t)diff_y | (uintptr_t)diff_x);
+        hipLaunchKernelGGL(V == 4 ? batchnorm_f32_backward_data_kernel<4> : batchnorm_f32_backward_data_kernel<1>, dim3(C, ranges), dim3(TBLOCK), 0,
+                           (hipStream_t)stream, d.q, splits, n, (const double*)workspace, (float)((size_t)B * H * W), x, scale, saved_mean, saved_variance,
+                           epsilon, diff_y, grads, diff_x);
+    } else if (diff_x)
         hipLaunchKernelGGL(batchnorm_f32_backward_data_flat_kernel, dim3(grid_for((size_t)B * C * plane)), dim3(TBLOCK), 0, (hipStream_t)stream,
                            (size_t)B * C * plane, C, plane, (float)((size_t)B * H * W), x, scale, saved_mean, saved_variance, epsilon, diff_y,
                            (const float*)diff_saved_mean, (const float*)diff_saved_variance, diff_x);

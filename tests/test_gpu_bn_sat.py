@@ -1,0 +1,72 @@
+"""Batch normalisation with the SAT quantizer applied on the way out against the two calls, bit for bit, and the sums of several
+blocks finished by the launch that follows them against one block's: planes below and at the line between the two ways of
+walking a tensor, of whole and broken quads, one and several blocks a channel, in place, learning and inference."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(3, 5, 1, 1), (2, 7, 9, 7), (40, 3, 7, 9), (2, 6, 8, 8), (5, 4, 10, 10), (3, 5, 9, 9), (130, 3, 9, 9), (140, 3, 7, 9), (33, 2, 16, 17), (20, 70, 32, 32)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("running", [0, 1])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_quantized_on_the_way_out(shape, running, in_place):
+    import torch
+    from n2d2_amd import capi, runtime as rt
+    print("bn sat", shape, running, in_place, flush=True)
+    B, C, H, W = shape
+    lib, rng = capi.lib, np.random.default_rng(B * C + H)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).cuda()
+    x, scale, bias = dev(rng.normal(1, 2, shape)), dev(rng.normal(1, .3, C)), dev(rng.normal(0, .3, C))
+    alpha, n = dev([1.7]), B * C * H * W
+    ws = torch.empty(int(lib.n2d2hip_batchnorm_f32_workspace_bytes(B, C, H, W)), dtype=torch.uint8, device="cuda")
+    out = {}
+    for fused in (False, True):
+        src = x.clone()
+        y, fp = (src if in_place else torch.empty_like(x)), torch.empty_like(x)
+        st = [dev(np.full(C, v)) for v in (0.2, 1.5, 9, 9)]
+        args = [B, C, H, W, src.data_ptr(), scale.data_ptr(), bias.data_ptr()] + [s.data_ptr() for s in st] + [1e-4, 0.1, running, y.data_ptr()]
+        if fused:
+            capi.check(lib.n2d2hip_batchnorm_f32_forward_sat(*args, fp.data_ptr(), 15.0, alpha.data_ptr(), ws.data_ptr(), ws.numel(), rt.stream_ptr()))
+        else:
+            capi.check(lib.n2d2hip_batchnorm_f32_forward(*args, ws.data_ptr(), ws.numel(), rt.stream_ptr()))
+            capi.check(lib.n2d2hip_sat_act_forward(y.data_ptr(), fp.data_ptr(), n, 15.0, alpha.data_ptr(), rt.stream_ptr()))
+        out[fused] = [t.cpu().numpy() for t in (y, fp, *st)]
+    for a, b in zip(out[False], out[True]):
+        assert np.array_equal(a, b)
+    if not running:                    # against 64 bits: x - mean over the root, its rounding errors and those of the statistics
+        x64 = x.cpu().numpy().astype(np.float64)
+        m, v = x64.mean((0, 2, 3)), x64.var((0, 2, 3))
+        want = (x64 - m[:, None, None]) / np.sqrt(v + 1e-4)[:, None, None] * scale.cpu().numpy().astype(np.float64)[:, None, None] + bias.cpu().numpy()[:, None, None]
+        assert np.max(np.abs(out[True][1] - want)) < 2e-5 * max(1.0, np.max(np.abs(want)))
+        assert np.max(np.abs(out[True][4] - m)) < 1e-6 * np.max(np.abs(x64)) and np.max(np.abs(out[True][5] - v)) < 1e-5 * np.max(v)
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("beta", [0.0, 0.5])
+@pytest.mark.parametrize("to_input", [False, True])
+def test_backward_finished_by_the_next_launch(shape, beta, to_input):
+    """With the workspace (several blocks a channel, finished by the launch that writes diff_x) and without one (a block a channel)."""
+    import torch
+    from n2d2_amd import capi, runtime as rt
+    print("bn backward", shape, beta, to_input, flush=True)
+    B, C, H, W = shape
+    lib, rng = capi.lib, np.random.default_rng(B * C + H)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).cuda()
+    x, dy = dev(rng.normal(1, 2, shape)), dev(rng.normal(0, 1, shape))
+    scale, m, v = dev(rng.normal(1, .3, C)), dev(rng.normal(1, .1, C)), dev(rng.uniform(3, 5, C))
+    ws = torch.empty(int(lib.n2d2hip_batchnorm_f32_workspace_bytes(B, C, H, W)), dtype=torch.uint8, device="cuda")
+    out = []
+    for w in (None, ws):
+        g = [dev(np.full(C, 0.25)) for _ in range(4)]
+        dx = dy.clone()                # (diff_x over diff_y, as the cells use it)
+        capi.check(lib.n2d2hip_batchnorm_f32_backward(B, C, H, W, x.data_ptr(), scale.data_ptr(), m.data_ptr(), v.data_ptr(), 1e-4, dx.data_ptr(), beta,
+                                                      g[0].data_ptr(), beta, g[1].data_ptr(), g[2].data_ptr(), g[3].data_ptr(),
+                                                      dx.data_ptr() if to_input else None, w.data_ptr() if w is not None else None,
+                                                      w.numel() if w is not None else 0, rt.stream_ptr()))
+        out.append([t.cpu().numpy() for t in (*g, dx)])
+    # the sums are double on both sides and differ in their order only: one rounding to float apart
+    for a, b in zip(*out):
+        assert np.max(np.abs(a - b)) <= 4 * 2.0 ** -24 * max(1.0, np.max(np.abs(a)))
