@@ -587,84 +587,124 @@ __global__ __launch_bounds__(256) void conv_f32_3x3_kernel(PixelGemm g, const fl
 }
 
 // A layer that spans its input, forward, in the reference's order of terms: y[b][o] = sum over k of x[b][k] w[o][k], one
-// after the other in float.  The chain of additions is what takes the time (a product and an addition behind another: 5.3 ns
-// a term on one wave, of which the addition's latency is 3.6), so everything else is kept off it: a block is one wave with 8
-// images x 8 outputs, its 16 rows of operands arrive in LDS two stages of 256 terms ahead, and in registers 32 terms ahead.
-// 16384 -> 10, 64 images: 2632 -> 116 us.
+// after the other in float.  The chain of additions is what takes the time: a wave alone on its SIMD issues an instruction in
+// about 8 cycles, an addition no sooner than the one before it, so everything else is kept off that wave.  A block is 8 images
+// x 8 outputs and three waves: two load the operands (16 rows, in LDS two stages of 256 terms ahead), multiply them, 64 terms of
+// 128 each, and leave the products in LDS; the third reads those a step later and only adds.  16384 -> 10, 64 images: 117 us
+// with one wave that did all (2632 before that), now 90: additions and their reads, an instruction in 8 cycles.  (One wave with
+// the products of the next 32 terms between its additions: 130.  Steps of 64 terms: 95, and the same up to 1600 terms.)
 constexpr int CHAIN_K = 256, CHAIN_ROW = CHAIN_K + 4, CHAIN_STAGES = 3;      // (rows 16 bytes apart in the banks)
-__global__ __launch_bounds__(64) void conv_f32_chain_kernel(int B, int O, int K, const float* __restrict__ x, const float* __restrict__ w,
-                                                            const float* __restrict__ bias, float beta, float* __restrict__ y)
+constexpr int CHAIN_T = 128, CHAIN_PROD = CHAIN_T + 4;                        // terms between two barriers; a lane's row of products
+__global__ __launch_bounds__(192) void conv_f32_chain_kernel(int B, int O, int K, const float* __restrict__ x, const float* __restrict__ w,
+                                                             const float* __restrict__ bias, float beta, float* __restrict__ y)
 {
-    __shared__ __attribute__((aligned(16))) float smem[CHAIN_STAGES * 16 * CHAIN_ROW];
-    const int lane = threadIdx.x, bi = lane >> 3, oi = lane & 7, b0 = blockIdx.x * 8, o0 = blockIdx.y * 8;
-    const __amdgpu_buffer_rsrc_t rsrcX = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x + (size_t)b0 * K), 0, min(8, B - b0) * K * 4, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rsrcW = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(w + (size_t)o0 * K), 0, min(8, O - o0) * K * 4, 0x00020000);
-    int soff = 0;
-    unsigned dst = 0;
-    auto load = [&]() {                          // (terms past a row: zeros, or of the next row; rows past the last: zeros; not used)
+    __shared__ __attribute__((aligned(16))) float smem[CHAIN_STAGES * 16 * CHAIN_ROW + 2 * 64 * CHAIN_PROD];
+    float* const products = smem + CHAIN_STAGES * 16 * CHAIN_ROW;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int bi = lane >> 3, oi = lane & 7, b0 = blockIdx.x * 8, o0 = blockIdx.y * 8;
+    const int steps = (K + CHAIN_T - 1) / CHAIN_T;
+    constexpr int PER_STAGE = CHAIN_K / CHAIN_T;
+    // both sides pass barrier 0, ..., steps: step t multiplies between barriers t and t + 1 and is added between t + 1 and the next
+    if (wave < 2) {
+        // wave 0 loads the images' rows and wave 1 the outputs' (terms past a row: zeros, or of the next row; rows past the last: zeros)
+        const float* const rows = wave ? w + (size_t)o0 * K : x + (size_t)b0 * K;
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(rows), 0, min(8, wave ? O - o0 : B - b0) * K * 4, 0x00020000);
+        int soff = 0;
+        unsigned dst = wave * 8u * CHAIN_ROW * 4u;
+        auto load = [&]() {
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const lds_ptr_t d = (lds_ptr_t)((char*)smem + dst + r * CHAIN_ROW * 4);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcX, d, 16, lane * 16, soff + r * K * 4, 0, 0);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcW, (lds_ptr_t)((char*)smem + dst + (r + 8) * CHAIN_ROW * 4), 16, lane * 16, soff + r * K * 4, 0, 0);
+            for (int r = 0; r < 8; ++r)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)((char*)smem + dst + r * CHAIN_ROW * 4), 16, lane * 16, soff + r * K * 4, 0, 0);
+            soff += CHAIN_K * 4;
+            dst = dst >= (CHAIN_STAGES - 1) * 16u * CHAIN_ROW * 4u ? wave * 8u * CHAIN_ROW * 4u : dst + 16u * CHAIN_ROW * 4u;
+        };
+        const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) float*)smem;
+        const unsigned first = lds0 + 2u * CHAIN_T * wave;       // this wave's terms of a step
+        unsigned src = first;
+        float* const out = products + lane * CHAIN_PROD + CHAIN_T / 2 * wave;
+        load();
+        load();
+        wait_loads_and_barrier<8>();             // (barrier 0: the first stage is there)
+        for (int t = 0; t < steps; ++t) {
+            if (t % PER_STAGE == 0) load();      // where the stage before this one was, which both waves have read
+            float* const to = out + (t & 1) * 64 * CHAIN_PROD;
+            v4f xv[2][8], wv[2][8];
+            const unsigned xa = src + 4u * bi * CHAIN_ROW, wa = src + 4u * (8 + oi) * CHAIN_ROW;
+            const auto read = [&](auto half) {
+                constexpr int h = decltype(half)::value, o = 128 * h;
+                lds_read128f<o>(xv[h][0], xa); lds_read128f<o>(wv[h][0], wa);
+                lds_read128f<o + 16>(xv[h][1], xa); lds_read128f<o + 16>(wv[h][1], wa);
+                lds_read128f<o + 32>(xv[h][2], xa); lds_read128f<o + 32>(wv[h][2], wa);
+                lds_read128f<o + 48>(xv[h][3], xa); lds_read128f<o + 48>(wv[h][3], wa);
+                lds_read128f<o + 64>(xv[h][4], xa); lds_read128f<o + 64>(wv[h][4], wa);
+                lds_read128f<o + 80>(xv[h][5], xa); lds_read128f<o + 80>(wv[h][5], wa);
+                lds_read128f<o + 96>(xv[h][6], xa); lds_read128f<o + 96>(wv[h][6], wa);
+                lds_read128f<o + 112>(xv[h][7], xa); lds_read128f<o + 112>(wv[h][7], wa);
+            };
+            read(std::integral_constant<int, 0>{});
+            wait_lgkm<0>();
+#pragma unroll
+            for (int i = 0; i < 8; ++i) { tie(xv[0][i]); tie(wv[0][i]); }
+            read(std::integral_constant<int, 1>{});
+#pragma unroll
+            for (int i = 0; i < 8; ++i) *(v4f*)(to + 4 * i) = wv[0][i] * xv[0][i];
+            wait_lgkm<0>();
+#pragma unroll
+            for (int i = 0; i < 8; ++i) { tie(xv[1][i]); tie(wv[1][i]); *(v4f*)(to + 32 + 4 * i) = wv[1][i] * xv[1][i]; }
+            src += 4u * CHAIN_T;
+            if ((t + 1) % PER_STAGE == 0)
+                src = t + 1 == PER_STAGE * CHAIN_STAGES * ((t + 1) / (PER_STAGE * CHAIN_STAGES)) ? first : src + 4u * (16 * CHAIN_ROW - CHAIN_K);
+            if ((t + 1) % PER_STAGE == 0) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");       // (the next stage is there)
+            else asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         }
-        soff += CHAIN_K * 4;
-        dst = dst == (CHAIN_STAGES - 1) * 16u * CHAIN_ROW * 4u ? 0u : dst + 16u * CHAIN_ROW * 4u;
-    };
-    const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) float*)smem;
-    const unsigned xrow = lds0 + 4u * bi * CHAIN_ROW, wrow = lds0 + 4u * (8 + oi) * CHAIN_ROW;
-    const int full = K / 32, rest = K % 32, groups = full + (rest > 0);
-    v4f xv[2][8], wv[2][8];
-    unsigned src = 0;
-    auto read = [&](int buf, int h) {            // the operands of the h-th 32 terms
-        const unsigned off = src + 128u * (h & 7);
-        const unsigned xa = xrow + off, wa = wrow + off;
-        lds_read128f<0>(xv[buf][0], xa); lds_read128f<0>(wv[buf][0], wa);
-        lds_read128f<16>(xv[buf][1], xa); lds_read128f<16>(wv[buf][1], wa);
-        lds_read128f<32>(xv[buf][2], xa); lds_read128f<32>(wv[buf][2], wa);
-        lds_read128f<48>(xv[buf][3], xa); lds_read128f<48>(wv[buf][3], wa);
-        lds_read128f<64>(xv[buf][4], xa); lds_read128f<64>(wv[buf][4], wa);
-        lds_read128f<80>(xv[buf][5], xa); lds_read128f<80>(wv[buf][5], wa);
-        lds_read128f<96>(xv[buf][6], xa); lds_read128f<96>(wv[buf][6], wa);
-        lds_read128f<112>(xv[buf][7], xa); lds_read128f<112>(wv[buf][7], wa);
-    };
-    float sum = 0.0f;
-    auto group = [&](auto bufc, int h) {
-        constexpr int buf = decltype(bufc)::value;
-        wait_lgkm<0>();
-#pragma unroll
-        for (int i = 0; i < 8; ++i) { tie(xv[buf][i]); tie(wv[buf][i]); }
-        if ((h & 7) == 7) {                      // the stage has been read: its place is free, and the next one is there
-            wait_loads_and_barrier<16 * (CHAIN_STAGES - 2)>();
-            load();
-            src = src == (CHAIN_STAGES - 1) * 16u * CHAIN_ROW * 4u ? 0u : src + 16u * CHAIN_ROW * 4u;
-        }
-        if (h + 1 < groups) read(1 - buf, h + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        if (h < full) {
-            float p[32];
-#pragma unroll
-            for (int i = 0; i < 32; ++i) p[i] = wv[buf][i >> 2][i & 3] * xv[buf][i >> 2][i & 3];
-#pragma unroll
-            for (int i = 0; i < 32; ++i) sum = sum + p[i];
-        } else {
-#pragma unroll
-            for (int i = 0; i < 31; ++i) {
-                const float t = sum + wv[buf][i >> 2][i & 3] * xv[buf][i >> 2][i & 3];
-                sum = i < rest ? t : sum;
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    };
-#pragma unroll
-    for (int st = 0; st < CHAIN_STAGES; ++st) load();
-    wait_loads_and_barrier<16 * (CHAIN_STAGES - 1)>();
-    read(0, 0);
-    for (int h = 0; h < groups; h += 2) {
-        group(std::integral_constant<int, 0>{}, h);
-        if (h + 1 < groups) group(std::integral_constant<int, 1>{}, h + 1);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        return;
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    float sum = 0.0f;
+    const unsigned in = (unsigned)(unsigned long)(__attribute__((address_space(3))) float*)(products + lane * CHAIN_PROD);
+    asm volatile("s_barrier" ::: "memory");
+    for (int t = 0; t < steps; ++t) {
+        asm volatile("s_barrier" ::: "memory");
+        const unsigned from = in + (t & 1) * 4u * 64u * CHAIN_PROD;
+        const int rest = K - t * CHAIN_T;
+        // quarters of 32 products, each requested a quarter ahead; the first adds as its reads arrive
+        v4f p[2][8];
+        const auto read = [&](auto quarter) {
+            constexpr int h = decltype(quarter)::value & 1, o = 128 * decltype(quarter)::value;
+            lds_read128f<o>(p[h][0], from); lds_read128f<o + 16>(p[h][1], from);
+            lds_read128f<o + 32>(p[h][2], from); lds_read128f<o + 48>(p[h][3], from);
+            lds_read128f<o + 64>(p[h][4], from); lds_read128f<o + 80>(p[h][5], from);
+            lds_read128f<o + 96>(p[h][6], from); lds_read128f<o + 112>(p[h][7], from);
+        };
+        const auto add = [&](auto quarter) {
+            constexpr int h = decltype(quarter)::value & 1, k0 = 32 * decltype(quarter)::value;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) tie(p[h][i]);
+            if (rest >= k0 + 32) {
+#pragma unroll
+                for (int i = 0; i < 32; ++i) sum = sum + p[h][i >> 2][i & 3];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 31; ++i) sum = k0 + i < rest ? sum + p[h][i >> 2][i & 3] : sum;
+            }
+        };
+        read(std::integral_constant<int, 0>{});
+        read(std::integral_constant<int, 1>{});
+        wait_lgkm<8>();
+        add(std::integral_constant<int, 0>{});
+        __builtin_amdgcn_sched_barrier(0);
+        read(std::integral_constant<int, 2>{});
+        wait_lgkm<8>();
+        add(std::integral_constant<int, 1>{});
+        __builtin_amdgcn_sched_barrier(0);
+        read(std::integral_constant<int, 3>{});
+        wait_lgkm<8>();
+        add(std::integral_constant<int, 2>{});
+        __builtin_amdgcn_sched_barrier(0);
+        wait_lgkm<0>();
+        add(std::integral_constant<int, 3>{});
+        __builtin_amdgcn_sched_barrier(0);
+    }
     const int b = b0 + bi, o = o0 + oi;
     if (b >= B || o >= O) return;
     const size_t idx = (size_t)b * O + o;

@@ -1,0 +1,29 @@
+"""The forward pass of a layer that spans its input against the same sum in float32 on the host, term for term: equal bits, at the
+remainders of the kernel's steps of 128 terms, stages of 256, 8 images and 8 outputs."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,K,O", [(1, 4, 1), (8, 124, 8), (9, 128, 7), (3, 132, 9), (8, 252, 16), (5, 256, 3), (2, 260, 8), (17, 384, 10), (8, 508, 8),
+                                   (1, 768, 12), (8, 772, 1), (4, 1020, 8), (7, 1024, 5), (3, 2308, 11)])
+def test_equals_ordered_float32_sum(B, K, O):
+    import torch
+    from n2d2_amd import capi, runtime as rt
+    print("chain", B, K, O, flush=True)
+    rng = np.random.default_rng(K + O)
+    x, w, bias, y0 = (rng.normal(size=s).astype(np.float32) for s in ((B, K), (O, K), (O,), (B, O)))
+    want = np.zeros((B, O), np.float32)
+    for k in range(K):
+        want = want + w[None, :, k] * x[:, k, None]
+    want = bias[None] + (want + np.float32(0.5) * y0)
+    d = capi.ConvDesc(K // 4, O, 2, 2, 1, 1, 0, 0, 0, 0, 1, 1, 1, 0, capi.KERNEL_F32_DIRECT)
+    dev = lambda a: torch.from_numpy(a).cuda()
+    dx, dw, db, dy = dev(x), dev(w), dev(bias), dev(y0)
+    capi.check(capi.lib.n2d2hip_conv2d_f32_forward(C.byref(d), B, 2, 2, dx.data_ptr(), dw.data_ptr(), db.data_ptr(), 0.5, dy.data_ptr(), None, 0,
+                                                   rt.stream_ptr()))
+    torch.cuda.synchronize()
+    assert np.array_equal(dy.cpu().numpy(), want)
