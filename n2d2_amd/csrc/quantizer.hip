@@ -130,8 +130,8 @@ struct SatLevels {
 // SAT weights of several tensors, in two launches at most: a learning net quantizes the weights of all its cells before a pass,
 // most of them few, and a launch each (three for many weights) was what bounded them.  16 tensors fit a launch's arguments.
 //  * Up to 16384 weights: one block computes the tensor, in the first launch.  Its tanh stay in registers (they were computed
-//    twice, and each pass went through memory): up to 1024 weights 3.7 us, 2400 4.2 and 10080, scaling included, 11.5; the blocks
-//    of several tensors run side by side.  (Instances by the weights per thread: skipping unused ones inside one instance
+//    twice, and each pass went through memory): up to 1024 weights 3.7 us, 2400 4.2 and 10080, scaling included, 11.6 in a
+//    batch (12.8 with an instance of 16 weights a thread); the blocks of several tensors run side by side.  (Instances by the weights per thread: skipping unused ones inside one instance
 //    made the compiler spill.)
 //  * More: the first launch leaves each block's max |tanh w|, and every block of the second one takes the maximum of those,
 //    at most 256, itself, instead of a launch of one block in between (48120 weights: 3 launches of 2.8, 1.8 and 2.4 us).
@@ -196,6 +196,8 @@ __global__ __launch_bounds__(1024) void sat_weight_first_kernel(const SatBatch<N
     const n2d2hip_sat_weight_item& t = b.item[k];
     if (t.n <= 1024) sat_weight_small<1>(t);
     else if (t.n <= 4 * 1024) sat_weight_small<4>(t);
+    else if (t.n <= 8 * 1024) sat_weight_small<8>(t);
+    else if (t.n <= 12 * 1024) sat_weight_small<12>(t);
     else if (sat_small(t.n)) sat_weight_small<SAT_SMALL>(t);
     else {
         float m = 0.0f;
