@@ -478,7 +478,7 @@ int n2d2hip_dw_pw_create(n2d2hip_conv_t dw, n2d2hip_conv_t pw, n2d2hip_dw_pw_t* 
         && (dd.strideX == 1 || dd.strideX == 2) && dw->act->args.kind == EPI_I24 && dw->act->cpad >= C && dw->in_cs == C
         && (C == 32 || C % 64 == 0) && dw->act->min_out >= -128 && dw->act->max_out <= 255
         && plain_1x1(dp) && dp.C == C && pw->in_cs == C && pw->in_dtype == byte_type_of(dw->act) && (O == 64 || O == 128 || O % 256 == 0)
-        && pw->act->args.kind == EPI_I24 && pw->bias_folded && pw->d_epi_tab && pw->act->min_out >= -128 && pw->act->max_out <= 255
+        && (int)dw->act->htab.size() >= 5 * dw->act->cpad && pw->act->args.kind == EPI_I24 && pw->bias_folded && pw->d_epi_tab && pw->act->min_out >= -128 && pw->act->max_out <= 255
         && !pw->sum && pw->ktot >= C;
     N2D2HIP_REQUIRE(ok, N2D2HIP_ERR_UNSUPPORTED,
                     "dw_pw_create: needs a 3x3 undilated depthwise convolution of stride 1 or 2 over 32 or a multiple of 64 channels and an "
@@ -522,26 +522,24 @@ int n2d2hip_dw_pw_create(n2d2hip_conv_t dw, n2d2hip_conv_t pw, n2d2hip_dw_pw_t* 
     const bool fast = dw->bias_folded && dw->d_epi_tab && !dw->preclamp && dw->act->args.lo == 0 && dw->act->args.hi == 255
         && !pw->preclamp && pw->act->args.lo == 0 && pw->act->args.hi == 255;
     {
-        const EpiArgs& t = dw->act->args;
         const int cpd = dw->act->cpad;
-        const int* w = dw->d_wdw;
-        const int* rows[] = {w, w + C, w + 2 * (size_t)C, fast ? dw->d_epi_tab + 2 * cpd : t.c, fast ? dw->d_epi_tab + 3 * cpd : t.d,
-                             w + 3 * (size_t)C, t.a, t.b, fast ? dw->d_epi_tab + 4 * cpd : t.e};     // in the order of DWT_*, then e
+        std::vector<int> wdw(4 * (size_t)C), rescale = dw->act->htab;      // a, b, c, d, e, each [cpad]
+        e = hipMemcpy(wdw.data(), dw->d_wdw, wdw.size() * sizeof(int), hipMemcpyDeviceToHost);
+        if (fast && e == hipSuccess) e = hipMemcpy(rescale.data(), dw->d_epi_tab, 5 * (size_t)cpd * sizeof(int), hipMemcpyDeviceToHost);
+        if (e != hipSuccess)
+            return fail(N2D2HIP_ERR_HIP, "dw_pw_create: reading the depthwise tables back failed: %s", hipGetErrorString(e));
         const size_t base = tab.size();
         tab.resize(base + (size_t)nchunks * DWT_ROWS * kc);
-        std::vector<int> row(C);
-        for (int r = 0; r <= DWT_USED; ++r) {
-            e = hipMemcpy(row.data(), rows[r], C * sizeof(int), hipMemcpyDeviceToHost);
-            if (e != hipSuccess)
-                return fail(N2D2HIP_ERR_HIP, "dw_pw_create: reading the depthwise tables back failed: %s", hipGetErrorString(e));
-            for (int c = 0; c < C; ++c) {
-                int* const t0 = tab.data() + base + (size_t)(c / kc) * DWT_ROWS * kc + c % kc;
-                if (r < 3)
-                    for (int kx = 0; kx < 3; ++kx)
-                        t0[(DWT_W + kx) * kc] |= (row[c] >> (8 * kx) & 255) << (8 * r);
-                else if (r == DWT_USED) t0[DWT_CE * kc] = with_shift(t0[DWT_CE * kc], row[c]);
-                else t0[r * kc] = row[c];
-            }
+        for (int c = 0; c < C; ++c) {
+            int* const t0 = tab.data() + base + (size_t)(c / kc) * DWT_ROWS * kc + c % kc;
+            for (int kx = 0; kx < 3; ++kx)
+                for (int ky = 0; ky < 3; ++ky)
+                    t0[(DWT_W + kx) * kc] |= (wdw[(size_t)ky * C + c] >> (8 * kx) & 255) << (8 * ky);
+            t0[DWT_CE * kc] = with_shift(rescale[2 * (size_t)cpd + c], rescale[4 * (size_t)cpd + c]);
+            t0[DWT_D * kc] = rescale[3 * (size_t)cpd + c];
+            t0[DWT_BIAS * kc] = wdw[3 * (size_t)C + c];
+            t0[DWT_A * kc] = rescale[c];
+            t0[DWT_B * kc] = rescale[(size_t)cpd + c];
         }
     }
     n2d2hip_dw_pw_s* h = new n2d2hip_dw_pw_s();

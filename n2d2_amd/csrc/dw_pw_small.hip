@@ -28,7 +28,9 @@ namespace {
 // general rescale needs
 enum { DWS_W, DWS_C = 3, DWS_D, DWS_E, DWS_BIAS, DWS_A, DWS_B, DWS_ROWS = 12 };
 constexpr int OUTS = 32, PIXELS = 16, MAX_PARTS = 8;
-constexpr int TILES_OUTS = 128;           // up to so many outputs the kernel for many pixels is considered too
+// the kernel for many pixels is considered too: up to 128 outputs at every size, up to 512 from so many pixels
+constexpr int TILES_OUTS = 128, TILES_WIDE_OUTS = 512;
+constexpr long long TILES_WIDE_PIXELS = 9216;
 constexpr int STAGE_PIXELS = 9 * PIXELS * 64, STAGE = STAGE_PIXELS + DWS_ROWS * 64 * 4;      // bytes of LDS of a wave
 
 struct DwPwSmallArgs {
@@ -183,6 +185,15 @@ struct n2d2hip_dw_pw_small_s {
     size_t dwt_at, pwt_at, fill_at;
 };
 
+// The other kernel's handle, or null where that does not take the pair
+static int make_tiles(n2d2hip_dw_pw_small_s* h)
+{
+    const int rc = n2d2hip_dw_pw_create(h->dw, h->pw, &h->tiles);
+    if (rc != N2D2HIP_OK)
+        h->tiles = nullptr;
+    return rc == N2D2HIP_ERR_UNSUPPORTED ? N2D2HIP_OK : rc;
+}
+
 extern "C" {
 
 int n2d2hip_dw_pw_small_destroy(n2d2hip_dw_pw_small_t h)
@@ -263,29 +274,27 @@ int n2d2hip_dw_pw_small_create(n2d2hip_conv_t dw, n2d2hip_conv_t pw, n2d2hip_dw_
         return fail(N2D2HIP_ERR_HIP, "dw_pw_small_create: device upload failed: %s", hipGetErrorString(e));
     }
     if (O <= TILES_OUTS) {
-        const int rc = n2d2hip_dw_pw_create(dw, pw, &h->tiles);
-        if (rc != N2D2HIP_OK && rc != N2D2HIP_ERR_UNSUPPORTED) {
+        const int rc = make_tiles(h);
+        if (rc != N2D2HIP_OK) {
             n2d2hip_dw_pw_small_destroy(h);
             return rc;
         }
-        if (rc != N2D2HIP_OK)
-            h->tiles = nullptr;
     }
     *out = h;
     return N2D2HIP_OK;
 }
 
-// 32 pixels' worth of outputs and more channels than a chunk fill the chip only with many pixels, 8 x 16 of which the other kernel
-// gives to a work-group; up to 128 outputs it needs no more of them than one image has.  us, that kernel / this one / two
-// launches: 32 -> 64 channels, 112 x 112 3.6 / 4.8 / 7.6, two images of 48 x 48 3.4 / 4.1 / 7.5; 64 -> 128 stride 2, 56 x 56
-// 4.6 / 4.3 / 8.1, two 4.6 / 5.1 / 8.2; 128 -> 128, 56 x 56 5.1 / 4.6 / 6.6, two 5.2 / 6.7 / 7.0, four 5.3 / 10.0 / 8.0, two of 24 x 24
-// 5.7 / 4.1 / 5.9.
-static bool choose_tiles(n2d2hip_dw_pw_small_t h, long long groups)
-{
-    return h->tiles && (h->dw->desc.C == 32 || groups > 1024);
-}
-
 static long long work_groups(n2d2hip_dw_pw_small_t h, long long pixels) { return (pixels + PIXELS - 1) / PIXELS * (h->pw->desc.O / OUTS); }
+
+// That kernel gives a work-group 8 x 16 pixels and all their outputs, up to 256.  us, that kernel / this one / two launches, up to
+// 128 outputs: 32 -> 64 channels, 112 x 112 3.6 / 4.8 / 7.6, two images of 48 x 48 3.4 / 4.1 / 7.5; 64 -> 128 stride 2, 56 x 56
+// 4.6 / 4.3 / 8.1, two 4.6 / 5.1 / 8.2; 128 -> 128, 56 x 56 5.1 / 4.6 / 6.6, two 5.2 / 6.7 / 7.0, four 5.3 / 10.0 / 8.0, two of 24 x 24
+// 5.7 / 4.1 / 5.9.  With 512 outputs it computes the depthwise part twice and fills the chip later; that kernel / two launches,
+// 512 -> 512 at 14 x 14: 32 images 14.3 / 12.9, 48 15.0 / 15.9, 64 15.8 / 17.9, 128 26.8 / 28.2 (1024 outputs: 24.7 / 15.0 at 64).
+static bool choose_tiles(n2d2hip_dw_pw_small_t h, long long pixels)
+{
+    return h->tiles && (h->pw->desc.O > TILES_OUTS ? pixels >= TILES_WIDE_PIXELS : h->dw->desc.C == 32 || work_groups(h, pixels) > 1024);
+}
 
 int n2d2hip_dw_pw_small_pays(n2d2hip_dw_pw_small_t h, int batch, int in_h, int in_w)
 {
@@ -294,8 +303,11 @@ int n2d2hip_dw_pw_small_pays(n2d2hip_dw_pw_small_t h, int batch, int in_h, int i
     int OH, OW;
     if (n2d2hip_conv_out_dims(&h->dw->desc, in_h, in_w, &OH, &OW) != N2D2HIP_OK)
         return 0;
-    const long long groups = work_groups(h, (long long)batch * OH * OW);
-    if (choose_tiles(h, groups))
+    const long long pixels = (long long)batch * OH * OW, groups = work_groups(h, pixels);
+    const int O = h->pw->desc.O;
+    if (!h->tiles && O > TILES_OUTS && O <= TILES_WIDE_OUTS && pixels >= TILES_WIDE_PIXELS && make_tiles(h) != N2D2HIP_OK)
+        return 0;
+    if (choose_tiles(h, pixels))
         return 1;
     // Where all work-groups are on the chip at once (by their LDS, 12 KB a wave).  us, one launch and two, for output planes of
     // 112 / 56 / 56 / 28 / 28 / 14 / 14 / 7 and 32 -> 64, 64 -> 128, 128 -> 128, 128 -> 256, 256 -> 256, 256 -> 512, 512 -> 512, 512 -> 1024 channels:
@@ -316,7 +328,7 @@ int n2d2hip_dw_pw_small_forward(n2d2hip_dw_pw_small_t h, const n2d2hip_tensor* i
     if (rc != N2D2HIP_OK)
         return rc;
     const long long pixels = (long long)in->B * OH * OW;
-    if (choose_tiles(h, work_groups(h, pixels)))
+    if (choose_tiles(h, pixels))
         return n2d2hip_dw_pw_forward(h->tiles, in, out, stream_);
     const int out_dtype = byte_type_of(h->pw->act);
     N2D2HIP_REQUIRE(in->layout == N2D2HIP_NHWC && out->layout == N2D2HIP_NHWC && in->halo == 0 && out->halo == 0, N2D2HIP_ERR_UNSUPPORTED,

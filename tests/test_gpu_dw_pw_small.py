@@ -17,6 +17,7 @@ pytestmark = pytest.mark.gpu
     (2, 64, 128, 1, 33, 31, 1),        # 256 + groups: all on the chip
     (2, 64, 128, 1, 48, 47, 1),        # 1128 work-groups: the kernel for many pixels
     (1, 32, 64, 1, 20, 9, 1),          # 32 channels: the kernel for many pixels
+    (6, 64, 512, 1, 40, 39, 1),        # 512 outputs, 9360 pixels: the kernel for many pixels, once asked for
 ])
 @pytest.mark.parametrize("rescale", ["plain", "clamped", "wide"])
 def test_small_equals_separate_launches(B, C, O, stride, H, W, pad, rescale):
@@ -44,6 +45,8 @@ def test_small_equals_separate_launches(B, C, O, stride, H, W, pad, rescale):
     fused = rt.DwPwSmall.create(dw, pw)
     assert fused is not None
     out = rt.DTensor(B, O, want.H, want.W, want.dtype)
+    assert np.array_equal(fused.forward(xin, out).to_numpy(), want.to_numpy())
+    fused.pays(B, H, W)
     assert np.array_equal(fused.forward(xin, out).to_numpy(), want.to_numpy())
 
 
