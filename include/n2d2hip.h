@@ -582,6 +582,16 @@ int n2d2hip_batchnorm_f32_backward(int B, int C, int H, int W, const float* x, c
                                    float* diff_scale, float beta_bias, float* diff_bias, float* diff_saved_mean,
                                    float* diff_saved_variance, float* diff_x, void* workspace, size_t workspace_bytes,
                                    n2d2hip_stream_t stream);
+/* The same behind the SAT quantizer of n2d2hip_batchnorm_f32_forward_sat(): diff_y first goes through
+ * n2d2hip_sat_act_backward(diff_y, full_precision, diff_y, ..., beta_alpha, diff_alpha), in place.  It always needs a
+ * workspace, of n2d2hip_batchnorm_f32_backward_sat_workspace_bytes(), which serves the calls above too. */
+size_t n2d2hip_batchnorm_f32_backward_sat_workspace_bytes(int B, int C, int H, int W);
+int n2d2hip_batchnorm_f32_backward_sat(int B, int C, int H, int W, const float* x, const float* scale, const float* saved_mean,
+                                       const float* saved_variance, double epsilon, const float* full_precision, float range,
+                                       const float* alpha, float beta_alpha, float* diff_alpha, float* diff_y,
+                                       float beta_scale, float* diff_scale, float beta_bias, float* diff_bias,
+                                       float* diff_saved_mean, float* diff_saved_variance, float* diff_x, void* workspace,
+                                       size_t workspace_bytes, n2d2hip_stream_t stream);
 /* Max pooling of float NCHW, one output per channel; output size as PoolCell computes it, (in + 2 pad - pool + stride) /
  * stride.  argmax {B,C,oH,oW} receives row * W + column of the first largest element of each window in row-major order,
  * -1 for a window that lies in the padding (output 0) (ref: PoolCell_Frame_Kernels::forwardMax with its ArgMax tensor,

@@ -1598,14 +1598,21 @@ void SATQuantizerActivation_Frame_HIP<T>::propagate(float* inOut, std::size_t si
 }
 
 template <class T>
-void SATQuantizerActivation_Frame_HIP<T>::back_propagate(const float* diffInput, float* diffOutput, std::size_t size)
+typename SATQuantizerActivation_Frame_HIP<T>::PreparedGradient SATQuantizerActivation_Frame_HIP<T>::prepareGradient(std::size_t size)
 {
     if (!mFp || mFpSize != size)
         throw std::runtime_error("SATQuantizerActivation_Frame_HIP::back_propagate(): no full-precision activations saved (propagate with inference = false first)");
     lazyInit(size, true);
+    return PreparedGradient{mFp, (float)mRange, mDev, (mSolver && !mSolver->isNewIteration()) ? 1.0f : 0.0f, mDev + 1};
+}
+
+template <class T>
+void SATQuantizerActivation_Frame_HIP<T>::back_propagate(const float* diffInput, float* diffOutput, std::size_t size)
+{
+    const PreparedGradient g = prepareGradient(size);
     ensureWorkspace(mWorkspace, mWorkspaceBytes, size);
-    const float beta = (mSolver && !mSolver->isNewIteration()) ? 1.0f : 0.0f;
-    checkStatus(n2d2hip_sat_act_backward(diffInput, mFp, diffOutput, size, (float)mRange, mDev, beta, mDev + 1, mWorkspace, mWorkspaceBytes, mStream));
+    checkStatus(n2d2hip_sat_act_backward(diffInput, g.fullPrecision, diffOutput, size, g.range, g.alpha, g.beta, g.diffAlpha, mWorkspace, mWorkspaceBytes,
+                                         mStream));
 }
 
 template <class T>

@@ -1058,6 +1058,9 @@ public:
     // (null in inference), the range and the device's alpha
     struct Prepared { float* fullPrecision; float range; const float* alpha; };
     Prepared prepare(std::size_t size, bool inference);
+    // the same for back_propagate(): what it reads, and where alpha's gradient goes (beta: the part of what is there that stays)
+    struct PreparedGradient { const float* fullPrecision; float range; const float* alpha; float beta; float* diffAlpha; };
+    PreparedGradient prepareGradient(std::size_t size);
 
 private:
     void lazyInit(std::size_t size, bool needCopy);

@@ -574,7 +574,7 @@ void BatchNormCell_FrameTrain_HIP<T>::initialize()
     }
     for (DeviceFloats* d : {&mSavedMean, &mSavedVariance, &mDiffSavedMean, &mDiffSavedVariance})
         d->resize(dims);
-    const size_t bytes = n2d2hip_batchnorm_f32_workspace_bytes((int)mIn->dimB(), (int)mNbOutputs, (int)mInH, (int)mInW);
+    const size_t bytes = n2d2hip_batchnorm_f32_backward_sat_workspace_bytes((int)mIn->dimB(), (int)mNbOutputs, (int)mInH, (int)mInW);
     mWorkspace.resize({(bytes + sizeof(float) - 1) / sizeof(float), 1, 1, 1});
 }
 
@@ -611,7 +611,9 @@ void BatchNormCell_FrameTrain_HIP<T>::backPropagate()
         return;
     if (!mLearned)
         throw std::runtime_error("BatchNormCell_FrameTrain_HIP " + mName + ": backPropagate() needs the batch statistics of a learning propagate()");
-    activationBackPropagate();
+    const std::shared_ptr<SATQuantizerActivation_Frame_HIP<float> > sat = lonelySatQuantizer();
+    if (!sat)
+        activationBackPropagate();
     const float betaScale = mScaleSolver->isNewIteration() ? 0.0f : 1.0f;
     const float betaBias = mBiasSolver->isNewIteration() ? 0.0f : 1.0f;
     const bool toInput = mDiffOut && !mDiffOut->empty();
@@ -622,10 +624,19 @@ void BatchNormCell_FrameTrain_HIP<T>::backPropagate()
     if (accumulate && mDiffOwn.size() != mDiffOut->size())
         mDiffOwn.resize(mDiffOut->dims());
     float* dst = !toInput ? nullptr : accumulate ? mDiffOwn.data() : mDiffOut->data();
-    checkStatus(n2d2hip_batchnorm_f32_backward((int)mIn->dimB(), (int)mNbOutputs, (int)mInH, (int)mInW, mIn->data(), mScale.data(), mSavedMean.data(),
-                                               mSavedVariance.data(), mEpsilon, mDiffInputs.data(), betaScale, mDiffScale.data(), betaBias,
-                                               mDiffBias.data(), mDiffSavedMean.data(), mDiffSavedVariance.data(), dst,
-                                               mWorkspace.data(), mWorkspace.size() * sizeof(float), mStream));
+    if (sat) {
+        const auto to = sat->prepareGradient(mDiffInputs.size());
+        checkStatus(n2d2hip_batchnorm_f32_backward_sat((int)mIn->dimB(), (int)mNbOutputs, (int)mInH, (int)mInW, mIn->data(), mScale.data(),
+                                                       mSavedMean.data(), mSavedVariance.data(), mEpsilon, to.fullPrecision, to.range, to.alpha, to.beta,
+                                                       to.diffAlpha, mDiffInputs.data(), betaScale, mDiffScale.data(), betaBias, mDiffBias.data(),
+                                                       mDiffSavedMean.data(), mDiffSavedVariance.data(), dst, mWorkspace.data(),
+                                                       mWorkspace.size() * sizeof(float), mStream));
+    } else {
+        checkStatus(n2d2hip_batchnorm_f32_backward((int)mIn->dimB(), (int)mNbOutputs, (int)mInH, (int)mInW, mIn->data(), mScale.data(), mSavedMean.data(),
+                                                   mSavedVariance.data(), mEpsilon, mDiffInputs.data(), betaScale, mDiffScale.data(), betaBias,
+                                                   mDiffBias.data(), mDiffSavedMean.data(), mDiffSavedVariance.data(), dst,
+                                                   mWorkspace.data(), mWorkspace.size() * sizeof(float), mStream));
+    }
     if (accumulate)
         checkStatus(n2d2hip_elemwise_sum_f32_backward(mDiffOut->size(), 1.0f, mDiffOwn.data(), 1.0f, mDiffOut->data(), mStream));
     if (toInput)

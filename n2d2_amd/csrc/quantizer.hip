@@ -352,13 +352,8 @@ __global__ __launch_bounds__(QBLOCK) void sat_act_backward_kernel(const float* d
         quad_load<N>(g, dy, i);
 #pragma unroll
         for (int j = 0; j < N; ++j) {
-            const float xc = (x[j] < 0.0f) ? 0.0f : (x[j] < a) ? x[j] : a;
-            const float q = xc / a;
-            const float qd = round_half_away(__fmul_rn(range, q)) / range;
-            const float dqa = (x[j] >= a) ? 1.0f : __fsub_rn(qd, q);
-            s += (double)__fmul_rn(dqa, g[j]);
-            const float dact = (x[j] <= 0.0f) ? 0.0f : (x[j] > a) ? 0.0f : 1.0f;
-            d[j] = __fmul_rn(dact, g[j]);
+            s += (double)__fmul_rn(sat_alpha_slope(x[j], range, a), g[j]);
+            d[j] = __fmul_rn(sat_input_slope(x[j], a), g[j]);
         }
         quad_store<N>(dx, i, d);
     });

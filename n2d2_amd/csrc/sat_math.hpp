@@ -15,5 +15,14 @@ __device__ __forceinline__ float sat_quantize(float v, float range, float a)
     q = round_half_away(__fmul_rn(range, q)) / range;
     return __fmul_rn(q, a);
 }
+// Its derivatives by alpha and by its input, ref: SATQuantizer_Frame_Kernels.cpp:410-448
+__device__ __forceinline__ float sat_alpha_slope(float v, float range, float a)
+{
+    const float xc = (v < 0.0f) ? 0.0f : (v < a) ? v : a;
+    const float q = xc / a;
+    const float qd = round_half_away(__fmul_rn(range, q)) / range;
+    return (v >= a) ? 1.0f : __fsub_rn(qd, q);
+}
+__device__ __forceinline__ float sat_input_slope(float v, float a) { return (v <= 0.0f) ? 0.0f : (v > a) ? 0.0f : 1.0f; }
 
 } // namespace n2d2hip

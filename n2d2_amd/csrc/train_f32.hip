@@ -635,21 +635,55 @@ __device__ __forceinline__ void bn_write_grads(int c, const double* t, float dme
     o.diff_scale[c] = sum_scale + (o.beta_scale != 0.0f ? o.beta_scale * o.diff_scale[c] : 0.0f);
     o.diff_bias[c] = sum_bias + (o.beta_bias != 0.0f ? o.beta_bias * o.diff_bias[c] : 0.0f);
 }
-template <int V>
+// The SAT activation quantizer behind a normalisation, backwards: fp what went into it, alpha's gradient summed by block (partial,
+// a value for each block of the sums) and finished by the launch that follows; alpha null: no quantizer
+struct BnSatGrad {
+    const float* fp;
+    float range;
+    const float* alpha;
+    double* partial;
+    int blocks;
+    float beta;
+    float* diff_alpha;
+};
+// (one block: the sum of the blocks' values + beta times what was there)
+__device__ __forceinline__ void bn_finish_alpha(const BnSatGrad& sat)
+{
+    double t[1] = {};
+    for (int i = threadIdx.x; i < sat.blocks; i += TBLOCK) t[0] += sat.partial[i];
+    bn_block_sums<1>(t);
+    if (threadIdx.x == 0) sat.diff_alpha[0] = (float)t[0] + (sat.beta != 0.0f ? sat.beta * sat.diff_alpha[0] : 0.0f);
+}
+__global__ __launch_bounds__(TBLOCK) void batchnorm_f32_alpha_kernel(BnSatGrad sat) { bn_finish_alpha(sat); }
+
+// SAT: dy is first taken through the quantizer's gradient, in place (64 x 64 x 32 x 32, us: the quantizer's own pass 10.0, its end
+// 4.6 and the sums 9.8; together 19.2)
+template <int V, bool SAT>
 __global__ __launch_bounds__(1024) void batchnorm_f32_backward_sums_kernel(BnRange q, double n, const float* __restrict__ x,
                                                                            const float* __restrict__ scale, const float* __restrict__ saved_mean,
                                                                            const float* __restrict__ saved_variance, double epsilon,
-                                                                           const float* __restrict__ dy, double* __restrict__ ws, BnGrads grads)
+                                                                           float* __restrict__ dy, double* __restrict__ ws, BnGrads grads, BnSatGrad sat)
 {
     constexpr int N = V ? V : 1;
     const int c = blockIdx.x;
     const float m = saved_mean[c], g = scale[c];
     const float var = (float)sqrt((double)saved_variance[c] + epsilon);
-    double t[5] = {};
+    const float a = SAT ? fabsf(sat.alpha[0]) : 0.0f;
+    double t[SAT ? 6 : 5] = {};
     bn_walk<V>(q, c, [&](size_t idx) {
         float xv[N], dv[N];
         bn_load<N>(xv, x, idx);
         bn_load<N>(dv, dy, idx);
+        if (SAT) {
+            float fp[N];
+            bn_load<N>(fp, sat.fp, idx);
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                t[5] += (double)__fmul_rn(sat_alpha_slope(fp[k], sat.range, a), dv[k]);
+                dv[k] = __fmul_rn(sat_input_slope(fp[k], a), dv[k]);
+            }
+            bn_store<N>(dy, idx, dv);
+        }
 #pragma unroll
         for (int k = 0; k < N; ++k) {
             const float centred = xv[k] - m;
@@ -662,8 +696,9 @@ __global__ __launch_bounds__(1024) void batchnorm_f32_backward_sums_kernel(BnRan
             t[4] += (double)(diff_normalized * centred);
         }
     });
-    bn_block_sums<5>(t);
+    bn_block_sums<SAT ? 6 : 5>(t);
     if (threadIdx.x) return;
+    if (SAT) sat.partial[(size_t)c * gridDim.y + blockIdx.y] = t[5];
     if (gridDim.y == 1) {
         float dmean, dvariance;
         bn_stats_grads(n, t, saved_variance[c], epsilon, &dmean, &dvariance);
@@ -696,9 +731,13 @@ template <int V>
 __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_backward_data_kernel(BnRange q, int splits, double n, const double* __restrict__ ws, float size,
                                                                             const float* __restrict__ x, const float* __restrict__ scale,
                                                                             const float* __restrict__ saved_mean, const float* __restrict__ saved_variance,
-                                                                            double epsilon, const float* dy, BnGrads grads, float* dx)
+                                                                            double epsilon, const float* dy, BnGrads grads, BnSatGrad sat, float* dx)
 {
     const int c = blockIdx.x;
+    if (sat.alpha && blockIdx.x == 0 && blockIdx.y == gridDim.y - 1) {
+        bn_finish_alpha(sat);
+        __syncthreads();
+    }
     float dmean, dvariance;
     if (splits > 1) {
         __shared__ float of_stats[2];
@@ -738,8 +777,9 @@ __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_backward_data_flat_kerne
                                                                             const float* __restrict__ scale, const float* __restrict__ saved_mean,
                                                                             const float* __restrict__ saved_variance, double epsilon, const float* dy,
                                                                             const float* __restrict__ diff_saved_mean,
-                                                                            const float* __restrict__ diff_saved_variance, float* dx)
+                                                                            const float* __restrict__ diff_saved_variance, BnSatGrad sat, float* dx)
 {
+    if (sat.alpha && blockIdx.x == 0) bn_finish_alpha(sat);
     for (size_t i = (size_t)blockIdx.x * TBLOCK + threadIdx.x; i < total; i += (size_t)gridDim.x * TBLOCK) {
         const int c = (int)((i / plane) % C);
         const float var = (float)sqrt((double)saved_variance[c] + epsilon);
@@ -1524,16 +1564,20 @@ int n2d2hip_rectifier_f32_backward(const float* output, const float* diff_in, fl
     return N2D2HIP_OK;
 }
 
-// Blocks per channel for the sums over batch and pixels: about 1024 blocks in all, at least 4096 values each, at most 64.
+// Planes below 64 values (a channel's values of one image are less than a cache line or two) are written value by value, others
+// channel by channel, with the sums' end
+constexpr int BN_WALK_PLANE = 64;
+// Blocks per channel for the sums over batch and pixels: one below 8192 values; then about 1024 blocks in all, at most 64, of at
+// least 1024 values each, or 4096 where their end is a launch of its own.
 static int bn_splits(int B, int C, int H, int W)
 {
     const size_t n = (size_t)B * H * W;
-    const size_t by_size = n / 4096;
+    const size_t by_size = n < 8192 ? 1 : n / ((size_t)H * W >= BN_WALK_PLANE ? 1024 : 4096);
     const size_t by_grid = (size_t)std::max(1024 / C, 1);
     return (int)std::max<size_t>(1, std::min<size_t>(std::min(by_size, by_grid), 64));
 }
 
-// Units of 16 bytes where the planes allow it; a block of 1024 threads where one of 256 would go round more than four times
+// Units of 16 bytes where the planes allow it; a block of 1024 threads where one of 256 would go round more than twice
 struct BnLaunch {
     BnRange q;
     int V, block;
@@ -1546,7 +1590,7 @@ static BnLaunch bn_launch(int B, int C, int plane, int splits, uintptr_t pointer
     if (n / l.V >= ((size_t)1 << 30)) l.V = 0;
     const int v = l.V ? l.V : 1;
     l.q = {C, plane, plane / v, div_of(plane / v), n / v, (n / v + splits - 1) / splits};
-    l.block = splits == 1 && l.q.units > 4 * TBLOCK ? 1024 : TBLOCK;
+    l.block = splits == 1 && l.q.units > 2 * TBLOCK ? 1024 : TBLOCK;
     return l;
 }
 
@@ -1557,9 +1601,7 @@ size_t n2d2hip_batchnorm_f32_workspace_bytes(int B, int C, int H, int W)
     return (size_t)C * bn_splits(B, C, H, W) * 5 * sizeof(double);
 }
 
-// Blocks a channel for the passes that write a tensor: about 2048 in all, none for less than a value or quad a thread.  Planes below
-// 64 values (a channel's values of one image are less than a cache line or two) go value by value instead.
-constexpr int BN_WALK_PLANE = 64;
+// Blocks a channel for the passes that write a tensor: about 2048 in all, none for less than a value or quad a thread
 static int bn_ranges(int B, int C, int plane, int V)
 {
     const size_t blocks = ((size_t)B * plane / std::max(V, 1) + TBLOCK - 1) / TBLOCK;
@@ -1625,41 +1667,81 @@ int n2d2hip_batchnorm_f32_forward_sat(int B, int C, int H, int W, const float* x
                              moving_average_momentum, use_running, y, BnSat{full_precision, range, alpha}, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
+size_t n2d2hip_batchnorm_f32_backward_sat_workspace_bytes(int B, int C, int H, int W)
+{
+    if (B <= 0 || C <= 0 || H <= 0 || W <= 0)
+        return 0;
+    return (size_t)C * bn_splits(B, C, H, W) * 6 * sizeof(double);
+}
+
+static int batchnorm_backward(const char* who, int B, int C, int H, int W, const float* x, const float* scale, const float* saved_mean,
+                              const float* saved_variance, double epsilon, BnSatGrad sat, float* diff_y, const BnGrads& grads, float* diff_x,
+                              void* workspace, int splits, hipStream_t stream)
+{
+    N2D2HIP_REQUIRE(B > 0 && C > 0 && H > 0 && W > 0 && x && scale && saved_mean && saved_variance && diff_y && grads.diff_scale && grads.diff_bias
+                        && grads.diff_saved_mean && grads.diff_saved_variance && epsilon > 0.0,
+                    N2D2HIP_ERR_INVALID, "%s: bad argument", who);
+    N2D2HIP_REQUIRE((size_t)B * C < ((size_t)1 << 31) && (size_t)H * W < ((size_t)1 << 31), N2D2HIP_ERR_INVALID, "%s: tensor too large", who);
+    const double n = (double)B * H * W;
+    const int plane = H * W;
+    const uintptr_t in = (uintptr_t)x | (uintptr_t)diff_y;
+    const BnLaunch l = bn_launch(B, C, plane, splits, in | (uintptr_t)sat.fp);
+    sat.partial = (double*)workspace + (size_t)C * splits * 5;
+    sat.blocks = C * splits;
+    const auto kernel = sat.alpha ? (l.V == 4 ? batchnorm_f32_backward_sums_kernel<4, true> : l.V == 1 ? batchnorm_f32_backward_sums_kernel<1, true>
+                                                                                                : batchnorm_f32_backward_sums_kernel<0, true>)
+                                  : (l.V == 4 ? batchnorm_f32_backward_sums_kernel<4, false> : l.V == 1 ? batchnorm_f32_backward_sums_kernel<1, false>
+                                                                                                 : batchnorm_f32_backward_sums_kernel<0, false>);
+    hipLaunchKernelGGL(kernel, dim3(C, splits), dim3(l.block), 0, stream, l.q, n, x, scale, saved_mean, saved_variance, epsilon, diff_y, (double*)workspace,
+                       grads, sat);
+    const int V = bn_launch(B, C, plane, 1, in | (uintptr_t)diff_x).V;
+    const bool walk = diff_x && plane >= BN_WALK_PLANE && V != 0;
+    if (splits > 1 && !walk)
+        hipLaunchKernelGGL(batchnorm_f32_backward_finish_kernel, dim3(C), dim3(64), 0, stream, n, splits, (const double*)workspace, saved_variance, epsilon,
+                           grads);
+    if (walk) {
+        const int ranges = bn_ranges(B, C, plane, V);
+        const BnLaunch d = bn_launch(B, C, plane, ranges, in | (uintptr_t)diff_x);
+        hipLaunchKernelGGL(V == 4 ? batchnorm_f32_backward_data_kernel<4> : batchnorm_f32_backward_data_kernel<1>, dim3(C, ranges), dim3(TBLOCK), 0, stream,
+                           d.q, splits, n, (const double*)workspace, (float)((size_t)B * H * W), x, scale, saved_mean, saved_variance, epsilon, diff_y, grads,
+                           sat, diff_x);
+    } else if (diff_x)
+        hipLaunchKernelGGL(batchnorm_f32_backward_data_flat_kernel, dim3(grid_for((size_t)B * C * plane)), dim3(TBLOCK), 0, stream, (size_t)B * C * plane, C,
+                           plane, (float)((size_t)B * H * W), x, scale, saved_mean, saved_variance, epsilon, diff_y, (const float*)grads.diff_saved_mean,
+                           (const float*)grads.diff_saved_variance, sat, diff_x);
+    else if (sat.alpha)
+        hipLaunchKernelGGL(batchnorm_f32_alpha_kernel, dim3(1), dim3(TBLOCK), 0, stream, sat);
+    N2D2HIP_HIP_CHECK(hipGetLastError());
+    return N2D2HIP_OK;
+}
+
 int n2d2hip_batchnorm_f32_backward(int B, int C, int H, int W, const float* x, const float* scale, const float* saved_mean,
                                    const float* saved_variance, double epsilon, const float* diff_y, float beta_scale, float* diff_scale,
                                    float beta_bias, float* diff_bias, float* diff_saved_mean, float* diff_saved_variance, float* diff_x,
                                    void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream)
 {
-    N2D2HIP_REQUIRE(B > 0 && C > 0 && H > 0 && W > 0 && x && scale && saved_mean && saved_variance && diff_y && diff_scale && diff_bias
-                        && diff_saved_mean && diff_saved_variance && epsilon > 0.0,
-                    N2D2HIP_ERR_INVALID, "n2d2hip_batchnorm_f32_backward: bad argument");
-    N2D2HIP_REQUIRE((size_t)B * C < ((size_t)1 << 31) && (size_t)H * W < ((size_t)1 << 31), N2D2HIP_ERR_INVALID,
-                    "n2d2hip_batchnorm_f32_backward: tensor too large");
-    const double n = (double)B * H * W;
-    const int plane = H * W;
+    const int splits = B > 0 && C > 0 && H > 0 && W > 0 && workspace && workspace_bytes >= n2d2hip_batchnorm_f32_workspace_bytes(B, C, H, W)
+                           ? bn_splits(B, C, H, W) : 1;
     const BnGrads grads = {diff_scale, diff_bias, diff_saved_mean, diff_saved_variance, beta_scale, beta_bias};
-    const int splits = workspace && workspace_bytes >= n2d2hip_batchnorm_f32_workspace_bytes(B, C, H, W) ? bn_splits(B, C, H, W) : 1;
-    const BnLaunch l = bn_launch(B, C, plane, splits, (uintptr_t)x | (uintptr_t)diff_y);
-    const auto kernel = l.V == 4 ? batchnorm_f32_backward_sums_kernel<4> : l.V == 1 ? batchnorm_f32_backward_sums_kernel<1> : batchnorm_f32_backward_sums_kernel<0>;
-    hipLaunchKernelGGL(kernel, dim3(C, splits), dim3(l.block), 0, (hipStream_t)stream, l.q, n, x, scale, saved_mean, saved_variance, epsilon, diff_y,
-                       (double*)workspace, grads);
-    const int V = bn_launch(B, C, plane, 1, (uintptr_t)x | (uintptr_t)diff_y | (uintptr_t)diff_x).V;
-    const bool walk = diff_x && plane >= BN_WALK_PLANE && V != 0;
-    if (splits > 1 && !walk)
-        hipLaunchKernelGGL(batchnorm_f32_backward_finish_kernel, dim3(C), dim3(64), 0, (hipStream_t)stream, n, splits, (const double*)workspace,
-                           saved_variance, epsilon, grads);
-    if (walk) {
-        const int ranges = bn_ranges(B, C, plane, V);
-        const BnLaunch d = bn_launch(B, C, plane, ranges, (uintptr_t)x | (uintptr_t)diff_y | (uintptr_t)diff_x);
-        hipLaunchKernelGGL(V == 4 ? batchnorm_f32_backward_data_kernel<4> : batchnorm_f32_backward_data_kernel<1>, dim3(C, ranges), dim3(TBLOCK), 0,
-                           (hipStream_t)stream, d.q, splits, n, (const double*)workspace, (float)((size_t)B * H * W), x, scale, saved_mean, saved_variance,
-                           epsilon, diff_y, grads, diff_x);
-    } else if (diff_x)
-        hipLaunchKernelGGL(batchnorm_f32_backward_data_flat_kernel, dim3(grid_for((size_t)B * C * plane)), dim3(TBLOCK), 0, (hipStream_t)stream,
-                           (size_t)B * C * plane, C, plane, (float)((size_t)B * H * W), x, scale, saved_mean, saved_variance, epsilon, diff_y,
-                           (const float*)diff_saved_mean, (const float*)diff_saved_variance, diff_x);
-    N2D2HIP_HIP_CHECK(hipGetLastError());
-    return N2D2HIP_OK;
+    // (without a quantizer diff_y is only read)
+    return batchnorm_backward("n2d2hip_batchnorm_f32_backward", B, C, H, W, x, scale, saved_mean, saved_variance, epsilon, BnSatGrad{},
+                              const_cast<float*>(diff_y), grads, diff_x, workspace, splits, (hipStream_t)stream);
+}
+
+int n2d2hip_batchnorm_f32_backward_sat(int B, int C, int H, int W, const float* x, const float* scale, const float* saved_mean,
+                                       const float* saved_variance, double epsilon, const float* full_precision, float range, const float* alpha,
+                                       float beta_alpha, float* diff_alpha, float* diff_y, float beta_scale, float* diff_scale, float beta_bias,
+                                       float* diff_bias, float* diff_saved_mean, float* diff_saved_variance, float* diff_x, void* workspace,
+                                       size_t workspace_bytes, n2d2hip_stream_t stream)
+{
+    N2D2HIP_REQUIRE(full_precision && alpha && diff_alpha && full_precision != diff_y && full_precision != diff_x, N2D2HIP_ERR_INVALID,
+                    "n2d2hip_batchnorm_f32_backward_sat: bad argument");
+    const size_t need = n2d2hip_batchnorm_f32_backward_sat_workspace_bytes(B, C, H, W);
+    N2D2HIP_REQUIRE(workspace && workspace_bytes >= need, N2D2HIP_ERR_WORKSPACE, "n2d2hip_batchnorm_f32_backward_sat: workspace of %zu bytes needed", need);
+    const BnGrads grads = {diff_scale, diff_bias, diff_saved_mean, diff_saved_variance, beta_scale, beta_bias};
+    return batchnorm_backward("n2d2hip_batchnorm_f32_backward_sat", B, C, H, W, x, scale, saved_mean, saved_variance, epsilon,
+                              BnSatGrad{full_precision, range, alpha, nullptr, 0, beta_alpha, diff_alpha}, diff_y, grads, diff_x, workspace,
+                              need ? bn_splits(B, C, H, W) : 1, (hipStream_t)stream);
 }
 
 static bool pool_small(const PoolF32& q) { return (size_t)q.B * q.C * std::max((size_t)q.H * q.W, (size_t)q.oH * q.oW) < ((size_t)1 << 31) - TBLOCK; }

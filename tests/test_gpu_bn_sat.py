@@ -70,3 +70,42 @@ def test_backward_finished_by_the_next_launch(shape, beta, to_input):
     # the sums are double on both sides and differ in their order only: one rounding to float apart
     for a, b in zip(*out):
         assert np.max(np.abs(a - b)) <= 4 * 2.0 ** -24 * max(1.0, np.max(np.abs(a)))
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("beta", [0.0, 1.0])
+@pytest.mark.parametrize("to_input", [False, True])
+def test_quantizer_gradient_on_the_way_in(shape, beta, to_input):
+    """The quantizer's gradient taken by the normalisation's sums against the two calls: the same bits but for alpha's gradient,
+    whose double sum has another order."""
+    import torch
+    from n2d2_amd import capi, runtime as rt
+    print("bn sat backward", shape, beta, to_input, flush=True)
+    B, C, H, W = shape
+    n = B * C * H * W
+    lib, rng = capi.lib, np.random.default_rng(B * C + H)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).cuda()
+    x, dy, fp, alpha = dev(rng.normal(1, 2, shape)), dev(rng.normal(0, 1, shape)), dev(rng.normal(0.8, 1, shape)), dev([1.7])
+    scale, m, v = dev(rng.normal(1, .3, C)), dev(rng.normal(1, .1, C)), dev(rng.uniform(3, 5, C))
+    ws = torch.empty(int(lib.n2d2hip_batchnorm_f32_backward_sat_workspace_bytes(B, C, H, W)), dtype=torch.uint8, device="cuda")
+    qws = torch.empty(int(lib.n2d2hip_quantizer_workspace_bytes(n)), dtype=torch.uint8, device="cuda")
+    out = []
+    for fused in (False, True):
+        g = [dev(np.full(C, 0.25)) for _ in range(4)]
+        d, dx, da = dy.clone(), torch.full_like(dy, 9.0), dev([0.5])
+        head = [B, C, H, W, x.data_ptr(), scale.data_ptr(), m.data_ptr(), v.data_ptr(), 1e-4]
+        tail = [beta, g[0].data_ptr(), beta, g[1].data_ptr(), g[2].data_ptr(), g[3].data_ptr(), dx.data_ptr() if to_input else None, ws.data_ptr(), ws.numel(),
+                rt.stream_ptr()]
+        if fused:
+            capi.check(lib.n2d2hip_batchnorm_f32_backward_sat(*head, fp.data_ptr(), 15.0, alpha.data_ptr(), beta, da.data_ptr(), d.data_ptr(), *tail))
+        else:
+            capi.check(lib.n2d2hip_sat_act_backward(d.data_ptr(), fp.data_ptr(), d.data_ptr(), n, 15.0, alpha.data_ptr(), beta, da.data_ptr(),
+                                                    qws.data_ptr(), qws.numel(), rt.stream_ptr()))
+            capi.check(lib.n2d2hip_batchnorm_f32_backward(*head, d.data_ptr(), *tail))
+        out.append([t.cpu().numpy() for t in (*g, d, dx, da)])
+    for a, b in zip(out[0][:-1], out[1][:-1]):
+        assert np.array_equal(a, b)
+    # one rounding to float apart (and one more where beta adds what was there)
+    assert abs(out[0][-1][0] - out[1][-1][0]) <= 2 * 2.0 ** -23 * max(1.0, abs(out[0][-1][0]))
+    assert lib.n2d2hip_batchnorm_f32_backward_sat(*head, fp.data_ptr(), 15.0, alpha.data_ptr(), beta, da.data_ptr(), d.data_ptr(), *tail[:-3], None, 0,
+                                                  rt.stream_ptr()) == capi.ERR_WORKSPACE
