@@ -308,11 +308,35 @@ __global__ __launch_bounds__(TBLOCK) void conv_f32_backward_bias_kernel(int B, i
 }
 
 // Softmax over the channels of each pixel: exp(x - max) / sum, zeros if the sum is not positive.
+// Bound by its chain of loads where there are few pixels and by reading x three times where there are many. N: channels held in
+// registers, at least C, loaded once and all before the first is waited for; 0: any number, read in three loops. Measured, loops ->
+// registers: 32 images of 10 classes 5.1 -> 3.4 us, 16 maps of 512 x 512 with 2 / 4 / 10 / 16 channels 21.0 -> 20.6, 39.5 -> 26.3,
+// 136.5 -> 60.7, 237.5 -> 100.7 us.
+template <int N>
 __global__ __launch_bounds__(TBLOCK) void softmax_f32_kernel(const float* __restrict__ x, float* __restrict__ y, int B, int C, int plane)
 {
     const size_t total = (size_t)B * plane;
     for (size_t idx = (size_t)blockIdx.x * TBLOCK + threadIdx.x; idx < total; idx += (size_t)gridDim.x * TBLOCK) {
         const size_t base = (idx / plane) * (size_t)C * plane + idx % plane;
+        if (N) {
+            float v[N ? N : 1];
+#pragma unroll
+            for (int c = 0; c < N; ++c) v[c] = x[base + (size_t)(c < C ? c : 0) * plane];
+            float m = v[0];
+#pragma unroll
+            for (int c = 1; c < N; ++c) m = fmaxf(m, v[c]);                  // (past C: the first again)
+            float s = 0.0f;
+#pragma unroll
+            for (int c = 0; c < N; ++c) {
+                if (c >= C) break;
+                v[c] = expf(v[c] - m);
+                s += v[c];
+            }
+#pragma unroll
+            for (int c = 0; c < N; ++c)
+                if (c < C) y[base + (size_t)c * plane] = s > 0.0f ? v[c] / s : 0.0f;
+            continue;
+        }
         float m = x[base];
         for (int c = 1; c < C; ++c) m = fmaxf(m, x[base + (size_t)c * plane]);
         float s = 0.0f;
@@ -323,7 +347,7 @@ __global__ __launch_bounds__(TBLOCK) void softmax_f32_kernel(const float* __rest
 
 // diff = target - output, formed in double; partial[block] = sum of squares (double).
 __global__ __launch_bounds__(TBLOCK) void loss_f32_kernel(const float* target, const float* __restrict__ out, float* diff,
-                                                          size_t n, double* __restrict__ partial)
+                                                          size_t n, double* __restrict__ partial, double inv_batch, double* __restrict__ loss)
 {
     double acc = 0.0;
     for (size_t i = (size_t)blockIdx.x * TBLOCK + threadIdx.x; i < n; i += (size_t)gridDim.x * TBLOCK) {
@@ -332,8 +356,13 @@ __global__ __launch_bounds__(TBLOCK) void loss_f32_kernel(const float* target, c
         acc += e * e;
     }
     acc = block_sum_d(acc);
-    if (threadIdx.x == 0) partial[blockIdx.x] = acc;
+    if (threadIdx.x) return;
+    if (gridDim.x == 1) loss[0] = acc * inv_batch;
+    else partial[blockIdx.x] = acc;
 }
+// Up to this many values one block goes over all of them and writes the loss itself, instead of a second launch that adds the blocks'
+// partial sums: 320 / 2560 / 4096 values 3.9 / 4.0 / 4.0 us against 6.3 / 7.1 / 6.9 in two launches.
+constexpr size_t LOSS_ONE_BLOCK = 4096;
 __global__ __launch_bounds__(TBLOCK) void loss_finish_kernel(const double* __restrict__ partial, int nb, double inv_batch, double* __restrict__ loss)
 {
     double acc = 0.0;
@@ -1541,7 +1570,7 @@ int n2d2hip_conv2d_f32_backward_bias(int B, int O, int oH, int oW, const float* 
 int n2d2hip_softmax_f32_forward(const float* x, float* y, int B, int C, int H, int W, n2d2hip_stream_t stream)
 {
     N2D2HIP_REQUIRE(B > 0 && C > 0 && H > 0 && W > 0 && x && y, N2D2HIP_ERR_INVALID, "n2d2hip_softmax_f32_forward: bad argument");
-    hipLaunchKernelGGL(softmax_f32_kernel, dim3(grid_for((size_t)B * H * W)), dim3(TBLOCK), 0, (hipStream_t)stream, x, y, B, C, H * W);
+    hipLaunchKernelGGL(C <= 16 ? softmax_f32_kernel<16> : softmax_f32_kernel<0>, dim3(grid_for((size_t)B * H * W)), dim3(TBLOCK), 0, (hipStream_t)stream, x, y, B, C, H * W);
     N2D2HIP_HIP_CHECK(hipGetLastError());
     return N2D2HIP_OK;
 }
@@ -1995,8 +2024,10 @@ int n2d2hip_loss_f32(const float* target, const float* output, float* diff, size
     const int nb = grid_for(n);
     N2D2HIP_REQUIRE(workspace && workspace_bytes >= (size_t)nb * sizeof(double), N2D2HIP_ERR_WORKSPACE,
                     "n2d2hip_loss_f32: workspace of %zu bytes, %zu needed", workspace_bytes, (size_t)nb * sizeof(double));
-    hipLaunchKernelGGL(loss_f32_kernel, dim3(nb), dim3(TBLOCK), 0, (hipStream_t)stream, target, output, diff, n, (double*)workspace);
-    hipLaunchKernelGGL(loss_finish_kernel, dim3(1), dim3(TBLOCK), 0, (hipStream_t)stream, (const double*)workspace, nb, 1.0 / batch, loss);
+    const int blocks = n <= LOSS_ONE_BLOCK ? 1 : nb;
+    hipLaunchKernelGGL(loss_f32_kernel, dim3(blocks), dim3(TBLOCK), 0, (hipStream_t)stream, target, output, diff, n, (double*)workspace, 1.0 / batch, loss);
+    if (blocks > 1)
+        hipLaunchKernelGGL(loss_finish_kernel, dim3(1), dim3(TBLOCK), 0, (hipStream_t)stream, (const double*)workspace, blocks, 1.0 / batch, loss);
     N2D2HIP_HIP_CHECK(hipGetLastError());
     return N2D2HIP_OK;
 }
