@@ -59,10 +59,11 @@ namespace {
 enum { DWT_W, DWT_CE = 3, DWT_D, DWT_BIAS, DWT_A, DWT_B, DWT_USED, DWT_ROWS = 8 };
 
 // 16 bytes a lane from its own address to 16 * lane bytes past LDS offset `lds`, which is the same in all lanes.  As text,
-// because the compiler would wait for every such load of the wave before the next LDS read of any buffer.
+// because the compiler would wait for every such load of the wave before the next LDS read of any buffer.  m0, which holds the
+// offset, is an operand: the compiler writes it and knows what is in it.
 __device__ __forceinline__ void load_to_lds(const void* src, unsigned lds)
 {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "{m0}"(lds) : "memory");
 }
 
 // (acc * c + d) >> e of the rescales on 32 bits.  acc comes from an instruction of the compiler's: it waits for a matrix
