@@ -588,13 +588,42 @@ __global__ __launch_bounds__(256) void conv_f32_3x3_kernel(PixelGemm g, const fl
 
 // A layer that spans its input, forward, in the reference's order of terms: y[b][o] = sum over k of x[b][k] w[o][k], one
 // after the other in float.  The chain of additions is what takes the time: a wave alone on its SIMD issues an instruction in
-// about 8 cycles, an addition no sooner than the one before it, so everything else is kept off that wave.  A block is 8 images
-// x 8 outputs and three waves: two load the operands (16 rows, in LDS two stages of 256 terms ahead), multiply them, 64 terms of
-// 128 each, and leave the products in LDS; the third reads those a step later and only adds.  16384 -> 10, 64 images: 117 us
-// with one wave that did all (2632 before that), now 90: additions and their reads, an instruction in 8 cycles.  (One wave with
-// the products of the next 32 terms between its additions: 130.  Steps of 64 terms: 95, and the same up to 1600 terms.)
+// about 8 cycles, an addition no sooner than the one before it.  A block is 8 images x 8 outputs in both kernels, its 16 rows of
+// operands in LDS two stages of 256 terms ahead; which of the two is the faster depends on how many blocks there are:
+//  * Up to one a compute unit, conv_f32_chain_kernel: everything but the additions is kept off the wave that does them.  Two waves
+//    load the operands, multiply them, 64 terms of 128 each, and leave the products in LDS; the third reads those a step later and
+//    only adds, 5.5 ns a term.  (One wave with the products of the next 32 terms between its additions: 130 us where this takes 90.
+//    Steps of 64 terms: 95, and the same up to 1600 terms.)
+//  * More, conv_f32_chain_wave_kernel: one wave multiplies and adds, 7.1 ns a term, but its 49 KB let three blocks share a unit
+//    where the other kernel's 115 KB let one.
+// us, conv_f32_chain_kernel / conv_f32_chain_wave_kernel (images x outputs, blocks, terms): 64 x 10, 16, 16384 88.8 / 116.3; 40 x 400,
+// 250, 25088 140.5 / 178.1; 128 x 120, 240, 400 5.8 / 5.4; 144 x 120, 270, 400 9.7 / 5.8; 192 x 96, 288, 1024 13.7 / 10.4; 48 x 400, 300,
+// 25088 272.5 / 198.7; 256 x 120, 480, 400 9.9 / 5.9; 64 x 1000, 1000, 25088 552.5 / 381.1; 1024 x 120, 1920, 400 35.0 / 14.5.
 constexpr int CHAIN_K = 256, CHAIN_ROW = CHAIN_K + 4, CHAIN_STAGES = 3;      // (rows 16 bytes apart in the banks)
 constexpr int CHAIN_T = 128, CHAIN_PROD = CHAIN_T + 4;                        // terms between two barriers; a lane's row of products
+
+// 32 terms of an image's row and of an output's, from OFF bytes on
+template <int OFF>
+__device__ __forceinline__ void chain_read(v4f (&xv)[8], v4f (&wv)[8], unsigned xa, unsigned wa)
+{
+    lds_read128f<OFF>(xv[0], xa); lds_read128f<OFF>(wv[0], wa);
+    lds_read128f<OFF + 16>(xv[1], xa); lds_read128f<OFF + 16>(wv[1], wa);
+    lds_read128f<OFF + 32>(xv[2], xa); lds_read128f<OFF + 32>(wv[2], wa);
+    lds_read128f<OFF + 48>(xv[3], xa); lds_read128f<OFF + 48>(wv[3], wa);
+    lds_read128f<OFF + 64>(xv[4], xa); lds_read128f<OFF + 64>(wv[4], wa);
+    lds_read128f<OFF + 80>(xv[5], xa); lds_read128f<OFF + 80>(wv[5], wa);
+    lds_read128f<OFF + 96>(xv[6], xa); lds_read128f<OFF + 96>(wv[6], wa);
+    lds_read128f<OFF + 112>(xv[7], xa); lds_read128f<OFF + 112>(wv[7], wa);
+}
+__device__ __forceinline__ void chain_store(int B, int O, int b, int o, float sum, const float* __restrict__ bias, float beta, float* __restrict__ y)
+{
+    if (b >= B || o >= O) return;
+    const size_t idx = (size_t)b * O + o;
+    float r = sum + (beta != 0.0f ? beta * y[idx] : 0.0f);
+    if (bias) r = bias[o] + r;
+    y[idx] = r;
+}
+
 __global__ __launch_bounds__(192) void conv_f32_chain_kernel(int B, int O, int K, const float* __restrict__ x, const float* __restrict__ w,
                                                              const float* __restrict__ bias, float beta, float* __restrict__ y)
 {
@@ -630,22 +659,11 @@ __global__ __launch_bounds__(192) void conv_f32_chain_kernel(int B, int O, int K
             float* const to = out + (t & 1) * 64 * CHAIN_PROD;
             v4f xv[2][8], wv[2][8];
             const unsigned xa = src + 4u * bi * CHAIN_ROW, wa = src + 4u * (8 + oi) * CHAIN_ROW;
-            const auto read = [&](auto half) {
-                constexpr int h = decltype(half)::value, o = 128 * h;
-                lds_read128f<o>(xv[h][0], xa); lds_read128f<o>(wv[h][0], wa);
-                lds_read128f<o + 16>(xv[h][1], xa); lds_read128f<o + 16>(wv[h][1], wa);
-                lds_read128f<o + 32>(xv[h][2], xa); lds_read128f<o + 32>(wv[h][2], wa);
-                lds_read128f<o + 48>(xv[h][3], xa); lds_read128f<o + 48>(wv[h][3], wa);
-                lds_read128f<o + 64>(xv[h][4], xa); lds_read128f<o + 64>(wv[h][4], wa);
-                lds_read128f<o + 80>(xv[h][5], xa); lds_read128f<o + 80>(wv[h][5], wa);
-                lds_read128f<o + 96>(xv[h][6], xa); lds_read128f<o + 96>(wv[h][6], wa);
-                lds_read128f<o + 112>(xv[h][7], xa); lds_read128f<o + 112>(wv[h][7], wa);
-            };
-            read(std::integral_constant<int, 0>{});
+            chain_read<0>(xv[0], wv[0], xa, wa);
             wait_lgkm<0>();
 #pragma unroll
             for (int i = 0; i < 8; ++i) { tie(xv[0][i]); tie(wv[0][i]); }
-            read(std::integral_constant<int, 1>{});
+            chain_read<128>(xv[1], wv[1], xa, wa);
 #pragma unroll
             for (int i = 0; i < 8; ++i) *(v4f*)(to + 4 * i) = wv[0][i] * xv[0][i];
             wait_lgkm<0>();
@@ -705,12 +723,71 @@ __global__ __launch_bounds__(192) void conv_f32_chain_kernel(int B, int O, int K
         add(std::integral_constant<int, 3>{});
         __builtin_amdgcn_sched_barrier(0);
     }
-    const int b = b0 + bi, o = o0 + oi;
-    if (b >= B || o >= O) return;
-    const size_t idx = (size_t)b * O + o;
-    float r = sum + (beta != 0.0f ? beta * y[idx] : 0.0f);
-    if (bias) r = bias[o] + r;
-    y[idx] = r;
+    chain_store(B, O, b0 + bi, o0 + oi, sum, bias, beta, y);
+}
+
+__global__ __launch_bounds__(64) void conv_f32_chain_wave_kernel(int B, int O, int K, const float* __restrict__ x, const float* __restrict__ w,
+                                                                 const float* __restrict__ bias, float beta, float* __restrict__ y)
+{
+    __shared__ __attribute__((aligned(16))) float smem[CHAIN_STAGES * 16 * CHAIN_ROW];
+    const int lane = threadIdx.x, bi = lane >> 3, oi = lane & 7, b0 = blockIdx.x * 8, o0 = blockIdx.y * 8;
+    const __amdgpu_buffer_rsrc_t rsrcX = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x + (size_t)b0 * K), 0, min(8, B - b0) * K * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrcW = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(w + (size_t)o0 * K), 0, min(8, O - o0) * K * 4, 0x00020000);
+    int soff = 0;
+    unsigned dst = 0;
+    auto load = [&]() {                          // (terms past a row: zeros, or of the next row; rows past the last: zeros; not used)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcX, (lds_ptr_t)((char*)smem + dst + r * CHAIN_ROW * 4), 16, lane * 16, soff + r * K * 4, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcW, (lds_ptr_t)((char*)smem + dst + (r + 8) * CHAIN_ROW * 4), 16, lane * 16, soff + r * K * 4, 0, 0);
+        }
+        soff += CHAIN_K * 4;
+        dst = dst == (CHAIN_STAGES - 1) * 16u * CHAIN_ROW * 4u ? 0u : dst + 16u * CHAIN_ROW * 4u;
+    };
+    const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) float*)smem;
+    const unsigned xrow = lds0 + 4u * bi * CHAIN_ROW, wrow = lds0 + 4u * (8 + oi) * CHAIN_ROW;
+    const int full = K / 32, rest = K % 32, groups = full + (rest > 0);
+    v4f xv[2][8], wv[2][8];                      // 32 terms each: those that are added, the next ones
+    unsigned src = 0;
+    float sum = 0.0f;
+    auto group = [&](auto bufc, int h) {
+        constexpr int buf = decltype(bufc)::value;
+        wait_lgkm<0>();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) { tie(xv[buf][i]); tie(wv[buf][i]); }
+        if ((h & 7) == 7) {                      // the stage has been read: its place is free, and the next one is there
+            wait_loads_and_barrier<16 * (CHAIN_STAGES - 2)>();
+            load();
+            src = src == (CHAIN_STAGES - 1) * 16u * CHAIN_ROW * 4u ? 0u : src + 16u * CHAIN_ROW * 4u;
+        }
+        const unsigned off = src + 128u * ((h + 1) & 7);
+        if (h + 1 < groups) chain_read<0>(xv[1 - buf], wv[1 - buf], xrow + off, wrow + off);
+        __builtin_amdgcn_sched_barrier(0);
+        if (h < full) {
+            float p[32];
+#pragma unroll
+            for (int i = 0; i < 32; ++i) p[i] = wv[buf][i >> 2][i & 3] * xv[buf][i >> 2][i & 3];
+#pragma unroll
+            for (int i = 0; i < 32; ++i) sum = sum + p[i];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 31; ++i) {
+                const float t = sum + wv[buf][i >> 2][i & 3] * xv[buf][i >> 2][i & 3];
+                sum = i < rest ? t : sum;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int st = 0; st < CHAIN_STAGES; ++st) load();
+    wait_loads_and_barrier<16 * (CHAIN_STAGES - 1)>();
+    chain_read<0>(xv[0], wv[0], xrow, wrow);
+    for (int h = 0; h < groups; h += 2) {
+        group(std::integral_constant<int, 0>{}, h);
+        if (h + 1 < groups) group(std::integral_constant<int, 1>{}, h + 1);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    chain_store(B, O, b0 + bi, o0 + oi, sum, bias, beta, y);
 }
 
 // Forward (BWD = false) and backward-data with K in the tensors' own order, (channel, tap).

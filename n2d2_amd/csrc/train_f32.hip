@@ -1071,7 +1071,12 @@ static int run_direct(const ConvF32& q, int pass, const float* x, const float* w
     // (a kernel of 3x3 has an order of its own; 16-byte loads)
     if (!bwd && !q.depthwise && q.dx == 1 && q.dy == 1 && spans_input(q) && (q.kH != 3 || q.kW != 3) && K % 4 == 0 && K < (1 << 22) && q.O <= 8 * GRID_Y
         && (((size_t)x | (size_t)w) & 15) == 0) {
-        hipLaunchKernelGGL(conv_f32_chain_kernel, dim3(ceil_div_i(q.B, 8), ceil_div_i(q.O, 8)), dim3(192), 0, st, q.B, q.O, (int)K, x, w, bias, beta, out);
+        const dim3 grid(ceil_div_i(q.B, 8), ceil_div_i(q.O, 8));
+        // (a unit holds one block of the kernel whose waves share the work, and three of the other; measured there)
+        if ((size_t)grid.x * grid.y <= (size_t)num_cus())
+            N2D2HIP_LAUNCH(conv_f32_chain_kernel, grid, dim3(192), 0, st, q.B, q.O, (int)K, x, w, bias, beta, out);
+        else
+            N2D2HIP_LAUNCH(conv_f32_chain_wave_kernel, grid, dim3(64), 0, st, q.B, q.O, (int)K, x, w, bias, beta, out);
         N2D2HIP_HIP_CHECK(hipGetLastError());
         return N2D2HIP_OK;
     }
