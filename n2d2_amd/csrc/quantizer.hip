@@ -135,8 +135,12 @@ struct SatLevels {
 //    made the compiler spill.)
 //  * More: the first launch leaves each block's max |tanh w|, and every block of the second one takes the maximum of those,
 //    at most 256, itself, instead of a launch of one block in between (48120 weights: 3 launches of 2.8, 1.8 and 2.4 us).
+//    The second launch fills the chip, 8 blocks a compute unit, and both deal the weights to the XCDs alike, in runs of 256 as
+//    the scaling's launches do, so that the weights come from the XCD's own L2 the second time.  us, with the launch in
+//    between / with 4 blocks a unit and runs of 1024 in the first launch / now: 16385 weights 11.6 / 9.5 / 8.8, 1048576 11.3 / 9.8 / 9.4,
+//    4194304 16.6 / 20.3 / 15.5, 16777216 52.8 / 62.5 / 52.4, 67108864 279 / 341 / 269.
 constexpr int SAT_SMALL = 16;                    // weights per thread of a block of 1024 at most
-constexpr int SAT_BLOCKS = 256;                  // blocks of a larger tensor's first launch at most
+constexpr int SAT_BLOCKS = 256, SAT_BLOCKS2 = 2048;     // blocks of a larger tensor's first and second launch at most
 constexpr int SAT_ITEMS = 16;
 template <int N>
 struct SatBatch {
@@ -200,11 +204,13 @@ __global__ __launch_bounds__(1024) void sat_weight_first_kernel(const SatBatch<N
     else if (t.n <= 12 * 1024) sat_weight_small<12>(t);
     else if (sat_small(t.n)) sat_weight_small<SAT_SMALL>(t);
     else {
+        // (blocks 8 apart run on the same XCD: of 8 blocks, a multiple of which there is, each takes every 8th run of 256)
+        const unsigned block = blockIdx.x - b.first[k], run = 8 * (4 * (block >> 3) + (threadIdx.x >> 8)) + (block & 7);
         float m = 0.0f;
-        for (size_t i = (size_t)(blockIdx.x - b.first[k]) * 1024 + threadIdx.x; i < t.n; i += (size_t)(b.first[k + 1] - b.first[k]) * 1024)
+        for (size_t i = (size_t)run * QBLOCK + (threadIdx.x & (QBLOCK - 1)); i < t.n; i += (size_t)(b.first[k + 1] - b.first[k]) * 1024)
             m = fmaxf(m, fabsf(tanhf(t.w[i])));
         m = block_max(m);
-        if (threadIdx.x == 0) ((float*)t.workspace)[blockIdx.x - b.first[k]] = m;
+        if (threadIdx.x == 0) ((float*)t.workspace)[block] = m;
     }
 }
 template <int N>
@@ -461,12 +467,12 @@ static void sat_weight_launch(const n2d2hip_sat_weight_item* items, int count, h
     for (int i = 0; i < count; ++i) {
         const size_t n = items[i].n;
         b.item[i] = items[i];
-        b.first[i + 1] = b.first[i] + (sat_small(n) ? 1u : (unsigned)std::min<size_t>((n + 1023) / 1024, SAT_BLOCKS));
-        b.first2[i + 1] = b.first2[i] + (sat_small(n) ? 0u : (unsigned)blocks_for(n));
+        b.first[i + 1] = b.first[i] + (sat_small(n) ? 1u : (unsigned)std::min<size_t>((n + 8191) / 8192 * 8, SAT_BLOCKS));
+        b.first2[i + 1] = b.first2[i] + (sat_small(n) ? 0u : (unsigned)std::min<size_t>((n + QBLOCK - 1) / QBLOCK, SAT_BLOCKS2));
     }
-    hipLaunchKernelGGL(sat_weight_first_kernel<N>, dim3(b.first[count]), dim3(1024), 0, st, b);
+    N2D2HIP_LAUNCH_T(sat_weight_first_kernel, (N), dim3(b.first[count]), dim3(1024), 0, st, b);
     if (b.first2[count])
-        hipLaunchKernelGGL(sat_weight_second_kernel<N>, dim3(b.first2[count]), dim3(QBLOCK), 0, st, b);
+        N2D2HIP_LAUNCH_T(sat_weight_second_kernel, (N), dim3(b.first2[count]), dim3(QBLOCK), 0, st, b);
     for (int i = 0; i < count; ++i) {
         const n2d2hip_sat_weight_item& t = items[i];
         if (!t.apply_scaling || sat_small(t.n))

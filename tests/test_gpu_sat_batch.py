@@ -54,3 +54,28 @@ def test_batch_refuses_what_a_single_call_refuses():
     call = lambda **kw: lib.n2d2hip_sat_weight_forward_batch((capi.SatWeightItem * 2)(capi.SatWeightItem(**good), capi.SatWeightItem(**{**good, **kw})), 2, None)
     assert call(n=0) and call(w=None) and call(mode=9) and call(range=0.5) and call(workspace_bytes=8) and call(n=1, apply_scaling=1)
     assert lib.n2d2hip_sat_weight_forward_batch((capi.SatWeightItem * 1)(capi.SatWeightItem(**good)), 0, None)
+
+
+@pytest.mark.parametrize("n", [16385, 262143, 262145, 2097153, 4194307])
+def test_many_weights_fill_the_chip_and_equal_the_formula(n):
+    """Tensors of many blocks, whose runs of 256 are dealt out by eights: every weight once, and the pass that writes them has as
+    many threads as the chip holds (2048 a compute unit) as soon as there are as many weights."""
+    import torch
+    from n2d2_amd import capi, runtime as rt
+    print("sat many", n, flush=True)
+    ws = torch.empty(int(capi.lib.n2d2hip_quantizer_workspace_bytes(n)), dtype=torch.uint8, device="cuda")
+    stats = torch.zeros(2, device="cuda")
+    w = torch.from_numpy(np.random.default_rng(n).normal(0, 0.4, n).astype(np.float32)).cuda()
+    for place in (0, n - 1, (n // 256 - 1) * 256 + 255, min(n - 1, 8 * 256 * 3 + 5)):          # the largest weight at either end and inside
+        x = w.clone()
+        x[place] = 2.5
+        out = torch.full_like(x, 7.0)
+        with capi.launch_log() as log:
+            capi.check(capi.lib.n2d2hip_sat_weight_forward(x.data_ptr(), out.data_ptr(), n, 15.0, 0, 0, 1, stats.data_ptr(), ws.data_ptr(), ws.numel(),
+                                                           rt.stream_ptr()))
+        t = torch.tanh(x.double())
+        assert abs(float(stats[0]) - float(np.tanh(2.5))) < 2.0 ** -23
+        assert float((out.double() - t / t.abs().max()).abs().max()) < 5 * 2.0 ** -24 * 2         # (tanhf 2 ulp, the quotient half of one)
+        (first, second) = log.entries
+        cus = torch.cuda.get_device_properties(0).multi_processor_count
+        assert first[0].startswith("sat_weight_first_kernel") and second[1] * second[2] >= min(n, 2048 * cus)
