@@ -419,6 +419,11 @@ int n2d2hip_dw_pw_destroy(n2d2hip_dw_pw_t fused);
  * at most 256 outputs and at least 32768 output pixels, 9216 with more than 128 outputs), else 0.  No counterpart in the
  * reference: a planner's question (DeepNet::planFusion asks it). */
 int n2d2hip_dw_pw_pays(n2d2hip_dw_pw_t fused, int batch, int in_h, int in_w);
+/* How the pair runs fastest on `batch` inputs of in_h x in_w, from the two cells and sizes alone (measured rules, at the function),
+ * before anything is laid out for either kernel: as two launches (also where neither kernel takes the pair), by n2d2hip_dw_pw_*
+ * or by n2d2hip_dw_pw_small_*, below. */
+enum { N2D2HIP_DW_PW_APART = 0, N2D2HIP_DW_PW_TILES = 1, N2D2HIP_DW_PW_SMALL = 2 };
+int n2d2hip_dw_pw_plan(n2d2hip_conv_t depthwise, n2d2hip_conv_t pointwise, int batch, int in_h, int in_w);
 /* `in`: input of `depthwise`; `out`: output of `pointwise`.  NHWC bytes without a border, channel stride equal to the
  * channel count. */
 int n2d2hip_dw_pw_forward(n2d2hip_dw_pw_t fused, const n2d2hip_tensor* in, const n2d2hip_tensor* out, n2d2hip_stream_t stream);

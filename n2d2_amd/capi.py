@@ -24,6 +24,7 @@ KERNEL_NO_PIPE, KERNEL_NO_STEM, KERNEL_NO_HI16, KERNEL_NO_SUM16, KERNEL_TILE_M64
     1, 2, 4, 8, 16, 32, 64, 128)
 KERNEL_NO_PATCH, KERNEL_PATCH, KERNEL_NO_DIRECT, KERNEL_DIRECT, KERNEL_TILE_M256 = 256, 512, 1024, 2048, 4096
 KERNEL_NO_SPLIT, KERNEL_SPLIT = 8192, 16384
+DW_PW_APART, DW_PW_TILES, DW_PW_SMALL = range(3)
 
 # every symbol include/n2d2hip.h declares
 SYMBOLS = [
@@ -33,7 +34,7 @@ SYMBOLS = [
     "n2d2hip_conv_create", "n2d2hip_conv_destroy", "n2d2hip_conv_out_dims", "n2d2hip_conv_forward", "n2d2hip_conv_s2d_halo", "n2d2hip_conv_accepts_halo", "n2d2hip_conv_desc_reads_halo",
     "n2d2hip_conv_fuse_sum", "n2d2hip_conv_forward_sum", "n2d2hip_conv_chain_supported", "n2d2hip_conv_chain_pays", "n2d2hip_conv_chain_forward", "n2d2hip_bottleneck_create", "n2d2hip_bottleneck_destroy", "n2d2hip_bottleneck_pays", "n2d2hip_bottleneck_forward",
     "n2d2hip_conv_accepts_maxpool", "n2d2hip_conv_forward_maxpool", 
-    "n2d2hip_dw_pw_create", "n2d2hip_dw_pw_destroy", "n2d2hip_dw_pw_forward", "n2d2hip_dw_pw_pays",
+    "n2d2hip_dw_pw_create", "n2d2hip_dw_pw_destroy", "n2d2hip_dw_pw_forward", "n2d2hip_dw_pw_pays", "n2d2hip_dw_pw_plan",
     "n2d2hip_dw_pw_small_create", "n2d2hip_dw_pw_small_destroy", "n2d2hip_dw_pw_small_forward", "n2d2hip_dw_pw_small_pays",
     "n2d2hip_fc_create", "n2d2hip_fc_destroy", "n2d2hip_fc_forward", "n2d2hip_fc_chain_create", "n2d2hip_fc_chain_destroy", "n2d2hip_fc_chain_forward",
     "n2d2hip_cell_run_create", "n2d2hip_cell_run_destroy", "n2d2hip_cell_run_forward",
@@ -141,6 +142,7 @@ def load():
     lib.n2d2hip_bottleneck_forward.argtypes = [P, P, P, P]
     lib.n2d2hip_conv_accepts_maxpool.argtypes = [P, P, C.c_int, C.c_int]
     lib.n2d2hip_conv_forward_maxpool.argtypes = [P, P, P, P, P]
+    lib.n2d2hip_dw_pw_plan.argtypes = [P, P, I, I, I]
     for size in ("dw_pw", "dw_pw_small"):
         getattr(lib, "n2d2hip_%s_create" % size).argtypes = [P, P, P]
         getattr(lib, "n2d2hip_%s_destroy" % size).argtypes = [P]

@@ -28,6 +28,7 @@
 
 #include "common.h"
 #include "conv_handle.hpp"
+#include "dw_pw.hpp"
 #include "epilogue.hpp"
 #include "mfma_util.hpp"
 
@@ -398,15 +399,6 @@ __global__ __launch_bounds__(64 * WAVES, (DwPwShape<S, KC, NB, WAVES, SINGLE, FA
     }
 }
 
-bool plain_1x1(const n2d2hip_conv_desc& d)
-{
-    return d.kW == 1 && d.kH == 1 && d.strideX == 1 && d.strideY == 1 && d.padL == 0 && d.padT == 0 && d.padR == 0 && d.padB == 0
-        && d.dilX == 1 && d.dilY == 1 && d.groups == 1 && d.weight_bits == 8;
-}
-
-int byte_type_of(const n2d2hip_act_s* a) { return a->min_out >= 0 ? N2D2HIP_U8B : N2D2HIP_I8; }
-
-
 template <int S, int KC, int NB, int WAVES, bool SINGLE, bool FAST>
 void launch_one(DwPwArgs a, int ytiles, hipStream_t stream)
 {
@@ -446,6 +438,15 @@ void launch_chunks(const DwPwArgs& a, bool fast, int nb, hipStream_t stream)
 }
 
 } // namespace
+
+bool dw_pw_takes(const n2d2hip_conv_s* dw, const n2d2hip_conv_s* pw)
+{
+    const int C = dw->desc.C, O = pw->desc.O;
+    return plain_3x3_depthwise(dw) && dw->act->args.kind == EPI_I24 && dw->act->min_out >= -128 && dw->act->max_out <= 255 && plain_1x1(pw->desc)
+        && !pw->sub_inner && pw->desc.C == C && pw->in_cs == C && pw->in_dtype == byte_type_of(dw->act) && (O == 64 || O == 128 || O % 256 == 0)
+        && pw->act->args.kind == EPI_I24 && pw->bias_folded && pw->d_epi_tab && pw->act->min_out >= -128 && pw->act->max_out <= 255 && !pw->sum && pw->ktot >= C;
+}
+
 } // namespace n2d2hip
 
 using namespace n2d2hip;
@@ -472,16 +473,8 @@ int n2d2hip_dw_pw_destroy(n2d2hip_dw_pw_t h)
 int n2d2hip_dw_pw_create(n2d2hip_conv_t dw, n2d2hip_conv_t pw, n2d2hip_dw_pw_t* out)
 {
     N2D2HIP_REQUIRE(dw && pw && out, N2D2HIP_ERR_INVALID, "dw_pw_create: null argument");
-    const n2d2hip_conv_desc& dd = dw->desc;
-    const n2d2hip_conv_desc& dp = pw->desc;
-    const int C = dd.C, O = dp.O;
-    const bool ok = dw->depthwise && dw->d_wdw && dd.kW == 3 && dd.kH == 3 && dd.dilX == 1 && dd.dilY == 1 && dd.strideX == dd.strideY
-        && (dd.strideX == 1 || dd.strideX == 2) && dw->act->args.kind == EPI_I24 && dw->act->cpad >= C && dw->in_cs == C
-        && (C == 32 || C % 64 == 0) && dw->act->min_out >= -128 && dw->act->max_out <= 255
-        && plain_1x1(dp) && dp.C == C && pw->in_cs == C && pw->in_dtype == byte_type_of(dw->act) && (O == 64 || O == 128 || O % 256 == 0)
-        && (int)dw->act->htab.size() >= 5 * dw->act->cpad && pw->act->args.kind == EPI_I24 && pw->bias_folded && pw->d_epi_tab && pw->act->min_out >= -128 && pw->act->max_out <= 255
-        && !pw->sum && pw->ktot >= C;
-    N2D2HIP_REQUIRE(ok, N2D2HIP_ERR_UNSUPPORTED,
+    const int C = dw->desc.C, O = pw->desc.O;
+    N2D2HIP_REQUIRE(dw_pw_takes(dw, pw), N2D2HIP_ERR_UNSUPPORTED,
                     "dw_pw_create: needs a 3x3 undilated depthwise convolution of stride 1 or 2 over 32 or a multiple of 64 channels and an "
                     "unpadded 1x1 convolution of stride 1 reading it, to 64, 128 or a multiple of 256 channels, both 8-bit with integer "
                     "rescales (32-bit multiply-add) and byte outputs, the second without a folded sum");

@@ -17,6 +17,7 @@
 
 #include "common.h"
 #include "conv_handle.hpp"
+#include "dw_pw.hpp"
 #include "epilogue.hpp"
 #include "mfma_util.hpp"
 
@@ -169,9 +170,39 @@ bool integer_bytes(const n2d2hip_act_s* a)
     return (a->args.kind == EPI_I24 || a->args.kind == EPI_I64) && a->min_out >= -128 && a->max_out <= 255;
 }
 
-int byte_type_of(const n2d2hip_act_s* a) { return a->min_out >= 0 ? N2D2HIP_U8B : N2D2HIP_I8; }
+long long work_groups(int O, long long pixels) { return (pixels + PIXELS - 1) / PIXELS * (O / OUTS); }
+
+// That kernel gives a work-group 8 x 16 pixels and all their outputs, up to 256.  us, that kernel / this one / two launches, up to
+// 128 outputs: 32 -> 64 channels, 112 x 112 3.6 / 4.8 / 7.6, two images of 48 x 48 3.4 / 4.1 / 7.5; 64 -> 128 stride 2, 56 x 56
+// 4.6 / 4.3 / 8.1, two 4.6 / 5.1 / 8.2; 128 -> 128, 56 x 56 5.1 / 4.6 / 6.6, two 5.2 / 6.7 / 7.0, four 5.3 / 10.0 / 8.0, two of 24 x 24
+// 5.7 / 4.1 / 5.9.  With 512 outputs it computes the depthwise part twice and fills the chip later; that kernel / two launches,
+// 512 -> 512 at 14 x 14: 32 images 14.3 / 12.9, 48 15.0 / 15.9, 64 15.8 / 17.9, 128 26.8 / 28.2 (1024 outputs: 24.7 / 15.0 at 64).
+bool tiles_first(int C, int O, long long pixels)
+{
+    return O <= TILES_OUTS ? C == 32 || work_groups(O, pixels) > 1024 : O <= TILES_WIDE_OUTS && pixels >= TILES_WIDE_PIXELS;
+}
+
+// Is this kernel faster than the cells' own launches?
+bool small_wins(int C, int O, long long pixels)
+{
+    // Where all work-groups are on the chip at once (by their LDS, 12 KB a wave).  us, one launch and two, for output planes of
+    // 112 / 56 / 56 / 28 / 28 / 14 / 14 / 7 and 32 -> 64, 64 -> 128, 128 -> 128, 128 -> 256, 256 -> 256, 256 -> 512, 512 -> 512, 512 -> 1024 channels:
+    //   one image    4.8 7.6   4.3 8.1   4.6 6.6   4.1 5.8   4.6 6.1   4.2 5.7   5.2 6.1   4.7 5.8
+    //   two images   7.2 7.8   5.0 8.2   6.7 7.0*  4.6 6.3   6.8 6.9*  4.6 5.9   8.8 6.2*  4.8 5.9     * the rule declines
+    //   four        11.0 9.3*  7.6 8.7  10.0 8.0*  6.7 6.8*  9.8 7.2*  6.8 6.4* 16.0 7.3*  8.0 5.9*
+    return work_groups(O, pixels) <= (long long)num_cus() * (163840 / (std::min(MAX_PARTS, (C + 63) / 64) * STAGE));
+}
 
 } // namespace
+
+bool dw_pw_small_takes(const n2d2hip_conv_s* dw, const n2d2hip_conv_s* pw)
+{
+    const int C = dw->desc.C, O = pw->desc.O;
+    return plain_3x3_depthwise(dw) && integer_bytes(dw->act) && plain_1x1(pw->desc) && !pw->depthwise && !pw->sub_inner && !pw->is_fc && pw->desc.C == C
+        && pw->in_cs == C && pw->in_dtype == byte_type_of(dw->act) && O % OUTS == 0 && integer_bytes(pw->act) && !pw->sum && pw->ktot >= C && pw->d_bias
+        && (int)pw->act->htab.size() >= 5 * pw->act->cpad;
+}
+
 } // namespace n2d2hip
 
 using namespace n2d2hip;
@@ -208,16 +239,8 @@ int n2d2hip_dw_pw_small_destroy(n2d2hip_dw_pw_small_t h)
 int n2d2hip_dw_pw_small_create(n2d2hip_conv_t dw, n2d2hip_conv_t pw, n2d2hip_dw_pw_small_t* out)
 {
     N2D2HIP_REQUIRE(dw && pw && out, N2D2HIP_ERR_INVALID, "dw_pw_small_create: null argument");
-    const n2d2hip_conv_desc& dd = dw->desc;
-    const n2d2hip_conv_desc& dp = pw->desc;
-    const int C = dd.C, O = dp.O;
-    const bool ok = dw->depthwise && dw->d_wdw && dd.kW == 3 && dd.kH == 3 && dd.dilX == 1 && dd.dilY == 1 && dd.strideX == dd.strideY
-        && (dd.strideX == 1 || dd.strideX == 2) && integer_bytes(dw->act) && dw->act->cpad >= C && dw->in_cs == C && (C == 32 || C % 64 == 0)
-        && dp.kW == 1 && dp.kH == 1 && dp.strideX == 1 && dp.strideY == 1 && dp.padL == 0 && dp.padT == 0 && dp.padR == 0 && dp.padB == 0
-        && dp.dilX == 1 && dp.dilY == 1 && dp.groups == 1 && dp.weight_bits == 8 && !pw->depthwise && !pw->sub_inner && !pw->is_fc
-        && dp.C == C && pw->in_cs == C && pw->in_dtype == byte_type_of(dw->act) && O % OUTS == 0 && integer_bytes(pw->act) && !pw->sum
-        && pw->ktot >= C && pw->d_bias && (int)dw->act->htab.size() >= 5 * dw->act->cpad && (int)pw->act->htab.size() >= 5 * pw->act->cpad;
-    N2D2HIP_REQUIRE(ok, N2D2HIP_ERR_UNSUPPORTED,
+    const int C = dw->desc.C, O = pw->desc.O;
+    N2D2HIP_REQUIRE(dw_pw_small_takes(dw, pw), N2D2HIP_ERR_UNSUPPORTED,
                     "dw_pw_small_create: needs a 3x3 undilated depthwise convolution of stride 1 or 2 over 32 or a multiple of 64 channels and an "
                     "unpadded 1x1 convolution of stride 1 reading it, to a multiple of 32 channels, both 8-bit with integer rescales and byte "
                     "outputs, the second without a folded sum");
@@ -243,11 +266,13 @@ int n2d2hip_dw_pw_small_create(n2d2hip_conv_t dw, n2d2hip_conv_t pw, n2d2hip_dw_
     h->fill_at = h->pwt_at + 6 * (size_t)O * sizeof(int);
     std::vector<signed char> img(h->fill_at + (size_t)nchunks * 64, 0);
     // lane (p, g) of an output block: output p, and in byte 4 * G + i channel 16 * G + 4 * g + i of the chunk
-    for (int o = 0; o < O; ++o)
-        for (int c = 0; c < C; c += 4) {
-            const int k = c / 64, G = c / 16 % 4, g = c / 4 % 4;
-            memcpy(img.data() + (((size_t)(o / 16) * nchunks + k) * 64 + g * 16 + o % 16) * 16 + 4 * G, w.data() + (size_t)o * pw->ktot + c, 4);
-        }
+    signed char* to = img.data();
+    for (int o0 = 0; o0 < O; o0 += 16)
+        for (int c0 = 0; c0 < C; c0 += 64)
+            for (int g = 0; g < 4; ++g)
+                for (int o = o0; o < o0 + 16; ++o, to += 16)
+                    for (int G = 0; G < (C == 32 ? 2 : 4); ++G)
+                        memcpy(to + 4 * G, w.data() + (size_t)o * pw->ktot + c0 + 16 * G + 4 * g, 4);
     int* const dwt = (int*)(img.data() + h->dwt_at);
     const std::vector<int>& tab = fast ? fold : dw->act->htab;
     for (int c = 0; c < C; ++c) {
@@ -284,16 +309,18 @@ int n2d2hip_dw_pw_small_create(n2d2hip_conv_t dw, n2d2hip_conv_t pw, n2d2hip_dw_
     return N2D2HIP_OK;
 }
 
-static long long work_groups(n2d2hip_dw_pw_small_t h, long long pixels) { return (pixels + PIXELS - 1) / PIXELS * (h->pw->desc.O / OUTS); }
+static bool choose_tiles(n2d2hip_dw_pw_small_t h, long long pixels) { return h->tiles && tiles_first(h->dw->desc.C, h->pw->desc.O, pixels); }
 
-// That kernel gives a work-group 8 x 16 pixels and all their outputs, up to 256.  us, that kernel / this one / two launches, up to
-// 128 outputs: 32 -> 64 channels, 112 x 112 3.6 / 4.8 / 7.6, two images of 48 x 48 3.4 / 4.1 / 7.5; 64 -> 128 stride 2, 56 x 56
-// 4.6 / 4.3 / 8.1, two 4.6 / 5.1 / 8.2; 128 -> 128, 56 x 56 5.1 / 4.6 / 6.6, two 5.2 / 6.7 / 7.0, four 5.3 / 10.0 / 8.0, two of 24 x 24
-// 5.7 / 4.1 / 5.9.  With 512 outputs it computes the depthwise part twice and fills the chip later; that kernel / two launches,
-// 512 -> 512 at 14 x 14: 32 images 14.3 / 12.9, 48 15.0 / 15.9, 64 15.8 / 17.9, 128 26.8 / 28.2 (1024 outputs: 24.7 / 15.0 at 64).
-static bool choose_tiles(n2d2hip_dw_pw_small_t h, long long pixels)
+int n2d2hip_dw_pw_plan(n2d2hip_conv_t dw, n2d2hip_conv_t pw, int batch, int in_h, int in_w)
 {
-    return h->tiles && (h->pw->desc.O > TILES_OUTS ? pixels >= TILES_WIDE_PIXELS : h->dw->desc.C == 32 || work_groups(h, pixels) > 1024);
+    int OH, OW;
+    if (!dw || !pw || batch <= 0 || n2d2hip_conv_out_dims(&dw->desc, in_h, in_w, &OH, &OW) != N2D2HIP_OK)
+        return N2D2HIP_DW_PW_APART;
+    const int C = dw->desc.C, O = pw->desc.O;
+    const long long pixels = (long long)batch * OH * OW;
+    if (dw_pw_takes(dw, pw) && tiles_first(C, O, pixels))
+        return N2D2HIP_DW_PW_TILES;
+    return dw_pw_small_takes(dw, pw) && small_wins(C, O, pixels) ? N2D2HIP_DW_PW_SMALL : N2D2HIP_DW_PW_APART;
 }
 
 int n2d2hip_dw_pw_small_pays(n2d2hip_dw_pw_small_t h, int batch, int in_h, int in_w)
@@ -303,18 +330,11 @@ int n2d2hip_dw_pw_small_pays(n2d2hip_dw_pw_small_t h, int batch, int in_h, int i
     int OH, OW;
     if (n2d2hip_conv_out_dims(&h->dw->desc, in_h, in_w, &OH, &OW) != N2D2HIP_OK)
         return 0;
-    const long long pixels = (long long)batch * OH * OW, groups = work_groups(h, pixels);
+    const long long pixels = (long long)batch * OH * OW;
     const int O = h->pw->desc.O;
     if (!h->tiles && O > TILES_OUTS && O <= TILES_WIDE_OUTS && pixels >= TILES_WIDE_PIXELS && make_tiles(h) != N2D2HIP_OK)
         return 0;
-    if (choose_tiles(h, pixels))
-        return 1;
-    // Where all work-groups are on the chip at once (by their LDS, 12 KB a wave).  us, one launch and two, for output planes of
-    // 112 / 56 / 56 / 28 / 28 / 14 / 14 / 7 and 32 -> 64, 64 -> 128, 128 -> 128, 128 -> 256, 256 -> 256, 256 -> 512, 512 -> 512, 512 -> 1024 channels:
-    //   one image    4.8 7.6   4.3 8.1   4.6 6.6   4.1 5.8   4.6 6.1   4.2 5.7   5.2 6.1   4.7 5.8
-    //   two images   7.2 7.8   5.0 8.2   6.7 7.0*  4.6 6.3   6.8 6.9*  4.6 5.9   8.8 6.2*  4.8 5.9     * the rule declines
-    //   four        11.0 9.3*  7.6 8.7  10.0 8.0*  6.7 6.8*  9.8 7.2*  6.8 6.4* 16.0 7.3*  8.0 5.9*
-    return groups <= (long long)num_cus() * (163840 / (std::min(MAX_PARTS, h->nchunks) * STAGE)) ? 1 : 0;
+    return choose_tiles(h, pixels) || small_wins(h->dw->desc.C, O, pixels) ? 1 : 0;
 }
 
 int n2d2hip_dw_pw_small_forward(n2d2hip_dw_pw_small_t h, const n2d2hip_tensor* in, const n2d2hip_tensor* out, n2d2hip_stream_t stream_)

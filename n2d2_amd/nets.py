@@ -403,7 +403,7 @@ class GpuNet:
         stem_pool: compute the max pooling behind a first-layer convolution in that convolution's launch
         (n2d2hip_conv_forward_maxpool) where the library takes the pair.
         dw_pw: run a 3x3 depthwise convolution and the 1x1 convolution that alone reads it as one launch (n2d2hip_dw_pw_*)
-        where the library takes the pair and expects the launch to be faster than the two (n2d2hip_dw_pw_pays); "all":
+        where the library takes the pair and expects the launch to be faster than the two (n2d2hip_dw_pw_plan); "all":
         wherever the library takes the pair.
         s2d: store the network input space-to-depth (16-byte pixels of 2 x 2 input pixels, with a border of zeros) when the
         one cell reading it is a first-layer convolution the library serves that way (n2d2hip_conv_s2d_halo).
@@ -544,7 +544,7 @@ class GpuNet:
                 self.folded.add(conv.name)
                 self.stem_pools[l.name] = conv
         # a 3x3 depthwise convolution and the 1x1 convolution that alone reads it as one launch (the depthwise output is
-        # never written)
+        # never written); dw_pws: those of 32768 pixels and more, or taken because all were asked for, dw_pws_small: the others
         self.dw_pws, self.dw_pws_small = {}, {}
         if fuse and dw_pw:
             step_index = {l.name: k for k, (l, c, f) in enumerate(self.steps)}
@@ -555,14 +555,16 @@ class GpuNet:
                 if (dw is None or dw.type != "conv" or len(dw.inputs) != 1 or dw.groups == 1 or len(consumers[dw.name]) != 1 or dw.name in self.folded
                         or ins_of[dw.name][0].halo or self.tensors[l.name].halo):
                     continue
-                # the library knows where one launch is faster than two: large tensors between the cells, and few pixels
-                x = ins_of[dw.name][0]
-                for kind, pairs in ((rt.DwPw, self.dw_pws), (rt.DwPwSmall, self.dw_pws_small)):
-                    fused_cell = kind.create(self.steps[step_index[dw.name]][1], self.steps[step_index[l.name]][1])
-                    if fused_cell is not None and (fused_cell.pays(batch, x.H, x.W) or dw_pw == "all" and kind is rt.DwPw):
-                        break
-                else:
-                    continue
+                # the library knows where one launch is faster than two, and which
+                x, out = ins_of[dw.name][0], self.tensors[l.name]
+                pair = self.steps[step_index[dw.name]][1], self.steps[step_index[l.name]][1]
+                fused_cell = rt.DwPw.create(*pair) if dw_pw == "all" else None
+                pairs = self.dw_pws if fused_cell is not None or batch * out.H * out.W >= 32768 else self.dw_pws_small
+                if fused_cell is None:
+                    kind = rt.dw_pw_kind(*pair, batch, x.H, x.W)
+                    if kind is None:
+                        continue
+                    fused_cell = kind.create(*pair)
                 self.steps[step_index[l.name]] = (l, fused_cell, (lambda c, i, o: c.forward(i[0], o)))
                 ins_of[l.name] = ins_of[dw.name]
                 self.folded.add(dw.name)

@@ -203,6 +203,13 @@ class DwPwSmall(DwPw):
     _NAME = "n2d2hip_dw_pw_small"
 
 
+def dw_pw_kind(depthwise, pointwise, batch, in_h, in_w):
+    """DwPw or DwPwSmall, whichever the library expects to be the fastest on inputs of this size, or None: two launches.  Nothing
+    is laid out for the question."""
+    plan = lib.n2d2hip_dw_pw_plan(depthwise.handle, pointwise.handle, batch, in_h, in_w)
+    return {capi.DW_PW_TILES: DwPw, capi.DW_PW_SMALL: DwPwSmall}.get(plan)
+
+
 def scaling_forward(act, x, out_dtype=None):
     out = DTensor(x.B, x.C, x.H, x.W, out_dtype if out_dtype is not None else act.out_dtype(), x.layout)
     check(lib.n2d2hip_scaling_forward(act.handle, x.ref, out.ref, stream_ptr()))

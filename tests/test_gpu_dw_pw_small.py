@@ -65,3 +65,16 @@ def test_small_declines_what_it_is_not_written_for():
     # one pixel pays, a batch that does not fit the chip does not
     h = rt.DwPwSmall.create(conv(512, 512, 3, 512, pad=(1,) * 4), conv(512, 512, 1))
     assert h.pays(1, 14, 14) and not h.pays(8, 14, 14)
+
+
+@pytest.mark.parametrize("batch,image", [(1, 224), (2, 96), (8, 160)])
+def test_network_lays_out_only_the_pairs_it_launches(batch, image, monkeypatch):
+    """The library says from the cells and sizes alone how a pair runs, so that no kernel's weights are laid out and thrown away."""
+    from n2d2_amd import nets, runtime as rt
+    made = []
+    create = rt.DwPw.create.__func__           # (DwPwSmall inherits it)
+    monkeypatch.setattr(rt.DwPw, "create", classmethod(lambda cls, dw, pw: made.append(cls) or create(cls, dw, pw)))
+    net = nets.GpuNet(nets.mobilenet_v1(image=image), batch)
+    fused = [cell for l, cell, fn in net.steps if isinstance(cell, rt.DwPw)]
+    assert len(fused) == len(net.dw_pws) + len(net.dw_pws_small) >= 3
+    assert made == [type(cell) for cell in fused]
