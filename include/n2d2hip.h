@@ -428,11 +428,10 @@ int n2d2hip_dw_pw_plan(n2d2hip_conv_t depthwise, n2d2hip_conv_t pointwise, int b
  * channel count. */
 int n2d2hip_dw_pw_forward(n2d2hip_dw_pw_t fused, const n2d2hip_tensor* in, const n2d2hip_tensor* out, n2d2hip_stream_t stream);
 /* The same for few pixels: work-groups of 16 pixels x 32 outputs, each of which computes the depthwise convolution of its
- * pixels itself, or the kernel above where that is faster (up to 512 outputs).  Taken are 8-bit cells with integer rescales
- * (of either width) and byte outputs, over 32 or a multiple of 64 channels, to a multiple of 32; tensors, results and the
- * handles' lifetimes as above.  _pays: 1 where the one launch is expected to be faster than the two cells' own (measured
- * rule, at the function); past 128 outputs it also lays out the weights for the kernel above, where that is the faster
- * one, so it is asked before the forwards and not while a graph is captured. */
+ * pixels itself; up to 128 outputs the handle holds the kernel above too and runs it where that is the faster one.  Taken are
+ * 8-bit cells with integer rescales (of either width) and byte outputs, over 32 or a multiple of 64 channels, to a multiple of
+ * 32; tensors, results and the handles' lifetimes as above.  _pays: 1 where this handle's launch is expected to be faster than
+ * the two cells' own (measured rule, at the function). */
 typedef struct n2d2hip_dw_pw_small_s* n2d2hip_dw_pw_small_t;
 int n2d2hip_dw_pw_small_create(n2d2hip_conv_t depthwise, n2d2hip_conv_t pointwise, n2d2hip_dw_pw_small_t* fused);
 int n2d2hip_dw_pw_small_destroy(n2d2hip_dw_pw_small_t fused);

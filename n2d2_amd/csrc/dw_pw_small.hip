@@ -44,6 +44,7 @@ struct DwPwSmallArgs {
     int C, O, nchunks, parts;
     int H, W, OH, OW, stride, padL, padT;
     int ntasks;                   // output pixels
+    int first;                    // of those, the launch's first
     unsigned ow_mul, ow_sh, oh_mul, oh_sh;
     unsigned mid_xor, out_xor;
     int dw_lo, dw_hi;
@@ -65,7 +66,7 @@ __global__ __launch_bounds__(64 * MAX_PARTS) void dw_pw_small_kernel(const DwPwS
     // the pixel this lane brings 16 bytes of, 4 lanes a pixel; a pixel's 16-channel groups are swizzled so that 16 pixels' bytes
     // of one group lie in different banks
     const int pl = lane >> 2, group = (lane & 3) ^ (pl >> 2 & 3);
-    const int task = min((int)blockIdx.y * PIXELS + pl, q.ntasks - 1);
+    const int task = min(q.first + (int)blockIdx.y * PIXELS + pl, q.ntasks - 1);
     const int t1 = div_magic(task, q.ow_mul, q.ow_sh), ox = task - t1 * q.OW;
     const int b = div_magic(t1, q.oh_mul, q.oh_sh), oy = t1 - b * q.OH;
     const int ix = ox * q.stride - q.padL, iy = oy * q.stride - q.padT;
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(64 * MAX_PARTS) void dw_pw_small_kernel(const DwPwS
         for (int e = 0; e < 4; ++e)
             v[e] = q.pw_kind == EPI_I24 ? epi_apply<EPI_I24>(s[e] + bias[e], a[e], bb[e], c[e], d[e], e5[e], q.pw_lo, q.pw_hi, 0)
                                         : epi_apply<EPI_I64>(s[e] + bias[e], a[e], bb[e], c[e], 0, e5[e], q.pw_lo, q.pw_hi, 0);
-        const int pix = (int)blockIdx.y * PIXELS + p;
+        const int pix = q.first + (int)blockIdx.y * PIXELS + p;
         if (pix < q.ntasks)
             *(unsigned*)(q.out + (long long)pix * q.O + ch) = pack_bytes(v[0], v[1], v[2], v[3]) ^ q.out_xor;
     }
@@ -209,21 +210,12 @@ using namespace n2d2hip;
 
 struct n2d2hip_dw_pw_small_s {
     n2d2hip_conv_t dw, pw;
-    n2d2hip_dw_pw_t tiles;        // the kernel for many pixels, where this handle may choose it, or null
+    n2d2hip_dw_pw_t tiles;        // the kernel for many pixels, where it takes the pair and there are at most TILES_OUTS outputs, or null
     bool fast;
     int nchunks;
     signed char* d_image;         // 1x1 weights, depthwise tables, 1x1 tables, the stored 0
     size_t dwt_at, pwt_at, fill_at;
 };
-
-// The other kernel's handle, or null where that does not take the pair
-static int make_tiles(n2d2hip_dw_pw_small_s* h)
-{
-    const int rc = n2d2hip_dw_pw_create(h->dw, h->pw, &h->tiles);
-    if (rc != N2D2HIP_OK)
-        h->tiles = nullptr;
-    return rc == N2D2HIP_ERR_UNSUPPORTED ? N2D2HIP_OK : rc;
-}
 
 extern "C" {
 
@@ -298,9 +290,10 @@ int n2d2hip_dw_pw_small_create(n2d2hip_conv_t dw, n2d2hip_conv_t pw, n2d2hip_dw_
         n2d2hip_dw_pw_small_destroy(h);
         return fail(N2D2HIP_ERR_HIP, "dw_pw_small_create: device upload failed: %s", hipGetErrorString(e));
     }
-    if (O <= TILES_OUTS) {
-        const int rc = make_tiles(h);
+    if (O <= TILES_OUTS && dw_pw_takes(dw, pw)) {
+        const int rc = n2d2hip_dw_pw_create(dw, pw, &h->tiles);
         if (rc != N2D2HIP_OK) {
+            h->tiles = nullptr;
             n2d2hip_dw_pw_small_destroy(h);
             return rc;
         }
@@ -331,10 +324,7 @@ int n2d2hip_dw_pw_small_pays(n2d2hip_dw_pw_small_t h, int batch, int in_h, int i
     if (n2d2hip_conv_out_dims(&h->dw->desc, in_h, in_w, &OH, &OW) != N2D2HIP_OK)
         return 0;
     const long long pixels = (long long)batch * OH * OW;
-    const int O = h->pw->desc.O;
-    if (!h->tiles && O > TILES_OUTS && O <= TILES_WIDE_OUTS && pixels >= TILES_WIDE_PIXELS && make_tiles(h) != N2D2HIP_OK)
-        return 0;
-    return choose_tiles(h, pixels) || small_wins(h->dw->desc.C, O, pixels) ? 1 : 0;
+    return choose_tiles(h, pixels) || small_wins(h->dw->desc.C, h->pw->desc.O, pixels) ? 1 : 0;
 }
 
 int n2d2hip_dw_pw_small_forward(n2d2hip_dw_pw_small_t h, const n2d2hip_tensor* in, const n2d2hip_tensor* out, n2d2hip_stream_t stream_)
@@ -359,7 +349,8 @@ int n2d2hip_dw_pw_small_forward(n2d2hip_dw_pw_small_t h, const n2d2hip_tensor* i
     N2D2HIP_REQUIRE(out->B == in->B && out->C == dp.O && out->cs == dp.O && out->H == OH && out->W == OW && out->dtype == out_dtype,
                     N2D2HIP_ERR_INVALID, "dw_pw_small_forward: output must be %dx%dx%dx%d bytes of type %d with a channel stride of %d", in->B,
                     dp.O, OH, OW, out_dtype, dp.O);
-    N2D2HIP_REQUIRE(pixels > 0 && (pixels + PIXELS - 1) / PIXELS <= 65535 && (long long)in->B * in->H * in->W * in->cs < (1ll << 31),
+    constexpr int SPAN = 65535 * PIXELS;         // pixels of a launch at most
+    N2D2HIP_REQUIRE(pixels > 0 && pixels < (1ll << 31) - SPAN && (long long)in->B * in->H * in->W * in->cs < (1ll << 31),
                     N2D2HIP_ERR_UNSUPPORTED, "dw_pw_small_forward: tensor too large");
     DwPwSmallArgs a;
     a.in = (const signed char*)in->data; a.out = (signed char*)out->data;
@@ -375,10 +366,12 @@ int n2d2hip_dw_pw_small_forward(n2d2hip_dw_pw_small_t h, const n2d2hip_tensor* i
     a.dw_lo = h->dw->act->args.lo; a.dw_hi = h->dw->act->args.hi;
     a.pw_kind = h->pw->act->args.kind; a.pw_lo = h->pw->act->args.lo; a.pw_hi = h->pw->act->args.hi;
     // (output tiles first: work-groups 8 apart share an XCD, whose L2 then holds an eighth of the 1x1 weights)
-    const dim3 grid((unsigned)(dp.O / OUTS), (unsigned)((pixels + PIXELS - 1) / PIXELS));
-    if (h->fast) launch_groups<EPI_I24, true>(a, grid, stream);
-    else if (h->dw->act->args.kind == EPI_I24) launch_groups<EPI_I24, false>(a, grid, stream);
-    else launch_groups<EPI_I64, false>(a, grid, stream);
+    for (a.first = 0; a.first < a.ntasks; a.first += SPAN) {
+        const dim3 grid((unsigned)(dp.O / OUTS), (unsigned)((std::min(SPAN, a.ntasks - a.first) + PIXELS - 1) / PIXELS));
+        if (h->fast) launch_groups<EPI_I24, true>(a, grid, stream);
+        else if (h->dw->act->args.kind == EPI_I24) launch_groups<EPI_I24, false>(a, grid, stream);
+        else launch_groups<EPI_I64, false>(a, grid, stream);
+    }
     N2D2HIP_HIP_CHECK(hipGetLastError());
     return N2D2HIP_OK;
 }

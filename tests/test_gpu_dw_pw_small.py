@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
     (2, 64, 128, 1, 33, 31, 1),        # 256 + groups: all on the chip
     (2, 64, 128, 1, 48, 47, 1),        # 1128 work-groups: the kernel for many pixels
     (1, 32, 64, 1, 20, 9, 1),          # 32 channels: the kernel for many pixels
-    (6, 64, 512, 1, 40, 39, 1),        # 512 outputs, 9360 pixels: the kernel for many pixels, once asked for
+    (6, 64, 512, 1, 40, 39, 1),        # 512 outputs, 9360 pixels
 ])
 @pytest.mark.parametrize("rescale", ["plain", "clamped", "wide"])
 def test_small_equals_separate_launches(B, C, O, stride, H, W, pad, rescale):
@@ -45,9 +45,33 @@ def test_small_equals_separate_launches(B, C, O, stride, H, W, pad, rescale):
     fused = rt.DwPwSmall.create(dw, pw)
     assert fused is not None
     out = rt.DTensor(B, O, want.H, want.W, want.dtype)
-    assert np.array_equal(fused.forward(xin, out).to_numpy(), want.to_numpy())
-    fused.pays(B, H, W)
-    assert np.array_equal(fused.forward(xin, out).to_numpy(), want.to_numpy())
+    launched = []
+    for _ in range(2):                 # (the question whether it pays, between the two, changes nothing)
+        with capi.launch_log() as log:
+            assert np.array_equal(fused.forward(xin, out).to_numpy(), want.to_numpy())
+        launched.append([e[0] for e in log.entries if e[0].startswith("dw_pw")])
+        fused.pays(B, H, W)
+    assert launched[0] == launched[1] and len(launched[0]) == 1
+
+
+def test_small_takes_more_pixels_than_a_grid():
+    """65535 work-groups of 16 pixels are one launch; 34 pixels more."""
+    from n2d2_amd import capi, runtime as rt
+    from oracle.cells import ActSpec
+    rng = np.random.default_rng(7)
+    H, W = 1023, 1025
+    x = rng.integers(0, 256, size=(1, 32, H, W)).astype(np.int32)
+    spec = ActSpec("Rectifier", "FixedMult32", rng.integers(2 ** 11, 2 ** 12, size=32), frac_bits=18, nb_bits=8, unsigned_out=True)
+    dw = rt.Conv(rng.integers(-128, 128, size=(32, 1, 3, 3)), None, rt.Act(32, **spec.kwargs()), capi.U8B, pad=(1,) * 4, groups=32)
+    pw = rt.Conv(rng.integers(-128, 128, size=(32, 32, 1, 1)), None, rt.Act(32, **spec.kwargs()), capi.U8B)
+    xin = rt.DTensor.from_numpy(x, capi.U8B)
+    want = pw.forward(dw.forward(xin))
+    out = rt.DTensor(1, 32, H, W, want.dtype)
+    with capi.launch_log() as log:
+        rt.DwPwSmall.create(dw, pw).forward(xin, out)
+    assert [e[1] for e in log.entries] == [65535, 1]
+    import torch
+    assert torch.equal(out.buf, want.buf)
 
 
 def test_small_declines_what_it_is_not_written_for():
