@@ -415,9 +415,8 @@ int n2d2hip_conv_chain_forward(n2d2hip_conv_t conv3x3, n2d2hip_conv_t expand, co
 typedef struct n2d2hip_dw_pw_s* n2d2hip_dw_pw_t;
 int n2d2hip_dw_pw_create(n2d2hip_conv_t depthwise, n2d2hip_conv_t pointwise, n2d2hip_dw_pw_t* fused);
 int n2d2hip_dw_pw_destroy(n2d2hip_dw_pw_t fused);
-/* 1 when the one launch is expected to be faster than the two cells' own on `batch` inputs of in_h x in_w (measured rule:
- * at most 256 outputs and at least 32768 output pixels, 9216 with more than 128 outputs), else 0.  No counterpart in the
- * reference: a planner's question (DeepNet::planFusion asks it). */
+/* 1 when the one launch is expected to be faster than the two cells' own on `batch` inputs of in_h x in_w (measured rule, at
+ * the function), else 0.  No counterpart in the reference: a planner's question. */
 int n2d2hip_dw_pw_pays(n2d2hip_dw_pw_t fused, int batch, int in_h, int in_w);
 /* How the pair runs fastest on `batch` inputs of in_h x in_w, from the two cells and sizes alone (measured rules, at the function),
  * before anything is laid out for either kernel: as two launches (also where neither kernel takes the pair), by n2d2hip_dw_pw_*

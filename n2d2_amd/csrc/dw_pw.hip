@@ -437,7 +437,49 @@ void launch_chunks(const DwPwArgs& a, bool fast, int nb, hipStream_t stream)
     else launch_fast<S, 64, false>(a, fast, nb, stream);
 }
 
+// columns of a tile: 16, or fewer when that leaves fewer idle columns in the last tile of a row
+int tile_columns(int OW)
+{
+    int best_tw = 16;
+    long long best_cols = ((OW + 15) / 16) * 16;
+    for (int tw = 15; tw >= 8; --tw) {
+        const long long cols = (long long)((OW + tw - 1) / tw) * 16;
+        if (cols < best_cols) { best_cols = cols; best_tw = tw; }
+    }
+    return best_tw;
+}
+
 } // namespace
+
+// A work-group goes through its tile's chunks of 64 channels one behind the other, about 1.1 us each, so a launch takes 3 us and
+// that for every round of work-groups, while the cells' own launches grow with the pixels from 5 or 6 us on.  us, this launch / the
+// cells' own two:
+//  * one chunk: 32 -> 64 one pixel 3.0 / 6.0, 32400 4.0 / 8.0; 64 -> 256 4.4 / 6.4 and, 16384, 5.4 / 7.9; 64 -> 512, 32400, 10.6 / 13.3
+//  * up to 128 outputs: 128 -> 128 one pixel 4.7 / 5.5; 192 -> 128 5.6 / 6.3; 256 -> 128 one pixel 6.4 / 5.3, 2304 6.8 / 6.9, 8192
+//    7.0 / 7.7; 320 -> 128, 2048, 7.7 / 7.7; 384 -> 128, 5184 8.6 / 8.0, 9408 8.7 / 9.5; 512 -> 128, 8192 10.5 / 9.0, 9408 10.5 / 10.8; 768 -> 128, 10000
+//    13.9 / 12.9, 16384 14.1 / 15.4; 1024 -> 64, 16384 20.9 / 19.9, 19600 21.0 / 22.1
+//  * 256 outputs, whose work-group has the compute unit to itself: 256 -> 256, 6272 8.2 / 8.0, 9408 8.4 / 9.9; 512 -> 256, 8192 11.8 / 9.6,
+//    9408 11.9 / 12.0; 1024 -> 256, 12800 21.8 / 19.9.  Two rounds, the second nearly empty: 25872 pixels 256 -> 256 14.0 / 14.0, 512 -> 256
+//    21.2 / 19.3; 37632 14.4 / 18.1 and 23.0 / 27.4; 1024 -> 256, 32400 44.9 / 38.5, 40000 45.2 / 47.5
+//  * 512 outputs, each tile's depthwise part computed twice: 512 -> 512 at 14 x 14, images: 40 12.7 / 12.3, 48 12.6 / 13.6, 64 (one round)
+//    13.0 / 15.4, 65 21.5 / 15.2, 96 21.8 / 21.4, 112 22.6 / 22.1, 128 (two) 22.6 / 24.2, 192 (three) 34.4 / 33.2; at 10 x 10, whose tiles are
+//    39 % full, 96 21.1 / 14.0; 1024 -> 512, 10000 pixels 23.3 / 22.5, 19600 44.0 / 36.0
+bool dw_pw_wins(int C, int O, int batch, int OH, int OW)
+{
+    const int chunks = (C + 63) / 64;
+    const long long pixels = (long long)batch * OH * OW;
+    if (chunks == 1)
+        return O <= 512;
+    if (O <= 128)
+        return pixels >= (chunks <= 3 ? 0 : chunks <= 5 ? 2304 : std::max(9216, 1200 * chunks));
+    if (O > 512 || (O == 512 && chunks > 8))
+        return false;
+    const int tw = tile_columns(OW);
+    const long long groups = (long long)batch * ((OH + 7) / 8) * ((OW + tw - 1) / tw) * (O / 256), rounds = (groups + num_cus() - 1) / num_cus();
+    if (rounds == 1)
+        return pixels >= std::max(9216, 1000 * chunks);
+    return O == 512 ? rounds == 2 && pixels >= 23400 : pixels >= rounds * (9600 + 800 * chunks);
+}
 
 bool dw_pw_takes(const n2d2hip_conv_s* dw, const n2d2hip_conv_s* pw)
 {
@@ -557,12 +599,7 @@ int n2d2hip_dw_pw_pays(n2d2hip_dw_pw_t h, int batch, int in_h, int in_w)
     int OH, OW;
     if (n2d2hip_conv_out_dims(&h->dw->desc, in_h, in_w, &OH, &OW) != N2D2HIP_OK)
         return 0;
-    const long long pixels = (long long)batch * OH * OW;
-    // With more than 256 outputs the depthwise part is computed once per 256 of them.  A work-group of 256 outputs takes 9 us for
-    // its first tile, so that launches of fewer than two thirds of a tile a unit lose: 256 -> 256 at 28 x 28, this and two
-    // launches, us: 8 images 9.4 8.4, 12 9.6 10.6, 16 9.8 10.9, 64 18.4 and 35.  Up to 128 outputs it wins at every size; below
-    // 32768 pixels n2d2hip_dw_pw_small_*, which knows one more kernel, decides.
-    return h->pw->desc.O <= 256 && pixels >= (h->pw->desc.O > 128 ? 9216 : 32768) ? 1 : 0;
+    return dw_pw_wins(h->dw->desc.C, h->pw->desc.O, batch, OH, OW) ? 1 : 0;
 }
 
 int n2d2hip_dw_pw_forward(n2d2hip_dw_pw_t h, const n2d2hip_tensor* in, const n2d2hip_tensor* out, n2d2hip_stream_t stream_)
@@ -594,14 +631,7 @@ int n2d2hip_dw_pw_forward(n2d2hip_dw_pw_t h, const n2d2hip_tensor* in, const n2d
     a.dw_lo = h->dw->act->args.lo; a.dw_hi = h->dw->act->args.hi;
     a.C = dd.C; a.O = dp.O;
     a.H = in->H; a.W = in->W; a.OH = OH; a.OW = OW; a.padL = dd.padL; a.padT = dd.padT;
-    // columns of a tile: 16, or fewer when that leaves fewer idle columns in the last tile of a row
-    int best_tw = 16;
-    long long best_cols = ((OW + 15) / 16) * 16;
-    for (int tw = 15; tw >= 8; --tw) {
-        const long long cols = (long long)((OW + tw - 1) / tw) * 16;
-        if (cols < best_cols) { best_cols = cols; best_tw = tw; }
-    }
-    a.tw = best_tw;
+    a.tw = tile_columns(OW);
     a.tiles_x = (OW + a.tw - 1) / a.tw;
     a.tiles_y = (OH + 7) / 8;
     const long long ntiles = (long long)in->B * a.tiles_y * a.tiles_x;

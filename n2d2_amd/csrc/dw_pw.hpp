@@ -1,5 +1,6 @@
 // Interface between the two kernels that run a 3x3 depthwise convolution and the 1x1 convolution that reads it in one launch,
-// dw_pw.hip for many pixels and dw_pw_small.hip for few: what they take, from the cells alone.
+// dw_pw.hip for many pixels and dw_pw_small.hip for few: what they take, from the cells alone, and where the first is faster
+// than the cells' own launches.
 #pragma once
 
 #include "conv_handle.hpp"
@@ -8,6 +9,7 @@ namespace n2d2hip {
 
 bool dw_pw_takes(const n2d2hip_conv_s* dw, const n2d2hip_conv_s* pw);
 bool dw_pw_small_takes(const n2d2hip_conv_s* dw, const n2d2hip_conv_s* pw);
+bool dw_pw_wins(int C, int O, int batch, int OH, int OW);
 
 inline int byte_type_of(const n2d2hip_act_s* a) { return a->min_out >= 0 ? N2D2HIP_U8B : N2D2HIP_I8; }
 inline bool plain_1x1(const n2d2hip_conv_desc& d)

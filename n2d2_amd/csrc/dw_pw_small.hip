@@ -29,9 +29,7 @@ namespace {
 // general rescale needs
 enum { DWS_W, DWS_C = 3, DWS_D, DWS_E, DWS_BIAS, DWS_A, DWS_B, DWS_ROWS = 12 };
 constexpr int OUTS = 32, PIXELS = 16, MAX_PARTS = 8;
-// the kernel for many pixels is considered too: up to 128 outputs at every size, up to 512 from so many pixels
-constexpr int TILES_OUTS = 128, TILES_WIDE_OUTS = 512;
-constexpr long long TILES_WIDE_PIXELS = 9216;
+constexpr int TILES_OUTS = 128;                   // a handle of at most so many outputs holds the kernel for many pixels too
 constexpr int STAGE_PIXELS = 9 * PIXELS * 64, STAGE = STAGE_PIXELS + DWS_ROWS * 64 * 4;      // bytes of LDS of a wave
 
 struct DwPwSmallArgs {
@@ -173,15 +171,11 @@ bool integer_bytes(const n2d2hip_act_s* a)
 
 long long work_groups(int O, long long pixels) { return (pixels + PIXELS - 1) / PIXELS * (O / OUTS); }
 
-// That kernel gives a work-group 8 x 16 pixels and all their outputs, up to 256.  us, that kernel / this one / two launches, up to
-// 128 outputs: 32 -> 64 channels, 112 x 112 3.6 / 4.8 / 7.6, two images of 48 x 48 3.4 / 4.1 / 7.5; 64 -> 128 stride 2, 56 x 56
-// 4.6 / 4.3 / 8.1, two 4.6 / 5.1 / 8.2; 128 -> 128, 56 x 56 5.1 / 4.6 / 6.6, two 5.2 / 6.7 / 7.0, four 5.3 / 10.0 / 8.0, two of 24 x 24
-// 5.7 / 4.1 / 5.9.  With 512 outputs it computes the depthwise part twice and fills the chip later; that kernel / two launches,
-// 512 -> 512 at 14 x 14: 32 images 14.3 / 12.9, 48 15.0 / 15.9, 64 15.8 / 17.9, 128 26.8 / 28.2 (1024 outputs: 24.7 / 15.0 at 64).
-bool tiles_first(int C, int O, long long pixels)
-{
-    return O <= TILES_OUTS ? C == 32 || work_groups(O, pixels) > 1024 : O <= TILES_WIDE_OUTS && pixels >= TILES_WIDE_PIXELS;
-}
+// Where both are faster than the cells' own launches: is the kernel for many pixels the faster one?  It gives a work-group 8 x 16
+// pixels and all their outputs, up to 256.  us, that kernel / this one: 32 -> 64 channels, 112 x 112 3.6 / 4.8, two images of 48 x 48
+// 3.4 / 4.1; 64 -> 128 stride 2, 56 x 56 4.6 / 4.3, two 4.6 / 5.1; 128 -> 128, 4096 pixels 5.1 / 4.7, 5184 5.1 / 5.2, two images of 56 x 56
+// 5.2 / 6.7, four 5.3 / 10.0; 64 -> 256, 2304 pixels 4.9 / 4.8, 4096 5.0 / 5.3; 64 -> 512, 1369 4.9 / 4.9, 2304 5.0 / 5.6.
+bool tiles_first(int C, int O, long long pixels) { return (C == 32 && O <= TILES_OUTS) || work_groups(O, pixels) > 1024; }
 
 // Is this kernel faster than the cells' own launches?
 bool small_wins(int C, int O, long long pixels)
@@ -311,9 +305,10 @@ int n2d2hip_dw_pw_plan(n2d2hip_conv_t dw, n2d2hip_conv_t pw, int batch, int in_h
         return N2D2HIP_DW_PW_APART;
     const int C = dw->desc.C, O = pw->desc.O;
     const long long pixels = (long long)batch * OH * OW;
-    if (dw_pw_takes(dw, pw) && tiles_first(C, O, pixels))
+    const bool tiles = dw_pw_takes(dw, pw) && dw_pw_wins(C, O, batch, OH, OW), small = dw_pw_small_takes(dw, pw) && small_wins(C, O, pixels);
+    if (tiles && (!small || tiles_first(C, O, pixels)))
         return N2D2HIP_DW_PW_TILES;
-    return dw_pw_small_takes(dw, pw) && small_wins(C, O, pixels) ? N2D2HIP_DW_PW_SMALL : N2D2HIP_DW_PW_APART;
+    return small ? N2D2HIP_DW_PW_SMALL : N2D2HIP_DW_PW_APART;
 }
 
 int n2d2hip_dw_pw_small_pays(n2d2hip_dw_pw_small_t h, int batch, int in_h, int in_w)
@@ -324,7 +319,8 @@ int n2d2hip_dw_pw_small_pays(n2d2hip_dw_pw_small_t h, int batch, int in_h, int i
     if (n2d2hip_conv_out_dims(&h->dw->desc, in_h, in_w, &OH, &OW) != N2D2HIP_OK)
         return 0;
     const long long pixels = (long long)batch * OH * OW;
-    return choose_tiles(h, pixels) || small_wins(h->dw->desc.C, h->pw->desc.O, pixels) ? 1 : 0;
+    const int C = h->dw->desc.C, O = h->pw->desc.O;
+    return choose_tiles(h, pixels) ? dw_pw_wins(C, O, batch, OH, OW) : small_wins(C, O, pixels);
 }
 
 int n2d2hip_dw_pw_small_forward(n2d2hip_dw_pw_small_t h, const n2d2hip_tensor* in, const n2d2hip_tensor* out, n2d2hip_stream_t stream_)

@@ -573,17 +573,12 @@ bool ConvCell_Frame_HIP<T>::fuseDepthwise(Cell_Frame_HIP* depthwise)
     if (mDwPw || !mConv || !depthwise || !depthwise->convHandle() || depthwise->foldedInto() || foldedInto() || mInputs.size() != 1
         || depthwise->parentCells().size() != 1 || depthwise->inputTensor(0)->desc().halo != 0)
         return false;
-    n2d2hip_dw_pw_t fused = nullptr;
-    const int rc = n2d2hip_dw_pw_create(depthwise->convHandle(), mConv, &fused);
-    if (rc == N2D2HIP_ERR_UNSUPPORTED)
+    // (the depthwise cell's output can no longer be read then: small pairs stay two launches, whatever the library would gain)
+    const n2d2hip_tensor &x = depthwise->inputTensor(0)->desc(), &y = mOutputs.desc();
+    if ((long long)y.B * y.H * y.W < (y.C > 128 ? 9216 : 32768)
+        || n2d2hip_dw_pw_plan(depthwise->convHandle(), mConv, x.B, x.H, x.W) != N2D2HIP_DW_PW_TILES)
         return false;
-    checkStatus(rc);
-    const n2d2hip_tensor& x = depthwise->inputTensor(0)->desc();
-    if (!n2d2hip_dw_pw_pays(fused, x.B, x.H, x.W)) {
-        n2d2hip_dw_pw_destroy(fused);
-        return false;
-    }
-    mDwPw = fused;
+    checkStatus(n2d2hip_dw_pw_create(depthwise->convHandle(), mConv, &mDwPw));
     mFusedDw = depthwise;
     depthwise->setFoldedInto(this);
     return true;

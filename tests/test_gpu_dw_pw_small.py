@@ -102,3 +102,37 @@ def test_network_lays_out_only_the_pairs_it_launches(batch, image, monkeypatch):
     fused = [cell for l, cell, fn in net.steps if isinstance(cell, rt.DwPw)]
     assert len(fused) == len(net.dw_pws) + len(net.dw_pws_small) >= 3
     assert made == [type(cell) for cell in fused]
+
+
+@pytest.mark.parametrize("C,O,stride,sizes", [
+    (32, 64, 1, {(1, 1): "tiles", (4, 28): "tiles"}),                                               # one chunk of channels: always ahead
+    (64, 128, 1, {(1, 7): "small", (1, 50): "small", (1, 70): "tiles", (1, 200): "tiles"}),
+    (128, 128, 2, {(1, 14): "small", (2, 56): "tiles", (16, 56): "tiles"}),
+    (512, 128, 1, {(1, 14): "small", (1, 56): "apart", (2, 64): "apart", (1, 100): "tiles"}),        # many chunks: the launch is as long as they are
+    (1024, 64, 1, {(1, 14): "small", (1, 100): "apart", (1, 128): "apart", (1, 140): "tiles"}),
+    (256, 256, 1, {(1, 14): "small", (8, 28): "apart", (12, 28): "tiles", (33, 28): "tiles", (65, 28): "tiles"}),
+    (512, 256, 1, {(1, 14): "small", (8, 28): "apart", (12, 28): "tiles", (32, 28): "tiles", (33, 28): "apart", (48, 28): "tiles"}),
+    (512, 512, 1, {(1, 14): "small", (32, 14): "apart", (48, 14): "tiles", (64, 14): "tiles", (65, 14): "apart", (96, 14): "apart", (128, 14): "tiles",
+                   (192, 14): "apart", (96, 10): "apart"}),
+    (1024, 512, 1, {(1, 7): "small", (64, 14): "apart"}),
+    (512, 1024, 1, {(1, 7): "small", (64, 14): "apart"}),
+])
+def test_plan_follows_the_measured_lines(C, O, stride, sizes):
+    """What the library plans on a chip of 256 compute units, (images, output rows and columns) by (images, rows and columns); the
+    handles' own questions agree with it."""
+    import torch
+    from n2d2_amd import capi, runtime as rt
+    from oracle.cells import ActSpec
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines were measured with 256 compute units")
+    rng = np.random.default_rng(3)
+    spec = lambda n: ActSpec("Rectifier", "FixedMult32", rng.integers(2 ** 7, 2 ** 8, size=n), frac_bits=16, nb_bits=8, unsigned_out=True)
+    dw = rt.Conv(rng.integers(-128, 128, size=(C, 1, 3, 3)), None, rt.Act(C, **spec(C).kwargs()), capi.U8B, stride=(stride,) * 2, pad=(1,) * 4, groups=C)
+    pw = rt.Conv(rng.integers(-128, 128, size=(O, C, 1, 1)), None, rt.Act(O, **spec(O).kwargs()), capi.U8B)
+    tiles, small = rt.DwPw.create(dw, pw), rt.DwPwSmall.create(dw, pw)
+    for (B, H), want in sizes.items():
+        kind = rt.dw_pw_kind(dw, pw, B, H * stride, H * stride)
+        assert {None: "apart", rt.DwPw: "tiles", rt.DwPwSmall: "small"}[kind] == want, (B, H)
+        pays = tiles.pays(B, H * stride, H * stride), small.pays(B, H * stride, H * stride)
+        assert any(pays) == (want != "apart") and (want != "tiles" or pays[0]) and (want != "small" or pays[1]), (B, H, pays)
+    assert capi.lib.n2d2hip_dw_pw_plan(None, pw.handle, 1, 8, 8) == capi.lib.n2d2hip_dw_pw_plan(dw.handle, pw.handle, 0, 8, 8) == capi.DW_PW_APART
