@@ -1126,6 +1126,10 @@ bool ElemWiseCell_Frame_HIP::fuseIntoConv(size_t k, Cell_Frame_HIP* conv)
 {
     if (!mEw || mInputs.size() != 2 || k > 1 || !conv || !conv->convHandle() || mFusedConv || conv->parentCells().size() != 1)
         return false;
+    // (a launch that computes a depthwise cell writes the convolution's own output)
+    const auto* pointwise = dynamic_cast<const ConvCell_Frame_HIP<float>*>(conv);
+    if (pointwise && pointwise->computesDepthwise())
+        return false;
     const int rc = n2d2hip_conv_fuse_sum(conv->convHandle(), mEw, (int)k, sourceOf(mFoldedScaling, mInputs, 1 - k)->desc().dtype);
     if (rc == N2D2HIP_ERR_UNSUPPORTED)
         return false;

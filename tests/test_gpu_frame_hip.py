@@ -979,3 +979,24 @@ def test_replace_input_before_initialize_changes_what_a_cell_reads(fh):
     rewired = cells.run_net(spec, x, keep=["c"])["c"]
     assert not np.array_equal(straight, rewired)
     assert np.array_equal(net.outputs("c"), rewired)
+
+
+@pytest.mark.parametrize("batch,size", [(4, 96), (2, 24)])
+def test_depthwise_pair_in_front_of_a_residual_sum(fh, batch, size):
+    """A depthwise ConvCell, the 1x1 ConvCell that reads it and the sum that reads that (an inverted residual block): the 1x1 cell
+    computes the depthwise cell or the sum in its launch, not both; large enough for the pair to be one launch, and not."""
+    from n2d2_amd import nets
+    from oracle import cells
+    b = nets._Builder("inverted", (3, size, size), 43, "SingleShift")
+    t = b.conv("stem", "input", 64, 3, pad=1)
+    u = b.conv("dw", t, 64, 3, pad=1, groups=64)
+    u = b.conv("pw", u, 64, 1, kind="Linear")
+    t = b.sum("sum", [u, t])
+    t = b.pool("pool", t, "avg", size, size)
+    b.fc("fc", t, 10, mode="None")
+    x = np.random.default_rng(43).integers(0, 256, size=(batch, 3, size, size))
+    net = _compare(fh, b.spec, x, ["sum", "fc"])
+    assert net.nb_folded == 1
+    gpu = nets.GpuNet(b.spec, batch)
+    gpu.set_input(x)
+    assert np.array_equal(gpu.forward().to_numpy(), cells.run_net(b.spec, x)["fc"].astype(np.int64))
