@@ -16,10 +16,14 @@ _TORCH_DT = {capi.U8: torch.uint8, capi.I8: torch.int8, capi.U8B: torch.int8, ca
 _NP_DT = {capi.U8: np.uint8, capi.I8: np.int8, capi.U8B: np.int8, capi.I32: np.int32, capi.F32: np.float32}
 
 
+# Asked of torch's binding itself: building a torch.cuda.Stream around it took 2.9 of the 6.9 us a small cell's launch costs the
+# host.  A torch without that (private) function has the stream object.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda device: torch.cuda.current_stream(device).cuda_stream)
+
+
 def stream_ptr():
-    """The current stream of the current device.  Asked of torch's binding itself: building a torch.cuda.Stream around it took
-    2.9 of the 6.9 us a small cell's launch costs the host."""
-    return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+    """The current stream of the current device."""
+    return C.c_void_p(_raw_stream(torch.cuda.current_device()))
 
 
 class DTensor:
