@@ -839,11 +839,12 @@ class GpuNet:
         return self.forward()
 
     def capture(self, forwards=1, with_input_conversion=False):
-        """Records `forwards` forwards, one behind the other, into a HIP graph (every launch of the C ABI goes to the
-        capturing stream and none of them allocates or clears memory) and returns a callable that replays it.  More than
-        one forward per graph spreads the cost of launching a graph over them: a network of one or two kernels is
-        otherwise timed by that cost.  with_input_conversion: each forward is preceded by the graph-edge conversion of the
-        byte planes set_input() left on the device."""
+        """Returns a callable that runs `forwards` forwards, one behind the other, with the buffers of now, on the stream that is
+        current when it is called: the replay of a HIP graph recorded here (every launch of the C ABI goes to the capturing
+        stream and none of them allocates or clears memory), or, for one forward that is a single launch, that launch itself.
+        More than one forward per graph spreads the cost of launching a graph over them: a network of one or two kernels is
+        otherwise timed by that cost.  with_input_conversion: each forward is preceded by the graph-edge conversion of the byte
+        planes set_input() left on the device."""
         import torch
         self.forward()
         torch.cuda.synchronize()
@@ -860,8 +861,9 @@ class GpuNet:
         self._graph = graph
         replay_graph = graph.replay
         if forwards == 1 and self._run_steps == len(self.steps) and self._run_steps > 0:
-            # a graph of one launch costs more than the launch (14.1 against 8.6 us for one LeNet image): the same launch, with
-            # the same buffers, without it
+            # a graph of one launch costs more than the launch (14.1 against 8.4 us for one LeNet image): the same launch, with
+            # the same buffers, without it.  (The graph is recorded all the same: this launch takes 8.40 us in a process that has
+            # recorded one and 8.48 in one that has not, six processes of each.)
             src = self.input_src if with_input_conversion else None
             if src is None or (self._input_plain is None and self.cell_run.takes_edge(src)):
                 replay_graph = lambda: self.cell_run.forward(src)      # noqa: E731

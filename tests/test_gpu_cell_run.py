@@ -57,7 +57,7 @@ def test_cells_in_one_launch_bit_exact(case, batch):
     got = run.tensors[b.spec.output].to_numpy()
     want = cells.run_net(b.spec, img[:3])[b.spec.output].astype(np.int64)
     assert np.array_equal(got[:3], want)
-    # from the byte planes, replayed from a graph with other work between the replays
+    # from the byte planes, replayed (from a graph where the conversion is a launch of its own) with other work between the replays
     edge_in_launch = run.cell_run.takes_edge(run.input_src)
     assert edge_in_launch == (shape[0] <= 4)
     replay = run.capture(1, with_input_conversion=True)
@@ -66,6 +66,26 @@ def test_cells_in_one_launch_bit_exact(case, batch):
             run.tensors[n].buf.fill_(7)
         assert np.array_equal(replay().to_numpy(), got)
         assert np.array_equal(run.input.buf.cpu().numpy(), apart.input.buf.cpu().numpy())
+
+
+def test_captured_forward_of_a_single_launch_is_that_launch():
+    """One forward of a network that is one launch is replayed as the launch itself, two as a graph; both on the stream that is
+    current at the call."""
+    import torch
+    from n2d2_amd import capi, nets
+    net = nets.GpuNet(nets.lenet(), 2)
+    net.set_input(np.random.default_rng(5).integers(0, 256, size=(2, 1, 32, 32)))
+    want = net.forward().to_numpy()
+    side = torch.cuda.Stream()
+    for replay, launches in ((net.capture(), 1), (net.capture(1, with_input_conversion=True), 1), (net.capture(2), 0)):
+        for stream in (torch.cuda.current_stream(), side):
+            net.tensors[net.spec.output].buf.fill_(7)
+            torch.cuda.synchronize()
+            with torch.cuda.stream(stream), capi.launch_log() as log:
+                replay()
+            torch.cuda.synchronize()
+            assert len(log.entries) == launches
+            assert np.array_equal(net.tensors[net.spec.output].to_numpy(), want)
 
 
 @pytest.mark.parametrize("shape", [(1, 1, 2, 2), (3, 1, 32, 32), (5, 3, 7, 4), (2, 4, 6, 10), (2, 2, 5, 5), (513, 3, 33, 36)])
