@@ -4,9 +4,9 @@
 // With 64 x 64 tiles such a layer is a few dozen work-groups, and each walks its K steps one behind the other: a step of the
 // pipelined kernel takes about 640 cycles there, most of them the LDS's latency and a barrier between four waves that have
 // their SIMDs to themselves (3 x 3, 512 -> 512, 7 x 7: 36 steps, 13 us on 32 of 256 compute units).  Here a work-group owns
-// 32 (or 64) pixels x 32 channels, so four times as many of them share the layer, and its waves share K: wave w takes
-// every NW-th step of 128 bytes through a ring of its own (direct loads to LDS, no barrier: a wave waits for its own
-// loads only), so that NW steps are under way at once.  At the end the partial sums, 32-bit integers, meet in LDS, and
+// 32 pixels x 32 channels, so four times as many of them share the layer, and its waves share K: wave w takes
+// every fourth step of 128 bytes through a ring of its own (direct loads to LDS, no barrier: a wave waits for its own
+// loads only), so that four steps are under way at once.  At the end the partial sums, 32-bit integers, meet in LDS, and
 // every thread finishes four channels of a pixel.  The same layer: 6.2 us.  Whole nets, us: ResNet-50 1 image 331 -> 239,
 // 5 of 193 x 193 341 -> 280, 16 403 -> 391; ResNet-18 W4A4 1 image 188 -> 114, 16 214 -> 180; MobileNet 1 image 114 -> 106.
 //
@@ -20,18 +20,21 @@ namespace n2d2hip {
 
 namespace {
 
-// NW: waves; NJ: 32-pixel blocks of a tile; S: ring stages of a wave; VALID, W4: as conv_pipe_kernel; RAW: no rescale
-template <int NW, int NJ, int S, int VALID, bool W4, bool RAW>
+// Four waves of two stages: eight of two, four of four (128 KB) and tiles of 64 pixels were nowhere ahead by more than 3 %.
+constexpr int NW = 4, S = 2;               // waves, ring stages of a wave
+
+// VALID, W4: as conv_pipe_kernel; RAW: no rescale
+template <int VALID, bool W4, bool RAW>
 __global__ __launch_bounds__(NW * 64) void conv_split_kernel(ConvPipeArgs q)
 {
     const ConvArgs& p = q.c;
     constexpr int BK = 128, KH = BK / 32;
-    constexpr int A_CH = 4 * NJ, B_CH = W4 ? 2 : 4;        // 1 KB loads per stage: 8 rows of pixels or weights, or half a weight chunk
+    constexpr int A_CH = 4, B_CH = W4 ? 2 : 4;             // 1 KB loads per stage: 8 rows of pixels or weights, or half a weight chunk
     constexpr int LPI = A_CH + B_CH;
     constexpr int STAGE = LPI * 1024;
     constexpr int RP = 36;                                 // ints per pixel of the partial sums: 32 and a pad that spreads the banks
-    constexpr int ITEMS = (32 * NJ * 8 + NW * 64 - 1) / (NW * 64);      // dwords of output per thread
-    static_assert(NW * 32 * NJ * RP * 4 <= NW * S * STAGE, "the partial sums fit the rings");
+    constexpr int ITEMS = 32 * 8 / (NW * 64);              // dwords of output per thread
+    static_assert(NW * 32 * RP * 4 <= NW * S * STAGE, "the partial sums fit the rings");
     static_assert(LPI * (S - 1) < 60, "vmcnt is a 6-bit counter");
     __shared__ __attribute__((aligned(16))) unsigned char smem[NW * S * STAGE];
     const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) unsigned char*)smem;
@@ -44,7 +47,7 @@ __global__ __launch_bounds__(NW * 64) void conv_split_kernel(ConvPipeArgs q)
     if (idx >= q.mtiles * p.ntiles_n)
         return;
     const int tile_n = div_magic(idx, q.xcd_mul, q.xcd_sh);
-    const int m0 = (idx - tile_n * q.mtiles) * 32 * NJ, n0 = tile_n * 32;
+    const int m0 = (idx - tile_n * q.mtiles) * 32, n0 = tile_n * 32;
 
     // ---- loads: lane l of a 1 KB load fills 16-byte slot l, row l / 8; swz_k() places logical slots
     const int lrow = lane >> 3;
@@ -119,7 +122,7 @@ __global__ __launch_bounds__(NW * 64) void conv_split_kernel(ConvPipeArgs q)
         const int oy = div_magic(rem, q.ow_mul, q.ow_sh);
         const int ox = rem - oy * p.OW;
         auto place = [&](int halo) { return (b * (p.OH + 2 * halo) + oy + halo) * (p.OW + 2 * halo) + ox + halo; };
-        pixel[u] = m < p.M && ch < p.out_cs && (tid >> 3) + u * (NW * 8) < 32 * NJ ? place(q.out_halo) : -1;
+        pixel[u] = m < p.M && ch < p.out_cs ? place(q.out_halo) : -1;
         other[u] = 0u;
         if (!RAW && q.res && pixel[u] >= 0)
             other[u] = *(const unsigned*)(q.res + (long long)place(q.res_halo) * q.res_cs + ch);
@@ -147,24 +150,20 @@ __global__ __launch_bounds__(NW * 64) void conv_split_kernel(ConvPipeArgs q)
         wa[kk] = lds0 + wave * (S * STAGE) + A_CH * 1024
                + (W4 ? (kk / 2) * 1024 + l32 * 32 + (((2 * (kk % 2) + lh) ^ ((l32 >> 3) & 3)) << 3) : swz_k<BK>(l32, 2 * kk + lh));
     }
-    v16i acc[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-        acc[j] = v16i{};
+    v16i acc = v16i{};
     int slot = 0;
     for (int i = 0; i < n; ++i) {
         // loads answer in order; the tables' and the residual's were issued behind the first S steps: at the latest after the first
         // wait of the tail everything has landed
         if (i + S <= n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPI * (S - 1)) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        v4i fp[NJ][KH], fw[KH];
+        v4i fp[KH], fw[KH];
         v2i fw4[KH];
 #pragma unroll
         for (int kk = 0; kk < KH; ++kk) {
             if (W4) lds_read64_nowait<0>(fw4[kk], wa[kk] + slot * STAGE);
             else lds_read128_nowait<0>(fw[kk], wa[kk] + slot * STAGE);
-            lds_read128_nowait<0>(fp[0][kk], pa[kk] + slot * STAGE);
-            if (NJ > 1) lds_read128_nowait<4096>(fp[NJ - 1][kk], pa[kk] + slot * STAGE);
+            lds_read128_nowait<0>(fp[kk], pa[kk] + slot * STAGE);
         }
         wait_lgkm<0>();
 #pragma unroll
@@ -179,35 +178,30 @@ __global__ __launch_bounds__(NW * 64) void conv_split_kernel(ConvPipeArgs q)
             } else {
                 tie(fw[kk]);
             }
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) tie(fp[j][kk]);
+            tie(fp[kk]);
         }
         if (i + S < n)
             issue(wave + (i + S) * NW, slot);
         slot = slot + 1 == S ? 0 : slot + 1;
 #pragma unroll
         for (int kk = 0; kk < KH; ++kk)
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-                acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fw[kk], fp[j][kk], acc[j], 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fw[kk], fp[kk], acc, 0, 0, 0);
     }
 
-    // ---- the partial sums meet: lane (l32, lh) holds, for pixel l32 of block j, channels 8 g + 4 lh + e in acc[j][4 g + e]
+    // ---- the partial sums meet: lane (l32, lh) holds, for pixel l32, channels 8 g + 4 lh + e in acc[4 g + e]
     __syncthreads();                                       // (every wave has read its last stage; no load is under way)
     int* red = (int*)smem;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-            *(v4i*)(red + ((wave * NJ + j) * 32 + l32) * RP + 8 * g + 4 * lh) = v4i{acc[j][4 * g], acc[j][4 * g + 1], acc[j][4 * g + 2], acc[j][4 * g + 3]};
+    for (int g = 0; g < 4; ++g)
+        *(v4i*)(red + (wave * 32 + l32) * RP + 8 * g + 4 * lh) = v4i{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < ITEMS; ++u) {
-        const int m = min((tid >> 3) + u * (NW * 8), 32 * NJ - 1);
+        const int m = (tid >> 3) + u * (NW * 8);
         v4i v = *(const v4i*)(red + m * RP + (tid & 7) * 4);
 #pragma unroll
         for (int w = 1; w < NW; ++w)
-            v += *(const v4i*)(red + (w * NJ * 32 + m) * RP + (tid & 7) * 4);
+            v += *(const v4i*)(red + (w * 32 + m) * RP + (tid & 7) * 4);
         if (pixel[u] < 0)
             continue;
         if (RAW) {
@@ -252,34 +246,33 @@ __global__ __launch_bounds__(NW * 64) void conv_split_kernel(ConvPipeArgs q)
     }
 }
 
-template <int NW, int NJ, int S, int VALID>
+template <int VALID>
 void launch_kind(const ConvPipeArgs& a, bool w4, int grid, hipStream_t stream)
 {
     if (a.c.epi.kind == EPI_RAW) {
         if constexpr (VALID == 1)
-            N2D2HIP_LAUNCH_T(conv_split_kernel, (NW, NJ, S, VALID, false, true), dim3(grid), dim3(NW * 64), 0, stream, a);
+            N2D2HIP_LAUNCH_T(conv_split_kernel, (VALID, false, true), dim3(grid), dim3(NW * 64), 0, stream, a);
     } else if (w4) {
-        N2D2HIP_LAUNCH_T(conv_split_kernel, (NW, NJ, S, VALID, true, false), dim3(grid), dim3(NW * 64), 0, stream, a);
+        N2D2HIP_LAUNCH_T(conv_split_kernel, (VALID, true, false), dim3(grid), dim3(NW * 64), 0, stream, a);
     } else {
-        N2D2HIP_LAUNCH_T(conv_split_kernel, (NW, NJ, S, VALID, false, false), dim3(grid), dim3(NW * 64), 0, stream, a);
+        N2D2HIP_LAUNCH_T(conv_split_kernel, (VALID, false, false), dim3(grid), dim3(NW * 64), 0, stream, a);
     }
 }
 
-template <int NW, int NJ, int S>
 void launch(ConvPipeArgs a, int valid, bool w4, hipStream_t stream)
 {
     a.c.niter = a.c.ktot / 128;
     a.cper = a.c.in_cs / 128;
-    a.mtiles = (a.c.M + 32 * NJ - 1) / (32 * NJ);
+    a.mtiles = (a.c.M + 31) / 32;
     const int tiles = a.mtiles * a.c.ntiles_n;
     a.mlanes = (tiles + 7) / 8;
     magic_div((unsigned)a.mtiles, &a.xcd_mul, &a.xcd_sh);
     magic_div((unsigned)a.cper, &a.cper_mul, &a.cper_sh);
     a.kw_mul = 65536 / a.kW + 1;
     const int grid = 8 * a.mlanes;
-    if (valid == 1) launch_kind<NW, NJ, S, 1>(a, w4, grid, stream);
-    else if (valid == 2) launch_kind<NW, NJ, S, 2>(a, w4, grid, stream);
-    else launch_kind<NW, NJ, S, 0>(a, w4, grid, stream);
+    if (valid == 1) launch_kind<1>(a, w4, grid, stream);
+    else if (valid == 2) launch_kind<2>(a, w4, grid, stream);
+    else launch_kind<0>(a, w4, grid, stream);
 }
 
 } // namespace
@@ -308,8 +301,7 @@ bool conv_split_pays(long long M, int O, int ktot, bool w4, bool sum)
 int conv_split_launch(ConvPipeArgs a, int valid, bool w4, hipStream_t stream)
 {
     N2D2HIP_REQUIRE(a.c.epi.kind == EPI_I24 || (a.c.epi.kind == EPI_RAW && valid == 1 && !w4), N2D2HIP_ERR_INVALID, "conv_split: rescale not served");
-    // four waves of two stages; eight of two, four of four (128 KB) and 64-pixel tiles were nowhere ahead by more than 3 %
-    launch<4, 1, 2>(a, valid, w4, stream);
+    launch(a, valid, w4, stream);
     N2D2HIP_HIP_CHECK(hipGetLastError());
     return N2D2HIP_OK;
 }
