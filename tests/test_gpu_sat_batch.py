@@ -1,5 +1,5 @@
 """The SAT weight quantizers of many tensors in one call: what one call for each tensor gives, bit for bit, at the sizes where a
-tensor changes from one block of 1, 4 or 16 values a thread to many blocks, and past one launch's 16 tensors."""
+tensor changes from one block of 1, 4, 8, 12 or 16 values a thread to many blocks, and past one launch's 16 tensors."""
 import ctypes as C
 
 import numpy as np
@@ -8,15 +8,16 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 SIZES = [1, 2, 1023, 1024, 1025, 4096, 4097, 16384, 16385, 16400, 70001, 300000, 5, 9, 333, 20000, 64, 17000]
+MORE = [12288, 8192, 8193, 12289]          # (the first of them, the 19th tensor, is compared with the formula)
 
 
-@pytest.mark.parametrize("count", [1, 3, 16, 18])
+@pytest.mark.parametrize("count", [1, 3, 16, 18, 22])
 def test_batch_equals_single_calls(count):
     import torch
     from n2d2_amd import capi, runtime as rt
     print("sat batch", count, flush=True)
     lib, rng = capi.lib, np.random.default_rng(count)
-    sizes = SIZES[-count:] if count < 16 else SIZES[:count]
+    sizes = SIZES[-count:] if count < 16 else (SIZES + MORE)[:count]
     ws = int(lib.n2d2hip_quantizer_workspace_bytes(max(sizes)))
     dev = lambda a: torch.from_numpy(a.astype(np.float32)).cuda()
     items, grads, one, keep = [], [], [], []
