@@ -315,6 +315,9 @@ typedef struct n2d2hip_run_cell { /* one of the three, the others NULL; fcs only
 typedef struct n2d2hip_cell_run_s* n2d2hip_cell_run_t;
 int n2d2hip_cell_run_create(int nb_cells, const n2d2hip_run_cell* cells, int H, int W, n2d2hip_cell_run_t* run);
 int n2d2hip_cell_run_destroy(n2d2hip_cell_run_t run);
+/* 1 where a run is expected to be faster than its cells' own launches on so many images (measured rule, at the function), else
+ * 0: a planner's question, before the run is created. */
+int n2d2hip_cell_run_pays(int images);
 /* `in`: the first cell's input (NHWC, no halo); `outs`: the output of every cell (nb_cells of them).  `edge`: NULL, or the
  * network's byte planes (NCHW U8 for a U8B input, I8 for I8, at most 4 channels): `in` is then written from them first, as
  * n2d2hip_convert(edge, in) does, in the same launch. */

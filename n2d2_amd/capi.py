@@ -37,7 +37,7 @@ SYMBOLS = [
     "n2d2hip_dw_pw_create", "n2d2hip_dw_pw_destroy", "n2d2hip_dw_pw_forward", "n2d2hip_dw_pw_pays", "n2d2hip_dw_pw_plan",
     "n2d2hip_dw_pw_small_create", "n2d2hip_dw_pw_small_destroy", "n2d2hip_dw_pw_small_forward", "n2d2hip_dw_pw_small_pays",
     "n2d2hip_fc_create", "n2d2hip_fc_destroy", "n2d2hip_fc_forward", "n2d2hip_fc_chain_create", "n2d2hip_fc_chain_destroy", "n2d2hip_fc_chain_forward",
-    "n2d2hip_cell_run_create", "n2d2hip_cell_run_destroy", "n2d2hip_cell_run_forward",
+    "n2d2hip_cell_run_create", "n2d2hip_cell_run_destroy", "n2d2hip_cell_run_forward", "n2d2hip_cell_run_pays",
     "n2d2hip_pool_out_dims", "n2d2hip_pool_forward", "n2d2hip_pool_writes_halo", "n2d2hip_pool_forward_mapped",
     "n2d2hip_elemwise_create", "n2d2hip_elemwise_destroy", "n2d2hip_elemwise_forward", "n2d2hip_elemwise_fold_input_scaling", "n2d2hip_concat_channels",
     "n2d2hip_quantizer_workspace_bytes", "n2d2hip_sat_weight_forward_batch", "n2d2hip_sat_weight_backward_batch",
@@ -156,6 +156,7 @@ def load():
     lib.n2d2hip_fc_chain_forward.argtypes = [P, P, P, P]
     lib.n2d2hip_cell_run_create.argtypes = [I, P, I, I, P]
     lib.n2d2hip_cell_run_destroy.argtypes = [P]
+    lib.n2d2hip_cell_run_pays.argtypes = [I]
     lib.n2d2hip_cell_run_forward.argtypes = [P, P, P, P, P]
     lib.n2d2hip_pool_out_dims.argtypes = [P, I, I, P, P]
     lib.n2d2hip_pool_forward.argtypes = [P, P, P, P]

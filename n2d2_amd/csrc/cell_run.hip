@@ -6,10 +6,11 @@
 // a work-group of 8 waves takes one image through all the cells with its tensors in LDS; what a cell hands to the next
 // costs a barrier instead of a launch.  Each cell's output is also stored to its tensor, as the cells run in turn do (the
 // stores wait for nobody), so a caller finds the same values everywhere.  LeNet, conversion of the bytes included: one image
-// 33.9 -> 8.6 us, 256 images launched one by one 45.7 -> 14.8 us, 2048 images 82 -> 66 us, 16384 images (64 one after the other on
-// a compute unit) 463 -> 456 us: the cells' own launches, which then fill the chip, are never ahead.  Of the launch's 8 us, 2 go by until the image and the weights
-// are there, 3 in the first convolution (instruction issue), and the other five cells take about 0.5 each: a descriptor, a
-// few dependent LDS reads and a barrier.  16 waves took as long (each pays for its cells' descriptors and set-up).
+// 33.9 -> 8.4 us, 256 images launched one by one 45.7 -> 11.4 us.  Of the launch's 8 us, 2 go by until the image and the weights are
+// there, 3 in the first convolution (instruction issue), and the other five cells take about 0.5 each: a descriptor, a few
+// dependent LDS reads and a barrier.  16 waves took as long (each pays for its cells' descriptors and set-up).  With many images
+// the cells' own launches fill the chip and overtake it: cells and run, us, 1024 images 56.4 and 35.3, 2048 82.2 and 66.2, 4096 130.1
+// and 127.6, 6144 179.0 and 188.5, 8192 230.7 and 249.8, 16384 458 and 495 (n2d2hip_cell_run_pays).
 //
 //  * Convolutions run on the matrix cores, 16 channels x 16 pixels a tile (v_mfma_i32_16x16x64_i8): a lane's 16 bytes of K
 //    are one tap of a 16-channel pixel, or four taps of a 4-channel pixel, read from LDS where they lie; the 16 x 16 tile
@@ -731,6 +732,11 @@ int n2d2hip_cell_run_create(int nb_cells, const n2d2hip_run_cell* cells, int H, 
     r->long_fc = a.kper > 32;
     *out = r;
     return N2D2HIP_OK;
+}
+
+int n2d2hip_cell_run_pays(int images)
+{
+    return images > 0 && images <= 16 * num_cus() ? 1 : 0;       // (16 images one after the other on a compute unit: measured above)
 }
 
 int n2d2hip_cell_run_forward(n2d2hip_cell_run_t r, const n2d2hip_tensor* edge, const n2d2hip_tensor* in, const n2d2hip_tensor* outs, n2d2hip_stream_t stream)

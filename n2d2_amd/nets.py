@@ -410,8 +410,8 @@ class GpuNet:
         fc_chains: run two or three fully-connected cells, each the only reader of the one before, as one launch
         (n2d2hip_fc_chain_*) where the library takes them.
         cell_runs: forward() runs the small convolutions, max poolings and fully-connected cells a network begins with as one
-        launch (n2d2hip_cell_run_*) where the library takes them; every tensor is written all the same, and what addresses
-        the cells one by one (forward_subset, forward_timed, kernel_names) still launches them one by one.
+        launch (n2d2hip_cell_run_*) where the library takes them and expects that to be faster; every tensor is written all the
+        same, and what addresses the cells one by one (forward_subset, forward_timed, kernel_names) still launches them one by one.
         chains: run a block's 3x3 convolution in the launch of the expanding 1x1 convolution + sum that alone reads it
         (n2d2hip_conv_chain_*) where the library takes the pair: the 3x3 convolution's output stays on the chip.  Where the
         library expects two launches to be faster (n2d2hip_conv_chain_pays) the step makes two."""
@@ -668,7 +668,7 @@ class GpuNet:
         self.launched = [spec.layers[k] for k in keep]
         # the cells the network begins with, each reading the one before, as one launch
         self.cell_run, self._run_steps = None, 0
-        if fuse and cell_runs:
+        if fuse and cell_runs and rt.CellRun.pays(batch):
             self._plan_cell_run()
 
     def _plan_cell_run(self):

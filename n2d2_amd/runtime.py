@@ -381,6 +381,11 @@ class CellRun:
         self._outs = (capi.Tensor * len(outs))(*[o.desc for o in outs])
 
     @staticmethod
+    def pays(images):
+        """Does the library expect a run to be faster than its cells' own launches on so many images?"""
+        return bool(lib.n2d2hip_cell_run_pays(images))
+
+    @staticmethod
     def create(cells, x, outs):
         """cells: Conv and Pool objects in order, a FcChain possibly last; x: the first one's input; outs: their outputs.
         None when the library keeps the cells apart."""

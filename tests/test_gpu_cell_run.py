@@ -68,6 +68,15 @@ def test_cells_in_one_launch_bit_exact(case, batch):
         assert np.array_equal(run.input.buf.cpu().numpy(), apart.input.buf.cpu().numpy())
 
 
+def test_run_is_planned_up_to_sixteen_images_a_compute_unit():
+    import torch
+    from n2d2_amd import nets, runtime as rt
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    spec = nets.lenet()
+    assert nets.GpuNet(spec, 16 * cus).cell_run is not None and nets.GpuNet(spec, 16 * cus + 1).cell_run is None
+    assert rt.CellRun.pays(1) and not rt.CellRun.pays(0)
+
+
 def test_captured_forward_of_a_single_launch_is_that_launch():
     """One forward of a network that is one launch is replayed as the launch itself, two as a graph; both on the stream that is
     current at the call."""
