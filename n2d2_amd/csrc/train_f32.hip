@@ -997,22 +997,33 @@ static bool depthwise_strips(const ConvF32& q)
 }
 static unsigned reduce_grid(size_t n) { return (unsigned)std::min<size_t>((n + 63) / 64, 16384); }
 
-// Short sums of a few dozen channels: a block of 1024 per channel and tap row, whose blocks find each other's strips in the
-// caches, is ahead of ranges and the launch that adds them up (64 channels, 112 x 112, stride 2, batch 8: 10.1 against 12.7 us),
-// while it has blocks for the chip and all run side by side.
-static bool depthwise_filter_by_rows(const ConvF32& q)
+// Short sums: a block per channel and tap row (of so many threads; 0: none), whose blocks find each other's strips in the caches.
+// Ahead of ranges of all taps, whose K * K sums take a block as long to add up as some hundred strips, and of the launch
+// that adds the ranges, until the strips are many or, with many channels, the tensors no longer lie in the L2.  us, a block of 256 /
+// 512 / 1024 per tap row / ranges:
+//   3x3, channels, strips: 8, 224 4.0 / 4.0 / 4.2 / 5.6; 8, 3136 9.3 / 6.7 / 6.2 / 11.0; 48, 6400 14.3 / 9.7 / 8.7 / 11.2; 128, 480 4.8 / 4.9 / 6.1 / 6.9;
+//     128, 12544 37.3 / 29.8 / 34.2 / 28.2; 256, 3200 12.2 / 11.1 / 11.6 / 13.6; 256, 12544 41.8 / 39.2 / 41.6 / 29.7; 512, 784 8.8 / 9.9 / 13.9 / 10.4;
+//     512, 3136 31.7 / 40.5 / 40.5 / 26.5; 1024, 448 9.1 / 13.1 / 22.6 / 9.7; 1024, 1568 21.1 / 25.1 / 28.7 / 19.9
+//   5x5: 8, 200 4.2 / 4.3 / 5.3 / 9.9; 8, 12800 29.1 / 19.8 / 17.3 / 20.1; 8, 25088 53.2 / 35.0 / 30.2 / 21.2; 128, 784 6.9 / 7.7 / 11.1 / 14.7;
+//     128, 12800 50.5 / 45.6 / 42.5 / 41.9; 512, 1568 20.5 / 21.4 / 31.6 / 25.3; 512, 6272 77.0 / 75.7 / 75.9 / 62.0; 1024, 1600 38.0 / 41.6 / 62.3 / 43.4;
+//     stride 2, 1024, 512 40.7 / 44.1 / 57.8 / 24.8
+static int depthwise_row_threads(const ConvF32& q)
 {
-    const int items = q.B * q.oH * ceil_div_i(q.oW, 4), blocks = q.C * q.kH;
-    return items > 6 * 256 && items <= 8 * 1024 && 2 * blocks >= num_cus() && blocks <= 2 * num_cus();
+    const long items = (long)q.B * q.oH * ceil_div_i(q.oW, 4), blocks = (long)q.C * q.kH;
+    if (items > (q.kH == 3 ? 8192 : 12800) || items * q.C > 1600000 / q.sx / (blocks > 2560 ? 2 : 1)) return 0;
+    if (items > 2048 && blocks <= 1024) return 1024;
+    return items > 512 && blocks <= 512 ? 512 : 256;
 }
 // Ranges the strips of a channel are split into for its filter gradient: enough for eight blocks of 256 on every compute unit,
 // but no fewer than six strips a thread.  us, at 2 / 3 / 6 / 12 strips: 128 channels, 56 x 56, batch 32 30.8 / 31.4 / 31.1 / 32.6;
 // 512, 14 x 14, batch 64 20.0 / 20.2 / 20.0 / 20.3; 8, 56 x 56, batch 32 10.3 / 10.0 / 11.9 / 15.4; 96, 5x5, 56 x 56, batch 16
 // 41.8 / 37.0 / 33.9 / 33.1 (a block per channel and tap row: 48.6, 27.6, 25.4, 36.2).
+// The workspace query answers for them; with few channels (blocks for less than half of the chip) also where a block per tap row
+// takes the sum without, as a batch that is a little larger will need it.
 static int depthwise_filter_ranges(const ConvF32& q)
 {
     const int items = q.B * q.oH * ceil_div_i(q.oW, 4);
-    return depthwise_filter_by_rows(q) ? 1 : std::max(1, std::min(ceil_div_i(items, 6 * 256), ceil_div_i(8 * num_cus(), q.C)));
+    return depthwise_row_threads(q) && 2 * q.C * q.kH >= num_cus() ? 1 : std::max(1, std::min(ceil_div_i(items, 6 * 256), ceil_div_i(8 * num_cus(), q.C)));
 }
 static size_t depthwise_filter_bytes(const ConvF32& q, int ranges) { return ranges > 1 ? (size_t)ranges * q.C * q.kH * q.kW * sizeof(double) : 0; }
 
@@ -1028,18 +1039,23 @@ static int run_depthwise(const ConvF32& q, int pass, const float* a, const float
         if (pass == PASS_FWD) hipLaunchKernelGGL((depthwise_f32_forward_kernel<K, S>), grid, dim3(256), 0, st, k, a, b, bias, beta, out);
         else if (pass == PASS_BWD_FILTER) {
             // (without the workspace that the query names, or with one that holds no doubles: one range)
-            int ranges = depthwise_filter_ranges(q);
+            const int row_threads = depthwise_row_threads(q);
+            int ranges = row_threads ? 1 : depthwise_filter_ranges(q);
             if (workspace_bytes < depthwise_filter_bytes(q, ranges) || (size_t)workspace % sizeof(double)) ranges = 1;
             const int per_range = ceil_div_i(k.items, ranges);
             ranges = ceil_div_i(k.items, per_range);
             constexpr int WIDE = K == 3 ? 1024 : 512;
-            if (depthwise_filter_by_rows(q))
-                hipLaunchKernelGGL((depthwise_f32_filter_kernel<K, S, 1024, 1>), dim3(q.C, 1, K), dim3(1024), 0, st, k, per_range, a, b, beta, out, nullptr);
+            const auto by_rows = [&](auto T) {
+                constexpr int THREADS = decltype(T)::value;
+                N2D2HIP_LAUNCH_T(depthwise_f32_filter_kernel, (K, S, THREADS, 1), dim3(q.C, 1, K), dim3(THREADS), 0, st, k, per_range, a, b, beta, out, (double*)nullptr);
+            };
+            if (row_threads == 1024) by_rows(std::integral_constant<int, 1024>{});
+            else if (row_threads == 512) by_rows(std::integral_constant<int, 512>{});
+            else if (row_threads == 256) by_rows(std::integral_constant<int, 256>{});
             else if (ranges == 1 && k.items > 6 * 256)
-                hipLaunchKernelGGL((depthwise_f32_filter_kernel<K, S, WIDE, K>), dim3(q.C), dim3(WIDE), 0, st, k, per_range, a, b, beta, out, nullptr);
+                N2D2HIP_LAUNCH_T(depthwise_f32_filter_kernel, (K, S, WIDE, K), dim3(q.C), dim3(WIDE), 0, st, k, per_range, a, b, beta, out, (double*)nullptr);
             else
-                hipLaunchKernelGGL((depthwise_f32_filter_kernel<K, S, 256, K>), dim3(q.C, ranges), dim3(256), 0, st, k, per_range, a, b, beta, out,
-                                   (double*)workspace);
+                N2D2HIP_LAUNCH_T(depthwise_f32_filter_kernel, (K, S, 256, K), dim3(q.C, ranges), dim3(256), 0, st, k, per_range, a, b, beta, out, (double*)workspace);
             const size_t n = (size_t)q.C * K * K;
             if (ranges > 1)
                 hipLaunchKernelGGL(conv_f32_reduce_partials_kernel<double>, dim3(reduce_grid(n)), dim3(256), 0, st, (const double*)workspace, ranges, n, beta, out,
