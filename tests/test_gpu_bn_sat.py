@@ -109,3 +109,23 @@ def test_quantizer_gradient_on_the_way_in(shape, beta, to_input):
     assert abs(out[0][-1][0] - out[1][-1][0]) <= 2 * 2.0 ** -23 * max(1.0, abs(out[0][-1][0]))
     assert lib.n2d2hip_batchnorm_f32_backward_sat(*head, fp.data_ptr(), 15.0, alpha.data_ptr(), beta, da.data_ptr(), d.data_ptr(), *tail[:-3], None, 0,
                                                   rt.stream_ptr()) == capi.ERR_WORKSPACE
+
+
+@pytest.mark.parametrize("B,Cn,H,W,block", [(64, 300, 3, 3, 256), (16, 5, 8, 8, 256), (16, 3, 8, 32, 256), (17, 3, 8, 32, 1024), (41, 7, 5, 5, 1024), (40, 7, 5, 5, 256)])
+def test_a_channel_of_few_units_is_added_by_a_small_block(B, Cn, H, W, block):
+    """A block of 1024 threads from 1025 units (values, or quads where the planes hold whole ones) a channel on; mean and variance
+    against 64 bits on either side of the line."""
+    import torch
+    from n2d2_amd import capi, runtime as rt
+    print("bn block", B, Cn, H, W, flush=True)
+    x = torch.from_numpy(np.random.default_rng(B).normal(2.0, 3.0, (B, Cn, H, W)).astype(np.float32)).cuda()
+    y, v = torch.empty_like(x), [torch.full((Cn,), float(i < 1 or i == 3), device="cuda") for i in range(6)]
+    ws = torch.empty(int(capi.lib.n2d2hip_batchnorm_f32_workspace_bytes(B, Cn, H, W)), dtype=torch.uint8, device="cuda")
+    with capi.launch_log() as log:
+        capi.check(capi.lib.n2d2hip_batchnorm_f32_forward(B, Cn, H, W, x.data_ptr(), *(t.data_ptr() for t in v), 1e-5, 0.1, 0, y.data_ptr(), ws.data_ptr(),
+                                                          ws.numel(), rt.stream_ptr()))
+    assert [e[2] for e in log.entries if e[0].startswith("batchnorm_f32_stats_kernel")] == [block]
+    x64 = x.double()
+    m64, v64 = x64.mean((0, 2, 3)), x64.var((0, 2, 3), unbiased=False)
+    assert float((v[4].double() - m64).abs().max()) <= float(m64.abs().max()) * 2.0 ** -23
+    assert float(((v[5].double() - v64) / v64).abs().max()) <= 2.0 ** -22
