@@ -177,8 +177,7 @@ int depthwise3x3_launch(DepthwiseArgs a, int stride, int num_cus, hipStream_t st
     N2D2HIP_REQUIRE((stride == 1 || stride == 2) && a.cs % 4 == 0, N2D2HIP_ERR_INVALID, "depthwise3x3: stride %d, channel stride %d", stride, a.cs);
     a.cq = (unsigned)(a.cs / 4);
     // A strip re-reads the two input rows above it and computes whole turns of the kernel's loop, and a compute unit needs
-    // some waves: strips of a multiple of a turn's rows, up to 8 (14 rows gain 2 % more on large planes and lose 4 % at
-    // 64 x 256 x 28 x 28), as long as the chip holds 400 threads a unit.  Strips that filled 1024 threads a unit were up to
+    // some waves: strips of a multiple of a turn's rows, up to 8, as long as the chip holds 400 threads a unit.  Strips that filled 1024 threads a unit were up to
     // four times as many, and of rows that left turns half empty.  us by rows of a strip, images x channels x height x width:
     //   64 x 512 x 14 x 14   2: 11.6   4: 7.7   5 (the former rule): 9.1   8: 7.3
     //   64 x 1024 x 7 x 7    2: 7.2    4: 5.2   3 (the former rule): 6.5   8: 4.9
@@ -194,6 +193,14 @@ int depthwise3x3_launch(DepthwiseArgs a, int stride, int num_cus, hipStream_t st
     const long long rows = (a.OH + nstrips - 1) / nstrips, whole = (rows + turn - 1) / turn * turn;
     // (with less than 100 threads a unit left, a turn is time to wait for and no work: 1 x 512 x 14 x 14 3.00 at 2 rows, 3.04 at 4)
     a.rows = (int)std::min<long long>(columns * ((a.OH + whole - 1) / whole) * 4 >= want ? whole : rows, 8);
+    // Layers that fill the chip several times over are bound by what they read: longer strips, up to 28 rows (14 with stride 2, there
+    // from 800 threads a row and unit), as long as 1600 threads a unit are left.  us, 8 rows and these: 64 x 512 x 56 x 56 59.2 / 46.4,
+    // 128 x 1024 x 28 x 28 62.4 / 46.2, 64 x 1024 x 28 x 28 30.7 / 26.6, 16 x 256 x 112 x 112 31.4 / 27.2, 64 x 128 x 56 x 56 18.4 / 17.5;
+    // stride 2, 128 x 256 x 28 x 28 23.3 / 21.6, 256 x 512 x 14 x 14 22.2 / 21.3.
+    if (stride == 1 || columns >= 2 * want) {
+        const long long most = stride == 1 ? 28 : 14, parts = std::max((4 * want + columns - 1) / columns, (a.OH + most - 1) / most);
+        a.rows = std::max(a.rows, (int)(((a.OH + parts - 1) / parts + turn - 1) / turn * turn));
+    }
     a.nstrips = (a.OH + a.rows - 1) / a.rows;
     const long long nthreads = columns * a.nstrips;
     N2D2HIP_REQUIRE(nthreads < (1ll << 31), N2D2HIP_ERR_UNSUPPORTED, "depthwise3x3: tensor too large");
