@@ -463,7 +463,8 @@ int tile_columns(int OW)
 //    21.2 / 19.3; 37632 14.4 / 18.1 and 23.0 / 27.4; 1024 -> 256, 32400 44.9 / 38.5, 40000 45.2 / 47.5
 //  * 512 outputs, each tile's depthwise part computed twice: 512 -> 512 at 14 x 14, images: 40 12.7 / 12.3, 48 12.6 / 13.6, 64 (one round)
 //    13.0 / 15.4, 65 21.5 / 15.2, 96 21.8 / 21.4, 112 22.6 / 22.1, 128 (two) 22.6 / 24.2, 192 (three) 34.4 / 33.2; at 10 x 10, whose tiles are
-//    39 % full, 96 21.1 / 14.0; 1024 -> 512, 10000 pixels 23.3 / 22.5, 19600 44.0 / 36.0
+//    39 % full, 96 21.1 / 14.0; at 13 x 13, 118 21.7 / 20.6, 128 21.6 / 21.7; 1024 -> 512, 10000 pixels 23.3 / 22.5, 19600 44.0 / 36.0.  (Level ones run as one
+//    launch: in MobileNet-v1, 128 images of 193 x 193, that is 383 us where two launches a pair are 395.)
 bool dw_pw_wins(int C, int O, int batch, int OH, int OW)
 {
     const int chunks = (C + 63) / 64;
@@ -478,7 +479,7 @@ bool dw_pw_wins(int C, int O, int batch, int OH, int OW)
     const long long groups = (long long)batch * ((OH + 7) / 8) * ((OW + tw - 1) / tw) * (O / 256), rounds = (groups + num_cus() - 1) / num_cus();
     if (rounds == 1)
         return pixels >= std::max(9216, 1000 * chunks);
-    return O == 512 ? rounds == 2 && pixels >= 23400 : pixels >= rounds * (9600 + 800 * chunks);
+    return O == 512 ? rounds == 2 && pixels >= 20800 : pixels >= rounds * (9600 + 800 * chunks);
 }
 
 bool dw_pw_takes(const n2d2hip_conv_s* dw, const n2d2hip_conv_s* pw)

@@ -112,7 +112,7 @@ def test_network_lays_out_only_the_pairs_it_launches(batch, image, monkeypatch):
     (1024, 64, 1, {(1, 14): "small", (1, 100): "apart", (1, 128): "apart", (1, 140): "tiles"}),
     (256, 256, 1, {(1, 14): "small", (8, 28): "apart", (12, 28): "tiles", (33, 28): "tiles", (65, 28): "tiles"}),
     (512, 256, 1, {(1, 14): "small", (8, 28): "apart", (12, 28): "tiles", (32, 28): "tiles", (33, 28): "apart", (48, 28): "tiles"}),
-    (512, 512, 1, {(1, 14): "small", (32, 14): "apart", (48, 14): "tiles", (64, 14): "tiles", (65, 14): "apart", (96, 14): "apart", (128, 14): "tiles",
+    (512, 512, 1, {(1, 14): "small", (32, 14): "apart", (48, 14): "tiles", (64, 14): "tiles", (65, 14): "apart", (96, 14): "apart", (128, 14): "tiles", (112, 14): "tiles",
                    (192, 14): "apart", (96, 10): "apart"}),
     (1024, 512, 1, {(1, 7): "small", (64, 14): "apart"}),
     (512, 1024, 1, {(1, 7): "small", (64, 14): "apart"}),
