@@ -1627,9 +1627,11 @@ static int bn_splits(int B, int C, int H, int W)
     return (int)std::max<size_t>(1, std::min<size_t>(std::min(by_size, by_grid), 64));
 }
 
-// Units of 16 bytes where the planes allow it; a block of 1024 threads where one of 256 would go round more than four times.  (More
-// than twice: no shape of 888 gained, forward and backward us with 256 and 1024 threads: 2048 channels, 64 x 3 x 3 13.9 / 21.3 and
-// 32.1 / 48.4, 512 channels 7.9 / 9.9 and 11.6 / 15.6, 16 channels, 8 x 9 x 9 7.2 / 8.5 and 8.2 / 10.0.)
+// Units of 16 bytes where the planes allow it.  One block a channel: 1024 threads where 256 would go round more than four times, and
+// 512 where they would more than twice and the channels leave every block a compute unit of its own.  us, forward / backward /
+// backward with the quantizer's gradient, 513 to 1024 units: 16 channels with 256 threads 7.4 / 8.5 / 11.0, 512 7.1 / 7.9 / 9.7, 1024
+// 8.3 / 10.4 / 12.3; 256 channels 8.1 / 9.5 / 12.1, 7.8 / 8.9 / 10.8, 9.0 / 11.4 / 13.5; 512 channels 9.0 / 11.0 / 14.6, 9.8 / 12.1 /
+// 14.9, 12.7 / 17.3 / 21.6; 2048 channels 16.7 / 24.2 / 32.3, 21.3 / 31.1 / 39.2, 34.7 / 53.3 / 67.6.
 struct BnLaunch {
     BnRange q;
     int V, block;
@@ -1642,7 +1644,7 @@ static BnLaunch bn_launch(int B, int C, int plane, int splits, uintptr_t pointer
     if (n / l.V >= ((size_t)1 << 30)) l.V = 0;
     const int v = l.V ? l.V : 1;
     l.q = {C, plane, plane / v, div_of(plane / v), n / v, (n / v + splits - 1) / splits};
-    l.block = splits == 1 && l.q.units > 4 * TBLOCK ? 1024 : TBLOCK;
+    l.block = splits > 1 || l.q.units <= 2 * TBLOCK ? TBLOCK : l.q.units > 4 * TBLOCK ? 1024 : C <= num_cus() ? 512 : TBLOCK;
     return l;
 }
 

@@ -6,7 +6,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(3, 5, 1, 1), (2, 7, 9, 7), (40, 3, 7, 9), (2, 6, 8, 8), (5, 4, 10, 10), (3, 5, 9, 9), (130, 3, 9, 9), (140, 3, 7, 9), (33, 2, 16, 17), (20, 70, 32, 32)]
+SHAPES = [(3, 5, 1, 1), (2, 7, 9, 7), (40, 3, 7, 9), (2, 6, 8, 8), (5, 4, 10, 10), (32, 6, 10, 10), (3, 5, 9, 9), (130, 3, 9, 9), (140, 3, 7, 9), (33, 2, 16, 17), (20, 70, 32, 32)]
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
@@ -111,10 +111,11 @@ def test_quantizer_gradient_on_the_way_in(shape, beta, to_input):
                                                   rt.stream_ptr()) == capi.ERR_WORKSPACE
 
 
-@pytest.mark.parametrize("B,Cn,H,W,block", [(64, 300, 3, 3, 256), (16, 5, 8, 8, 256), (16, 3, 8, 32, 256), (17, 3, 8, 32, 1024), (41, 7, 5, 5, 1024), (40, 7, 5, 5, 256)])
+@pytest.mark.parametrize("B,Cn,H,W,block", [(64, 300, 3, 3, 256), (16, 5, 8, 8, 256), (32, 2, 8, 8, 256), (27, 256, 1, 19, 512),
+                                              (27, 257, 1, 19, 256), (16, 3, 8, 32, 512), (17, 3, 8, 32, 1024), (41, 7, 5, 5, 1024), (40, 7, 5, 5, 512)])
 def test_a_channel_of_few_units_is_added_by_a_small_block(B, Cn, H, W, block):
-    """A block of 1024 threads from 1025 units (values, or quads where the planes hold whole ones) a channel on; mean and variance
-    against 64 bits on either side of the line."""
+    """A block of 1024 threads from 1025 units (values, or quads where the planes hold whole ones) a channel on, of 512 from 513 where
+    256 compute units hold a channel each; mean and variance against 64 bits on either side of the lines."""
     import torch
     from n2d2_amd import capi, runtime as rt
     print("bn block", B, Cn, H, W, flush=True)
