@@ -169,8 +169,9 @@ __global__ __launch_bounds__(256) void depthwise_f32_data_kernel(DepthwiseF32 q,
 // What bounds it is the vector ALU: four instructions a product (multiply, select, conversion, addition in double).
 // 128 channels, 3x3, 56 x 56, batch 32: a block per channel and tap row, which loaded and converted dy's strip once per row
 // and stood on 384 blocks, 48.6 us; now 31.1 with the launch that adds the ranges up.
-// THREADS: 256; more where a range is a whole channel because the caller gave no workspace.  ROWS: tap rows of a block, all K or
-// one (blockIdx.z is which).
+// ROWS: tap rows of a block, all K, or one (blockIdx.z is which) where a channel's strips are few: depthwise_row_threads() in
+// train_f32.hip says where and measures both.  THREADS: 256; of one row, where blocks are few, 512 or 1024, and so of all rows where
+// a range is a whole channel because the caller gave no workspace.
 template <int K, int S, int THREADS, int ROWS>
 __global__ __launch_bounds__(THREADS) void depthwise_f32_filter_kernel(DepthwiseF32 q, int per_range, const float* __restrict__ x, const float* __restrict__ dy,
                                                                    float beta, float* __restrict__ dw, double* __restrict__ partial)
