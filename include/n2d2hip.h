@@ -194,6 +194,9 @@ enum {
     N2D2HIP_KERNEL_NO_DIRECT = 1024,/* integer cells with at most 4 input channels and 32 outputs: matrix-core kernel instead of the direct one */
     N2D2HIP_KERNEL_DIRECT = 2048,   /* the direct kernel wherever it can run (up to 16 input channels), also where the library finds the matrix cores faster */
     N2D2HIP_KERNEL_NO_SPLIT = 8192, /* integer cells: no kernel whose waves share K (layers of few output tiles) */
+    N2D2HIP_KERNEL_F32_TERMS = 32768, /* float passes: no forward sum on the bf16 matrix cores in parts.  Those are nearer to the sum in 64 bits than
+                                        the float kernels', but not the same, and a quantizer behind the layer turns the last bit into a level
+                                        now and then: for programs that compare a learning net's state with one kept before */
     N2D2HIP_KERNEL_SPLIT = 16384,   /* that kernel wherever it can run, also where the library finds the others faster */
     N2D2HIP_KERNEL_TILE_M256 = 4096 /* patch kernel: tiles of 256 positions (N2D2HIP_KERNEL_TILE_M128: of 128; _M64: four waves of 64 positions) instead of its own choice */
 };
@@ -522,7 +525,9 @@ int n2d2hip_lsq_backward(const float* diff_q, const float* fp_x, float* diff_fp,
  *
  * Ungrouped convolutions without dilation, of up to 64 taps or spanning their input, run on the matrix cores: forward from
  * 2e7 flops (spanning: up to 64 taps), backward-data, and backward-filter (in double below 2e7 flops and for spanning
- * kernels of more than 64 taps).  There sums are added in an order that follows from the sizes, not in the reference's.
+ * kernels of more than 64 taps).  There sums are added in an order that follows from the sizes, not in the reference's; forward
+ * and backward-data of several taps multiply on the bf16 matrix cores, each float as three bf16 numbers that add up to it, where
+ * that is faster (infinities and NaN come out as in float).
  * All others, and tensors of 2 GiB and more, run on direct kernels, which add forward and backward-data in the
  * reference's order and backward-filter in double.  kernel_choice N2D2HIP_KERNEL_F32_DIRECT asks for the direct
  * kernels, N2D2HIP_KERNEL_F32_GEMM for the matrix cores at any size.

@@ -13,6 +13,8 @@
 //  * operands go global -> LDS by direct loads (no registers on the way), into a ring of stages, and everything that does not
 //    differ from lane to lane is scalar: a load adds a scalar offset to a per-lane one.  What does not exist (padding, edges
 //    of tile and K range) is requested past the end of the buffer descriptor; the LDS receives 0.
+//  * kernels of several taps, forward and at stride 1 backward, are mostly left to the bf16 matrix cores (conv_f32_patch.hpp); what that
+//    kernel does not take (long rows, few channels), and forward where the caller asks for a rounding a term, stays here.
 //  * 3x3 kernels, forward and at stride 1 backward, keep a lane's nine offsets in registers, so that a load costs no vector
 //    instruction; 1x1 kernels and strided backward-data run K over chunks of 16 channels at one tap, so that the test whether
 //    the tap lies inside the input is made once per step.  A small kernel lays the weights out for both first.  Any other
@@ -31,7 +33,7 @@
 // Backward-filter, whose K is the whole batch of pixels and whose output is small, splits K over blockIdx.z into partial
 // results that a second kernel adds up in a fixed order; forward and backward-data do the same when their tiles alone would
 // not fill the chip.
-// Measured (us, forward / data / filter, before: 128 x 128 tiles, operands through registers, one test per load; now):
+// Measured on these kernels (us, forward / data / filter, before: 128 x 128 tiles, operands through registers, one test per load; now):
 //   64 -> 64, 3x3, 56 x 56, batch 64             236 / 284 / 263    149 / 157 / 180   (15 GFLOP: 99, 94, 82 TFLOP/s of 154)
 //   128 -> 256, 3x3 stride 2, 27 x 27, batch 33   80 / 277 /  76     55 /  54 /  58
 //   a layer spanning its input, 16384 -> 10, 64  2632 /  27 / 222    116 /   7 /   8
@@ -80,6 +82,9 @@ struct PixelGemm {
     int ptiles, ptiles8, qtiles;
     int qpad, T;               // chunked K: rows of q in the laid-out weights, taps of the kernel
     unsigned bytesX, bytesW;   // sizes of the operand tensors (below 2 GiB)
+    unsigned bytesO;           // of the result
+    int npos;                  // source pixels over all images
+    DivF32 dplane;             // by the source plane
     int nclass;
     PixelClass c[PIXEL_CLASSES];
 };

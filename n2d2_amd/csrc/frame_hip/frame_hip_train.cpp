@@ -355,6 +355,8 @@ n2d2hip_conv_desc ConvCell_FrameTrain_HIP<T>::desc() const
     d.dilX = (int)mDilationDims[0];
     d.dilY = (int)mDilationDims[1];
     d.groups = (int)mNbGroups;
+    // a level that a sum in parts moves is a step of the weights from then on
+    d.kernel_choice = N2D2HIP_KERNEL_F32_TERMS;
     return d;
 }
 

@@ -12,6 +12,7 @@
 
 #include "common.h"
 #include "conv_f32_gemm.hpp"
+#include "conv_f32_patch.hpp"
 #include "sat_math.hpp"
 #include "depthwise_f32.hpp"
 
@@ -1148,10 +1149,17 @@ static ConvF32 product_of(const ConvF32& q, int pass, int* as_pass)
 }
 
 // ---- forward and backward-data: tile shape and K ranges of a launch
+struct PatchShape {
+    int wq, wp, mq, np;        // a tile: 16 wq mq rows of q x 16 wp np pixels
+    int nu;                    // units of 128 source positions that hold what a tile's taps read; 0: more than the kernel takes
+    int pixels() const { return 16 * np * wp; }
+    int rows() const { return 16 * wq * mq; }
+};
 struct PixelPlan {
     bool small_q;              // tiles of 32 q x 128 pixels instead of 64 x 64
     int splits;                // K ranges that leave partial results
     int kind;                  // PIXELS_*
+    PatchShape patch;          // (PIXELS_PATCH)
     bool many;                 // a class has more tap rows and columns than a mask of 31 bits
     PixelGemm g;
 };
@@ -1196,7 +1204,47 @@ static std::vector<PixelClass> pixel_classes(const ConvF32& q, int pass)
     return v;
 }
 
-enum { PIXELS_TAPS, PIXELS_CHUNK, PIXELS_3X3 };
+enum { PIXELS_TAPS, PIXELS_CHUNK, PIXELS_3X3, PIXELS_PATCH };
+// Units of 128 source positions that hold what the taps of any `pixels` consecutive pixels of the class read: every step to the
+// next pixel is at least 0 and at most one of a row's, a row's end's and an image's end's.  0: a step back.
+static int patch_units(const ConvF32& q, int pass, const PixelClass& c, int pixels)
+{
+    const long sy = pass == PASS_FWD ? q.sy : 1, sx = pass == PASS_FWD ? q.sx : 1;
+    const long Hs = pass == PASS_FWD ? q.H : q.oH, Ws = pass == PASS_FWD ? q.W : q.oW, gH = c.gHW / c.gW, ny = c.nT / c.nx;
+    const long row = sy * Ws - c.gW * sx, image = Hs * Ws - gH * sy * Ws;        // beyond a step of sx; beyond that and `row`
+    if (sx + row < 0 || sx + row + image < 0) return 0;
+    const long n = pixels - 1;
+    const long span = n * sx + (n / c.gW + 1) * std::max(0L, row) + (n / c.gHW + 1) * std::max(0L, image) + (ny - 1) * Ws + c.nx;
+    return span <= 128 * 3 ? ceil_div_i(span, 128) : 0;
+}
+// Chunks of a class after which a float sum of the patch kernel is added to the one in double: where it has been rounded as often as
+// the longest float sum of the other kernels.  Theirs round once a term, this one 5 times in 32.
+static int patch_fold(const ConvF32& q, int pass, const PixelClass& c)
+{
+    const bool fwd = pass == PASS_FWD;
+    const long K = (long)(fwd ? q.C : q.O) * q.kH * q.kW;
+    const long ranges = pass_ranges((long)q.B * (fwd ? q.oH * q.oW : q.H * q.W), fwd ? q.O : q.C, K);
+    return (int)std::max(4 * (K / ranges) / (PK * c.nT), 1L);
+}
+// Tiles of 64 rows x 128 pixels where they fill three quarters of the chip's two blocks to a CU and need no sums in double (whose
+// registers they lack); else of 64 x 64.  us, 64 x 128 / 64 x 64, forward: 64 -> 64, 56 x 56, batch 64 (1568 of the larger tiles)
+// 90 / 105; 64 -> 64, 32 x 32, batch 64 (512) 34 / 38; 256 -> 256, 14 x 14, batch 32 (196) 65 / 60; 48 -> 96, 5x5, 30 x 30, batch
+// 16 (226) 54 / 42.  No shape for runs of more than 384 positions, which would leave one block to a CU: 64 -> 128, stride 2, 56 x
+// 56, batch 16 (456) 40 against 31 of the chunk kernel.
+static PatchShape patch_shape(const ConvF32& q, int pass, const PixelClass& c)
+{
+    const int Q = pass == PASS_FWD ? q.O : q.C, chunks = ceil_div_i(pass == PASS_FWD ? q.C : q.O, PK);
+    auto fit = [&](PatchShape s) {
+        s.nu = c.nx + c.nT / c.nx > 31 ? 0 : patch_units(q, pass, c, s.pixels());
+        return s;
+    };
+    if (Q <= 32) return fit(PatchShape{1, 4, 2, 2, 0});
+    if (patch_fold(q, pass, c) >= chunks && (long)ceil_div_i(c.P, 128) * ceil_div_i(Q, 64) >= 384) {
+        const PatchShape s = fit(PatchShape{2, 2, 2, 4, 0});
+        if (s.nu) return s;
+    }
+    return fit(PatchShape{2, 2, 2, 2, 0});
+}
 static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass> cls, int kind)
 {
     PixelPlan pl = {};
@@ -1215,16 +1263,20 @@ static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass>
     // tile shape
     long P = 0, kmax = 0;
     const int nchunks = ceil_div_i(g.Ch, GK);
-    const int kch = kind == PIXELS_CHUNK && (!fwd || T > 1) ? nchunks * GK : g.Ch;
+    const int kch = kind == PIXELS_PATCH ? round_up(g.Ch, PK) : kind == PIXELS_CHUNK && (!fwd || T > 1) ? nchunks * GK : g.Ch;
     for (const PixelClass& c : cls) { P += c.P; kmax = std::max(kmax, (long)kch * c.nT); }
     // (64 x 64 tiles, four to a CU, lost at most 4 % to the best of 32 x 128, 64 x 128 and 128 x 128 on every shape with Q
     // over 32 that was timed, and gained up to 70 % where the larger tiles are few)
     pl.small_q = g.Q <= 32;
-    const int PT = pl.small_q ? 128 : 64, QT = pl.small_q ? 32 : 64;
+    if (kind == PIXELS_PATCH) pl.patch = patch_shape(q, pass, cls[0]);
+    const int PT = kind == PIXELS_PATCH ? pl.patch.pixels() : pl.small_q ? 128 : 64, QT = kind == PIXELS_PATCH ? pl.patch.rows() : pl.small_q ? 32 : 64;
     g.qtiles = ceil_div_i(g.Q, QT);
     pl.kind = kind;
     g.T = T;
-    g.qpad = g.qtiles * QT;
+    g.qpad = kind == PIXELS_PATCH ? round_up(g.Q, 128) : g.qtiles * QT;
+    g.npos = q.B * g.planeS;
+    g.bytesO = (unsigned)(4 * (size_t)q.B * g.Q * g.planeO);
+    g.dplane = div_of(g.planeS);
     long tiles = 0;
     g.nclass = (int)cls.size();
     for (int i = 0; i < g.nclass; ++i) {
@@ -1236,6 +1288,17 @@ static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass>
     g.ptiles8 = ceil_div_i(tiles, 8);
     const long blocks = tiles * g.qtiles;
     g.nz = 1;
+    if (kind == PIXELS_PATCH) {
+        // ranges (of chunks) where the tiles alone would not give every CU a block
+        const int chunks = ceil_div_i(g.Ch, PK);
+        const int each = ceil_div_i(chunks, blocks >= 256 ? 1 : std::min<long>(chunks, std::max(1L, 512 / std::max(blocks, 1L))));
+        pl.splits = ceil_div_i(chunks, each);
+        const int fold = patch_fold(q, pass, cls[0]);
+        g.c[0] = cls[0];
+        g.c[0].kchunk = each;
+        g.c[0].fold = fold < each ? fold : 0;
+        return pl;
+    }
     long splits, least = q.ranges;
     if (fwd) {
         // The ranges of a forward sum follow from its sizes alone: with another order of additions the quantizer behind it would
@@ -1268,11 +1331,40 @@ static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass>
     return pl;
 }
 
+template <int WQ, int WP, int MQ, int NP, bool FOLDS>
+static void launch_patch(const PixelPlan& pl, dim3 grid, const float* x, const float* w, const float* wt, const float* bias, float beta, float* out, size_t partial,
+                         hipStream_t st)
+{
+    grid.x = std::min(grid.x, 8u * 32u * 2u);    // (two blocks to a CU)
+    const auto run = [&](auto nu_, auto nt_, auto fold_) {
+        hipLaunchKernelGGL((conv_f32_patch_kernel<WQ, WP, MQ, NP, 2 * decltype(nu_)::value, decltype(nt_)::value, decltype(fold_)::value>), grid, dim3(256), 0,
+                           st, pl.g, x, w, (const v4u*)wt, bias, beta, out, partial);
+    };
+    const auto taps = [&](auto nu_, auto fold_) {
+        pl.g.c[0].nT == 9 && pl.g.c[0].nx == 3 ? run(nu_, std::integral_constant<int, 9>{}, fold_)
+                                                                   : run(nu_, std::integral_constant<int, 0>{}, fold_);
+    };
+    const auto units = [&](auto fold_) {
+        pl.patch.nu <= 2 ? taps(std::integral_constant<int, 2>{}, fold_) : taps(std::integral_constant<int, 3>{}, fold_);
+    };
+    if constexpr (FOLDS) {
+        if (pl.g.c[0].fold) return units(std::true_type{});
+    }
+    units(std::false_type{});
+}
+
 template <bool BWD>
-static void launch_pixels(PixelPlan& pl, int splits, const float* x, const float* w, const float* bias, float beta, float* out, size_t partial,
+static void launch_pixels(PixelPlan& pl, int splits, const float* x, const float* w, const float* wt, const float* bias, float beta, float* out, size_t partial,
                           hipStream_t st)
 {
     const dim3 grid(pl.g.ptiles8 * 8 * pl.g.qtiles, 1, splits);
+    if (pl.kind == PIXELS_PATCH) {
+        if (pl.patch.wq == 1) launch_patch<1, 4, 2, 2, true>(pl, grid, x, w, wt, bias, beta, out, partial, st);
+        else if (pl.patch.np == 2) launch_patch<2, 2, 2, 2, true>(pl, grid, x, w, wt, bias, beta, out, partial, st);
+        else launch_patch<2, 2, 2, 4, false>(pl, grid, x, w, wt, bias, beta, out, partial, st);
+        return;
+    }
+    if (pl.kind != PIXELS_TAPS) w = wt;
     if (pl.kind == PIXELS_3X3) {
         if (pl.small_q) hipLaunchKernelGGL((conv_f32_3x3_kernel<1, 4>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
         else hipLaunchKernelGGL((conv_f32_3x3_kernel<2, 2>), grid, dim3(256), 0, st, pl.g, x, w, bias, beta, out, partial);
@@ -1376,7 +1468,8 @@ static void launch_filter(const FilterPlan& pl, const float* x, const float* dy,
     pl.g.kH + pl.g.kW > 31 ? pick(std::true_type{}) : pick(std::false_type{});
 }
 
-// The order of K.  3x3 kernels, forward or at stride 1: four channels with their taps at a time.  Chunks of 16 channels at one
+// The kernel and its order of K.  Kernels of several taps whose tiles read runs of source pixels that fit its LDS, with less than 2 / 5
+// of padding to 32 channels: the patch kernel, on the bf16 matrix cores.  Else 3x3 kernels, forward or at stride 1: four channels with their taps at a time.  Chunks of 16 channels at one
 // tap: 1x1 kernels, kernels of more than 31 rows and columns (1 x 64, 128 -> 128: 138 -> 113 us) and backward-data, where padding
 // the channels to them costs less than testing every load (about a fifth).  Both lay the weights out first (a launch of 3 us: even at 3 to 7e8 flops).
 static int pixels_kind(const ConvF32& q, int pass)
@@ -1384,6 +1477,10 @@ static int pixels_kind(const ConvF32& q, int pass)
     const int ch = pass == PASS_FWD ? q.C : q.O, T = q.kH * q.kW;
     if (2.0 * q.B * q.O * q.oH * q.oW * q.C * T < 5.0e8 || (size_t)(q.O + 64) * (q.C + 64) * (T + 2) >= ((size_t)1 << 28))
         return PIXELS_TAPS;
+    if (T > 1 && round_up(ch, PK) * 5 <= ch * 7 && !(pass == PASS_FWD && (q.choice & N2D2HIP_KERNEL_F32_TERMS))) {
+        // (backward-data at strides: the classes are few taps to a step each; 128 <- 256, stride 2, 27 x 27, batch 33: 58 us against 53)
+        if ((pass == PASS_FWD || (q.sx == 1 && q.sy == 1)) && patch_shape(q, pass, pixel_classes(q, pass)[0]).nu) return PIXELS_PATCH;
+    }
     if (q.kH == 3 && q.kW == 3 && (pass == PASS_FWD || (q.sx == 1 && q.sy == 1)) && round_up(ch, 4) * 5 <= ch * 7)
         return PIXELS_3X3;
     return (pass == PASS_BWD_DATA || T == 1 || q.kH + q.kW > 31) && round_up(ch, GK) * 5 <= ch * 6 ? PIXELS_CHUNK : PIXELS_TAPS;
@@ -1392,6 +1489,7 @@ static size_t laid_weights(const ConvF32& q, int pass, int kind)
 {
     const int ch = pass == PASS_FWD ? q.C : q.O, rows = pass == PASS_FWD ? q.O : q.C, qpad = round_up(rows, rows <= 32 ? 32 : 64);
     if (kind == PIXELS_TAPS) return 0;
+    if (kind == PIXELS_PATCH) return (size_t)ceil_div_i(ch, PK) * q.kH * q.kW * (round_up(rows, 128) / 16) * (PATCH_FRAG / 4);
     return kind == PIXELS_3X3 ? (size_t)(ch + 3) / 4 * qpad * W33 : (size_t)round_up(ch, GK) * q.kH * q.kW * qpad;
 }
 
@@ -1446,14 +1544,15 @@ static int run_pass(const ConvF32& q, int pass, const float* a, const float* b, 
         plans.push_back(plan_pixels(q, pass, std::vector<PixelClass>(cls.begin() + i, cls.begin() + std::min(cls.size(), i + PIXEL_CLASSES)), kind));
         splits = std::max(splits, plans.back().splits);
     }
-    const float* w = b;
+    const float* wt = ws;
     if (kind != PIXELS_TAPS) {
         const PixelGemm& g = plans[0].g;
-        const int total = (int)(kind == PIXELS_3X3 ? nlaid : nlaid / 4);
+        const int total = (int)(kind == PIXELS_3X3 ? nlaid : kind == PIXELS_PATCH ? nlaid / 12 : nlaid / 4);
         const dim3 grid(std::min((total + 255) / 256, 4096));
         if (kind == PIXELS_3X3) hipLaunchKernelGGL(conv_f32_lay_weights3x3_kernel, grid, dim3(256), 0, st, b, ws, total, g.Q, g.qpad, g.Ch, g.qs, g.chs);
+        else if (kind == PIXELS_PATCH)
+            hipLaunchKernelGGL(conv_f32_lay_parts_kernel, grid, dim3(256), 0, st, b, (v4u*)ws, total, g.Q, g.qpad / 16, g.Ch, g.T, g.qs, g.chs);
         else hipLaunchKernelGGL(conv_f32_lay_weights_kernel, grid, dim3(256), 0, st, b, ws, total, g.Q, g.qpad, g.Ch, g.T, g.qs, g.chs);
-        w = ws;
         ws += nlaid;
         ws_floats -= nlaid;
     }
@@ -1464,8 +1563,8 @@ static int run_pass(const ConvF32& q, int pass, const float* a, const float* b, 
     for (PixelPlan& pl : plans) {
         float* dst = splits > 1 ? ws : out;
         // (every launch runs the ranges of the pass, so that each partial result is complete)
-        if (pass == PASS_FWD) launch_pixels<false>(pl, splits, a, w, splits > 1 ? nullptr : bias, splits > 1 ? 0.0f : beta, dst, splits > 1 ? n : 0, st);
-        else launch_pixels<true>(pl, splits, a, w, nullptr, splits > 1 ? 0.0f : beta, dst, splits > 1 ? n : 0, st);
+        if (pass == PASS_FWD) launch_pixels<false>(pl, splits, a, b, wt, splits > 1 ? nullptr : bias, splits > 1 ? 0.0f : beta, dst, splits > 1 ? n : 0, st);
+        else launch_pixels<true>(pl, splits, a, b, wt, nullptr, splits > 1 ? 0.0f : beta, dst, splits > 1 ? n : 0, st);
     }
     if (splits > 1)
         hipLaunchKernelGGL(conv_f32_reduce_partials_kernel<float>, dim3(reduce_grid(n)), dim3(256), 0, st, (const float*)ws, splits, n, beta, out, bias,

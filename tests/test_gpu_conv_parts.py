@@ -1,0 +1,94 @@
+"""Float convolutions on the bf16 matrix cores, operands in three parts: forward and data gradient against float64 at the edges of the
+tiles, runs and channel chunks, and infinities, NaN and floats near the largest where a float sum has them."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# B, C, H, W, O, kH, kW, stride, pad, data gradient: rows and channels left over (97 rows, 39 channels), runs that cross images, pixels past
+# the last tile, 32 rows and less, other kernels than 3x3, strides, K ranges, sums in double
+CASES = [(33, 64, 32, 32, 64, 3, 3, 1, 1), (9, 39, 31, 33, 97, 3, 3, 1, 1), (70, 32, 13, 11, 31, 3, 3, 1, 1), (5, 64, 20, 112, 40, 3, 3, 1, 0), (21, 128, 27, 27, 70, 3, 3, 2, 1),
+         (12, 48, 29, 17, 80, 5, 5, 1, 2), (17, 64, 15, 40, 64, 2, 7, 1, 0), (2, 256, 14, 14, 256, 3, 3, 1, 1), (40, 96, 14, 15, 160, 3, 3, 1, 1), (64, 512, 7, 7, 129, 3, 3, 1, 1),
+         (4, 64, 60, 61, 33, 1, 9, 1, 4)]
+
+
+def _passes(x, w, dy, s, pad):
+    import torch
+    x64, w64 = (torch.from_numpy(v).double().requires_grad_() for v in (x, w))
+    y = torch.nn.functional.conv2d(x64, w64, stride=s, padding=pad)
+    y.backward(torch.from_numpy(dy).double())
+    return y.detach().numpy(), x64.grad.numpy()
+
+
+def _run(x, w, dy, s, pad, bias=None, beta=0.0, start=0.0, workspace=True):
+    import torch
+    from n2d2_amd import capi, runtime as rt
+    (B, Ci, H, W), (O, _, kH, kW) = x.shape, w.shape
+    d = capi.ConvDesc(Ci, O, kW, kH, s, s, pad[1], pad[0], pad[1], pad[0], 1, 1, 1, 0, 0)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    x_, w_, dy_, y, dx = dev(x), dev(w), dev(dy), torch.full(dy.shape, start, device="cuda"), torch.full(x.shape, start, device="cuda")
+    b_ = None if bias is None else dev(bias)
+    n = int(capi.lib.n2d2hip_conv2d_f32_workspace_bytes(C.byref(d), B, H, W)) if workspace else 0
+    ws = torch.empty(max(n, 16), dtype=torch.uint8, device="cuda")
+    p = ws.data_ptr() if n else None
+    capi.check(capi.lib.n2d2hip_conv2d_f32_forward(C.byref(d), B, H, W, x_.data_ptr(), w_.data_ptr(), None if b_ is None else b_.data_ptr(), beta, y.data_ptr(), p, n,
+                                                   rt.stream_ptr()))
+    capi.check(capi.lib.n2d2hip_conv2d_f32_backward_data(C.byref(d), B, H, W, w_.data_ptr(), dy_.data_ptr(), beta, dx.data_ptr(), p, n, rt.stream_ptr()))
+    torch.cuda.synchronize()
+    return y.cpu().numpy(), dx.cpu().numpy()
+
+
+def _inputs(case, seed=0):
+    B, Ci, H, W, O, kH, kW, s, p = case
+    pad = (p if kH > 1 else 0, p if kW > 1 else 0)
+    rng = np.random.default_rng(sum(case) + seed)
+    x, w = rng.normal(size=(B, Ci, H, W)).astype(np.float32), rng.normal(size=(O, Ci, kH, kW)).astype(np.float32)
+    dy = rng.normal(size=(B, O, (H + 2 * pad[0] - kH) // s + 1, (W + 2 * pad[1] - kW) // s + 1)).astype(np.float32)
+    return x, w, dy, s, pad, rng
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_against_float64(case):
+    """A sum of K terms is rounded 5 times in 32 terms (and no longer than the sums in float that it stands for, K times), each time by
+    2.53e-8 of it in the root mean square; the i-th of L equal steps is sqrt(i / L) of the last."""
+    print("parts", case, flush=True)
+    x, w, dy, s, pad, rng = _inputs(case)
+    want, mag = _passes(x, w, dy, s, pad), _passes(np.abs(x), np.abs(w), np.abs(dy), s, pad)
+    got = _run(x, w, dy, s, pad)
+    T = w.shape[2] * w.shape[3]
+    for g, t, m, k in zip(got, want, mag, (w.shape[1] * T, w.shape[0] * T)):
+        assert (np.abs(g - t) <= 2.0 ** -24 * (np.abs(t) + (k + 4) * m)).all()
+    # (the other kernels, which take short and padded passes, round once a term)
+    for g, t, k in zip(got, want, (w.shape[1] * T, w.shape[0] * T)):
+        assert np.linalg.norm(g - t) <= 1.1 * 2.53e-8 * np.sqrt(1 + k / 2) * np.linalg.norm(t)
+    bias = rng.normal(size=w.shape[0]).astype(np.float32)
+    y, dx = _run(x, w, dy, s, pad, bias=bias, beta=0.5, start=3.0)
+    assert np.abs(y - (got[0] + np.float32(1.5) + bias[None, :, None, None])).max() <= 2.0 ** -22 * (np.abs(got[0]).max() + 5)
+    assert np.abs(dx - (got[1] + np.float32(1.5))).max() <= 2.0 ** -22 * (np.abs(got[1]).max() + 2)
+
+
+@pytest.mark.parametrize("case", [(9, 39, 31, 33, 97, 3, 3, 1, 1), (40, 96, 14, 15, 160, 3, 3, 1, 1), (21, 128, 27, 27, 70, 3, 3, 2, 1)])
+def test_infinities_nan_and_the_largest_floats(case):
+    """An infinity in one operand gives infinities of the products' signs, NaN only against a zero or another infinity; a float that
+    rounds to infinity in bf16 is finite here."""
+    print("parts, special values", case, flush=True)
+    x, w, dy, s, pad, rng = _inputs(case, 1)
+    big = np.float32(3.4e38)
+    w *= np.float32(1e-3)
+    w[np.abs(w) < 1e-5] = 1e-5
+    w[3, 5, 1, 1] = 0.0
+    for t in (x, dy):
+        flat = t.reshape(-1)
+        at = rng.permutation(flat.size)[:12]
+        flat[at] = [np.inf, -np.inf, np.nan, big, -big, big, -big, big, np.inf, -big, 1e-42, -1e-42]
+    got = _run(x, w, dy, s, pad)
+    want = _passes(x, w, dy, s, pad)
+    fin = _passes(np.where(np.isfinite(x), x, 0), w, np.where(np.isfinite(dy), dy, 0), s, pad)
+    mag = _passes(np.abs(np.where(np.isfinite(x), x, 0)), np.abs(w), np.abs(np.where(np.isfinite(dy), dy, 0)), s, pad)
+    k = w.shape[1] * 9, w.shape[0] * 9
+    for g, t, f, m, n in zip(got, want, fin, mag, k):
+        assert np.array_equal(np.isnan(g), np.isnan(t)) and np.array_equal(g == np.inf, t == np.inf) and np.array_equal(g == -np.inf, t == -np.inf)
+        ok = np.isfinite(t)
+        assert (np.abs(g - f)[ok] <= 2.0 ** -24 * (np.abs(f) + (n + 4) * m)[ok]).all()
