@@ -13,6 +13,7 @@
 #include "common.h"
 #include "conv_f32_gemm.hpp"
 #include "conv_f32_patch.hpp"
+#include "conv_f32_filter_rows.hpp"
 #include "sat_math.hpp"
 #include "depthwise_f32.hpp"
 
@@ -1423,6 +1424,63 @@ static FilterPlan plan_filter(const ConvF32& q)
     pl.splits = ceil_div_i(g.K, g.kchunk);
     return pl;
 }
+// ---- backward-filter of 3x3 kernels on the bf16 matrix cores
+struct RowsPlan {
+    int nol;                   // log2 of a step's octets of a row; -1: not this kernel
+    int qtiles, ctiles, splits;
+    FilterRows g;
+    size_t values() const { return (size_t)qtiles * ctiles * ROWS_TILE; }
+};
+static RowsPlan plan_rows(const ConvF32& q)
+{
+    RowsPlan pl = {};
+    pl.nol = -1;
+    if (q.kH != 3 || q.kW != 3 || q.sx != q.sy || q.sx > 2 || q.pl != 1 || q.pt > 2 || q.ranges) return pl;
+    FilterRows& g = pl.g;
+    g.B = q.B; g.C = q.C; g.Q = q.O; g.H = q.H; g.W = q.W; g.oH = q.oH; g.oW = q.oW; g.pt = q.pt;
+    // an image's rows of x, the padding above the next one's, and all that the last output row reads
+    g.D = std::max(ceil_div_i(q.H + q.pt, q.sy), ceil_div_i((q.oH - 1) * q.sy - q.pt + 3, q.sy));
+    const int octets = ceil_div_i(q.oW, 8);
+    pl.qtiles = ceil_div_i(q.O, ROWS_Q); pl.ctiles = ceil_div_i(q.C, ROWS_C);
+    // Where the layer is large and fills the tiles and octets (us, fp32 kernel / this one): 64 <- 64, 28 x 28, batch 8, 4.6e8 flops 17 / 22;
+    // 128 <- 128, 56 x 56, 9.2e8 25 / 26; 64 <- 32, 112 x 112, batch 4, 1.8e9 34 / 28; 71 <- 37 channels, 113 x 75, batch 5, 0.3 filled
+    // 52 / 54; 100 <- 48, 56 x 56, batch 16, 0.59 filled 69 / 61.
+    const double flops = 2.0 * q.B * q.O * q.oH * q.oW * q.C * 9;
+    if (flops < 1.5e9 || (double)q.O * q.C * q.oW < 0.4 * pl.qtiles * ROWS_Q * (double)pl.ctiles * ROWS_C * octets * 8) return pl;
+    // a step has 8 octets (4 at stride 2): as many of a row as leave the fewest beyond its end; rows that follow each other share theirs of x
+    int best = 1 << 30;
+    for (int nol = q.sx == 1 ? 3 : 2; nol >= 0; --nol)
+        if (round_up(octets, 1 << nol) < best) {
+            best = round_up(octets, 1 << nol);
+            pl.nol = nol;
+        }
+    const int rows = (q.sx == 1 ? 8 : 4) >> pl.nol;
+    g.pieces = best >> pl.nol;
+    g.chunks = ceil_div_i((long)q.B * g.D, rows) * g.pieces;
+    pl.splits = (int)std::min<long>(std::max(256L / ((long)pl.qtiles * pl.ctiles), 1L), ceil_div_i(g.chunks, 4));
+    g.per = ceil_div_i(g.chunks, pl.splits);
+    pl.splits = ceil_div_i(g.chunks, g.per);
+    g.masked = q.oW % 8 != 0 || q.W % (8 * q.sx) != 0;
+    g.bytesX = (unsigned)(4 * (size_t)q.B * q.C * q.H * q.W); g.bytesY = (unsigned)(4 * (size_t)q.B * q.O * q.oH * q.oW);
+    g.dD = div_of(g.D); g.dSD = div_of(q.sx * g.D); g.dpieces = div_of(g.pieces);
+    return pl;
+}
+static void launch_rows(const RowsPlan& pl, int s, const float* x, const float* dy, float beta, float* dw, float* ws, hipStream_t st)
+{
+    const dim3 grid(pl.ctiles, pl.qtiles, pl.splits);
+    const auto run = [&](auto s_, auto nol_) {
+        hipLaunchKernelGGL((conv_f32_filter_rows_kernel<decltype(s_)::value, decltype(nol_)::value>), grid, dim3(512), 0, st, pl.g, x, dy, ws);
+    };
+    const auto octets = [&](auto s_) {
+        if (pl.nol == 0) run(s_, std::integral_constant<int, 0>{});
+        else if (pl.nol == 1) run(s_, std::integral_constant<int, 1>{});
+        else if (pl.nol == 2) run(s_, std::integral_constant<int, 2>{});
+        else if constexpr (decltype(s_)::value == 1) run(s_, std::integral_constant<int, 3>{});
+    };
+    s == 1 ? octets(std::integral_constant<int, 1>{}) : octets(std::integral_constant<int, 2>{});
+    hipLaunchKernelGGL(conv_f32_reduce_rows_kernel, dim3((unsigned)(pl.values() / 64)), dim3(256), 0, st, (const float*)ws, pl.splits, pl.ctiles, pl.values(), pl.g.Q,
+                       pl.g.C, beta, dw);
+}
 // What the small filter kernel runs of a pass: backward-filter, or backward-data of a spanning kernel as a sum over "pixels" o,
 // dx[b][k] = sum_o dy[b][o] w[o][k], with the images as rows of q and the weights of an output as columns of p.
 static FilterGemm small_gemm(const ConvF32& q, int pass)
@@ -1497,6 +1555,8 @@ static size_t laid_weights(const ConvF32& q, int pass, int kind)
 static size_t pass_workspace(const ConvF32& q, int pass)
 {
     if (pass == PASS_BWD_FILTER) {
+        const RowsPlan rows = plan_rows(q);
+        if (rows.nol >= 0) return rows.splits * rows.values();
         const FilterPlan pl = plan_filter(q);
         return (size_t)pl.splits * pl.g.Q * pl.g.P;
     }
@@ -1515,6 +1575,12 @@ static int run_pass(const ConvF32& q, int pass, const float* a, const float* b, 
                     float* out, float* ws, size_t ws_floats, hipStream_t st)
 {
     if (pass == PASS_BWD_FILTER) {
+        const RowsPlan rows = plan_rows(q);
+        if (rows.nol >= 0 && rows.splits * rows.values() <= ws_floats) {
+            launch_rows(rows, q.sx, a, b, beta, out, ws, st);
+            N2D2HIP_HIP_CHECK(hipGetLastError());
+            return N2D2HIP_OK;
+        }
         FilterPlan pl = plan_filter(q);
         const size_t n = (size_t)pl.g.Q * pl.g.P;
         bool direct = false;

@@ -1,4 +1,4 @@
-"""Float convolutions on the bf16 matrix cores, operands in three parts: forward and data gradient against float64 at the edges of the
+"""Float convolutions on the bf16 matrix cores, operands in three parts: forward, data and filter gradient against float64 at the edges of the
 tiles, runs and channel chunks, and infinities, NaN and floats near the largest where a float sum has them."""
 import ctypes as C
 
@@ -92,3 +92,75 @@ def test_infinities_nan_and_the_largest_floats(case):
         assert np.array_equal(np.isnan(g), np.isnan(t)) and np.array_equal(g == np.inf, t == np.inf) and np.array_equal(g == -np.inf, t == -np.inf)
         ok = np.isfinite(t)
         assert (np.abs(g - f)[ok] <= 2.0 ** -24 * (np.abs(f) + (n + 4) * m)[ok]).all()
+
+
+# B, C, H, W, O, stride, pad y: rows of one octet, of two, three (a step of one each, of two with one left over), four and eight, ends inside an
+# octet, tiles left over in both directions, no padding and two rows above, images whose last row no output reads
+FILTER = [(260, 64, 7, 7, 128, 1, 1), (70, 64, 13, 15, 100, 1, 1), (44, 70, 19, 24, 64, 1, 1), (33, 64, 31, 30, 64, 1, 1), (11, 32, 40, 57, 120, 1, 0), (6, 64, 64, 64, 64, 1, 2),
+          (290, 96, 14, 14, 64, 2, 1), (33, 128, 27, 27, 120, 2, 1), (21, 64, 41, 50, 128, 2, 0), (22, 64, 57, 64, 64, 2, 2), (300, 64, 9, 16, 128, 2, 1)]
+
+
+def _filter(x, w_shape, dy, s, pt, beta=0.0, start=0.0):
+    import torch
+    from n2d2_amd import capi, runtime as rt
+    B, Ci, H, W = x.shape
+    d = capi.ConvDesc(Ci, w_shape[0], 3, 3, s, s, 1, pt, 1, pt, 1, 1, 1, 0, 0)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    x_, dy_, dw = dev(x), dev(dy), torch.full(w_shape, start, device="cuda")
+    n = int(capi.lib.n2d2hip_conv2d_f32_workspace_bytes(C.byref(d), B, H, W))
+    ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+    capi.check(capi.lib.n2d2hip_conv2d_f32_backward_filter(C.byref(d), B, H, W, x_.data_ptr(), dy_.data_ptr(), beta, dw.data_ptr(), ws.data_ptr(), n, rt.stream_ptr()))
+    torch.cuda.synchronize()
+    return dw.cpu().numpy()
+
+
+def _filter64(x, dy, s, pt):
+    B, Ci, H, W = x.shape
+    xp = np.zeros((B, Ci, dy.shape[2] * s + 2, dy.shape[3] * s + 2))
+    h, w = min(H, xp.shape[2] - pt), min(W, xp.shape[3] - 1)
+    xp[:, :, pt:pt + h, 1:1 + w] = x[:, :, :h, :w]
+    dw = np.empty((dy.shape[1], Ci, 3, 3))
+    d = dy.astype(np.float64).transpose(1, 0, 2, 3).reshape(dy.shape[1], -1)
+    for i in range(3):
+        for j in range(3):
+            dw[:, :, i, j] = d @ xp[:, :, i:i + s * dy.shape[2]:s, j:j + s * dy.shape[3]:s].transpose(1, 0, 2, 3).reshape(Ci, -1).T
+    return dw
+
+
+@pytest.mark.parametrize("case", FILTER)
+def test_filter_gradient_against_float64(case):
+    B, Ci, H, W, O, s, pt = case
+    print("parts, filter gradient", case, flush=True)
+    rng = np.random.default_rng(sum(case))
+    oH, oW = (H + 2 * pt - 3) // s + 1, (W - 1) // s + 1
+    assert 2.0 * B * O * oH * oW * Ci * 9 >= 1.5e9
+    x, dy = rng.normal(size=(B, Ci, H, W)).astype(np.float32), rng.normal(size=(B, O, oH, oW)).astype(np.float32)
+    want, mag = _filter64(x, dy, s, pt), _filter64(np.abs(x), np.abs(dy), s, pt)
+    got = _filter(x, (O, Ci, 3, 3), dy, s, pt)
+    # (ranges, of which each is a sum in float, are added in double; one range is at most all pixels: 5 roundings in 32)
+    K = B * oH * oW
+    assert (np.abs(got - want) <= 2.0 ** -24 * (np.abs(want) + (5 * K / 32 + 4) * mag)).all()
+    assert np.linalg.norm(got - want) <= 1.1 * 2.53e-8 * np.sqrt(1 + 5 * K / 64) * np.linalg.norm(want)
+    again = _filter(x, (O, Ci, 3, 3), dy, s, pt, beta=0.5, start=2.0)
+    assert np.abs(again - (got + np.float32(1.0))).max() <= 2.0 ** -23 * (np.abs(got).max() + 2)
+
+
+def test_filter_gradient_infinities_nan_and_the_largest_floats():
+    B, Ci, H, W, O, s, pt = 33, 128, 27, 27, 120, 2, 1
+    print("parts, filter gradient, special values", flush=True)
+    rng = np.random.default_rng(5)
+    x, dy = rng.normal(size=(B, Ci, H, W)).astype(np.float32), (1e-3 * rng.normal(size=(B, O, 14, 14))).astype(np.float32)
+    dy[np.abs(dy) < 1e-5] = 1e-5
+    dy[2, 7] = 0.0
+    for c, v in enumerate([np.inf, -np.inf, np.nan, 3.4e38, -3.4e38, 1e-42]):
+        x[rng.integers(B), 3 * c + 1, rng.integers(H), rng.integers(W)] = v
+    x[2, 50, 5, 6] = np.inf
+    with np.errstate(invalid="ignore"):
+        want = _filter64(x, dy, s, pt)
+    got = _filter(x, (O, Ci, 3, 3), dy, s, pt)
+    # (a padded position is no product here, in the reference a zero: only NaN of `want` against infinities outside the windows would differ)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got == np.inf, want == np.inf) and np.array_equal(got == -np.inf, want == -np.inf)
+    ok = np.isfinite(want)
+    fin = np.where(np.isfinite(x), x, 0)
+    mag = _filter64(np.abs(fin), np.abs(dy), s, pt)
+    assert (np.abs(got - _filter64(fin, dy, s, pt))[ok] <= 2.0 ** -24 * ((5 * B * 196 / 32 + 4) * mag)[ok]).all()
