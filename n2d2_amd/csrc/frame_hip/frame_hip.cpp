@@ -3,6 +3,9 @@
 
 #include <hip/hip_runtime_api.h>
 #include <omp.h>
+#if defined(__x86_64__)
+#include <immintrin.h>
+#endif
 
 #include <algorithm>
 #include <functional>
@@ -1891,7 +1894,7 @@ void DeepNet::setStimuliData(const Tensor<Float_T>& data)
     setStimuliData(data.data(), data.dimX(), data.dimY(), data.dimZ(), data.dimB());
 }
 
-// Integer-valued floats in [lo, hi] -> bytes; false if a value is not one.  One pass at the rate of memory.
+// Integer-valued floats in [lo, hi] -> bytes; false if a value is not one.
 static bool narrowToBytes(const Float_T* x, unsigned char* out, size_t n, int lo, int hi)
 {
     int bad = 0;
@@ -1903,11 +1906,39 @@ static bool narrowToBytes(const Float_T* x, unsigned char* out, size_t n, int lo
     }
     return bad == 0;
 }
+#if defined(__x86_64__)
+// 32 values at a time, twice as fast as with 16-byte vectors.  (What is no integer of 32 bits is converted to the smallest one, which
+// is out of every range here.)
+__attribute__((target("avx2"))) static bool narrowToBytesAvx2(const Float_T* x, unsigned char* out, size_t n, int lo, int hi)
+{
+    __m256 bad = _mm256_setzero_ps();
+    __m256i least = _mm256_set1_epi32(lo), most = _mm256_set1_epi32(hi);
+    // (the packs interleave the halves of their operands: dwords 0, 4, 1, 5, ... are the order of the values)
+    const __m256i order = _mm256_setr_epi32(0, 4, 1, 5, 2, 6, 3, 7), low = _mm256_set1_epi32(255);
+    size_t i = 0;
+    for (; i + 32 <= n; i += 32) {
+        __m256i v[4];
+        for (int k = 0; k < 4; ++k) {
+            const __m256 f = _mm256_loadu_ps(x + i + 8 * k);
+            v[k] = _mm256_cvttps_epi32(f);
+            bad = _mm256_or_ps(bad, _mm256_cmp_ps(_mm256_cvtepi32_ps(v[k]), f, _CMP_NEQ_UQ));
+            least = _mm256_min_epi32(least, v[k]);
+            most = _mm256_max_epi32(most, v[k]);
+            v[k] = _mm256_and_si256(v[k], low);
+        }
+        const __m256i bytes = _mm256_packus_epi16(_mm256_packus_epi32(v[0], v[1]), _mm256_packus_epi32(v[2], v[3]));
+        _mm256_storeu_si256((__m256i*)(out + i), _mm256_permutevar8x32_epi32(bytes, order));
+    }
+    const __m256i outside = _mm256_or_si256(_mm256_cmpgt_epi32(_mm256_set1_epi32(lo), least), _mm256_cmpgt_epi32(most, _mm256_set1_epi32(hi)));
+    return _mm256_movemask_ps(_mm256_or_ps(bad, _mm256_castsi256_ps(outside))) == 0 && narrowToBytes(x + i, out + i, n - i, lo, hi);
+}
+#endif
 
 // The stimuli arrive as floats in ordinary host memory.  A few threads check and narrow them to bytes in pinned memory, so
 // that a quarter of the bytes cross to the device, and the conversion to the first cell's layout reads those.  Bound by
-// reading the floats and by the copy.  16 x 3 x 224 x 224 values: 12.4 ms -> 0.135 ms (before: one thread testing value by
-// value, three copies of the floats on the host, a device buffer allocated and freed on each call).
+// reading the floats and by the copy (2.4 MB: 50 us).  16 x 3 x 224 x 224 values: 12.4 ms -> 0.128 ms (before: one thread testing value by
+// value, three copies of the floats on the host, a device buffer allocated and freed on each call) -> 0.090 ms (16-byte vectors and 8
+// threads before; half the values copied while the other half is narrowed: the same 0.090).
 void DeepNet::setStimuliData(const Float_T* data, size_t dimX, size_t dimY, size_t dimZ, size_t dimB)
 {
     // network input unsigned <=> DeepNetExport::mEnvDataUnsigned (StimuliProviderExport::unsignedStimuli)
@@ -1932,10 +1963,15 @@ void DeepNet::setStimuliData(const Float_T* data, size_t dimX, size_t dimY, size
     // (slices of 64 K values, about 15 us of one thread's work: less is not worth waking a second one)
     const size_t slice = (size_t)1 << 16;
     const long slices = (long)((nbValues + slice - 1) / slice);
+    const int threads = (int)std::min<long>(slices, std::min(omp_get_max_threads(), 16));
+    auto narrow = narrowToBytes;
+#if defined(__x86_64__)
+    if (__builtin_cpu_supports("avx2")) narrow = narrowToBytesAvx2;
+#endif
     bool good = true;
-#pragma omp parallel for schedule(static) reduction(&& : good) num_threads((int)std::min<long>(slices, std::min(omp_get_max_threads(), 8))) if (slices > 1)
+#pragma omp parallel for schedule(static) reduction(&& : good) num_threads(threads) if (threads > 1)
     for (long k = 0; k < slices; ++k)
-        good = narrowToBytes(data + k * slice, mStimuliBytes + k * slice, std::min(slice, nbValues - k * slice), lo, hi) && good;
+        good = narrow(data + k * slice, mStimuliBytes + k * slice, std::min(slice, nbValues - k * slice), lo, hi) && good;
     if (!good)          // (the device keeps the stimuli it has)
         for (size_t i = 0; i < nbValues; ++i)
             toInteger(data[i], lo, hi, "stimuli");

@@ -90,6 +90,21 @@ def test_stimuli_are_checked_and_narrowed_in_slices(fh, batch):
     assert np.array_equal(net.outputs("fc3"), before)
 
 
+def test_stimuli_of_any_count_are_narrowed(fh):
+    """Groups of 32 values and what is left over: every byte, and what is none in each place of a group and behind the last."""
+    from n2d2_amd import nets
+    b = nets._Builder("ragged", (3, 9, 7), seed=4, scaling_mode="DoubleShift")
+    b.fc("fc", b.conv("c", "input", 8, 3), 10, mode="None")
+    x = np.arange(5 * 189).reshape(5, 3, 9, 7) * 7 % 256         # 29 groups and 17 values
+    net = _compare(fh, b.spec, x, ["c", "fc"])
+    for at in list(range(32, 64)) + [0, 927, 928, 944]:
+        for bad in (-1.0, 256.0, 7.5, float("nan"), -3e9):
+            y = x.astype(np.float32)
+            y.reshape(-1)[at] = bad
+            with pytest.raises(fh.FrameHipError):
+                net.set_stimuli(y)
+
+
 def test_resnet50_through_the_registrar(fh):
     from n2d2_amd import nets
     spec = nets.resnet50()
