@@ -105,6 +105,7 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
     const int nchunks = (g.Ch + PK - 1) / PK, plane4 = g.planeS * 4, tstep = g.qpad / 16 * PATCH_FRAG;
     const unsigned zaddr = lo * OCT + 64 * PB * 16;
     const __amdgpu_buffer_rsrc_t rsrcX = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(srcX), 0, g.bytesX, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrcW = __builtin_amdgcn_make_buffer_rsrc(const_cast<v4u*>(wt), 0, nchunks * g.T * tstep, 0x00020000);
     if (threadIdx.x < 12) *(v4u*)(smem + threadIdx.x * OCT + 64 * PB * 16) = v4u{0, 0, 0, 0};
 
     const PixelClass& c = g.c[0];                // (forward, or backward-data at stride 1)
@@ -164,18 +165,17 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
     // a wave's weights: consecutive taps of a chunk are a fragment of every 16 rows of q apart
     v4u a[3][MQ][3], b[2][3];
     auto weights = [&](v4u (&w)[MQ][3], int qtile, int chunk, int t) {
-        const char* at = (const char*)wt + (size_t)(qtile * (QT / 16) + wq * MQ) * PATCH_FRAG + lane * 16
-                         + (size_t)(chunk * nT + t) * tstep;
+        const int at = (qtile * (QT / 16) + wq * MQ) * PATCH_FRAG + (chunk * nT + t) * tstep;
 #pragma unroll
         for (int m = 0; m < MQ; ++m)
 #pragma unroll
-            for (int p = 0; p < 3; ++p) w[m][p] = *(const v4u*)(at + m * PATCH_FRAG + p * 1024);
+            for (int p = 0; p < 3; ++p) w[m][p] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(rsrcW, lane * 16, at + m * PATCH_FRAG + p * 1024, 0));
     };
     auto first_weights = [&](int qtile) {
         weights(a[0], qtile, cbeg, 0);
         if (NT == 9) weights(a[1], qtile, cbeg, 1);
     };
-    unsigned xaddr[NP], mask[NP], obase[NP];     // of a lane's pixels: where tap (0, 0) is in LDS; the taps that exist; in `out`
+    unsigned xaddr[NP], mask[NP];                // of a lane's pixels: where tap (0, 0) is in LDS; the taps that exist
 
     // (before its first tile a block runs through one step that only loads: its code is that of the others)
     PatchItem it, to;
@@ -191,22 +191,20 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
         if (live) {
             // a lane works out one of the wave's pixels, and hands it to those that take it
             const int run0 = source(p0) - back;
-            const int p = p0 + wp * NP * 16 + lane, pp = min(p, c.P - 1);
-            const int img = div_f32(pp, c.ghw), rem = pp - img * c.gHW, py = div_f32(rem, c.gw), px = rem - py * c.gW;
-            const int y = py * g.sy + c.y0, x = px * g.sx + c.x0;
             // taps first .. end - 1 of an axis lie inside it
             auto inside = [&](int at, int size, int n) {
                 const int first = min(max(g.d > 0 ? -at : at - size + 1, 0), n), end = min(max(g.d > 0 ? size - at : at + 1, 0), n);
                 return ((1u << end) - 1u) & ~((1u << first) - 1u);
             };
+            const int p = p0 + wp * NP * 16 + lane, pp = min(p, c.P - 1);
+            const int img = div_f32(pp, c.ghw), rem = pp - img * c.gHW, py = div_f32(rem, c.gw), px = rem - py * c.gW;
+            const int y = py * g.sy + c.y0, x = px * g.sx + c.x0;
             const unsigned m = p < c.P ? inside(x, g.Ws, nx) | (inside(y, g.Hs, ny) << nx) : 0u;
             const unsigned at = 16 * (img * g.planeS + y * g.Ws + x - run0);
-            const unsigned o = p < c.P ? 4u * (unsigned)(img * g.Q * g.planeO + rem) : F32_OOB;
 #pragma unroll
             for (int n = 0; n < NP; ++n) {
                 mask[n] = __shfl((int)m, n * 16 + l16);
                 xaddr[n] = lo * OCT + __shfl((int)at, n * 16 + l16);
-                obase[n] = __shfl((int)o, n * 16 + l16);
             }
         }
         each([&](int m, int n, int r) {
@@ -307,6 +305,11 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
         // A lane holds pixel .. + lane % 16 and rows qn + 16 m + r.
         if (live) {
             const size_t zoff = (size_t)blockIdx.z * partial;
+            unsigned obase[NP];                  // of the pixels, in `out`
+            const int p = p0 + wp * NP * 16 + lane, pp = min(p, c.P - 1), img = div_f32(pp, c.ghw);
+            const unsigned o = p < c.P ? 4u * (unsigned)(img * (g.Q - 1) * g.planeO + pp) : F32_OOB;
+#pragma unroll
+            for (int n = 0; n < NP; ++n) obase[n] = __shfl((int)o, n * 16 + l16);
             const __amdgpu_buffer_rsrc_t rsrcO = __builtin_amdgcn_make_buffer_rsrc(out + zoff, 0, g.bytesO, 0x00020000);
             const int planeO4 = 4 * g.planeO;
             const unsigned qrow = qn * planeO4;

@@ -1342,8 +1342,7 @@ static void launch_patch(const PixelPlan& pl, dim3 grid, const float* x, const f
                            st, pl.g, x, w, (const v4u*)wt, bias, beta, out, partial);
     };
     const auto taps = [&](auto nu_, auto fold_) {
-        pl.g.c[0].nT == 9 && pl.g.c[0].nx == 3 ? run(nu_, std::integral_constant<int, 9>{}, fold_)
-                                                                   : run(nu_, std::integral_constant<int, 0>{}, fold_);
+        pl.g.c[0].nT == 9 && pl.g.c[0].nx == 3 ? run(nu_, std::integral_constant<int, 9>{}, fold_) : run(nu_, std::integral_constant<int, 0>{}, fold_);
     };
     const auto units = [&](auto fold_) {
         pl.patch.nu <= 2 ? taps(std::integral_constant<int, 2>{}, fold_) : taps(std::integral_constant<int, 3>{}, fold_);
