@@ -524,7 +524,7 @@ int n2d2hip_lsq_backward(const float* diff_q, const float* fp_x, float* diff_fp,
  * (target - output at the loss), so the solver adds rate * diff.
  *
  * Ungrouped convolutions without dilation, of up to 64 taps or spanning their input, run on the matrix cores: forward from
- * 2e7 flops (spanning: up to 64 taps), backward-data, and backward-filter (in double below 2e7 flops and for spanning
+ * 2e7 flops (spanning: up to 64 taps), backward-data (in double where small), and backward-filter (in double below 2e7 flops and for spanning
  * kernels of more than 64 taps).  There sums are added in an order that follows from the sizes, not in the reference's; forward
  * and backward-data of several taps multiply on the bf16 matrix cores, each float as three bf16 numbers that add up to it, where
  * that is faster (infinities and NaN come out as in float).

@@ -1132,6 +1132,80 @@ __global__ __launch_bounds__(256) void conv_f32_filter_small_kernel(FilterGemm g
     else out[idx] = (float)v + (beta != 0.0f ? beta * out[idx] : 0.0f);
 }
 
+// Backward-data of small problems, the same way: dx[c][pixel] adds w[o][c][tap] dy[o][the pixel that the tap reaches] over (o, tap)
+// in double.  A block is 16 channels x 16 input pixels; its waves take 16 terms in turn.  Bound by the latency of its loads, a
+// microsecond for each wave's two rounds of them: 8 waves where K is more than four waves take in two.  Which pixel a tap reaches
+// is worked out once for the block (for every term: 12.1 us where this takes 8.6).
+// us, the pixel kernel with its ranges / this with 4 / 8 waves (error against 64 bits 1.4e-7, 2.5e-8):
+//   6 <- 16, 5x5, 14 x 14, batch 32, K 400   14.5 /  8.6 /  7.8      16 <- 16, 3x3, 28 x 28, batch 8, K 144    12.3 /  5.3 /  5.6
+//   8 <- 16, 3x3, 32 x 32, batch 16, K 144   12.4 /  6.5 /  7.7      64 <- 64, 3x3, 28 x 28, K 576             11.8 /  8.6 /  6.7
+//   64 <- 64, 3x3 stride 2, 14 x 14, batch 4 10.5 /  8.5 /  6.7      256 <- 256, 3x3, 7 x 7, K 2304            20.1 / 24.0 / 16.5
+//   8 <- 512, 3x3, 7 x 7, K 4608             15.5 / 43.9 / 29.1      8 <- 8, 3x3, 32 x 32, batch 64, K 72      12.2 / 13.7 / 18.8
+struct DataSmall {
+    int P, C, O, T, K;                           // input pixels over all images; taps; O * T
+    int kW, HW, W, oH, oW, sy, sx, pt, pl;
+    DivF32 dHW, dW, dT, dkW, dsy, dsx;
+};
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void conv_f32_data_small_kernel(DataSmall g, const float* __restrict__ w, const float* __restrict__ dy, float beta,
+                                                                  float* __restrict__ dx)
+{
+    __shared__ double red[WAVES][256];
+    __shared__ int reach[64 * 16];               // where in a channel's image a pixel's tap is; -1: outside
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane & 15, kg = lane >> 4;
+    const int c = blockIdx.y * 16 + row, plane = g.oH * g.oW;
+    {
+        const int p = min((int)(blockIdx.x * 16 + (threadIdx.x & 15)), g.P - 1), rem = p - div_f32(p, g.dHW) * g.HW, iy = div_f32(rem, g.dW), ix = rem - iy * g.W;
+        for (int t = threadIdx.x >> 4; t < g.T; t += 4 * WAVES) {
+            const int ty = div_f32(t, g.dkW), y = iy + g.pt - ty, x = ix + g.pl - (t - ty * g.kW);
+            const int oy = div_f32(max(y, 0), g.dsy), ox = div_f32(max(x, 0), g.dsx);
+            reach[t * 16 + (threadIdx.x & 15)] = y >= 0 && x >= 0 && oy * g.sy == y && ox * g.sx == x && oy < g.oH && ox < g.oW ? oy * g.oW + ox : -1;
+        }
+    }
+    __syncthreads();
+    const float* wb = w + (size_t)min(c, g.C - 1) * g.T;
+    const float* yb = dy + (size_t)div_f32(min((int)(blockIdx.x * 16 + row), g.P - 1), g.dHW) * g.O * plane;
+    float a[2][4], b[2][4];
+    const int adv_o = div_f32(16 * WAVES, g.dT), adv_t = 16 * WAVES - adv_o * g.T;
+    int ko = div_f32(wave * 16 + kg * 4, g.dT), kt = wave * 16 + kg * 4 - ko * g.T;     // this lane's next term
+    auto load = [&](float (&av)[4], float (&bv)[4]) {
+        int o = ko, t = kt;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int at = o < g.O ? reach[t * 16 + row] : -1;
+            av[j] = o < g.O ? wb[(size_t)o * g.C * g.T + t] : 0.0f;
+            bv[j] = at >= 0 ? yb[(size_t)o * plane + at] : 0.0f;
+            if (++t == g.T) { t = 0; ++o; }
+        }
+        ko += adv_o;
+        kt += adv_t;
+        if (kt >= g.T) { kt -= g.T; ++ko; }
+    };
+    v4d acc = {0.0, 0.0, 0.0, 0.0};
+    load(a[0], b[0]);
+    for (int s = wave * 16; s < g.K; s += 32 * WAVES) {
+        load(a[1], b[1]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[0][j], (double)b[0][j], acc, 0, 0, 0);
+        load(a[0], b[0]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[1][j], (double)b[1][j], acc, 0, 0, 0);
+    }
+    // lane holds column p = lane % 16 and rows c = 4 r + lane / 16
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wave][(4 * r + kg) * 16 + row] = acc[r];
+    __syncthreads();
+    if (threadIdx.x >= 256) return;
+    const int oc = blockIdx.y * 16 + threadIdx.x / 16, op = blockIdx.x * 16 + threadIdx.x % 16;
+    if (oc >= g.C || op >= g.P) return;
+    double v = red[0][threadIdx.x];
+#pragma unroll
+    for (int i = 1; i < WAVES; ++i) v += red[i][threadIdx.x];
+    const int oi = div_f32(op, g.dHW);
+    const size_t idx = ((size_t)oi * g.C + oc) * g.HW + (op - oi * g.HW);
+    dx[idx] = (float)v + (beta != 0.0f ? beta * dx[idx] : 0.0f);
+}
+
 // out[i] = sum over the K ranges + beta * out[i] (+ bias of element i's channel, NCHW with `plane` pixels per channel and O
 // channels).  A block adds 64 elements: each of its four waves a quarter of the ranges in double, in their order, then the
 // four in order, so the result does not depend on timing.

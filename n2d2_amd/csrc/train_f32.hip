@@ -938,7 +938,7 @@ static bool spans_input(const ConvF32& q)
 }
 
 enum { PASS_FWD = 0, PASS_BWD_DATA = 1, PASS_BWD_FILTER = 2 };
-enum { F32_PATH_DIRECT, F32_PATH_GEMM, F32_PATH_SMALL };
+enum { F32_PATH_DIRECT, F32_PATH_GEMM, F32_PATH_SMALL, F32_PATH_SMALL_DATA };
 
 // More than the pixel kernels have lanes and the filter kernel has mask bits for
 static bool many_taps(const ConvF32& q) { return (long)q.kH * q.kW > 64; }
@@ -949,7 +949,7 @@ constexpr long GRID_Y = 65535;
 // The kernels of a pass.  The matrix cores serve ungrouped convolutions without dilation; the direct kernels keep the rest
 // (depthwise, dilated) and the forward sums below 2e7 flops or of kernels over 64 taps, which stay in the reference's order
 // of terms (quantizers turn the last bit of a sum into a level now and then).  Backward-filter below 2e7 flops, and of a
-// spanning kernel over 64 taps, adds in double (F32_PATH_SMALL).  The descriptor's kernel_choice (N2D2HIP_KERNEL_F32_DIRECT /
+// spanning kernel over 64 taps, and small data gradients add in double (F32_PATH_SMALL, _SMALL_DATA).  The descriptor's kernel_choice (N2D2HIP_KERNEL_F32_DIRECT /
 // _GEMM) overrides the size rules.
 static int f32_path(const ConvF32& q, int pass)
 {
@@ -975,6 +975,17 @@ static int f32_path(const ConvF32& q, int pass)
     if (pass == PASS_BWD_DATA && (forced || !small) && flops < 5.0e8 && !many_taps(q) && q.kH * q.kW > 1 && q.B <= 16 * GRID_Y && spans_input(q))
         return F32_PATH_SMALL;
     if (forced) return F32_PATH_GEMM;
+    // Small data gradients add in double.  Spanning layers below 2e7 flops (us, product in float / this): 16 x 5 x 5 <- 120, batch 32 8.4 / 4.2;
+    // 120 <- 84, batch 32 8.5 / 4.2; 512 x 1 x 1 <- 64, batch 2 7.7 / 3.9; 64 <- 10, batch 96 5.5 / 4.0.  Others by the rounds of loads
+    // of all blocks and of one (conv_f32_data_small_kernel has the times).
+    if (pass == PASS_BWD_DATA && !many_taps(q)) {
+        if (spans_input(q)) {
+            if (small && q.B <= 16 * GRID_Y) return F32_PATH_SMALL;
+        } else {
+            const long K = (long)q.O * q.kH * q.kW;
+            if (K <= 2304 && (double)ceil_div_i((long)q.B * q.H * q.W, 16) * ceil_div_i(q.C, 16) * K <= 2.3e5) return F32_PATH_SMALL_DATA;
+        }
+    }
     if (pass == PASS_FWD) return small || many_taps(q) ? F32_PATH_DIRECT : F32_PATH_GEMM;
     if (small && pass == PASS_BWD_FILTER) return q.O <= 16 * GRID_Y ? F32_PATH_SMALL : F32_PATH_DIRECT;
     return F32_PATH_GEMM;
@@ -1678,6 +1689,16 @@ int n2d2hip_conv2d_f32_backward_data(const n2d2hip_conv_desc* desc, int B, int H
     const int path = f32_path(q, PASS_BWD_DATA);
     if (path == F32_PATH_SMALL)
         return run_small_filter(small_gemm(q, PASS_BWD_DATA), w, diff_y, beta, diff_x, (double*)workspace, workspace ? workspace_bytes : 0, (hipStream_t)stream);
+    if (path == F32_PATH_SMALL_DATA) {
+        const int T = q.kH * q.kW;
+        const DataSmall g = {q.B * q.H * q.W, q.C, q.O, T, q.O * T, q.kW, q.H * q.W, q.W, q.oH, q.oW, q.sy, q.sx, q.pt, q.pl,
+                             div_of(q.H * q.W), div_of(q.W), div_of(T), div_of(q.kW), div_of(q.sy), div_of(q.sx)};
+        const dim3 grid(ceil_div_i(g.P, 16), ceil_div_i(g.C, 16));
+        if (g.K <= 256) hipLaunchKernelGGL(conv_f32_data_small_kernel<4>, grid, dim3(256), 0, (hipStream_t)stream, g, w, diff_y, beta, diff_x);
+        else hipLaunchKernelGGL(conv_f32_data_small_kernel<8>, grid, dim3(512), 0, (hipStream_t)stream, g, w, diff_y, beta, diff_x);
+        N2D2HIP_HIP_CHECK(hipGetLastError());
+        return N2D2HIP_OK;
+    }
     if (path == F32_PATH_GEMM) {
         float* ws = (float*)workspace;
         const size_t nws = workspace ? workspace_bytes / sizeof(float) : 0;
