@@ -592,16 +592,22 @@ __global__ __launch_bounds__(256) void conv_f32_3x3_kernel(PixelGemm g, const fl
 }
 
 // A layer that spans its input, forward, in the reference's order of terms: y[b][o] = sum over k of x[b][k] w[o][k], one
-// after the other in float.  The chain of additions is what takes the time: a wave alone on its SIMD issues an instruction in
-// about 8 cycles, an addition no sooner than the one before it.  A block is 8 images x 8 outputs in both kernels, its 16 rows of
-// operands in LDS two stages of 256 terms ahead; which of the two is the faster depends on how many blocks there are:
-//  * Up to one a compute unit, conv_f32_chain_kernel: everything but the additions is kept off the wave that does them.  Two waves
-//    load the operands, multiply them, 64 terms of 128 each, and leave the products in LDS; the third reads those a step later and
-//    only adds, 5.5 ns a term.  (One wave with the products of the next 32 terms between its additions: 130 us where this takes 90.
-//    Steps of 64 terms: 95, and the same up to 1600 terms.)
-//  * More, conv_f32_chain_wave_kernel: one wave multiplies and adds, 7.1 ns a term, but its 49 KB let three blocks share a unit
+// after the other in float.  The chain of additions is what takes the time: a wave alone on its SIMD issues one in 6 to 8 cycles, and
+// every other instruction between two of them costs about as much.  Which kernel is the fastest depends on how many sums there are:
+//  * Up to two waves a SIMD (32 sums a compute unit), conv_f32_chain_kernel<4>: a wave holds four sums, one to a row of 16 lanes.  The lanes
+//    of a row multiply 64 terms, four each, straight from memory, and an addition takes its product out of the lane that has it by a broadcast
+//    within the row: 64 additions for 4 multiplications and 2 loads, 2.5 ns a term.  With LDS between (the next kernel) 16 reads of
+//    about 15 cycles each stood between 64 additions.
+//  * Up to one block of 8 images x 8 outputs a compute unit, conv_f32_chain_kernel<64>: a lane holds a sum, and everything but the additions
+//    is kept off the wave that does them.  Two waves load the operands, two stages of 256 terms ahead, multiply them, 64 terms of 128 each, and
+//    leave the products in LDS; the third reads those a step later and only adds, 5.5 ns a term.  (Steps of 64 terms: 95 us where
+//    this takes 90.)
+//  * More, conv_f32_chain_wave_kernel: one wave multiplies and adds 64 sums, 7.1 ns a term, but its 49 KB let three blocks share a unit
 //    where the other kernel's 115 KB let one.
-// us, conv_f32_chain_kernel / conv_f32_chain_wave_kernel (images x outputs, blocks, terms): 64 x 10, 16, 16384 88.8 / 116.3; 40 x 400,
+// us, conv_f32_chain_kernel<4> / <64> (images x outputs, terms): 64 x 10, 16384 41.7 / 88.9; 64 x 10, 1024 4.5 / 7.5; 32 x 120, 400 4.0 / 5.5;
+// 32 x 84, 120 4.0 / 4.0; 40 x 100, 25088 63.5 / 139; 64 x 64, 4096 13.0 / 23.7; 64 x 100 21.0 / 24.0; 64 x 128 21.0 / 23.8; 96 x 120
+// 29.0 / 24.0; 40 x 400, 25088 196 / 140.
+// us, conv_f32_chain_kernel<64> / conv_f32_chain_wave_kernel (images x outputs, blocks, terms): 40 x 400,
 // 250, 25088 140.5 / 178.1; 128 x 120, 240, 400 5.8 / 5.4; 144 x 120, 270, 400 9.7 / 5.8; 192 x 96, 288, 1024 13.7 / 10.4; 48 x 400, 300,
 // 25088 272.5 / 198.7; 256 x 120, 480, 400 9.9 / 5.9; 64 x 1000, 1000, 25088 552.5 / 381.1; 1024 x 120, 1920, 400 35.0 / 14.5.
 constexpr int CHAIN_K = 256, CHAIN_ROW = CHAIN_K + 4, CHAIN_STAGES = 3;      // (rows 16 bytes apart in the banks)
@@ -629,8 +635,78 @@ __device__ __forceinline__ void chain_store(int B, int O, int b, int o, float su
     y[idx] = r;
 }
 
-__global__ __launch_bounds__(192) void conv_f32_chain_kernel(int B, int O, int K, const float* __restrict__ x, const float* __restrict__ w,
-                                                             const float* __restrict__ bias, float beta, float* __restrict__ y)
+// The products of a row's 16 lanes, four each, one after the other: each addition takes a lane's for the whole row.  (In assembly:
+// the compiler puts a wait before each, as if the lanes' operand had just been written.)
+#define N2D2HIP_CHAIN_LANE(I)                                                                                                   \
+    "v_add_f32_dpp %0, %1, %0 row_newbcast:" #I " row_mask:0xf bank_mask:0xf\n\tv_add_f32_dpp %0, %2, %0 row_newbcast:" #I     \
+    " row_mask:0xf bank_mask:0xf\n\tv_add_f32_dpp %0, %3, %0 row_newbcast:" #I " row_mask:0xf bank_mask:0xf\n\t"              \
+    "v_add_f32_dpp %0, %4, %0 row_newbcast:" #I " row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ void chain_add_row(float& sum, const v4f& p)
+{
+    const float p0 = p[0], p1 = p[1], p2 = p[2], p3 = p[3];
+    asm volatile("s_nop 1\n\t" N2D2HIP_CHAIN_LANE(0) N2D2HIP_CHAIN_LANE(1) N2D2HIP_CHAIN_LANE(2) N2D2HIP_CHAIN_LANE(3) N2D2HIP_CHAIN_LANE(4)
+                 N2D2HIP_CHAIN_LANE(5) N2D2HIP_CHAIN_LANE(6) N2D2HIP_CHAIN_LANE(7) N2D2HIP_CHAIN_LANE(8) N2D2HIP_CHAIN_LANE(9)
+                 N2D2HIP_CHAIN_LANE(10) N2D2HIP_CHAIN_LANE(11) N2D2HIP_CHAIN_LANE(12) N2D2HIP_CHAIN_LANE(13) N2D2HIP_CHAIN_LANE(14)
+                 N2D2HIP_CHAIN_LANE(15)
+                 : "+v"(sum) : "v"(p0), "v"(p1), "v"(p2), "v"(p3));
+}
+// The first `lanes` lanes' products
+__device__ __forceinline__ void chain_add_lanes(float& sum, const v4f& p, int lanes)
+{
+    const float p0 = p[0], p1 = p[1], p2 = p[2], p3 = p[3];
+#define N2D2HIP_CHAIN_ONE(I) if (lanes > I) asm volatile("s_nop 1\n\t" N2D2HIP_CHAIN_LANE(I) : "+v"(sum) : "v"(p0), "v"(p1), "v"(p2), "v"(p3))
+    N2D2HIP_CHAIN_ONE(0); N2D2HIP_CHAIN_ONE(1); N2D2HIP_CHAIN_ONE(2); N2D2HIP_CHAIN_ONE(3); N2D2HIP_CHAIN_ONE(4);
+    N2D2HIP_CHAIN_ONE(5); N2D2HIP_CHAIN_ONE(6); N2D2HIP_CHAIN_ONE(7); N2D2HIP_CHAIN_ONE(8); N2D2HIP_CHAIN_ONE(9);
+    N2D2HIP_CHAIN_ONE(10); N2D2HIP_CHAIN_ONE(11); N2D2HIP_CHAIN_ONE(12); N2D2HIP_CHAIN_ONE(13); N2D2HIP_CHAIN_ONE(14);
+#undef N2D2HIP_CHAIN_ONE
+}
+#undef N2D2HIP_CHAIN_LANE
+// (SUMS: of a work-group; the two have nothing but the name in common)
+template <int SUMS>
+__global__ void conv_f32_chain_kernel(int B, int O, int K, const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float beta,
+                                      float* __restrict__ y);
+template <>
+__global__ __launch_bounds__(64) void conv_f32_chain_kernel<4>(int B, int O, int K, const float* __restrict__ x, const float* __restrict__ w,
+                                                               const float* __restrict__ bias, float beta, float* __restrict__ y)
+{
+    constexpr int D = 8;                         // groups of 64 terms requested ahead
+    const int lane = threadIdx.x, li = lane & 15, bi = lane >> 5, oi = lane >> 4 & 1, b0 = blockIdx.x * 2, o0 = blockIdx.y * 2;
+    const __amdgpu_buffer_rsrc_t rsrcX = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x + (size_t)b0 * K), 0, min(2, B - b0) * K * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrcW = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(w + (size_t)o0 * K), 0, min(2, O - o0) * K * 4, 0x00020000);
+    const int xoff = (bi * K + li * 4) * 4, woff = (oi * K + li * 4) * 4;
+    v4f xv[D], wv[D];
+    float sum = 0.0f;
+    // (terms past a row: of the next row, or zeros; rows past the last: zeros; not used)
+    const auto load = [&](v4f& xr, v4f& wr, int group) {
+        xr = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrcX, xoff, group * 256, 0));
+        wr = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrcW, woff, group * 256, 0));
+    };
+    const int full = K / 64, rest = K % 64 / 4;
+#pragma unroll
+    for (int u = 0; u < D; ++u) load(xv[u], wv[u], u);
+    int g = 0;
+    for (; g + D <= full; g += D) {
+#pragma unroll
+        for (int u = 0; u < D; ++u) {
+            tie(xv[u]); tie(wv[u]);
+            const v4f p = wv[u] * xv[u];
+            load(xv[u], wv[u], g + D + u);
+            __builtin_amdgcn_sched_barrier(0);
+            chain_add_row(sum, p);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+        if (g + u < full) chain_add_row(sum, wv[u] * xv[u]);
+        else if (g + u == full) chain_add_lanes(sum, wv[u] * xv[u], rest);
+    }
+    if (li == 0) chain_store(B, O, b0 + bi, o0 + oi, sum, bias, beta, y);
+}
+
+template <>
+__global__ __launch_bounds__(192) void conv_f32_chain_kernel<64>(int B, int O, int K, const float* __restrict__ x, const float* __restrict__ w,
+                                                                 const float* __restrict__ bias, float beta, float* __restrict__ y)
 {
     __shared__ __attribute__((aligned(16))) float smem[CHAIN_STAGES * 16 * CHAIN_ROW + 2 * 64 * CHAIN_PROD];
     float* const products = smem + CHAIN_STAGES * 16 * CHAIN_ROW;

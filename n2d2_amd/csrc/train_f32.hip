@@ -1101,9 +1101,12 @@ static int run_direct(const ConvF32& q, int pass, const float* x, const float* w
     if (!bwd && !q.depthwise && q.dx == 1 && q.dy == 1 && spans_input(q) && (q.kH != 3 || q.kW != 3) && K % 4 == 0 && K < (1 << 22) && q.O <= 8 * GRID_Y
         && (((size_t)x | (size_t)w) & 15) == 0) {
         const dim3 grid(ceil_div_i(q.B, 8), ceil_div_i(q.O, 8));
-        // (a unit holds one block of the kernel whose waves share the work, and three of the other; measured there)
-        if ((size_t)grid.x * grid.y <= (size_t)num_cus())
-            N2D2HIP_LAUNCH(conv_f32_chain_kernel, grid, dim3(192), 0, st, q.B, q.O, (int)K, x, w, bias, beta, out);
+        // (the first up to two of its waves a SIMD; a unit holds one block of the second, and three of the third; measured at the kernels)
+        const dim3 small(ceil_div_i(q.B, 2), ceil_div_i(q.O, 2));
+        if ((size_t)small.x * small.y <= 8 * (size_t)num_cus())
+            N2D2HIP_LAUNCH(conv_f32_chain_kernel<4>, small, dim3(64), 0, st, q.B, q.O, (int)K, x, w, bias, beta, out);
+        else if ((size_t)grid.x * grid.y <= (size_t)num_cus())
+            N2D2HIP_LAUNCH(conv_f32_chain_kernel<64>, grid, dim3(192), 0, st, q.B, q.O, (int)K, x, w, bias, beta, out);
         else
             N2D2HIP_LAUNCH(conv_f32_chain_wave_kernel, grid, dim3(64), 0, st, q.B, q.O, (int)K, x, w, bias, beta, out);
         N2D2HIP_HIP_CHECK(hipGetLastError());
