@@ -647,9 +647,25 @@ __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_apply_flat_kernel(size_t
     }
 }
 
-// The five sums of BatchNormCell_Frame<T>::backPropagate over one channel, and what follows from them, in blocks as above.
-// 128 channels, 56 x 56, batch 32: 40.7 us and the last step 7.0, now 20.6 and 4.9.
+// The sums of BatchNormCell_Frame<T>::backPropagate over one channel, and what follows from them, in blocks as above.  Its five are
+// multiples of three, d the values of dy and c those of x - mean: the sums of d c, of d and of c.  Those are what the blocks add up, in
+// double and the products unrounded; the factors (scale, 1 / sigma, -2) come in once a channel.  With a division and five conversions
+// a value the vector units took longer than the memory.  This pass and the next, us, before / now: 64 x 64 x 32 x 32 19.7 / 15.7,
+// behind a quantizer 27.7 / 23.5; 128 channels, 56 x 56, batch 32 45.6 / 42.2; 256, 14 x 14, batch 33 14.5 / 11.1; 32, 112 x 112, batch 8
+// 18.7 / 13.4; 6, 28 x 28, batch 32 9.7 / 7.5.  Errors against 64 bits are the same or smaller (dx 1.1e-7 / 0.7e-7).
+constexpr int BN_SUMS = 3;
 struct BnGrads { float* diff_scale; float* diff_bias; float* diff_saved_mean; float* diff_saved_variance; float beta_scale, beta_bias; };
+// (sigma is rounded to float, as the forward pass has it)
+__device__ __forceinline__ double bn_inv_sigma(float saved_variance, double epsilon) { return 1.0 / (double)(float)sqrt((double)saved_variance + epsilon); }
+// -> the reference's five: of d c / sigma, d, d scale, -2 c, d scale c
+__device__ __forceinline__ void bn_five_sums(double* t, const double* s, float scale, double inv_sigma)
+{
+    t[0] = s[0] * inv_sigma;
+    t[1] = s[1];
+    t[2] = (double)scale * s[1];
+    t[3] = -2.0 * s[2];
+    t[4] = (double)scale * s[0];
+}
 __device__ __forceinline__ void bn_stats_grads(double n, const double* t, float saved_variance, double epsilon, float* dmean, float* dvariance)
 {
     const float sum_mean1 = (float)t[2], sum_mean2 = (float)t[3], sum_var = (float)t[4];
@@ -688,7 +704,7 @@ __device__ __forceinline__ void bn_finish_alpha(const BnSatGrad& sat)
 __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_alpha_kernel(BnSatGrad sat) { bn_finish_alpha(sat); }
 
 // SAT: dy is first taken through the quantizer's gradient, in place (64 x 64 x 32 x 32, us: the quantizer's own pass 10.0, its end
-// 4.6 and the sums 9.8; together 19.2)
+// 4.6 and the sums, then 9.8; together then 19.2)
 template <int V, bool SAT>
 __global__ __launch_bounds__(1024) void batchnorm_f32_backward_sums_kernel(BnRange q, double n, const float* __restrict__ x,
                                                                            const float* __restrict__ scale, const float* __restrict__ saved_mean,
@@ -697,10 +713,10 @@ __global__ __launch_bounds__(1024) void batchnorm_f32_backward_sums_kernel(BnRan
 {
     constexpr int N = V ? V : 1;
     const int c = blockIdx.x;
-    const float m = saved_mean[c], g = scale[c];
-    const float var = (float)sqrt((double)saved_variance[c] + epsilon);
+    const float m = saved_mean[c], g = scale[c], variance = saved_variance[c];
+    const double inv_sigma = bn_inv_sigma(variance, epsilon);
     const float a = SAT ? fabsf(sat.alpha[0]) : 0.0f;
-    double t[SAT ? 6 : 5] = {};
+    double s[SAT ? BN_SUMS + 1 : BN_SUMS] = {};
     bn_walk<V>(q, c, [&](size_t idx) {
         float xv[N], dv[N];
         bn_load<N>(xv, x, idx);
@@ -710,54 +726,49 @@ __global__ __launch_bounds__(1024) void batchnorm_f32_backward_sums_kernel(BnRan
             bn_load<N>(fp, sat.fp, idx);
 #pragma unroll
             for (int k = 0; k < N; ++k) {
-                t[5] += (double)__fmul_rn(sat_alpha_slope(fp[k], sat.range, a), dv[k]);
+                s[BN_SUMS] += (double)__fmul_rn(sat_alpha_slope(fp[k], sat.range, a), dv[k]);
                 dv[k] = __fmul_rn(sat_input_slope(fp[k], a), dv[k]);
             }
             bn_store<N>(dy, idx, dv);
         }
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-            const float centred = xv[k] - m;
-            const float normalized = centred / var;
-            const float diff_normalized = dv[k] * g;
-            t[0] += (double)(dv[k] * normalized);
-            t[1] += (double)dv[k];
-            t[2] += (double)diff_normalized;
-            t[3] += (double)(-2.0f * centred);
-            t[4] += (double)(diff_normalized * centred);
+            const double centred = (double)(xv[k] - m), d = (double)dv[k];
+            s[0] = __fma_rn(d, centred, s[0]);
+            s[1] += d;
+            s[2] += centred;
         }
     });
-    bn_block_sums<SAT ? 6 : 5>(t);
+    bn_block_sums<SAT ? BN_SUMS + 1 : BN_SUMS>(s);
     if (threadIdx.x) return;
-    if (SAT) sat.partial[(size_t)c * gridDim.y + blockIdx.y] = t[5];
+    if (SAT) sat.partial[(size_t)c * gridDim.y + blockIdx.y] = s[BN_SUMS];
     if (gridDim.y == 1) {
+        double t[5];
         float dmean, dvariance;
-        bn_stats_grads(n, t, saved_variance[c], epsilon, &dmean, &dvariance);
+        bn_five_sums(t, s, g, inv_sigma);
+        bn_stats_grads(n, t, variance, epsilon, &dmean, &dvariance);
         bn_write_grads(c, t, dmean, dvariance, grads);
     } else {
-        double* o = ws + ((size_t)c * gridDim.y + blockIdx.y) * 5;
-        o[0] = t[0]; o[1] = t[1]; o[2] = t[2]; o[3] = t[3]; o[4] = t[4];
+        double* o = ws + ((size_t)c * gridDim.y + blockIdx.y) * BN_SUMS;
+        o[0] = s[0]; o[1] = s[1]; o[2] = s[2];
     }
 }
-__global__ __launch_bounds__(64) void batchnorm_f32_backward_finish_kernel(double n, int splits, const double* __restrict__ ws,
+__global__ __launch_bounds__(64) void batchnorm_f32_backward_finish_kernel(double n, int splits, const double* __restrict__ ws, const float* __restrict__ scale,
                                                                            const float* __restrict__ saved_variance, double epsilon, BnGrads grads)
 {
     const int c = blockIdx.x;
-    double t[5];
-    bn_partial_sums<5>(t, ws + (size_t)c * splits * 5, splits);
+    double s[BN_SUMS], t[5];
+    bn_partial_sums<BN_SUMS>(s, ws + (size_t)c * splits * BN_SUMS, splits);
     if (threadIdx.x) return;
+    bn_five_sums(t, s, scale[c], bn_inv_sigma(saved_variance[c], epsilon));
     float dmean, dvariance;
     bn_stats_grads(n, t, saved_variance[c], epsilon, &dmean, &dvariance);
     bn_write_grads(c, t, dmean, dvariance, grads);
 }
 
 // dx = dy * scale / sigma + dVar * 2 (x - mean) / size + dMean / size, in ranges of a channel as the apply kernel, the end of the
-// sums before it with it: 4.8 + 8.7 us at 64 x 64 x 32 x 32, now 10.5
-__device__ __forceinline__ float bn_dx(float x, float d, float g, float var, float m, double dv2, double size, double dmean_over_size)
-{
-    const float diff_normalized = d * g;
-    return (float)((double)(diff_normalized / var) + dv2 * (double)(x - m) / size + dmean_over_size);
-}
+// sums before it with it.  In double, what a channel's values share worked out once a block: dx = kd d + kc (x - mean) + k, where
+// there were two divisions a value, one of them in double (figures at the sums).
 template <int V>
 __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_backward_data_kernel(BnRange q, int splits, double n, const double* __restrict__ ws, float size,
                                                                             const float* __restrict__ x, const float* __restrict__ scale,
@@ -769,17 +780,17 @@ __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_backward_data_kernel(BnR
         bn_finish_alpha(sat);
         __syncthreads();
     }
+    const float m = saved_mean[c], g = scale[c], variance = saved_variance[c];
+    const double inv_sigma = bn_inv_sigma(variance, epsilon);
     float dmean, dvariance;
     if (splits > 1) {
         __shared__ float of_stats[2];
         if (threadIdx.x < 64) {
-            double t[5];
-            const double* const p = ws + (size_t)c * splits * 5;
-#pragma unroll
-            for (int k = 0; k < 5; ++k)           // (the first two are the scale's and the bias's)
-                if (k >= 2 || blockIdx.y == 0) t[k] = wave_sum_d((int)threadIdx.x < splits ? p[(size_t)threadIdx.x * 5 + k] : 0.0);
+            double s[BN_SUMS], t[5];
+            bn_partial_sums<BN_SUMS>(s, ws + (size_t)c * splits * BN_SUMS, splits);
             if (threadIdx.x == 0) {
-                bn_stats_grads(n, t, saved_variance[c], epsilon, &dmean, &dvariance);
+                bn_five_sums(t, s, g, inv_sigma);
+                bn_stats_grads(n, t, variance, epsilon, &dmean, &dvariance);
                 of_stats[0] = dmean; of_stats[1] = dvariance;
                 if (blockIdx.y == 0) bn_write_grads(c, t, dmean, dvariance, grads);
             }
@@ -790,15 +801,13 @@ __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_backward_data_kernel(BnR
         dmean = grads.diff_saved_mean[c];
         dvariance = grads.diff_saved_variance[c];
     }
-    const float var = (float)sqrt((double)saved_variance[c] + epsilon);
-    const float m = saved_mean[c], g = scale[c];
-    const double dv2 = (double)dvariance * 2.0, sz = (double)size, dm = (double)(dmean / size);
+    const double kd = (double)g * inv_sigma, kc = (double)dvariance * 2.0 / (double)size, k0 = (double)(dmean / size);
     bn_walk<V>(q, c, [&](size_t idx) {
         float xv[V], dv[V];
         bn_load<V>(xv, x, idx);
         bn_load<V>(dv, dy, idx);
 #pragma unroll
-        for (int k = 0; k < V; ++k) dv[k] = bn_dx(xv[k], dv[k], g, var, m, dv2, sz, dm);
+        for (int k = 0; k < V; ++k) dv[k] = (float)__fma_rn(kd, (double)dv[k], __fma_rn(kc, (double)(xv[k] - m), k0));
         bn_store<V>(dx, idx, dv);
     });
 }
@@ -1933,7 +1942,7 @@ static int batchnorm_backward(const char* who, int B, int C, int H, int W, const
     const int plane = H * W;
     const uintptr_t in = (uintptr_t)x | (uintptr_t)diff_y;
     const BnLaunch l = bn_launch(B, C, plane, splits, in | (uintptr_t)sat.fp);
-    sat.partial = (double*)workspace + (size_t)C * splits * 5;
+    sat.partial = (double*)workspace + (size_t)C * splits * BN_SUMS;
     sat.blocks = C * splits;
     const auto kernel = sat.alpha ? (l.V == 4 ? batchnorm_f32_backward_sums_kernel<4, true> : l.V == 1 ? batchnorm_f32_backward_sums_kernel<1, true>
                                                                                                 : batchnorm_f32_backward_sums_kernel<0, true>)
@@ -1944,7 +1953,7 @@ static int batchnorm_backward(const char* who, int B, int C, int H, int W, const
     const int V = bn_launch(B, C, plane, 1, in | (uintptr_t)diff_x).V;
     const bool walk = diff_x && plane >= BN_WALK_PLANE && V != 0;
     if (splits > 1 && !walk)
-        hipLaunchKernelGGL(batchnorm_f32_backward_finish_kernel, dim3(C), dim3(64), 0, stream, n, splits, (const double*)workspace, saved_variance, epsilon,
+        hipLaunchKernelGGL(batchnorm_f32_backward_finish_kernel, dim3(C), dim3(64), 0, stream, n, splits, (const double*)workspace, scale, saved_variance, epsilon,
                            grads);
     if (walk) {
         const int ranges = bn_ranges(B, C, plane, V);

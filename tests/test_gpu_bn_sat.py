@@ -130,3 +130,35 @@ def test_a_channel_of_few_units_is_added_by_a_small_block(B, Cn, H, W, block):
     m64, v64 = x64.mean((0, 2, 3)), x64.var((0, 2, 3), unbiased=False)
     assert float((v[4].double() - m64).abs().max()) <= float(m64.abs().max()) * 2.0 ** -23
     assert float(((v[5].double() - v64) / v64).abs().max()) <= 2.0 ** -22
+
+
+@pytest.mark.parametrize("shape", SHAPES + [(64, 2, 64, 64)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("workspace", [False, True])
+def test_backward_against_64_bits(shape, workspace):
+    """A channel's sums are formed in double of x - mean as rounded to float (2^-24 of each) with 1 / sigma of a sigma rounded to float,
+    and rounded once; dx then takes them as they were stored.  Bounds accordingly, twice 2^-24 for each rounding beside the sums."""
+    import torch
+    from n2d2_amd import capi, runtime as rt
+    print("bn backward in 64 bits", shape, workspace, flush=True)
+    B, C, H, W = shape
+    lib, rng, u = capi.lib, np.random.default_rng(B + C * H), 2.0 ** -24
+    x, dy = (rng.normal(k, 2 - k, shape).astype(np.float32) for k in (1, 0))
+    scale, m, v = rng.normal(1, .3, C).astype(np.float32), rng.normal(1, .1, C).astype(np.float32), rng.uniform(.5, 5, C).astype(np.float32)
+    dev = lambda a: torch.from_numpy(a).cuda()
+    X, D, S, M, V = map(dev, (x, dy, scale, m, v))
+    ds, db, dm, dv, dx = (torch.empty(n, device="cuda") for n in (C, C, C, C, x.size))
+    ws = torch.empty(int(lib.n2d2hip_batchnorm_f32_workspace_bytes(*shape)), dtype=torch.uint8, device="cuda")
+    capi.check(lib.n2d2hip_batchnorm_f32_backward(*shape, X.data_ptr(), S.data_ptr(), M.data_ptr(), V.data_ptr(), 1e-5, D.data_ptr(), 0.0, ds.data_ptr(), 0.0,
+                                                  db.data_ptr(), dm.data_ptr(), dv.data_ptr(), dx.data_ptr(), ws.data_ptr() if workspace else None,
+                                                  ws.numel() if workspace else 0, rt.stream_ptr()))
+    ds, db, dm, dv, dx = (t.cpu().numpy().astype(np.float64) for t in (ds, db, dm, dv, dx))
+    d, n, at = dy.astype(np.float64), B * H * W, lambda a: a[:, None, None]
+    c, g, sigma = x.astype(np.float64) - at(m.astype(np.float64)), scale.astype(np.float64), np.sqrt(v.astype(np.float64) + 1e-5)
+    total = lambda a: a.sum((0, 2, 3))
+    near = lambda got, want, terms: np.testing.assert_array_less(np.abs(got - want), u * terms + 1e-30)
+    near(ds, total(d * c) / sigma, 4 * total(np.abs(d * c)) / sigma)
+    near(db, total(d), total(np.abs(d)))
+    near(dv, -.5 * g * total(d * c) / sigma ** 3, 4 * np.abs(g) * total(np.abs(d * c)) / sigma ** 3)
+    near(dm, -g * total(d) / sigma - 2 * dv * total(c) / n, 8 * (np.abs(g) * total(np.abs(d)) / sigma + 2 * np.abs(dv) * total(np.abs(c)) / n))
+    parts = [d * at(g / sigma), 2 * at(dv) * c / n, np.broadcast_to(at(dm) / n, shape)]
+    near(dx.reshape(shape), sum(parts), 6 * sum(np.abs(p) for p in parts))
