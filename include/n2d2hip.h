@@ -552,6 +552,11 @@ size_t n2d2hip_conv2d_f32_workspace_bytes(const n2d2hip_conv_desc* desc, int B, 
 int n2d2hip_conv2d_f32_backward_filter(const n2d2hip_conv_desc* desc, int B, int H, int W, const float* x,
                                        const float* diff_y, float beta, float* diff_w, void* workspace,
                                        size_t workspace_bytes, n2d2hip_stream_t stream);
+/* Both of the above, equal to n2d2hip_conv2d_f32_backward_filter followed by n2d2hip_conv2d_f32_backward_data, bit for bit (small
+ * layers that span their input: in one launch). */
+int n2d2hip_conv2d_f32_backward(const n2d2hip_conv_desc* desc, int B, int H, int W, const float* x, const float* w,
+                                const float* diff_y, float beta_w, float* diff_w, float beta_x, float* diff_x,
+                                void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream);
 /* diff_bias[o] = sum over batch and pixels of diff_y + beta * diff_bias (ref: ...ConvCell_Frame_Kernels.cpp:429-452). */
 int n2d2hip_conv2d_f32_backward_bias(int B, int O, int oH, int oW, const float* diff_y, float beta, float* diff_bias,
                                      n2d2hip_stream_t stream);

@@ -252,23 +252,22 @@ void WeightedCell_FrameTrain_HIP::backPropagateWeighted(bool noBias)
     activationBackPropagate();
     const n2d2hip_conv_desc d = desc();
     const int B = (int)mIn->dimB();
-    {
-        const float beta = mWeightsSolver->isNewIteration() ? 0.0f : 1.0f;
+    const float beta = mWeightsSolver->isNewIteration() ? 0.0f : 1.0f;
+    if (mDiffOut && !mDiffOut->empty()) {
+        const float* w = mQuantizer ? mQuantizer->getQuantizedWeights(0) : mDevW.data();
+        checkStatus(n2d2hip_conv2d_f32_backward(&d, B, (int)mInH, (int)mInW, mIn->data(), w, mDiffInputs.data(), beta, mDevDiffW.data(),
+                                                mDiffOut->isValid() ? 1.0f : 0.0f, mDiffOut->data(), mWorkspace.data(),
+                                                mWorkspace.size() * sizeof(float), mStream));
+        mDiffOut->setValid();
+    } else {
         checkStatus(n2d2hip_conv2d_f32_backward_filter(&d, B, (int)mInH, (int)mInW, mIn->data(), mDiffInputs.data(), beta, mDevDiffW.data(),
                                                        mWorkspace.data(), mWorkspace.size() * sizeof(float), mStream));
-        mDevDiffW.setValid();
     }
+    mDevDiffW.setValid();
     if (!noBias) {
         const float beta = mBiasSolver->isNewIteration() ? 0.0f : 1.0f;
         checkStatus(n2d2hip_conv2d_f32_backward_bias(B, (int)mNbOutputs, (int)mOutH, (int)mOutW, mDiffInputs.data(), beta, mDevDiffBias.data(), mStream));
         mDevDiffBias.setValid();
-    }
-    if (mDiffOut && !mDiffOut->empty()) {
-        const float beta = mDiffOut->isValid() ? 1.0f : 0.0f;
-        const float* w = mQuantizer ? mQuantizer->getQuantizedWeights(0) : mDevW.data();
-        checkStatus(n2d2hip_conv2d_f32_backward_data(&d, B, (int)mInH, (int)mInW, w, mDiffInputs.data(), beta, mDiffOut->data(),
-                                                     mWorkspace.data(), mWorkspace.size() * sizeof(float), mStream));
-        mDiffOut->setValid();
     }
     if (mQuantizer)
         mQuantizer->back_propagate();

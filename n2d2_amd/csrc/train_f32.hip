@@ -1529,7 +1529,8 @@ static int run_small_filter(FilterGemm g, const float* x, const float* dy, float
     if (splits * n * sizeof(double) > ws_bytes || ((size_t)ws & 7)) splits = 1;
     g.kchunk = round_up(ceil_div_i(g.K, splits), 64);
     splits = ceil_div_i(g.K, g.kchunk);
-    hipLaunchKernelGGL(conv_f32_filter_small_kernel, dim3(ceil_div_i(g.P, 16), ceil_div_i(g.Q, 16), splits), dim3(256), 0, st, g, x, dy, ws, beta, out);
+    hipLaunchKernelGGL(conv_f32_filter_small_kernel, dim3(ceil_div_i(g.P, 16), ceil_div_i(g.Q, 16), splits), dim3(256), 0, st, g, x, dy,
+                       splits > 1 ? ws : (double*)nullptr, beta, out);
     if (splits > 1)
         hipLaunchKernelGGL(conv_f32_reduce_partials_kernel<double>, dim3(reduce_grid(n)), dim3(256), 0, st, (const double*)ws, splits, n, beta, out,
                            (const float*)nullptr, 1, 1);
@@ -1775,6 +1776,47 @@ int n2d2hip_conv2d_f32_backward_filter(const n2d2hip_conv_desc* desc, int B, int
     hipLaunchKernelGGL(conv_f32_backward_filter_kernel, dim3((unsigned)nw), dim3(TBLOCK), 0, (hipStream_t)stream, q, x, diff_y, beta, diff_w);
     N2D2HIP_HIP_CHECK(hipGetLastError());
     return N2D2HIP_OK;
+}
+
+// (neither product in ranges, whose partial results a second launch adds up; 2^30 tiles at most)
+static bool small_pair(const ConvF32& q, SmallPair* a, long* blocks)
+{
+    if (f32_path(q, PASS_BWD_FILTER) != F32_PATH_SMALL || f32_path(q, PASS_BWD_DATA) != F32_PATH_SMALL) return false;
+    *blocks = 0;
+    for (int k = 0; k < 2; ++k) {
+        SmallProduct& s = a->of[k];
+        s.g = small_gemm(q, k ? PASS_BWD_DATA : PASS_BWD_FILTER);
+        if (small_filter_splits(s.g) > 1) return false;
+        s.g.kchunk = round_up(s.g.K, 64);
+        s.ptiles = ceil_div_i(s.g.P, 16);
+        if (k) a->first = (unsigned)*blocks;
+        *blocks += (long)s.ptiles * ceil_div_i(s.g.Q, 16);
+        if (*blocks >= 1L << 30) return false;
+    }
+    return true;
+}
+int n2d2hip_conv2d_f32_backward(const n2d2hip_conv_desc* desc, int B, int H, int W, const float* x, const float* w, const float* diff_y, float beta_w,
+                                float* diff_w, float beta_x, float* diff_x, void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream)
+{
+    ConvF32 q;
+    const int st = make_conv(desc, B, H, W, true, &q, "n2d2hip_conv2d_f32_backward");
+    if (st != N2D2HIP_OK) return st;
+    N2D2HIP_REQUIRE(x && w && diff_y && diff_w && diff_x, N2D2HIP_ERR_INVALID, "n2d2hip_conv2d_f32_backward: null pointer");
+    const size_t nx = (size_t)q.B * q.C * q.H * q.W, nw = (size_t)q.O * q.Cw * q.kH * q.kW, ny = (size_t)q.B * q.O * q.oH * q.oW;
+    const auto apart = [](const float* a, size_t na, const float* b, size_t nb) { return a + na <= b || b + nb <= a; };
+    SmallPair a;
+    long blocks;
+    // (results over the operands, as the two passes one behind the other allow: in that order)
+    if (small_pair(q, &a, &blocks) && apart(diff_w, nw, x, nx) && apart(diff_w, nw, w, nw) && apart(diff_w, nw, diff_y, ny) && apart(diff_x, nx, x, nx)
+        && apart(diff_x, nx, w, nw) && apart(diff_x, nx, diff_y, ny) && apart(diff_x, nx, diff_w, nw)) {
+        a.of[0].srcX = x; a.of[0].srcY = diff_y; a.of[0].beta = beta_w; a.of[0].out = diff_w;
+        a.of[1].srcX = w; a.of[1].srcY = diff_y; a.of[1].beta = beta_x; a.of[1].out = diff_x;
+        N2D2HIP_LAUNCH(conv_f32_small_pair_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a);
+        N2D2HIP_HIP_CHECK(hipGetLastError());
+        return N2D2HIP_OK;
+    }
+    const int rc = n2d2hip_conv2d_f32_backward_filter(desc, B, H, W, x, diff_y, beta_w, diff_w, workspace, workspace_bytes, stream);
+    return rc != N2D2HIP_OK ? rc : n2d2hip_conv2d_f32_backward_data(desc, B, H, W, w, diff_y, beta_x, diff_x, workspace, workspace_bytes, stream);
 }
 
 int n2d2hip_conv2d_f32_backward_bias(int B, int O, int oH, int oW, const float* diff_y, float beta, float* diff_bias, n2d2hip_stream_t stream)
