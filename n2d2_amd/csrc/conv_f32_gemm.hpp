@@ -1158,13 +1158,16 @@ __global__ __launch_bounds__(256) void conv_f32_filter_kernel(FilterGemm g, cons
 // 16 x 16: 50 -> 12 us.  Spanning layers, whose K is the batch: 16384 -> 10, 64 images: 211 -> 8.2 us; 20736 -> 64, 64 images:
 // 1690 -> 22 (fp32 matrix instructions take 10, with four times the error of a sum in double: 1.4e-7 against 2.5e-8).
 typedef double v4d __attribute__((ext_vector_type(4)));
+// (WAVES: of the block, the first four take part)
+template <int WAVES>
 __device__ __forceinline__ void filter_small_tile(const FilterGemm& g, int tp, int tq, int range, const float* __restrict__ srcX, const float* __restrict__ srcY,
                                                   double* __restrict__ partial, float beta, float* __restrict__ out)
 {
     __shared__ double red[4][256];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane & 15, kg = lane >> 4;
     const int p = tp * 16 + row, q = tq * 16 + row;
-    const int kbeg = range * g.kchunk, kend = min(kbeg + g.kchunk, g.K);
+    const bool takes = WAVES == 4 || wave < 4;
+    const int kbeg = range * g.kchunk, kend = takes ? min(kbeg + g.kchunk, g.K) : kbeg;
     const int kHW = g.kH * g.kW, pp = min(p, g.P - 1);
     const int ch = pp / kHW, t = pp - ch * kHW, ty = t / g.kW, tx = t - ty * g.kW;
     const float* xb = srcX + (size_t)ch * g.H * g.W;
@@ -1198,8 +1201,10 @@ __device__ __forceinline__ void filter_small_tile(const FilterGemm& g, int tp, i
     }
     // lane holds column p = lane % 16 and rows q = 4 r + lane / 16
 #pragma unroll
-    for (int r = 0; r < 4; ++r) red[wave][(4 * r + kg) * 16 + row] = acc[r];
+    for (int r = 0; r < 4; ++r)
+        if (takes) red[wave][(4 * r + kg) * 16 + row] = acc[r];
     __syncthreads();
+    if (!takes) return;
     const int oq = tq * 16 + threadIdx.x / 16, op = tp * 16 + threadIdx.x % 16;
     if (oq >= g.Q || op >= g.P) return;
     const double v = ((red[0][threadIdx.x] + red[1][threadIdx.x]) + red[2][threadIdx.x]) + red[3][threadIdx.x];
@@ -1210,7 +1215,7 @@ __device__ __forceinline__ void filter_small_tile(const FilterGemm& g, int tp, i
 __global__ __launch_bounds__(256) void conv_f32_filter_small_kernel(FilterGemm g, const float* __restrict__ srcX, const float* __restrict__ srcY,
                                                                     double* __restrict__ partial, float beta, float* __restrict__ out)
 {
-    filter_small_tile(g, blockIdx.x, blockIdx.y, blockIdx.z, srcX, srcY, partial, beta, out);
+    filter_small_tile<4>(g, blockIdx.x, blockIdx.y, blockIdx.z, srcX, srcY, partial, beta, out);
 }
 // Both gradients of a small spanning layer in one launch: two such products, of which neither reads what the other writes, and a launch
 // each was what they took.  us, two launches / one: 84 <- 120, 32 images 8.4 / 4.5; 120 <- 16 x 5 x 5 8.3 / 4.6; 64 <- 512, 255 images
@@ -1231,7 +1236,7 @@ __global__ __launch_bounds__(256) void conv_f32_small_pair_kernel(const SmallPai
     const int k = blockIdx.x >= a.first;
     const SmallProduct& s = a.of[k];
     const int block = blockIdx.x - (k ? a.first : 0), tq = block / s.ptiles;
-    filter_small_tile(s.g, block - tq * s.ptiles, tq, 0, s.srcX, s.srcY, nullptr, s.beta, s.out);
+    filter_small_tile<4>(s.g, block - tq * s.ptiles, tq, 0, s.srcX, s.srcY, nullptr, s.beta, s.out);
 }
 
 // Backward-data of small problems, the same way: dx[c][pixel] adds w[o][c][tap] dy[o][the pixel that the tap reaches] over (o, tap)
@@ -1249,15 +1254,15 @@ struct DataSmall {
     DivF32 dHW, dW, dT, dkW, dsy, dsx;
 };
 template <int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void conv_f32_data_small_kernel(DataSmall g, const float* __restrict__ w, const float* __restrict__ dy, float beta,
-                                                                  float* __restrict__ dx)
+__device__ __forceinline__ void data_small_tile(const DataSmall& g, int tp, int tc, const float* __restrict__ w, const float* __restrict__ dy, float beta,
+                                                float* __restrict__ dx)
 {
     __shared__ double red[WAVES][256];
     __shared__ int reach[64 * 16];               // where in a channel's image a pixel's tap is; -1: outside
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane & 15, kg = lane >> 4;
-    const int c = blockIdx.y * 16 + row, plane = g.oH * g.oW;
+    const int c = tc * 16 + row, plane = g.oH * g.oW;
     {
-        const int p = min((int)(blockIdx.x * 16 + (threadIdx.x & 15)), g.P - 1), rem = p - div_f32(p, g.dHW) * g.HW, iy = div_f32(rem, g.dW), ix = rem - iy * g.W;
+        const int p = min(tp * 16 + (int)(threadIdx.x & 15), g.P - 1), rem = p - div_f32(p, g.dHW) * g.HW, iy = div_f32(rem, g.dW), ix = rem - iy * g.W;
         for (int t = threadIdx.x >> 4; t < g.T; t += 4 * WAVES) {
             const int ty = div_f32(t, g.dkW), y = iy + g.pt - ty, x = ix + g.pl - (t - ty * g.kW);
             const int oy = div_f32(max(y, 0), g.dsy), ox = div_f32(max(x, 0), g.dsx);
@@ -1266,7 +1271,7 @@ __global__ __launch_bounds__(64 * WAVES) void conv_f32_data_small_kernel(DataSma
     }
     __syncthreads();
     const float* wb = w + (size_t)min(c, g.C - 1) * g.T;
-    const float* yb = dy + (size_t)div_f32(min((int)(blockIdx.x * 16 + row), g.P - 1), g.dHW) * g.O * plane;
+    const float* yb = dy + (size_t)div_f32(min(tp * 16 + row, g.P - 1), g.dHW) * g.O * plane;
     float a[2][4], b[2][4];
     const int adv_o = div_f32(16 * WAVES, g.dT), adv_t = 16 * WAVES - adv_o * g.T;
     int ko = div_f32(wave * 16 + kg * 4, g.dT), kt = wave * 16 + kg * 4 - ko * g.T;     // this lane's next term
@@ -1298,7 +1303,7 @@ __global__ __launch_bounds__(64 * WAVES) void conv_f32_data_small_kernel(DataSma
     for (int r = 0; r < 4; ++r) red[wave][(4 * r + kg) * 16 + row] = acc[r];
     __syncthreads();
     if (threadIdx.x >= 256) return;
-    const int oc = blockIdx.y * 16 + threadIdx.x / 16, op = blockIdx.x * 16 + threadIdx.x % 16;
+    const int oc = tc * 16 + threadIdx.x / 16, op = tp * 16 + threadIdx.x % 16;
     if (oc >= g.C || op >= g.P) return;
     double v = red[0][threadIdx.x];
 #pragma unroll
@@ -1306,6 +1311,37 @@ __global__ __launch_bounds__(64 * WAVES) void conv_f32_data_small_kernel(DataSma
     const int oi = div_f32(op, g.dHW);
     const size_t idx = ((size_t)oi * g.C + oc) * g.HW + (op - oi * g.HW);
     dx[idx] = (float)v + (beta != 0.0f ? beta * dx[idx] : 0.0f);
+}
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void conv_f32_data_small_kernel(DataSmall g, const float* __restrict__ w, const float* __restrict__ dy, float beta,
+                                                                         float* __restrict__ dx)
+{
+    data_small_tile<WAVES>(g, blockIdx.x, blockIdx.y, w, dy, beta, dx);
+}
+// Both gradients of a small layer in one launch, the blocks of the data first, which take longer, then those of the weights, whose ranges
+// are added by the launch that follows.  us, two launches / one, with the one that adds: 6 <- 16, 5x5, 14 x 14, batch 32 15.5 / 12.4; 64 <- 64,
+// 3x3 stride 2, 14 x 14, batch 4 12.1 / 8.5; 8 <- 8, 3x3, 16 x 16, batch 2 11.3 / 7.4.
+struct SmallBoth {
+    DataSmall data;
+    int dtiles;                                  // of 16 pixels
+    unsigned first;                              // first block of the weights'
+    SmallProduct filter;
+    int ftiles;                                  // tiles of a range
+    const float *w, *dy;
+    float beta;
+    float* dx;
+    double* partial;
+};
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void conv_f32_small_both_kernel(const SmallBoth a)
+{
+    if (blockIdx.x < a.first) {
+        const int tc = blockIdx.x / a.dtiles;
+        data_small_tile<WAVES>(a.data, blockIdx.x - tc * a.dtiles, tc, a.w, a.dy, a.beta, a.dx);
+    } else {
+        const int block = blockIdx.x - a.first, range = block / a.ftiles, tile = block - range * a.ftiles, tq = tile / a.filter.ptiles;
+        filter_small_tile<WAVES>(a.filter.g, tile - tq * a.filter.ptiles, tq, range, a.filter.srcX, a.filter.srcY, a.partial, a.filter.beta, a.filter.out);
+    }
 }
 
 // out[i] = sum over the K ranges + beta * out[i] (+ bias of element i's channel, NCHW with `plane` pixels per channel and O

@@ -1521,14 +1521,18 @@ static int small_filter_splits(const FilterGemm& g)
     const long tiles = (long)ceil_div_i(g.P, 16) * ceil_div_i(g.Q, 16);
     return (int)std::max(1L, std::min<long>(512 / tiles, g.K / 128));
 }
-// (a workspace too small for the partial results: one range)
-static int run_small_filter(FilterGemm g, const float* x, const float* dy, float beta, float* out, double* ws, size_t ws_bytes, hipStream_t st)
+// -> ranges, and their length in g (a workspace too small for the partial results: one range)
+static int small_filter_ranges(FilterGemm& g, size_t n, const double* ws, size_t ws_bytes)
 {
-    const size_t n = (size_t)g.Q * g.P;
     int splits = small_filter_splits(g);
     if (splits * n * sizeof(double) > ws_bytes || ((size_t)ws & 7)) splits = 1;
     g.kchunk = round_up(ceil_div_i(g.K, splits), 64);
-    splits = ceil_div_i(g.K, g.kchunk);
+    return ceil_div_i(g.K, g.kchunk);
+}
+static int run_small_filter(FilterGemm g, const float* x, const float* dy, float beta, float* out, double* ws, size_t ws_bytes, hipStream_t st)
+{
+    const size_t n = (size_t)g.Q * g.P;
+    const int splits = small_filter_ranges(g, n, ws, ws_bytes);
     hipLaunchKernelGGL(conv_f32_filter_small_kernel, dim3(ceil_div_i(g.P, 16), ceil_div_i(g.Q, 16), splits), dim3(256), 0, st, g, x, dy,
                        splits > 1 ? ws : (double*)nullptr, beta, out);
     if (splits > 1)
@@ -1692,6 +1696,12 @@ int n2d2hip_conv2d_f32_forward(const n2d2hip_conv_desc* desc, int B, int H, int 
     return run_direct(q, PASS_FWD, x, w, bias, beta, y, (hipStream_t)stream);
 }
 
+static DataSmall small_data(const ConvF32& q)
+{
+    const int T = q.kH * q.kW;
+    return DataSmall{q.B * q.H * q.W, q.C, q.O, T, q.O * T, q.kW, q.H * q.W, q.W, q.oH, q.oW, q.sy, q.sx, q.pt, q.pl,
+                     div_of(q.H * q.W), div_of(q.W), div_of(T), div_of(q.kW), div_of(q.sy), div_of(q.sx)};
+}
 int n2d2hip_conv2d_f32_backward_data(const n2d2hip_conv_desc* desc, int B, int H, int W, const float* w, const float* diff_y, float beta,
                                      float* diff_x, void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream)
 {
@@ -1703,9 +1713,7 @@ int n2d2hip_conv2d_f32_backward_data(const n2d2hip_conv_desc* desc, int B, int H
     if (path == F32_PATH_SMALL)
         return run_small_filter(small_gemm(q, PASS_BWD_DATA), w, diff_y, beta, diff_x, (double*)workspace, workspace ? workspace_bytes : 0, (hipStream_t)stream);
     if (path == F32_PATH_SMALL_DATA) {
-        const int T = q.kH * q.kW;
-        const DataSmall g = {q.B * q.H * q.W, q.C, q.O, T, q.O * T, q.kW, q.H * q.W, q.W, q.oH, q.oW, q.sy, q.sx, q.pt, q.pl,
-                             div_of(q.H * q.W), div_of(q.W), div_of(T), div_of(q.kW), div_of(q.sy), div_of(q.sx)};
+        const DataSmall g = small_data(q);
         const dim3 grid(ceil_div_i(g.P, 16), ceil_div_i(g.C, 16));
         if (g.K <= 256) hipLaunchKernelGGL(conv_f32_data_small_kernel<4>, grid, dim3(256), 0, (hipStream_t)stream, g, w, diff_y, beta, diff_x);
         else hipLaunchKernelGGL(conv_f32_data_small_kernel<8>, grid, dim3(512), 0, (hipStream_t)stream, g, w, diff_y, beta, diff_x);
@@ -1803,17 +1811,43 @@ int n2d2hip_conv2d_f32_backward(const n2d2hip_conv_desc* desc, int B, int H, int
     if (st != N2D2HIP_OK) return st;
     N2D2HIP_REQUIRE(x && w && diff_y && diff_w && diff_x, N2D2HIP_ERR_INVALID, "n2d2hip_conv2d_f32_backward: null pointer");
     const size_t nx = (size_t)q.B * q.C * q.H * q.W, nw = (size_t)q.O * q.Cw * q.kH * q.kW, ny = (size_t)q.B * q.O * q.oH * q.oW;
-    const auto apart = [](const float* a, size_t na, const float* b, size_t nb) { return a + na <= b || b + nb <= a; };
+    const auto disjoint = [](const float* a, size_t na, const float* b, size_t nb) { return a + na <= b || b + nb <= a; };
+    // (results over the operands, as the two passes one behind the other allow: in that order)
+    const bool apart = disjoint(diff_w, nw, x, nx) && disjoint(diff_w, nw, w, nw) && disjoint(diff_w, nw, diff_y, ny) && disjoint(diff_x, nx, x, nx)
+                       && disjoint(diff_x, nx, w, nw) && disjoint(diff_x, nx, diff_y, ny) && disjoint(diff_x, nx, diff_w, nw);
     SmallPair a;
     long blocks;
-    // (results over the operands, as the two passes one behind the other allow: in that order)
-    if (small_pair(q, &a, &blocks) && apart(diff_w, nw, x, nx) && apart(diff_w, nw, w, nw) && apart(diff_w, nw, diff_y, ny) && apart(diff_x, nx, x, nx)
-        && apart(diff_x, nx, w, nw) && apart(diff_x, nx, diff_y, ny) && apart(diff_x, nx, diff_w, nw)) {
+    if (apart && small_pair(q, &a, &blocks)) {
         a.of[0].srcX = x; a.of[0].srcY = diff_y; a.of[0].beta = beta_w; a.of[0].out = diff_w;
         a.of[1].srcX = w; a.of[1].srcY = diff_y; a.of[1].beta = beta_x; a.of[1].out = diff_x;
         N2D2HIP_LAUNCH(conv_f32_small_pair_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a);
         N2D2HIP_HIP_CHECK(hipGetLastError());
         return N2D2HIP_OK;
+    }
+    if (apart && f32_path(q, PASS_BWD_FILTER) == F32_PATH_SMALL && f32_path(q, PASS_BWD_DATA) == F32_PATH_SMALL_DATA) {
+        SmallBoth b = {};
+        b.data = small_data(q);
+        b.dtiles = ceil_div_i(b.data.P, 16);
+        b.first = (unsigned)(b.dtiles * ceil_div_i(b.data.C, 16));               // (2.3e5 / K at most)
+        b.filter.g = small_gemm(q, PASS_BWD_FILTER);
+        const size_t n = (size_t)b.filter.g.Q * b.filter.g.P;
+        const int ranges = small_filter_ranges(b.filter.g, n, (const double*)workspace, workspace ? workspace_bytes : 0);
+        b.filter.ptiles = ceil_div_i(b.filter.g.P, 16);
+        const long ftiles = (long)b.filter.ptiles * ceil_div_i(b.filter.g.Q, 16);
+        if (ftiles * ranges < 1L << 30) {
+            b.ftiles = (int)ftiles;
+            b.filter.srcX = x; b.filter.srcY = diff_y; b.filter.beta = beta_w; b.filter.out = diff_w;
+            b.w = w; b.dy = diff_y; b.beta = beta_x; b.dx = diff_x;
+            b.partial = ranges > 1 ? (double*)workspace : nullptr;
+            const dim3 grid(b.first + (unsigned)(ftiles * ranges));
+            if (b.data.K <= 256) N2D2HIP_LAUNCH(conv_f32_small_both_kernel<4>, grid, dim3(256), 0, (hipStream_t)stream, b);
+            else N2D2HIP_LAUNCH(conv_f32_small_both_kernel<8>, grid, dim3(512), 0, (hipStream_t)stream, b);
+            if (ranges > 1)
+                hipLaunchKernelGGL(conv_f32_reduce_partials_kernel<double>, dim3(reduce_grid(n)), dim3(256), 0, (hipStream_t)stream, (const double*)workspace,
+                                   ranges, n, beta_w, diff_w, (const float*)nullptr, 1, 1);
+            N2D2HIP_HIP_CHECK(hipGetLastError());
+            return N2D2HIP_OK;
+        }
     }
     const int rc = n2d2hip_conv2d_f32_backward_filter(desc, B, H, W, x, diff_y, beta_w, diff_w, workspace, workspace_bytes, stream);
     return rc != N2D2HIP_OK ? rc : n2d2hip_conv2d_f32_backward_data(desc, B, H, W, w, diff_y, beta_x, diff_x, workspace, workspace_bytes, stream);
