@@ -19,6 +19,7 @@ struct DepthwiseF32 {
     int strips;                                  // strips of a row
     int nx, ny;                                  // values of x (or dx) and y (or dy)
     DivF32 dstrips, drows;
+    int narrow;                                  // backward-filter: strips are whole, and reach at most K / 2 columns past a row's ends
 };
 
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
@@ -166,7 +167,11 @@ __global__ __launch_bounds__(256) void depthwise_f32_data_kernel(DepthwiseF32 q,
 // Backward-filter: a block adds the products of all K^2 taps over one range of a channel's strips in double, so both tensors
 // are read once (x's rows K times, out of the caches).  gridDim.y is the number of ranges; one: the sums are the gradient,
 // more: they go to partial[range][channel][tap], which conv_f32_reduce_partials_kernel adds up.
-// What bounds it is the vector ALU: four instructions a product (multiply, select, conversion, addition in double).
+// What bounds it is the vector ALU: four instructions a product (multiply, select, conversion, addition in double), three where the
+// product's column is in the row for certain: rows of whole strips with at most K / 2 columns of padding on either side (q.narrow)
+// select for the K / 2 outer columns of a strip alone.  us, all / these: 128 channels, 3x3, 56 x 56, batch 32 30.3 / 25.8; 64 channels,
+// 112 x 112 46.7 / 38.5, at stride 2 28.4 / 27.0; 96 channels, 5x5, 56 x 56, batch 16 28.3 / 23.5.  (Multiply-adds in double, an
+// instruction a product behind the conversions: 40.6 for the first.)
 // 128 channels, 3x3, 56 x 56, batch 32: a block per channel and tap row, which loaded and converted dy's strip once per row
 // and stood on 384 blocks, 48.6 us; now 31.1 with the launch that adds the ranges up.
 // ROWS: tap rows of a block, all K, or one (blockIdx.z is which) where a channel's strips are few: depthwise_row_threads() in
@@ -179,33 +184,38 @@ __global__ __launch_bounds__(THREADS) void depthwise_f32_filter_kernel(Depthwise
     constexpr int NX = 3 * S + K;
     const int c = blockIdx.x, end = min(q.items, ((int)blockIdx.y + 1) * per_range), ty0 = ROWS == K ? 0 : (int)blockIdx.z;
     double acc[ROWS][K] = {};
-    for (int i = (int)blockIdx.y * per_range + threadIdx.x; i < end; i += THREADS) {
-        const int r = div_f32(i, q.dstrips), ox0 = (i - r * q.strips) * 4, b = div_f32(r, q.drows), oy = r - b * q.oH;
-        const int iy0 = oy * S - q.pt + ty0, ix0 = ox0 * S - q.pl, img = b * q.C + c;
-        float xv[ROWS][NX], dv[4];
-        strip_load<4>(dv, dy, (img * q.oH + oy) * q.oW + ox0, q.ny);
+    const auto add = [&](auto narrow) {
+        for (int i = (int)blockIdx.y * per_range + threadIdx.x; i < end; i += THREADS) {
+            const int r = div_f32(i, q.dstrips), ox0 = (i - r * q.strips) * 4, b = div_f32(r, q.drows), oy = r - b * q.oH;
+            const int iy0 = oy * S - q.pt + ty0, ix0 = ox0 * S - q.pl, img = b * q.C + c;
+            float xv[ROWS][NX], dv[4];
+            strip_load<4>(dv, dy, (img * q.oH + oy) * q.oW + ox0, q.ny);
 #pragma unroll
-        for (int ty = 0; ty < ROWS; ++ty)
-            if ((unsigned)(iy0 + ty) < (unsigned)q.H)
-                strip_load<NX>(xv[ty], x, (img * q.H + iy0 + ty) * q.W + ix0, q.nx);
-        bool inside[4][K];
+            for (int ty = 0; ty < ROWS; ++ty)
+                if ((unsigned)(iy0 + ty) < (unsigned)q.H)
+                    strip_load<NX>(xv[ty], x, (img * q.H + iy0 + ty) * q.W + ix0, q.nx);
+            bool inside[4][K];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+            for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int t = 0; t < K; ++t)
-                inside[u][t] = ox0 + u < q.oW && (unsigned)(ix0 + u * S + t) < (unsigned)q.W;
+                for (int t = 0; t < K; ++t)
+                    inside[u][t] = (decltype(narrow)::value && u * S + t >= K / 2 && u * S + t < NX - K / 2)
+                                   || (ox0 + u < q.oW && (unsigned)(ix0 + u * S + t) < (unsigned)q.W);
 #pragma unroll
-        for (int ty = 0; ty < ROWS; ++ty)
-            if ((unsigned)(iy0 + ty) < (unsigned)q.H) {
+            for (int ty = 0; ty < ROWS; ++ty)
+                if ((unsigned)(iy0 + ty) < (unsigned)q.H) {
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
+                    for (int u = 0; u < 4; ++u)
 #pragma unroll
-                    for (int t = 0; t < K; ++t) {
-                        const float p = xv[ty][u * S + t] * dv[u];
-                        acc[ty][t] += (double)(inside[u][t] ? p : 0.0f);
-                    }
-            }
-    }
+                        for (int t = 0; t < K; ++t) {
+                            const float p = xv[ty][u * S + t] * dv[u];
+                            acc[ty][t] += (double)(inside[u][t] ? p : 0.0f);
+                        }
+                }
+        }
+    };
+    if (q.narrow) add(std::true_type{});
+    else add(std::false_type{});
     __shared__ double red[THREADS / 64][ROWS * K];
 #pragma unroll
     for (int t = 0; t < ROWS * K; ++t) {

@@ -721,7 +721,7 @@ __global__ __launch_bounds__(1024) void batchnorm_f32_backward_sums_kernel(BnRan
         float xv[N], dv[N];
         bn_load<N>(xv, x, idx);
         bn_load<N>(dv, dy, idx);
-        if (SAT) {
+        if constexpr (SAT) {
             float fp[N];
             bn_load<N>(fp, sat.fp, idx);
 #pragma unroll
@@ -1054,7 +1054,8 @@ static int run_depthwise(const ConvF32& q, int pass, const float* a, const float
 {
     const int rows = pass == PASS_BWD_DATA ? q.H : q.oH, cols = pass == PASS_BWD_DATA ? q.W : q.oW, strips = ceil_div_i(cols, 4);
     const DepthwiseF32 k = {q.C, q.H, q.W, q.oH, q.oW, q.pl, q.pt, q.B * rows * strips, strips, q.B * q.C * q.H * q.W, q.B * q.C * q.oH * q.oW,
-                            div_of(strips), div_of(rows)};
+                            div_of(strips), div_of(rows),
+                            q.oW % 4 == 0 && q.pl <= q.kW / 2 && (q.oW - 1) * q.sx - q.pl + q.kW - 1 < q.W + q.kW / 2};
     const dim3 grid(ceil_div_i(k.items, 256), q.C);
     const auto run = [&](auto K_, auto S_) {
         constexpr int K = decltype(K_)::value, S = decltype(S_)::value;
