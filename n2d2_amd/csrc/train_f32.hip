@@ -912,6 +912,39 @@ __global__ __launch_bounds__(TBLOCK) void pool_max_f32_backward_kernel(PoolF32 q
     }
 }
 
+// The same for rows of whole quads: a lane takes four inputs of a row and goes through the windows that hold one of them, so that a
+// window's two loads and the places are worked out once for the four.  (Of the same windows an input adds the same values in the same
+// order.)  us, an input / a quad a lane: 64 x 64 x 32 x 32, 2x2 11.6 / 6.6 (42 MB); 32 x 64 x 112 x 112, 3x3 at 2 123 / 45; 32 x 64 x 56 x 56, 3x3
+// at 1 72 / 57; 16 x 32 x 64 x 64, 7x7 at 7 7.7 / 4.3; 2 x 8 x 8 x 8 4.0 / 3.8.
+__global__ __launch_bounds__(TBLOCK) void pool_max_f32_backward_quads_kernel(PoolF32 q, DivF32 dquads, const float* __restrict__ dy, const int* __restrict__ argmax,
+                                                                             float beta, float* __restrict__ dx)
+{
+    const int quads = q.W / 4, total = q.B * q.C * q.H * quads;
+    for (int i = (int)(blockIdx.x * TBLOCK + threadIdx.x); i < total; i += (int)gridDim.x * TBLOCK) {
+        const int row = div_f32(i, dquads), ix = (i - row * quads) * 4, bc = div_f32(row, q.dh), iy = row - bc * q.H;
+        // windows that begin at or before the last of the four, and end behind the first
+        const int iy_pad = iy + q.py, oy0 = div_f32(iy_pad, q.dsy), ox0 = min(div_f32(ix + 3 + q.px, q.dsx), q.oW - 1);
+        const int place = iy * q.W + ix;
+        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int oy = oy0, sy = iy_pad - oy0 * q.sy; sy < q.ph && oy >= 0; sy += q.sy, --oy) {
+            if (oy >= q.oH) continue;
+            const int base = (bc * q.oH + oy) * q.oW;
+            for (int ox = ox0; ox >= 0 && ox * q.sx + q.pw > ix + q.px; --ox) {
+                const int at = argmax[base + ox] - place;
+                const float d = dy[base + ox];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) acc[u] = at == u ? acc[u] + d : acc[u];
+            }
+        }
+        float4* const out = (float4*)dx + i;
+        if (beta != 0.0f) {
+            const float4 o = *out;
+            acc[0] += beta * o.x; acc[1] += beta * o.y; acc[2] += beta * o.z; acc[3] += beta * o.w;
+        }
+        *out = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    }
+}
+
 static int grid_for(size_t total)
 {
     const size_t blocks = (total + TBLOCK - 1) / TBLOCK;
@@ -2113,6 +2146,12 @@ int n2d2hip_pool_max_f32_backward(int B, int C, int H, int W, int pool_w, int po
     const int rc = make_pool(B, C, H, W, pool_w, pool_h, stride_x, stride_y, pad_x, pad_y, &q, "n2d2hip_pool_max_f32_backward");
     if (rc != N2D2HIP_OK) return rc;
     N2D2HIP_REQUIRE(diff_y && argmax && diff_x, N2D2HIP_ERR_INVALID, "n2d2hip_pool_max_f32_backward: null pointer");
+    if (pool_small(q) && W % 4 == 0 && ((size_t)diff_x & 15) == 0) {
+        hipLaunchKernelGGL(pool_max_f32_backward_quads_kernel, dim3(grid_for((size_t)B * C * H * W / 4)), dim3(TBLOCK), 0, (hipStream_t)stream, q, div_of(W / 4), diff_y,
+                           argmax, beta, diff_x);
+        N2D2HIP_HIP_CHECK(hipGetLastError());
+        return N2D2HIP_OK;
+    }
     hipLaunchKernelGGL(pool_small(q) ? pool_max_f32_backward_kernel<true> : pool_max_f32_backward_kernel<false>, dim3(grid_for((size_t)B * C * H * W)),
                        dim3(TBLOCK), 0, (hipStream_t)stream, q, diff_y, argmax, beta, diff_x);
     N2D2HIP_HIP_CHECK(hipGetLastError());
