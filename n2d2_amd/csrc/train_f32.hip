@@ -1684,7 +1684,15 @@ static int run_pass(const ConvF32& q, int pass, const float* a, const float* b, 
         ws_floats -= nlaid;
     }
     if (splits * n > ws_floats) {                           // no room for partial results: a block takes all ranges
-        for (PixelPlan& pl : plans) pl.g.nz *= pl.splits;
+        for (PixelPlan& pl : plans) {
+            if (kind == PIXELS_PATCH) {          // (whose ranges are not walked one by one: a single one of all chunks)
+                const int fold = patch_fold(q, pass, cls[0]), chunks = ceil_div_i(pl.g.Ch, PK);
+                pl.g.c[0].kchunk = chunks;
+                pl.g.c[0].fold = fold < chunks ? fold : 0;
+            } else {
+                pl.g.nz *= pl.splits;
+            }
+        }
         splits = 1;
     }
     for (PixelPlan& pl : plans) {

@@ -22,7 +22,7 @@ def _passes(x, w, dy, s, pad):
     return y.detach().numpy(), x64.grad.numpy()
 
 
-def _run(x, w, dy, s, pad, bias=None, beta=0.0, start=0.0, workspace=True):
+def _run(x, w, dy, s, pad, bias=None, beta=0.0, start=0.0, workspace=True, less=0):
     import torch
     from n2d2_amd import capi, runtime as rt
     (B, Ci, H, W), (O, _, kH, kW) = x.shape, w.shape
@@ -31,6 +31,7 @@ def _run(x, w, dy, s, pad, bias=None, beta=0.0, start=0.0, workspace=True):
     x_, w_, dy_, y, dx = dev(x), dev(w), dev(dy), torch.full(dy.shape, start, device="cuda"), torch.full(x.shape, start, device="cuda")
     b_ = None if bias is None else dev(bias)
     n = int(capi.lib.n2d2hip_conv2d_f32_workspace_bytes(C.byref(d), B, H, W)) if workspace else 0
+    n = max(0, n - (less(n) if callable(less) else less))
     ws = torch.empty(max(n, 16), dtype=torch.uint8, device="cuda")
     p = ws.data_ptr() if n else None
     capi.check(capi.lib.n2d2hip_conv2d_f32_forward(C.byref(d), B, H, W, x_.data_ptr(), w_.data_ptr(), None if b_ is None else b_.data_ptr(), beta, y.data_ptr(), p, n,
@@ -92,6 +93,19 @@ def test_infinities_nan_and_the_largest_floats(case):
         assert np.array_equal(np.isnan(g), np.isnan(t)) and np.array_equal(g == np.inf, t == np.inf) and np.array_equal(g == -np.inf, t == -np.inf)
         ok = np.isfinite(t)
         assert (np.abs(g - f)[ok] <= 2.0 ** -24 * (np.abs(f) + (n + 4) * m)[ok]).all()
+
+
+@pytest.mark.parametrize("case", [(2, 256, 14, 14, 256, 3, 3, 1, 1), (40, 96, 14, 15, 160, 3, 3, 1, 1), (21, 128, 27, 27, 70, 3, 3, 2, 1), (64, 512, 7, 7, 129, 3, 3, 1, 1)])
+def test_workspaces_of_every_size(case):
+    """A workspace that holds the laid-out weights but not the partial results, half of it, and none: all of K, within the bound of a sum that
+    rounds every term."""
+    print("parts, workspaces", case, flush=True)
+    x, w, dy, s, pad, rng = _inputs(case, 2)
+    want, mag = _passes(x, w, dy, s, pad), _passes(np.abs(x), np.abs(w), np.abs(dy), s, pad)
+    T = w.shape[2] * w.shape[3]
+    for less in (16, 4 * dy.size + 16, lambda n: n // 2, lambda n: n):
+        for g, t, m, k in zip(_run(x, w, dy, s, pad, less=less), want, mag, (w.shape[1] * T, w.shape[0] * T)):
+            assert (np.abs(g - t) <= 2.0 ** -24 * (np.abs(t) + (k + 4) * m)).all(), less
 
 
 # B, C, H, W, O, stride, pad y: rows of one octet, of two, three (a step of one each, of two with one left over), four and eight, ends inside an
