@@ -1,4 +1,4 @@
-// Float32 convolution, forward and backward-data at stride 1, on the bf16 matrix cores with every operand in three parts.
+// Float32 convolution, forward, backward-data at stride 1 and of 3x3 kernels at stride 2, on the bf16 matrix cores with every operand in three parts.
 //
 // A float is the sum of three bf16 numbers without a rest (8 + 8 + 8 bits of mantissa, each part the rounded rest of the ones
 // before): a = a0 + a1 + a2.  Of the nine products of a b, a2 b2, a1 b2 and a2 b1 are below 2^-25 of it, less than what a float
@@ -16,6 +16,8 @@
 //   512 -> 512, 3x3, 14 x 14, batch 8           115 / 103     80 /  75
 //   48 -> 96, 5x5, 30 x 30, batch 16             71 /  64     43 /  44
 //   128 -> 256, 3x3 stride 2, 27 x 27, batch 33  53 /         42
+//   256 -> 512, 3x3 stride 2, 28 x 28, batch 8      /  75        /  54      (data: four pixels a place, below)
+//   128 -> 128, 3x3 stride 2, 56 x 56, batch 64     / 152        / 109
 // 64 -> 64 on 56 x 56 is 42 us of matrix instructions at the 2.0 GHz that they leave; what is beside them, in a block's cycles (of
 // 160000, two blocks to a CU): 8 steps of 13700 that are matrix instructions of both blocks, 8 x 1700 that take a step's floats
 // apart, 4 x 9000 for a tile's results and the next one's addresses, 15000 until the first step is there; and 6.1 tiles to a CU take
@@ -88,7 +90,10 @@ struct PatchItem {
 // are consecutive, and so are a channel's images, up to the other channels between them): a step brings 32 channels of that
 // run into LDS, in parts, 16 bytes to 8 channels of a position, and runs through the taps from there; a tap outside the
 // source reads a position that holds zeros.  A block stays for a run of tiles, whose loads go on across their ends.
-template <int WQ, int WP, int MQ, int NP, int PB, int NT, bool FOLD>
+// CL 4: backward-data of a 3x3 kernel at stride 2.  A tile's pixels are places of a grid of half the resolution, and each is the four
+// pixels (2 py, 2 px) ... (2 py + 1, 2 px + 1): every tap belongs to one of them, and all read from 2 x 2 source positions.  Axis by axis, taps 0 and 2
+// go to the pixel c.ry (c.rx) and tap 1 to the other.
+template <int WQ, int WP, int MQ, int NP, int PB, int NT, bool FOLD, int CL = 1>
 __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, const float* __restrict__ srcX, const float* __restrict__ srcW,
                                                                 const v4u* __restrict__ wt, const float* __restrict__ bias, float beta,
                                                                 float* __restrict__ out, size_t partial)
@@ -109,7 +114,13 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
     if (threadIdx.x < 12) *(v4u*)(smem + threadIdx.x * OCT + 64 * PB * 16) = v4u{0, 0, 0, 0};
 
     const PixelClass& c = g.c[0];                // (forward, or backward-data at stride 1)
-    const int nT = NT ? NT : c.nT, nx = NT == 9 ? 3 : c.nx, ny = NT == 9 ? 3 : div_f32(c.nT, c.nxd);
+    static_assert(CL == 1 || (NT == 9 && !FOLD), "3x3 kernels, float sums");
+    const int nT = NT ? NT : c.nT;
+    const int nx = CL == 4 ? 2 : NT == 9 ? 3 : c.nx, ny = CL == 4 ? 2 : NT == 9 ? 3 : div_f32(c.nT, c.nxd);      // source positions of the taps
+    // of tap (i, j): its source row and column, and which of the four pixels it belongs to
+    auto row_of = [&](int i) { return CL == 4 ? (i == 1 ? c.ry : i >> 1) : i; };
+    auto column_of = [&](int j) { return CL == 4 ? (j == 1 ? c.rx : j >> 1) : j; };
+    auto class_of = [](int i, int j) { return CL == 4 ? 2 * (i == 1) + (j == 1) : 0; };
     const int reach = (ny - 1) * g.Ws + nx - 1, back = g.d > 0 ? 0 : reach, ahead = reach - back;
     const int cbeg = blockIdx.z * c.kchunk, cend = min(cbeg + c.kchunk, nchunks);
     // a tile's run: source positions of its first pixel's first tap to its last pixel's last one, counted over a channel's images
@@ -149,18 +160,20 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
             for (int p = 0; p < 3; ++p) *(v4u*)(smem + p * PART + wave * OCT + (u * 64 + lane) * 16) = parts[p];
         }
     };
-    v4f acc[MQ][NP];
+    v4f acc[CL][MQ][NP];
     double folded[FOLD ? MQ : 1][NP][4];
     auto each = [&](auto&& f) {
 #pragma unroll
-        for (int m = 0; m < MQ; ++m)
+        for (int k = 0; k < CL; ++k)
 #pragma unroll
-            for (int n = 0; n < NP; ++n)
+            for (int m = 0; m < MQ; ++m)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) f(m, n, r);
+                for (int n = 0; n < NP; ++n)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) f(k, m, n, r);
     };
     auto fold = [&]() {
-        each([&](int m, int n, int r) { folded[m][n][r] += (double)acc[m][n][r]; acc[m][n][r] = 0.0f; });
+        each([&](int k, int m, int n, int r) { folded[m][n][r] += (double)acc[k][m][n][r]; acc[k][m][n][r] = 0.0f; });
     };
     // a wave's weights: consecutive taps of a chunk are a fragment of every 16 rows of q apart
     v4u a[3][MQ][3], b[2][3];
@@ -207,18 +220,19 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
                 xaddr[n] = lo * OCT + __shfl((int)at, n * 16 + l16);
             }
         }
-        each([&](int m, int n, int r) {
-            acc[m][n][r] = 0.0f;
+        each([&](int k, int m, int n, int r) {
+            acc[k][m][n][r] = 0.0f;
             if (FOLD) folded[m][n][r] = 0.0;
         });
         auto pixels = [&](v4u (&x)[3], int n, int i, int j) {
-            const unsigned bit = (1u << j) | (1u << (nx + i));
-            const unsigned at = (mask[n] & bit) == bit ? xaddr[n] + 16 * g.d * (i * g.Ws + j) : zaddr;
+            const int row = row_of(i), column = column_of(j);
+            const unsigned bit = (1u << column) | (1u << (nx + row));
+            const unsigned at = (mask[n] & bit) == bit ? xaddr[n] + 16 * g.d * (row * g.Ws + column) : zaddr;
 #pragma unroll
             for (int p = 0; p < 3; ++p) x[p] = *(const v4u*)(smem + at + p * PART);
         };
         // the products but the largest in a sum of their own: a matrix instruction rounds its sum four times
-        auto products = [&](const v4u (&w)[MQ][3], const v4u (&x)[3], int n) {
+        auto products = [&](const v4u (&w)[MQ][3], const v4u (&x)[3], int n, int k) {
             v4f small[MQ];
 #pragma unroll
             for (int m = 0; m < MQ; ++m) small[m] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
@@ -231,11 +245,11 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
             }
 #pragma unroll
             for (int m = 0; m < MQ; ++m)
-                acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, w[m][0]), __builtin_bit_cast(v8bf, x[0]), acc[m][n], 0, 0, 0);
+                acc[k][m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, w[m][0]), __builtin_bit_cast(v8bf, x[0]), acc[k][m][n], 0, 0, 0);
 #pragma unroll
             for (int m = 0; m < MQ; ++m)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) acc[m][n][r] += small[m][r];
+                for (int r = 0; r < 4; ++r) acc[k][m][n][r] += small[m][r];
         };
         // a tap's products, 16 pixels at a time, the next 16 (of tap (i1, j1) after the last) on their way from LDS
         auto tap = [&](const v4u (&w)[MQ][3], int i, int j, int i1, int j1, bool last) {
@@ -244,7 +258,7 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
                 if (n + 1 < NP) pixels(b[(n + 1) & 1], n + 1, i, j);
                 else if (!last) pixels(b[(n + 1) & 1], 0, i1, j1);
                 __builtin_amdgcn_sched_barrier(0);
-                products(w, b[n & 1], n);
+                products(w, b[n & 1], n, class_of(i, j));
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
@@ -258,7 +272,7 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
             if constexpr (NT == 9) {
                 if (live) {
                     pixels(b[0], 0, 0, 0);
-                    for (int i = 0; i < 3; ++i)
+                    auto row = [&](int i) {
 #pragma unroll
                         for (int j = 0; j < 3; ++j) {
                             if (i == 0) load_part(lchunk, j * LOADS / 3, (j + 1) * LOADS / 3);
@@ -266,6 +280,14 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
                             weights(a[(j + 2) % 3], on ? lqtile : it.qtile, on ? lchunk : chunk, on ? j - 1 : 3 * i + j + 2);
                             tap(a[j], i, j, j == 2 ? i + 1 : i, (j + 1) % 3, i == 2 && j == 2);
                         }
+                    };
+                    if constexpr (CL == 4) {     // (which sums a row's taps go to is in the code)
+                        row(0);
+                        row(1);
+                        row(2);
+                    } else {
+                        for (int i = 0; i < 3; ++i) row(i);
+                    }
                 } else {
                     load_part(lchunk, 0, LOADS);
                     if (next_tile) first_weights(to.qtile);
@@ -300,27 +322,42 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
         }
         if (FOLD) {
             fold();
-            each([&](int m, int n, int r) { acc[m][n][r] = (float)folded[m][n][r]; });
+            each([&](int k, int m, int n, int r) { acc[k][m][n][r] = (float)folded[m][n][r]; });
         }
         // A lane holds pixel .. + lane % 16 and rows qn + 16 m + r.
         if (live) {
             const size_t zoff = (size_t)blockIdx.z * partial;
-            unsigned obase[NP];                  // of the pixels, in `out`
+            unsigned obase[NP];                  // of the pixels, in `out`; CL 4: of (2 py, 2 px), and whether row 2 py + 1 and column 2 px + 1 are there
             const int p = p0 + wp * NP * 16 + lane, pp = min(p, c.P - 1), img = div_f32(pp, c.ghw);
-            const unsigned o = p < c.P ? 4u * (unsigned)(img * (g.Q - 1) * g.planeO + pp) : F32_OOB;
+            unsigned o;
+            if constexpr (CL == 4) {
+                const int rem = pp - img * c.gHW, py = div_f32(rem, c.gw), px = rem - py * c.gW;
+                o = 4u * (unsigned)(img * g.Q * g.planeO + 2 * py * g.Wo + 2 * px) | (2 * px + 1 < g.Wo ? 2u : 0u)
+                    | ((2 * py + 1) * g.Wo < g.planeO ? 1u : 0u);
+            } else {
+                o = 4u * (unsigned)(img * (g.Q - 1) * g.planeO + pp);
+            }
+            if (p >= c.P) o = F32_OOB;
 #pragma unroll
             for (int n = 0; n < NP; ++n) obase[n] = __shfl((int)o, n * 16 + l16);
+            auto place = [&](int k, int n) {     // of one of a place's pixels; F32_OOB: there is none
+                if (CL == 1 || obase[n] == F32_OOB) return obase[n];
+                const unsigned ry = k & 2 ? 1 - c.ry : c.ry, rx = k & 1 ? 1 - c.rx : c.rx, needs = ry | rx << 1;
+                return (obase[n] & needs) == needs ? (obase[n] & ~3u) + 4u * (ry * g.Wo + rx) : F32_OOB;
+            };
             const __amdgpu_buffer_rsrc_t rsrcO = __builtin_amdgcn_make_buffer_rsrc(out + zoff, 0, g.bytesO, 0x00020000);
             const int planeO4 = 4 * g.planeO;
             const unsigned qrow = qn * planeO4;
             float finite = 0.0f;
-            each([&](int m, int n, int r) { finite = __builtin_fmaf(acc[m][n][r], 0.0f, finite); });
+            each([&](int k, int m, int n, int r) { finite = __builtin_fmaf(acc[k][m][n][r], 0.0f, finite); });
             const bool plain = partial != 0 || (beta == 0.0f && !bias);
             if (plain) {
-                each([&](int m, int n, int r) {
+                unsigned at = F32_OOB;
+                each([&](int k, int m, int n, int r) {
                     if (q0 + wq * MQ * 16 + 16 * m + r >= g.Q) return;
-                    const float s = acc[m][n][r];        // (the cast of a vector's element reads its first one)
-                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, s), rsrcO, qn + 16 * m + r < g.Q ? obase[n] + qrow : F32_OOB,
+                    if (CL == 1 || r == 0) at = place(k, n);
+                    const float s = acc[k][m][n][r];     // (the cast of a vector's element reads its first one)
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, s), rsrcO, qn + 16 * m + r < g.Q && at != F32_OOB ? at + qrow : F32_OOB,
                                                           (16 * m + r) * planeO4, 0);
                 });
             }
@@ -328,40 +365,44 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
                 // Infinities, and what rounds to one in bf16, leave NaN where float products might not: such sums are added again,
                 // in float.
 #pragma unroll
-                for (int n = 0; n < NP; ++n) {
-                    if (obase[n] == F32_OOB) continue;
-                    unsigned redo = 0;
-                    auto store = [&](int m, int r, float s) {
-                        float* at = out + zoff + obase[n] / 4u + (size_t)(qn + 16 * m + r) * g.planeO;
-                        if (partial == 0) {
-                            if (beta != 0.0f) s += beta * *at;
-                            if (bias) s = bias[qn + 16 * m + r] + s;
-                        }
-                        *at = s;
-                    };
+                for (int k = 0; k < CL; ++k)
 #pragma unroll
-                    for (int m = 0; m < MQ; ++m)
+                    for (int n = 0; n < NP; ++n) {
+                        const unsigned base = place(k, n);
+                        if (base == F32_OOB) continue;
+                        unsigned redo = 0;
+                        auto store = [&](int m, int r, float s) {
+                            float* at = out + zoff + base / 4u + (size_t)(qn + 16 * m + r) * g.planeO;
+                            if (partial == 0) {
+                                if (beta != 0.0f) s += beta * *at;
+                                if (bias) s = bias[qn + 16 * m + r] + s;
+                            }
+                            *at = s;
+                        };
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            if (qn + 16 * m + r >= g.Q) continue;
-                            if (!(__builtin_fabsf(acc[m][n][r]) < __builtin_inff())) redo |= 1u << (4 * m + r);
-                            else if (!plain) store(m, r, acc[m][n][r]);
+                        for (int m = 0; m < MQ; ++m)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) {
+                                if (qn + 16 * m + r >= g.Q) continue;
+                                if (!(__builtin_fabsf(acc[k][m][n][r]) < __builtin_inff())) redo |= 1u << (4 * m + r);
+                                else if (!plain) store(m, r, acc[k][m][n][r]);
+                            }
+                        const int p = p0 + (wp * NP + n) * 16 + l16, img = div_f32(p, c.ghw), rem = p - img * c.gHW, py = div_f32(rem, c.gw), px = rem - py * c.gW;
+                        const int rows = CL == 4 ? 3 : ny, columns = CL == 4 ? 3 : nx;
+                        for (; redo; redo &= redo - 1) {
+                            const int at = __builtin_ctz(redo), q = qn + 16 * (at >> 2) + (at & 3);
+                            float s = 0.0f;
+                            for (int ch = cbeg * PK; ch < min(cend * PK, g.Ch); ++ch)
+                                for (int i = 0; i < rows; ++i)
+                                    for (int j = 0; j < columns; ++j) {
+                                        const int y = py * g.sy + c.y0 + g.d * row_of(i), x = px * g.sx + c.x0 + g.d * column_of(j);
+                                        if (y < 0 || y >= g.Hs || x < 0 || x >= g.Ws || class_of(i, j) != k) continue;
+                                        s += srcW[(size_t)q * g.qs + (size_t)ch * g.chs + i * columns + j]
+                                             * srcX[((size_t)img * g.Ch + ch) * g.planeS + y * g.Ws + x];
+                                    }
+                            store(at >> 2, at & 3, s);
                         }
-                    const int p = p0 + (wp * NP + n) * 16 + l16, img = div_f32(p, c.ghw), rem = p - img * c.gHW, py = div_f32(rem, c.gw), px = rem - py * c.gW;
-                    for (; redo; redo &= redo - 1) {
-                        const int at = __builtin_ctz(redo), q = qn + 16 * (at >> 2) + (at & 3);
-                        float s = 0.0f;
-                        for (int ch = cbeg * PK; ch < min(cend * PK, g.Ch); ++ch)
-                            for (int i = 0; i < ny; ++i)
-                                for (int j = 0; j < nx; ++j) {
-                                    const int y = py * g.sy + c.y0 + g.d * i, x = px * g.sx + c.x0 + g.d * j;
-                                    if (y < 0 || y >= g.Hs || x < 0 || x >= g.Ws) continue;
-                                    s += srcW[(size_t)q * g.qs + (size_t)ch * g.chs + i * nx + j]
-                                         * srcX[((size_t)img * g.Ch + ch) * g.planeS + y * g.Ws + x];
-                                }
-                        store(at >> 2, at & 3, s);
                     }
-                }
             }
         }
         if (!again) return;

@@ -1282,7 +1282,20 @@ static int patch_fold(const ConvF32& q, int pass, const PixelClass& c)
     const bool fwd = pass == PASS_FWD;
     const long K = (long)(fwd ? q.C : q.O) * q.kH * q.kW;
     const long ranges = pass_ranges((long)q.B * (fwd ? q.oH * q.oW : q.H * q.W), fwd ? q.O : q.C, K);
-    return (int)std::max(4 * (K / ranges) / (PK * c.nT), 1L);
+    const long T = fwd ? (long)c.nT : (long)ceil_div_i(q.kH, q.sy) * ceil_div_i(q.kW, q.sx);     // taps of the longest sum
+    return (int)std::max(4 * (K / ranges) / (PK * T), 1L);
+}
+// Backward-data of a 3x3 kernel at stride 2 as one class whose every place is four pixels
+static bool patch_fours(const ConvF32& q, int pass) { return pass == PASS_BWD_DATA && q.kH == 3 && q.kW == 3 && q.sx == 2 && q.sy == 2; }
+static PixelClass fours_class(const ConvF32& q)
+{
+    PixelClass c = {};
+    c.gW = (q.W + 1) / 2; c.gHW = (q.H + 1) / 2 * c.gW; c.P = q.B * c.gHW;
+    c.nx = 3; c.nT = 9;
+    c.ry = q.pt & 1; c.rx = q.pl & 1;            // the pixel of taps 0 and 2
+    c.y0 = (c.ry + q.pt) / 2; c.x0 = (c.rx + q.pl) / 2;
+    c.ghw = div_of(c.gHW); c.gw = div_of(c.gW); c.nt = div_of(c.nT); c.nxd = div_of(c.nx);
+    return c;
 }
 // Tiles of 64 rows x 128 pixels where they fill three quarters of the chip's two blocks to a CU and need no sums in double (whose
 // registers they lack); else of 64 x 64.  us, 64 x 128 / 64 x 64, forward: 64 -> 64, 56 x 56, batch 64 (1568 of the larger tiles)
@@ -1296,6 +1309,20 @@ static PatchShape patch_shape(const ConvF32& q, int pass, const PixelClass& c)
         s.nu = c.nx + c.nT / c.nx > 31 ? 0 : patch_units(q, pass, c, s.pixels());
         return s;
     };
+    if (patch_fours(q, pass)) {
+        // No sums in double (the float ones take the registers).  Where the tiles give every CU a block, or are so few that the chunk
+        // kernel's longest class leaves most of the chip idle; between, partial results of two ranges cost more than it saves.
+        // us, chunk kernel / this: 64 <- 64, 56 x 56, batch 128 (1568 tiles) 98 / 74; 256 <- 512, 14 x 14, batch 128 (392) 145 / 106; 64 <- 128,
+        // 32 x 32, batch 64 (256) 34.4 / 29.1; 128 <- 256, 27 x 27, batch 33 (202) 52.3 / 54.7; 64 <- 128, 56 x 56, batch 16 (196) 32.5 / 47.7; 320 <- 384,
+        // 13 x 13, batch 33 (130 of 12 chunks) 62 / 54; 128 <- 256, 16 x 16, batch 64 (128 of 8) 42.5 / 43.1; 256 <- 512, 28 x 28, batch 8 (100 of
+        // 16) 75 / 54; half of a tile padding: 40 <- 48, 48 x 48, batch 64 33.3 / 34.1.
+        PatchShape s = fit(PatchShape{2, 2, 2, 2, 0});
+        const long tiles = (long)ceil_div_i(c.P, 64) * ceil_div_i(Q, 64);
+        if (s.nu > 2 || Q <= 32 || patch_fold(q, pass, c) < chunks || (tiles < 256 && !(tiles <= 160 && chunks >= 12))
+            || 2L * Q * q.O < (long)ceil_div_i(Q, 64) * 64 * chunks * PK)
+            s.nu = 0;
+        return s;
+    }
     if (Q <= 32) return fit(PatchShape{1, 4, 2, 2, 0});
     if (patch_fold(q, pass, c) >= chunks && (long)ceil_div_i(c.P, 128) * ceil_div_i(Q, 64) >= 384) {
         const PatchShape s = fit(PatchShape{2, 2, 2, 4, 0});
@@ -1416,7 +1443,13 @@ static void launch_pixels(PixelPlan& pl, int splits, const float* x, const float
 {
     const dim3 grid(pl.g.ptiles8 * 8 * pl.g.qtiles, 1, splits);
     if (pl.kind == PIXELS_PATCH) {
-        if (pl.patch.wq == 1) launch_patch<1, 4, 2, 2, true>(pl, grid, x, w, wt, bias, beta, out, partial, st);
+        if (BWD && pl.g.osx == 2) {
+            const dim3 most(std::min(grid.x, 8u * 32u * 2u), 1, grid.z);
+            if (pl.patch.nu == 1)
+                N2D2HIP_LAUNCH_T(conv_f32_patch_kernel, (2, 2, 2, 2, 2, 9, false, 4), most, dim3(256), 0, st, pl.g, x, w, (const v4u*)wt, bias, beta, out, partial);
+            else
+                N2D2HIP_LAUNCH_T(conv_f32_patch_kernel, (2, 2, 2, 2, 4, 9, false, 4), most, dim3(256), 0, st, pl.g, x, w, (const v4u*)wt, bias, beta, out, partial);
+        } else if (pl.patch.wq == 1) launch_patch<1, 4, 2, 2, true>(pl, grid, x, w, wt, bias, beta, out, partial, st);
         else if (pl.patch.np == 2) launch_patch<2, 2, 2, 2, true>(pl, grid, x, w, wt, bias, beta, out, partial, st);
         else launch_patch<2, 2, 2, 4, false>(pl, grid, x, w, wt, bias, beta, out, partial, st);
         return;
@@ -1597,12 +1630,18 @@ static int pixels_kind(const ConvF32& q, int pass)
     if (2.0 * q.B * q.O * q.oH * q.oW * q.C * T < 5.0e8 || (size_t)(q.O + 64) * (q.C + 64) * (T + 2) >= ((size_t)1 << 28))
         return PIXELS_TAPS;
     if (T > 1 && round_up(ch, PK) * 5 <= ch * 7 && !(pass == PASS_FWD && (q.choice & N2D2HIP_KERNEL_F32_TERMS))) {
-        // (backward-data at strides: the classes are few taps to a step each; 128 <- 256, stride 2, 27 x 27, batch 33: 58 us against 53)
-        if ((pass == PASS_FWD || (q.sx == 1 && q.sy == 1)) && patch_shape(q, pass, pixel_classes(q, pass)[0]).nu) return PIXELS_PATCH;
+        // (backward-data at other strides and kernels: the classes are few taps to a step each; 128 <- 256, stride 2, 27 x 27, batch 33, a class a
+        // launch: 58 us against 53)
+        if (patch_fours(q, pass) ? patch_shape(q, pass, fours_class(q)).nu
+            : (pass == PASS_FWD || (q.sx == 1 && q.sy == 1)) && patch_shape(q, pass, pixel_classes(q, pass)[0]).nu) return PIXELS_PATCH;
     }
     if (q.kH == 3 && q.kW == 3 && (pass == PASS_FWD || (q.sx == 1 && q.sy == 1)) && round_up(ch, 4) * 5 <= ch * 7)
         return PIXELS_3X3;
     return (pass == PASS_BWD_DATA || T == 1 || q.kH + q.kW > 31) && round_up(ch, GK) * 5 <= ch * 6 ? PIXELS_CHUNK : PIXELS_TAPS;
+}
+static std::vector<PixelClass> launch_classes(const ConvF32& q, int pass, int kind)
+{
+    return kind == PIXELS_PATCH && patch_fours(q, pass) ? std::vector<PixelClass>{fours_class(q)} : pixel_classes(q, pass);
 }
 static size_t laid_weights(const ConvF32& q, int pass, int kind)
 {
@@ -1622,7 +1661,7 @@ static size_t pass_workspace(const ConvF32& q, int pass)
         return (size_t)pl.splits * pl.g.Q * pl.g.P;
     }
     const int kind = pixels_kind(q, pass);
-    const std::vector<PixelClass> cls = pixel_classes(q, pass);
+    const std::vector<PixelClass> cls = launch_classes(q, pass, kind);
     const size_t n = (size_t)q.B * (pass == PASS_FWD ? (size_t)q.O * q.oH * q.oW : (size_t)q.C * q.H * q.W);
     int splits = 1;
     for (size_t i = 0; i < cls.size(); i += PIXEL_CLASSES)
@@ -1664,7 +1703,7 @@ static int run_pass(const ConvF32& q, int pass, const float* a, const float* b, 
     int kind = pixels_kind(q, pass);
     const size_t nlaid = laid_weights(q, pass, kind);
     if (nlaid > ws_floats || ((size_t)ws & 15)) kind = PIXELS_TAPS;
-    const std::vector<PixelClass> cls = pixel_classes(q, pass);
+    const std::vector<PixelClass> cls = launch_classes(q, pass, kind);
     std::vector<PixelPlan> plans;
     int splits = 1;
     for (size_t i = 0; i < cls.size(); i += PIXEL_CLASSES) {

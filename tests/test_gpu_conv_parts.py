@@ -108,6 +108,28 @@ def test_workspaces_of_every_size(case):
             assert (np.abs(g - t) <= 2.0 ** -24 * (np.abs(t) + (k + 4) * m)).all(), less
 
 
+# Data gradients at stride 2 whose four pixels a place run together: odd and even sizes, rows, channels and pixels left over, 0 to 2 of padding, K
+# ranges, runs of one unit and of two, each beside a neighbour that does not qualify (tiles between the limits, long sums, a step back, few rows)
+FOURS = [((64, 64, 32, 32, 128, 3, 3, 2, 1), 2), ((66, 100, 31, 33, 70, 3, 3, 2, 1), 2), ((12, 70, 31, 30, 390, 3, 3, 2, 1), 2), ((70, 64, 32, 32, 64, 3, 3, 2, 1), 2),
+         ((10, 128, 40, 41, 400, 3, 3, 2, 2), 4), ((3, 100, 57, 100, 385, 3, 3, 2, 1), 4), ((3, 64, 16, 200, 512, 3, 3, 2, 1), 0),
+         ((33, 128, 27, 27, 256, 3, 3, 2, 1), 0), ((9, 70, 29, 30, 390, 3, 3, 2, 1), 0), ((70, 64, 33, 33, 64, 3, 3, 2, 0), 0), ((128, 32, 32, 32, 128, 3, 3, 2, 1), 0), ((64, 36, 48, 48, 48, 3, 3, 2, 1), 0)]
+
+
+@pytest.mark.parametrize("case,units", FOURS, ids=str)
+def test_strided_data_gradient_of_four_pixels_a_place(case, units):
+    from n2d2_amd import capi
+    with capi.launch_log() as log:
+        test_against_float64(case)
+        test_workspaces_of_every_size(case)
+    kernels = {e[0] for e in log.entries if e[0].endswith("4>") and e[0].startswith("conv_f32_patch_kernel")}
+    assert kernels == ({"conv_f32_patch_kernel<2, 2, 2, 2, %d, 9, false, 4>" % units} if units else set())
+
+
+@pytest.mark.parametrize("case", [(66, 100, 31, 33, 70, 3, 3, 2, 1), (10, 128, 40, 41, 400, 3, 3, 2, 2)])
+def test_strided_data_gradient_infinities_nan_and_the_largest_floats(case):
+    test_infinities_nan_and_the_largest_floats(case)
+
+
 # B, C, H, W, O, stride, pad y: rows of one octet, of two, three (a step of one each, of two with one left over), four and eight, ends inside an
 # octet, tiles left over in both directions, no padding and two rows above, images whose last row no output reads
 FILTER = [(260, 64, 7, 7, 128, 1, 1), (70, 64, 13, 15, 100, 1, 1), (44, 70, 19, 24, 64, 1, 1), (33, 64, 31, 30, 64, 1, 1), (11, 32, 40, 57, 120, 1, 0), (6, 64, 64, 64, 64, 1, 2),
