@@ -648,13 +648,13 @@ __device__ __forceinline__ void chain_add_row(float& sum, const v4f& p)
                  N2D2HIP_CHAIN_LANE(5) N2D2HIP_CHAIN_LANE(6) N2D2HIP_CHAIN_LANE(7) N2D2HIP_CHAIN_LANE(8) N2D2HIP_CHAIN_LANE(9)
                  N2D2HIP_CHAIN_LANE(10) N2D2HIP_CHAIN_LANE(11) N2D2HIP_CHAIN_LANE(12) N2D2HIP_CHAIN_LANE(13) N2D2HIP_CHAIN_LANE(14)
                  N2D2HIP_CHAIN_LANE(15)
-                 : "+v"(sum) : "v"(p0), "v"(p1), "v"(p2), "v"(p3));
+                 : "+&v"(sum) : "v"(p0), "v"(p1), "v"(p2), "v"(p3));
 }
 // The first `lanes` lanes' products
 __device__ __forceinline__ void chain_add_lanes(float& sum, const v4f& p, int lanes)
 {
     const float p0 = p[0], p1 = p[1], p2 = p[2], p3 = p[3];
-#define N2D2HIP_CHAIN_ONE(I) if (lanes > I) asm volatile("s_nop 1\n\t" N2D2HIP_CHAIN_LANE(I) : "+v"(sum) : "v"(p0), "v"(p1), "v"(p2), "v"(p3))
+#define N2D2HIP_CHAIN_ONE(I) if (lanes > I) asm volatile("s_nop 1\n\t" N2D2HIP_CHAIN_LANE(I) : "+&v"(sum) : "v"(p0), "v"(p1), "v"(p2), "v"(p3))
     N2D2HIP_CHAIN_ONE(0); N2D2HIP_CHAIN_ONE(1); N2D2HIP_CHAIN_ONE(2); N2D2HIP_CHAIN_ONE(3); N2D2HIP_CHAIN_ONE(4);
     N2D2HIP_CHAIN_ONE(5); N2D2HIP_CHAIN_ONE(6); N2D2HIP_CHAIN_ONE(7); N2D2HIP_CHAIN_ONE(8); N2D2HIP_CHAIN_ONE(9);
     N2D2HIP_CHAIN_ONE(10); N2D2HIP_CHAIN_ONE(11); N2D2HIP_CHAIN_ONE(12); N2D2HIP_CHAIN_ONE(13); N2D2HIP_CHAIN_ONE(14);
