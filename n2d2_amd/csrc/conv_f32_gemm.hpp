@@ -1312,11 +1312,13 @@ __device__ __forceinline__ void data_small_tile(const DataSmall& g, int tp, int 
     const size_t idx = ((size_t)oi * g.C + oc) * g.HW + (op - oi * g.HW);
     dx[idx] = (float)v + (beta != 0.0f ? beta * dx[idx] : 0.0f);
 }
+// (dtiles: of 16 pixels.  The tiles of both directions are in the grid's first: channels alone can be more than 16 x 65535)
 template <int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void conv_f32_data_small_kernel(DataSmall g, const float* __restrict__ w, const float* __restrict__ dy, float beta,
-                                                                         float* __restrict__ dx)
+__global__ __launch_bounds__(64 * WAVES) void conv_f32_data_small_kernel(DataSmall g, int dtiles, const float* __restrict__ w, const float* __restrict__ dy,
+                                                                         float beta, float* __restrict__ dx)
 {
-    data_small_tile<WAVES>(g, blockIdx.x, blockIdx.y, w, dy, beta, dx);
+    const int tc = blockIdx.x / dtiles;
+    data_small_tile<WAVES>(g, blockIdx.x - tc * dtiles, tc, w, dy, beta, dx);
 }
 // Both gradients of a small layer in one launch, the blocks of the data first, which take longer, then those of the weights, whose ranges
 // are added by the launch that follows.  us, two launches / one, with the one that adds: 6 <- 16, 5x5, 14 x 14, batch 32 15.5 / 12.4; 64 <- 64,

@@ -1795,9 +1795,10 @@ int n2d2hip_conv2d_f32_backward_data(const n2d2hip_conv_desc* desc, int B, int H
         return run_small_filter(small_gemm(q, PASS_BWD_DATA), w, diff_y, beta, diff_x, (double*)workspace, workspace ? workspace_bytes : 0, (hipStream_t)stream);
     if (path == F32_PATH_SMALL_DATA) {
         const DataSmall g = small_data(q);
-        const dim3 grid(ceil_div_i(g.P, 16), ceil_div_i(g.C, 16));
-        if (g.K <= 256) hipLaunchKernelGGL(conv_f32_data_small_kernel<4>, grid, dim3(256), 0, (hipStream_t)stream, g, w, diff_y, beta, diff_x);
-        else hipLaunchKernelGGL(conv_f32_data_small_kernel<8>, grid, dim3(512), 0, (hipStream_t)stream, g, w, diff_y, beta, diff_x);
+        const int dtiles = ceil_div_i(g.P, 16);
+        const dim3 grid(dtiles * ceil_div_i(g.C, 16));       // (2.3e5 / K at most)
+        if (g.K <= 256) N2D2HIP_LAUNCH_T(conv_f32_data_small_kernel, (4), grid, dim3(256), 0, (hipStream_t)stream, g, dtiles, w, diff_y, beta, diff_x);
+        else N2D2HIP_LAUNCH_T(conv_f32_data_small_kernel, (8), grid, dim3(512), 0, (hipStream_t)stream, g, dtiles, w, diff_y, beta, diff_x);
         N2D2HIP_HIP_CHECK(hipGetLastError());
         return N2D2HIP_OK;
     }

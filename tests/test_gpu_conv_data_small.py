@@ -44,3 +44,29 @@ def test_adds_in_double(case, beta):
         want = want + 0.5 * start
         bound = bound + 2.0 ** -24 * (np.abs(want) + bound) + 2.0 ** -25 * np.abs(start)
     assert (np.abs(got - want) <= bound).all()
+
+
+@pytest.mark.parametrize("joint", [False, True])
+def test_more_channel_tiles_than_a_grids_second_dimension(joint):
+    """One output, 1x1: a gradient is one product.  65537 tiles of channels and the rest of one, two pixels."""
+    import torch
+    from n2d2_amd import capi, runtime as rt
+    Ci = 16 * 65535 + 17
+    print("small data gradient, channels", Ci, joint, flush=True)
+    rng = np.random.default_rng(7)
+    d = capi.ConvDesc(Ci, 1, 1, 1, 1, 1, 0, 0, 0, 0, 1, 1, 1, 0, 0)
+    dev = lambda *n: torch.from_numpy(rng.normal(size=n).astype(np.float32)).cuda()
+    x, w, dy = dev(1, Ci, 1, 2), dev(1, Ci, 1, 1), dev(1, 1, 1, 2)
+    dw, dx = torch.full_like(w, np.nan), torch.full_like(x, np.nan)
+    with capi.launch_log() as log:
+        if joint:
+            capi.check(capi.lib.n2d2hip_conv2d_f32_backward(C.byref(d), 1, 1, 2, x.data_ptr(), w.data_ptr(), dy.data_ptr(), 0.0, dw.data_ptr(), 0.0, dx.data_ptr(),
+                                                            None, 0, rt.stream_ptr()))
+        else:
+            capi.check(capi.lib.n2d2hip_conv2d_f32_backward_data(C.byref(d), 1, 1, 2, w.data_ptr(), dy.data_ptr(), 0.0, dx.data_ptr(), None, 0, rt.stream_ptr()))
+    torch.cuda.synchronize()
+    assert any("small" in e[0] for e in log.entries)
+    assert torch.equal(dx, w.reshape(1, Ci, 1, 1) * dy)
+    if joint:
+        want = (x.double() * dy.double()).sum(dim=3).reshape(w.shape)
+        assert bool(((dw.double() - want).abs() <= 2.0 ** -24 * want.abs()).all())
