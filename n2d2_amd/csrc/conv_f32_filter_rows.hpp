@@ -229,7 +229,7 @@ __global__ __launch_bounds__(512, 2) void conv_f32_filter_rows_kernel(FilterRows
 #pragma unroll
     for (int t = 0; t < 9; ++t) {
         // (the sums of the first half first, in both)
-        const v4f other = *(const v4f*)(red + (((1 - half) * 9 + t) * 256 + tid) * 4), sum = half ? other + acc[t][1] : acc[t][0] + other;
+        const v4f other = *(const v4f*)(red + (((1 - half) * 9 + t) * 256 + tid) * 4), sum = (half ? other + acc[t][1] : acc[t][0] + other) * PARTS_UNSCALE;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             finite = __builtin_fmaf(sum[r], 0.0f, finite);

@@ -1,8 +1,8 @@
 // Float32 convolution, forward, backward-data at stride 1 and of 3x3 kernels at stride 2, on the bf16 matrix cores with every operand in three parts.
 //
 // A float is the sum of three bf16 numbers without a rest (8 + 8 + 8 bits of mantissa, each part the rounded rest of the ones
-// before): a = a0 + a1 + a2.  Of the nine products of a b, a2 b2, a1 b2 and a2 b1 are below 2^-25 of it, less than what a float
-// addition rounds off; the other six are matrix instructions.  Random data, two waves to a SIMD, register operands only: 16x16x32
+// before; scaled, so that the parts of small floats keep their bits): a = a0 + a1 + a2.  Of the nine products of a b, a1 b2 and a2 b1 are
+// below 2^-25 of it and a2 b2 below 2^-34: left out, all three are 2^-24.4 of a b at most.  The other six are matrix instructions.  Random data, two waves to a SIMD, register operands only: 16x16x32
 // bf16 2040 TFLOP/s, 340 of six products; 32x32x16 bf16 1350 (two waves in turn slow it down; one alone has 1800); 32x32x2 fp32 98.
 // An instruction adds its 32 products to the sum in four roundings: the five smaller products have a sum of their own, which one
 // addition brings to that of the largest, so that a sum is rounded 5 times in 32 terms where the fp32 instructions round it 32
@@ -33,6 +33,11 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
+// What operands are multiplied by before they are taken apart, and sums afterwards: a bf16 has no bits below 2^-133, which is 2^-149, a
+// float's last, 2^16 larger.  Error of sums of 32 products, one operand of size 2^-112 / 2^-116 / 2^-120 / 2^-124, without: 1.4e-7 / 2.2e-6 /
+// 3.5e-5 / 5.7e-4, with: as of size 1.
+constexpr float PARTS_SCALE = 0x1p16f, PARTS_UNSCALE = 0x1p-32f;
+
 // (a, b) -> their first parts, packed; a and b become the rests
 __device__ __forceinline__ unsigned bf16_part(float& a, float& b)
 {
@@ -45,7 +50,7 @@ __device__ __forceinline__ void bf16_parts(float (&v)[8], v4u (&parts)[3])
 {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        float a = v[2 * j], b = v[2 * j + 1];
+        float a = v[2 * j] * PARTS_SCALE, b = v[2 * j + 1] * PARTS_SCALE;
         parts[0][j] = bf16_part(a, b);
         parts[1][j] = bf16_part(a, b);
         parts[2][j] = __builtin_bit_cast(unsigned, __builtin_convertvector(v2f{a, b}, v2bf));
@@ -320,10 +325,11 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
             __syncthreads();
             if (more || next_tile) put();
         }
-        if (FOLD) {
-            fold();
-            each([&](int k, int m, int n, int r) { acc[k][m][n][r] = (float)folded[m][n][r]; });
-        }
+        if (FOLD) fold();
+        each([&](int k, int m, int n, int r) {
+            if constexpr (FOLD) acc[k][m][n][r] = (float)(folded[m][n][r] * (double)PARTS_UNSCALE);
+            else acc[k][m][n][r] *= PARTS_UNSCALE;
+        });
         // A lane holds pixel .. + lane % 16 and rows qn + 16 m + r.
         if (live) {
             const size_t zoff = (size_t)blockIdx.z * partial;

@@ -200,3 +200,22 @@ def test_filter_gradient_infinities_nan_and_the_largest_floats():
     fin = np.where(np.isfinite(x), x, 0)
     mag = _filter64(np.abs(fin), np.abs(dy), s, pt)
     assert (np.abs(got - _filter64(fin, dy, s, pt))[ok] <= 2.0 ** -24 * ((5 * B * 196 / 32 + 4) * mag)[ok]).all()
+
+
+@pytest.mark.parametrize("small", [2.0 ** -112, 2.0 ** -118, 2.0 ** -126])
+def test_small_floats_keep_their_bits(small):
+    """One operand of a size whose parts would lie below the smallest bf16, against the other of size 1, and of 2^100: the bound of
+    values of size 1, and half a step of the results where they are below the normal floats."""
+    case = (33, 64, 32, 32, 64, 3, 3, 1, 1)
+    print("parts, small floats", small, flush=True)
+    x, w, dy, s, pad, rng = _inputs(case, 3)
+    small = np.float32(small)
+    for of_x, of_w in ((small, 1), (1, small), (small, np.float32(2.0 ** 100)), (np.float32(2.0 ** 100), small)):
+        a, b, d = x * of_x, w * of_w, dy * of_x
+        for g, t, k in zip(_run(a, b, d, s, pad), _passes(a, b, d, s, pad), (64 * 9, 64 * 9)):
+            assert np.linalg.norm(g - t) <= 1.1 * 2.53e-8 * np.sqrt(1 + k / 2) * np.linalg.norm(t) + 2.0 ** -150 * np.sqrt(t.size)
+    K = dy.size // 64
+    for of_x, of_dy in ((small, 1), (1, small), (small, np.float32(2.0 ** 100)), (np.float32(2.0 ** 100), small)):
+        a, d = x * of_x, dy * of_dy
+        got, want = _filter(a, w.shape, d, 1, 1), _filter64(a, d, 1, 1)
+        assert np.linalg.norm(got - want) <= 1.1 * 2.53e-8 * np.sqrt(1 + 5 * K / 64) * np.linalg.norm(want) + 2.0 ** -150 * np.sqrt(want.size)
