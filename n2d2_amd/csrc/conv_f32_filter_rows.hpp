@@ -226,41 +226,65 @@ __global__ __launch_bounds__(512, 2) void conv_f32_filter_rows_kernel(FilterRows
     __syncthreads();
     float* const out = partial + ((size_t)blockIdx.z * gridDim.y * gridDim.x + blockIdx.y * gridDim.x + blockIdx.x) * ROWS_TILE;
     float finite = 0.0f;
+    v4f sum[9];
 #pragma unroll
     for (int t = 0; t < 9; ++t) {
         // (the sums of the first half first, in both)
-        const v4f other = *(const v4f*)(red + (((1 - half) * 9 + t) * 256 + tid) * 4), sum = (half ? other + acc[t][1] : acc[t][0] + other) * PARTS_UNSCALE;
+        const v4f other = *(const v4f*)(red + (((1 - half) * 9 + t) * 256 + tid) * 4);
+        sum[t] = (half ? other + acc[t][1] : acc[t][0] + other) * PARTS_UNSCALE;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            finite = __builtin_fmaf(sum[r], 0.0f, finite);
-            out[((t * 2 + half) * 4 + r) * 256 + tid] = sum[r];
-        }
+        for (int r = 0; r < 4; ++r) finite = __builtin_fmaf(sum[t][r], 0.0f, finite);
     }
-    if (!__any(finite != finite)) return;
-    // Infinities, and what rounds to one in bf16, leave NaN where float products might not: such sums are added again, in float.
-    for (int k = 0; k < 72; ++k) {
-        if ((k >> 2 & 1) != half || __builtin_fabsf(out[k * 256 + tid]) < __builtin_inff()) continue;
-        int q, c, tap;
-        rows_place(k, tid, &q, &c, &tap);
-        q += q0;
-        c += c0;
-        if (q >= g.Q || c >= g.C) continue;
-        float s = 0.0f;
+    if (__any(finite != finite)) {
+        // Infinities, and what rounds to one in bf16, leave NaN where float products might not: a wave that holds such sums adds them
+        // again, on the fp32 matrix cores straight from memory, in double from eight pixels to the next.  Where a tap lies outside x
+        // both operands are 0.
+        // us of 64 <- 64, 56 x 56, batch 64: finite 118; NaN throughout 960; a channel of x NaN 704 (a sum after the other by the lane that
+        // held it: 15570, 9030).
+        int here = lane;                         // (opaque: nothing of this is worked out ahead, and held, by waves that never come here)
+        asm volatile("" : "+v"(here));
+        const int l16 = here & 15, lo = here >> 4, q = q0 + wq * 32 + half * 16 + l16, ch = c0 + wc * 16 + l16;
+        double folded[9][4] = {};
+#pragma unroll 1
         for (int chunk = beg; chunk < end; ++chunk) {
-            const int row = chunk / g.pieces, piece = chunk - row * g.pieces;
+            const int row = div_f32(chunk, g.dpieces), piece = chunk - row * g.pieces;
+#pragma unroll 1
             for (int e = 0; e < NE; ++e) {
-                const int v = row * RW + (e >> NOL), img = v / g.D, oy = v - img * g.D, y = oy * S - g.pt + tap / 3;
-                if (img >= g.B || oy >= g.oH || y < 0 || y >= g.H) continue;
-                const int ox0 = 8 * (piece * NO + (e & (NO - 1)));
-                for (int ox = ox0; ox < min(ox0 + 8, g.oW); ++ox) {
-                    const int xx = ox * S - 1 + tap % 3;
-                    if (xx >= 0 && xx < g.W)
-                        s += dy[((size_t)(img * g.Q + q) * g.oH + oy) * g.oW + ox] * x[((size_t)(img * g.C + c) * g.H + y) * g.W + xx];
+                const int v = row * RW + (e >> NOL), img = div_f32(v, g.dD), oy = v - img * g.D;
+                if (img >= g.B || oy >= g.oH) continue;
+                v4f part[9];
+#pragma unroll
+                for (int t = 0; t < 9; ++t) part[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+                for (int h = 0; h < 8; h += 4) {
+                    const int ox = 8 * (piece * NO + (e & (NO - 1))) + h + lo;
+                    const float d = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                        rsrcY, q < g.Q && ox < g.oW ? 4u * (unsigned)(((img * g.Q + q) * g.oH + oy) * g.oW + ox) : F32_OOB, 0, 0));
+#pragma unroll
+                    for (int t = 0; t < 9; ++t) {
+                        const int y = oy * S - g.pt + t / 3, col = ox * S - 1 + t % 3;
+                        const bool there = ox < g.oW && (unsigned)y < (unsigned)g.H && (unsigned)col < (unsigned)g.W;
+                        const float u = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                            rsrcX, there && ch < g.C ? 4u * (unsigned)(((img * g.C + ch) * g.H + y) * g.W + col) : F32_OOB, 0, 0));
+                        part[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(there ? d : 0.0f, u, part[t], 0, 0, 0);
+                    }
                 }
+#pragma unroll
+                for (int t = 0; t < 9; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) folded[t][r] += (double)part[t][r];
             }
         }
-        out[k * 256 + tid] = s;
+#pragma unroll
+        for (int t = 0; t < 9; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (!(__builtin_fabsf(sum[t][r]) < __builtin_inff())) sum[t][r] = (float)folded[t][r];
     }
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[((t * 2 + half) * 4 + r) * 256 + tid] = sum[t][r];
 }
 
 // dw[q][c][tap] = sum over the ranges + beta * dw: 64 values of a tile to a block, each of its four waves a quarter of the ranges, in

@@ -104,7 +104,7 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
                                                                 float* __restrict__ out, size_t partial)
 {
     static_assert(WQ * WP == 4, "four waves, one to 8 channels of a step");
-    static_assert(NP % 2 == 0 && NP <= 4, "a tap's first 16 pixels are in b[0]; a lane for each of a wave's pixels");
+    static_assert(NP == 2 || NP == 4, "a tap's first 16 pixels are in b[0]; a lane for each of a wave's pixels");
     constexpr int QT = 16 * MQ * WQ, PT = 16 * NP * WP;
     constexpr int POS = 64 * PB + 16;            // positions of 8 channels, zeros behind them (16: what lanes of an LDS read share no banks)
     constexpr int OCT = POS * 16, PART = 4 * OCT;
@@ -194,6 +194,106 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
         if (NT == 9) weights(a[1], qtile, cbeg, 1);
     };
     unsigned xaddr[NP], mask[NP];                // of a lane's pixels: where tap (0, 0) is in LDS; the taps that exist
+
+    // Infinities, and what rounds to one in bf16, leave NaN where float products might not.  A wave that holds such sums adds them
+    // again, on the fp32 matrix cores straight from memory, in double from four channels to the next.
+    // us of 64 -> 64, 56 x 56, batch 64, forward / data: finite 96 / 95; NaN throughout 830 / 700; a channel of the input NaN 650 / 520; one weight
+    // NaN 1240 / 1260 (a sum after the other by the lane that held it: 6520 / 6570, 6500 / 6590, 970 / 1500).
+    // (32 pixels of one class at a time: of more the sums would take the registers that hold the next step's operands)
+    auto again_in_float = [&](auto k_, auto n_, int p0, int q0) {
+        constexpr int k = decltype(k_)::value, n0 = decltype(n_)::value;
+        int here = lane;                         // (opaque: nothing of this is worked out ahead, and held, by waves that never come here)
+        const float* weights_ = srcW;
+        asm volatile("" : "+v"(here), "+s"(weights_));
+        const int l16 = here & 15, lo = here >> 4;
+        const int rows = CL == 4 ? 3 : ny, columns = CL == 4 ? 3 : nx, chend = min(cend * PK, g.Ch);
+        const __amdgpu_buffer_rsrc_t rsrcV = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(weights_), 0, g.bytesW, 0x00020000);
+        int img[2], y0[2], x0[2];
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            const int p = p0 + (wp * NP + n0 + n) * 16 + l16;
+            img[n] = div_f32(min(p, c.P - 1), c.ghw);
+            const int rem = p - img[n] * c.gHW, py = div_f32(rem, c.gw);
+            y0[n] = p < c.P ? py * g.sy + c.y0 : -(1 << 24);         // (no row at all)
+            x0[n] = (rem - py * c.gW) * g.sx + c.x0;
+        }
+        auto there = [&](int n, int i, int j) {
+            return (unsigned)(y0[n] + g.d * row_of(i)) < (unsigned)g.Hs && (unsigned)(x0[n] + g.d * column_of(j)) < (unsigned)g.Ws;
+        };
+        auto source_of = [&](int n, int ch, int i, int j) { return (img[n] * g.Ch + ch) * g.planeS + (y0[n] + g.d * row_of(i)) * g.Ws + x0[n] + g.d * column_of(j); };
+        double sum[MQ][2][4] = {};
+        bool odd = false;                        // a weight is not finite
+#pragma unroll 1
+        for (int ch0 = cbeg * PK; ch0 < chend; ch0 += 4) {
+            const int ch = ch0 + lo;
+            v4f part[MQ][2];
+#pragma unroll
+            for (int m = 0; m < MQ; ++m)
+#pragma unroll
+                for (int n = 0; n < 2; ++n) part[m][n] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+            for (int i = 0; i < rows; ++i)
+#pragma unroll 1
+                for (int j = 0; j < columns; ++j) {
+                    if (class_of(i, j) != k) continue;
+                    float w[MQ], x[2];
+#pragma unroll
+                    for (int m = 0; m < MQ; ++m) {
+                        const int q = q0 + (wq * MQ + m) * 16 + l16;
+                        w[m] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                            rsrcV, q < g.Q && ch < chend ? 4u * (unsigned)(q * g.qs + ch * g.chs + i * columns + j) : F32_OOB, 0, 0));
+                        odd |= !(__builtin_fabsf(w[m]) < __builtin_inff());
+                    }
+#pragma unroll
+                    for (int n = 0; n < 2; ++n)
+                        x[n] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                            rsrcX, ch < chend && there(n, i, j) ? 4u * (unsigned)source_of(n, ch, i, j) : F32_OOB, 0, 0));
+#pragma unroll
+                    for (int m = 0; m < MQ; ++m)
+#pragma unroll
+                        for (int n = 0; n < 2; ++n) part[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[m], x[n], part[m][n], 0, 0, 0);
+                }
+#pragma unroll
+            for (int m = 0; m < MQ; ++m)
+#pragma unroll
+                for (int n = 0; n < 2; ++n)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sum[m][n][r] += (double)part[m][n][r];
+        }
+        odd = __any(odd);
+#pragma unroll
+        for (int m = 0; m < MQ; ++m)
+#pragma unroll
+            for (int n = 0; n < 2; ++n)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (__builtin_fabsf(acc[k][m][n0 + n][r]) < __builtin_inff()) continue;
+                    float s = (float)sum[m][n][r];
+                    const int q = q0 + (wq * MQ + m) * 16 + 4 * lo + r;
+                    if (odd && s != s && q < g.Q) {
+                        // (of a tap outside the source there is no product, above there was one with 0)
+                        s = 0.0f;
+                        for (int i = 0; i < rows; ++i)
+                            for (int j = 0; j < columns; ++j) {
+                                if (class_of(i, j) != k || !there(n, i, j)) continue;
+                                for (int ch = cbeg * PK; ch < chend && s == s; ch += 8) {
+                                    float w[8], x[8];
+#pragma unroll
+                                    for (int u = 0; u < 8; ++u) {
+                                        const bool is = ch + u < chend;
+                                        w[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                            rsrcV, is ? 4u * (unsigned)(q * g.qs + (ch + u) * g.chs + i * columns + j) : F32_OOB, 0, 0));
+                                        x[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                            rsrcX, is ? 4u * (unsigned)source_of(n, ch + u, i, j) : F32_OOB, 0, 0));
+                                    }
+#pragma unroll
+                                    for (int u = 0; u < 8; ++u) s += w[u] * x[u];
+                                }
+                            }
+                    }
+                    acc[k][m][n0 + n][r] = s;
+                }
+    };
 
     // (before its first tile a block runs through one step that only loads: its code is that of the others)
     PatchItem it, to;
@@ -356,8 +456,19 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
             const unsigned qrow = qn * planeO4;
             float finite = 0.0f;
             each([&](int k, int m, int n, int r) { finite = __builtin_fmaf(acc[k][m][n][r], 0.0f, finite); });
-            const bool plain = partial != 0 || (beta == 0.0f && !bias);
-            if (plain) {
+            if (__any(finite != finite)) {
+                const auto pixels_of = [&](auto k_) {
+                    again_in_float(k_, std::integral_constant<int, 0>{}, p0, q0);
+                    if constexpr (NP == 4) again_in_float(k_, std::integral_constant<int, 2>{}, p0, q0);
+                };
+                pixels_of(std::integral_constant<int, 0>{});
+                if constexpr (CL == 4) {
+                    pixels_of(std::integral_constant<int, 1>{});
+                    pixels_of(std::integral_constant<int, 2>{});
+                    pixels_of(std::integral_constant<int, 3>{});
+                }
+            }
+            if (partial != 0 || (beta == 0.0f && !bias)) {
                 unsigned at = F32_OOB;
                 each([&](int k, int m, int n, int r) {
                     if (q0 + wq * MQ * 16 + 16 * m + r >= g.Q) return;
@@ -366,49 +477,16 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
                     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, s), rsrcO, qn + 16 * m + r < g.Q && at != F32_OOB ? at + qrow : F32_OOB,
                                                           (16 * m + r) * planeO4, 0);
                 });
-            }
-            if (!plain || __any(finite != finite)) {
-                // Infinities, and what rounds to one in bf16, leave NaN where float products might not: such sums are added again,
-                // in float.
-#pragma unroll
-                for (int k = 0; k < CL; ++k)
-#pragma unroll
-                    for (int n = 0; n < NP; ++n) {
-                        const unsigned base = place(k, n);
-                        if (base == F32_OOB) continue;
-                        unsigned redo = 0;
-                        auto store = [&](int m, int r, float s) {
-                            float* at = out + zoff + base / 4u + (size_t)(qn + 16 * m + r) * g.planeO;
-                            if (partial == 0) {
-                                if (beta != 0.0f) s += beta * *at;
-                                if (bias) s = bias[qn + 16 * m + r] + s;
-                            }
-                            *at = s;
-                        };
-#pragma unroll
-                        for (int m = 0; m < MQ; ++m)
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) {
-                                if (qn + 16 * m + r >= g.Q) continue;
-                                if (!(__builtin_fabsf(acc[k][m][n][r]) < __builtin_inff())) redo |= 1u << (4 * m + r);
-                                else if (!plain) store(m, r, acc[k][m][n][r]);
-                            }
-                        const int p = p0 + (wp * NP + n) * 16 + l16, img = div_f32(p, c.ghw), rem = p - img * c.gHW, py = div_f32(rem, c.gw), px = rem - py * c.gW;
-                        const int rows = CL == 4 ? 3 : ny, columns = CL == 4 ? 3 : nx;
-                        for (; redo; redo &= redo - 1) {
-                            const int at = __builtin_ctz(redo), q = qn + 16 * (at >> 2) + (at & 3);
-                            float s = 0.0f;
-                            for (int ch = cbeg * PK; ch < min(cend * PK, g.Ch); ++ch)
-                                for (int i = 0; i < rows; ++i)
-                                    for (int j = 0; j < columns; ++j) {
-                                        const int y = py * g.sy + c.y0 + g.d * row_of(i), x = px * g.sx + c.x0 + g.d * column_of(j);
-                                        if (y < 0 || y >= g.Hs || x < 0 || x >= g.Ws || class_of(i, j) != k) continue;
-                                        s += srcW[(size_t)q * g.qs + (size_t)ch * g.chs + i * columns + j]
-                                             * srcX[((size_t)img * g.Ch + ch) * g.planeS + y * g.Ws + x];
-                                    }
-                            store(at >> 2, at & 3, s);
-                        }
-                    }
+            } else {
+                each([&](int k, int m, int n, int r) {
+                    const unsigned base = place(k, n);
+                    if (base == F32_OOB || qn + 16 * m + r >= g.Q) return;
+                    float* at = out + base / 4u + (size_t)(qn + 16 * m + r) * g.planeO;
+                    float s = acc[k][m][n][r];
+                    if (beta != 0.0f) s += beta * *at;
+                    if (bias) s = bias[qn + 16 * m + r] + s;
+                    *at = s;
+                });
             }
         }
         if (!again) return;

@@ -219,3 +219,55 @@ def test_small_floats_keep_their_bits(small):
         a, d = x * of_x, dy * of_dy
         got, want = _filter(a, w.shape, d, 1, 1), _filter64(a, d, 1, 1)
         assert np.linalg.norm(got - want) <= 1.1 * 2.53e-8 * np.sqrt(1 + 5 * K / 64) * np.linalg.norm(want) + 2.0 ** -150 * np.sqrt(want.size)
+
+
+def _clipped(x, w, dy, s, pad):
+    """Forward and data gradient in float64 whose windows end at the borders: of a tap outside there is no product, not one with 0."""
+    (B, Ci, H, W), (O, _, kH, kW), (oH, oW) = x.shape, w.shape, dy.shape[2:]
+    y, dx, w64 = np.zeros(dy.shape), np.zeros(x.shape), w.astype(np.float64)
+
+    def axis(t, p, size, out):
+        at = [o for o in range(out) if 0 <= o * s + t - p < size]
+        return slice(at[0], at[-1] + 1), slice(at[0] * s + t - p, at[-1] * s + t - p + 1, s)
+    for i in range(kH):
+        for j in range(kW):
+            (oy, iy), (ox, ix) = axis(i, pad[0], H, oH), axis(j, pad[1], W, oW)
+            xs, ds = x[:, :, iy, ix].astype(np.float64), dy[:, :, oy, ox].astype(np.float64)
+            y[:, :, oy, ox] += np.matmul(w64[:, :, i, j], xs.reshape(B, Ci, -1)).reshape(ds.shape)
+            dx[:, :, iy, ix] += np.matmul(w64[:, :, i, j].T, ds.reshape(B, O, -1)).reshape(xs.shape)
+    return y, dx
+
+
+@pytest.mark.parametrize("weights", ["some", "every weight NaN"])
+@pytest.mark.parametrize("case", [(9, 47, 31, 33, 97, 3, 3, 1, 1), (66, 100, 31, 33, 70, 3, 3, 2, 1)])
+def test_weights_that_are_not_finite(case, weights):
+    """What is NaN or infinite follows from the products inside the borders alone: beside them a weight meets no zero."""
+    print("parts, weights not finite", case, weights, flush=True)
+    x, w, dy, s, pad, rng = _inputs(case, 4)
+    x[1, 5], dy[1, 3, ::2] = 0.0, 0.0
+    if weights == "some":
+        w[3, 5, 1, 1], w[7, 2, 0, 2], w[9, 1, 2, 2], w[12, 3, 0, 0], w[12, 30, 2, 1], w[60, 46, 2, 2] = np.inf, np.nan, -np.inf, np.inf, -np.inf, np.nan
+    else:
+        w[:] = np.nan
+    with np.errstate(invalid="ignore"):
+        want = _clipped(x, w, dy, s, pad)
+    fin = np.where(np.isfinite(w), w, np.float32(0))
+    mag = _clipped(np.abs(x), np.abs(fin), np.abs(dy), s, pad)
+    for g, t, m, k in zip(_run(x, w, dy, s, pad), want, mag, (w.shape[1] * 9, w.shape[0] * 9)):
+        assert np.array_equal(np.isnan(g), np.isnan(t)) and np.array_equal(g == np.inf, t == np.inf) and np.array_equal(g == -np.inf, t == -np.inf)
+        ok = np.isfinite(t)
+        assert (np.abs(g[ok] - t[ok]) <= 2.0 ** -24 * (np.abs(t) + (k + 4) * m)[ok]).all()
+
+
+def test_sums_beyond_the_scaled_range():
+    """Operands of size 2^50 and 1e30, whose sums are past 2^96: added again, no further off than the sums of ordinary size."""
+    case = (33, 64, 32, 32, 64, 3, 3, 1, 1)
+    print("parts, large sums", flush=True)
+    x, w, dy, s, pad, rng = _inputs(case, 5)
+    for of_x, of_w in ((np.float32(1e30), np.float32(1)), (np.float32(2.0 ** 50), np.float32(2.0 ** 50)), (np.float32(2.0 ** 115), np.float32(2.0 ** -20))):
+        a, b, d = x * of_x, w * of_w, dy * of_x
+        for g, t in zip(_run(a, b, d, s, pad), _passes(a, b, d, s, pad)):
+            assert np.linalg.norm(g / 1e30 - t / 1e30) <= 1.1 * 2.53e-8 * np.sqrt(1 + 5 * 64 * 9 / 64) * np.linalg.norm(t / 1e30)
+        d = dy * of_w
+        got, want = _filter(a, w.shape, d, 1, 1) / 1e30, _filter64(a, d, 1, 1) / 1e30
+        assert np.linalg.norm(got - want) <= 1.1 * 2.53e-8 * np.sqrt(1 + 5 * 33 * 1024 / 64) * np.linalg.norm(want)
