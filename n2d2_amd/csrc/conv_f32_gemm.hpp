@@ -1241,47 +1241,56 @@ __global__ __launch_bounds__(256) void conv_f32_small_pair_kernel(const SmallPai
 
 // Backward-data of small problems, the same way: dx[c][pixel] adds w[o][c][tap] dy[o][the pixel that the tap reaches] over (o, tap)
 // in double.  A block is 16 channels x 16 input pixels; its waves take 16 terms in turn.  Bound by the latency of its loads, a
-// microsecond for each wave's two rounds of them: 8 waves where K is more than four waves take in two.  Which pixel a tap reaches
-// is worked out once for the block (for every term: 12.1 us where this takes 8.6).
-// us, the pixel kernel with its ranges / this with 4 / 8 waves (error against 64 bits 1.4e-7, 2.5e-8):
-//   6 <- 16, 5x5, 14 x 14, batch 32, K 400   14.5 /  8.6 /  7.8      16 <- 16, 3x3, 28 x 28, batch 8, K 144    12.3 /  5.3 /  5.6
-//   8 <- 16, 3x3, 32 x 32, batch 16, K 144   12.4 /  6.5 /  7.7      64 <- 64, 3x3, 28 x 28, K 576             11.8 /  8.6 /  6.7
-//   64 <- 64, 3x3 stride 2, 14 x 14, batch 4 10.5 /  8.5 /  6.7      256 <- 256, 3x3, 7 x 7, K 2304            20.1 / 24.0 / 16.5
-//   8 <- 512, 3x3, 7 x 7, K 4608             15.5 / 43.9 / 29.1      8 <- 8, 3x3, 32 x 32, batch 64, K 72      12.2 / 13.7 / 18.8
+// microsecond for each wave's two rounds of them: 8 waves where K is more than four waves take in two, 16 from 1025 terms; and where
+// the tiles are more than the chip holds blocks, a tile to each wave.  Which pixel a tap reaches is worked out once for the tile
+// (for every term: half as long again).  Beyond the range of the rule: 8 <- 512, 3x3, 7 x 7, K 4608 15.5 us on the pixel kernel and 29.1 on this; 8 <- 8,
+// 3x3, 32 x 32, batch 64, 2.9e5 11.5 / 13.7.
+// us, the pixel kernel with its ranges / this (error against 64 bits 1.4e-7, 2.5e-8):
+//   6 <- 16, 5x5, 14 x 14, batch 32, K 400   14.1 /  6.8             16 <- 16, 3x3, 28 x 28, batch 8, K 144    12.0 /  4.6
+//   8 <- 16, 3x3, 32 x 32, batch 16, K 144   12.0 /  5.8             64 <- 64, 3x3, 28 x 28, K 576             11.4 /  6.0
+//   64 <- 64, 3x3 stride 2, 14 x 14, batch 4 10.3 /  6.0             256 <- 256, 3x3, 7 x 7, K 2304            20.1 / 14.9
+//   477 <- 11, 1x1 stride 2, 17 x 78, batch 7, 17430 tiles 12.1 / 12.0 (four waves to a tile 28.0)
+//   121 <- 13, 1x1, 26 x 36, batch 31, 14512 tiles 10.3 / 10.1 (23.3)
 struct DataSmall {
     int P, C, O, T, K;                           // input pixels over all images; taps; O * T
     int kW, HW, W, oH, oW, sy, sx, pt, pl;
+    unsigned bytesW, bytesY;
     DivF32 dHW, dW, dT, dkW, dsy, dsx;
 };
-template <int WAVES>
+// (TILES: a block's, 1, or one to each of its waves, which then takes all of K; `tp` is the first)
+template <int WAVES, int TILES>
 __device__ __forceinline__ void data_small_tile(const DataSmall& g, int tp, int tc, const float* __restrict__ w, const float* __restrict__ dy, float beta,
                                                 float* __restrict__ dx)
 {
-    __shared__ double red[WAVES][256];
-    __shared__ int reach[64 * 16];               // where in a channel's image a pixel's tap is; -1: outside
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane & 15, kg = lane >> 4;
-    const int c = tc * 16 + row, plane = g.oH * g.oW;
+    static_assert(TILES == 1 || TILES == WAVES, "a tile of the block or of a wave");
+    constexpr int SHARE = WAVES / TILES;         // waves of a tile
+    __shared__ double red[TILES == 1 ? WAVES : 1][256];
+    __shared__ int reach_of[TILES][64 * 16];     // where in a channel's image a pixel's tap is; -1: outside
+    const int lane = threadIdx.x & 63, wave = TILES == 1 ? threadIdx.x >> 6 : 0, row = lane & 15, kg = lane >> 4;
+    int* const reach = reach_of[TILES == 1 ? 0 : threadIdx.x >> 6];
+    if (TILES > 1) tp += threadIdx.x >> 6;
+    const __amdgpu_buffer_rsrc_t rsrcW = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(w), 0, g.bytesW, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrcY = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(dy), 0, g.bytesY, 0x00020000);
+    const int c = tc * 16 + row, plane = g.oH * g.oW, p = min(tp * 16 + row, g.P - 1), img = div_f32(p, g.dHW);
     {
-        const int p = min(tp * 16 + (int)(threadIdx.x & 15), g.P - 1), rem = p - div_f32(p, g.dHW) * g.HW, iy = div_f32(rem, g.dW), ix = rem - iy * g.W;
-        for (int t = threadIdx.x >> 4; t < g.T; t += 4 * WAVES) {
+        const int rem = p - img * g.HW, iy = div_f32(rem, g.dW), ix = rem - iy * g.W;
+        for (int t = TILES == 1 ? threadIdx.x >> 4 : kg; t < g.T; t += 4 * SHARE) {
             const int ty = div_f32(t, g.dkW), y = iy + g.pt - ty, x = ix + g.pl - (t - ty * g.kW);
             const int oy = div_f32(max(y, 0), g.dsy), ox = div_f32(max(x, 0), g.dsx);
-            reach[t * 16 + (threadIdx.x & 15)] = y >= 0 && x >= 0 && oy * g.sy == y && ox * g.sx == x && oy < g.oH && ox < g.oW ? oy * g.oW + ox : -1;
+            reach[t * 16 + row] = y >= 0 && x >= 0 && oy * g.sy == y && ox * g.sx == x && oy < g.oH && ox < g.oW ? oy * g.oW + ox : -1;
         }
     }
     __syncthreads();
-    const float* wb = w + (size_t)min(c, g.C - 1) * g.T;
-    const float* yb = dy + (size_t)div_f32(min(tp * 16 + row, g.P - 1), g.dHW) * g.O * plane;
     float a[2][4], b[2][4];
-    const int adv_o = div_f32(16 * WAVES, g.dT), adv_t = 16 * WAVES - adv_o * g.T;
+    const int adv_o = div_f32(16 * SHARE, g.dT), adv_t = 16 * SHARE - adv_o * g.T;
     int ko = div_f32(wave * 16 + kg * 4, g.dT), kt = wave * 16 + kg * 4 - ko * g.T;     // this lane's next term
     auto load = [&](float (&av)[4], float (&bv)[4]) {
         int o = ko, t = kt;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int at = o < g.O ? reach[t * 16 + row] : -1;
-            av[j] = o < g.O ? wb[(size_t)o * g.C * g.T + t] : 0.0f;
-            bv[j] = at >= 0 ? yb[(size_t)o * plane + at] : 0.0f;
+            av[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrcW, o < g.O && c < g.C ? 4u * (unsigned)((o * g.C + c) * g.T + t) : F32_OOB, 0, 0));
+            bv[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrcY, at >= 0 ? 4u * (unsigned)((img * g.O + o) * plane + at) : F32_OOB, 0, 0));
             if (++t == g.T) { t = 0; ++o; }
         }
         ko += adv_o;
@@ -1289,43 +1298,54 @@ __device__ __forceinline__ void data_small_tile(const DataSmall& g, int tp, int 
         if (kt >= g.T) { kt -= g.T; ++ko; }
     };
     v4d acc = {0.0, 0.0, 0.0, 0.0};
+    auto multiply = [&](const float (&av)[4], const float (&bv)[4]) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)av[j], (double)bv[j], acc, 0, 0, 0);
+    };
     load(a[0], b[0]);
-    for (int s = wave * 16; s < g.K; s += 32 * WAVES) {
-        load(a[1], b[1]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[0][j], (double)b[0][j], acc, 0, 0, 0);
+    for (int s = wave * 16; s < g.K; s += 32 * SHARE) {
+        const bool second = s + 16 * SHARE < g.K;
+        if (second) load(a[1], b[1]);
+        multiply(a[0], b[0]);
+        if (!second) break;
         load(a[0], b[0]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[1][j], (double)b[1][j], acc, 0, 0, 0);
+        multiply(a[1], b[1]);
     }
+    const auto store = [&](int oc, int op, double v) {
+        if (oc >= g.C || op >= g.P) return;
+        const int oi = div_f32(op, g.dHW);
+        const size_t idx = ((size_t)oi * g.C + oc) * g.HW + (op - oi * g.HW);
+        dx[idx] = (float)v + (beta != 0.0f ? beta * dx[idx] : 0.0f);
+    };
     // lane holds column p = lane % 16 and rows c = 4 r + lane / 16
+    if constexpr (TILES > 1) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) store(tc * 16 + 4 * r + kg, tp * 16 + row, acc[r]);
+        return;
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) red[wave][(4 * r + kg) * 16 + row] = acc[r];
     __syncthreads();
     if (threadIdx.x >= 256) return;
-    const int oc = tc * 16 + threadIdx.x / 16, op = tp * 16 + threadIdx.x % 16;
-    if (oc >= g.C || op >= g.P) return;
     double v = red[0][threadIdx.x];
 #pragma unroll
-    for (int i = 1; i < WAVES; ++i) v += red[i][threadIdx.x];
-    const int oi = div_f32(op, g.dHW);
-    const size_t idx = ((size_t)oi * g.C + oc) * g.HW + (op - oi * g.HW);
-    dx[idx] = (float)v + (beta != 0.0f ? beta * dx[idx] : 0.0f);
+    for (int i = 1; i < (TILES == 1 ? WAVES : 1); ++i) v += red[i][threadIdx.x];
+    store(tc * 16 + threadIdx.x / 16, tp * 16 + threadIdx.x % 16, v);
 }
-// (dtiles: of 16 pixels.  The tiles of both directions are in the grid's first: channels alone can be more than 16 x 65535)
-template <int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void conv_f32_data_small_kernel(DataSmall g, int dtiles, const float* __restrict__ w, const float* __restrict__ dy,
+// (across: blocks along the pixels.  Those of both directions are in the grid's first: channels alone can be more than 16 x 65535)
+template <int WAVES, int TILES>
+__global__ __launch_bounds__(64 * WAVES) void conv_f32_data_small_kernel(DataSmall g, int across, const float* __restrict__ w, const float* __restrict__ dy,
                                                                          float beta, float* __restrict__ dx)
 {
-    const int tc = blockIdx.x / dtiles;
-    data_small_tile<WAVES>(g, blockIdx.x - tc * dtiles, tc, w, dy, beta, dx);
+    const int tc = blockIdx.x / across;
+    data_small_tile<WAVES, TILES>(g, (blockIdx.x - tc * across) * TILES, tc, w, dy, beta, dx);
 }
 // Both gradients of a small layer in one launch, the blocks of the data first, which take longer, then those of the weights, whose ranges
 // are added by the launch that follows.  us, two launches / one, with the one that adds: 6 <- 16, 5x5, 14 x 14, batch 32 15.5 / 12.4; 64 <- 64,
 // 3x3 stride 2, 14 x 14, batch 4 12.1 / 8.5; 8 <- 8, 3x3, 16 x 16, batch 2 11.3 / 7.4.
 struct SmallBoth {
     DataSmall data;
-    int dtiles;                                  // of 16 pixels
+    int across;                                  // the data's blocks along the pixels
     unsigned first;                              // first block of the weights'
     SmallProduct filter;
     int ftiles;                                  // tiles of a range
@@ -1334,12 +1354,12 @@ struct SmallBoth {
     float* dx;
     double* partial;
 };
-template <int WAVES>
+template <int WAVES, int TILES>
 __global__ __launch_bounds__(64 * WAVES) void conv_f32_small_both_kernel(const SmallBoth a)
 {
     if (blockIdx.x < a.first) {
-        const int tc = blockIdx.x / a.dtiles;
-        data_small_tile<WAVES>(a.data, blockIdx.x - tc * a.dtiles, tc, a.w, a.dy, a.beta, a.dx);
+        const int tc = blockIdx.x / a.across;
+        data_small_tile<WAVES, TILES>(a.data, (blockIdx.x - tc * a.across) * TILES, tc, a.w, a.dy, a.beta, a.dx);
     } else {
         const int block = blockIdx.x - a.first, range = block / a.ftiles, tile = block - range * a.ftiles, tq = tile / a.filter.ptiles;
         filter_small_tile<WAVES>(a.filter.g, tile - tq * a.filter.ptiles, tq, range, a.filter.srcX, a.filter.srcY, a.partial, a.filter.beta, a.filter.out);

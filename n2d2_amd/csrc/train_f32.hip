@@ -741,7 +741,7 @@ __global__ __launch_bounds__(1024) void batchnorm_f32_backward_sums_kernel(BnRan
     });
     bn_block_sums<SAT ? BN_SUMS + 1 : BN_SUMS>(s);
     if (threadIdx.x) return;
-    if (SAT) sat.partial[(size_t)c * gridDim.y + blockIdx.y] = s[BN_SUMS];
+    if constexpr (SAT) sat.partial[(size_t)c * gridDim.y + blockIdx.y] = s[BN_SUMS];
     if (gridDim.y == 1) {
         double t[5];
         float dmean, dvariance;
@@ -1019,7 +1019,8 @@ static int f32_path(const ConvF32& q, int pass)
     if (forced) return F32_PATH_GEMM;
     // Small data gradients add in double.  Spanning layers below 2e7 flops (us, product in float / this): 16 x 5 x 5 <- 120, batch 32 8.4 / 4.2;
     // 120 <- 84, batch 32 8.5 / 4.2; 512 x 1 x 1 <- 64, batch 2 7.7 / 3.9; 64 <- 10, batch 96 5.5 / 4.0.  Others by the rounds of loads
-    // of all blocks and of one (conv_f32_data_small_kernel has the times).
+    // of all blocks and of one (data_small_tile has the times).  (Of 430 drawn layers those of 2x2 at stride 2 with products of 1.9e5 and
+    // more, and strided ones of K from 1800, take up to 1.2 times as long as the sums in float.)
     if (pass == PASS_BWD_DATA && !many_taps(q)) {
         if (spans_input(q)) {
             if (small && q.B <= 16 * GRID_Y) return F32_PATH_SMALL;
@@ -1747,6 +1748,39 @@ static int run_pass(const ConvF32& q, int pass, const float* a, const float* b, 
     return N2D2HIP_OK;
 }
 
+static DataSmall small_data(const ConvF32& q)
+{
+    const int T = q.kH * q.kW;
+    return DataSmall{q.B * q.H * q.W, q.C, q.O, T, q.O * T, q.kW, q.H * q.W, q.W, q.oH, q.oW, q.sy, q.sx, q.pt, q.pl,
+                     (unsigned)(4 * (size_t)q.O * q.C * T), (unsigned)(4 * (size_t)q.B * q.O * q.oH * q.oW),
+                     div_of(q.H * q.W), div_of(q.W), div_of(T), div_of(q.kW), div_of(q.sy), div_of(q.sx)};
+}
+// Waves of a block, and tiles: of the block, or one of each wave: where the tiles are more than the chip holds blocks, and a wave's share of K
+// is short.  us, all of a block / one of a wave (tiles, K): 804, 14 4.0 / 4.0; 1296, 64 4.5 / 5.8; 1674, 128 7.6 / 8.3; 1785, 36 5.1 / 4.9; 1890, 28
+// 4.8 / 4.6; 2232, 53 6.1 / 6.7; 2444, 16 5.5 / 4.0; 2366, 91 8.8 / 8.4; 4200, 9 7.1 / 4.6; 23674, 9 28.2 / 14.3.
+struct SmallDataShape {
+    int waves, tiles, across;
+    unsigned blocks;                             // (2.3e5 / K at most)
+};
+static SmallDataShape small_data_shape(const DataSmall& g)
+{
+    const int dtiles = ceil_div_i(g.P, 16), ctiles = ceil_div_i(g.C, 16);
+    SmallDataShape s = {};
+    s.waves = g.K <= 256 ? 4 : g.K <= 1024 ? 8 : 16;
+    s.tiles = s.waves == 4 && (long)dtiles * ctiles > 1792 && g.K <= 112 ? 4 : 1;
+    s.across = ceil_div_i(dtiles, s.tiles);
+    s.blocks = (unsigned)(s.across * ctiles);
+    return s;
+}
+template <class F>
+static void small_data_kernel(const SmallDataShape& s, F&& f)
+{
+    if (s.tiles == 4) f(std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
+    else if (s.waves == 4) f(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{});
+    else if (s.waves == 8) f(std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{});
+    else f(std::integral_constant<int, 16>{}, std::integral_constant<int, 1>{});
+}
+
 } // namespace n2d2hip
 
 using namespace n2d2hip;
@@ -1777,12 +1811,6 @@ int n2d2hip_conv2d_f32_forward(const n2d2hip_conv_desc* desc, int B, int H, int 
     return run_direct(q, PASS_FWD, x, w, bias, beta, y, (hipStream_t)stream);
 }
 
-static DataSmall small_data(const ConvF32& q)
-{
-    const int T = q.kH * q.kW;
-    return DataSmall{q.B * q.H * q.W, q.C, q.O, T, q.O * T, q.kW, q.H * q.W, q.W, q.oH, q.oW, q.sy, q.sx, q.pt, q.pl,
-                     div_of(q.H * q.W), div_of(q.W), div_of(T), div_of(q.kW), div_of(q.sy), div_of(q.sx)};
-}
 int n2d2hip_conv2d_f32_backward_data(const n2d2hip_conv_desc* desc, int B, int H, int W, const float* w, const float* diff_y, float beta,
                                      float* diff_x, void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream)
 {
@@ -1795,10 +1823,12 @@ int n2d2hip_conv2d_f32_backward_data(const n2d2hip_conv_desc* desc, int B, int H
         return run_small_filter(small_gemm(q, PASS_BWD_DATA), w, diff_y, beta, diff_x, (double*)workspace, workspace ? workspace_bytes : 0, (hipStream_t)stream);
     if (path == F32_PATH_SMALL_DATA) {
         const DataSmall g = small_data(q);
-        const int dtiles = ceil_div_i(g.P, 16);
-        const dim3 grid(dtiles * ceil_div_i(g.C, 16));       // (2.3e5 / K at most)
-        if (g.K <= 256) N2D2HIP_LAUNCH_T(conv_f32_data_small_kernel, (4), grid, dim3(256), 0, (hipStream_t)stream, g, dtiles, w, diff_y, beta, diff_x);
-        else N2D2HIP_LAUNCH_T(conv_f32_data_small_kernel, (8), grid, dim3(512), 0, (hipStream_t)stream, g, dtiles, w, diff_y, beta, diff_x);
+        const SmallDataShape shape = small_data_shape(g);
+        small_data_kernel(shape, [&](auto waves_, auto tiles_) {
+            constexpr int WAVES = decltype(waves_)::value, TILES = decltype(tiles_)::value;
+            N2D2HIP_LAUNCH_T(conv_f32_data_small_kernel, (WAVES, TILES), dim3(shape.blocks), dim3(64 * WAVES), 0, (hipStream_t)stream, g, shape.across, w, diff_y, beta,
+                             diff_x);
+        });
         N2D2HIP_HIP_CHECK(hipGetLastError());
         return N2D2HIP_OK;
     }
@@ -1909,8 +1939,9 @@ int n2d2hip_conv2d_f32_backward(const n2d2hip_conv_desc* desc, int B, int H, int
     if (apart && f32_path(q, PASS_BWD_FILTER) == F32_PATH_SMALL && f32_path(q, PASS_BWD_DATA) == F32_PATH_SMALL_DATA) {
         SmallBoth b = {};
         b.data = small_data(q);
-        b.dtiles = ceil_div_i(b.data.P, 16);
-        b.first = (unsigned)(b.dtiles * ceil_div_i(b.data.C, 16));               // (2.3e5 / K at most)
+        const SmallDataShape shape = small_data_shape(b.data);
+        b.across = shape.across;
+        b.first = shape.blocks;
         b.filter.g = small_gemm(q, PASS_BWD_FILTER);
         const size_t n = (size_t)b.filter.g.Q * b.filter.g.P;
         const int ranges = small_filter_ranges(b.filter.g, n, (const double*)workspace, workspace ? workspace_bytes : 0);
@@ -1922,8 +1953,10 @@ int n2d2hip_conv2d_f32_backward(const n2d2hip_conv_desc* desc, int B, int H, int
             b.w = w; b.dy = diff_y; b.beta = beta_x; b.dx = diff_x;
             b.partial = ranges > 1 ? (double*)workspace : nullptr;
             const dim3 grid(b.first + (unsigned)(ftiles * ranges));
-            if (b.data.K <= 256) N2D2HIP_LAUNCH(conv_f32_small_both_kernel<4>, grid, dim3(256), 0, (hipStream_t)stream, b);
-            else N2D2HIP_LAUNCH(conv_f32_small_both_kernel<8>, grid, dim3(512), 0, (hipStream_t)stream, b);
+            small_data_kernel(shape, [&](auto waves_, auto tiles_) {
+                constexpr int WAVES = decltype(waves_)::value, TILES = decltype(tiles_)::value;
+                N2D2HIP_LAUNCH_T(conv_f32_small_both_kernel, (WAVES, TILES), grid, dim3(64 * WAVES), 0, (hipStream_t)stream, b);
+            });
             if (ranges > 1)
                 hipLaunchKernelGGL(conv_f32_reduce_partials_kernel<double>, dim3(reduce_grid(n)), dim3(256), 0, (hipStream_t)stream, (const double*)workspace,
                                    ranges, n, beta_w, diff_w, (const float*)nullptr, 1, 1);

@@ -14,6 +14,7 @@ CASES = [(32, 84, 10, 1, 1, 1, 1, 0, 1, PAIR), (32, 120, 84, 1, 1, 1, 1, 0, 1, P
          (600, 8, 8, 1, 1, 1, 1, 0, 1, None), (4, 2, 3000, 1, 1, 1, 1, 0, 1, None),           # (sums in ranges)
          (8, 6, 16, 5, 14, 14, 1, 0, 1, BOTH), (4, 16, 16, 3, 12, 10, 2, 1, 1, BOTH), (1, 17, 28, 3, 9, 9, 1, 1, 1, BOTH), (2, 16, 29, 3, 9, 9, 1, 0, 1, BOTH),
          (1, 1, 1, 2, 3, 3, 1, 0, 1, BOTH), (32, 3, 8, 3, 15, 17, 1, 1, 1, BOTH), (32, 6, 16, 5, 14, 14, 1, 0, 1, BOTH),
+         (31, 20, 8, 1, 40, 47, 1, 0, 1, BOTH), (9, 5, 3, 3, 71, 64, 1, 1, 1, BOTH), (1, 9, 130, 3, 9, 9, 1, 1, 1, BOTH),      # (a tile to a wave; sixteen waves to a tile)
          (4, 16, 16, 3, 12, 10, 1, 1, 16, None),
          (64, 64, 64, 3, 24, 24, 1, 1, 1, None), (64, 512, 1000, 1, 1, 1, 1, 0, 1, None), (2, 4, 10, 16, 16, 16, 1, 0, 1, None)]
 

@@ -12,6 +12,12 @@ pytestmark = pytest.mark.gpu
 CASES = [(32, 6, 14, 14, 16, 5, 5, 1, 1, 0, 0), (1, 1, 1, 1, 1, 1, 1, 1, 1, 0, 0), (3, 17, 9, 11, 5, 3, 3, 1, 1, 1, 1), (2, 16, 13, 7, 29, 3, 3, 2, 2, 1, 1), (5, 33, 8, 8, 40, 1, 1, 1, 1, 0, 0),
          (4, 3, 10, 9, 8, 2, 3, 3, 2, 0, 1), (1, 64, 14, 14, 256, 3, 3, 1, 1, 1, 1), (2, 5, 30, 4, 33, 31, 2, 1, 1, 1, 15), (2, 20, 7, 7, 11, 3, 3, 1, 3, 2, 0),
          (32, 16, 5, 5, 120, 5, 5, 1, 1, 0, 0), (7, 30, 1, 1, 9, 1, 1, 1, 1, 0, 0), (3, 2, 8, 8, 100, 8, 8, 1, 1, 0, 0)]
+# A tile to each wave: tiles and channels left over, one term and the most, a tap and nine; beside them one tile and one term less or more than
+# the line.  Sixteen waves to a tile, and the last K of eight.
+WAVES = [((1, 17, 151, 190, 1, 1, 1, 1, 1, 0, 0), "<4, 4>"), ((31, 20, 40, 47, 8, 1, 1, 1, 1, 0, 0), "<4, 4>"), ((33, 16, 31, 30, 12, 3, 3, 2, 2, 1, 1), "<4, 4>"),
+         ((7, 9, 64, 65, 112, 1, 1, 1, 1, 0, 0), "<4, 4>"), ((7, 9, 64, 65, 113, 1, 1, 1, 1, 0, 0), "<4, 1>"), ((28, 16, 32, 32, 9, 3, 3, 1, 1, 1, 1), "<4, 1>"),
+         ((1, 16, 64, 449, 9, 3, 3, 1, 1, 1, 1), "<4, 4>"), ((2, 30, 9, 7, 1025, 1, 1, 1, 1, 0, 0), "<16, 1>"), ((1, 17, 5, 9, 256, 3, 3, 1, 1, 1, 1), "<16, 1>"),
+         ((2, 30, 9, 7, 1024, 1, 1, 1, 1, 0, 0), "<8, 1>")]
 
 
 @pytest.mark.parametrize("beta", [0.0, 0.5])
@@ -44,6 +50,15 @@ def test_adds_in_double(case, beta):
         want = want + 0.5 * start
         bound = bound + 2.0 ** -24 * (np.abs(want) + bound) + 2.0 ** -25 * np.abs(start)
     assert (np.abs(got - want) <= bound).all()
+
+
+@pytest.mark.parametrize("case,shape", WAVES, ids=str)
+def test_waves_of_a_tile(case, shape):
+    from n2d2_amd import capi
+    with capi.launch_log() as log:
+        test_adds_in_double(case, 0.0)
+        test_adds_in_double(case, 0.5)
+    assert [e[0] for e in log.entries] == ["conv_f32_data_small_kernel" + shape] * 2
 
 
 @pytest.mark.parametrize("joint", [False, True])
