@@ -197,8 +197,8 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
 
     // Infinities, and what rounds to one in bf16, leave NaN where float products might not.  A wave that holds such sums adds them
     // again, on the fp32 matrix cores straight from memory, in double from four channels to the next.
-    // us of 64 -> 64, 56 x 56, batch 64, forward / data: finite 96 / 95; NaN throughout 830 / 700; a channel of the input NaN 650 / 520; one weight
-    // NaN 1240 / 1260 (a sum after the other by the lane that held it: 6520 / 6570, 6500 / 6590, 970 / 1500).
+    // us of 64 -> 64, 56 x 56, batch 64, forward / data: finite 93 / 85; NaN throughout 624 / 507; a channel of the input NaN 617 / 505; one weight
+    // NaN 852 / 815 (a sum after the other by the lane that held it: 6520 / 6570, 6500 / 6590, 970 / 1500).
     // (32 pixels of one class at a time: of more the sums would take the registers that hold the next step's operands)
     auto again_in_float = [&](auto k_, auto n_, int p0, int q0) {
         constexpr int k = decltype(k_)::value, n0 = decltype(n_)::value;
@@ -261,6 +261,7 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
                     for (int r = 0; r < 4; ++r) sum[m][n][r] += (double)part[m][n][r];
         }
         odd = __any(odd);
+        unsigned nans = 0;                       // sums that a tap outside the source may have made NaN: above there was a product with 0, of which there is none
 #pragma unroll
         for (int m = 0; m < MQ; ++m)
 #pragma unroll
@@ -268,31 +269,49 @@ __global__ __launch_bounds__(256, 2) void conv_f32_patch_kernel(PixelGemm g, con
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     if (__builtin_fabsf(acc[k][m][n0 + n][r]) < __builtin_inff()) continue;
-                    float s = (float)sum[m][n][r];
-                    const int q = q0 + (wq * MQ + m) * 16 + 4 * lo + r;
-                    if (odd && s != s && q < g.Q) {
-                        // (of a tap outside the source there is no product, above there was one with 0)
-                        s = 0.0f;
-                        for (int i = 0; i < rows; ++i)
-                            for (int j = 0; j < columns; ++j) {
-                                if (class_of(i, j) != k || !there(n, i, j)) continue;
-                                for (int ch = cbeg * PK; ch < chend && s == s; ch += 8) {
-                                    float w[8], x[8];
-#pragma unroll
-                                    for (int u = 0; u < 8; ++u) {
-                                        const bool is = ch + u < chend;
-                                        w[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                            rsrcV, is ? 4u * (unsigned)(q * g.qs + (ch + u) * g.chs + i * columns + j) : F32_OOB, 0, 0));
-                                        x[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                            rsrcX, is ? 4u * (unsigned)source_of(n, ch + u, i, j) : F32_OOB, 0, 0));
-                                    }
-#pragma unroll
-                                    for (int u = 0; u < 8; ++u) s += w[u] * x[u];
-                                }
-                            }
-                    }
+                    const float s = (float)sum[m][n][r];
                     acc[k][m][n0 + n][r] = s;
+                    if (odd && s != s && q0 + (wq * MQ + m) * 16 + 4 * lo + r < g.Q) nans |= 1u << ((m * 2 + n) * 4 + r);
                 }
+        // (one after the other, and the code once: sixteen times, in each of the kernel's instances, the compiler takes seven minutes for the file
+        // instead of 40 s, and one weight NaN is 1240 / 1260 us)
+#pragma unroll 1
+        for (int at = 0; at < 8 * MQ; ++at) {
+            if (!__any(nans >> at & 1)) continue;
+            const int n = at >> 2 & 1, q = q0 + (wq * MQ + (at >> 3)) * 16 + 4 * lo + (at & 3);
+            const int y = n ? y0[1] : y0[0], x_ = n ? x0[1] : x0[0], b = n ? img[1] : img[0];
+            float s = 0.0f;
+            if (nans >> at & 1) {
+#pragma unroll 1
+                for (int i = 0; i < rows; ++i)
+#pragma unroll 1
+                    for (int j = 0; j < columns; ++j) {
+                        const int ys = y + g.d * row_of(i), xs = x_ + g.d * column_of(j);
+                        if (class_of(i, j) != k || (unsigned)ys >= (unsigned)g.Hs || (unsigned)xs >= (unsigned)g.Ws) continue;
+#pragma unroll 1
+                        for (int ch = cbeg * PK; ch < chend && s == s; ch += 8) {
+                            float w[8], x[8];
+#pragma unroll
+                            for (int u = 0; u < 8; ++u) {
+                                const bool is = ch + u < chend;
+                                w[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                    rsrcV, is ? 4u * (unsigned)(q * g.qs + (ch + u) * g.chs + i * columns + j) : F32_OOB, 0, 0));
+                                x[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                    rsrcX, is ? 4u * (unsigned)((b * g.Ch + ch + u) * g.planeS + ys * g.Ws + xs) : F32_OOB, 0, 0));
+                            }
+#pragma unroll
+                            for (int u = 0; u < 8; ++u) s += w[u] * x[u];
+                        }
+                    }
+            }
+#pragma unroll
+            for (int m = 0; m < MQ; ++m)
+#pragma unroll
+                for (int n = 0; n < 2; ++n)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (at == (m * 2 + n) * 4 + r && (nans >> at & 1)) acc[k][m][n0 + n][r] = s;
+        }
     };
 
     // (before its first tile a block runs through one step that only loads: its code is that of the others)
