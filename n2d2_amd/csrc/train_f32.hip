@@ -1423,8 +1423,9 @@ static void launch_patch(const PixelPlan& pl, dim3 grid, const float* x, const f
 {
     grid.x = std::min(grid.x, 8u * 32u * 2u);    // (two blocks to a CU)
     const auto run = [&](auto nu_, auto nt_, auto fold_) {
-        hipLaunchKernelGGL((conv_f32_patch_kernel<WQ, WP, MQ, NP, 2 * decltype(nu_)::value, decltype(nt_)::value, decltype(fold_)::value>), grid, dim3(256), 0,
-                           st, pl.g, x, w, (const v4u*)wt, bias, beta, out, partial);
+        constexpr int PB = 2 * decltype(nu_)::value, NT = decltype(nt_)::value;
+        constexpr bool FOLD = decltype(fold_)::value;
+        N2D2HIP_LAUNCH_T(conv_f32_patch_kernel, (WQ, WP, MQ, NP, PB, NT, FOLD), grid, dim3(256), 0, st, pl.g, x, w, (const v4u*)wt, bias, beta, out, partial);
     };
     const auto taps = [&](auto nu_, auto fold_) {
         pl.g.c[0].nT == 9 && pl.g.c[0].nx == 3 ? run(nu_, std::integral_constant<int, 9>{}, fold_) : run(nu_, std::integral_constant<int, 0>{}, fold_);
@@ -1559,7 +1560,8 @@ static void launch_rows(const RowsPlan& pl, int s, const float* x, const float* 
 {
     const dim3 grid(pl.ctiles, pl.qtiles, pl.splits);
     const auto run = [&](auto s_, auto nol_) {
-        hipLaunchKernelGGL((conv_f32_filter_rows_kernel<decltype(s_)::value, decltype(nol_)::value>), grid, dim3(512), 0, st, pl.g, x, dy, ws);
+        constexpr int S = decltype(s_)::value, NOL = decltype(nol_)::value;
+        N2D2HIP_LAUNCH_T(conv_f32_filter_rows_kernel, (S, NOL), grid, dim3(512), 0, st, pl.g, x, dy, ws);
     };
     const auto octets = [&](auto s_) {
         if (pl.nol == 0) run(s_, std::integral_constant<int, 0>{});
@@ -1568,8 +1570,8 @@ static void launch_rows(const RowsPlan& pl, int s, const float* x, const float* 
         else if constexpr (decltype(s_)::value == 1) run(s_, std::integral_constant<int, 3>{});
     };
     s == 1 ? octets(std::integral_constant<int, 1>{}) : octets(std::integral_constant<int, 2>{});
-    hipLaunchKernelGGL(conv_f32_reduce_rows_kernel, dim3((unsigned)(pl.values() / 64)), dim3(256), 0, st, (const float*)ws, pl.splits, pl.ctiles, pl.values(), pl.g.Q,
-                       pl.g.C, beta, dw);
+    N2D2HIP_LAUNCH(conv_f32_reduce_rows_kernel, dim3((unsigned)(pl.values() / 64)), dim3(256), 0, st, (const float*)ws, pl.splits, pl.ctiles, pl.values(), pl.g.Q,
+                   pl.g.C, beta, dw);
 }
 // What the small filter kernel runs of a pass: backward-filter, or backward-data of a spanning kernel as a sum over "pixels" o,
 // dx[b][k] = sum_o dy[b][o] w[o][k], with the images as rows of q and the weights of an output as columns of p.
@@ -1718,7 +1720,7 @@ static int run_pass(const ConvF32& q, int pass, const float* a, const float* b, 
         const dim3 grid(std::min((total + 255) / 256, 4096));
         if (kind == PIXELS_3X3) hipLaunchKernelGGL(conv_f32_lay_weights3x3_kernel, grid, dim3(256), 0, st, b, ws, total, g.Q, g.qpad, g.Ch, g.qs, g.chs);
         else if (kind == PIXELS_PATCH)
-            hipLaunchKernelGGL(conv_f32_lay_parts_kernel, grid, dim3(256), 0, st, b, (v4u*)ws, total, g.Q, g.qpad / 16, g.Ch, g.T, g.qs, g.chs);
+            N2D2HIP_LAUNCH(conv_f32_lay_parts_kernel, grid, dim3(256), 0, st, b, (v4u*)ws, total, g.Q, g.qpad / 16, g.Ch, g.T, g.qs, g.chs);
         else hipLaunchKernelGGL(conv_f32_lay_weights_kernel, grid, dim3(256), 0, st, b, ws, total, g.Q, g.qpad, g.Ch, g.T, g.qs, g.chs);
         ws += nlaid;
         ws_floats -= nlaid;

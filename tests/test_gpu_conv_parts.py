@@ -7,7 +7,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-# B, C, H, W, O, kH, kW, stride, pad, data gradient: rows and channels left over (97 rows, 39 channels), runs that cross images, pixels past
+# B, C, H, W, O, kH, kW, stride, pad, forward and data gradient, whichever kernel takes them (ROUTES names those of the parts): rows and channels left over (97 rows, 39 channels), runs that cross images, pixels past
 # the last tile, 32 rows and less, other kernels than 3x3, strides, K ranges, sums in double
 CASES = [(33, 64, 32, 32, 64, 3, 3, 1, 1), (9, 39, 31, 33, 97, 3, 3, 1, 1), (70, 32, 13, 11, 31, 3, 3, 1, 1), (5, 64, 20, 112, 40, 3, 3, 1, 0), (21, 128, 27, 27, 70, 3, 3, 2, 1),
          (12, 48, 29, 17, 80, 5, 5, 1, 2), (17, 64, 15, 40, 64, 2, 7, 1, 0), (2, 256, 14, 14, 256, 3, 3, 1, 1), (40, 96, 14, 15, 160, 3, 3, 1, 1), (64, 512, 7, 7, 129, 3, 3, 1, 1),
@@ -22,11 +22,11 @@ def _passes(x, w, dy, s, pad):
     return y.detach().numpy(), x64.grad.numpy()
 
 
-def _run(x, w, dy, s, pad, bias=None, beta=0.0, start=0.0, workspace=True, less=0):
+def _run(x, w, dy, s, pad, bias=None, beta=0.0, start=0.0, workspace=True, less=0, choice=0):
     import torch
     from n2d2_amd import capi, runtime as rt
     (B, Ci, H, W), (O, _, kH, kW) = x.shape, w.shape
-    d = capi.ConvDesc(Ci, O, kW, kH, s, s, pad[1], pad[0], pad[1], pad[0], 1, 1, 1, 0, 0)
+    d = capi.ConvDesc(Ci, O, kW, kH, s, s, pad[1], pad[0], pad[1], pad[0], 1, 1, 1, 0, choice)
     dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
     x_, w_, dy_, y, dx = dev(x), dev(w), dev(dy), torch.full(dy.shape, start, device="cuda"), torch.full(x.shape, start, device="cuda")
     b_ = None if bias is None else dev(bias)
@@ -108,6 +108,83 @@ def test_workspaces_of_every_size(case):
             assert (np.abs(g - t) <= 2.0 ** -24 * (np.abs(t) + (k + 4) * m)).all(), less
 
 
+# The kernel's stride-1 instances: tiles of 32 rows x 128 pixels, 64 x 64 and 64 x 128, runs of up to 256 positions (4) and 384 (6), nine taps and any (0), with
+# sums in double and without.  Odd batches, rows, pixels and channels left over, runs of 256, 260 and 384 positions, images with and
+# without rows between them; beside them what the kernel leaves to the others: too much padding of channels, too few flops, runs of 385.
+ROUTES = [((65, 64, 31, 33, 70, 3, 3, 1, 1), "2, 2, 2, 4, 4, 9, false", "2, 2, 2, 4, 4, 9, false"), ((9, 64, 60, 100, 70, 3, 3, 1, 1), "2, 2, 2, 4, 6, 9, false", "2, 2, 2, 4, 6, 9, false"),
+          ((40, 48, 37, 41, 80, 5, 5, 1, 2), "2, 2, 2, 4, 6, 0, false", "2, 2, 2, 4, 6, 0, false"), ((65, 64, 31, 33, 64, 2, 5, 1, 0), "2, 2, 2, 4, 4, 0, false", None),
+          ((22, 256, 28, 28, 64, 1, 5, 1, 2), "2, 2, 2, 2, 4, 0, true", "2, 2, 2, 4, 4, 0, false"), ((22, 160, 28, 28, 64, 9, 1, 1, 4), "2, 2, 2, 2, 6, 0, true", "2, 2, 2, 4, 6, 0, false"),
+          ((4, 160, 43, 100, 64, 3, 3, 1, 1), "2, 2, 2, 2, 6, 9, true", "2, 2, 2, 4, 6, 9, false"), ((40, 96, 14, 15, 160, 3, 3, 1, 1), "2, 2, 2, 2, 4, 9, false", "2, 2, 2, 2, 4, 9, true"),
+          ((6, 64, 22, 100, 48, 3, 3, 1, 1), "2, 2, 2, 2, 6, 9, false", "2, 2, 2, 2, 6, 9, false"), ((12, 48, 29, 17, 80, 5, 5, 1, 2), "2, 2, 2, 2, 4, 0, false", "2, 2, 2, 2, 4, 0, false"),
+          ((9, 47, 31, 33, 97, 3, 3, 1, 1), "2, 2, 2, 2, 4, 9, false", "2, 2, 2, 2, 4, 9, false"), ((5, 256, 14, 14, 256, 3, 3, 1, 1), "2, 2, 2, 2, 4, 9, false", "2, 2, 2, 2, 4, 9, false"),
+          ((3, 64, 40, 159, 40, 3, 3, 1, 1), "2, 2, 2, 2, 6, 9, false", None), ((3, 64, 40, 160, 40, 3, 3, 1, 1), None, None),
+          ((200, 32, 13, 11, 31, 3, 3, 1, 1), "1, 4, 2, 2, 4, 9, false", "1, 4, 2, 2, 4, 9, false"), ((5, 32, 71, 90, 31, 3, 3, 1, 1), "1, 4, 2, 2, 6, 9, false", "1, 4, 2, 2, 6, 9, false"),
+          ((40, 32, 29, 31, 32, 5, 5, 1, 2), "1, 4, 2, 2, 4, 0, false", "1, 4, 2, 2, 4, 0, false"), ((38, 32, 29, 32, 24, 5, 5, 1, 2), "1, 4, 2, 2, 6, 0, false", "1, 4, 2, 2, 6, 0, false"),
+          ((28, 160, 16, 28, 32, 9, 1, 1, 4), "1, 4, 2, 2, 6, 0, false", "2, 2, 2, 2, 6, 0, false"), ((21, 128, 27, 27, 70, 3, 3, 2, 1), "2, 2, 2, 2, 6, 9, false", None),
+          ((9, 39, 31, 33, 97, 3, 3, 1, 1), None, "2, 2, 2, 2, 4, 9, false"), ((70, 32, 13, 11, 31, 3, 3, 1, 1), None, None), ((2, 256, 14, 14, 256, 3, 3, 1, 1), None, None)]
+
+
+def _patch_kernels(log):
+    return [e[0][len("conv_f32_patch_kernel<"):-1] for e in log.entries if e[0].startswith("conv_f32_patch_kernel")]
+
+
+@pytest.mark.parametrize("case,forward,data", ROUTES, ids=str)
+def test_kernel_of_every_tile_and_run(case, forward, data):
+    """The kernel that each pass is to take, and what only that one gives: 5 roundings in 32 terms, of which the rests of channels are some."""
+    from n2d2_amd import capi
+    print("parts, kernels", case, flush=True)
+    x, w, dy, s, pad, rng = _inputs(case, 6)
+    want, T = _passes(x, w, dy, s, pad), w.shape[2] * w.shape[3]
+    with capi.launch_log() as log:
+        got = _run(x, w, dy, s, pad)
+    assert _patch_kernels(log) == [k for k in (forward, data) if k]
+    assert [e[0] for e in log.entries].count("conv_f32_lay_parts_kernel") == (forward is not None) + (data is not None)
+    for g, t, kernel, channels in zip(got, want, (forward, data), (w.shape[1], w.shape[0])):
+        roundings = 5 * -(-channels // 32) * T if kernel else channels * T
+        assert np.linalg.norm(g - t) <= 1.1 * 2.53e-8 * np.sqrt(1 + roundings / 2) * np.linalg.norm(t)
+    bias = rng.normal(size=w.shape[0]).astype(np.float32)
+    y, dx = _run(x, w, dy, s, pad, bias=bias, beta=0.5, start=3.0)
+    assert np.abs(y - (got[0] + np.float32(1.5) + bias[None, :, None, None])).max() <= 2.0 ** -22 * (np.abs(got[0]).max() + 5)
+    assert np.abs(dx - (got[1] + np.float32(1.5))).max() <= 2.0 ** -22 * (np.abs(got[1]).max() + 2)
+
+
+# Forward with room for the laid-out weights alone, which adds all of K in one range: tiles of 32 rows with sums in double
+@pytest.mark.parametrize("case,forward", [((50, 160, 16, 16, 32, 3, 3, 1, 1), "1, 4, 2, 2, 4, 9, true"), ((2, 160, 64, 100, 32, 3, 3, 1, 1), "1, 4, 2, 2, 6, 9, true"),
+                                          ((50, 256, 16, 16, 32, 1, 5, 1, 2), "1, 4, 2, 2, 4, 0, true"), ((28, 160, 16, 28, 32, 9, 1, 1, 4), "1, 4, 2, 2, 6, 0, true")], ids=str)
+def test_rows_of_32_in_one_range(case, forward):
+    from n2d2_amd import capi
+    print("parts, one range", case, flush=True)
+    x, w, dy, s, pad, rng = _inputs(case, 7)
+    want = _passes(x, w, dy, s, pad)[0]
+    with capi.launch_log() as log:
+        got = _run(x, w, dy, s, pad, less=4 * dy.size + 16)[0]
+    assert _patch_kernels(log)[0] == forward
+    assert np.linalg.norm(got - want) <= 1.1 * 2.53e-8 * np.sqrt(1 + 5 * w.shape[1] * w.shape[2] * w.shape[3] / 64) * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("case", [(65, 64, 31, 33, 70, 3, 3, 1, 1), (9, 47, 31, 33, 97, 3, 3, 1, 1), (200, 32, 13, 11, 31, 3, 3, 1, 1)])
+def test_infinities_nan_and_the_largest_floats_of_every_tile(case):
+    """(the kernels of these are in ROUTES)"""
+    assert any(r[0] == case and r[1] and r[2] for r in ROUTES)
+    test_infinities_nan_and_the_largest_floats(case)
+
+
+def test_sums_term_by_term_where_they_are_asked_for():
+    """N2D2HIP_KERNEL_F32_TERMS: forward rounds once a term, on the kernel that has no parts; backward is as without it."""
+    import torch
+    from n2d2_amd import capi, runtime as rt
+    case = (33, 64, 32, 32, 64, 3, 3, 1, 1)
+    print("parts, sums term by term", case, flush=True)
+    x, w, dy, s, pad, rng = _inputs(case, 8)
+    plain = _run(x, w, dy, s, pad)
+    with capi.launch_log() as log:
+        got = _run(x, w, dy, s, pad, choice=capi.KERNEL_F32_TERMS)
+    assert _patch_kernels(log) == ["2, 2, 2, 2, 4, 9, false"]        # (of the data gradient)
+    assert np.array_equal(got[1], plain[1]) and not np.array_equal(got[0], plain[0])
+    want = _passes(x, w, dy, s, pad)[0]
+    assert np.linalg.norm(got[0] - want) <= 1.1 * 2.53e-8 * np.sqrt(1 + 64 * 9 / 2) * np.linalg.norm(want)
+
+
 # Data gradients at stride 2 whose four pixels a place run together: odd and even sizes, rows, channels and pixels left over, 0 to 2 of padding, K
 # ranges, runs of one unit and of two, each beside a neighbour that does not qualify (tiles between the limits, long sums, a step back, few rows)
 FOURS = [((64, 64, 32, 32, 128, 3, 3, 2, 1), 2), ((66, 100, 31, 33, 70, 3, 3, 2, 1), 2), ((12, 70, 31, 30, 390, 3, 3, 2, 1), 2), ((70, 64, 32, 32, 64, 3, 3, 2, 1), 2),
@@ -165,14 +242,19 @@ def _filter64(x, dy, s, pt):
 
 @pytest.mark.parametrize("case", FILTER)
 def test_filter_gradient_against_float64(case):
+    from n2d2_amd import capi
     B, Ci, H, W, O, s, pt = case
     print("parts, filter gradient", case, flush=True)
     rng = np.random.default_rng(sum(case))
     oH, oW = (H + 2 * pt - 3) // s + 1, (W - 1) // s + 1
     assert 2.0 * B * O * oH * oW * Ci * 9 >= 1.5e9
+    octets = -(-oW // 8)                         # a step has 8 of them, 4 at stride 2: the most of a row that leave the fewest beyond its end
+    nol = min(range(4 - s, -1, -1), key=lambda n: -(-octets // 2 ** n) * 2 ** n)
     x, dy = rng.normal(size=(B, Ci, H, W)).astype(np.float32), rng.normal(size=(B, O, oH, oW)).astype(np.float32)
     want, mag = _filter64(x, dy, s, pt), _filter64(np.abs(x), np.abs(dy), s, pt)
-    got = _filter(x, (O, Ci, 3, 3), dy, s, pt)
+    with capi.launch_log() as log:
+        got = _filter(x, (O, Ci, 3, 3), dy, s, pt)
+    assert [e[0] for e in log.entries] == ["conv_f32_filter_rows_kernel<%d, %d>" % (s, nol), "conv_f32_reduce_rows_kernel"]
     # (ranges, of which each is a sum in float, are added in double; one range is at most all pixels: 5 roundings in 32)
     K = B * oH * oW
     assert (np.abs(got - want) <= 2.0 ** -24 * (np.abs(want) + (5 * K / 32 + 4) * mag)).all()
