@@ -1302,7 +1302,8 @@ static PixelClass fours_class(const ConvF32& q)
 // registers they lack); else of 64 x 64.  us, 64 x 128 / 64 x 64, forward: 64 -> 64, 56 x 56, batch 64 (1568 of the larger tiles)
 // 90 / 105; 64 -> 64, 32 x 32, batch 64 (512) 34 / 38; 256 -> 256, 14 x 14, batch 32 (196) 65 / 60; 48 -> 96, 5x5, 30 x 30, batch
 // 16 (226) 54 / 42.  No shape for runs of more than 384 positions, which would leave one block to a CU: 64 -> 128, stride 2, 56 x
-// 56, batch 16 (456) 40 against 31 of the chunk kernel.
+// 56, batch 16 (456) 40 against 31 of the chunk kernel.  (All counts of tiles are for 256 CUs, wherever they run: the order of a sum's
+// additions follows from the sizes alone.)
 static PatchShape patch_shape(const ConvF32& q, int pass, const PixelClass& c)
 {
     const int Q = pass == PASS_FWD ? q.O : q.C, chunks = ceil_div_i(pass == PASS_FWD ? q.C : q.O, PK);
@@ -1375,7 +1376,7 @@ static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass>
     const long blocks = tiles * g.qtiles;
     g.nz = 1;
     if (kind == PIXELS_PATCH) {
-        // ranges (of chunks) where the tiles alone would not give every CU a block
+        // ranges (of chunks) where the tiles alone would not give each of 256 CUs a block
         const int chunks = ceil_div_i(g.Ch, PK);
         const int each = ceil_div_i(chunks, blocks >= 256 ? 1 : std::min<long>(chunks, std::max(1L, 512 / std::max(blocks, 1L))));
         pl.splits = ceil_div_i(chunks, each);
@@ -1417,11 +1418,13 @@ static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass>
     return pl;
 }
 
+// Blocks of the patch kernel: those of all items, or two to a CU that stay for several (a multiple of 8, one to each XCD)
+static unsigned patch_blocks(unsigned items) { return std::min(items, (unsigned)std::max(2 * num_cus() / 8, 1) * 8); }
 template <int WQ, int WP, int MQ, int NP, bool FOLDS>
 static void launch_patch(const PixelPlan& pl, dim3 grid, const float* x, const float* w, const float* wt, const float* bias, float beta, float* out, size_t partial,
                          hipStream_t st)
 {
-    grid.x = std::min(grid.x, 8u * 32u * 2u);    // (two blocks to a CU)
+    grid.x = patch_blocks(grid.x);
     const auto run = [&](auto nu_, auto nt_, auto fold_) {
         constexpr int PB = 2 * decltype(nu_)::value, NT = decltype(nt_)::value;
         constexpr bool FOLD = decltype(fold_)::value;
@@ -1446,7 +1449,7 @@ static void launch_pixels(PixelPlan& pl, int splits, const float* x, const float
     const dim3 grid(pl.g.ptiles8 * 8 * pl.g.qtiles, 1, splits);
     if (pl.kind == PIXELS_PATCH) {
         if (BWD && pl.g.osx == 2) {
-            const dim3 most(std::min(grid.x, 8u * 32u * 2u), 1, grid.z);
+            const dim3 most(patch_blocks(grid.x), 1, grid.z);
             if (pl.patch.nu == 1)
                 N2D2HIP_LAUNCH_T(conv_f32_patch_kernel, (2, 2, 2, 2, 2, 9, false, 4), most, dim3(256), 0, st, pl.g, x, w, (const v4u*)wt, bias, beta, out, partial);
             else
