@@ -526,8 +526,10 @@ int n2d2hip_lsq_backward(const float* diff_q, const float* fp_x, float* diff_fp,
  * Ungrouped convolutions without dilation, of up to 64 taps or spanning their input, run on the matrix cores: forward from
  * 2e7 flops (spanning: up to 64 taps), backward-data (in double where small), and backward-filter (in double below 2e7 flops and for spanning
  * kernels of more than 64 taps).  There sums are added in an order that follows from the sizes, not in the reference's; forward
- * and backward-data of several taps multiply on the bf16 matrix cores, each float as three bf16 numbers that add up to it, where
- * that is faster (infinities and NaN come out as in float).
+ * and backward-data of several taps, and backward-filter of 3x3 kernels, multiply on the bf16 matrix cores where that is faster, each float
+ * as three bf16 numbers that add up to it, whatever its size.  A product is then off by up to 2^-24 of it before the sum is rounded: a sum
+ * of one product that is not zero can be 1.9 half units of the last place from it, where a float product is 1.0 at most; from four products on
+ * sums are nearer to 64 bits than in float.  Infinities and NaN come out as in float.  N2D2HIP_KERNEL_F32_TERMS keeps forward off them.
  * All others, and tensors of 2 GiB and more, run on direct kernels, which add forward and backward-data in the
  * reference's order and backward-filter in double.  kernel_choice N2D2HIP_KERNEL_F32_DIRECT asks for the direct
  * kernels, N2D2HIP_KERNEL_F32_GEMM for the matrix cores at any size.
@@ -552,8 +554,8 @@ size_t n2d2hip_conv2d_f32_workspace_bytes(const n2d2hip_conv_desc* desc, int B, 
 int n2d2hip_conv2d_f32_backward_filter(const n2d2hip_conv_desc* desc, int B, int H, int W, const float* x,
                                        const float* diff_y, float beta, float* diff_w, void* workspace,
                                        size_t workspace_bytes, n2d2hip_stream_t stream);
-/* Both of the above, equal to n2d2hip_conv2d_f32_backward_filter followed by n2d2hip_conv2d_f32_backward_data, bit for bit (small
- * layers that span their input: in one launch). */
+/* Both of the above, equal to n2d2hip_conv2d_f32_backward_filter followed by n2d2hip_conv2d_f32_backward_data, bit for bit (of small
+ * layers, whose two gradients add in double: in one launch, and one more where the weights' sums are split into ranges). */
 int n2d2hip_conv2d_f32_backward(const n2d2hip_conv_desc* desc, int B, int H, int W, const float* x, const float* w,
                                 const float* diff_y, float beta_w, float* diff_w, float beta_x, float* diff_x,
                                 void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream);

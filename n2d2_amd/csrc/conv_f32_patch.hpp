@@ -2,19 +2,21 @@
 //
 // A float is the sum of three bf16 numbers without a rest (8 + 8 + 8 bits of mantissa, each part the rounded rest of the ones
 // before; scaled, so that the parts of small floats keep their bits): a = a0 + a1 + a2.  Of the nine products of a b, a1 b2 and a2 b1 are
-// below 2^-25 of it and a2 b2 below 2^-34: left out, all three are 2^-24.4 of a b at most.  The other six are matrix instructions.  Random data, two waves to a SIMD, register operands only: 16x16x32
-// bf16 2040 TFLOP/s, 340 of six products; 32x32x16 bf16 1350 (two waves in turn slow it down; one alone has 1800); 32x32x2 fp32 98.
+// below 2^-25 of it and a2 b2 below 2^-34: left out, all three are just below 2^-24 of a b at most (a sum of one product that is not zero is off by
+// up to 1.9 half units of the last place, a float product by 1.0; the sums of more terms are below).  The other six are matrix
+// instructions.  Random data, two waves to a SIMD, register operands only: 16x16x32 bf16 2040 TFLOP/s, 340 of six products; 32x32x16
+// bf16 1350 (two waves in turn slow it down; one alone has 1800); 32x32x2 fp32 98.
 // An instruction adds its 32 products to the sum in four roundings: the five smaller products have a sum of their own, which one
 // addition brings to that of the largest, so that a sum is rounded 5 times in 32 terms where the fp32 instructions round it 32
 // times.  Error against 64 bits, random data (forward; before, now): 64 channels, 3x3 4.3e-7, 1.5e-7; 256 channels, 3x3, 14 x 14
 // 3.2e-7, 2.2e-7; 48 channels, 5x5 3.0e-7, 1.7e-7.  All six in one sum: 3.6e-7, 3.5e-7, 3.8e-7.
 //
 // us, forward / data, fp32 matrix cores (conv_f32_3x3_kernel, conv_f32_pixel_kernel), now:
-//   64 -> 64, 3x3, 56 x 56, batch 64            139 / 138     89 /  89
+//   64 -> 64, 3x3, 56 x 56, batch 64            139 / 138     93 /  85
 //   64 -> 64, 3x3, 32 x 32, batch 64             48 /  49     36 /  35
-//   256 -> 256, 3x3, 14 x 14, batch 32          100 /  91     65 /  63
-//   512 -> 512, 3x3, 14 x 14, batch 8           115 / 103     80 /  75
-//   48 -> 96, 5x5, 30 x 30, batch 16             71 /  64     43 /  44
+//   256 -> 256, 3x3, 14 x 14, batch 32          100 /  91     63 /  62
+//   512 -> 512, 3x3, 14 x 14, batch 8           115 / 103     80 /  73
+//   48 -> 96, 5x5, 30 x 30, batch 16             71 /  64     41 /  43
 //   128 -> 256, 3x3 stride 2, 27 x 27, batch 33  53 /         42
 //   256 -> 512, 3x3 stride 2, 28 x 28, batch 8      /  75        /  54      (data: four pixels a place, below)
 //   128 -> 128, 3x3 stride 2, 56 x 56, batch 64     / 152        / 109
