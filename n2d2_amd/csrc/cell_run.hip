@@ -6,9 +6,11 @@
 // a work-group of 8 waves takes one image through all the cells with its tensors in LDS; what a cell hands to the next
 // costs a barrier instead of a launch.  Each cell's output is also stored to its tensor, as the cells run in turn do (the
 // stores wait for nobody), so a caller finds the same values everywhere.  LeNet, conversion of the bytes included: one image
-// 33.9 -> 8.4 us, 256 images launched one by one 45.7 -> 11.4 us.  Of the launch's 8 us, 2 go by until the image and the weights are
-// there, 3 in the first convolution (instruction issue), and the other five cells take about 0.5 each: a descriptor, a few
-// dependent LDS reads and a barrier.  16 waves took as long (each pays for its cells' descriptors and set-up).  With many images
+// 33.9 -> 7.1 us, 256 images launched one by one 45.7 -> 11.2 us (the host's two calls).  Of a launch's 16000 cycles 4200 go by until the image
+// and the weights are there, 2900 in the first convolution (6600 before its pixels went in pairs), and the other cells take 750 to 2200 each: a
+// descriptor, a few dependent LDS reads and a barrier.  16 waves took as long (each pays for its cells' descriptors and set-up); so did
+// the fully-connected weights requested four loads at a time behind the first cells (the compiler waits for them there), and the next
+// cell's descriptor loaded a cell ahead (its registers are spilled).  With many images
 // the cells' own launches fill the chip and overtake it: cells and run, us, 1024 images 56.4 and 35.3, 2048 82.2 and 66.2, 4096 130.1
 // and 127.6, 6144 179.0 and 188.5, 8192 230.7 and 249.8, 16384 458 and 495 (n2d2hip_cell_run_pays).
 //
@@ -37,18 +39,19 @@ namespace n2d2hip {
 
 enum { RUN_CELLS = 8, RUN_THREADS = 512, RUN_WAVES = RUN_THREADS / 64, RUN_LDS = 65536, RUN_TAB = 6 /* bias, a, b, c, d, e */ };
 
-enum { RUN_CONV16, RUN_CONV16_PADDED, RUN_CONV4, RUN_CONV4_PADDED, RUN_POOL, RUN_POOL_PADDED };
+enum { RUN_CONV16, RUN_CONV16_PADDED, RUN_CONV4, RUN_CONV4_PADDED, RUN_POOL, RUN_POOL_PADDED, RUN_CONV4_PAIRS, RUN_CONV4_PAIRS_FAST };
 
 // (What a wave needs before its first pixel is computed by the host as far as it goes: the scalar unit, too, issues one
 // instruction a clock for all waves.)
 struct RunCell {
     int op;                              // RUN_*; padded: some window reaches outside the input
-    int H, W, OW, npix, out_cs;          // input size, output columns and pixels, channel stride of the output
+    int H, W, OW, npix, out_cs;          // input size, output columns and pixels (RUN_CONV4_PAIRS: pairs of them), channel stride of the output
+    int out_bytes;                       // of an image's output
     int in_off, out_off;                 // LDS offsets of the two tensors
     int sx, sy, px, py;                  // stride, padding
     unsigned ow_mul, ow_sh;              // p / OW == p * ow_mul >> ow_sh for every output pixel p, the product below 2^32
     int tap_off;                         // LDS offset of the taps: bytes from the window's origin, or (padded) row << 16 | column.  Convolution:
-                                         // [K step][lane / 16], one (16 channels) or four (4 channels) each; pooling: a multiple of 4
+                                         // [K step][lane / 16], one (16 channels), four (4 channels) or two (pairs: of two columns) each; pooling: a multiple of 4
     int nk;                              // convolution: K steps of 64 bytes (16 channels: a multiple of 4); pooling: groups of 4 taps
     int hop_x;                           // columns between a pixel of a wave's tile and that of its next tile, less than OW
     int hop, wrap, last;                 // the same in bytes of the window's origin, what a step into the next row adds, the last pixel's origin
@@ -252,10 +255,11 @@ __device__ __forceinline__ void run_conv(const RunCell& c, signed char* out, uns
 #pragma unroll
             for (int u = 0; u < N; ++u) {
                 int r[4];
+                // (clamp_i32 on the accumulators: what assembly reads of a matrix instruction's result the compiler does not wait for)
                 if (c.kind == EPI_I24) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                        r[i] = med3_i32((__mul24(med3_i32(acc[u][i], tq[1][i], tq[2][i]), tq[3][i]) + tq[4][i]) >> tq[5][i], c.lo, c.hi);
+                        r[i] = med3_i32((__mul24(clamp_i32(acc[u][i], tq[1][i], tq[2][i]), tq[3][i]) + tq[4][i]) >> tq[5][i], c.lo, c.hi);
                 } else {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
@@ -286,11 +290,142 @@ __device__ __forceinline__ void run_conv(const RunCell& c, signed char* out, uns
     }
 }
 
+// A convolution of 4 channels to at most 8, whose windows lie inside the input: a tile's 16 rows are 8 outputs of a pixel and 8 of the one to its
+// right.  Both windows together are one column (at stride 1) wider than one, which costs no K step where the taps did not fill theirs (5 x 5:
+// 30 of 32), and half as many tiles are read, multiplied and rescaled, with no row of them for outputs that do not exist.  Pairs begin 8 bytes
+// apart, so that a lane's 16 bytes of K are two reads of two columns each, and the weights of the first two steps stay in registers.
+// Bound by the latencies of a tile's chain and by instruction issue: a wave has up to four tiles under way together, and what differs from
+// network to network (the rescale's kind) is decided outside the tiles.  LeNet, one image, us: a pixel a column 8.39, pairs, two tiles
+// at a time 7.71, four and FAST 7.25 (with the poolings' pixels a thread each, and the arguments asked for together, 7.1).
+// FAST: two K steps, rescale EPI_I24
+template <bool FAST>
+__device__ __forceinline__ void run_conv_pairs(const RunCell& c, signed char* out, unsigned char* smem, int wave, int lane)
+{
+    const int l16 = lane & 15, kg = lane >> 4, half = kg >> 1, ch = 4 * (kg & 1);
+    const int ntiles = (c.npix + 15) >> 4;
+    const unsigned char* x = smem + c.in_off;
+    const unsigned char* taps = smem + c.tap_off + kg * 8;
+    const unsigned char* wf = smem + c.w_off + lane * 16;
+    const int* tab = (const int*)(smem + c.tab_off) + ch;
+    // (the host has them be an even number)
+    const v4i w0 = *(const v4i*)wf, w1 = *(const v4i*)(wf + 1024);
+    const v2i t0 = *(const v2i*)taps, t1 = *(const v2i*)(taps + 32);
+    v4i tq[6];
+#pragma unroll
+    for (int r = 0; r < RUN_TAB; ++r)
+        tq[r] = *(const v4i*)(tab + r * 32);
+    const int live = c.O - ch;
+    const unsigned keep = live >= 4 ? 0xffffffffu : live <= 0 ? 0u : (1u << (8 * live)) - 1u;
+    RunPixel<false> px;
+    px.pix = wave * 16 + l16;
+    {
+        const int pc = min(px.pix, c.npix - 1), oy = (int)(__umul24((unsigned)pc, c.ow_mul) >> c.ow_sh);
+        px.ox = pc - __mul24(oy, c.OW);
+        px.iy0 = px.ix0 = 0;
+        px.origin = (__mul24(oy, __mul24(c.sy, c.W)) + __mul24(px.ox, c.sx)) * 4;
+    }
+    // N tiles, RUN_WAVES apart
+    auto tiles = [&](auto n) {
+        constexpr int N = decltype(n)::value;
+        v4i acc[N], p0[N], p1[N];
+        const unsigned char* at[N];
+        int pix[N];
+        auto read = [&](const unsigned char* from, v2i t) {
+            const v2i a = *(const v2i*)(from + t[0]), b = *(const v2i*)(from + t[1]);
+            return v4i{a[0], a[1], b[0], b[1]};
+        };
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            at[u] = x + min(px.origin, c.last);
+            pix[u] = px.pix;
+            p0[u] = read(at[u], t0);
+            p1[u] = read(at[u], t1);
+            px.hop(c);
+        }
+#pragma unroll
+        for (int u = 0; u < N; ++u)
+            acc[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0, p0[u], tq[0], 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < N; ++u)
+            acc[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w1, p1[u], acc[u], 0, 0, 0);
+        if (!FAST) {
+#pragma unroll 1
+            for (int s = 2; s < c.nk; ++s) {
+                const v4i w = *(const v4i*)(wf + s * 1024);
+                const v2i t = *(const v2i*)(taps + s * 32);
+#pragma unroll
+                for (int u = 0; u < N; ++u)
+                    acc[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w, read(at[u], t), acc[u], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            int r[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (FAST) {
+                    r[i] = med3_i32((__mul24(clamp_i32(acc[u][i], tq[1][i], tq[2][i]), tq[3][i]) + tq[4][i]) >> tq[5][i], c.lo, c.hi);
+                } else {
+                    const int tr[RUN_TAB] = {0, tq[1][i], tq[2][i], tq[3][i], tq[4][i], tq[5][i]};
+                    r[i] = run_rescale(tr, c.kind, c.lo, c.hi, c.relu, acc[u][i]);
+                }
+            }
+            const unsigned v = (pack_bytes(r[0], r[1], r[2], r[3]) & keep) ^ c.out_xor;
+            const unsigned to = __umul24((unsigned)(2 * pix[u] + half), (unsigned)c.out_cs);
+            if (c.out_cs == 16) {
+                // channels 0 .. 7 of a pixel in the lanes that have its first four, and 8 .. 15, which hold the stored 0, in the others
+                const auto both = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+                const v2i w2 = ch ? v2i{(int)c.out_xor, (int)c.out_xor} : v2i{(int)both[0], (int)both[1]};
+                if (pix[u] < c.npix) {
+                    *(v2i*)(smem + c.out_off + to + 2 * ch) = w2;
+                    *(v2i*)(out + to + 2 * ch) = w2;
+                }
+            } else if (pix[u] < c.npix && ch == 0) {
+                *(unsigned*)(smem + c.out_off + to) = v;
+                *(unsigned*)(out + to) = v;
+            }
+        }
+    };
+    for (int t = wave; t < ntiles; t += 4 * RUN_WAVES) {
+        const int left = ntiles - t;
+        if (left > 3 * RUN_WAVES) tiles(std::integral_constant<int, 4>());
+        else if (left > 2 * RUN_WAVES) tiles(std::integral_constant<int, 3>());
+        else if (left > RUN_WAVES) tiles(std::integral_constant<int, 2>());
+        else tiles(std::integral_constant<int, 1>());
+    }
+}
+
 // Max pooling, four channels a thread, four taps in flight.  A tap outside the input is replaced by the nearest one inside,
 // which cannot change a maximum; the host knows that every window has one.
 template <bool PADDED>
 __device__ __forceinline__ void run_pool(const RunCell& c, signed char* out, unsigned char* smem, int tid)
 {
+    if (!PADDED && c.out_cs == 16 && c.nk == 1) {
+        // (2 x 2 and the like, 16 channels: a pixel a thread, whose reads are four of 16 bytes in place of sixteen of four)
+        const v4i tap = *(const v4i*)(smem + c.tap_off);
+#pragma unroll 1
+        for (int pix = tid; pix < c.npix; pix += RUN_THREADS) {
+            const int oy = (int)(__umul24((unsigned)pix, c.ow_mul) >> c.ow_sh), ox = pix - __mul24(oy, c.OW);
+            const unsigned char* origin = smem + c.in_off + ((__mul24(__mul24(oy, c.sy), c.W) + __mul24(ox, c.sx)) << 4);
+            v4i w[4], v;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                w[j] = *(const v4i*)(origin + tap[j]);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                v2s me = as_v2s((int)((unsigned)w[0][k] << 8)), mo = as_v2s(w[0][k]);
+#pragma unroll
+                for (int j = 1; j < 4; ++j) {
+                    me = __builtin_elementwise_max(me, as_v2s((int)((unsigned)w[j][k] << 8)));
+                    mo = __builtin_elementwise_max(mo, as_v2s(w[j][k]));
+                }
+                v[k] = (int)((((unsigned)__builtin_bit_cast(int, me) >> 8) & 0x00FF00FFu) | ((unsigned)__builtin_bit_cast(int, mo) & 0xFF00FF00u));
+            }
+            *(v4i*)(smem + c.out_off + 16 * pix) = v;
+            *(v4i*)(out + 16 * pix) = v;
+        }
+        return;
+    }
     const int q = c.out_cs >> 2;                        // 1, 4 or 8
     const int qs = q == 1 ? 0 : q == 4 ? 2 : 3;
     const unsigned char* taps = smem + c.tap_off;
@@ -318,9 +453,9 @@ __device__ __forceinline__ void run_pool(const RunCell& c, signed char* out, uns
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                // a signed byte in the high half of each 16 bits: the 16-bit maximum orders them as bytes
-                me = __builtin_elementwise_max(me, as_v2s((int)((w[j] << 8) & 0xFF00FF00u)));
-                mo = __builtin_elementwise_max(mo, as_v2s((int)(w[j] & 0xFF00FF00u)));
+                // a signed byte in the high half of each 16 bits: the 16-bit maximum orders them as bytes, whatever the low halves hold
+                me = __builtin_elementwise_max(me, as_v2s((int)(w[j] << 8)));
+                mo = __builtin_elementwise_max(mo, as_v2s((int)w[j]));
             }
             if (++k >= c.nk)
                 break;
@@ -350,18 +485,11 @@ __global__ __launch_bounds__(RUN_THREADS) void cell_run_kernel(const CellRunArgs
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = blockIdx.x;
+    // (what the first loads need of the arguments, asked for together: one after the other, each waits for the last)
+    asm volatile("" ::"s"(q.in), "s"(q.edge), "s"(q.in_w), "s"(q.edge_xor), "s"(q.in_cs), "s"(q.C), "s"(q.H), "s"(q.W), "s"(q.blob), "s"(q.blob_bytes),
+                 "s"(q.in_off), "s"(q.nfc), "s"(q.kper), "s"(q.fc_w[0]), "s"(q.fc_w[1]), "s"(q.fc_w[FC_CHAIN_MAX - 1]));
     // (the plan does not change while kernels run: scalar loads)
     const auto* plan = (const RunPlan __attribute__((address_space(4)))*)(unsigned long long)q.blob;
-    // What is read by scalar loads later on is touched here, a word of every 64 bytes, while the image is on its way: the
-    // arguments lie in host memory, the plan in the device's, and each miss would hold all waves up (2000 and 500 cycles).
-    if (wave == 0) {
-        int touched = 0;
-#pragma unroll
-        for (unsigned i = 0; i < sizeof(RunPlan) / 4; i += 16)
-            touched |= ((const int __attribute__((address_space(4)))*)plan)[i];
-        asm volatile("" ::"s"(touched), "s"(q.outs[0]), "s"(q.outs[RUN_CELLS - 1]), "s"(q.out), "s"(q.x_off), "s"(q.kper));
-    }
-
     // ---- the image, the convolutions' weights and all tables
     for (int c = wave; c < q.blob_bytes / 1024; c += RUN_WAVES)
         __builtin_amdgcn_global_load_lds((gbl_ptr_t)(q.blob + c * 1024 + lane * 16), (lds_ptr_t)(smem + c * 1024), 16, 0, 0);
@@ -412,6 +540,17 @@ __global__ __launch_bounds__(RUN_THREADS) void cell_run_kernel(const CellRunArgs
             for (int j = 0; j < 2; ++j)
                 wn[l - 1][j] = *((const v4i*)(q.blob + q.fc_w[l]) + (wave * 2 + j) * 64 + lane);
     }
+    // What is read by scalar loads later on is touched here, a word of every 64 bytes, while the image is on its way (behind its loads:
+    // ahead of them it held them up by a microsecond): the arguments lie in host memory, the plan in the device's, and each miss would
+    // hold all waves up (2000 and 500 cycles).
+    {
+        constexpr int LINES = (sizeof(RunPlan) + 63) / 64;
+        int touched = 0;
+#pragma unroll
+        for (int i = 0; i < LINES; i += RUN_WAVES)          // (each wave an eighth of the plan)
+            touched |= ((const int __attribute__((address_space(4)))*)plan)[min(i + wave, LINES - 1) * 16];
+        asm volatile("" ::"s"(touched), "s"(q.outs[0]), "s"(q.outs[RUN_CELLS - 1]), "s"(q.out), "s"(q.x_off), "s"(q.kper));
+    }
 #pragma unroll
     for (int j = 0; j < AHEAD; ++j)
         if (tid + j * RUN_THREADS < words)
@@ -428,12 +567,14 @@ __global__ __launch_bounds__(RUN_THREADS) void cell_run_kernel(const CellRunArgs
 
     for (int i = 0; i < q.ncells; ++i) {
         const RunCell c = scalar_load(&plan->cell[i]);
-        signed char* out = q.outs[i] + (size_t)b * (unsigned)(c.npix * c.out_cs);
+        signed char* out = q.outs[i] + (size_t)b * (unsigned)c.out_bytes;
         switch (c.op) {
         case RUN_CONV16: run_conv<16, false>(c, out, smem, wave, lane); break;
         case RUN_CONV16_PADDED: run_conv<16, true>(c, out, smem, wave, lane); break;
         case RUN_CONV4: run_conv<4, false>(c, out, smem, wave, lane); break;
         case RUN_CONV4_PADDED: run_conv<4, true>(c, out, smem, wave, lane); break;
+        case RUN_CONV4_PAIRS: run_conv_pairs<false>(c, out, smem, wave, lane); break;
+        case RUN_CONV4_PAIRS_FAST: run_conv_pairs<true>(c, out, smem, wave, lane); break;
         case RUN_POOL: run_pool<false>(c, out, smem, tid); break;
         default: run_pool<true>(c, out, smem, tid); break;
         }
@@ -573,7 +714,7 @@ int n2d2hip_cell_run_create(int nb_cells, const n2d2hip_run_cell* cells, int H, 
         }
         c.H = h; c.W = w;
         int OH, OW, taps, kW, dy = 1, dx = 1, listed;
-        bool padded;
+        bool padded, pairs = false;
         const int in_cs = cs;
         if (cv) {
             const n2d2hip_conv_desc& d = cv->desc;
@@ -593,6 +734,13 @@ int n2d2hip_cell_run_create(int nb_cells, const n2d2hip_run_cell* cells, int H, 
             listed = c.nk * (cs == 4 ? 16 : 4);
             c.O = d.O; c.mblocks = (d.O + 15) / 16;
             padded = d.padL > 0 || d.padT > 0 || (OH - 1) * d.strideY - d.padT + (d.kH - 1) * d.dilY >= h || (OW - 1) * d.strideX - d.padL + (d.kW - 1) * d.dilX >= w;
+            // two columns of a window to a read; the K steps of a pair are no more than those of two pixels
+            const int columns = (d.kW + d.strideX + 1) / 2, pair_steps = round_up((d.kH * columns + 7) / 8, 2);
+            pairs = cs == 4 && d.O <= 8 && !padded && OW % 2 == 0 && w % 2 == 0 && dy == 1 && dx == 1 && pair_steps <= 2 * c.nk;
+            if (pairs) {
+                c.nk = pair_steps;
+                listed = c.nk * 8;
+            }
             c.kind = cv->act->args.kind; c.lo = cv->act->args.lo; c.hi = cv->act->args.hi; c.relu = cv->act->args.relu;
             c.fill = stored_zero(dtype);
             // weights as matrix-core fragments: [block of 16 outputs][K step][lane][16 bytes], lane l output l % 16, bytes 16 * (l / 16) of the step
@@ -604,7 +752,12 @@ int n2d2hip_cell_run_create(int nb_cells, const n2d2hip_run_cell* cells, int H, 
                 for (int s = 0; s < c.nk; ++s)
                     for (int l = 0; l < 64; ++l)
                         for (int k = 0; k < 16; ++k) {
-                            const int o = 16 * mb + (l & 15), kb = 64 * s + 16 * (l >> 4) + k, tap = kb / cs;
+                            int o = 16 * mb + (l & 15), kb = 64 * s + 16 * (l >> 4) + k, tap = kb / cs;
+                            if (pairs) {        // (column 2 (tap / 2 % columns) + tap % 2 of the first pixel's window)
+                                const int x = 2 * (tap / 2 % columns) + tap % 2 - (o >= 8 ? d.strideX : 0), y = tap / 2 / columns;
+                                tap = y < d.kH && x >= 0 && x < d.kW ? y * d.kW + x : taps;
+                                o &= 7;
+                            }
                             if (o < d.O && tap < taps)
                                 blob[(size_t)c.w_off + ((size_t)(mb * c.nk + s) * 64 + l) * 16 + k] = img[((size_t)tap * rows + o) * cs + kb % cs];
                         }
@@ -629,19 +782,26 @@ int n2d2hip_cell_run_create(int nb_cells, const n2d2hip_run_cell* cells, int H, 
         }
         N2D2HIP_RUN_NEEDS(cs == 4 || cs == 16 || cs == 32, "a tensor has more than 32 channels");
         N2D2HIP_RUN_NEEDS((long long)OH * OW * cs <= RUN_LDS, "a tensor does not fit");
-        c.OW = OW; c.npix = OH * OW; c.out_cs = cs;
-        c.op = (cv ? (in_cs == 16 ? RUN_CONV16 : RUN_CONV4) : RUN_POOL) + (padded ? 1 : 0);
-        const int hop_y = RUN_WAVES * 16 / OW;
-        c.hop_x = RUN_WAVES * 16 % OW;
+        c.out_bytes = OH * OW * cs; c.out_cs = cs;
+        const int columns_out = pairs ? OW / 2 : OW;
+        if (pairs) c.sx *= 2;
+        c.OW = columns_out; c.npix = OH * columns_out;
+        c.op = pairs ? (c.nk == 2 && c.kind == EPI_I24 ? RUN_CONV4_PAIRS_FAST : RUN_CONV4_PAIRS) : (cv ? (in_cs == 16 ? RUN_CONV16 : RUN_CONV4) : RUN_POOL) + (padded ? 1 : 0);
+        const int hop_y = RUN_WAVES * 16 / columns_out;
+        c.hop_x = RUN_WAVES * 16 % columns_out;
         c.hop = (hop_y * c.sy * w + c.hop_x * c.sx) * in_cs;
-        c.wrap = (c.sy * w - OW * c.sx) * in_cs;
-        c.last = ((OH - 1) * c.sy * w + (OW - 1) * c.sx) * in_cs;
+        c.wrap = (c.sy * w - columns_out * c.sx) * in_cs;
+        c.last = ((OH - 1) * c.sy * w + (columns_out - 1) * c.sx) * in_cs;
         c.hop_y = hop_y * c.sy;
         // K position (step, lane / 16, i) is tap 4 * step + lane / 16, or with 4 channels tap 16 * step + 4 * (lane / 16) + i; behind the
         // last tap it is listed again (a convolution has zero weights there, a maximum does not change)
         std::vector<int> tap(listed);
         for (int t = 0; t < listed; ++t) {
-            const int k = std::min(t, taps - 1), ty = k / kW * dy, tx = k % kW * dx;
+            int k = std::min(t, taps - 1), ty = k / kW * dy, tx = k % kW * dx;
+            if (pairs) {            // (pairs of columns; behind the last one: of the last)
+                const int columns = (kW + c.sx / 2 + 1) / 2;
+                k = std::min(t, columns * (taps / kW) - 1); ty = k / columns; tx = 2 * (k % columns);
+            }
             tap[t] = padded ? ty << 16 | tx : (ty * w + tx) * in_cs;
         }
         c.tap_off = (int)blob.size();
@@ -650,10 +810,10 @@ int n2d2hip_cell_run_create(int nb_cells, const n2d2hip_run_cell* cells, int H, 
         // (at most 16384 pixels: tried on every one of them)
         bool divides = false;
         for (c.ow_sh = 8; c.ow_sh <= 22 && !divides; ++c.ow_sh) {
-            c.ow_mul = (1u << c.ow_sh) / (unsigned)OW + 1u;
-            divides = (unsigned long long)c.ow_mul * (unsigned)(OH * OW) < (1ull << 32);
-            for (unsigned p = 0; p < (unsigned)(OH * OW) && divides; ++p)
-                divides = (p * c.ow_mul) >> c.ow_sh == p / (unsigned)OW;
+            c.ow_mul = (1u << c.ow_sh) / (unsigned)c.OW + 1u;
+            divides = (unsigned long long)c.ow_mul * (unsigned)c.npix < (1ull << 32);
+            for (unsigned p = 0; p < (unsigned)c.npix && divides; ++p)
+                divides = (p * c.ow_mul) >> c.ow_sh == p / (unsigned)c.OW;
         }
         --c.ow_sh;
         N2D2HIP_RUN_NEEDS(divides, "a tensor's rows do not divide");

@@ -68,6 +68,25 @@ def test_cells_in_one_launch_bit_exact(case, batch):
         assert np.array_equal(run.input.buf.cpu().numpy(), apart.input.buf.cpu().numpy())
 
 
+# Pairs of pixels a column of the matrix instruction: convolutions of 4 channels to at most 8 outputs, unpadded, rows of even length in and out
+PAIRS = [
+    # one tile and one pair behind it (17 pairs), 8 outputs, stride 1; then the same from a row of its own (1 x 2 pixels)
+    ("eight_of_five", (4, 5, 38), True, "FixedMult32", [("conv", 8, 5, 1, 0), ("conv", 4, 1, 1, 0), ("conv", 3, 1, 1, 0)]),
+    # three outputs (a channel stride of 4), float rescale, four K steps; a pair alone
+    ("three_of_seven", (1, 7, 8), False, "FloatMult", [("conv", 3, 7, 1, 0), ("conv", 5, 1, 1, 0), ("fc", 12), ("fc", 6)]),
+    # strides 2 and 3, 64-bit rescale; more tiles than two a wave
+    ("stride_two", (3, 40, 42), True, "DoubleShift", [("conv", 4, 4, 2, 0), ("pool", 2, 2, 0), ("conv", 5, 3, 1, 0)]),
+    ("stride_three", (2, 32, 50), True, "FixedMult16", [("conv", 6, 5, 3, 0), ("pool", 2, 2, 0), ("fc", 12), ("fc", 9)]),
+    ("last_pair_of_two", (1, 37, 34), True, "SingleShift", [("conv", 6, 3, 1, 0), ("pool", 2, 2, 0), ("conv", 16, 3, 1, 0)]),
+]
+
+
+@pytest.mark.parametrize("batch", [1, 3])
+@pytest.mark.parametrize("case", PAIRS, ids=[c[0] for c in PAIRS])
+def test_pairs_of_pixels_bit_exact(case, batch):
+    test_cells_in_one_launch_bit_exact(case, batch)
+
+
 def test_run_is_planned_up_to_sixteen_images_a_compute_unit():
     import torch
     from n2d2_amd import nets, runtime as rt
