@@ -66,6 +66,7 @@ struct PixelClass {
     int y0, x0;                // source position of tap (0, 0) for grid pixel (0, 0)
     int stepy, stepx;          // element offset from one tap to the next in the source plane
     int soff0, bias;           // element offset of tap (0, 0) against the moved base `src - bias`; both make every offset >= 0
+    int w0;                    // conv_f32_taps_kernel: steps of the classes before this one
     int ry, rx;                // output position of grid pixel (py, px): (py * osy + ry, px * osx + rx)
     DivF32 ghw, gw, nt, nxd;
 };

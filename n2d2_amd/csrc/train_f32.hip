@@ -13,6 +13,7 @@
 #include "common.h"
 #include "conv_f32_gemm.hpp"
 #include "conv_f32_patch.hpp"
+#include "conv_f32_taps.hpp"
 #include "conv_f32_filter_rows.hpp"
 #include "sat_math.hpp"
 #include "depthwise_f32.hpp"
@@ -1219,7 +1220,8 @@ struct PixelPlan {
     bool small_q;              // tiles of 32 q x 128 pixels instead of 64 x 64
     int splits;                // K ranges that leave partial results
     int kind;                  // PIXELS_*
-    PatchShape patch;          // (PIXELS_PATCH)
+    PatchShape patch;          // (PIXELS_PATCH, PIXELS_PARTS)
+    bool chunks;               // (PIXELS_PARTS) a step is channels at one tap
     bool many;                 // a class has more tap rows and columns than a mask of 31 bits
     PixelGemm g;
 };
@@ -1264,7 +1266,7 @@ static std::vector<PixelClass> pixel_classes(const ConvF32& q, int pass)
     return v;
 }
 
-enum { PIXELS_TAPS, PIXELS_CHUNK, PIXELS_3X3, PIXELS_PATCH };
+enum { PIXELS_TAPS, PIXELS_CHUNK, PIXELS_3X3, PIXELS_PATCH, PIXELS_PARTS };
 // Units of 128 source positions that hold what the taps of any `pixels` consecutive pixels of the class read: every step to the
 // next pixel is at least 0 and at most one of a row's, a row's end's and an image's end's.  0: a step back.
 static int patch_units(const ConvF32& q, int pass, const PixelClass& c, int pixels)
@@ -1333,6 +1335,33 @@ static PatchShape patch_shape(const ConvF32& q, int pass, const PixelClass& c)
     }
     return fit(PatchShape{2, 2, 2, 2, 0});
 }
+// conv_f32_taps_kernel: whether a step is 32 channels at one tap, and the steps of a class
+static bool taps_chunks(const ConvF32& q, int pass) { const int ch = pass == PASS_FWD ? q.C : q.O; return round_up(ch, PK) * 5 <= ch * 6; }
+static int taps_steps(const ConvF32& q, int pass, const PixelClass& c)
+{
+    const int ch = pass == PASS_FWD ? q.C : q.O;
+    return taps_chunks(q, pass) ? ceil_div_i(ch, PK) * c.nT : ceil_div_i((long)ch * c.nT, PK);
+}
+// Steps after which its float sums go to those in double: as patch_fold
+static int taps_fold(const ConvF32& q, int pass)
+{
+    const bool fwd = pass == PASS_FWD;
+    const long K = (long)(fwd ? q.C : q.O) * q.kH * q.kW;
+    return (int)std::max(4 * (K / pass_ranges((long)q.B * (fwd ? q.oH * q.oW : q.H * q.W), fwd ? q.O : q.C, K)) / PK, 1L);
+}
+// Tiles of 128 rows x 64 pixels, whose waves read each weight once and take each value of the source apart for twice as many products, where they fill
+// 128 rows and give every CU a block or K is long enough to be split; of 64 x 64 else, and where several classes of different length share
+// the chip.  us, 128 / 64 rows: forward 164 -> 377, 5x5 stride 2, 9 x 85, batch 16 (162 blocks of 128 rows, K 4100) 99 / 124; 64 -> 256, 1x1, 56 x 56,
+// batch 64 (6272) 87 / 95; 1024 -> 256, 1x1, 14 x 14, batch 32 (196, K 1024) 45 / 40; 512 -> 2048, 7 x 7, batch 16 (208, K 512) 39 / 31; data 128 <- 256, 3x3
+// stride 2, 27 x 27, batch 33, four classes 48.6 / 46.6.
+static PatchShape taps_shape(const ConvF32& q, int pass, const std::vector<PixelClass>& cls)
+{
+    const int Q = pass == PASS_FWD ? q.O : q.C;
+    if (Q <= 16) return PatchShape{1, 4, 1, 2, 0};
+    if (Q <= 32) return PatchShape{1, 4, 2, 2, 0};
+    const long blocks = (long)ceil_div_i(cls[0].P, 64) * ceil_div_i(Q, 128), K = (long)(pass == PASS_FWD ? q.C : q.O) * cls[0].nT;
+    return cls.size() == 1 && round_up(Q, 128) * 8 <= round_up(Q, 64) * 9 && (blocks >= 256 || K >= 2048) ? PatchShape{4, 1, 2, 4, 0} : PatchShape{2, 2, 2, 2, 0};
+}
 static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass> cls, int kind)
 {
     PixelPlan pl = {};
@@ -1357,7 +1386,9 @@ static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass>
     // over 32 that was timed, and gained up to 70 % where the larger tiles are few)
     pl.small_q = g.Q <= 32;
     if (kind == PIXELS_PATCH) pl.patch = patch_shape(q, pass, cls[0]);
-    const int PT = kind == PIXELS_PATCH ? pl.patch.pixels() : pl.small_q ? 128 : 64, QT = kind == PIXELS_PATCH ? pl.patch.rows() : pl.small_q ? 32 : 64;
+    if (kind == PIXELS_PARTS) pl.patch = taps_shape(q, pass, cls);
+    const bool parts = kind == PIXELS_PATCH || kind == PIXELS_PARTS;
+    const int PT = parts ? pl.patch.pixels() : pl.small_q ? 128 : 64, QT = parts ? pl.patch.rows() : pl.small_q ? 32 : 64;
     g.qtiles = ceil_div_i(g.Q, QT);
     pl.kind = kind;
     g.T = T;
@@ -1385,6 +1416,25 @@ static PixelPlan plan_pixels(const ConvF32& q, int pass, std::vector<PixelClass>
         g.c[0] = cls[0];
         g.c[0].kchunk = each;
         g.c[0].fold = fold < each ? fold : 0;
+        return pl;
+    }
+    if (kind == PIXELS_PARTS) {
+        int most = 1, w0 = 0;
+        for (const PixelClass& c : cls) most = std::max(most, taps_steps(q, pass, c));
+        const int fold = taps_fold(q, pass);
+        pl.chunks = taps_chunks(q, pass);
+        // (ranges of four steps at least, where the tiles alone would not give each of 256 CUs a block)
+        const int splits = blocks >= 256 ? 1 : (int)std::max(1L, std::min<long>(512 / std::max(blocks, 1L), most / 4));
+        const int each = ceil_div_i(most, splits);
+        pl.splits = ceil_div_i(most, each);
+        for (int i = 0; i < g.nclass; ++i) {
+            g.c[i] = cls[i];
+            g.c[i].w0 = w0;
+            const int steps = taps_steps(q, pass, cls[i]);
+            w0 += steps;
+            g.c[i].kchunk = std::max(ceil_div_i(steps, pl.splits), 1);
+            g.c[i].fold = fold < each ? fold : 0;
+        }
         return pl;
     }
     long splits, least = q.ranges;
@@ -1458,6 +1508,28 @@ static void launch_pixels(PixelPlan& pl, int splits, const float* x, const float
         } else if (pl.patch.wq == 1) launch_patch<1, 4, 2, 2, true>(pl, grid, x, w, wt, bias, beta, out, partial, st);
         else if (pl.patch.np == 2) launch_patch<2, 2, 2, 2, true>(pl, grid, x, w, wt, bias, beta, out, partial, st);
         else launch_patch<2, 2, 2, 4, false>(pl, grid, x, w, wt, bias, beta, out, partial, st);
+        return;
+    }
+    if (pl.kind == PIXELS_PARTS) {
+        const auto run = [&](auto wq_, auto mq_, auto np_, auto chunk_, auto fold_) {
+            constexpr int WQ = decltype(wq_)::value, MQ = decltype(mq_)::value, NP = decltype(np_)::value;
+            constexpr bool CHUNK = decltype(chunk_)::value, FOLD = decltype(fold_)::value;
+            N2D2HIP_LAUNCH_T(conv_f32_taps_kernel, (WQ, 4 / WQ, MQ, NP, CHUNK, FOLD), grid, dim3(256), 0, st, pl.g, x, w, (const v4u*)wt, bias, beta, out, partial);
+        };
+        using I1 = std::integral_constant<int, 1>;
+        using I2 = std::integral_constant<int, 2>;
+        using I4 = std::integral_constant<int, 4>;
+        const auto shape = [&](auto chunk_, auto fold_) {
+            if (pl.patch.wq == 4) run(I4{}, I2{}, I4{}, chunk_, fold_);
+            else if (pl.patch.wq == 1 && pl.patch.mq == 1) run(I1{}, I1{}, I2{}, chunk_, fold_);
+            else if (pl.patch.wq == 1) run(I1{}, I2{}, I2{}, chunk_, fold_);
+            else run(I2{}, I2{}, I2{}, chunk_, fold_);
+        };
+        const auto folds = [&](auto chunk_) {
+            if (pl.g.c[0].fold) shape(chunk_, std::true_type{});
+            else shape(chunk_, std::false_type{});
+        };
+        pl.chunks ? folds(std::true_type{}) : folds(std::false_type{});
         return;
     }
     if (pl.kind != PIXELS_TAPS) w = wt;
@@ -1642,6 +1714,13 @@ static int pixels_kind(const ConvF32& q, int pass)
         if (patch_fours(q, pass) ? patch_shape(q, pass, fours_class(q)).nu
             : (pass == PASS_FWD || (q.sx == 1 && q.sy == 1)) && patch_shape(q, pass, pixel_classes(q, pass)[0]).nu) return PIXELS_PATCH;
     }
+    // The other large ones whose K is more than a few steps: conv_f32_taps_kernel, but where a third of a tile's rows is empty (17 <- 253, 5x5: 149 us, pixel
+    // kernel 140).  us, fp32 kernels / this: below the rule 33 -> 79, 3x3, 55 x 72, batch 6, 1.1e9 flops 23.7 / 27.4; 16 -> 54, 3x3, 97 x 27, batch 14, 5.7e8
+    // 15.4 / 22; 64 -> 64, 1x1, 56 x 56, batch 64, K 64 31.2 / 31; others at the kernel.
+    const int rows = pass == PASS_FWD ? q.O : q.C;
+    if (!(pass == PASS_FWD && (q.choice & N2D2HIP_KERNEL_F32_TERMS)) && q.kH + q.kW <= 31 && !q.ranges && q.sx * q.sy <= PIXEL_CLASSES
+        && 2.0 * q.B * q.O * q.oH * q.oW * q.C * T >= 1.5e9 && (long)ch * T >= 200 && (rows <= 16 || rows >= 22))
+        return PIXELS_PARTS;
     if (q.kH == 3 && q.kW == 3 && (pass == PASS_FWD || (q.sx == 1 && q.sy == 1)) && round_up(ch, 4) * 5 <= ch * 7)
         return PIXELS_3X3;
     return (pass == PASS_BWD_DATA || T == 1 || q.kH + q.kW > 31) && round_up(ch, GK) * 5 <= ch * 6 ? PIXELS_CHUNK : PIXELS_TAPS;
@@ -1654,6 +1733,12 @@ static size_t laid_weights(const ConvF32& q, int pass, int kind)
 {
     const int ch = pass == PASS_FWD ? q.C : q.O, rows = pass == PASS_FWD ? q.O : q.C, qpad = round_up(rows, rows <= 32 ? 32 : 64);
     if (kind == PIXELS_TAPS) return 0;
+    if (kind == PIXELS_PARTS) {
+        const std::vector<PixelClass> cls = pixel_classes(q, pass);
+        size_t steps = 0;
+        for (const PixelClass& c : cls) steps += taps_steps(q, pass, c);
+        return steps * (round_up(rows, taps_shape(q, pass, cls).rows()) / 16) * (PATCH_FRAG / 4);
+    }
     if (kind == PIXELS_PATCH) return (size_t)ceil_div_i(ch, PK) * q.kH * q.kW * (round_up(rows, 128) / 16) * (PATCH_FRAG / 4);
     return kind == PIXELS_3X3 ? (size_t)(ch + 3) / 4 * qpad * W33 : (size_t)round_up(ch, GK) * q.kH * q.kW * qpad;
 }
@@ -1720,12 +1805,15 @@ static int run_pass(const ConvF32& q, int pass, const float* a, const float* b, 
     const float* wt = ws;
     if (kind != PIXELS_TAPS) {
         const PixelGemm& g = plans[0].g;
-        const int total = (int)(kind == PIXELS_3X3 ? nlaid : kind == PIXELS_PATCH ? nlaid / 12 : nlaid / 4);
+        const int total = (int)(kind == PIXELS_3X3 ? nlaid : kind == PIXELS_PATCH || kind == PIXELS_PARTS ? nlaid / 12 : nlaid / 4);
         const dim3 grid(std::min((total + 255) / 256, 4096));
         if (kind == PIXELS_3X3) hipLaunchKernelGGL(conv_f32_lay_weights3x3_kernel, grid, dim3(256), 0, st, b, ws, total, g.Q, g.qpad, g.Ch, g.qs, g.chs);
         else if (kind == PIXELS_PATCH)
             N2D2HIP_LAUNCH(conv_f32_lay_parts_kernel, grid, dim3(256), 0, st, b, (v4u*)ws, total, g.Q, g.qpad / 16, g.Ch, g.T, g.qs, g.chs);
-        else hipLaunchKernelGGL(conv_f32_lay_weights_kernel, grid, dim3(256), 0, st, b, ws, total, g.Q, g.qpad, g.Ch, g.T, g.qs, g.chs);
+        else if (kind == PIXELS_PARTS) {
+            if (plans[0].chunks) N2D2HIP_LAUNCH_T(conv_f32_lay_taps_kernel, (true), grid, dim3(256), 0, st, g, b, (v4u*)ws, total);
+            else N2D2HIP_LAUNCH_T(conv_f32_lay_taps_kernel, (false), grid, dim3(256), 0, st, g, b, (v4u*)ws, total);
+        } else hipLaunchKernelGGL(conv_f32_lay_weights_kernel, grid, dim3(256), 0, st, b, ws, total, g.Q, g.qpad, g.Ch, g.T, g.qs, g.chs);
         ws += nlaid;
         ws_floats -= nlaid;
     }
@@ -1735,6 +1823,14 @@ static int run_pass(const ConvF32& q, int pass, const float* a, const float* b, 
                 const int fold = patch_fold(q, pass, cls[0]), chunks = ceil_div_i(pl.g.Ch, PK);
                 pl.g.c[0].kchunk = chunks;
                 pl.g.c[0].fold = fold < chunks ? fold : 0;
+            } else if (kind == PIXELS_PARTS) {
+                const int fold = taps_fold(q, pass);
+                int most = 0;
+                for (int i = 0; i < pl.g.nclass; ++i) {
+                    pl.g.c[i].kchunk = taps_steps(q, pass, pl.g.c[i]);
+                    most = std::max(most, pl.g.c[i].kchunk);
+                }
+                for (int i = 0; i < pl.g.nclass; ++i) pl.g.c[i].fold = fold < most ? fold : 0;
             } else {
                 pl.g.nz *= pl.splits;
             }
