@@ -1,4 +1,6 @@
 // Float cells of the Frame_HIP model for quantization-aware training (see frame_hip_train.hpp).
+#include <cstring>
+
 #include <hip/hip_runtime_api.h>
 
 #include "frame_hip_train.hpp"
@@ -69,6 +71,39 @@ void DeviceFloats::toHost(float* host, size_t n) const
     if (n != size())
         throw std::runtime_error("DeviceFloats::toHost(): size mismatch");
     checkHipT(hipMemcpy(host, mData, n * sizeof(float), hipMemcpyDeviceToHost), "DeviceFloats::toHost()");
+}
+
+// -------------------------------------------------------------- PinnedFloats
+PinnedFloats::~PinnedFloats()
+{
+    if (mData) (void)hipHostFree(mData);
+}
+
+void PinnedFloats::reserve(size_t n)
+{
+    if (n <= mSize)
+        return;
+    if (mData) (void)hipHostFree(mData);
+    mData = nullptr;
+    mSize = 0;
+    checkHipT(hipHostMalloc((void**)&mData, n * sizeof(float), hipHostMallocDefault), "PinnedFloats::reserve()");
+    mSize = n;
+}
+
+void PinnedFloats::read(float* host, const float* device, size_t n, void* stream)
+{
+    hipStream_t st = (hipStream_t)stream;
+    if (n <= FEW || n > READ) {
+        if (st) checkHipT(hipStreamSynchronize(st), "PinnedFloats::read()");
+        checkHipT(hipMemcpy(host, device, n * sizeof(float), hipMemcpyDeviceToHost), "PinnedFloats::read()");
+        return;
+    }
+    std::lock_guard<std::mutex> lock(mReading);
+    reserve(READ);
+    const hipError_t copied = hipMemcpyAsync(mData, device, n * sizeof(float), hipMemcpyDeviceToHost, st);
+    const hipError_t waited = hipStreamSynchronize(st);      // (also where the copy failed: nothing writes here afterwards)
+    checkHipT(copied != hipSuccess ? copied : waited, "PinnedFloats::read()");
+    std::memcpy(host, mData, n * sizeof(float));
 }
 
 // -------------------------------------------------------- Cell_FrameTrain_HIP
@@ -283,6 +318,13 @@ void WeightedCell_FrameTrain_HIP::updateWeighted(bool noBias)
     if (mQuantizer)
         mQuantizer->update(batch);
     activationUpdate();
+}
+
+void WeightedCell_FrameTrain_HIP::readWeights(float* host, size_t n, PinnedFloats& through) const
+{
+    if (n != mDevW.size())
+        throw std::runtime_error("DeviceFloats::toHost(): size mismatch");
+    through.read(host, mDevW.data(), n, mStream);
 }
 
 Tensor<Float_T> WeightedCell_FrameTrain_HIP::getQuantizedWeights() const
@@ -526,12 +568,12 @@ std::vector<Float_T> BatchNormCell_FrameTrain_HIP<T>::get(const DeviceFloats& de
 }
 
 template <class T>
-void BatchNormCell_FrameTrain_HIP<T>::readParameters(float* host) const
+void BatchNormCell_FrameTrain_HIP<T>::readParameters(float* host, PinnedFloats& through) const
 {
     if (mParameters.empty())
         throw std::runtime_error("BatchNormCell_FrameTrain_HIP " + mName + ": readParameters() before initialize()");
-    checkHipT(hipStreamSynchronize((hipStream_t)mStream), "BatchNormCell_FrameTrain_HIP: synchronize");
-    const Tensor<Float_T> all = mParameters.toHost();
+    std::vector<Float_T> all(mParameters.size());
+    through.read(all.data(), mParameters.data(), all.size(), mStream);
     for (size_t k = 0; k < 6; ++k)
         std::copy(all.data() + k * parameterStride(), all.data() + k * parameterStride() + mNbOutputs, host + k * mNbOutputs);
 }

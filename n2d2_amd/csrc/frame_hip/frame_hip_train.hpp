@@ -8,6 +8,8 @@
 #ifndef N2D2_FRAME_HIP_TRAIN_HPP
 #define N2D2_FRAME_HIP_TRAIN_HPP
 
+#include <mutex>
+
 #include "frame_hip.hpp"
 
 namespace N2D2 {
@@ -46,6 +48,28 @@ private:
     bool mValid;
 };
 
+// Page-locked host memory: what a net's reads come through, and what goes to its device without a wait.  A copy to or from
+// pageable memory is staged by the runtime piece by piece: reading 40 KB took 25.0 us, 147 KB 68.9, and 9.7 and 14.7 this way, the
+// copy on to the caller's memory with it; 10 KB 16.5 / 12.1.  Up to 4 KB and from 512 KB on both take as long (13.5 / 11.8, 37.8 / 39.3).
+// A net's tensors belong to the stream given.
+class PinnedFloats {
+public:
+    static constexpr size_t FEW = 1 << 10, READ = 1 << 17;       // reads of more than FEW and up to READ floats come through
+    PinnedFloats() : mData(nullptr), mSize(0) {}
+    ~PinnedFloats();
+    PinnedFloats(const PinnedFloats&) = delete;
+    PinnedFloats& operator=(const PinnedFloats&) = delete;
+    void reserve(size_t n);              // n floats at least; not while a copy is under way
+    float* data() { return mData; }
+    // n floats of device memory to host memory, behind the stream's work; waits.  From several threads one after the other.
+    void read(float* host, const float* device, size_t n, void* stream);
+
+private:
+    float* mData;
+    size_t mSize;
+    std::mutex mReading;
+};
+
 // Common part of the float cells (the role of Cell_Frame<T>, src/Cell/Cell_Frame.cpp:100-160 and :474-492): one input
 // tensor and the tensor its gradient goes to, own outputs and the gradient with respect to them, the activation
 // applied in place.
@@ -73,6 +97,8 @@ public:
     // wait for the value.  A learning loop that reads only its last loss need not stop the device for the others.
     void launchLoss(const float* targets);
     double readLoss() const;
+    // the value's place in device memory, null before the first launchLoss()
+    const double* lossOnDevice() const { return mLoss; }
     bool isCuda() const { return false; }
     std::string getPyModel() const { return "Frame_HIP_QAT"; }
     // The stream this cell's kernels are launched on: whatever a caller copies into the cell's tensors between two of its
@@ -120,7 +146,7 @@ public:
     void quantizeWeights();
     void forgetQuantizedWeights() { mWeightsQuantized = false; }
     // the device's weights, without the host tensors
-    void readWeights(float* host, size_t n) const { mDevW.toHost(host, n); }
+    void readWeights(float* host, size_t n, PinnedFloats& through) const;
 
 protected:
     WeightedCell_FrameTrain_HIP();
@@ -272,7 +298,7 @@ public:
     std::vector<Float_T> getDiffScales() const { return get(mDiffScale, std::vector<Float_T>()); }
     std::vector<Float_T> getDiffBiases() const { return get(mDiffBias, std::vector<Float_T>()); }
     // the six vectors above, one behind the other (6 x nbOutputs values), in one copy from the device
-    void readParameters(float* host) const;
+    void readParameters(float* host, PinnedFloats& through) const;
     void setScaleSolver(const std::shared_ptr<SGDSolver>& solver) { mScaleSolver = solver; }
     void setBiasSolver(const std::shared_ptr<SGDSolver>& solver) { mBiasSolver = solver; }
     const std::shared_ptr<SGDSolver>& getScaleSolver() const { return mScaleSolver; }

@@ -28,6 +28,7 @@ struct TrainNet {
     Network net;
     DeepNet deepNet;
     DeviceFloats input, inputDiff, inputDiffPreset, targets;
+    PinnedFloats reads, toDevice;             // toDevice: the loss (a double), then the targets
     std::vector<std::shared_ptr<Cell_FrameTrain_HIP> > cells;
     std::map<std::string, std::shared_ptr<SATQuantizerActivation_Frame_HIP<float> > > satAct;
     std::map<std::string, std::shared_ptr<LSQQuantizerActivation_Frame_HIP<float> > > lsqAct;
@@ -144,6 +145,7 @@ int fh_train_net_create(const char* model, const float* input, int B, int C, int
         n->input.fromHost(input, n->input.size());
         if (propagateGradient)
             n->inputDiff.resize(dims);
+        n->reads.reserve(PinnedFloats::READ);
         *out = n.release();
     });
 }
@@ -284,7 +286,7 @@ int fh_train_get_batchnorm_all(void* net, const char* cell, float* out, size_t n
         auto bn = dynamic_cast<BatchNormCell_FrameTrain_HIP<float>*>(find(*(TrainNet*)net, cell));
         if (!bn) throw std::runtime_error("Not a BatchNorm cell: " + std::string(cell));
         if (n != bn->getNbOutputs()) throw std::runtime_error("fh_train_get_batchnorm_all(): size mismatch");
-        bn->readParameters(out);
+        bn->readParameters(out, ((TrainNet*)net)->reads);
     });
 }
 
@@ -379,8 +381,19 @@ int fh_train_learn(void* net, const float* targets, size_t nTargets, int iterati
         if (n.cells.empty()) throw std::runtime_error("Empty net");
         Cell_FrameTrain_HIP* last = n.last();
         if (nTargets != last->getOutputs().size()) throw std::runtime_error("fh_train_learn(): wrong number of targets");
-        n.targets.resize(last->getOutputs().dims());
-        n.targets.fromHost(targets, nTargets);
+        if (n.targets.dims() != last->getOutputs().dims())
+            n.targets.resize(last->getOutputs().dims());
+        // (the host does not wait for the targets' copy; whoever writes to this memory again has waited for the device first)
+        constexpr size_t LOSS = sizeof(double) / sizeof(float);
+        n.toDevice.reserve(LOSS + nTargets);
+        struct Wait {
+            bool pending = true;
+            ~Wait() { if (pending) (void)hipDeviceSynchronize(); }
+        } copies;
+        std::memcpy(n.toDevice.data() + LOSS, targets, nTargets * sizeof(float));
+        if (hipMemcpyAsync(n.targets.data(), n.toDevice.data() + LOSS, nTargets * sizeof(float), hipMemcpyHostToDevice, (hipStream_t)last->stream())
+            != hipSuccess)
+            throw std::runtime_error("fh_train_learn(): copy of the targets failed");
         for (int it = 0; it < iterations; ++it) {
             // the gradient towards the net's input is this iteration's: empty, or what another consumer of the input has
             // already put there (fh_train_preset_input_gradient)
@@ -411,8 +424,13 @@ int fh_train_learn(void* net, const float* targets, size_t nTargets, int iterati
             updates.flush();
         }
         // (only the last iteration's loss is asked for: the device runs through the others without a stop)
-        const double l = iterations > 0 ? last->readLoss() : 0.0;
+        if (iterations > 0
+            && hipMemcpyAsync(n.toDevice.data(), last->lossOnDevice(), sizeof(double), hipMemcpyDeviceToHost, (hipStream_t)last->stream()) != hipSuccess)
+            throw std::runtime_error("fh_train_learn(): copy of the loss failed");
+        copies.pending = false;
         if (hipDeviceSynchronize() != hipSuccess) throw std::runtime_error("fh_train_learn(): device error");
+        double l = 0.0;
+        if (iterations > 0) std::memcpy(&l, n.toDevice.data(), sizeof(double));
         if (loss) *loss = l;
     });
 }
@@ -490,7 +508,7 @@ int fh_train_get(void* net, const char* cell, int what, float* out, size_t n)
         Tensor<Float_T> t;
         auto conv = dynamic_cast<WeightedCell_FrameTrain_HIP*>(c);
         if (what == 2 && conv) {
-            conv->readWeights(out, n);
+            conv->readWeights(out, n, ((TrainNet*)net)->reads);
             return;
         }
         if (what == 0) t = c->getOutputs().toHost();
