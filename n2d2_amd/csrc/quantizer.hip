@@ -42,6 +42,17 @@ __device__ __forceinline__ double block_sum(double v)
     for (int i = 0; i < (int)(blockDim.x >> 6); ++i) t += red[i];
     return t;
 }
+// Both sums over the block, with one wait
+__device__ __forceinline__ void block_sums(double& a, double& b)
+{
+    __shared__ double red[16][2];
+    a = wave_sum(a);
+    b = wave_sum(b);
+    if ((threadIdx.x & 63) == 0) { red[threadIdx.x >> 6][0] = a; red[threadIdx.x >> 6][1] = b; }
+    __syncthreads();
+    a = b = 0.0;
+    for (int i = 0; i < (int)(blockDim.x >> 6); ++i) { a += red[i][0]; b += red[i][1]; }
+}
 __device__ __forceinline__ float block_max(float v)
 {
     __shared__ float redm[16];
@@ -127,28 +138,44 @@ struct SatLevels {
         }
     }
 };
-// SAT weights of several tensors, in two launches at most: a learning net quantizes the weights of all its cells before a pass,
-// most of them few, and a launch each (three for many weights) was what bounded them.  16 tensors fit a launch's arguments.
-//  * Up to 16384 weights: one block computes the tensor, in the first launch.  Its tanh stay in registers (they were computed
-//    twice, and each pass went through memory): up to 1024 weights 3.7 us, 2400 4.2 and 10080, scaling included, 11.6 in a
-//    batch (12.8 with an instance of 16 weights a thread); the blocks of several tensors run side by side.  (Instances by the weights per thread: skipping unused ones inside one instance
-//    made the compiler spill.)
+// SAT weights of several tensors, in three launches at most: a learning net quantizes the weights of all its cells before a pass,
+// most of them few, and a launch each (seven for many weights with scaling) was what bounded them.  16 tensors fit a launch's arguments.
+//  * Few: one block computes the tensor, in the first launch.  Its tanh stay in registers; the blocks of several tensors run side by
+//    side.  (Instances by the weights per thread: skipping unused ones inside one instance made the compiler spill.)  What bounds it is
+//    that one compute unit's arithmetic, so it ends where two or three launches of many blocks take as long: us, one block / many, 6000
+//    weights 5.5 / 5.7, 8192 5.9 / 5.6, 10080 7.0 / 5.6, 16384 8.8 / 5.8; with scaling 8192 7.7 / 10.0, 12288 9.4 / 10.1, 16384 11.1 / 10.0.
 //  * More: the first launch leaves each block's max |tanh w|, and every block of the second one takes the maximum of those,
-//    at most 256, itself, instead of a launch of one block in between (48120 weights: 3 launches of 2.8, 1.8 and 2.4 us).
-//    The second launch fills the chip, 8 blocks a compute unit, and both deal the weights to the XCDs alike, in runs of 256 as
-//    the scaling's launches do, so that the weights come from the XCD's own L2 the second time.  us, with the launch in
-//    between / with 4 blocks a unit and runs of 1024 in the first launch / now: 16385 weights 11.6 / 9.5 / 8.8, 1048576 11.3 / 9.8 / 9.4,
-//    4194304 16.6 / 20.3 / 15.5, 16777216 52.8 / 62.5 / 52.4, 67108864 279 / 341 / 269.
-constexpr int SAT_SMALL = 16;                    // weights per thread of a block of 1024 at most
-constexpr int SAT_BLOCKS = 256, SAT_BLOCKS2 = 2048;     // blocks of a larger tensor's first and second launch at most
+//    at most 256, itself.  The second launch fills the chip, 8 blocks a compute unit, and all deal the weights to the XCDs alike, in
+//    runs of 256, so that the weights come from the XCD's own L2 the second time.  us: 16385 weights 5.8, 1048576 8.5, 4194304
+//    14.6, 16777216 52.
+//  * With scaling the second leaves each block's sums of the levels' differences from the first level and of their squares, in double, and a
+//    third divides the levels: every block adds the sums up itself.  (One pass for the mean, one for the squares, a block's launch
+//    behind each and the division before: 16385 weights 15.6 us, now 10.1; 163840 17.4 / 11.8; 1048576 22.2 / 17.4; 4194304 36.1 / 28.3;
+//    16777216 121.5 / 82.3.)  The workspace holds the sums of 448 blocks; from 2 M weights on those are of 1024 threads, which 16777216 need
+//    (124.5 with 256; 1048576 18.7 with 1024).
+constexpr int SAT_SMALL = 8, SAT_SMALL_SCALED = 12;     // weights per thread of a block of 1024 at most
+constexpr int SAT_BLOCKS = 256, SAT_BLOCKS2 = 2048;     // blocks of a larger tensor's first, and second or third launch at most
+constexpr int SAT_BLOCKS_SUMS = 448;             // of the second where each leaves its sums in the workspace
+constexpr size_t SAT_MANY = 2 << 20;             // scaled weights from which their blocks have 1024 threads
 constexpr int SAT_ITEMS = 16;
+constexpr size_t SAT_SUMS = (SAT_BLOCKS + 4) * sizeof(float);       // place of the blocks' sums, behind their maxima and the first weight's tanh
 template <int N>
 struct SatBatch {
     n2d2hip_sat_weight_item item[N];
-    unsigned first[N + 1], first2[N + 1];        // first block of a tensor in the first and the second launch
+    unsigned first[N + 1], first2[N + 1], first3[N + 1];        // first block of a tensor in each launch
     int count;
 };
-__host__ __device__ inline bool sat_small(size_t n) { return n <= (size_t)SAT_SMALL * 1024; }
+__host__ __device__ inline bool sat_small(const n2d2hip_sat_weight_item& t) { return t.n <= (size_t)(t.apply_scaling ? SAT_SMALL_SCALED : SAT_SMALL) * 1024; }
+
+// SAT scaling, ref: SATQuantizer_Frame_Kernels.cpp:244-262: the n levels' mean, their unbiased variance about that mean rounded to
+// float, scaling = sqrt(var * outputs_size); from the sums of their differences d from one of them and of d * d, in double
+__device__ __forceinline__ float sat_scaling(double sum, double squares, float shift, size_t n, unsigned outputs_size)
+{
+    const float mean = (float)(sum + (double)n * (double)shift) / (float)n;
+    const double e = (double)mean - (double)shift, about = squares - 2.0 * e * sum + (double)n * e * e;
+    const float var = (float)(about < 0.0 ? 0.0 : about) / ((float)n - 1.0f);       // (NaN stays)
+    return sqrtf(var * (float)outputs_size);
+}
 
 template <int K>
 __device__ __forceinline__ void sat_weight_small(const n2d2hip_sat_weight_item& t)
@@ -156,6 +183,7 @@ __device__ __forceinline__ void sat_weight_small(const n2d2hip_sat_weight_item& 
     const float* __restrict__ w = t.w;
     float* __restrict__ wq = t.wq;
     const int n = (int)t.n;
+    __shared__ float first;
     float v[K];
     float m = 0.0f;
 #pragma unroll
@@ -164,25 +192,25 @@ __device__ __forceinline__ void sat_weight_small(const n2d2hip_sat_weight_item& 
         v[k] = i < n ? tanhf(w[i]) : 0.0f;
         m = fmaxf(m, fabsf(v[k]));
     }
+    if (threadIdx.x == 0) first = v[0];
     m = block_max(m);
     const SatLevels level(t.range, t.mode, m);
-    double sum = 0.0;
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-        v[k] = level(v[k]);
-        if (k * 1024 + (int)threadIdx.x < n) sum += (double)v[k];
-    }
+    for (int k = 0; k < K; ++k) v[k] = level(v[k]);
     float scaling = 1.0f;
-    if (t.apply_scaling) {                       // (the formulas of mean_final, sqdev_partial and sat_scaling_final)
-        const float mean = (float)block_sum(sum) / (float)n;
-        double squares = 0.0;
+    if (t.apply_scaling) {
+        const float shift = level(first);
+        double sum = 0.0, squares = 0.0;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            const float d = __fsub_rn(v[k], mean);
-            if (k * 1024 + (int)threadIdx.x < n) squares += (double)__fmul_rn(d, d);
+            const double d = (double)v[k] - (double)shift;
+            if (k * 1024 + (int)threadIdx.x < n) {
+                sum += d;
+                squares += d * d;
+            }
         }
-        const float var = (float)block_sum(squares) / ((float)n - 1.0f);
-        scaling = sqrtf(var * (float)t.outputs_size);
+        block_sums(sum, squares);
+        scaling = sat_scaling(sum, squares, shift, t.n, t.outputs_size);
     }
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -198,12 +226,12 @@ __global__ __launch_bounds__(1024) void sat_weight_first_kernel(const SatBatch<N
     if (N > 1)
         while (k + 1 < b.count && blockIdx.x >= b.first[k + 1]) ++k;
     const n2d2hip_sat_weight_item& t = b.item[k];
-    if (t.n <= 1024) sat_weight_small<1>(t);
-    else if (t.n <= 4 * 1024) sat_weight_small<4>(t);
-    else if (t.n <= 8 * 1024) sat_weight_small<8>(t);
-    else if (t.n <= 12 * 1024) sat_weight_small<12>(t);
-    else if (sat_small(t.n)) sat_weight_small<SAT_SMALL>(t);
-    else {
+    if (sat_small(t)) {
+        if (t.n <= 1024) sat_weight_small<1>(t);
+        else if (t.n <= 4 * 1024) sat_weight_small<4>(t);
+        else if (t.n <= 8 * 1024) sat_weight_small<8>(t);
+        else sat_weight_small<SAT_SMALL_SCALED>(t);
+    } else {
         // (blocks 8 apart run on the same XCD: of 8 blocks, a multiple of which there is, each takes every 8th run of 256)
         const unsigned block = blockIdx.x - b.first[k], run = 8 * (4 * (block >> 3) + (threadIdx.x >> 8)) + (block & 7);
         float m = 0.0f;
@@ -211,10 +239,16 @@ __global__ __launch_bounds__(1024) void sat_weight_first_kernel(const SatBatch<N
             m = fmaxf(m, fabsf(tanhf(t.w[i])));
         m = block_max(m);
         if (threadIdx.x == 0) ((float*)t.workspace)[block] = m;
+        if (block == 0 && threadIdx.x == 0) ((float*)t.workspace)[SAT_BLOCKS] = tanhf(t.w[0]);
     }
 }
+// A thread's first weight where a tensor's blocks, of 256 or 1024 threads, take every 8th run of 256 from their own on, as the first launch's do
+__device__ __forceinline__ size_t sat_first_weight(unsigned block)
+{
+    return (size_t)(8 * ((blockDim.x >> 8) * (block >> 3) + (threadIdx.x >> 8)) + (block & 7)) * QBLOCK + (threadIdx.x & (QBLOCK - 1));
+}
 template <int N>
-__global__ __launch_bounds__(QBLOCK) void sat_weight_second_kernel(const SatBatch<N> b)
+__global__ __launch_bounds__(1024) void sat_weight_second_kernel(const SatBatch<N> b)
 {
     int k = 0;
     if (N > 1)
@@ -222,59 +256,53 @@ __global__ __launch_bounds__(QBLOCK) void sat_weight_second_kernel(const SatBatc
     const n2d2hip_sat_weight_item& t = b.item[k];
     const float* __restrict__ w = t.w;
     float* __restrict__ wq = t.wq;
+    const unsigned block = blockIdx.x - b.first2[k];
+    const size_t step = (size_t)(b.first2[k + 1] - b.first2[k]) * blockDim.x;
     static_assert(SAT_BLOCKS <= QBLOCK, "a thread takes one block's maximum");
     const float m = block_max(threadIdx.x < b.first[k + 1] - b.first[k] ? ((const float*)t.workspace)[threadIdx.x] : 0.0f);
     const SatLevels level(t.range, t.mode, m);
-    for (size_t i = (size_t)(blockIdx.x - b.first2[k]) * QBLOCK + threadIdx.x; i < t.n; i += (size_t)(b.first2[k + 1] - b.first2[k]) * QBLOCK)
-        wq[i] = level(tanhf(w[i]));
-    if (blockIdx.x == b.first2[k] && threadIdx.x == 0) { t.stats[0] = m; t.stats[1] = 1.0f; }
+    if (block == 0 && threadIdx.x == 0) { t.stats[0] = m; t.stats[1] = 1.0f; }
+    if (!t.apply_scaling) {
+        for (size_t i = sat_first_weight(block); i < t.n; i += step) wq[i] = level(tanhf(w[i]));
+        return;
+    }
+    const float shift = level(((const float*)t.workspace)[SAT_BLOCKS]);
+    double sum = 0.0, squares = 0.0;
+#pragma unroll 4
+    for (size_t i = sat_first_weight(block); i < t.n; i += step) {
+        const float q = level(tanhf(w[i]));
+        const double d = (double)q - (double)shift;
+        wq[i] = q;
+        sum += d;
+        squares += d * d;
+    }
+    block_sums(sum, squares);
+    if (threadIdx.x == 0) ((double2*)((char*)t.workspace + SAT_SUMS))[block] = make_double2(sum, squares);
 }
 
-// SAT scaling, ref: SATQuantizer_Frame_Kernels.cpp:244-262: mean, unbiased variance about that
-// mean, scaling = sqrt(var * outputs_size).
-__global__ __launch_bounds__(QBLOCK) void sum_partial(const float* __restrict__ x, size_t n, double* __restrict__ partial)
+// The division of the levels by their scaling.  The second launch leaves each block's sums; every block of this one adds them up itself
+// and divides its share.  (A pass for the sum, one for the squares, a block's launch behind each and the division were five launches.)
+template <int N>
+__global__ __launch_bounds__(1024) void sat_weight_scale_kernel(const SatBatch<N> b)
 {
-    double s = 0.0;
-    for (size_t i = (size_t)blockIdx.x * QBLOCK + threadIdx.x; i < n; i += (size_t)gridDim.x * QBLOCK)
-        s += (double)x[i];
-    s = block_sum(s);
-    if (threadIdx.x == 0) partial[blockIdx.x] = s;
-}
-__global__ __launch_bounds__(QBLOCK) void mean_final(const double* __restrict__ partial, int count, size_t n, float* __restrict__ mean)
-{
-    double s = 0.0;
-    for (int i = threadIdx.x; i < count; i += QBLOCK) s += partial[i];
-    s = block_sum(s);
-    if (threadIdx.x == 0) mean[0] = (float)((float)s / (float)n);
-}
-__global__ __launch_bounds__(QBLOCK) void sqdev_partial(const float* __restrict__ x, size_t n, const float* __restrict__ mean,
-                                                        double* __restrict__ partial)
-{
-    const float m = mean[0];
-    double s = 0.0;
-    for (size_t i = (size_t)blockIdx.x * QBLOCK + threadIdx.x; i < n; i += (size_t)gridDim.x * QBLOCK) {
-        const float d = __fsub_rn(x[i], m);
-        s += (double)__fmul_rn(d, d);
+    int k = 0;
+    if (N > 1)
+        while (k + 1 < b.count && blockIdx.x >= b.first3[k + 1]) ++k;
+    const n2d2hip_sat_weight_item& t = b.item[k];
+    float* __restrict__ wq = t.wq;
+    const unsigned block = blockIdx.x - b.first3[k], count = b.first2[k + 1] - b.first2[k];
+    const double2* sums = (const double2*)((const char*)t.workspace + SAT_SUMS);
+    const float shift = SatLevels(t.range, t.mode, t.stats[0])(((const float*)t.workspace)[SAT_BLOCKS]);
+    double sum = 0.0, squares = 0.0;
+    for (unsigned i = threadIdx.x; i < count; i += blockDim.x) {
+        const double2 v = sums[i];
+        sum += v.x;
+        squares += v.y;
     }
-    s = block_sum(s);
-    if (threadIdx.x == 0) partial[blockIdx.x] = s;
-}
-__global__ __launch_bounds__(QBLOCK) void sat_scaling_final(const double* __restrict__ partial, int count, size_t n, unsigned factor,
-                                                            float* __restrict__ stats)
-{
-    double s = 0.0;
-    for (int i = threadIdx.x; i < count; i += QBLOCK) s += partial[i];
-    s = block_sum(s);
-    if (threadIdx.x == 0) {
-        const float var = (float)s / ((float)n - 1.0f);
-        stats[1] = sqrtf(var * (float)factor);
-    }
-}
-__global__ __launch_bounds__(QBLOCK) void divide_by_stat(float* __restrict__ x, size_t n, const float* __restrict__ stat)
-{
-    const float s = stat[0];
-    for (size_t i = (size_t)blockIdx.x * QBLOCK + threadIdx.x; i < n; i += (size_t)gridDim.x * QBLOCK)
-        x[i] = x[i] / s;
+    block_sums(sum, squares);
+    const float scaling = sat_scaling(sum, squares, shift, t.n, t.outputs_size);
+    if (block == 0 && threadIdx.x == 0) t.stats[1] = scaling;
+    for (size_t i = sat_first_weight(block); i < t.n; i += (size_t)(b.first3[k + 1] - b.first3[k]) * blockDim.x) wq[i] = wq[i] / scaling;
 }
 
 // ref: SATQuantizer_Frame_Kernels.cpp:349-404
@@ -464,28 +492,27 @@ static void sat_weight_launch(const n2d2hip_sat_weight_item* items, int count, h
 {
     SatBatch<N> b = {};
     b.count = count;
+    int threads = QBLOCK;
+    for (int i = 0; i < count; ++i)
+        if (items[i].apply_scaling && items[i].n >= SAT_MANY) threads = 1024;
+    const auto blocks = [&](size_t n, int most) {
+        return (unsigned)std::min<size_t>(threads == QBLOCK ? (n + QBLOCK - 1) / QBLOCK : (n + 8191) / 8192 * 8, most);
+    };
     for (int i = 0; i < count; ++i) {
         const size_t n = items[i].n;
+        const bool small = sat_small(items[i]), scaled = items[i].apply_scaling && !small;
         b.item[i] = items[i];
-        b.first[i + 1] = b.first[i] + (sat_small(n) ? 1u : (unsigned)std::min<size_t>((n + 8191) / 8192 * 8, SAT_BLOCKS));
-        b.first2[i + 1] = b.first2[i] + (sat_small(n) ? 0u : (unsigned)std::min<size_t>((n + QBLOCK - 1) / QBLOCK, SAT_BLOCKS2));
+        b.first[i + 1] = b.first[i] + (small ? 1u : (unsigned)std::min<size_t>((n + 8191) / 8192 * 8, SAT_BLOCKS));
+        b.first2[i + 1] = b.first2[i] + (small ? 0u : blocks(n, scaled ? SAT_BLOCKS_SUMS : SAT_BLOCKS2 * QBLOCK / threads));
+        b.first3[i + 1] = b.first3[i] + (scaled ? blocks(n, SAT_BLOCKS2 * QBLOCK / threads) : 0u);
     }
+    static_assert(SAT_SUMS % sizeof(double2) == 0 && SAT_SUMS + SAT_BLOCKS_SUMS * sizeof(double2) <= (size_t)PARTIALS * sizeof(double) + 256,
+                  "a workspace holds the maxima and the sums");
     N2D2HIP_LAUNCH_T(sat_weight_first_kernel, (N), dim3(b.first[count]), dim3(1024), 0, st, b);
     if (b.first2[count])
-        N2D2HIP_LAUNCH_T(sat_weight_second_kernel, (N), dim3(b.first2[count]), dim3(QBLOCK), 0, st, b);
-    for (int i = 0; i < count; ++i) {
-        const n2d2hip_sat_weight_item& t = items[i];
-        if (!t.apply_scaling || sat_small(t.n))
-            continue;
-        const int nb = blocks_for(t.n);
-        double* partial = (double*)t.workspace;
-        float* mean = (float*)((char*)t.workspace + (size_t)PARTIALS * sizeof(double));
-        hipLaunchKernelGGL(sum_partial, dim3(nb), dim3(QBLOCK), 0, st, (const float*)t.wq, t.n, partial);
-        hipLaunchKernelGGL(mean_final, dim3(1), dim3(QBLOCK), 0, st, (const double*)partial, nb, t.n, mean);
-        hipLaunchKernelGGL(sqdev_partial, dim3(nb), dim3(QBLOCK), 0, st, (const float*)t.wq, t.n, (const float*)mean, partial);
-        hipLaunchKernelGGL(sat_scaling_final, dim3(1), dim3(QBLOCK), 0, st, (const double*)partial, nb, t.n, t.outputs_size, t.stats);
-        hipLaunchKernelGGL(divide_by_stat, dim3(ew_grid(t.n)), dim3(QBLOCK), 0, st, t.wq, t.n, (const float*)(t.stats + 1));
-    }
+        N2D2HIP_LAUNCH_T(sat_weight_second_kernel, (N), dim3(b.first2[count]), dim3(threads), 0, st, b);
+    if (b.first3[count])
+        N2D2HIP_LAUNCH_T(sat_weight_scale_kernel, (N), dim3(b.first3[count]), dim3(threads), 0, st, b);
 }
 
 template <int N>
