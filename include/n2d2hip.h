@@ -539,6 +539,11 @@ int n2d2hip_lsq_backward(const float* diff_q, const float* fp_x, float* diff_fp,
 int n2d2hip_conv2d_f32_forward(const n2d2hip_conv_desc* desc, int B, int H, int W, const float* x, const float* w,
                                const float* bias, float beta, float* y, void* workspace, size_t workspace_bytes,
                                n2d2hip_stream_t stream);
+/* The same without beta and with the SAT activation quantizer of n2d2hip_sat_act_forward() behind it: y receives the quantized
+ * values, full_precision (or NULL) what goes into the quantizer.  full_precision is none of the other tensors. */
+int n2d2hip_conv2d_f32_forward_sat(const n2d2hip_conv_desc* desc, int B, int H, int W, const float* x, const float* w,
+                                   const float* bias, float* y, float* full_precision, float range, const float* alpha,
+                                   void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream);
 /* diff_x = backwardData(w, diff_y) + beta * diff_x (ref: src/Cell/ConvCell_Frame_Kernels.cpp:176-333).  Dilation
  * must be 1: the reference's backward kernels do not read it. */
 int n2d2hip_conv2d_f32_backward_data(const n2d2hip_conv_desc* desc, int B, int H, int W, const float* w,
@@ -652,6 +657,11 @@ int n2d2hip_softmax_f32_forward(const float* x, float* y, int B, int C, int H, i
 size_t n2d2hip_loss_workspace_bytes(size_t n);
 int n2d2hip_loss_f32(const float* target, const float* output, float* diff, size_t n, int batch, double* loss,
                      void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream);
+/* A SoftmaxCell with loss at the end of a learning net in one call: y = n2d2hip_softmax_f32_forward(x), then
+ * n2d2hip_loss_f32(target, y, diff, ...) with batch B, and diff once more in diff_x (or NULL), the gradient of the cell
+ * below.  The tensors do not overlap; the workspace is n2d2hip_loss_workspace_bytes()'s. */
+int n2d2hip_softmax_loss_f32(const float* x, const float* target, float* y, float* diff, float* diff_x, int B, int C, int H,
+                             int W, double* loss, void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream);
 /* One SGDSolver_Frame<float>::update on a device tensor (ref: include/Solver/SGDSolver_Frame.hpp:77-146):
  * momentum_data == NULL: data += rate_diff * diff; otherwise m = m * momentum + rate_diff * diff
  * - decay_times_rate * data, data += m.  rate_diff = rate / (batchSize * IterationSize), computed by the caller from

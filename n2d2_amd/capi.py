@@ -44,7 +44,7 @@ SYMBOLS = [
     "n2d2hip_sat_weight_forward", "n2d2hip_sat_weight_forward_static", "n2d2hip_sat_weight_backward",
     "n2d2hip_sat_act_forward", "n2d2hip_sat_act_backward", "n2d2hip_lsq_forward", "n2d2hip_lsq_backward",
     "n2d2hip_conv2d_f32_forward", "n2d2hip_conv2d_f32_backward_data", "n2d2hip_conv2d_f32_backward_filter", "n2d2hip_conv2d_f32_backward", "n2d2hip_conv2d_f32_workspace_bytes",
-    "n2d2hip_conv2d_f32_backward_bias", "n2d2hip_softmax_f32_forward", "n2d2hip_loss_workspace_bytes", "n2d2hip_loss_f32",
+    "n2d2hip_conv2d_f32_backward_bias", "n2d2hip_softmax_f32_forward", "n2d2hip_loss_workspace_bytes", "n2d2hip_loss_f32", "n2d2hip_softmax_loss_f32", "n2d2hip_conv2d_f32_forward_sat",
     "n2d2hip_sgd_update_f32", "n2d2hip_sgd_update_f32_batch", "n2d2hip_rectifier_f32_forward", "n2d2hip_rectifier_f32_backward",
     "n2d2hip_batchnorm_f32_workspace_bytes", "n2d2hip_batchnorm_f32_forward_sat",
     "n2d2hip_batchnorm_f32_backward_sat_workspace_bytes", "n2d2hip_batchnorm_f32_backward_sat",
@@ -186,6 +186,8 @@ def load():
     lib.n2d2hip_loss_workspace_bytes.restype = C.c_size_t
     lib.n2d2hip_loss_workspace_bytes.argtypes = [SZ]
     lib.n2d2hip_loss_f32.argtypes = [P, P, P, SZ, I, P, P, SZ, P]
+    lib.n2d2hip_softmax_loss_f32.argtypes = [P, P, P, P, P, I, I, I, I, P, P, SZ, P]
+    lib.n2d2hip_conv2d_f32_forward_sat.argtypes = [P, I, I, I, P, P, P, P, P, F, P, P, SZ, P]
     lib.n2d2hip_sgd_update_f32.argtypes = [P, P, SZ, F, F, F, P, I, F, F, P]
     lib.n2d2hip_sgd_update_f32_batch.argtypes = [C.POINTER(SgdItem), I, P]
     lib.n2d2hip_rectifier_f32_forward.argtypes = [P, SZ, F, F, P]

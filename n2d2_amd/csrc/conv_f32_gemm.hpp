@@ -44,6 +44,7 @@
 
 #include "common.h"
 #include "mfma_util.hpp"
+#include "sat_math.hpp"
 
 namespace n2d2hip {
 
@@ -627,12 +628,19 @@ __device__ __forceinline__ void chain_read(v4f (&xv)[8], v4f (&wv)[8], unsigned 
     lds_read128f<OFF + 96>(xv[6], xa); lds_read128f<OFF + 96>(wv[6], wa);
     lds_read128f<OFF + 112>(xv[7], xa); lds_read128f<OFF + 112>(wv[7], wa);
 }
-__device__ __forceinline__ void chain_store(int B, int O, int b, int o, float sum, const float* __restrict__ bias, float beta, float* __restrict__ y)
+// (The SAT quantizer that follows on the way out, a: its |alpha|.  32 x 84 and 32 x 10 sums: 2.9 + 2.6 and 2.6 + 1.9 us in two kernels each, 3.7 and
+// 3.1 in one.)
+__device__ __forceinline__ void chain_store(int B, int O, int b, int o, float sum, const float* __restrict__ bias, float beta, const SatStore& sat, float a,
+                                            float* __restrict__ y)
 {
     if (b >= B || o >= O) return;
     const size_t idx = (size_t)b * O + o;
     float r = sum + (beta != 0.0f ? beta * y[idx] : 0.0f);
     if (bias) r = bias[o] + r;
+    if (sat.alpha) {
+        if (sat.fp) sat.fp[idx] = r;
+        r = sat_quantize(r, sat.range, a);
+    }
     y[idx] = r;
 }
 
@@ -665,11 +673,12 @@ __device__ __forceinline__ void chain_add_lanes(float& sum, const v4f& p, int la
 // (SUMS: of a work-group; the two have nothing but the name in common)
 template <int SUMS>
 __global__ void conv_f32_chain_kernel(int B, int O, int K, const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float beta,
-                                      float* __restrict__ y);
+                                      SatStore sat, float* __restrict__ y);
 template <>
 __global__ __launch_bounds__(64) void conv_f32_chain_kernel<4>(int B, int O, int K, const float* __restrict__ x, const float* __restrict__ w,
-                                                               const float* __restrict__ bias, float beta, float* __restrict__ y)
+                                                               const float* __restrict__ bias, float beta, SatStore sat, float* __restrict__ y)
 {
+    const float a = sat.alpha ? fabsf(sat.alpha[0]) : 0.0f;
     constexpr int D = 8;                         // groups of 64 terms requested ahead
     const int lane = threadIdx.x, li = lane & 15, bi = lane >> 5, oi = lane >> 4 & 1, b0 = blockIdx.x * 2, o0 = blockIdx.y * 2;
     const __amdgpu_buffer_rsrc_t rsrcX = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x + (size_t)b0 * K), 0, min(2, B - b0) * K * 4, 0x00020000);
@@ -702,13 +711,14 @@ __global__ __launch_bounds__(64) void conv_f32_chain_kernel<4>(int B, int O, int
         if (g + u < full) chain_add_row(sum, wv[u] * xv[u]);
         else if (g + u == full) chain_add_lanes(sum, wv[u] * xv[u], rest);
     }
-    if (li == 0) chain_store(B, O, b0 + bi, o0 + oi, sum, bias, beta, y);
+    if (li == 0) chain_store(B, O, b0 + bi, o0 + oi, sum, bias, beta, sat, a, y);
 }
 
 template <>
 __global__ __launch_bounds__(192) void conv_f32_chain_kernel<64>(int B, int O, int K, const float* __restrict__ x, const float* __restrict__ w,
-                                                                 const float* __restrict__ bias, float beta, float* __restrict__ y)
+                                                                 const float* __restrict__ bias, float beta, SatStore sat, float* __restrict__ y)
 {
+    const float a = sat.alpha ? fabsf(sat.alpha[0]) : 0.0f;
     __shared__ __attribute__((aligned(16))) float smem[CHAIN_STAGES * 16 * CHAIN_ROW + 2 * 64 * CHAIN_PROD];
     float* const products = smem + CHAIN_STAGES * 16 * CHAIN_ROW;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -805,12 +815,13 @@ __global__ __launch_bounds__(192) void conv_f32_chain_kernel<64>(int B, int O, i
         add(std::integral_constant<int, 3>{});
         __builtin_amdgcn_sched_barrier(0);
     }
-    chain_store(B, O, b0 + bi, o0 + oi, sum, bias, beta, y);
+    chain_store(B, O, b0 + bi, o0 + oi, sum, bias, beta, sat, a, y);
 }
 
 __global__ __launch_bounds__(64) void conv_f32_chain_wave_kernel(int B, int O, int K, const float* __restrict__ x, const float* __restrict__ w,
-                                                                 const float* __restrict__ bias, float beta, float* __restrict__ y)
+                                                                 const float* __restrict__ bias, float beta, SatStore sat, float* __restrict__ y)
 {
+    const float a = sat.alpha ? fabsf(sat.alpha[0]) : 0.0f;
     __shared__ __attribute__((aligned(16))) float smem[CHAIN_STAGES * 16 * CHAIN_ROW];
     const int lane = threadIdx.x, bi = lane >> 3, oi = lane & 7, b0 = blockIdx.x * 8, o0 = blockIdx.y * 8;
     const __amdgpu_buffer_rsrc_t rsrcX = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x + (size_t)b0 * K), 0, min(8, B - b0) * K * 4, 0x00020000);
@@ -869,7 +880,7 @@ __global__ __launch_bounds__(64) void conv_f32_chain_wave_kernel(int B, int O, i
         if (h + 1 < groups) group(std::integral_constant<int, 1>{}, h + 1);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    chain_store(B, O, b0 + bi, o0 + oi, sum, bias, beta, y);
+    chain_store(B, O, b0 + bi, o0 + oi, sum, bias, beta, sat, a, y);
 }
 
 // Forward (BWD = false) and backward-data with K in the tensors' own order, (channel, tap).

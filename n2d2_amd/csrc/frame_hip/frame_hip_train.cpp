@@ -199,9 +199,8 @@ void Cell_FrameTrain_HIP::activationUpdate()
         mActivation->getQuantizer()->update((unsigned int)mIn->dimB());
 }
 
-void Cell_FrameTrain_HIP::launchLoss(const float* targets)
+void Cell_FrameTrain_HIP::allocateLoss(size_t n)
 {
-    const size_t n = mOutputs.size();
     if (!mLoss)
         checkHipT(hipMalloc((void**)&mLoss, sizeof(double)), "Cell_FrameTrain_HIP::launchLoss()");
     const size_t need = n2d2hip_loss_workspace_bytes(n);
@@ -211,6 +210,12 @@ void Cell_FrameTrain_HIP::launchLoss(const float* targets)
         checkHipT(hipMalloc(&mLossWorkspace, need), "Cell_FrameTrain_HIP::launchLoss()");
         mLossWorkspaceBytes = need;
     }
+}
+
+void Cell_FrameTrain_HIP::launchLoss(const float* targets)
+{
+    const size_t n = mOutputs.size();
+    allocateLoss(n);
     // (target and diff may be the same buffer: each element is read, then written, by one thread)
     checkStatus(n2d2hip_loss_f32(targets, mOutputs.data(), mDiffInputs.data(), n, (int)mOutputs.dimB(), mLoss,
                                  mLossWorkspace, mLossWorkspaceBytes, mStream));
@@ -272,9 +277,17 @@ void WeightedCell_FrameTrain_HIP::propagateWeighted(bool inference, bool noBias)
     if (need > mWorkspace.size() * sizeof(float))
         mWorkspace.resize({(need + sizeof(float) - 1) / sizeof(float)});
     // a quantizer passes the biases through (quantize_bias_propagate copies them)
-    checkStatus(n2d2hip_conv2d_f32_forward(&d, (int)mIn->dimB(), (int)mInH, (int)mInW, mIn->data(), w, noBias ? nullptr : mDevBias.data(), 0.0f,
-                                           mOutputs.data(), mWorkspace.data(), mWorkspace.size() * sizeof(float), mStream));
-    activationPropagate(inference);
+    const float* bias = noBias ? nullptr : mDevBias.data();
+    // (a SAT quantizer alone behind the cell is applied as its sums leave)
+    if (const std::shared_ptr<SATQuantizerActivation_Frame_HIP<float> > sat = lonelySatQuantizer()) {
+        const auto to = sat->prepare(mOutputs.size(), inference);
+        checkStatus(n2d2hip_conv2d_f32_forward_sat(&d, (int)mIn->dimB(), (int)mInH, (int)mInW, mIn->data(), w, bias, mOutputs.data(), to.fullPrecision, to.range,
+                                                   to.alpha, mWorkspace.data(), mWorkspace.size() * sizeof(float), mStream));
+    } else {
+        checkStatus(n2d2hip_conv2d_f32_forward(&d, (int)mIn->dimB(), (int)mInH, (int)mInW, mIn->data(), w, bias, 0.0f, mOutputs.data(), mWorkspace.data(),
+                                               mWorkspace.size() * sizeof(float), mStream));
+        activationPropagate(inference);
+    }
     mDiffInputs.clearValid();
     mDevDiffW.clearValid();
     mDevDiffBias.clearValid();
@@ -873,7 +886,7 @@ const char* SoftmaxCell::Type = "Softmax";
 template <class T>
 SoftmaxCell_FrameTrain_HIP<T>::SoftmaxCell_FrameTrain_HIP(const DeepNet& /*deepNet*/, const std::string& name, unsigned int nbOutputs, bool withLoss,
                                                           unsigned int groupSize)
-    : Cell(name, nbOutputs), SoftmaxCell(withLoss, groupSize)
+    : Cell(name, nbOutputs), SoftmaxCell(withLoss, groupSize), mDiffOutWritten(false)
 {
     if (groupSize != 0 && groupSize != nbOutputs)
         throw std::runtime_error("SoftmaxCell_FrameTrain_HIP " + name + ": GroupSize is not supported by the float Frame_HIP cells");
@@ -892,18 +905,32 @@ void SoftmaxCell_FrameTrain_HIP<T>::propagate(bool /*inference*/)
 {
     checkStatus(n2d2hip_softmax_f32_forward(mIn->data(), mOutputs.data(), (int)mIn->dimB(), (int)mNbOutputs, (int)mOutH, (int)mOutW, mStream));
     mDiffInputs.clearValid();
+    mDiffOutWritten = false;
+}
+
+template <class T>
+void SoftmaxCell_FrameTrain_HIP<T>::propagateWithLoss(const float* targets)
+{
+    // (a gradient that is already there is added to, by backPropagate())
+    mDiffOutWritten = mWithLoss && mDiffOut && !mDiffOut->empty() && !mDiffOut->isValid();
+    allocateLoss(mOutputs.size());
+    checkStatus(n2d2hip_softmax_loss_f32(mIn->data(), targets, mOutputs.data(), mDiffInputs.data(), mDiffOutWritten ? mDiffOut->data() : nullptr,
+                                         (int)mIn->dimB(), (int)mNbOutputs, (int)mOutH, (int)mOutW, mLoss, mLossWorkspace, mLossWorkspaceBytes, mStream));
+    mDiffInputs.setValid();
 }
 
 template <class T>
 void SoftmaxCell_FrameTrain_HIP<T>::backPropagate()
 {
+    const bool written = mDiffOutWritten;
+    mDiffOutWritten = false;
     if (!mDiffOut || mDiffOut->empty() || !mDiffInputs.isValid())
         return;
     if (!mWithLoss)
         throw std::runtime_error("SoftmaxCell_FrameTrain_HIP " + mName + ": backPropagate() without WithLoss is not supported by the float Frame_HIP cells");
     if (mDiffOut->isValid())       // another consumer of the input has written its part: add to it
         checkStatus(n2d2hip_elemwise_sum_f32_backward(mDiffInputs.size(), 1.0f, mDiffInputs.data(), 1.0f, mDiffOut->data(), mStream));
-    else
+    else if (!written)
         checkHipT(hipMemcpyAsync(mDiffOut->data(), mDiffInputs.data(), mDiffInputs.size() * sizeof(float), hipMemcpyDeviceToDevice, (hipStream_t)mStream),
                   "SoftmaxCell_FrameTrain_HIP::backPropagate()");
     mDiffOut->setValid();

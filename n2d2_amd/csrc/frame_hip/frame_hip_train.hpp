@@ -85,6 +85,8 @@ public:
     // (SATWeightsScope); forgetQuantizedWeights() before the weights may change.
     virtual void quantizeWeights() {}
     virtual void forgetQuantizedWeights() {}
+    // The last cell's propagate(false) and launchLoss() in a learning iteration
+    virtual void propagateWithLoss(const float* targets) { propagate(false); launchLoss(targets); }
     virtual void backPropagate() = 0;
     virtual void update() = 0;
     DeviceFloats& getOutputs() { return mOutputs; }
@@ -120,11 +122,12 @@ protected:
     DeviceFloats* mDiffOut;
     DeviceFloats mOutputs, mDiffInputs;
     void* mStream;                  // the default stream: the quantizers attached to a cell launch there too
-
-private:
+    // places for the loss and its partial sums
+    void allocateLoss(size_t n);
     double* mLoss;
     void* mLossWorkspace;
     size_t mLossWorkspaceBytes;
+
 };
 
 // What ConvCell_Frame and FcCell_Frame share when they learn: device weights and biases with their gradients, the weight
@@ -409,6 +412,7 @@ public:
     }
     void initialize();
     void propagate(bool inference = false);
+    void propagateWithLoss(const float* targets);
     void backPropagate();
     void update() {}
 
@@ -416,6 +420,7 @@ protected:
     void setOutputsDims() { mOutW = mInW; mOutH = mInH; }
 
 private:
+    bool mDiffOutWritten;           // by propagateWithLoss(), for the next backPropagate()
     static Registrar<SoftmaxCell> mRegistrar;
 };
 

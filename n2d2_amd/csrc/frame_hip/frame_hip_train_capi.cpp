@@ -411,9 +411,12 @@ int fh_train_learn(void* net, const float* targets, size_t nTargets, int iterati
             }
             {
                 QuantizedWeights quantized(n);   // (all cells' in one launch or two)
-                for (auto& c : n.cells) c->propagate(false);
+                for (auto& c : n.cells) {
+                    if (c.get() == last && c == n.cells.back()) c->propagateWithLoss(n.targets.data());
+                    else c->propagate(false);
+                }
             }
-            last->launchLoss(n.targets.data());
+            if (last != n.cells.back().get()) last->launchLoss(n.targets.data());
             {
                 SATWeightsScope gradients;
                 for (auto c = n.cells.rbegin(); c != n.cells.rend(); ++c) (*c)->backPropagate();

@@ -15,6 +15,13 @@ __device__ __forceinline__ float sat_quantize(float v, float range, float a)
     q = round_half_away(__fmul_rn(range, q)) / range;
     return __fmul_rn(q, a);
 }
+// The quantizer behind a kernel that writes a tensor: fp receives what goes into it (or null), the output what comes out;
+// alpha null: no quantizer
+struct SatStore {
+    float* fp;
+    float range;
+    const float* alpha;
+};
 // Its derivatives by alpha and by its input, ref: SATQuantizer_Frame_Kernels.cpp:410-448
 __device__ __forceinline__ float sat_alpha_slope(float v, float range, float a)
 {

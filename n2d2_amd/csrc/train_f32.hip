@@ -374,6 +374,50 @@ __global__ __launch_bounds__(TBLOCK) void loss_finish_kernel(const double* __res
     if (threadIdx.x == 0) loss[0] = acc * inv_batch;
 }
 
+// The head of a learning net in one launch: softmax of few pixels, a thread each, targets - outputs and the loss from it, the
+// gradient where the cell below reads it too (diff_x, or null).  The start of a launch bounds each of softmax, loss and copy: 32 images
+// of 10 classes 2.9, 1.8 and 1.2 us in the kernels and as much between them, together 3.6.
+template <int N>
+__global__ __launch_bounds__(TBLOCK) void softmax_loss_f32_kernel(const float* __restrict__ x, const float* __restrict__ target, float* __restrict__ y,
+                                                                  float* __restrict__ diff, float* __restrict__ diff_x, int total, int C, int plane, double inv_batch,
+                                                                  double* __restrict__ loss)
+{
+    double acc = 0.0;
+    for (int idx = threadIdx.x; idx < total; idx += TBLOCK) {
+        const size_t base = (size_t)(idx / plane) * C * plane + idx % plane;
+        float v[N], t[N];
+#pragma unroll
+        for (int c = 0; c < N; ++c) {
+            const size_t at = base + (size_t)(c < C ? c : 0) * plane;
+            v[c] = x[at];
+            t[c] = target[at];
+        }
+        float m = v[0];
+#pragma unroll
+        for (int c = 1; c < N; ++c) m = fmaxf(m, v[c]);
+        float s = 0.0f;
+#pragma unroll
+        for (int c = 0; c < N; ++c) {
+            if (c >= C) break;
+            v[c] = expf(v[c] - m);
+            s += v[c];
+        }
+#pragma unroll
+        for (int c = 0; c < N; ++c) {
+            if (c >= C) break;
+            const size_t at = base + (size_t)c * plane;
+            const float o = s > 0.0f ? v[c] / s : 0.0f;
+            const double e = (double)t[c] - (double)o;
+            y[at] = o;
+            diff[at] = (float)e;
+            if (diff_x) diff_x[at] = (float)e;
+            acc += e * e;
+        }
+    }
+    acc = block_sum_d(acc);
+    if (threadIdx.x == 0) loss[0] = acc * inv_batch;
+}
+
 // SGDSolver_Frame::update for one tensor.
 // SGD updates of up to SGD_ITEMS tensors.  Most tensors of a net are small (scales, biases, steps), and a launch for each is
 // what bounds an update; the blocks of one launch find their tensor in the table that comes with the arguments.  16 tensors
@@ -565,13 +609,6 @@ __global__ __launch_bounds__(64) void batchnorm_f32_stats_finish_kernel(double n
     if (threadIdx.x == 0) bn_write_stats(c, n, m, v, mean, variance, saved_mean, saved_variance, momentum);
 }
 
-// The SAT activation quantizer behind a normalisation: fp receives what goes into it (or null), the output what comes out;
-// alpha null: no quantizer
-struct BnSat {
-    float* fp;
-    float range;
-    const float* alpha;
-};
 template <int V>
 __device__ __forceinline__ void bn_store(float* p, size_t idx, const float* v)
 {
@@ -591,7 +628,7 @@ __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_apply_kernel(BnRange q, 
                                                                      float* __restrict__ variance, float* __restrict__ saved_mean,
                                                                      float* __restrict__ saved_variance, double momentum, int running,
                                                                      const float* __restrict__ x, const float* __restrict__ scale, const float* __restrict__ bias, double epsilon,
-                                                                     BnSat sat, float* __restrict__ y)
+                                                                     SatStore sat, float* __restrict__ y)
 {
     const int c = blockIdx.x;
     float m, v;
@@ -632,7 +669,7 @@ __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_apply_kernel(BnRange q, 
 __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_apply_flat_kernel(size_t total, int C, int plane, const float* __restrict__ x,
                                                                      const float* __restrict__ scale, const float* __restrict__ bias,
                                                                      const float* __restrict__ mean, const float* __restrict__ variance, double epsilon,
-                                                                     int eps_in_float, BnSat sat, float* __restrict__ y)
+                                                                     int eps_in_float, SatStore sat, float* __restrict__ y)
 {
     const float a = sat.alpha ? fabsf(sat.alpha[0]) : 0.0f;
     for (size_t i = (size_t)blockIdx.x * TBLOCK + threadIdx.x; i < total; i += (size_t)gridDim.x * TBLOCK) {
@@ -1135,7 +1172,9 @@ static int run_depthwise(const ConvF32& q, int pass, const float* a, const float
 
 // The direct kernel of forward and backward-data: the walk with 32-bit offsets and one mask bit per tap row and column, or
 // (dilated, larger) one load after the other.
-static int run_direct(const ConvF32& q, int pass, const float* x, const float* w, const float* bias, float beta, float* out, hipStream_t st)
+// (sat: done by the kernels of a spanning layer, which say so)
+static int run_direct(const ConvF32& q, int pass, const float* x, const float* w, const float* bias, float beta, float* out, hipStream_t st, const SatStore& sat = {},
+                      bool* sat_done = nullptr)
 {
     if (depthwise_strips(q)) return run_depthwise(q, pass, x, w, bias, beta, out, nullptr, 0, st);
     const bool bwd = pass == PASS_BWD_DATA;
@@ -1150,11 +1189,12 @@ static int run_direct(const ConvF32& q, int pass, const float* x, const float* w
         // (the first up to two of its waves a SIMD; a unit holds one block of the second, and three of the third; measured at the kernels)
         const dim3 small(ceil_div_i(q.B, 2), ceil_div_i(q.O, 2));
         if ((size_t)small.x * small.y <= 8 * (size_t)num_cus())
-            N2D2HIP_LAUNCH(conv_f32_chain_kernel<4>, small, dim3(64), 0, st, q.B, q.O, (int)K, x, w, bias, beta, out);
+            N2D2HIP_LAUNCH(conv_f32_chain_kernel<4>, small, dim3(64), 0, st, q.B, q.O, (int)K, x, w, bias, beta, sat, out);
         else if ((size_t)grid.x * grid.y <= (size_t)num_cus())
-            N2D2HIP_LAUNCH(conv_f32_chain_kernel<64>, grid, dim3(192), 0, st, q.B, q.O, (int)K, x, w, bias, beta, out);
+            N2D2HIP_LAUNCH(conv_f32_chain_kernel<64>, grid, dim3(192), 0, st, q.B, q.O, (int)K, x, w, bias, beta, sat, out);
         else
-            N2D2HIP_LAUNCH(conv_f32_chain_wave_kernel, grid, dim3(64), 0, st, q.B, q.O, (int)K, x, w, bias, beta, out);
+            N2D2HIP_LAUNCH(conv_f32_chain_wave_kernel, grid, dim3(64), 0, st, q.B, q.O, (int)K, x, w, bias, beta, sat, out);
+        if (sat_done) *sat_done = true;
         N2D2HIP_HIP_CHECK(hipGetLastError());
         return N2D2HIP_OK;
     }
@@ -1889,28 +1929,48 @@ using namespace n2d2hip;
 
 extern "C" {
 
+static int conv_forward(const char* who, const n2d2hip_conv_desc* desc, int B, int H, int W, const float* x, const float* w, const float* bias, float beta, float* y,
+                        const SatStore& sat, void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream)
+{
+    ConvF32 q;
+    int st = make_conv(desc, B, H, W, false, &q, who);
+    if (st != N2D2HIP_OK) return st;
+    N2D2HIP_REQUIRE(x && w && y, N2D2HIP_ERR_INVALID, "%s: null pointer", who);
+    bool sat_done = false;
+    const auto forward = [&] {
+        if (f32_path(q, PASS_FWD) == F32_PATH_GEMM) {
+            float* ws = (float*)workspace;
+            const size_t nws = workspace ? workspace_bytes / sizeof(float) : 0;
+            if (spans_input(q)) {
+                int pass;
+                const ConvF32 m = product_of(q, PASS_FWD, &pass);
+                // (without a workspace that holds its partial results: the convolution as it stands, whose kernels keep a tap in each
+                // of a wave's 64 lanes, or the direct kernels)
+                if (q.B <= 64 * GRID_Y && pass_workspace(m, pass) <= nws)
+                    return run_pass(m, pass, w, x, bias, 1, q.O, beta, y, ws, nws, (hipStream_t)stream);
+                if (many_taps(q)) return run_direct(q, PASS_FWD, x, w, bias, beta, y, (hipStream_t)stream, sat, &sat_done);
+            }
+            return run_pass(q, PASS_FWD, x, w, bias, q.oH * q.oW, q.O, beta, y, ws, nws, (hipStream_t)stream);
+        }
+        return run_direct(q, PASS_FWD, x, w, bias, beta, y, (hipStream_t)stream, sat, &sat_done);
+    };
+    st = forward();
+    if (st != N2D2HIP_OK || !sat.alpha || sat_done) return st;
+    return n2d2hip_sat_act_forward(y, sat.fp, (size_t)q.B * q.O * q.oH * q.oW, sat.range, sat.alpha, stream);
+}
+
 int n2d2hip_conv2d_f32_forward(const n2d2hip_conv_desc* desc, int B, int H, int W, const float* x, const float* w, const float* bias,
                                float beta, float* y, void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream)
 {
-    ConvF32 q;
-    const int st = make_conv(desc, B, H, W, false, &q, "n2d2hip_conv2d_f32_forward");
-    if (st != N2D2HIP_OK) return st;
-    N2D2HIP_REQUIRE(x && w && y, N2D2HIP_ERR_INVALID, "n2d2hip_conv2d_f32_forward: null pointer");
-    if (f32_path(q, PASS_FWD) == F32_PATH_GEMM) {
-        float* ws = (float*)workspace;
-        const size_t nws = workspace ? workspace_bytes / sizeof(float) : 0;
-        if (spans_input(q)) {
-            int pass;
-            const ConvF32 m = product_of(q, PASS_FWD, &pass);
-            // (without a workspace that holds its partial results: the convolution as it stands, whose kernels keep a tap in each
-            // of a wave's 64 lanes, or the direct kernels)
-            if (q.B <= 64 * GRID_Y && pass_workspace(m, pass) <= nws)
-                return run_pass(m, pass, w, x, bias, 1, q.O, beta, y, ws, nws, (hipStream_t)stream);
-            if (many_taps(q)) return run_direct(q, PASS_FWD, x, w, bias, beta, y, (hipStream_t)stream);
-        }
-        return run_pass(q, PASS_FWD, x, w, bias, q.oH * q.oW, q.O, beta, y, ws, nws, (hipStream_t)stream);
-    }
-    return run_direct(q, PASS_FWD, x, w, bias, beta, y, (hipStream_t)stream);
+    return conv_forward("n2d2hip_conv2d_f32_forward", desc, B, H, W, x, w, bias, beta, y, SatStore{}, workspace, workspace_bytes, stream);
+}
+
+int n2d2hip_conv2d_f32_forward_sat(const n2d2hip_conv_desc* desc, int B, int H, int W, const float* x, const float* w, const float* bias, float* y,
+                                   float* full_precision, float range, const float* alpha, void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream)
+{
+    N2D2HIP_REQUIRE(alpha && full_precision != y, N2D2HIP_ERR_INVALID, "n2d2hip_conv2d_f32_forward_sat: bad argument");
+    return conv_forward("n2d2hip_conv2d_f32_forward_sat", desc, B, H, W, x, w, bias, 0.0f, y, SatStore{full_precision, range, alpha}, workspace, workspace_bytes,
+                        stream);
 }
 
 int n2d2hip_conv2d_f32_backward_data(const n2d2hip_conv_desc* desc, int B, int H, int W, const float* w, const float* diff_y, float beta,
@@ -2154,7 +2214,7 @@ static int bn_ranges(int B, int C, int plane, int V)
 
 static int batchnorm_forward(const char* who, int B, int C, int H, int W, const float* x, const float* scale, const float* bias, float* mean, float* variance,
                              float* saved_mean, float* saved_variance, double epsilon, double moving_average_momentum, int use_running, float* y,
-                             const BnSat& sat, void* workspace, size_t workspace_bytes, hipStream_t stream)
+                             const SatStore& sat, void* workspace, size_t workspace_bytes, hipStream_t stream)
 {
     N2D2HIP_REQUIRE(B > 0 && C > 0 && H > 0 && W > 0 && x && scale && bias && mean && variance && y && epsilon > 0.0, N2D2HIP_ERR_INVALID,
                     "%s: bad argument", who);
@@ -2203,7 +2263,7 @@ int n2d2hip_batchnorm_f32_forward(int B, int C, int H, int W, const float* x, co
                                   int use_running, float* y, void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream)
 {
     return batchnorm_forward("n2d2hip_batchnorm_f32_forward", B, C, H, W, x, scale, bias, mean, variance, saved_mean, saved_variance, epsilon,
-                             moving_average_momentum, use_running, y, BnSat{nullptr, 0.0f, nullptr}, workspace, workspace_bytes, (hipStream_t)stream);
+                             moving_average_momentum, use_running, y, SatStore{nullptr, 0.0f, nullptr}, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 int n2d2hip_batchnorm_f32_forward_sat(int B, int C, int H, int W, const float* x, const float* scale, const float* bias, float* mean,
@@ -2213,7 +2273,7 @@ int n2d2hip_batchnorm_f32_forward_sat(int B, int C, int H, int W, const float* x
 {
     N2D2HIP_REQUIRE(alpha && range >= 1.0f && full_precision != y, N2D2HIP_ERR_INVALID, "n2d2hip_batchnorm_f32_forward_sat: bad argument");
     return batchnorm_forward("n2d2hip_batchnorm_f32_forward_sat", B, C, H, W, x, scale, bias, mean, variance, saved_mean, saved_variance, epsilon,
-                             moving_average_momentum, use_running, y, BnSat{full_precision, range, alpha}, workspace, workspace_bytes, (hipStream_t)stream);
+                             moving_average_momentum, use_running, y, SatStore{full_precision, range, alpha}, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 size_t n2d2hip_batchnorm_f32_backward_sat_workspace_bytes(int B, int C, int H, int W)
@@ -2556,6 +2616,24 @@ int n2d2hip_loss_f32(const float* target, const float* output, float* diff, size
         hipLaunchKernelGGL(loss_finish_kernel, dim3(1), dim3(TBLOCK), 0, (hipStream_t)stream, (const double*)workspace, blocks, 1.0 / batch, loss);
     N2D2HIP_HIP_CHECK(hipGetLastError());
     return N2D2HIP_OK;
+}
+
+int n2d2hip_softmax_loss_f32(const float* x, const float* target, float* y, float* diff, float* diff_x, int B, int C, int H, int W, double* loss, void* workspace,
+                             size_t workspace_bytes, n2d2hip_stream_t stream)
+{
+    N2D2HIP_REQUIRE(B > 0 && C > 0 && H > 0 && W > 0 && x && target && y && diff && loss, N2D2HIP_ERR_INVALID, "n2d2hip_softmax_loss_f32: bad argument");
+    const size_t n = (size_t)B * C * H * W;
+    N2D2HIP_REQUIRE(workspace && workspace_bytes >= n2d2hip_loss_workspace_bytes(n), N2D2HIP_ERR_WORKSPACE,
+                    "n2d2hip_softmax_loss_f32: workspace of %zu bytes, %zu needed", workspace_bytes, n2d2hip_loss_workspace_bytes(n));
+    if (n <= LOSS_ONE_BLOCK && C <= 16) {
+        N2D2HIP_LAUNCH_T(softmax_loss_f32_kernel, (16), dim3(1), dim3(TBLOCK), 0, (hipStream_t)stream, x, target, y, diff, diff_x, B * H * W, C, H * W, 1.0 / B, loss);
+        N2D2HIP_HIP_CHECK(hipGetLastError());
+        return N2D2HIP_OK;
+    }
+    int st = n2d2hip_softmax_f32_forward(x, y, B, C, H, W, stream);
+    if (st == N2D2HIP_OK) st = n2d2hip_loss_f32(target, y, diff, n, B, loss, workspace, workspace_bytes, stream);
+    if (st == N2D2HIP_OK && diff_x) st = n2d2hip_elemwise_sum_f32_backward(n, 1.0f, diff, 0.0f, diff_x, stream);
+    return st;
 }
 
 int n2d2hip_sgd_update_f32_batch(const n2d2hip_sgd_item* items, int count, n2d2hip_stream_t stream)
