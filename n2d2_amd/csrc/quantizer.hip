@@ -140,20 +140,26 @@ struct SatLevels {
 };
 // SAT weights of several tensors, in three launches at most: a learning net quantizes the weights of all its cells before a pass,
 // most of them few, and a launch each (seven for many weights with scaling) was what bounded them.  16 tensors fit a launch's arguments.
-//  * Few: one block computes the tensor, in the first launch.  Its tanh stay in registers; the blocks of several tensors run side by
-//    side.  (Instances by the weights per thread: skipping unused ones inside one instance made the compiler spill.)  What bounds it is
-//    that one compute unit's arithmetic, so it ends where two or three launches of many blocks take as long: us, one block / many, 6000
-//    weights 5.5 / 5.7, 8192 5.9 / 5.6, 10080 7.0 / 5.6, 16384 8.8 / 5.8; with scaling 8192 7.7 / 10.0, 12288 9.4 / 10.1, 16384 11.1 / 10.0.
+//  * From 1025 (with scaling 8193) to SAT_SELF weights, in the first launch: every block looks for the largest weight of the whole tensor itself, 16
+//    bytes a load, and computes 1024 levels.  tanh is taken of that one weight and of the block's own: it does not decrease (tanhf of
+//    every positive float compared with the next one's), so the largest weight has the largest tanh.  It ends where reading the tensor from
+//    L2 takes as long as the launch that leaves the blocks' maxima to a second one.  us, one block's or two launches / now: 2400 weights
+//    4.1 / 3.5, 10080 6.8 / 3.9, 36864 5.8 / 4.6, 65536 5.9 / 5.4; with scaling, three launches 16384 10.0 / 8.9.
+//  * Up to 1024, and 8192 with scaling: one block computes the tensor, in the first launch, its tanh in registers (instances by the
+//    weights per thread: skipping unused ones inside one instance made the compiler spill).  One compute unit's arithmetic bounds it; from
+//    there on many blocks are as fast (with scaling 8192 weights 7.8, 10080 9.4 / 8.5; without 1024 3.2 / 3.4).  So are up to 8192
+//    weights that are overwritten by their levels, which another block must not be reading, and those that are only divided by the
+//    largest (SAT_NONE, where nothing is quantized), whose launches the log has always had one by one.
 //  * More: the first launch leaves each block's max |tanh w|, and every block of the second one takes the maximum of those,
 //    at most 256, itself.  The second launch fills the chip, 8 blocks a compute unit, and all deal the weights to the XCDs alike, in
-//    runs of 256, so that the weights come from the XCD's own L2 the second time.  us: 16385 weights 5.8, 1048576 8.5, 4194304
-//    14.6, 16777216 52.
-//  * With scaling the second leaves each block's sums of the levels' differences from the first level and of their squares, in double, and a
-//    third divides the levels: every block adds the sums up itself.  (One pass for the mean, one for the squares, a block's launch
-//    behind each and the division before: 16385 weights 15.6 us, now 10.1; 163840 17.4 / 11.8; 1048576 22.2 / 17.4; 4194304 36.1 / 28.3;
+//    runs of 256, so that the weights come from the XCD's own L2 the second time.
+//  * With scaling the blocks that computed the levels leave the sums of the levels' differences from the first level and of their squares,
+//    in double, and a last launch divides the levels: every block adds the sums up itself.  (One pass for the mean, one for the squares, a
+//    block's launch behind each and the division before: 163840 weights 17.4 us, with sums 11.8; 1048576 22.2 / 17.4; 4194304 36.1 / 28.3;
 //    16777216 121.5 / 82.3.)  The workspace holds the sums of 448 blocks; from 2 M weights on those are of 1024 threads, which 16777216 need
 //    (124.5 with 256; 1048576 18.7 with 1024).
-constexpr int SAT_SMALL = 8, SAT_SMALL_SCALED = 12;     // weights per thread of a block of 1024 at most
+constexpr size_t SAT_SMALL = 8 * 1024;           // weights of one block's tensor at most
+constexpr size_t SAT_SELF = 64 * 1024;           // weights among which every block looks for the largest itself
 constexpr int SAT_BLOCKS = 256, SAT_BLOCKS2 = 2048;     // blocks of a larger tensor's first, and second or third launch at most
 constexpr int SAT_BLOCKS_SUMS = 448;             // of the second where each leaves its sums in the workspace
 constexpr size_t SAT_MANY = 2 << 20;             // scaled weights from which their blocks have 1024 threads
@@ -165,7 +171,13 @@ struct SatBatch {
     unsigned first[N + 1], first2[N + 1], first3[N + 1];        // first block of a tensor in each launch
     int count;
 };
-__host__ __device__ inline bool sat_small(const n2d2hip_sat_weight_item& t) { return t.n <= (size_t)(t.apply_scaling ? SAT_SMALL_SCALED : SAT_SMALL) * 1024; }
+enum class SatKind { SELF, SMALL, MANY };
+__host__ __device__ inline SatKind sat_kind(const n2d2hip_sat_weight_item& t)
+{
+    const bool in_place = (uintptr_t)t.w < (uintptr_t)(t.wq + t.n) && (uintptr_t)t.wq < (uintptr_t)(t.w + t.n);
+    if (!in_place && t.mode != N2D2HIP_SAT_NONE && t.n > (t.apply_scaling ? SAT_SMALL : 1024) && t.n <= SAT_SELF) return SatKind::SELF;
+    return t.n <= SAT_SMALL ? SatKind::SMALL : SatKind::MANY;
+}
 
 // SAT scaling, ref: SATQuantizer_Frame_Kernels.cpp:244-262: the n levels' mean, their unbiased variance about that mean rounded to
 // float, scaling = sqrt(var * outputs_size); from the sums of their differences d from one of them and of d * d, in double
@@ -219,6 +231,34 @@ __device__ __forceinline__ void sat_weight_small(const n2d2hip_sat_weight_item& 
     }
     if (threadIdx.x == 0) { t.stats[0] = m; t.stats[1] = scaling; }
 }
+// A block of 1024 threads of those that look for the largest weight themselves: a level a thread
+__device__ __forceinline__ void sat_weight_self(const n2d2hip_sat_weight_item& t, unsigned block)
+{
+    const float* __restrict__ w = t.w;
+    const int n = (int)t.n, own = (int)(block * 1024 + threadIdx.x), quads = ((uintptr_t)w & 15) == 0 ? n / 4 : 0;
+    const float mine = own < n ? w[own] : 0.0f, zeroth = w[0];
+    float m = 0.0f;
+#pragma unroll 8
+    for (int i = threadIdx.x; i < quads; i += 1024) {
+        const float4 v = ((const float4*)w)[i];
+        m = fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+    }
+#pragma unroll 4
+    for (int i = quads * 4 + threadIdx.x; i < n; i += 1024) m = fmaxf(m, fabsf(w[i]));
+    m = tanhf(block_max(m));
+    const SatLevels level(t.range, t.mode, m);
+    const float q = level(tanhf(mine));
+    if (own < n) t.wq[own] = q;
+    if (block == 0 && threadIdx.x == 0) { t.stats[0] = m; t.stats[1] = 1.0f; }
+    if (!t.apply_scaling) return;
+    const float tanh0 = tanhf(zeroth);
+    const double d = (double)q - (double)level(tanh0);
+    double sum = own < n ? d : 0.0, squares = own < n ? d * d : 0.0;
+    block_sums(sum, squares);
+    if (threadIdx.x) return;
+    ((double2*)((char*)t.workspace + SAT_SUMS))[block] = make_double2(sum, squares);
+    if (block == 0) ((float*)t.workspace)[SAT_BLOCKS] = tanh0;
+}
 template <int N>
 __global__ __launch_bounds__(1024) void sat_weight_first_kernel(const SatBatch<N> b)
 {
@@ -226,11 +266,13 @@ __global__ __launch_bounds__(1024) void sat_weight_first_kernel(const SatBatch<N
     if (N > 1)
         while (k + 1 < b.count && blockIdx.x >= b.first[k + 1]) ++k;
     const n2d2hip_sat_weight_item& t = b.item[k];
-    if (sat_small(t)) {
+    const SatKind kind = sat_kind(t);
+    if (kind == SatKind::SELF) {
+        sat_weight_self(t, blockIdx.x - b.first[k]);
+    } else if (kind == SatKind::SMALL) {
         if (t.n <= 1024) sat_weight_small<1>(t);
         else if (t.n <= 4 * 1024) sat_weight_small<4>(t);
-        else if (t.n <= 8 * 1024) sat_weight_small<8>(t);
-        else sat_weight_small<SAT_SMALL_SCALED>(t);
+        else sat_weight_small<SAT_SMALL / 1024>(t);
     } else {
         // (blocks 8 apart run on the same XCD: of 8 blocks, a multiple of which there is, each takes every 8th run of 256)
         const unsigned block = blockIdx.x - b.first[k], run = 8 * (4 * (block >> 3) + (threadIdx.x >> 8)) + (block & 7);
@@ -290,7 +332,8 @@ __global__ __launch_bounds__(1024) void sat_weight_scale_kernel(const SatBatch<N
         while (k + 1 < b.count && blockIdx.x >= b.first3[k + 1]) ++k;
     const n2d2hip_sat_weight_item& t = b.item[k];
     float* __restrict__ wq = t.wq;
-    const unsigned block = blockIdx.x - b.first3[k], count = b.first2[k + 1] - b.first2[k];
+    const unsigned block = blockIdx.x - b.first3[k];
+    const unsigned count = sat_kind(t) == SatKind::SELF ? b.first[k + 1] - b.first[k] : b.first2[k + 1] - b.first2[k];
     const double2* sums = (const double2*)((const char*)t.workspace + SAT_SUMS);
     const float shift = SatLevels(t.range, t.mode, t.stats[0])(((const float*)t.workspace)[SAT_BLOCKS]);
     double sum = 0.0, squares = 0.0;
@@ -500,14 +543,17 @@ static void sat_weight_launch(const n2d2hip_sat_weight_item* items, int count, h
     };
     for (int i = 0; i < count; ++i) {
         const size_t n = items[i].n;
-        const bool small = sat_small(items[i]), scaled = items[i].apply_scaling && !small;
+        const SatKind kind = sat_kind(items[i]);
+        const bool scaled = items[i].apply_scaling && kind != SatKind::SMALL;
         b.item[i] = items[i];
-        b.first[i + 1] = b.first[i] + (small ? 1u : (unsigned)std::min<size_t>((n + 8191) / 8192 * 8, SAT_BLOCKS));
-        b.first2[i + 1] = b.first2[i] + (small ? 0u : blocks(n, scaled ? SAT_BLOCKS_SUMS : SAT_BLOCKS2 * QBLOCK / threads));
+        b.first[i + 1] = b.first[i] + (kind == SatKind::SMALL ? 1u : kind == SatKind::SELF ? (unsigned)((n + 1023) / 1024)
+                                                                                           : (unsigned)std::min<size_t>((n + 8191) / 8192 * 8, SAT_BLOCKS));
+        b.first2[i + 1] = b.first2[i] + (kind != SatKind::MANY ? 0u : blocks(n, scaled ? SAT_BLOCKS_SUMS : SAT_BLOCKS2 * QBLOCK / threads));
         b.first3[i + 1] = b.first3[i] + (scaled ? blocks(n, SAT_BLOCKS2 * QBLOCK / threads) : 0u);
     }
     static_assert(SAT_SUMS % sizeof(double2) == 0 && SAT_SUMS + SAT_BLOCKS_SUMS * sizeof(double2) <= (size_t)PARTIALS * sizeof(double) + 256,
                   "a workspace holds the maxima and the sums");
+    static_assert((SAT_SELF + 1023) / 1024 <= SAT_BLOCKS_SUMS, "of the blocks that look for the largest weight themselves too");
     N2D2HIP_LAUNCH_T(sat_weight_first_kernel, (N), dim3(b.first[count]), dim3(1024), 0, st, b);
     if (b.first2[count])
         N2D2HIP_LAUNCH_T(sat_weight_second_kernel, (N), dim3(b.first2[count]), dim3(threads), 0, st, b);
