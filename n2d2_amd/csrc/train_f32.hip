@@ -557,16 +557,13 @@ __device__ __forceinline__ void bn_write_stats(int c, double n, float m, float v
     mean[c] = (float)((double)m * momentum + (double)mean[c] * (1.0 - momentum));
     variance[c] = (float)((double)unbiased * momentum + (double)variance[c] * (1.0 - momentum));
 }
-// A channel per blockIdx.x in gridDim.y blocks: one finishes by itself, several leave their sums in ws
+// -> the shift, and in t the block's sums of x, x - shift and (x - shift)^2 over its range of channel c
 template <int V>
-__global__ __launch_bounds__(1024) void batchnorm_f32_stats_kernel(BnRange q, double n, const float* __restrict__ x, double* __restrict__ ws,
-                                                                   float* __restrict__ mean, float* __restrict__ variance, float* __restrict__ saved_mean,
-                                                                   float* __restrict__ saved_variance, double momentum)
+__device__ __forceinline__ float bn_channel_sums(const BnRange& q, int c, const float* __restrict__ x, double* t)
 {
     constexpr int N = V ? V : 1;
-    const int c = blockIdx.x;
     const float shift = x[(size_t)c * q.plane];
-    double t[3] = {};
+    t[0] = t[1] = t[2] = 0.0;
     bn_walk<V>(q, c, [&](size_t idx) {
         float v[N];
         bn_load<N>(v, x, idx);
@@ -579,14 +576,59 @@ __global__ __launch_bounds__(1024) void batchnorm_f32_stats_kernel(BnRange q, do
         }
     });
     bn_block_sums<3>(t);
-    if (threadIdx.x) return;
-    if (gridDim.y == 1) {
-        float m, v;
-        bn_stats(n, shift, t, &m, &v);
-        bn_write_stats(c, n, m, v, mean, variance, saved_mean, saved_variance, momentum);
-    } else {
+    return shift;
+}
+template <int V>
+__device__ __forceinline__ void bn_store(float* p, size_t idx, const float* v)
+{
+    if (V == 4) *(float4*)(p + idx) = make_float4(v[0], v[1], v[2], v[3]);
+    else p[idx] = v[0];
+}
+
+// V values normalised (mean m, var the root), scaled by g, b added, and quantized
+template <int V, bool SAT>
+__device__ __forceinline__ void bn_apply(size_t idx, const float* __restrict__ x, float m, float var, float g, float b, const SatStore& sat, float a,
+                                         float* __restrict__ y)
+{
+    float t[V];
+    bn_load<V>(t, x, idx);
+#pragma unroll
+    for (int k = 0; k < V; ++k) t[k] = g * ((t[k] - m) / var) + b;
+    if (SAT) {
+        if (sat.fp) bn_store<V>(sat.fp, idx, t);
+#pragma unroll
+        for (int k = 0; k < V; ++k) t[k] = sat_quantize(t[k], sat.range, a);
+    }
+    bn_store<V>(y, idx, t);
+}
+
+// A channel per blockIdx.x in gridDim.y blocks: one finishes by itself, several leave their sums in ws.  With BN_APPLY or BN_APPLY_SAT the
+// one block normalises its channel too, as the kernel below does, and reads it again mostly from its cache (when, and what it gives: bn_whole()).
+enum { BN_SUMS_ONLY, BN_APPLY, BN_APPLY_SAT };
+template <int V, int THEN>
+__global__ __launch_bounds__(1024) void batchnorm_f32_stats_kernel(BnRange q, double n, const float* __restrict__ x, double* __restrict__ ws,
+                                                                   float* __restrict__ mean, float* __restrict__ variance, float* __restrict__ saved_mean,
+                                                                   float* __restrict__ saved_variance, double momentum, const float* __restrict__ scale,
+                                                                   const float* __restrict__ bias, double epsilon, SatStore sat, float* __restrict__ y)
+{
+    const int c = blockIdx.x;
+    float g = 0.0f, b = 0.0f, a = 0.0f;          // (loaded ahead of the sums)
+    if constexpr (THEN != BN_SUMS_ONLY) { g = scale[c]; b = bias[c]; }
+    if constexpr (THEN == BN_APPLY_SAT) a = fabsf(sat.alpha[0]);
+    double t[3];
+    const float shift = bn_channel_sums<V>(q, c, x, t);
+    if (THEN == BN_SUMS_ONLY && threadIdx.x) return;
+    if (THEN == BN_SUMS_ONLY && gridDim.y > 1) {
         double* o = ws + ((size_t)c * gridDim.y + blockIdx.y) * 4;
         o[0] = t[0]; o[1] = t[1]; o[2] = t[2]; o[3] = (double)shift;
+        return;
+    }
+    float m, v;
+    bn_stats(n, shift, t, &m, &v);
+    if (threadIdx.x == 0) bn_write_stats(c, n, m, v, mean, variance, saved_mean, saved_variance, momentum);
+    if constexpr (THEN != BN_SUMS_ONLY) {
+        const float var = (float)sqrt((double)v + epsilon);
+        bn_walk<V>(q, c, [&](size_t idx) { bn_apply<V, THEN == BN_APPLY_SAT>(idx, x, m, var, g, b, sat, a, y); });
     }
 }
 // The statistics of a channel from its blocks' sums, by the first wavefront of the block that asks
@@ -607,13 +649,6 @@ __global__ __launch_bounds__(64) void batchnorm_f32_stats_finish_kernel(double n
     float m, v;
     bn_split_stats(c, n, splits, ws, &m, &v);
     if (threadIdx.x == 0) bn_write_stats(c, n, m, v, mean, variance, saved_mean, saved_variance, momentum);
-}
-
-template <int V>
-__device__ __forceinline__ void bn_store(float* p, size_t idx, const float* v)
-{
-    if (V == 4) *(float4*)(p + idx) = make_float4(v[0], v[1], v[2], v[3]);
-    else p[idx] = v[0];
 }
 
 // y = scale * (x - mean) / sqrt(variance + epsilon) + bias.  eps_in_float: the inference branch of the reference adds
@@ -650,18 +685,7 @@ __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_apply_kernel(BnRange q, 
     const float var = running ? sqrtf(v + (float)epsilon) : (float)sqrt((double)v + epsilon);
     const float g = scale[c], b = bias[c];
     const float a = SAT ? fabsf(sat.alpha[0]) : 0.0f;
-    bn_walk<V>(q, c, [&](size_t idx) {
-        float t[V];
-        bn_load<V>(t, x, idx);
-#pragma unroll
-        for (int k = 0; k < V; ++k) t[k] = g * ((t[k] - m) / var) + b;
-        if (SAT) {
-            if (sat.fp) bn_store<V>(sat.fp, idx, t);
-#pragma unroll
-            for (int k = 0; k < V; ++k) t[k] = sat_quantize(t[k], sat.range, a);
-        }
-        bn_store<V>(y, idx, t);
-    });
+    bn_walk<V>(q, c, [&](size_t idx) { bn_apply<V, SAT>(idx, x, m, var, g, b, sat, a, y); });
 }
 
 // The same for small planes, whose channels lie in pieces, and for channels past 32-bit counts: one lane per value, the
@@ -2212,6 +2236,18 @@ static int bn_ranges(int B, int C, int plane, int V)
     return (int)std::min<size_t>(std::max(2048 / C, 1), blocks);
 }
 
+// Whether one block takes each channel, statistics and normalisation in one launch.  The second launch, and the statistics on their way
+// to it, take longer than what one block has to do while a channel is short, or while there are blocks for every compute unit; until the tensors
+// (three with a quantizer) outgrow the 256 MB of the last cache, where the many blocks of two launches keep the memory busier.  Single values
+// and pieces of a few a plane it would write line by line with other blocks: only where they are few in all.  us, two launches / one,
+// batch x channels x plane: 32 x 16 x 10^2 6.8 / 5.1, 33 x 256 x 14^2 10.1 / 7.8, 128 x 512 x 7^2 22.3 / 14.9, 64 x 512 x 14^2 22.0 / 17.1,
+// 32 x 512 x 28^2 29.2 / 25.6, with the quantizer 38.7 / 34.3, 256 x 2048 x 7^2 with it 114 / 126; 256 x 512 x 1 7.2 / 6.1, 256 x 2048 x 1 11.1 / 11.6.
+static bool bn_whole(int B, int C, int plane, int tensors)
+{
+    const size_t n = (size_t)B * plane;
+    return (n < 8192 || (C >= num_cus() && n < 65536)) && n * C * tensors <= ((size_t)64 << 20) && (plane >= 16 || n * C <= 128 * 1024);
+}
+
 static int batchnorm_forward(const char* who, int B, int C, int H, int W, const float* x, const float* scale, const float* bias, float* mean, float* variance,
                              float* saved_mean, float* saved_variance, double epsilon, double moving_average_momentum, int use_running, float* y,
                              const SatStore& sat, void* workspace, size_t workspace_bytes, hipStream_t stream)
@@ -2229,15 +2265,25 @@ static int batchnorm_forward(const char* who, int B, int C, int H, int W, const 
         N2D2HIP_REQUIRE(saved_mean && saved_variance, N2D2HIP_ERR_INVALID, "%s: the learning pass needs saved_mean and saved_variance", who);
         N2D2HIP_REQUIRE((size_t)B * H * W > 1, N2D2HIP_ERR_INVALID, "%s: batch statistics need more than one value per channel", who);
         splits = workspace && workspace_bytes >= n2d2hip_batchnorm_f32_workspace_bytes(B, C, H, W) ? bn_splits(B, C, H, W) : 1;
-        const BnLaunch l = bn_launch(B, C, plane, splits, (uintptr_t)x);
-        const auto stats = [&](auto W) {
-            constexpr int VEC = decltype(W)::value;
-            N2D2HIP_LAUNCH_T(batchnorm_f32_stats_kernel, (VEC), dim3(C, splits), dim3(l.block), 0, stream, l.q, n, x, (double*)workspace, mean, variance,
-                             saved_mean, saved_variance, moving_average_momentum);
+        const bool whole = bn_whole(B, C, plane, sat.fp ? 3 : 2);
+        if (whole) splits = 1;
+        const BnLaunch l = bn_launch(B, C, plane, splits, (uintptr_t)x | (whole ? (uintptr_t)y | (uintptr_t)sat.fp : 0));
+        const auto stats = [&](auto W, auto then) {
+            N2D2HIP_LAUNCH_T(batchnorm_f32_stats_kernel, (decltype(W)::value, decltype(then)::value), dim3(C, splits), dim3(l.block), 0, stream, l.q, n, x,
+                             (double*)workspace, mean, variance, saved_mean, saved_variance, moving_average_momentum, scale, bias, epsilon, sat, y);
         };
-        if (l.V == 4) stats(std::integral_constant<int, 4>{});
-        else if (l.V == 1) stats(std::integral_constant<int, 1>{});
-        else stats(std::integral_constant<int, 0>{});
+        const auto then = [&](auto W) {
+            if (!whole) stats(W, std::integral_constant<int, BN_SUMS_ONLY>{});
+            else if (sat.alpha) stats(W, std::integral_constant<int, BN_APPLY_SAT>{});
+            else stats(W, std::integral_constant<int, BN_APPLY>{});
+        };
+        if (l.V == 4) then(std::integral_constant<int, 4>{});
+        else if (l.V == 1) then(std::integral_constant<int, 1>{});
+        else stats(std::integral_constant<int, 0>{}, std::integral_constant<int, BN_SUMS_ONLY>{});       // (2^30 values a channel: never whole)
+        if (whole) {
+            N2D2HIP_HIP_CHECK(hipGetLastError());
+            return N2D2HIP_OK;
+        }
         if (splits > 1 && !walk)
             hipLaunchKernelGGL(batchnorm_f32_stats_finish_kernel, dim3(C), dim3(64), 0, stream, n, splits, (const double*)workspace, mean, variance,
                                saved_mean, saved_variance, moving_average_momentum);

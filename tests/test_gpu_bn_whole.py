@@ -1,0 +1,50 @@
+"""Batch normalisation whose statistics and values come from one launch: at the edges of the rule that chooses it, with planes and outputs that
+16-byte accesses do not fit, against 64 bits.  The statistics are sums in double (2^-24 relative for the one rounding of each, and of their
+moving averages); a value takes four roundings from them: 4 x 2^-24 of its terms, which are below 6 sigma here, 2e-6 absolute."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,C,H,W", [(1, 3, 1, 2), (2, 5, 3, 5), (2, 5, 4, 4), (13, 7, 3, 5), (31, 6, 16, 16), (32, 6, 16, 16), (1, 3, 1, 8191),
+                                     (128, 1024, 1, 1), (129, 1024, 1, 1), (42, 256, 14, 14), (8, 300, 13, 9)])
+@pytest.mark.parametrize("sat", [False, True])
+def test_forward(B, C, H, W, sat):
+    import torch
+    from n2d2_amd import capi, runtime
+    rng = np.random.default_rng(B * C + H)
+    x = rng.normal(1.5, 2.0, size=(B, C, H, W)).astype(np.float32)
+    scale, bias = rng.uniform(0.5, 1.5, C).astype(np.float32), rng.normal(0, 0.3, C).astype(np.float32)
+    n = B * H * W
+    x64 = x.astype(np.float64)
+    mean, var = x64.mean(axis=(0, 2, 3)), x64.var(axis=(0, 2, 3))
+    per = lambda v: v.astype(np.float64)[:, None, None]  # noqa: E731
+    want = per(scale) * (x64 - per(mean)) / np.sqrt(per(var) + 1e-5) + per(bias)
+    for offset in (0, 1):                        # of the tensors that are written: their loads and stores by 16 bytes or by 4
+        dev = lambda v: torch.from_numpy(v).cuda()  # noqa: E731
+        dx, ds, db, rm, rv = dev(x), dev(scale), dev(bias), torch.zeros(C, device="cuda"), torch.ones(C, device="cuda")
+        sm, sv = torch.empty(C, device="cuda"), torch.empty(C, device="cuda")
+        y, fp = (torch.full((x.size + 1,), -7.0, device="cuda")[offset:offset + x.size] for _ in range(2))
+        alpha = torch.full((1,), 1.25, device="cuda")
+        ws = torch.empty(int(capi.lib.n2d2hip_batchnorm_f32_workspace_bytes(B, C, H, W)), dtype=torch.uint8, device="cuda")
+        p = [t.data_ptr() for t in (dx, ds, db, rm, rv, sm, sv)]
+        if sat:
+            capi.check(capi.lib.n2d2hip_batchnorm_f32_forward_sat(B, C, H, W, *p, 1e-5, 0.25, 0, y.data_ptr(), fp.data_ptr(), 15.0, alpha.data_ptr(),
+                                                                  ws.data_ptr(), ws.numel(), runtime.stream_ptr()))
+        else:
+            capi.check(capi.lib.n2d2hip_batchnorm_f32_forward(B, C, H, W, *p, 1e-5, 0.25, 0, y.data_ptr(), ws.data_ptr(), ws.numel(), runtime.stream_ptr()))
+        torch.cuda.synchronize()
+        got = (fp if sat else y).cpu().numpy().reshape(x.shape)
+        tol = 2e-6 * max(1.0, np.abs(want).max())
+        if n > 2:
+            assert np.abs(got - want).max() <= tol
+        np.testing.assert_allclose(sm.cpu().numpy(), mean, rtol=2e-7, atol=2e-7)
+        np.testing.assert_allclose(sv.cpu().numpy(), var, rtol=1e-6)
+        np.testing.assert_allclose(rm.cpu().numpy(), 0.25 * mean, rtol=4e-7, atol=2e-7)
+        np.testing.assert_allclose(rv.cpu().numpy(), 0.25 * var * n / (n - 1) + 0.75, rtol=2e-6)
+        if sat:                                  # the quantizer of the values that were kept, in 32 bits as the kernel has it
+            c = np.clip(got, np.float32(0), np.float32(1.25))
+            q = np.floor(np.float32(15) * (c / np.float32(1.25)) + np.float32(0.5)) / np.float32(15) * np.float32(1.25)
+            z = y.cpu().numpy().reshape(x.shape)
+            assert (np.abs(z - q) > 1e-6).sum() <= 2 + x.size // 100000      # (ties)
