@@ -649,6 +649,18 @@ int n2d2hip_elemwise_sum_f32_forward(int nb_inputs, const float* const* inputs, 
  * ElemWiseCell_Frame::backPropagate, Sum, src/Cell/ElemWiseCell_Frame.cpp:194-233). */
 int n2d2hip_elemwise_sum_f32_backward(size_t n, float weight, const float* diff_y, float beta, float* diff_x,
                                       n2d2hip_stream_t stream);
+/* The sum and the SAT activation quantizer behind it in one pass: n2d2hip_elemwise_sum_f32_forward() and n2d2hip_sat_act_forward() on y, with
+ * full_precision (or NULL) as its copy. */
+int n2d2hip_elemwise_sum_f32_forward_sat(int nb_inputs, const float* const* inputs, size_t n, const float* weights,
+                                         const float* shifts, float* y, float* full_precision, float range, const float* alpha,
+                                         n2d2hip_stream_t stream);
+/* Backwards: n2d2hip_sat_act_backward() in place on diff_y, then n2d2hip_elemwise_sum_f32_backward() for input 0, 1, ..., with weights[k] and
+ * betas[k] into diff_x[k] (host arrays; the same tensor may come twice, as long as it is not diff_y).  The workspace is
+ * n2d2hip_quantizer_workspace_bytes()'s. */
+int n2d2hip_elemwise_sum_f32_backward_sat(int nb_inputs, size_t n, const float* weights, const float* betas,
+                                          float* const* diff_x, float* diff_y, const float* full_precision, float range,
+                                          const float* alpha, float beta_alpha, float* diff_alpha, void* workspace,
+                                          size_t workspace_bytes, n2d2hip_stream_t stream);
 /* Softmax over the channels of each pixel, one group (ref: src/Cell/SoftmaxCell_Frame.cpp:93-137). */
 int n2d2hip_softmax_f32_forward(const float* x, float* y, int B, int C, int H, int W, n2d2hip_stream_t stream);
 /* diff = target - output, formed in double; loss[0] (device double) = sum of squares / batch

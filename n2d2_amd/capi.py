@@ -50,6 +50,7 @@ SYMBOLS = [
     "n2d2hip_batchnorm_f32_backward_sat_workspace_bytes", "n2d2hip_batchnorm_f32_backward_sat",
     "n2d2hip_batchnorm_f32_forward", "n2d2hip_batchnorm_f32_backward", "n2d2hip_pool_max_f32_forward", "n2d2hip_pool_max_f32_backward",
     "n2d2hip_pool_average_f32_forward", "n2d2hip_pool_average_f32_backward", "n2d2hip_elemwise_sum_f32_forward", "n2d2hip_elemwise_sum_f32_backward",
+    "n2d2hip_elemwise_sum_f32_forward_sat", "n2d2hip_elemwise_sum_f32_backward_sat",
 ]
 
 
@@ -207,6 +208,8 @@ def load():
     lib.n2d2hip_pool_average_f32_backward.argtypes = [I, I, I, I, I, I, I, I, I, I, I, P, F, P, P]
     lib.n2d2hip_elemwise_sum_f32_forward.argtypes = [I, C.POINTER(C.c_void_p), SZ, C.POINTER(C.c_float), C.POINTER(C.c_float), P, P]
     lib.n2d2hip_elemwise_sum_f32_backward.argtypes = [SZ, F, P, F, P, P]
+    lib.n2d2hip_elemwise_sum_f32_forward_sat.argtypes = [I, C.POINTER(C.c_void_p), SZ, C.POINTER(C.c_float), C.POINTER(C.c_float), P, P, F, P, P]
+    lib.n2d2hip_elemwise_sum_f32_backward_sat.argtypes = [I, SZ, C.POINTER(C.c_float), C.POINTER(C.c_float), C.POINTER(C.c_void_p), P, P, F, P, F, P, P, SZ, P]
     return lib
 
 

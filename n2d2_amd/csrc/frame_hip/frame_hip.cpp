@@ -1618,6 +1618,16 @@ void SATQuantizerActivation_Frame_HIP<T>::back_propagate(const float* diffInput,
 }
 
 template <class T>
+void SATQuantizerActivation_Frame_HIP<T>::back_propagate_sum(float* diff, std::size_t size, const std::vector<float>& weights, const std::vector<float>& betas,
+                                                             const std::vector<float*>& diffInputs)
+{
+    const PreparedGradient g = prepareGradient(size);
+    ensureWorkspace(mWorkspace, mWorkspaceBytes, size);
+    checkStatus(n2d2hip_elemwise_sum_f32_backward_sat((int)diffInputs.size(), size, weights.data(), betas.data(), diffInputs.data(), diff, g.fullPrecision,
+                                                      g.range, g.alpha, g.beta, g.diffAlpha, mWorkspace, mWorkspaceBytes, mStream));
+}
+
+template <class T>
 float SATQuantizerActivation_Frame_HIP<T>::getAlpha()
 {
     lazyInit(0, false);

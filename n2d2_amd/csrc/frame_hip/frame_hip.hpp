@@ -1061,6 +1061,10 @@ public:
     // the same for back_propagate(): what it reads, and where alpha's gradient goes (beta: the part of what is there that stays)
     struct PreparedGradient { const float* fullPrecision; float range; const float* alpha; float beta; float* diffAlpha; };
     PreparedGradient prepareGradient(std::size_t size);
+    // back_propagate() in place on diff, the gradient of a sum's outputs, and from there to the sum's inputs: weights[k] times it + betas[k]
+    // times what is in diffInputs[k], in one pass
+    void back_propagate_sum(float* diff, std::size_t size, const std::vector<float>& weights, const std::vector<float>& betas,
+                            const std::vector<float*>& diffInputs);
 
 private:
     void lazyInit(std::size_t size, bool needCopy);

@@ -856,9 +856,16 @@ void ElemWiseCell_FrameTrain_HIP::propagate(bool inference)
     std::vector<const float*> ins;
     for (const DeviceFloats* t : mIns)
         ins.push_back(t->data());
-    checkStatus(n2d2hip_elemwise_sum_f32_forward((int)ins.size(), ins.data(), mOutputs.size(), mWeights.data(), mShifts.data(), mOutputs.data(),
-                                                 mStream));
-    activationPropagate(inference);
+    // (a SAT quantizer alone behind the sum is applied as that leaves)
+    if (const std::shared_ptr<SATQuantizerActivation_Frame_HIP<float> > sat = lonelySatQuantizer()) {
+        const auto to = sat->prepare(mOutputs.size(), inference);
+        checkStatus(n2d2hip_elemwise_sum_f32_forward_sat((int)ins.size(), ins.data(), mOutputs.size(), mWeights.data(), mShifts.data(), mOutputs.data(),
+                                                         to.fullPrecision, to.range, to.alpha, mStream));
+    } else {
+        checkStatus(n2d2hip_elemwise_sum_f32_forward((int)ins.size(), ins.data(), mOutputs.size(), mWeights.data(), mShifts.data(), mOutputs.data(),
+                                                     mStream));
+        activationPropagate(inference);
+    }
     mDiffInputs.clearValid();
 }
 
@@ -866,6 +873,22 @@ void ElemWiseCell_FrameTrain_HIP::backPropagate()
 {
     if (!mDiffInputs.isValid())
         return;
+    if (const std::shared_ptr<SATQuantizerActivation_Frame_HIP<float> > sat = lonelySatQuantizer()) {
+        // the quantizer's gradient and the inputs' in one pass
+        std::vector<float> weights, betas;
+        std::vector<float*> diffs;
+        for (size_t k = 0; k < mIns.size(); ++k) {
+            DeviceFloats* d = mDiffOuts[k];
+            if (!d || d->empty())
+                continue;
+            weights.push_back(mWeights[k]);
+            betas.push_back(d->isValid() ? 1.0f : 0.0f);
+            diffs.push_back(d->data());
+            d->setValid();
+        }
+        sat->back_propagate_sum(mDiffInputs.data(), mDiffInputs.size(), weights, betas, diffs);
+        return;
+    }
     activationBackPropagate();
     for (size_t k = 0; k < mIns.size(); ++k) {
         DeviceFloats* d = mDiffOuts[k];
