@@ -692,6 +692,10 @@ typedef struct {
     int clamp;
 } n2d2hip_sgd_item;
 int n2d2hip_sgd_update_f32_batch(const n2d2hip_sgd_item* items, int count, n2d2hip_stream_t stream);
+/* n2d2hip_sat_weight_backward_batch(grads), then that; an item that updates a gradient's weights (its data and diff are the gradient's w
+ * and diff_w) does so in the launch that computes the gradient. */
+int n2d2hip_sgd_update_f32_batch_sat(const n2d2hip_sgd_item* items, int count, const n2d2hip_sat_weight_grad_item* grads,
+                                     int nb_grads, n2d2hip_stream_t stream);
 
 #ifdef __cplusplus
 }

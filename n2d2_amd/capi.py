@@ -45,7 +45,7 @@ SYMBOLS = [
     "n2d2hip_sat_act_forward", "n2d2hip_sat_act_backward", "n2d2hip_lsq_forward", "n2d2hip_lsq_backward",
     "n2d2hip_conv2d_f32_forward", "n2d2hip_conv2d_f32_backward_data", "n2d2hip_conv2d_f32_backward_filter", "n2d2hip_conv2d_f32_backward", "n2d2hip_conv2d_f32_workspace_bytes",
     "n2d2hip_conv2d_f32_backward_bias", "n2d2hip_softmax_f32_forward", "n2d2hip_loss_workspace_bytes", "n2d2hip_loss_f32", "n2d2hip_softmax_loss_f32", "n2d2hip_conv2d_f32_forward_sat",
-    "n2d2hip_sgd_update_f32", "n2d2hip_sgd_update_f32_batch", "n2d2hip_rectifier_f32_forward", "n2d2hip_rectifier_f32_backward",
+    "n2d2hip_sgd_update_f32", "n2d2hip_sgd_update_f32_batch", "n2d2hip_sgd_update_f32_batch_sat", "n2d2hip_rectifier_f32_forward", "n2d2hip_rectifier_f32_backward",
     "n2d2hip_batchnorm_f32_workspace_bytes", "n2d2hip_batchnorm_f32_forward_sat",
     "n2d2hip_batchnorm_f32_backward_sat_workspace_bytes", "n2d2hip_batchnorm_f32_backward_sat",
     "n2d2hip_batchnorm_f32_forward", "n2d2hip_batchnorm_f32_backward", "n2d2hip_pool_max_f32_forward", "n2d2hip_pool_max_f32_backward",
@@ -191,6 +191,7 @@ def load():
     lib.n2d2hip_conv2d_f32_forward_sat.argtypes = [P, I, I, I, P, P, P, P, P, F, P, P, SZ, P]
     lib.n2d2hip_sgd_update_f32.argtypes = [P, P, SZ, F, F, F, P, I, F, F, P]
     lib.n2d2hip_sgd_update_f32_batch.argtypes = [C.POINTER(SgdItem), I, P]
+    lib.n2d2hip_sgd_update_f32_batch_sat.argtypes = [C.POINTER(SgdItem), I, C.POINTER(SatWeightGradItem), I, P]
     lib.n2d2hip_rectifier_f32_forward.argtypes = [P, SZ, F, F, P]
     lib.n2d2hip_rectifier_f32_backward.argtypes = [P, P, P, SZ, F, F, P]
     D = C.c_double

@@ -1342,7 +1342,12 @@ SGDUpdateScope::~SGDUpdateScope()
     if (!mOuter) return;
     sgdScope = nullptr;
     // (left by an exception: what came before it is still done; its own error is the one to report)
-    if (!mItems.empty()) (void)n2d2hip_sgd_update_f32_batch(mItems.data(), (int)mItems.size(), mStream);
+    if (mItems.empty()) return;
+    std::vector<n2d2hip_sat_weight_grad_item> grads;
+    try {
+        if (SATWeightsScope* scope = SATWeightsScope::current()) grads = scope->takeGradients(mStream);
+    } catch (const std::exception&) {}
+    (void)n2d2hip_sgd_update_f32_batch_sat(mItems.data(), (int)mItems.size(), grads.data(), (int)grads.size(), mStream);
 }
 
 void SGDUpdateScope::flush()
@@ -1351,7 +1356,10 @@ void SGDUpdateScope::flush()
     if (mItems.empty()) return;
     std::vector<n2d2hip_sgd_item> items;
     items.swap(mItems);
-    checkStatus(n2d2hip_sgd_update_f32_batch(items.data(), (int)items.size(), mStream));
+    // (gradients that wait for their launch go along with the weights' updates)
+    std::vector<n2d2hip_sat_weight_grad_item> grads;
+    if (SATWeightsScope* scope = SATWeightsScope::current()) grads = scope->takeGradients(mStream);
+    checkStatus(n2d2hip_sgd_update_f32_batch_sat(items.data(), (int)items.size(), grads.data(), (int)grads.size(), mStream));
 }
 
 SGDUpdateScope* SGDUpdateScope::current() { return sgdScope; }
@@ -1382,8 +1390,12 @@ void SGDSolver::update(float* data, const float* diff, std::size_t n, unsigned i
         mMomentumSize = n;
     }
     const n2d2hip_sgd_item item = {data, diff, n, plain ? nullptr : mMomentumData, rateDiff, (float)mMomentum, (float)mDecay * rate, 0.0f, 0.0f, 0};
-    if (SGDUpdateScope* scope = SGDUpdateScope::current()) scope->add(item, stream);
-    else checkStatus(n2d2hip_sgd_update_f32_batch(&item, 1, stream));
+    if (SGDUpdateScope* scope = SGDUpdateScope::current()) {
+        scope->add(item, stream);
+    } else {
+        if (SATWeightsScope* scope = SATWeightsScope::current()) scope->flush();
+        checkStatus(n2d2hip_sgd_update_f32_batch(&item, 1, stream));
+    }
 }
 
 template <> Registrar<SGDSolver> SGDSolver_Frame_HIP<float>::mRegistrar("Frame_HIP", SGDSolver_Frame_HIP<float>::create,
@@ -1446,6 +1458,15 @@ void SATWeightsScope::flush()
 }
 
 SATWeightsScope* SATWeightsScope::current() { return satScope; }
+
+std::vector<n2d2hip_sat_weight_grad_item> SATWeightsScope::takeGradients(void* stream)
+{
+    // (weights that are still to be quantized come before their update)
+    if (!mItems.empty() || stream != mStream) flush();
+    std::vector<n2d2hip_sat_weight_grad_item> grads;
+    grads.swap(mGrads);
+    return grads;
+}
 
 void SATWeightsScope::add(const n2d2hip_sat_weight_item& item, void* stream)
 {

@@ -886,6 +886,8 @@ public:
     static SATWeightsScope* current();
     void add(const n2d2hip_sat_weight_item& item, void* stream);
     void add(const n2d2hip_sat_weight_grad_item& item, void* stream);
+    // the gradients that are not launched yet, for the launch that updates their weights; those of another stream are launched
+    std::vector<n2d2hip_sat_weight_grad_item> takeGradients(void* stream);
 
 private:
     void launch(const std::vector<n2d2hip_sat_weight_item>& items, const std::vector<n2d2hip_sat_weight_grad_item>& grads, bool throws);

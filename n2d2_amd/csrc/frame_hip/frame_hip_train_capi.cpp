@@ -417,14 +417,13 @@ int fh_train_learn(void* net, const float* targets, size_t nTargets, int iterati
                 }
             }
             if (last != n.cells.back().get()) last->launchLoss(n.targets.data());
-            {
-                SATWeightsScope gradients;
-                for (auto c = n.cells.rbegin(); c != n.cells.rend(); ++c) (*c)->backPropagate();
-                gradients.flush();
-            }
-            SGDUpdateScope updates;              // (all tensors of the net in one launch)
+            // (all tensors' updates in one launch, the gradients of their weights' quantizers with them)
+            SATWeightsScope gradients;
+            for (auto c = n.cells.rbegin(); c != n.cells.rend(); ++c) (*c)->backPropagate();
+            SGDUpdateScope updates;
             for (auto c = n.cells.rbegin(); c != n.cells.rend(); ++c) (*c)->update();
             updates.flush();
+            gradients.flush();
         }
         // (only the last iteration's loss is asked for: the device runs through the others without a stop)
         if (iterations > 0

@@ -366,16 +366,9 @@ __global__ __launch_bounds__(QBLOCK) void sat_weight_backward_kernel(const SatGr
     const float* __restrict__ dq = t.diff_wq;
     const float* __restrict__ w = t.w;
     float* __restrict__ dw = t.diff_w;
-    const float mode_factor = b.mode_factor[k];
-    const float factor = t.apply_scaling ? __fmul_rn(t.stats[0], t.stats[1]) : t.stats[0];
-    const float inv_factor = 1.0f / factor;
-    for (size_t i = (size_t)(blockIdx.x - b.first[k]) * QBLOCK + threadIdx.x; i < t.n; i += (size_t)(b.first[k + 1] - b.first[k]) * QBLOCK) {
-        const float inv_cosh = 1.0f / coshf(w[i]);
-        float grad = __fmul_rn(__fmul_rn(inv_cosh, inv_cosh), inv_factor);
-        if (mode_factor != 0.0f)
-            grad = __fmul_rn(grad, mode_factor);
-        dw[i] = __fmul_rn(dq[i], grad);
-    }
+    const float mode_factor = b.mode_factor[k], inv_factor = sat_weight_inv_factor(t);
+    for (size_t i = (size_t)(blockIdx.x - b.first[k]) * QBLOCK + threadIdx.x; i < t.n; i += (size_t)(b.first[k + 1] - b.first[k]) * QBLOCK)
+        dw[i] = sat_weight_gradient(w[i], dq[i], inv_factor, mode_factor);
 }
 
 // -------------------------------------------------------- SAT activations
@@ -505,6 +498,14 @@ __global__ __launch_bounds__(QBLOCK) void lsq_backward_kernel(const float* dq, c
     end_of_pass(acc, partial, accumulate);
 }
 
+int sat_weight_grad_check(const n2d2hip_sat_weight_grad_item& t)
+{
+    N2D2HIP_REQUIRE(t.diff_wq && t.w && t.diff_w && t.stats, N2D2HIP_ERR_INVALID, "sat_weight_backward: null argument");
+    N2D2HIP_REQUIRE(t.n > 0, N2D2HIP_ERR_INVALID, "sat_weight_backward: empty tensor");
+    N2D2HIP_REQUIRE(t.mode >= N2D2HIP_SAT_NONE && t.mode <= N2D2HIP_SAT_NONE_ASYM, N2D2HIP_ERR_INVALID, "sat_weight_backward: bad mode %d", t.mode);
+    return N2D2HIP_OK;
+}
+
 } // namespace n2d2hip
 
 using namespace n2d2hip;
@@ -593,9 +594,7 @@ static void sat_weight_backward_launch(const n2d2hip_sat_weight_grad_item* items
         const n2d2hip_sat_weight_grad_item& t = items[i];
         b.item[i] = t;
         b.first[i + 1] = b.first[i] + ew_grid(t.n);
-        // ref: SATQuantizerCell_Frame.cpp:249-283: Asymmetric and FullRange have their own slope factor
-        if (t.mode == N2D2HIP_SAT_FULLRANGE) b.mode_factor[i] = 1.0f + 0.9998f / t.range;
-        else if (t.mode == N2D2HIP_SAT_ASYMRANGE || t.mode == N2D2HIP_SAT_NONE_ASYM) { const float r2 = floorf(t.range / 2.0f); b.mode_factor[i] = 1.0f + 1.0f / (2.0f * r2); }
+        b.mode_factor[i] = sat_weight_mode_factor(t);
     }
     hipLaunchKernelGGL(sat_weight_backward_kernel<N>, dim3(b.first[count]), dim3(QBLOCK), 0, st, b);
 }
@@ -665,10 +664,8 @@ int n2d2hip_sat_weight_backward_batch(const n2d2hip_sat_weight_grad_item* items,
 {
     N2D2HIP_REQUIRE(items && count > 0, N2D2HIP_ERR_INVALID, "sat_weight_backward: bad argument");
     for (int i = 0; i < count; ++i) {
-        const n2d2hip_sat_weight_grad_item& t = items[i];
-        N2D2HIP_REQUIRE(t.diff_wq && t.w && t.diff_w && t.stats, N2D2HIP_ERR_INVALID, "sat_weight_backward: null argument");
-        N2D2HIP_REQUIRE(t.n > 0, N2D2HIP_ERR_INVALID, "sat_weight_backward: empty tensor");
-        N2D2HIP_REQUIRE(t.mode >= N2D2HIP_SAT_NONE && t.mode <= N2D2HIP_SAT_NONE_ASYM, N2D2HIP_ERR_INVALID, "sat_weight_backward: bad mode %d", t.mode);
+        const int rc = sat_weight_grad_check(items[i]);
+        if (rc != N2D2HIP_OK) return rc;
     }
     for (int i = 0; i < count; i += SAT_ITEMS) {
         const int nb = std::min(count - i, SAT_ITEMS);

@@ -430,6 +430,23 @@ struct SgdBatch {
     unsigned first[N + 1];                       // first block of a tensor; the grid behind the last
     int count;
 };
+// The update of value i
+__device__ __forceinline__ void sgd_one(const n2d2hip_sgd_item& t, size_t i, float diff)
+{
+    float* __restrict__ data = t.data;
+    float* __restrict__ mom = t.momentum_data;
+    float v;
+    if (mom) {
+        float m = mom[i] * t.momentum;
+        m += t.rate_diff * diff;
+        if (t.decay_times_rate != 0.0f) m += -t.decay_times_rate * data[i];
+        mom[i] = m;
+        v = data[i] + m;
+    } else {
+        v = data[i] + t.rate_diff * diff;
+    }
+    data[i] = t.clamp ? fminf(fmaxf(v, t.clamp_min), t.clamp_max) : v;
+}
 template <int N>
 __global__ __launch_bounds__(TBLOCK) void sgd_f32_kernel(SgdBatch<N> b)
 {
@@ -437,22 +454,37 @@ __global__ __launch_bounds__(TBLOCK) void sgd_f32_kernel(SgdBatch<N> b)
     if (N > 1)
         while (k + 1 < b.count && blockIdx.x >= b.first[k + 1]) ++k;
     const n2d2hip_sgd_item& t = b.item[k];
-    float* __restrict__ data = t.data;
-    const float* __restrict__ diff = t.diff;
-    float* __restrict__ mom = t.momentum_data;
     const size_t n = t.n, step = (size_t)(b.first[k + 1] - b.first[k]) * TBLOCK;
-    for (size_t i = (size_t)(blockIdx.x - b.first[k]) * TBLOCK + threadIdx.x; i < n; i += step) {
-        float v;
-        if (mom) {
-            float m = mom[i] * t.momentum;
-            m += t.rate_diff * diff[i];
-            if (t.decay_times_rate != 0.0f) m += -t.decay_times_rate * data[i];
-            mom[i] = m;
-            v = data[i] + m;
-        } else {
-            v = data[i] + t.rate_diff * diff[i];
+    for (size_t i = (size_t)(blockIdx.x - b.first[k]) * TBLOCK + threadIdx.x; i < n; i += step) sgd_one(t, i, t.diff[i]);
+}
+// With the SAT quantizers' gradients, which the update alone waits for: grad_of says which of `grad` an item's diff is, -1: it is there
+// already.  A launch less at the end of every learning iteration, and one pass over the weights (240000 in six tensors, us: 4.8 + 5.2, now 6.1).
+constexpr int SGD_GRADS = 16;
+struct SgdSatBatch {
+    SgdBatch<SGD_ITEMS> sgd;
+    n2d2hip_sat_weight_grad_item grad[SGD_GRADS];
+    float mode_factor[SGD_GRADS];
+    signed char grad_of[SGD_ITEMS];
+};
+static_assert(sizeof(SgdSatBatch) <= 4096, "a launch's arguments");
+__global__ __launch_bounds__(TBLOCK) void sgd_sat_f32_kernel(SgdSatBatch b)
+{
+    int k = 0;
+    while (k + 1 < b.sgd.count && blockIdx.x >= b.sgd.first[k + 1]) ++k;
+    const n2d2hip_sgd_item& t = b.sgd.item[k];
+    const int from = b.grad_of[k];
+    const size_t n = t.n, step = (size_t)(b.sgd.first[k + 1] - b.sgd.first[k]) * TBLOCK;
+    const size_t i0 = (size_t)(blockIdx.x - b.sgd.first[k]) * TBLOCK + threadIdx.x;
+    if (from < 0) {
+        for (size_t i = i0; i < n; i += step) sgd_one(t, i, t.diff[i]);
+    } else {
+        const n2d2hip_sat_weight_grad_item& s = b.grad[from];
+        const float inv_factor = sat_weight_inv_factor(s), mode_factor = b.mode_factor[from];
+        for (size_t i = i0; i < n; i += step) {
+            const float d = sat_weight_gradient(t.data[i], s.diff_wq[i], inv_factor, mode_factor);
+            s.diff_w[i] = d;
+            sgd_one(t, i, d);
         }
-        data[i] = t.clamp ? fminf(fmaxf(v, t.clamp_min), t.clamp_max) : v;
     }
 }
 
@@ -2620,6 +2652,18 @@ __global__ __launch_bounds__(TBLOCK) void elemwise_sum_f32_backward_kernel(size_
     }
 }
 
+template <int N>
+static SgdBatch<N> sgd_batch(const n2d2hip_sgd_item* item, int count)
+{
+    SgdBatch<N> b = {};
+    b.count = count;
+    for (int i = 0; i < count; ++i) {
+        b.item[i] = item[i];
+        b.first[i + 1] = b.first[i] + (unsigned)grid_for(item[i].n);
+    }
+    return b;
+}
+
 extern "C" {
 
 static int elemwise_sum_forward(const char* who, int nb_inputs, const float* const* inputs, size_t n, const float* weights, const float* shifts, float* y,
@@ -2708,7 +2752,7 @@ int n2d2hip_softmax_loss_f32(const float* x, const float* target, float* y, floa
     return st;
 }
 
-int n2d2hip_sgd_update_f32_batch(const n2d2hip_sgd_item* items, int count, n2d2hip_stream_t stream)
+static int sgd_check(const n2d2hip_sgd_item* items, int count)
 {
     N2D2HIP_REQUIRE(items && count > 0, N2D2HIP_ERR_INVALID, "n2d2hip_sgd_update_f32: bad argument");
     for (int k = 0; k < count; ++k) {
@@ -2716,20 +2760,61 @@ int n2d2hip_sgd_update_f32_batch(const n2d2hip_sgd_item* items, int count, n2d2h
         N2D2HIP_REQUIRE(items[k].momentum_data || (items[k].momentum == 0.0f && items[k].decay_times_rate == 0.0f), N2D2HIP_ERR_INVALID,
                         "n2d2hip_sgd_update_f32: momentum or decay without a momentum buffer");
     }
-    const auto launch = [&](auto N_, const n2d2hip_sgd_item* item, int nb) {
-        constexpr int N = decltype(N_)::value;
-        SgdBatch<N> b = {};
-        b.count = nb;
-        for (int i = 0; i < nb; ++i) {
-            b.item[i] = item[i];
-            b.first[i + 1] = b.first[i] + (unsigned)grid_for(item[i].n);
-        }
-        hipLaunchKernelGGL(sgd_f32_kernel<N>, dim3(b.first[nb]), dim3(TBLOCK), 0, (hipStream_t)stream, b);
-    };
+    return N2D2HIP_OK;
+}
+int n2d2hip_sgd_update_f32_batch(const n2d2hip_sgd_item* items, int count, n2d2hip_stream_t stream)
+{
+    const int rc = sgd_check(items, count);
+    if (rc != N2D2HIP_OK) return rc;
     for (int k = 0; k < count; k += SGD_ITEMS) {
         const int nb = std::min(count - k, SGD_ITEMS);
-        if (nb == 1) launch(std::integral_constant<int, 1>{}, items + k, nb);
-        else launch(std::integral_constant<int, SGD_ITEMS>{}, items + k, nb);
+        if (nb == 1) {
+            const SgdBatch<1> b = sgd_batch<1>(items + k, nb);
+            hipLaunchKernelGGL(sgd_f32_kernel<1>, dim3(b.first[nb]), dim3(TBLOCK), 0, (hipStream_t)stream, b);
+        } else {
+            const SgdBatch<SGD_ITEMS> b = sgd_batch<SGD_ITEMS>(items + k, nb);
+            hipLaunchKernelGGL(sgd_f32_kernel<SGD_ITEMS>, dim3(b.first[nb]), dim3(TBLOCK), 0, (hipStream_t)stream, b);
+        }
+    }
+    N2D2HIP_HIP_CHECK(hipGetLastError());
+    return N2D2HIP_OK;
+}
+
+int n2d2hip_sgd_update_f32_batch_sat(const n2d2hip_sgd_item* items, int count, const n2d2hip_sat_weight_grad_item* grads, int nb_grads, n2d2hip_stream_t stream)
+{
+    int rc = sgd_check(items, count);
+    if (rc != N2D2HIP_OK) return rc;
+    N2D2HIP_REQUIRE(nb_grads >= 0 && (grads || nb_grads == 0), N2D2HIP_ERR_INVALID, "n2d2hip_sgd_update_f32_batch_sat: bad argument");
+    // whose gradient an item's is: at most one item's each; the others are computed first
+    std::vector<int> grad_of(count, -1);
+    std::vector<n2d2hip_sat_weight_grad_item> others;
+    for (int g = 0; g < nb_grads; ++g) {
+        rc = sat_weight_grad_check(grads[g]);
+        if (rc != N2D2HIP_OK) return rc;
+        int item = 0;
+        while (item < count && !(items[item].diff == grads[g].diff_w && items[item].data == grads[g].w && items[item].n == grads[g].n && grad_of[item] < 0)) ++item;
+        if (item < count) grad_of[item] = g;
+        else others.push_back(grads[g]);
+    }
+    if (!others.empty()) {
+        rc = n2d2hip_sat_weight_backward_batch(others.data(), (int)others.size(), stream);
+        if (rc != N2D2HIP_OK) return rc;
+    }
+    if ((int)others.size() == nb_grads) return n2d2hip_sgd_update_f32_batch(items, count, stream);
+    for (int k = 0; k < count;) {
+        int nb = 0, nb_sat = 0;
+        SgdSatBatch b = {};
+        for (; nb < SGD_ITEMS && k + nb < count; ++nb) {
+            const int g = grad_of[k + nb];
+            if (g >= 0 && nb_sat == SGD_GRADS) break;
+            b.grad_of[nb] = (signed char)(g < 0 ? -1 : nb_sat);
+            if (g < 0) continue;
+            b.grad[nb_sat] = grads[g];
+            b.mode_factor[nb_sat++] = sat_weight_mode_factor(grads[g]);
+        }
+        b.sgd = sgd_batch<SGD_ITEMS>(items + k, nb);
+        hipLaunchKernelGGL(sgd_sat_f32_kernel, dim3(b.sgd.first[nb]), dim3(TBLOCK), 0, (hipStream_t)stream, b);
+        k += nb;
     }
     N2D2HIP_HIP_CHECK(hipGetLastError());
     return N2D2HIP_OK;
