@@ -797,6 +797,39 @@ __device__ __forceinline__ void bn_finish_alpha(const BnSatGrad& sat)
 }
 __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_alpha_kernel(BnSatGrad sat) { bn_finish_alpha(sat); }
 
+// Three sums of V values of x and of the gradient in dv
+template <int N>
+__device__ __forceinline__ void bn_grad_terms(double* s, const float* xv, const float* dv, float m)
+{
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const double centred = (double)(xv[k] - m), d = (double)dv[k];
+        s[0] = __fma_rn(d, centred, s[0]);
+        s[1] += d;
+        s[2] += centred;
+    }
+}
+// dx = dy * scale / sigma + dVar * 2 (x - mean) / size + dMean / size.  In double, what a channel's values share worked out once a block:
+// dx = kd d + kc (x - mean) + k0, where there were two divisions a value, one of them in double (figures at the sums).
+struct BnData {
+    float m;
+    double kd, kc, k0;
+    __device__ BnData(float mean, float scale, double inv_sigma, float dmean, float dvariance, float size)
+        : m(mean), kd((double)scale * inv_sigma), kc((double)dvariance * 2.0 / (double)size), k0((double)(dmean / size))
+    {
+    }
+    template <int V>
+    __device__ void value(size_t idx, const float* __restrict__ x, const float* dy, float* dx) const
+    {
+        float xv[V], dv[V];
+        bn_load<V>(xv, x, idx);
+        bn_load<V>(dv, dy, idx);
+#pragma unroll
+        for (int k = 0; k < V; ++k) dv[k] = (float)__fma_rn(kd, (double)dv[k], __fma_rn(kc, (double)(xv[k] - m), k0));
+        bn_store<V>(dx, idx, dv);
+    }
+};
+
 // SAT: dy is first taken through the quantizer's gradient, in place (64 x 64 x 32 x 32, us: the quantizer's own pass 10.0, its end
 // 4.6 and the sums, then 9.8; together then 19.2)
 template <int V, bool SAT>
@@ -825,13 +858,7 @@ __global__ __launch_bounds__(1024) void batchnorm_f32_backward_sums_kernel(BnRan
             }
             bn_store<N>(dy, idx, dv);
         }
-#pragma unroll
-        for (int k = 0; k < N; ++k) {
-            const double centred = (double)(xv[k] - m), d = (double)dv[k];
-            s[0] = __fma_rn(d, centred, s[0]);
-            s[1] += d;
-            s[2] += centred;
-        }
+        bn_grad_terms<N>(s, xv, dv, m);
     });
     bn_block_sums<SAT ? BN_SUMS + 1 : BN_SUMS>(s);
     if (threadIdx.x) return;
@@ -860,9 +887,33 @@ __global__ __launch_bounds__(64) void batchnorm_f32_backward_finish_kernel(doubl
     bn_write_grads(c, t, dmean, dvariance, grads);
 }
 
-// dx = dy * scale / sigma + dVar * 2 (x - mean) / size + dMean / size, in ranges of a channel as the apply kernel, the end of the
-// sums before it with it.  In double, what a channel's values share worked out once a block: dx = kd d + kc (x - mean) + k, where
-// there were two divisions a value, one of them in double (figures at the sums).
+// Sums and values of channels that one block adds up, in one launch (when, and what it gives: bn_whole()).  dx may be dy.
+template <int V>
+__global__ __launch_bounds__(1024) void batchnorm_f32_backward_whole_kernel(BnRange q, double n, float size, const float* __restrict__ x,
+                                                                            const float* __restrict__ scale, const float* __restrict__ saved_mean,
+                                                                            const float* __restrict__ saved_variance, double epsilon, const float* dy,
+                                                                            BnGrads grads, float* dx)
+{
+    const int c = blockIdx.x;
+    const float m = saved_mean[c], g = scale[c], variance = saved_variance[c];
+    double s[BN_SUMS] = {}, t[5];
+    bn_walk<V>(q, c, [&](size_t idx) {
+        float xv[V], dv[V];
+        bn_load<V>(xv, x, idx);
+        bn_load<V>(dv, dy, idx);
+        bn_grad_terms<V>(s, xv, dv, m);
+    });
+    const double inv_sigma = bn_inv_sigma(variance, epsilon);
+    bn_block_sums<BN_SUMS>(s);
+    float dmean, dvariance;
+    bn_five_sums(t, s, g, inv_sigma);
+    bn_stats_grads(n, t, variance, epsilon, &dmean, &dvariance);
+    if (threadIdx.x == 0) bn_write_grads(c, t, dmean, dvariance, grads);
+    const BnData data(m, g, inv_sigma, dmean, dvariance, size);
+    bn_walk<V>(q, c, [&](size_t idx) { data.value<V>(idx, x, dy, dx); });
+}
+
+// The values (BnData), in ranges of a channel as the apply kernel, the end of the sums before it with it.
 template <int V>
 __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_backward_data_kernel(BnRange q, int splits, double n, const double* __restrict__ ws, float size,
                                                                             const float* __restrict__ x, const float* __restrict__ scale,
@@ -895,15 +946,8 @@ __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_backward_data_kernel(BnR
         dmean = grads.diff_saved_mean[c];
         dvariance = grads.diff_saved_variance[c];
     }
-    const double kd = (double)g * inv_sigma, kc = (double)dvariance * 2.0 / (double)size, k0 = (double)(dmean / size);
-    bn_walk<V>(q, c, [&](size_t idx) {
-        float xv[V], dv[V];
-        bn_load<V>(xv, x, idx);
-        bn_load<V>(dv, dy, idx);
-#pragma unroll
-        for (int k = 0; k < V; ++k) dv[k] = (float)__fma_rn(kd, (double)dv[k], __fma_rn(kc, (double)(xv[k] - m), k0));
-        bn_store<V>(dx, idx, dv);
-    });
+    const BnData data(m, g, inv_sigma, dmean, dvariance, size);
+    bn_walk<V>(q, c, [&](size_t idx) { data.value<V>(idx, x, dy, dx); });
 }
 
 // The same for small planes: one lane per value.
@@ -916,11 +960,8 @@ __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_backward_data_flat_kerne
     if (sat.alpha && blockIdx.x == 0) bn_finish_alpha(sat);
     for (size_t i = (size_t)blockIdx.x * TBLOCK + threadIdx.x; i < total; i += (size_t)gridDim.x * TBLOCK) {
         const int c = (int)((i / plane) % C);
-        const float var = (float)sqrt((double)saved_variance[c] + epsilon);
-        const float diff_normalized = dy[i] * scale[c];
-        const double gradient = (double)(diff_normalized / var) + (double)diff_saved_variance[c] * 2.0 * (double)(x[i] - saved_mean[c]) / (double)size
-                                + (double)(diff_saved_mean[c] / size);
-        dx[i] = (float)gradient;
+        const BnData data(saved_mean[c], scale[c], bn_inv_sigma(saved_variance[c], epsilon), diff_saved_mean[c], diff_saved_variance[c], size);
+        data.value<1>(i, x, dy, dx);
     }
 }
 
@@ -2274,6 +2315,8 @@ static int bn_ranges(int B, int C, int plane, int V)
 // and pieces of a few a plane it would write line by line with other blocks: only where they are few in all.  us, two launches / one,
 // batch x channels x plane: 32 x 16 x 10^2 6.8 / 5.1, 33 x 256 x 14^2 10.1 / 7.8, 128 x 512 x 7^2 22.3 / 14.9, 64 x 512 x 14^2 22.0 / 17.1,
 // 32 x 512 x 28^2 29.2 / 25.6, with the quantizer 38.7 / 34.3, 256 x 2048 x 7^2 with it 114 / 126; 256 x 512 x 1 7.2 / 6.1, 256 x 2048 x 1 11.1 / 11.6.
+// Backwards (three tensors): 32 x 16 x 10^2 6.5 / 4.7, 33 x 256 x 14^2 10.7 / 8.1, 128 x 512 x 7^2 27.5 / 17.9, 64 x 512 x 14^2 27.9 / 22.3, 32 x 512 x 28^2
+// 43.5 / 37.9.  (Behind a SAT quantizer alpha's gradient waits for every channel, so those stay two launches.)
 static bool bn_whole(int B, int C, int plane, int tensors)
 {
     const size_t n = (size_t)B * plane;
@@ -2372,6 +2415,13 @@ static int batchnorm_backward(const char* who, int B, int C, int H, int W, const
     const double n = (double)B * H * W;
     const int plane = H * W;
     const uintptr_t in = (uintptr_t)x | (uintptr_t)diff_y;
+    if (!sat.alpha && diff_x && bn_whole(B, C, plane, 3)) {
+        const BnLaunch w = bn_launch(B, C, plane, 1, in | (uintptr_t)diff_x);
+        hipLaunchKernelGGL(w.V == 4 ? batchnorm_f32_backward_whole_kernel<4> : batchnorm_f32_backward_whole_kernel<1>, dim3(C), dim3(w.block), 0, stream, w.q,
+                           n, (float)((size_t)B * H * W), x, scale, saved_mean, saved_variance, epsilon, (const float*)diff_y, grads, diff_x);
+        N2D2HIP_HIP_CHECK(hipGetLastError());
+        return N2D2HIP_OK;
+    }
     const BnLaunch l = bn_launch(B, C, plane, splits, in | (uintptr_t)sat.fp);
     sat.partial = (double*)workspace + (size_t)C * splits * BN_SUMS;
     sat.blocks = C * splits;
