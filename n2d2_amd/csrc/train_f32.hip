@@ -430,20 +430,19 @@ struct SgdBatch {
     unsigned first[N + 1];                       // first block of a tensor; the grid behind the last
     int count;
 };
-// The update of value i
-__device__ __forceinline__ void sgd_one(const n2d2hip_sgd_item& t, size_t i, float diff)
+// The update of value i by diff(i)
+template <class F>
+__device__ __forceinline__ void sgd_one(const n2d2hip_sgd_item& t, float* __restrict__ data, float* __restrict__ mom, size_t i, F diff)
 {
-    float* __restrict__ data = t.data;
-    float* __restrict__ mom = t.momentum_data;
     float v;
     if (mom) {
         float m = mom[i] * t.momentum;
-        m += t.rate_diff * diff;
+        m += t.rate_diff * diff(i);
         if (t.decay_times_rate != 0.0f) m += -t.decay_times_rate * data[i];
         mom[i] = m;
         v = data[i] + m;
     } else {
-        v = data[i] + t.rate_diff * diff;
+        v = data[i] + t.rate_diff * diff(i);
     }
     data[i] = t.clamp ? fminf(fmaxf(v, t.clamp_min), t.clamp_max) : v;
 }
@@ -454,8 +453,12 @@ __global__ __launch_bounds__(TBLOCK) void sgd_f32_kernel(SgdBatch<N> b)
     if (N > 1)
         while (k + 1 < b.count && blockIdx.x >= b.first[k + 1]) ++k;
     const n2d2hip_sgd_item& t = b.item[k];
+    float* __restrict__ data = t.data;
+    const float* __restrict__ diff = t.diff;
+    float* __restrict__ mom = t.momentum_data;
     const size_t n = t.n, step = (size_t)(b.first[k + 1] - b.first[k]) * TBLOCK;
-    for (size_t i = (size_t)(blockIdx.x - b.first[k]) * TBLOCK + threadIdx.x; i < n; i += step) sgd_one(t, i, t.diff[i]);
+    for (size_t i = (size_t)(blockIdx.x - b.first[k]) * TBLOCK + threadIdx.x; i < n; i += step)
+        sgd_one(t, data, mom, i, [=](size_t j) { return diff[j]; });
 }
 // With the SAT quantizers' gradients, which the update alone waits for: grad_of says which of `grad` an item's diff is, -1: it is there
 // already.  A launch less at the end of every learning iteration, and one pass over the weights (240000 in six tensors, us: 4.8 + 5.2, now 6.1).
@@ -473,17 +476,20 @@ __global__ __launch_bounds__(TBLOCK) void sgd_sat_f32_kernel(SgdSatBatch b)
     while (k + 1 < b.sgd.count && blockIdx.x >= b.sgd.first[k + 1]) ++k;
     const n2d2hip_sgd_item& t = b.sgd.item[k];
     const int from = b.grad_of[k];
+    float* __restrict__ data = t.data;
+    float* __restrict__ mom = t.momentum_data;
     const size_t n = t.n, step = (size_t)(b.sgd.first[k + 1] - b.sgd.first[k]) * TBLOCK;
     const size_t i0 = (size_t)(blockIdx.x - b.sgd.first[k]) * TBLOCK + threadIdx.x;
     if (from < 0) {
-        for (size_t i = i0; i < n; i += step) sgd_one(t, i, t.diff[i]);
+        const float* __restrict__ diff = t.diff;
+        for (size_t i = i0; i < n; i += step) sgd_one(t, data, mom, i, [=](size_t j) { return diff[j]; });
     } else {
         const n2d2hip_sat_weight_grad_item& s = b.grad[from];
         const float inv_factor = sat_weight_inv_factor(s), mode_factor = b.mode_factor[from];
         for (size_t i = i0; i < n; i += step) {
-            const float d = sat_weight_gradient(t.data[i], s.diff_wq[i], inv_factor, mode_factor);
+            const float d = sat_weight_gradient(data[i], s.diff_wq[i], inv_factor, mode_factor);
             s.diff_w[i] = d;
-            sgd_one(t, i, d);
+            sgd_one(t, data, mom, i, [=](size_t) { return d; });
         }
     }
 }
