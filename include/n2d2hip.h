@@ -615,6 +615,20 @@ int n2d2hip_batchnorm_f32_backward_sat(int B, int C, int H, int W, const float* 
                                        float beta_scale, float* diff_scale, float beta_bias, float* diff_bias,
                                        float* diff_saved_mean, float* diff_saved_variance, float* diff_x, void* workspace,
                                        size_t workspace_bytes, n2d2hip_stream_t stream);
+/* n2d2hip_batchnorm_f32_forward_sat() and the 2x2 max pooling of its y at stride 2, over planes of even sides, as n2d2hip_pool_max_f32_forward()
+ * does it, in the launches of the first where those write channel by channel.  Backwards: n2d2hip_pool_max_f32_backward() into diff_y, then
+ * n2d2hip_batchnorm_f32_backward_sat(). */
+int n2d2hip_batchnorm_f32_forward_sat_pool(int B, int C, int H, int W, const float* x, const float* scale, const float* bias,
+                                           float* mean, float* variance, float* saved_mean, float* saved_variance, double epsilon,
+                                           double moving_average_momentum, int use_running, float* y, float* full_precision,
+                                           float range, const float* alpha, float* pooled, int* argmax, void* workspace,
+                                           size_t workspace_bytes, n2d2hip_stream_t stream);
+int n2d2hip_batchnorm_f32_backward_sat_pool(int B, int C, int H, int W, const float* x, const float* scale, const float* saved_mean,
+                                            const float* saved_variance, double epsilon, const float* full_precision, float range,
+                                            const float* alpha, float beta_alpha, float* diff_alpha, const float* diff_pooled,
+                                            const int* argmax, float* diff_y, float beta_scale, float* diff_scale, float beta_bias,
+                                            float* diff_bias, float* diff_saved_mean, float* diff_saved_variance, float* diff_x,
+                                            void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream);
 /* Max pooling of float NCHW, one output per channel; output size as PoolCell computes it, (in + 2 pad - pool + stride) /
  * stride.  argmax {B,C,oH,oW} receives row * W + column of the first largest element of each window in row-major order,
  * -1 for a window that lies in the padding (output 0) (ref: PoolCell_Frame_Kernels::forwardMax with its ArgMax tensor,

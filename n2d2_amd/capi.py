@@ -46,7 +46,8 @@ SYMBOLS = [
     "n2d2hip_conv2d_f32_forward", "n2d2hip_conv2d_f32_backward_data", "n2d2hip_conv2d_f32_backward_filter", "n2d2hip_conv2d_f32_backward", "n2d2hip_conv2d_f32_workspace_bytes",
     "n2d2hip_conv2d_f32_backward_bias", "n2d2hip_softmax_f32_forward", "n2d2hip_loss_workspace_bytes", "n2d2hip_loss_f32", "n2d2hip_softmax_loss_f32", "n2d2hip_conv2d_f32_forward_sat",
     "n2d2hip_sgd_update_f32", "n2d2hip_sgd_update_f32_batch", "n2d2hip_sgd_update_f32_batch_sat", "n2d2hip_rectifier_f32_forward", "n2d2hip_rectifier_f32_backward",
-    "n2d2hip_batchnorm_f32_workspace_bytes", "n2d2hip_batchnorm_f32_forward_sat",
+    "n2d2hip_batchnorm_f32_workspace_bytes", "n2d2hip_batchnorm_f32_forward_sat", "n2d2hip_batchnorm_f32_forward_sat_pool",
+    "n2d2hip_batchnorm_f32_backward_sat_pool",
     "n2d2hip_batchnorm_f32_backward_sat_workspace_bytes", "n2d2hip_batchnorm_f32_backward_sat",
     "n2d2hip_batchnorm_f32_forward", "n2d2hip_batchnorm_f32_backward", "n2d2hip_pool_max_f32_forward", "n2d2hip_pool_max_f32_backward",
     "n2d2hip_pool_average_f32_forward", "n2d2hip_pool_average_f32_backward", "n2d2hip_elemwise_sum_f32_forward", "n2d2hip_elemwise_sum_f32_backward",
@@ -201,6 +202,8 @@ def load():
     lib.n2d2hip_batchnorm_f32_backward_sat_workspace_bytes.argtypes = [I, I, I, I]
     lib.n2d2hip_batchnorm_f32_backward_sat_workspace_bytes.restype = SZ
     lib.n2d2hip_batchnorm_f32_backward_sat.argtypes = [I, I, I, I, P, P, P, P, D, P, F, P, F, P, P, F, P, F, P, P, P, P, P, SZ, P]
+    lib.n2d2hip_batchnorm_f32_forward_sat_pool.argtypes = [I, I, I, I, P, P, P, P, P, P, P, D, D, I, P, P, F, P, P, P, P, SZ, P]
+    lib.n2d2hip_batchnorm_f32_backward_sat_pool.argtypes = [I, I, I, I, P, P, P, P, D, P, F, P, F, P, P, P, P, F, P, F, P, P, P, P, P, SZ, P]
     lib.n2d2hip_batchnorm_f32_forward_sat.argtypes = [I, I, I, I, P, P, P, P, P, P, P, D, D, I, P, P, F, P, P, SZ, P]
     lib.n2d2hip_batchnorm_f32_backward.argtypes = [I, I, I, I, P, P, P, P, D, P, F, P, F, P, P, P, P, P, SZ, P]
     lib.n2d2hip_pool_max_f32_forward.argtypes = [I, I, I, I, I, I, I, I, I, I, P, P, P, P]

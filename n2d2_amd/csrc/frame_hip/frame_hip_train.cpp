@@ -554,7 +554,7 @@ void BatchNormCell::setParameter(const std::string& name, double value)
 template <class T>
 BatchNormCell_FrameTrain_HIP<T>::BatchNormCell_FrameTrain_HIP(const DeepNet& /*deepNet*/, const std::string& name, unsigned int nbOutputs,
                                                               const std::shared_ptr<Activation>& activation)
-    : Cell(name, nbOutputs), mScaleSolver(std::make_shared<SGDSolver_Frame_HIP<float> >()),
+    : Cell(name, nbOutputs), mJoined(nullptr), mScaleSolver(std::make_shared<SGDSolver_Frame_HIP<float> >()),
       mBiasSolver(std::make_shared<SGDSolver_Frame_HIP<float> >()), mLearned(false)
 {
     mActivation = activation;
@@ -635,11 +635,30 @@ void BatchNormCell_FrameTrain_HIP<T>::initialize()
 }
 
 template <class T>
+bool BatchNormCell_FrameTrain_HIP<T>::joinConsumer(Cell_FrameTrain_HIP* consumer)
+{
+    if (mJoined) mJoined->mJoined = mJoined->mGradientWaits = false;
+    PoolCell_FrameTrain_HIP<T>* const pool = dynamic_cast<PoolCell_FrameTrain_HIP<T>*>(consumer);
+    const std::vector<unsigned int> two(2, 2), none(2, 0);
+    mJoined = pool && pool->mPooling == PoolCell::Max && pool->mPoolDims == two && pool->mStrideDims == two && pool->mPaddingDims == none && mOutW % 2 == 0
+                      && mOutH % 2 == 0 && lonelySatQuantizer() ? pool : nullptr;
+    if (mJoined) mJoined->mJoined = true;
+    return mJoined != nullptr;
+}
+
+template <class T>
 void BatchNormCell_FrameTrain_HIP<T>::propagate(bool inference)
 {
     // (a SAT quantizer alone behind the normalisation is applied as that leaves)
     const std::shared_ptr<SATQuantizerActivation_Frame_HIP<float> > sat = lonelySatQuantizer();
-    if (sat) {
+    if (sat && mJoined) {
+        const auto to = sat->prepare(mOutputs.size(), inference);
+        checkStatus(n2d2hip_batchnorm_f32_forward_sat_pool((int)mIn->dimB(), (int)mNbOutputs, (int)mInH, (int)mInW, mIn->data(), mScale.data(), mBias.data(),
+                                                           mMean.data(), mVariance.data(), mSavedMean.data(), mSavedVariance.data(), mEpsilon,
+                                                           mMovingAverageMomentum, inference ? 1 : 0, mOutputs.data(), to.fullPrecision, to.range, to.alpha,
+                                                           mJoined->mOutputs.data(), mJoined->mArgMax, mWorkspace.data(), mWorkspace.size() * sizeof(float),
+                                                           mStream));
+    } else if (sat) {
         const auto to = sat->prepare(mOutputs.size(), inference);
         checkStatus(n2d2hip_batchnorm_f32_forward_sat((int)mIn->dimB(), (int)mNbOutputs, (int)mInH, (int)mInW, mIn->data(), mScale.data(), mBias.data(),
                                                       mMean.data(), mVariance.data(), mSavedMean.data(), mSavedVariance.data(), mEpsilon,
@@ -680,7 +699,15 @@ void BatchNormCell_FrameTrain_HIP<T>::backPropagate()
     if (accumulate && mDiffOwn.size() != mDiffOut->size())
         mDiffOwn.resize(mDiffOut->dims());
     float* dst = !toInput ? nullptr : accumulate ? mDiffOwn.data() : mDiffOut->data();
-    if (sat) {
+    if (sat && mJoined && mJoined->mGradientWaits) {
+        mJoined->mGradientWaits = false;
+        const auto to = sat->prepareGradient(mDiffInputs.size());
+        checkStatus(n2d2hip_batchnorm_f32_backward_sat_pool((int)mIn->dimB(), (int)mNbOutputs, (int)mInH, (int)mInW, mIn->data(), mScale.data(),
+                                                            mSavedMean.data(), mSavedVariance.data(), mEpsilon, to.fullPrecision, to.range, to.alpha, to.beta,
+                                                            to.diffAlpha, mJoined->mDiffInputs.data(), mJoined->mArgMax, mDiffInputs.data(), betaScale,
+                                                            mDiffScale.data(), betaBias, mDiffBias.data(), mDiffSavedMean.data(), mDiffSavedVariance.data(), dst,
+                                                            mWorkspace.data(), mWorkspace.size() * sizeof(float), mStream));
+    } else if (sat) {
         const auto to = sat->prepareGradient(mDiffInputs.size());
         checkStatus(n2d2hip_batchnorm_f32_backward_sat((int)mIn->dimB(), (int)mNbOutputs, (int)mInH, (int)mInW, mIn->data(), mScale.data(),
                                                        mSavedMean.data(), mSavedVariance.data(), mEpsilon, to.fullPrecision, to.range, to.alpha, to.beta,
@@ -722,7 +749,7 @@ PoolCell_FrameTrain_HIP<T>::PoolCell_FrameTrain_HIP(const DeepNet& /*deepNet*/, 
                                                     unsigned int nbOutputs, const std::vector<unsigned int>& strideDims,
                                                     const std::vector<unsigned int>& paddingDims, Pooling pooling,
                                                     const std::shared_ptr<Activation>& activation)
-    : Cell(name, nbOutputs), PoolCell(poolDims, strideDims, paddingDims, pooling), mArgMax(nullptr)
+    : Cell(name, nbOutputs), PoolCell(poolDims, strideDims, paddingDims, pooling), mArgMax(nullptr), mJoined(false), mGradientWaits(false)
 {
     if (poolDims.size() != 2 || strideDims.size() != 2 || paddingDims.size() != 2)
         throw std::runtime_error("PoolCell_FrameTrain_HIP " + name + ": two-dimensional pooling expected");
@@ -761,7 +788,9 @@ void PoolCell_FrameTrain_HIP<T>::initialize()
 template <class T>
 void PoolCell_FrameTrain_HIP<T>::propagate(bool inference)
 {
-    if (mPooling == Max)
+    if (mJoined) {
+        // (the cell before has pooled as it wrote)
+    } else if (mPooling == Max)
         checkStatus(n2d2hip_pool_max_f32_forward((int)mIn->dimB(), (int)mNbOutputs, (int)mInH, (int)mInW, (int)mPoolDims[0], (int)mPoolDims[1],
                                                  (int)mStrideDims[0], (int)mStrideDims[1], (int)mPaddingDims[0], (int)mPaddingDims[1], mIn->data(),
                                                  mOutputs.data(), mArgMax, mStream));
@@ -782,7 +811,9 @@ void PoolCell_FrameTrain_HIP<T>::backPropagate()
     if (!mDiffOut || mDiffOut->empty())
         return;
     const float beta = mDiffOut->isValid() ? 1.0f : 0.0f;
-    if (mPooling == Max)
+    if (mJoined && !mDiffOut->isValid())
+        mGradientWaits = true;
+    else if (mPooling == Max)
         checkStatus(n2d2hip_pool_max_f32_backward((int)mIn->dimB(), (int)mNbOutputs, (int)mInH, (int)mInW, (int)mPoolDims[0], (int)mPoolDims[1],
                                                   (int)mStrideDims[0], (int)mStrideDims[1], (int)mPaddingDims[0], (int)mPaddingDims[1],
                                                   mDiffInputs.data(), mArgMax, beta, mDiffOut->data(), mStream));

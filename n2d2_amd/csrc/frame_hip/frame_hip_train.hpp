@@ -8,6 +8,7 @@
 #ifndef N2D2_FRAME_HIP_TRAIN_HPP
 #define N2D2_FRAME_HIP_TRAIN_HPP
 
+#include <algorithm>
 #include <mutex>
 
 #include "frame_hip.hpp"
@@ -106,6 +107,11 @@ public:
     // The stream this cell's kernels are launched on: whatever a caller copies into the cell's tensors between two of its
     // passes goes to the same stream, so that the order does not depend on a stream's implicit synchronisation.
     void* stream() const { return mStream; }
+    // Does the cell read that tensor?
+    virtual bool reads(const DeviceFloats& outputs) const { return mIn == &outputs; }
+    // A learning iteration in which `consumer`, the only reader of this cell's outputs, may be computed in this cell's launches:
+    // true, and from then on it is, until joinConsumer(nullptr).
+    virtual bool joinConsumer(Cell_FrameTrain_HIP* /*consumer*/) { return false; }
 
 protected:
     Cell_FrameTrain_HIP() : mIn(nullptr), mDiffOut(nullptr), mStream(nullptr), mLoss(nullptr), mLossWorkspace(nullptr), mLossWorkspaceBytes(0) {}
@@ -256,6 +262,9 @@ private:
     static Registrar<ActivationCell> mRegistrar;
 };
 
+template <class T>
+class PoolCell_FrameTrain_HIP;
+
 // include/Cell/BatchNormCell.hpp:36-160: Epsilon (1.0e-5), MovingAverageMomentum (0.1); scales 1, biases 0, means 0,
 // variances 0 until set or learned
 class BatchNormCell : public virtual Cell {
@@ -309,11 +318,14 @@ public:
     // What DeepNetQAT reads of this cell: the four vectors, Epsilon, and range and alpha of the SAT quantizer of its
     // activation (range 0 without one)
     BatchNormParameters getBatchNormParameters() const;
+    // a 2x2 max pooling of whole windows behind a SAT quantizer
+    bool joinConsumer(Cell_FrameTrain_HIP* consumer);
 
 protected:
     void setOutputsDims() { mOutW = mInW; mOutH = mInH; }
 
 private:
+    PoolCell_FrameTrain_HIP<T>* mJoined;
     void set(DeviceFloats& dev, std::vector<Float_T>& host, const std::vector<Float_T>& v);
     std::vector<Float_T> get(const DeviceFloats& dev, const std::vector<Float_T>& host) const;
     size_t parameterStride() const { return ((size_t)mNbOutputs + 63) / 64 * 64; }
@@ -351,7 +363,10 @@ protected:
     void setOutputsDims();
 
 private:
+    friend class BatchNormCell_FrameTrain_HIP<T>;
     int* mArgMax;
+    // joined to the cell whose outputs it pools: that one's next backPropagate() takes the gradient from here
+    bool mJoined, mGradientWaits;
     static Registrar<PoolCell> mRegistrar;
 };
 
@@ -372,6 +387,7 @@ public:
     // every input has the size of the first one
     void addInput(Cell_FrameTrain_HIP* parent);
     void addInput(DeviceFloats& inputs, DeviceFloats& diffOutputs);
+    bool reads(const DeviceFloats& outputs) const { return std::find(mIns.begin(), mIns.end(), &outputs) != mIns.end(); }
     void initialize();
     void propagate(bool inference = false);
     void backPropagate();

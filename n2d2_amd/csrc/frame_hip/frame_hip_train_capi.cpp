@@ -108,6 +108,22 @@ struct QuantizedWeights {
     TrainNet& n;
 };
 
+// Cells computed in the launches of the cell before, while it lives
+struct JoinedCells {
+    explicit JoinedCells(TrainNet& net) : n(net)
+    {
+        for (auto& c : n.cells) {
+            Cell_FrameTrain_HIP* reader = nullptr;
+            int readers = 0;
+            for (auto& o : n.cells)
+                if (o->reads(c->getOutputs())) { reader = o.get(); ++readers; }
+            if (readers == 1) c->joinConsumer(reader);
+        }
+    }
+    ~JoinedCells() { for (auto& c : n.cells) c->joinConsumer(nullptr); }
+    TrainNet& n;
+};
+
 Cell_FrameTrain_HIP* find(TrainNet& n, const char* name)
 {
     for (auto& c : n.cells)
@@ -394,6 +410,7 @@ int fh_train_learn(void* net, const float* targets, size_t nTargets, int iterati
         if (hipMemcpyAsync(n.targets.data(), n.toDevice.data() + LOSS, nTargets * sizeof(float), hipMemcpyHostToDevice, (hipStream_t)last->stream())
             != hipSuccess)
             throw std::runtime_error("fh_train_learn(): copy of the targets failed");
+        JoinedCells joined(n);
         for (int it = 0; it < iterations; ++it) {
             // the gradient towards the net's input is this iteration's: empty, or what another consumer of the input has
             // already put there (fh_train_preset_input_gradient)

@@ -640,19 +640,93 @@ __device__ __forceinline__ void bn_apply(size_t idx, const float* __restrict__ x
     bn_store<V>(y, idx, t);
 }
 
+// The 2x2 max pooling behind a normalisation and its quantizer: planes of whole windows, taken in units of two rows by VW columns.  On its own
+// the pooling of a small net is a launch that lasts as long as a launch does, each way; here it comes from values that are in registers.
+// us, launches one behind the other / joined: 32 x 6 x 28 x 28 forwards 4.5 + 4.8 + 3.4 / 4.6 + 5.6, backwards 3.2 + 6.1 / 5.7; 32 x 16 x 10 x 10 5.9 + 3.3 / 7.2,
+// 3.2 + 6.3 / 6.6; a LeNet iteration of 32 images 167 / 154.
+struct BnPool {
+    BnRange units;                               // unit_plane and dplane: the units of a plane; plane: its values
+    int W, row_units;                            // columns of a plane, units of two rows
+    DivF32 drow;                                 // division by row_units
+    float* y;
+    int* argmax;
+};
+// f(first value of a unit, the same within its plane, its first window) over the block's range of channel c
+template <int VW, class F>
+__device__ __forceinline__ void bn_walk_windows(const BnPool& p, int c, F f)
+{
+    const BnRange& q = p.units;
+    const size_t u0 = (size_t)blockIdx.y * q.chunk, u1 = u0 + q.chunk < q.units ? u0 + q.chunk : q.units;
+    for (int u = (int)u0 + (int)threadIdx.x; u < (int)u1; u += (int)blockDim.x) {
+        const int b = div_f32(u, q.dplane), in = u - b * q.unit_plane, row = div_f32(in, p.drow), col = in - row * p.row_units;
+        const size_t plane = (size_t)b * q.C + c;
+        const int first = 2 * row * p.W + col * VW;
+        f(plane * q.plane + first, first, plane * (q.plane / 4) + (size_t)row * (p.W / 2) + col * (VW / 2));
+    }
+}
+template <int VW>
+__device__ __forceinline__ void bn_load_row(float* dst, const float* __restrict__ p, size_t idx)
+{
+    if (VW == 4) {
+        bn_load<4>(dst, p, idx);
+    } else {
+        const float2 v = *(const float2*)(p + idx);
+        dst[0] = v.x; dst[1] = v.y;
+    }
+}
+template <int VW>
+__device__ __forceinline__ void bn_store_row(float* p, size_t idx, const float* v)
+{
+    if (VW == 4) bn_store<4>(p, idx, v);
+    else *(float2*)(p + idx) = make_float2(v[0], v[1]);
+}
+// A unit normalised, quantized and pooled: of a window's values the first largest in row-major order
+template <int VW>
+__device__ __forceinline__ void bn_apply_windows(size_t idx, int first, size_t window, const BnPool& p, const float* __restrict__ x, float m, float var,
+                                                 float g, float b, const SatStore& sat, float a, float* __restrict__ y)
+{
+    float t[2][VW];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) bn_load_row<VW>(t[r], x, idx + r * p.W);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+#pragma unroll
+        for (int k = 0; k < VW; ++k) t[r][k] = g * ((t[r][k] - m) / var) + b;
+        if (sat.fp) bn_store_row<VW>(sat.fp, idx + r * p.W, t[r]);
+#pragma unroll
+        for (int k = 0; k < VW; ++k) t[r][k] = sat_quantize(t[r][k], sat.range, a);
+        bn_store_row<VW>(y, idx + r * p.W, t[r]);
+    }
+#pragma unroll
+    for (int w = 0; w < VW / 2; ++w) {
+        float best = t[0][2 * w];
+        int where = first + 2 * w;
+#pragma unroll
+        for (int k = 1; k < 4; ++k)
+            if (t[k / 2][2 * w + k % 2] > best) {
+                best = t[k / 2][2 * w + k % 2];
+                where = first + (k / 2) * p.W + 2 * w + k % 2;
+            }
+        p.y[window + w] = best;
+        p.argmax[window + w] = where;
+    }
+}
+
 // A channel per blockIdx.x in gridDim.y blocks: one finishes by itself, several leave their sums in ws.  With BN_APPLY or BN_APPLY_SAT the
 // one block normalises its channel too, as the kernel below does, and reads it again mostly from its cache (when, and what it gives: bn_whole()).
-enum { BN_SUMS_ONLY, BN_APPLY, BN_APPLY_SAT };
+// BN_APPLY_SAT_POOL + VW: and pools, in units of VW columns.
+enum { BN_SUMS_ONLY, BN_APPLY, BN_APPLY_SAT, BN_APPLY_SAT_POOL };
 template <int V, int THEN>
 __global__ __launch_bounds__(1024) void batchnorm_f32_stats_kernel(BnRange q, double n, const float* __restrict__ x, double* __restrict__ ws,
                                                                    float* __restrict__ mean, float* __restrict__ variance, float* __restrict__ saved_mean,
                                                                    float* __restrict__ saved_variance, double momentum, const float* __restrict__ scale,
-                                                                   const float* __restrict__ bias, double epsilon, SatStore sat, float* __restrict__ y)
+                                                                   const float* __restrict__ bias, double epsilon, SatStore sat, float* __restrict__ y,
+                                                                   BnPool pool)
 {
     const int c = blockIdx.x;
     float g = 0.0f, b = 0.0f, a = 0.0f;          // (loaded ahead of the sums)
     if constexpr (THEN != BN_SUMS_ONLY) { g = scale[c]; b = bias[c]; }
-    if constexpr (THEN == BN_APPLY_SAT) a = fabsf(sat.alpha[0]);
+    if constexpr (THEN >= BN_APPLY_SAT) a = fabsf(sat.alpha[0]);
     double t[3];
     const float shift = bn_channel_sums<V>(q, c, x, t);
     if (THEN == BN_SUMS_ONLY && threadIdx.x) return;
@@ -666,7 +740,12 @@ __global__ __launch_bounds__(1024) void batchnorm_f32_stats_kernel(BnRange q, do
     if (threadIdx.x == 0) bn_write_stats(c, n, m, v, mean, variance, saved_mean, saved_variance, momentum);
     if constexpr (THEN != BN_SUMS_ONLY) {
         const float var = (float)sqrt((double)v + epsilon);
-        bn_walk<V>(q, c, [&](size_t idx) { bn_apply<V, THEN == BN_APPLY_SAT>(idx, x, m, var, g, b, sat, a, y); });
+        if constexpr (THEN > BN_APPLY_SAT_POOL) {
+            constexpr int VW = THEN - BN_APPLY_SAT_POOL;
+            bn_walk_windows<VW>(pool, c, [&](size_t idx, int first, size_t window) { bn_apply_windows<VW>(idx, first, window, pool, x, m, var, g, b, sat, a, y); });
+        } else {
+            bn_walk<V>(q, c, [&](size_t idx) { bn_apply<V, THEN == BN_APPLY_SAT>(idx, x, m, var, g, b, sat, a, y); });
+        }
     }
 }
 // The statistics of a channel from its blocks' sums, by the first wavefront of the block that asks
@@ -696,12 +775,13 @@ __global__ __launch_bounds__(64) void batchnorm_f32_stats_finish_kernel(double n
 // range writes the statistics.  The quantizer that follows a normalisation in a learning net is applied on the way out; it read
 // and wrote the tensor again.  64 x 64 x 32 x 32, us: statistics, their end, this and the quantizer 5.8 + 4.8 + 6.1 + 10.5, now
 // 6.0 + 12.9, of which 10 are the 50 MB.
-template <int V, bool SAT>
+// POOL: 0, or the columns of a unit of windows, which are pooled on the way out too (SAT only).
+template <int V, bool SAT, int POOL = 0>
 __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_apply_kernel(BnRange q, int splits, double n, const double* __restrict__ ws, float* __restrict__ mean,
                                                                      float* __restrict__ variance, float* __restrict__ saved_mean,
                                                                      float* __restrict__ saved_variance, double momentum, int running,
                                                                      const float* __restrict__ x, const float* __restrict__ scale, const float* __restrict__ bias, double epsilon,
-                                                                     SatStore sat, float* __restrict__ y)
+                                                                     SatStore sat, float* __restrict__ y, BnPool pool)
 {
     const int c = blockIdx.x;
     float m, v;
@@ -723,7 +803,10 @@ __global__ __launch_bounds__(TBLOCK) void batchnorm_f32_apply_kernel(BnRange q, 
     const float var = running ? sqrtf(v + (float)epsilon) : (float)sqrt((double)v + epsilon);
     const float g = scale[c], b = bias[c];
     const float a = SAT ? fabsf(sat.alpha[0]) : 0.0f;
-    bn_walk<V>(q, c, [&](size_t idx) { bn_apply<V, SAT>(idx, x, m, var, g, b, sat, a, y); });
+    if constexpr (POOL != 0)
+        bn_walk_windows<POOL>(pool, c, [&](size_t idx, int first, size_t window) { bn_apply_windows<POOL>(idx, first, window, pool, x, m, var, g, b, sat, a, y); });
+    else
+        bn_walk<V>(q, c, [&](size_t idx) { bn_apply<V, SAT>(idx, x, m, var, g, b, sat, a, y); });
 }
 
 // The same for small planes, whose channels lie in pieces, and for channels past 32-bit counts: one lane per value, the
@@ -838,11 +921,14 @@ struct BnData {
 
 // SAT: dy is first taken through the quantizer's gradient, in place (64 x 64 x 32 x 32, us: the quantizer's own pass 10.0, its end
 // 4.6 and the sums, then 9.8; together then 19.2)
-template <int V, bool SAT>
+// POOL: 0, or the columns of a unit of the windows behind the quantizer: dy is not read but made from the pooled tensor's gradient (in
+// pool.y), whose window chose one value each.
+template <int V, bool SAT, int POOL = 0>
 __global__ __launch_bounds__(1024) void batchnorm_f32_backward_sums_kernel(BnRange q, double n, const float* __restrict__ x,
                                                                            const float* __restrict__ scale, const float* __restrict__ saved_mean,
                                                                            const float* __restrict__ saved_variance, double epsilon,
-                                                                           float* __restrict__ dy, double* __restrict__ ws, BnGrads grads, BnSatGrad sat)
+                                                                           float* __restrict__ dy, double* __restrict__ ws, BnGrads grads, BnSatGrad sat,
+                                                                           BnPool pool)
 {
     constexpr int N = V ? V : 1;
     const int c = blockIdx.x;
@@ -850,7 +936,27 @@ __global__ __launch_bounds__(1024) void batchnorm_f32_backward_sums_kernel(BnRan
     const double inv_sigma = bn_inv_sigma(variance, epsilon);
     const float a = SAT ? fabsf(sat.alpha[0]) : 0.0f;
     double s[SAT ? BN_SUMS + 1 : BN_SUMS] = {};
-    bn_walk<V>(q, c, [&](size_t idx) {
+    if constexpr (POOL != 0) bn_walk_windows<POOL>(pool, c, [&](size_t idx, int first, size_t window) {
+        float d[POOL / 2], xv[2][POOL], fp[2][POOL];
+        int at[POOL / 2];
+#pragma unroll
+        for (int w = 0; w < POOL / 2; ++w) { d[w] = pool.y[window + w]; at[w] = pool.argmax[window + w] - first; }
+#pragma unroll
+        for (int r = 0; r < 2; ++r) { bn_load_row<POOL>(xv[r], x, idx + r * pool.W); bn_load_row<POOL>(fp[r], sat.fp, idx + r * pool.W); }
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            float dv[POOL];
+#pragma unroll
+            for (int k = 0; k < POOL; ++k) {
+                dv[k] = at[k / 2] == r * pool.W + k ? d[k / 2] : 0.0f;
+                s[BN_SUMS] += (double)__fmul_rn(sat_alpha_slope(fp[r][k], sat.range, a), dv[k]);
+                dv[k] = __fmul_rn(sat_input_slope(fp[r][k], a), dv[k]);
+            }
+            bn_store_row<POOL>(dy, idx + r * pool.W, dv);
+            bn_grad_terms<POOL>(s, xv[r], dv, m);
+        }
+    });
+    else bn_walk<V>(q, c, [&](size_t idx) {
         float xv[N], dv[N];
         bn_load<N>(xv, x, idx);
         bn_load<N>(dv, dy, idx);
@@ -2329,9 +2435,25 @@ static bool bn_whole(int B, int C, int plane, int tensors)
     return (n < 8192 || (C >= num_cus() && n < 65536)) && n * C * tensors <= ((size_t)64 << 20) && (plane >= 16 || n * C <= 128 * 1024);
 }
 
+// Windows that tile planes of even sides, from and to memory that the loads of `columns` allow: 4 or 2, 0: neither
+static int bn_pool_columns(int B, int H, int W, uintptr_t pointers)
+{
+    if (H % 2 || W % 2 || (size_t)B * H * W >= ((size_t)1 << 31)) return 0;
+    return W % 4 == 0 && pointers % 16 == 0 ? 4 : pointers % 8 == 0 ? 2 : 0;
+}
+static BnPool bn_pool(int B, int C, int H, int W, int columns, int blocks, float* y, int* argmax)
+{
+    BnPool p;
+    const int row = W / columns, plane = H / 2 * row;
+    p.units = {C, H * W, plane, div_of(plane), (size_t)B * plane, ((size_t)B * plane + blocks - 1) / blocks};
+    p.W = W; p.row_units = row; p.drow = div_of(row); p.y = y; p.argmax = argmax;
+    return p;
+}
+
 static int batchnorm_forward(const char* who, int B, int C, int H, int W, const float* x, const float* scale, const float* bias, float* mean, float* variance,
                              float* saved_mean, float* saved_variance, double epsilon, double moving_average_momentum, int use_running, float* y,
-                             const SatStore& sat, void* workspace, size_t workspace_bytes, hipStream_t stream)
+                             const SatStore& sat, void* workspace, size_t workspace_bytes, hipStream_t stream, int columns = 0, float* pooled = nullptr,
+                             int* argmax = nullptr)
 {
     N2D2HIP_REQUIRE(B > 0 && C > 0 && H > 0 && W > 0 && x && scale && bias && mean && variance && y && epsilon > 0.0, N2D2HIP_ERR_INVALID,
                     "%s: bad argument", who);
@@ -2351,10 +2473,13 @@ static int batchnorm_forward(const char* who, int B, int C, int H, int W, const 
         const BnLaunch l = bn_launch(B, C, plane, splits, (uintptr_t)x | (whole ? (uintptr_t)y | (uintptr_t)sat.fp : 0));
         const auto stats = [&](auto W, auto then) {
             N2D2HIP_LAUNCH_T(batchnorm_f32_stats_kernel, (decltype(W)::value, decltype(then)::value), dim3(C, splits), dim3(l.block), 0, stream, l.q, n, x,
-                             (double*)workspace, mean, variance, saved_mean, saved_variance, moving_average_momentum, scale, bias, epsilon, sat, y);
+                             (double*)workspace, mean, variance, saved_mean, saved_variance, moving_average_momentum, scale, bias, epsilon, sat, y,
+                             columns ? bn_pool(B, C, H, plane / H, columns, 1, pooled, argmax) : BnPool{});
         };
         const auto then = [&](auto W) {
             if (!whole) stats(W, std::integral_constant<int, BN_SUMS_ONLY>{});
+            else if (columns == 4) stats(W, std::integral_constant<int, BN_APPLY_SAT_POOL + 4>{});
+            else if (columns == 2) stats(W, std::integral_constant<int, BN_APPLY_SAT_POOL + 2>{});
             else if (sat.alpha) stats(W, std::integral_constant<int, BN_APPLY_SAT>{});
             else stats(W, std::integral_constant<int, BN_APPLY>{});
         };
@@ -2372,10 +2497,12 @@ static int batchnorm_forward(const char* who, int B, int C, int H, int W, const 
     if (walk) {
         const int ranges = bn_ranges(B, C, plane, V);
         const BnLaunch l = bn_launch(B, C, plane, ranges, (uintptr_t)x | (uintptr_t)y | (uintptr_t)sat.fp);
-        const auto kernel = V == 4 ? (sat.alpha ? batchnorm_f32_apply_kernel<4, true> : batchnorm_f32_apply_kernel<4, false>)
-                                   : (sat.alpha ? batchnorm_f32_apply_kernel<1, true> : batchnorm_f32_apply_kernel<1, false>);
+        const auto kernel = columns == 4 ? batchnorm_f32_apply_kernel<1, true, 4> : columns == 2 ? batchnorm_f32_apply_kernel<1, true, 2>
+                            : V == 4 ? (sat.alpha ? batchnorm_f32_apply_kernel<4, true> : batchnorm_f32_apply_kernel<4, false>)
+                                     : (sat.alpha ? batchnorm_f32_apply_kernel<1, true> : batchnorm_f32_apply_kernel<1, false>);
         hipLaunchKernelGGL(kernel, dim3(C, ranges), dim3(TBLOCK), 0, stream, l.q, splits, n, (const double*)workspace, mean, variance, saved_mean,
-                           saved_variance, moving_average_momentum, running ? 1 : 0, x, scale, bias, epsilon, sat, y);
+                           saved_variance, moving_average_momentum, running ? 1 : 0, x, scale, bias, epsilon, sat, y,
+                           columns ? bn_pool(B, C, H, W, columns, ranges, pooled, argmax) : BnPool{});
     } else {
         hipLaunchKernelGGL(batchnorm_f32_apply_flat_kernel, dim3(grid_for((size_t)B * C * plane)), dim3(TBLOCK), 0, stream, (size_t)B * C * plane, C, plane, x,
                            scale, bias, running ? (const float*)mean : (const float*)saved_mean, running ? (const float*)variance : (const float*)saved_variance,
@@ -2403,6 +2530,26 @@ int n2d2hip_batchnorm_f32_forward_sat(int B, int C, int H, int W, const float* x
                              moving_average_momentum, use_running, y, SatStore{full_precision, range, alpha}, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
+int n2d2hip_batchnorm_f32_forward_sat_pool(int B, int C, int H, int W, const float* x, const float* scale, const float* bias, float* mean,
+                                           float* variance, float* saved_mean, float* saved_variance, double epsilon, double moving_average_momentum,
+                                           int use_running, float* y, float* full_precision, float range, const float* alpha, float* pooled, int* argmax,
+                                           void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream)
+{
+    const char* who = "n2d2hip_batchnorm_f32_forward_sat_pool";
+    N2D2HIP_REQUIRE(alpha && range >= 1.0f && full_precision != y && pooled && argmax, N2D2HIP_ERR_INVALID, "%s: bad argument", who);
+    N2D2HIP_REQUIRE(B > 0 && C > 0 && H > 1 && W > 1 && H % 2 == 0 && W % 2 == 0, N2D2HIP_ERR_INVALID, "%s: planes of whole 2x2 windows expected", who);
+    const uintptr_t pointers = (uintptr_t)x | (uintptr_t)y | (uintptr_t)full_precision;
+    const int V = bn_launch(B, C, H * W, 1, pointers).V, columns = bn_pool_columns(B, H, W, pointers);
+    // (in one pass where the values are written channel by channel)
+    const bool learns = !use_running && moving_average_momentum != 0.0;
+    if (columns && V != 0 && (H * W >= BN_WALK_PLANE || (learns && bn_whole(B, C, H * W, full_precision ? 3 : 2))))
+        return batchnorm_forward(who, B, C, H, W, x, scale, bias, mean, variance, saved_mean, saved_variance, epsilon, moving_average_momentum, use_running, y,
+                                 SatStore{full_precision, range, alpha}, workspace, workspace_bytes, (hipStream_t)stream, columns, pooled, argmax);
+    const int rc = n2d2hip_batchnorm_f32_forward_sat(B, C, H, W, x, scale, bias, mean, variance, saved_mean, saved_variance, epsilon, moving_average_momentum,
+                                                     use_running, y, full_precision, range, alpha, workspace, workspace_bytes, stream);
+    return rc == N2D2HIP_OK ? n2d2hip_pool_max_f32_forward(B, C, H, W, 2, 2, 2, 2, 0, 0, y, pooled, argmax, stream) : rc;
+}
+
 size_t n2d2hip_batchnorm_f32_backward_sat_workspace_bytes(int B, int C, int H, int W)
 {
     if (B <= 0 || C <= 0 || H <= 0 || W <= 0)
@@ -2412,7 +2559,8 @@ size_t n2d2hip_batchnorm_f32_backward_sat_workspace_bytes(int B, int C, int H, i
 
 static int batchnorm_backward(const char* who, int B, int C, int H, int W, const float* x, const float* scale, const float* saved_mean,
                               const float* saved_variance, double epsilon, BnSatGrad sat, float* diff_y, const BnGrads& grads, float* diff_x,
-                              void* workspace, int splits, hipStream_t stream)
+                              void* workspace, int splits, hipStream_t stream, int columns = 0, const float* diff_pooled = nullptr,
+                              const int* argmax = nullptr)
 {
     N2D2HIP_REQUIRE(B > 0 && C > 0 && H > 0 && W > 0 && x && scale && saved_mean && saved_variance && diff_y && grads.diff_scale && grads.diff_bias
                         && grads.diff_saved_mean && grads.diff_saved_variance && epsilon > 0.0,
@@ -2431,12 +2579,13 @@ static int batchnorm_backward(const char* who, int B, int C, int H, int W, const
     const BnLaunch l = bn_launch(B, C, plane, splits, in | (uintptr_t)sat.fp);
     sat.partial = (double*)workspace + (size_t)C * splits * BN_SUMS;
     sat.blocks = C * splits;
-    const auto kernel = sat.alpha ? (l.V == 4 ? batchnorm_f32_backward_sums_kernel<4, true> : l.V == 1 ? batchnorm_f32_backward_sums_kernel<1, true>
+    const auto kernel = columns == 4 ? batchnorm_f32_backward_sums_kernel<1, true, 4> : columns == 2 ? batchnorm_f32_backward_sums_kernel<1, true, 2>
+                        : sat.alpha ? (l.V == 4 ? batchnorm_f32_backward_sums_kernel<4, true> : l.V == 1 ? batchnorm_f32_backward_sums_kernel<1, true>
                                                                                                 : batchnorm_f32_backward_sums_kernel<0, true>)
                                   : (l.V == 4 ? batchnorm_f32_backward_sums_kernel<4, false> : l.V == 1 ? batchnorm_f32_backward_sums_kernel<1, false>
                                                                                                  : batchnorm_f32_backward_sums_kernel<0, false>);
     hipLaunchKernelGGL(kernel, dim3(C, splits), dim3(l.block), 0, stream, l.q, n, x, scale, saved_mean, saved_variance, epsilon, diff_y, (double*)workspace,
-                       grads, sat);
+                       grads, sat, columns ? bn_pool(B, C, H, W, columns, splits, const_cast<float*>(diff_pooled), const_cast<int*>(argmax)) : BnPool{});
     const int V = bn_launch(B, C, plane, 1, in | (uintptr_t)diff_x).V;
     const bool walk = diff_x && plane >= BN_WALK_PLANE && V != 0;
     if (splits > 1 && !walk)
@@ -2485,6 +2634,31 @@ int n2d2hip_batchnorm_f32_backward_sat(int B, int C, int H, int W, const float* 
     return batchnorm_backward("n2d2hip_batchnorm_f32_backward_sat", B, C, H, W, x, scale, saved_mean, saved_variance, epsilon,
                               BnSatGrad{full_precision, range, alpha, nullptr, 0, beta_alpha, diff_alpha}, diff_y, grads, diff_x, workspace,
                               need ? bn_splits(B, C, H, W) : 1, (hipStream_t)stream);
+}
+
+int n2d2hip_batchnorm_f32_backward_sat_pool(int B, int C, int H, int W, const float* x, const float* scale, const float* saved_mean,
+                                            const float* saved_variance, double epsilon, const float* full_precision, float range, const float* alpha,
+                                            float beta_alpha, float* diff_alpha, const float* diff_pooled, const int* argmax, float* diff_y, float beta_scale,
+                                            float* diff_scale, float beta_bias, float* diff_bias, float* diff_saved_mean, float* diff_saved_variance,
+                                            float* diff_x, void* workspace, size_t workspace_bytes, n2d2hip_stream_t stream)
+{
+    const char* who = "n2d2hip_batchnorm_f32_backward_sat_pool";
+    N2D2HIP_REQUIRE(full_precision && alpha && diff_alpha && full_precision != diff_y && full_precision != diff_x && diff_pooled && argmax && diff_y,
+                    N2D2HIP_ERR_INVALID, "%s: bad argument", who);
+    N2D2HIP_REQUIRE(B > 0 && C > 0 && H > 1 && W > 1 && H % 2 == 0 && W % 2 == 0, N2D2HIP_ERR_INVALID, "%s: planes of whole 2x2 windows expected", who);
+    const size_t need = n2d2hip_batchnorm_f32_backward_sat_workspace_bytes(B, C, H, W);
+    N2D2HIP_REQUIRE(workspace && workspace_bytes >= need, N2D2HIP_ERR_WORKSPACE, "%s: workspace of %zu bytes needed", who, need);
+    const int columns = bn_pool_columns(B, H, W, (uintptr_t)x | (uintptr_t)full_precision | (uintptr_t)diff_y);
+    if (!columns) {
+        const int rc = n2d2hip_pool_max_f32_backward(B, C, H, W, 2, 2, 2, 2, 0, 0, diff_pooled, argmax, 0.0f, diff_y, stream);
+        return rc == N2D2HIP_OK ? n2d2hip_batchnorm_f32_backward_sat(B, C, H, W, x, scale, saved_mean, saved_variance, epsilon, full_precision, range, alpha,
+                                                                     beta_alpha, diff_alpha, diff_y, beta_scale, diff_scale, beta_bias, diff_bias,
+                                                                     diff_saved_mean, diff_saved_variance, diff_x, workspace, workspace_bytes, stream) : rc;
+    }
+    const BnGrads grads = {diff_scale, diff_bias, diff_saved_mean, diff_saved_variance, beta_scale, beta_bias};
+    return batchnorm_backward(who, B, C, H, W, x, scale, saved_mean, saved_variance, epsilon,
+                              BnSatGrad{full_precision, range, alpha, nullptr, 0, beta_alpha, diff_alpha}, diff_y, grads, diff_x, workspace,
+                              bn_splits(B, C, H, W), (hipStream_t)stream, columns, diff_pooled, argmax);
 }
 
 static bool pool_small(const PoolF32& q) { return (size_t)q.B * q.C * std::max((size_t)q.H * q.W, (size_t)q.oH * q.oW) < ((size_t)1 << 31) - TBLOCK; }
