@@ -2,7 +2,8 @@
 // image.  There both launches are mostly their fixed cost (2.5 us of 4 on this chip), and the kernel for many pixels
 // (dw_pw.hip), whose work-groups own 128 pixels and all their outputs, would leave most of the chip idle.
 //
-// A work-group owns 16 pixels x 32 outputs and computes the depthwise convolution of its pixels itself, once per 32 outputs:
+// A work-group owns 16 pixels x 32 outputs (64 or 128 where there are more images) and computes the depthwise convolution of its
+// pixels itself, once per 32 outputs:
 // what is computed again is 9 products an element, and shared are the latencies of one launch.  Its waves share the channels,
 // a chunk of 64 each (or two, past 512 channels), and work alone until their sums meet in LDS:
 //  * the 9 pixels of each output pixel and the chunk's tables go to the wave's own part of LDS by direct loads, 64 contiguous
@@ -29,6 +30,7 @@ namespace {
 // general rescale needs
 enum { DWS_W, DWS_C = 3, DWS_D, DWS_E, DWS_BIAS, DWS_A, DWS_B, DWS_ROWS = 12 };
 constexpr int OUTS = 32, PIXELS = 16, MAX_PARTS = 8;
+constexpr int MAX_BLOCKS = 8;                     // blocks of 16 outputs of a work-group at most
 constexpr int TILES_OUTS = 128;                   // a handle of at most so many outputs holds the kernel for many pixels too
 constexpr int STAGE_PIXELS = 9 * PIXELS * 64, STAGE = STAGE_PIXELS + DWS_ROWS * 64 * 4;      // bytes of LDS of a wave
 
@@ -50,12 +52,11 @@ struct DwPwSmallArgs {
 };
 
 // KIND of the depthwise cell's rescale (FAST: EPI_I24 with the bias folded in, no clamp before it, saturating to [0, 255]); GN:
-// groups of 16 channels in a chunk
-template <int KIND, bool FAST, int GN>
+// groups of 16 channels in a chunk; OB: blocks of 16 outputs
+template <int KIND, bool FAST, int GN, int OB>
 __global__ __launch_bounds__(64 * MAX_PARTS) void dw_pw_small_kernel(const DwPwSmallArgs q)
 {
     typedef const v4i __attribute__((address_space(1))) * GlobalQuad;
-    constexpr int OB = OUTS / 16;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];       // STAGE bytes a wave
     const int lane = threadIdx.x & 63, p = lane & 15, g = lane >> 4;
     const int part = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -158,10 +159,14 @@ __global__ __launch_bounds__(64 * MAX_PARTS) void dw_pw_small_kernel(const DwPwS
 }
 
 template <int KIND, bool FAST>
-void launch_groups(const DwPwSmallArgs& a, dim3 grid, hipStream_t stream)
+void launch_groups(const DwPwSmallArgs& a, int blocks, unsigned pixel_groups, hipStream_t stream)
 {
-    if (a.C == 32) N2D2HIP_LAUNCH_T(dw_pw_small_kernel, (KIND, FAST, 2), grid, dim3(64 * a.parts), a.parts * STAGE, stream, a);
-    else N2D2HIP_LAUNCH_T(dw_pw_small_kernel, (KIND, FAST, 4), grid, dim3(64 * a.parts), a.parts * STAGE, stream, a);
+    static_assert(MAX_BLOCKS * 1024 <= STAGE, "a wave's sums lie where its pixels were");
+    const dim3 grid((unsigned)(a.O / (16 * blocks)), pixel_groups), waves(64 * a.parts);
+    if (a.C == 32) N2D2HIP_LAUNCH_T(dw_pw_small_kernel, (KIND, FAST, 2, 2), grid, waves, a.parts * STAGE, stream, a);
+    else if (blocks == 2) N2D2HIP_LAUNCH_T(dw_pw_small_kernel, (KIND, FAST, 4, 2), grid, waves, a.parts * STAGE, stream, a);
+    else if (blocks == 4) N2D2HIP_LAUNCH_T(dw_pw_small_kernel, (KIND, FAST, 4, 4), grid, waves, a.parts * STAGE, stream, a);
+    else N2D2HIP_LAUNCH_T(dw_pw_small_kernel, (KIND, FAST, 4, MAX_BLOCKS), grid, waves, a.parts * STAGE, stream, a);
 }
 
 bool integer_bytes(const n2d2hip_act_s* a)
@@ -169,7 +174,18 @@ bool integer_bytes(const n2d2hip_act_s* a)
     return (a->args.kind == EPI_I24 || a->args.kind == EPI_I64) && a->min_out >= -128 && a->max_out <= 255;
 }
 
-long long work_groups(int O, long long pixels) { return (pixels + PIXELS - 1) / PIXELS * (O / OUTS); }
+long long work_groups(int O, long long pixels, int blocks = OUTS / 16) { return (pixels + PIXELS - 1) / PIXELS * (O / (16 * blocks)); }
+// of those, as many as are on the chip at once (by their LDS, 12 KB a wave)
+long long on_chip(int C) { return (long long)num_cus() * (163840 / (std::min(MAX_PARTS, (C + 63) / 64) * STAGE)); }
+// Blocks of 16 outputs of a work-group: the fewest with which all are on the chip at once.  More outputs share one depthwise convolution, and
+// fewer work-groups the chip.  us, 2 / 4 / 8 blocks: 512 -> 512, 14 x 14, one image 4.9 / 5.2 / 5.5, two 8.1 / 5.3 / 5.5, four 14.5 / 9.0 / 5.7.  (Up to 128 outputs the plan's lines
+// are those of 32, with the kernel for many pixels behind them.)
+int output_blocks(int C, int O, long long pixels)
+{
+    int blocks = OUTS / 16;
+    while (O > TILES_OUTS && C != 32 && blocks < MAX_BLOCKS && O % (32 * blocks) == 0 && work_groups(O, pixels, blocks) > on_chip(C)) blocks *= 2;
+    return blocks;
+}
 
 // Where both are faster than the cells' own launches: is the kernel for many pixels the faster one?  It gives a work-group 8 x 16
 // pixels and all their outputs, up to 256.  us, that kernel / this one: 32 -> 64 channels, 112 x 112 3.6 / 4.8, two images of 48 x 48
@@ -180,12 +196,14 @@ bool tiles_first(int C, int O, long long pixels) { return (C == 32 && O <= TILES
 // Is this kernel faster than the cells' own launches?
 bool small_wins(int C, int O, long long pixels)
 {
-    // Where all work-groups are on the chip at once (by their LDS, 12 KB a wave).  us, one launch and two, for output planes of
-    // 112 / 56 / 56 / 28 / 28 / 14 / 14 / 7 and 32 -> 64, 64 -> 128, 128 -> 128, 128 -> 256, 256 -> 256, 256 -> 512, 512 -> 512, 512 -> 1024 channels:
-    //   one image    4.8 7.6   4.3 8.1   4.6 6.6   4.1 5.8   4.6 6.1   4.2 5.7   5.2 6.1   4.7 5.8
-    //   two images   7.2 7.8   5.0 8.2   6.7 7.0*  4.6 6.3   6.8 6.9*  4.6 5.9   8.8 6.2*  4.8 5.9     * the rule declines
-    //   four        11.0 9.3*  7.6 8.7  10.0 8.0*  6.7 6.8*  9.8 7.2*  6.8 6.4* 16.0 7.3*  8.0 5.9*
-    return work_groups(O, pixels) <= (long long)num_cus() * (163840 / (std::min(MAX_PARTS, (C + 63) / 64) * STAGE));
+    // Where all work-groups are on the chip at once.  us, one launch / two, for one, two, four, eight and sixteen images (* the rule declines):
+    //   256 -> 256, 28 x 28   4.7 6.2   5.1 7.0   6.0 7.0   9.8 8.1*  14.6 10.5*
+    //   256 -> 512, 14 x 14   4.2 5.8   4.6 5.8   5.1 6.5   6.1 6.8   9.9 7.9*
+    //   512 -> 512, 14 x 14   4.9 6.1   5.3 6.3   5.7 7.3   9.7 7.8*  18.0 9.2*
+    //   512 -> 1024, 7 x 7    4.8 5.8   4.9 5.9   5.3 6.0   5.7 6.7   9.7 7.4*
+    //   1024 -> 1024, 7 x 7   5.9 6.4   6.0 6.5   6.5 6.7   6.9 7.8   12.0 8.9*
+    //   128 -> 256, 28 x 28   4.2 5.8   4.7 6.4   5.6 6.6   7.1 7.5   (from 9216 pixels on the kernel for many)
+    return work_groups(O, pixels, output_blocks(C, O, pixels)) <= on_chip(C);
 }
 
 } // namespace
@@ -361,12 +379,13 @@ int n2d2hip_dw_pw_small_forward(n2d2hip_dw_pw_small_t h, const n2d2hip_tensor* i
     a.out_xor = out_dtype == N2D2HIP_U8B ? 0x80808080u : 0u;
     a.dw_lo = h->dw->act->args.lo; a.dw_hi = h->dw->act->args.hi;
     a.pw_kind = h->pw->act->args.kind; a.pw_lo = h->pw->act->args.lo; a.pw_hi = h->pw->act->args.hi;
+    const int blocks = output_blocks(dd.C, dp.O, pixels);
     // (output tiles first: work-groups 8 apart share an XCD, whose L2 then holds an eighth of the 1x1 weights)
     for (a.first = 0; a.first < a.ntasks; a.first += SPAN) {
-        const dim3 grid((unsigned)(dp.O / OUTS), (unsigned)((std::min(SPAN, a.ntasks - a.first) + PIXELS - 1) / PIXELS));
-        if (h->fast) launch_groups<EPI_I24, true>(a, grid, stream);
-        else if (h->dw->act->args.kind == EPI_I24) launch_groups<EPI_I24, false>(a, grid, stream);
-        else launch_groups<EPI_I64, false>(a, grid, stream);
+        const unsigned groups = (unsigned)((std::min(SPAN, a.ntasks - a.first) + PIXELS - 1) / PIXELS);
+        if (h->fast) launch_groups<EPI_I24, true>(a, blocks, groups, stream);
+        else if (h->dw->act->args.kind == EPI_I24) launch_groups<EPI_I24, false>(a, blocks, groups, stream);
+        else launch_groups<EPI_I64, false>(a, blocks, groups, stream);
     }
     N2D2HIP_HIP_CHECK(hipGetLastError());
     return N2D2HIP_OK;
