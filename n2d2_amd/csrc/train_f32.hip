@@ -2058,7 +2058,7 @@ static int run_pass(const ConvF32& q, int pass, const float* a, const float* b, 
         const dim3 grid(std::min((total + 255) / 256, 4096));
         if (kind == PIXELS_3X3) hipLaunchKernelGGL(conv_f32_lay_weights3x3_kernel, grid, dim3(256), 0, st, b, ws, total, g.Q, g.qpad, g.Ch, g.qs, g.chs);
         else if (kind == PIXELS_PATCH)
-            N2D2HIP_LAUNCH(conv_f32_lay_parts_kernel, grid, dim3(256), 0, st, b, (v4u*)ws, total, g.Q, g.qpad / 16, g.Ch, g.T, g.qs, g.chs);
+            N2D2HIP_LAUNCH(conv_f32_lay_parts_kernel, dim3(std::min(ceil_div_i(total, LAY_THREADS), 16384)), dim3(LAY_THREADS), 0, st, b, (v4u*)ws, total, g.Q, g.qpad / 16, g.Ch, g.T, g.qs, g.chs);
         else if (kind == PIXELS_PARTS) {
             if (plans[0].chunks) N2D2HIP_LAUNCH_T(conv_f32_lay_taps_kernel, (true), grid, dim3(256), 0, st, g, b, (v4u*)ws, total);
             else N2D2HIP_LAUNCH_T(conv_f32_lay_taps_kernel, (false), grid, dim3(256), 0, st, g, b, (v4u*)ws, total);
